@@ -121,8 +121,8 @@ __global__ __launch_bounds__(kSmallThreads) void gms_small_kernel(
   // the weight addresses are scalar
   const unsigned long long mask_v = (size_t)block * 64 < (size_t)n_dst ? block_masks[block] : 0ull;
   const unsigned long long mask =
-      ((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(mask_v >> 32)) << 32) |
-      (unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)mask_v);
+      ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(mask_v >> 32)) << 32) |
+      (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(mask_v & 0xffffffffu));
   // this wave's share: the set bits number part, part + parts, ...
   unsigned long long todo = mask;
   if (parts > 1) {
