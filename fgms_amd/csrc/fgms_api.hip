@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <initializer_list>
 #include <map>
 #include <mutex>
 #include <utility>
@@ -477,9 +478,72 @@ Route route_of(const GmsArgs &a, const Plan *plan) {
 
 int run_gms_one(GmsArgs a, const Plan *plan);
 
+// ---- channel counts no tuned kernel takes: padded copies (fgms_pad.hip) -----------------------
+// Workspace slots of the copies (slots 0 .. 3: see fgms_internal.h).
+constexpr int kSlotPadIn = 4, kSlotPadOut = 5, kSlotPadWeights = 6, kSlotPadResult = 7;
+
+// May the call grow the stream's workspaces?  (Not under stream capture: the shape-agnostic
+// kernels, which need none, then serve it unless an earlier call has left them big enough.)
+bool workspaces_fit(hipStream_t s, std::initializer_list<std::pair<int, size_t>> wanted) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (!s || hipStreamIsCapturing(s, &st) != hipSuccess || st == hipStreamCaptureStatusNone) return true;
+  for (const auto &w : wanted)
+    if (workspace_bytes(s, w.first) < w.second) return false;
+  return true;
+}
+
+int up_to_power_of_two(int c, int least) {
+  int p = least;
+  while (p < c) p *= 2;
+  return p;
+}
+int up_to_32(int c) { return (c + 31) / 32 * 32; }
+
+size_t elem_size(int dtype) { return dtype == FGMS_F16 ? 2 : 4; }
+
+// `a` as it would look over padded copies (aligned, so any address will do).
+GmsArgs with_channels(GmsArgs a, int c_in, int c_out) {
+  a.c_in = c_in;
+  a.c_out = c_out;
+  a.src = a.w = (const void *)4096;
+  a.dst = (void *)4096;
+  return a;
+}
+
+bool tuned_gms(const GmsArgs &a, const Plan *plan) {
+  if (plan && !plan->groups.empty() && a.dense_k < 0) {
+    GmsArgs g = a;
+    g.k_vol = plan->groups.front()->k_vol;
+    return route_of(g, plan->groups.front()) != Route::kGeneric;
+  }
+  return route_of(a, plan) != Route::kGeneric;
+}
+
+// Widened channels of a forward / input-gradient pass that no tuned kernel takes as it is: the
+// skinny kernel's where its products are no more than the padded MFMA tile's eighth (it runs on
+// the vector ALUs), else multiples of the MFMA kernels' 32.
+bool padded_gms_channels(const GmsArgs &a, const Plan *plan, int *c_in, int *c_out) {
+  if (g_policy != 0 || tuned_gms(a, plan)) return false;
+  const int si = up_to_power_of_two(a.c_in, 4), so = up_to_power_of_two(a.c_out, 4);
+  if (si * so <= 256 && tuned_gms(with_channels(a, si, so), plan)) {
+    *c_in = si; *c_out = so;
+    return true;
+  }
+  *c_in = up_to_32(a.c_in); *c_out = up_to_32(a.c_out);
+  return tuned_gms(with_channels(a, *c_in, *c_out), plan);
+}
+
 // A pass over all offsets: one walk for plans of up to 64 offsets (or none), one per group of 64
 // offsets for larger kernels (the groups' results add up in the destination rows).
+int run_gms_padded(const GmsArgs &a, const Plan *plan, int c_in, int c_out, bool *done);
+
 int run_gms(GmsArgs a, const Plan *plan) {
+  int pi, po;
+  if ((a.dense_k >= 0 ? a.n_dense : a.n_pairs) > 0 && padded_gms_channels(a, plan, &pi, &po)) {
+    bool done = false;
+    const int rc = run_gms_padded(a, plan, pi, po, &done);
+    if (rc != FGMS_OK || done) return rc;
+  }
   if (!plan || plan->groups.empty() || a.dense_k >= 0) return run_gms_one(a, plan);
   plan_touch(plan, a.stream);
   const size_t esz = a.dtype == FGMS_F16 ? 2 : 4;
@@ -510,11 +574,179 @@ int run_gms_one(GmsArgs a, const Plan *plan) {
   }
 }
 
+// The pass over copies padded to c_in x c_out channels; *done = false (and nothing launched)
+// where their workspaces cannot be had now.
+int run_gms_padded(const GmsArgs &a, const Plan *plan, int c_in, int c_out, bool *done) {
+  const size_t esz = elem_size(a.dtype);
+  const int c_src = a.transpose_w ? a.c_out : a.c_in, c_dst = a.transpose_w ? a.c_in : a.c_out;
+  const int p_src = a.transpose_w ? c_out : c_in, p_dst = a.transpose_w ? c_in : c_out;
+  const size_t src_bytes = (size_t)a.n_src * p_src * esz, w_bytes = (size_t)a.k_vol * c_in * c_out * esz,
+               dst_bytes = (size_t)a.n_dst * p_dst * esz;
+  const int src_slot = a.transpose_w ? kSlotPadOut : kSlotPadIn;
+  *done = workspaces_fit(a.stream, {{src_slot, src_bytes}, {kSlotPadWeights, w_bytes}, {kSlotPadResult, dst_bytes}});
+  if (!*done) return FGMS_OK;
+  GmsArgs p = a;
+  p.c_in = c_in;
+  p.c_out = c_out;
+  void *src = nullptr, *w = nullptr, *dst = nullptr;
+  int rc;
+  if ((rc = workspace_get(a.stream, src_slot, src_bytes, &src)) || (rc = workspace_get(a.stream, kSlotPadWeights, w_bytes, &w)) ||
+      (rc = workspace_get(a.stream, kSlotPadResult, dst_bytes, &dst)))
+    return rc;
+  PadBatch pads{};
+  pads.add(a.src, src, (size_t)a.n_src, 1, 1, c_src, p_src, (int)esz);
+  pads.add(a.w, w, (size_t)a.k_vol, a.c_in, c_in, a.c_out, c_out, (int)esz);
+  pads.add(nullptr, dst, (size_t)a.n_dst, 1, 1, p_dst, p_dst, (int)esz);
+  if ((rc = launch_pad(pads, a.dtype, a.stream))) return rc;
+  p.src = src;
+  p.w = w;
+  p.dst = dst;
+  if ((rc = run_gms(p, plan))) return rc;
+  return launch_crop_add(dst, a.dst, (size_t)a.n_dst, c_dst, p_dst, a.dtype, a.stream);
+}
+
+// Widened channels of a weight gradient no MFMA / skinny kernel takes as it is.
+bool padded_wgrad_channels(const WgradArgs &a, int *c_in, int *c_out) {
+  if (g_policy != 0 || mfma_wgrad_supported(a)) return false;
+  WgradArgs p = a;
+  p.in = p.gout = (const void *)4096;
+  if (a.c_in <= 16 && a.c_out <= 64) {
+    p.c_in = up_to_power_of_two(a.c_in, 4);
+    p.c_out = up_to_power_of_two(a.c_out, 16);
+  } else {
+    p.c_in = up_to_32(a.c_in);
+    p.c_out = up_to_32(a.c_out);
+  }
+  *c_in = p.c_in; *c_out = p.c_out;
+  return mfma_wgrad_supported(p);
+}
+
+// The weight gradient over padded copies of the rows (as above); its fp32 sums are cropped when
+// they are added to the caller's tensor.
+int run_wgrad_padded(const WgradArgs &a, int c_in, int c_out, bool *done) {
+  const size_t esz = elem_size(a.dtype);
+  const size_t in_bytes = (size_t)a.n_in * c_in * esz, gout_bytes = (size_t)a.n_out * c_out * esz;
+  *done = workspaces_fit(a.stream, {{kSlotPadIn, in_bytes}, {kSlotPadOut, gout_bytes}, {1, (size_t)a.k_vol * c_in * c_out * sizeof(float)}});
+  if (!*done) return FGMS_OK;
+  void *in = nullptr, *gout = nullptr;
+  int rc;
+  if ((rc = workspace_get(a.stream, kSlotPadIn, in_bytes, &in)) || (rc = workspace_get(a.stream, kSlotPadOut, gout_bytes, &gout)))
+    return rc;
+  PadBatch pads{};
+  pads.add(a.in, in, (size_t)a.n_in, 1, 1, a.c_in, c_in, (int)esz);
+  pads.add(a.gout, gout, (size_t)a.n_out, 1, 1, a.c_out, c_out, (int)esz);
+  if ((rc = launch_pad(pads, a.dtype, a.stream))) return rc;
+  WgradArgs p = a;
+  p.in = in;
+  p.gout = gout;
+  p.c_in = c_in;
+  p.c_out = c_out;
+  p.crop_in = a.c_in;
+  p.crop_out = a.c_out;
+  return launch_mfma_wgrad(p);
+}
+
 int run_wgrad(const WgradArgs &a) {
   if (a.n_pairs == 0) return FGMS_OK;
   if (a.plan) plan_touch(a.plan, a.stream);
+  int pi, po;
+  if (padded_wgrad_channels(a, &pi, &po)) {
+    bool done = false;
+    const int rc = run_wgrad_padded(a, pi, po, &done);
+    if (rc != FGMS_OK || done) return rc;
+  }
   if (g_policy != 1 && mfma_wgrad_supported(a)) return launch_mfma_wgrad(a);
   return launch_generic_wgrad(a);
+}
+
+// Both gradients.
+int run_bwd(GmsArgs d, const Plan *p, WgradArgs w) {
+  int rc;
+  // Both gradients through their main kernels: two launches instead of four.  The weight
+  // gradient goes first and its launch also re-lays the weights for the input gradient,
+  // whose launch in turn also rounds the weight gradient's fp32 sums into the caller's
+  // fp16 tensor.  (The two gradients do not depend on each other.)
+  if (d.n_pairs > 0 && (!p || p->groups.empty()) && route_of(d, p) == Route::kRows && g_policy != 1 && mfma_wgrad_supported(w)) {
+    plan_touch(p, d.stream);
+    // one launch for both where the shapes allow (and a small one that rounds an fp16
+    // weight gradient), else two
+    bool fused = false;
+    if ((rc = launch_fused_bwd(d, p, w, &fused))) return rc;
+    if (fused) return FGMS_OK;
+    SideJob pack{}, flush{};
+    const void *packed = nullptr;
+    if ((rc = planned_pack_job(d, &pack, &packed))) return rc;
+    w.side = pack;
+    w.deferred_flush = &flush;
+    if ((rc = launch_mfma_wgrad(w))) return rc;
+    d.prepacked = packed;
+    d.side = flush;
+    if ((rc = launch_planned_gms(d, p))) {
+      (void)launch_side_job(flush, d.stream);   // the accumulator must not stay filled
+      return rc;
+    }
+    return FGMS_OK;
+  }
+  if ((rc = run_gms(d, p))) return rc;
+  return run_wgrad(w);
+}
+
+// Widened channels for a backward pass one of whose gradients no tuned kernel takes as it is: the
+// narrow layers' kernels up to 16 x 64, else multiples of 32 for both, which the one-grid launch takes.
+bool padded_bwd_channels(const GmsArgs &d, const Plan *p, const WgradArgs &w, int *c_in, int *c_out) {
+  if (g_policy != 0 || (tuned_gms(d, p) && mfma_wgrad_supported(w))) return false;
+  for (int narrow = w.c_in <= 16 && w.c_out <= 64 ? 1 : 0; narrow >= 0; --narrow) {
+    *c_in = narrow ? up_to_power_of_two(w.c_in, 4) : up_to_32(w.c_in);
+    *c_out = narrow ? up_to_power_of_two(w.c_out, 16) : up_to_32(w.c_out);
+    WgradArgs pw = w;
+    pw.in = pw.gout = (const void *)4096;
+    pw.c_in = *c_in;
+    pw.c_out = *c_out;
+    if (tuned_gms(with_channels(d, *c_in, *c_out), p) && mfma_wgrad_supported(pw)) return true;
+  }
+  return false;
+}
+
+// The backward pass over padded copies; the copies of the output gradient's rows serve both gradients.
+int run_bwd_padded(const GmsArgs &d, const Plan *p, const WgradArgs &w, int c_in, int c_out, bool *done) {
+  const size_t esz = elem_size(d.dtype);
+  const size_t in_bytes = (size_t)w.n_in * c_in * esz, gout_bytes = (size_t)w.n_out * c_out * esz,
+               w_bytes = (size_t)w.k_vol * c_in * c_out * esz;
+  *done = workspaces_fit(d.stream, {{kSlotPadIn, in_bytes}, {kSlotPadOut, gout_bytes}, {kSlotPadWeights, w_bytes},
+                                    {kSlotPadResult, in_bytes}, {1, (size_t)w.k_vol * c_in * c_out * sizeof(float)}});
+  if (!*done) return FGMS_OK;
+  GmsArgs pd = d;
+  WgradArgs pw = w;
+  pd.c_in = pw.c_in = c_in;
+  pd.c_out = pw.c_out = c_out;
+  pw.crop_in = w.c_in;
+  pw.crop_out = w.c_out;
+  void *in = nullptr, *gout = nullptr, *weights = nullptr, *gin = nullptr;
+  hipStream_t s = d.stream;
+  int rc;
+  PadBatch pads{};
+  if ((rc = workspace_get(s, kSlotPadWeights, w_bytes, &weights))) return rc;
+  pads.add(d.w, weights, (size_t)d.k_vol, d.c_in, c_in, d.c_out, c_out, (int)esz);
+  pd.w = weights;
+  if (c_out != d.c_out || reinterpret_cast<uintptr_t>(d.src) % 16) {
+    if ((rc = workspace_get(s, kSlotPadOut, gout_bytes, &gout))) return rc;
+    pads.add(d.src, gout, (size_t)w.n_out, 1, 1, d.c_out, c_out, (int)esz);
+    pd.src = pw.gout = gout;
+  }
+  if (c_in != d.c_in || reinterpret_cast<uintptr_t>(w.in) % 16) {
+    if ((rc = workspace_get(s, kSlotPadIn, in_bytes, &in))) return rc;
+    pads.add(w.in, in, (size_t)w.n_in, 1, 1, d.c_in, c_in, (int)esz);
+    pw.in = in;
+  }
+  const bool crop_result = c_in != d.c_in || reinterpret_cast<uintptr_t>(d.dst) % 16;
+  if (crop_result) {
+    if ((rc = workspace_get(s, kSlotPadResult, in_bytes, &gin))) return rc;
+    pads.add(nullptr, gin, (size_t)w.n_in, 1, 1, c_in, c_in, (int)esz);
+    pd.dst = gin;
+  }
+  if ((rc = launch_pad(pads, d.dtype, s))) return rc;
+  if ((rc = run_bwd(pd, p, pw))) return rc;
+  return crop_result ? launch_crop_add(gin, d.dst, (size_t)w.n_in, d.c_in, c_in, d.dtype, s) : FGMS_OK;
 }
 
 int mid_of(int k_vol) { return (k_vol % 2 == 1) ? k_vol / 2 : 0; }
@@ -745,33 +977,13 @@ int fgms_bwd(const void *out_feats_grad, const void *in_feats, const void *kerne
   w.stream = (hipStream_t)stream;
   w.plan = p;
   w.reduced = d.reduced;
-  // Both gradients through their main kernels: two launches instead of four.  The weight
-  // gradient goes first and its launch also re-lays the weights for the input gradient,
-  // whose launch in turn also rounds the weight gradient's fp32 sums into the caller's
-  // fp16 tensor.  (The two gradients do not depend on each other.)
-  if (n_pairs > 0 && (!p || p->groups.empty()) && route_of(d, p) == Route::kRows && g_policy != 1 && mfma_wgrad_supported(w)) {
-    plan_touch(p, d.stream);
-    // one launch for both where the shapes allow (and a small one that rounds an fp16
-    // weight gradient), else two
-    bool fused = false;
-    if ((rc = launch_fused_bwd(d, p, w, &fused))) return rc;
-    if (fused) return FGMS_OK;
-    SideJob pack{}, flush{};
-    const void *packed = nullptr;
-    if ((rc = planned_pack_job(d, &pack, &packed))) return rc;
-    w.side = pack;
-    w.deferred_flush = &flush;
-    if ((rc = launch_mfma_wgrad(w))) return rc;
-    d.prepacked = packed;
-    d.side = flush;
-    if ((rc = launch_planned_gms(d, p))) {
-      (void)launch_side_job(flush, d.stream);   // the accumulator must not stay filled
-      return rc;
-    }
-    return FGMS_OK;
+  int pi, po;
+  if (n_pairs > 0 && padded_bwd_channels(d, p, w, &pi, &po)) {
+    bool done = false;
+    rc = run_bwd_padded(d, p, w, pi, po, &done);
+    if (rc || done) return rc;
   }
-  if ((rc = run_gms(d, p))) return rc;
-  return run_wgrad(w);
+  return run_bwd(d, p, w);
 }
 
 int fgms_build_kernel_map(const int32_t *in_coords, int64_t n_in, const int32_t *out_coords,

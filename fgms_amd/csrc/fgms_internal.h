@@ -98,6 +98,8 @@ struct WgradArgs {
   // MFMA kernels, fp16: use this fp32 accumulator (k_vol * c_in * c_out floats, all zero)
   // instead of the stream's workspace; nothing is allocated then
   float *acc_override;
+  // the rows are padded copies: the caller's tensor is [k_vol, crop_in, crop_out] (0: [k_vol, c_in, c_out])
+  int crop_in, crop_out;
 };
 
 constexpr int kPlanFlags = 16;      // ints the plan build reports back (see fgms_plan.hip)
@@ -184,7 +186,8 @@ struct Plan {
 
 // Fp32 scratch that outlives a call (per device and stream, grown on demand).
 // slot 0: packed weights, slot 1: fp32 weight-gradient accumulator of the MFMA kernels (kept
-// all-zero between calls), slot 2: the generic kernel's accumulator, slot 3: the gather probe's sink.
+// all-zero between calls), slot 2: the generic kernel's accumulator, slot 3: the gather probe's sink,
+// slots 4 .. 7: padded copies of input rows, output rows, weights and a result (fgms_pad.hip).
 // *fresh (optional) is set when the buffer was (re)allocated by this call.
 int workspace_get(hipStream_t stream, int slot, size_t bytes, void **ptr, bool *fresh = nullptr);
 // Buffer for a re-laid copy of a.w in `layout` (any number that tells the layouts of one weight
@@ -206,6 +209,24 @@ struct ProfileScope {
 
 // ---- launchers (each returns an FGMS_* code) ----
 int launch_fill_zero(void *ptr, size_t bytes, hipStream_t stream);
+// Padded copies (fgms_pad.hip): dst[outer][r_to][c_to] = src[outer][r][c] and zeros (no src: all
+// zeros), up to four copies in a launch; dst[rows][c] += the first c of src's c_from columns; the
+// weight gradient's sums cropped, rounded and cleared.
+struct PadJob {
+  const void *src;
+  void *dst;
+  size_t chunks;
+  int r, r_to, c, c_to, first_block, blocks;
+  bool wide, whole;      // 16-byte stores; every chunk all data or all padding
+};
+struct PadBatch {
+  PadJob job[4];
+  int count, total_blocks;
+  void add(const void *src, void *dst, size_t outer, int r, int r_to, int c, int c_to, int elem_size);
+};
+int launch_pad(const PadBatch &batch, int dtype, hipStream_t s);
+int launch_crop_add(const void *src, void *dst, size_t rows, int c, int c_from, int dtype, hipStream_t s);
+int launch_crop_sums(float *sums, void *dst, size_t k_vol, int r, int r_from, int c, int c_from, int dtype, hipStream_t s);
 int launch_generic_gms(const GmsArgs &a);
 int launch_generic_wgrad(const WgradArgs &a);
 bool mfma_gms_supported(const GmsArgs &a);

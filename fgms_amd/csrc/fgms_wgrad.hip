@@ -447,7 +447,7 @@ int wgrad_geometry(const WgradArgs &a, WgradGeometry *g, bool shares_grid) {
 }
 
 int wgrad_accumulator(const WgradArgs &a, float **acc32) {
-  if (a.dtype != FGMS_F16) {
+  if (a.dtype != FGMS_F16 && !a.crop_in) {
     *acc32 = (float *)a.gw;
     return FGMS_OK;
   }
@@ -469,6 +469,7 @@ int wgrad_accumulator(const WgradArgs &a, float **acc32) {
 }
 
 int wgrad_finish(const WgradArgs &a, float *acc32) {
+  if (a.crop_in) return launch_crop_sums(acc32, a.gw, (size_t)a.k_vol, a.crop_in, a.c_in, a.crop_out, a.c_out, a.dtype, a.stream);
   if (a.dtype != FGMS_F16) return FGMS_OK;
   const size_t n = (size_t)a.k_vol * a.c_in * a.c_out;
   add_and_clear_kernel<<<(unsigned)((n + 255) / 256), 256, 0, a.stream>>>((__half *)a.gw, acc32, n);
@@ -480,14 +481,14 @@ int launch_mfma_wgrad(const WgradArgs &a) {
   float *acc32 = nullptr;
   int rc = wgrad_accumulator(a, &acc32);
   if (rc != FGMS_OK) return rc;
-  if (a.dtype != FGMS_F16) return dispatch<float>(a, acc32);
-  if ((rc = dispatch<__half>(a, acc32))) {
+  if (a.dtype != FGMS_F16 && !a.crop_in) return dispatch<float>(a, acc32);
+  if ((rc = a.dtype == FGMS_F16 ? dispatch<__half>(a, acc32) : dispatch<float>(a, acc32))) {
     const size_t bytes = a.acc_override ? (size_t)a.k_vol * a.c_in * a.c_out * sizeof(float)
                                         : workspace_bytes(a.stream, 1);
     (void)launch_fill_zero(acc32, bytes, a.stream);
     return rc;
   }
-  if (a.deferred_flush) {
+  if (a.deferred_flush && !a.crop_in) {
     // the caller attaches the flush to its next launch on the stream
     const size_t n = (size_t)a.k_vol * a.c_in * a.c_out;
     SideJob &f = *a.deferred_flush;

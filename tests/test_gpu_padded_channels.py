@@ -1,0 +1,52 @@
+"""Channel counts that run over padded copies: one off the kernels' multiples on either side, one
+channel, a kernel of more than 64 offsets, with and without a plan, results added to what the
+buffers hold -- against the CPU oracle."""
+import numpy as np
+import pytest
+import torch
+
+from fgms_amd import clouds
+from tests import gpu_util as G
+from tests.test_gpu_parity import layer
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("use_plan", [True, False], ids=["plan", "no_plan"])
+@pytest.mark.parametrize("dtype", [np.float16, np.float32], ids=["fp16", "fp32"])
+@pytest.mark.parametrize("shape", [(1, 1), (3, 32), (5, 17), (16, 65), (17, 16), (31, 33), (33, 31), (95, 20), (127, 129)])
+def test_against_oracle(oracle, shape, dtype, use_plan):
+    from fgms_amd import capi
+    capi.set_kernel_policy(0)
+    L = layer(400 + shape[0], *shape, dtype)
+    D = G.to_dev(L)
+    mode = G.mode_of(L["in_feats"].dtype)
+    args = (L["knnz"], L["imap"], L["omap"])
+    plan = capi.Plan(D["kpos"], D["imap"], D["omap"], D["n_in"], D["n_out"]) if use_plan else None
+    init = torch.randn(D["n_out"], D["c_out"], device="cuda").to(D["in_feats"].dtype)
+    ref = oracle.np_fwd(L["in_feats"], L["kernel"], *args, L["n_out"]) + init.cpu().numpy().astype(np.float64)
+    G.assert_close(G.run_fwd(capi, D, plan=plan, out_init=init), ref, mode, "fwd")
+    for split in (False, True):
+        gi, gw = G.run_bwd(capi, D, plan=plan, split=split)
+        G.assert_close(gi, oracle.np_dgrad(L["out_grad"], L["kernel"], *args, L["n_in"]), mode, "dgrad")
+        G.assert_close(gw, oracle.np_wgrad(L["in_feats"], L["out_grad"], *args, L["k_vol"]), mode, "wgrad")
+
+
+@pytest.mark.parametrize("dtype", [np.float16, np.float32], ids=["fp16", "fp32"])
+@pytest.mark.parametrize("c_in", [3, 4])
+def test_wide_kernel(oracle, dtype, c_in):
+    """125 offsets: the copies are made once, the offset groups run over them."""
+    from fgms_amd import capi
+    capi.set_kernel_policy(0)
+    rng = np.random.default_rng(5)
+    vox = clouds.cloud_planes_spheres(rng, 40, 1501)
+    imap, omap, knnz, kpos = clouds.build_kernel_map(vox, vox, clouds.offsets_cube(5))
+    L = clouds.make_layer(rng, imap, omap, knnz, kpos, len(vox), len(vox), c_in, 32, dtype)
+    D = G.to_dev(L)
+    mode = G.mode_of(L["in_feats"].dtype)
+    args = (L["knnz"], L["imap"], L["omap"])
+    plan = capi.Plan(D["kpos"], D["imap"], D["omap"], D["n_in"], D["n_out"])
+    G.assert_close(G.run_fwd(capi, D, plan=plan), oracle.np_fwd(L["in_feats"], L["kernel"], *args, L["n_out"]), mode, "fwd")
+    gi, gw = G.run_bwd(capi, D, plan=plan)
+    G.assert_close(gi, oracle.np_dgrad(L["out_grad"], L["kernel"], *args, L["n_in"]), mode, "dgrad")
+    G.assert_close(gw, oracle.np_wgrad(L["in_feats"], L["out_grad"], *args, L["k_vol"]), mode, "wgrad")
