@@ -1158,8 +1158,10 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
 // dealing the two kinds alternately or the weight gradient first measured 1-2 us slower).
 // Their count is a multiple of 8, so that a workgroup's index mod 8, its XCD, is what the
 // plan's XCD-aware orders of either kind assume.
+// (2 waves per SIMD where the weight gradient's tile is 128 x 128: its 64 accumulators per lane and
+// the rows in flight spill at 3.  128 -> 128 over 40k voxels, forward and backward: tf32 mode 477 -> 327 us.)
 template <typename T, int NT, int S, int BI, int BJ, int RAWD, int MT = 2>
-__global__ __launch_bounds__(kThreads, NT == 4 ? 2 : 3) void bwd_fused_kernel(
+__global__ __launch_bounds__(kThreads, NT == 4 || BI * BJ == 16 ? 2 : 3) void bwd_fused_kernel(
     const T *__restrict__ gout, const T *__restrict__ w, T *__restrict__ gin,
     const int32_t *__restrict__ nbr, const unsigned long long *__restrict__ block_masks,
     const int32_t *__restrict__ perm, const int32_t *__restrict__ tile_order, int n_in, int k_vol,
