@@ -1,9 +1,9 @@
 """Autograd wrapper over ``FGMS.backend``: the caller side that hkeee21/FGMS leaves to
 an external library (``README.md:3``).  It owns exactly what the reference's scripts
 repeat by hand before every call: the padded offset table ``qkpos``
-(``cpu-check.py:6-14``), zero-initialised outputs (``cpu-check.py:107-108``,
+(``cpu-check.py:6-14``), the outputs (``cpu-check.py:107-108``,
 ``cpu-check-back.py:104-107``) and the pairing of the forward call with the backward one
-(``spconv-test.py:96-120``).
+(``spconv-test.py:96-120``), as one native autograd node (``FGMS.backend.sparse_conv``).
 
     y = sparse_conv(feats, weight, kmap)          # differentiable in feats and weight
     layer = SparseConv(64, 64, k_vol=27); y = layer(feats, kmap)
@@ -60,38 +60,10 @@ class KernelMap:
         return t
 
 
-class _SparseConvFunction(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, feats, weight, kmap, allow_tf32):
-        if feats.dim() != 2 or weight.dim() != 3 or weight.shape[0] != kmap.k_vol:
-            raise ValueError("expected feats [N, Cin] and weight [K, Cin, Cout] with K = the map's offsets")
-        if feats.shape[0] != kmap.n_in:
-            raise ValueError("feats has %d rows, the kernel map expects %d" % (feats.shape[0], kmap.n_in))
-        feats = feats.contiguous()
-        weight = weight.contiguous()
-        out = torch.zeros(kmap.n_out, weight.shape[2], dtype=feats.dtype, device=feats.device)
-        backend.fgms_fusion_fwd_cuda(feats, weight, kmap.qsum, out, kmap.kpos, kmap.qkpos,
-                                     kmap.in_map, kmap.out_map, False, bool(allow_tf32))
-        ctx.save_for_backward(feats, weight)
-        ctx.kmap = kmap
-        ctx.allow_tf32 = bool(allow_tf32)
-        return out
-
-    @staticmethod
-    def backward(ctx, grad_out):
-        feats, weight = ctx.saved_tensors
-        kmap = ctx.kmap
-        grad_out = grad_out.contiguous()
-        grad_feats = torch.zeros_like(feats)
-        grad_weight = torch.zeros_like(weight)
-        backend.fgms_bwd_cuda(grad_out, feats, weight, kmap.qsum, grad_feats, grad_weight,
-                              kmap.kpos, kmap.qkpos, kmap.in_map, kmap.out_map, False, ctx.allow_tf32)
-        return grad_feats, grad_weight, None, None
-
-
 def sparse_conv(feats, weight, kmap, allow_tf32=False):
     """out[out_map[j]] += feats[in_map[j]] @ weight[k]; differentiable in feats and weight."""
-    return _SparseConvFunction.apply(feats, weight, kmap, allow_tf32)
+    return backend.sparse_conv(feats, weight, kmap.kpos, kmap.in_map, kmap.out_map, kmap.n_in, kmap.n_out,
+                               bool(allow_tf32))
 
 
 class SparseConv(torch.nn.Module):

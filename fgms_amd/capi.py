@@ -15,7 +15,7 @@ LIB_PATH = os.path.join(_HERE, "lib", "libfgms_hip.so")
 F32, F16 = 0, 1
 SYMBOLS = [
     "fgms_version", "fgms_last_error", "fgms_plan_create", "fgms_plan_check", "fgms_plan_transposed", "fgms_plan_destroy",
-    "fgms_plan_usable", "fgms_plan_stats", "fgms_fusion_fwd", "fgms_fwd", "fgms_bwd", "fgms_dgrad",
+    "fgms_plan_usable", "fgms_plan_stats", "fgms_conv_fwd", "fgms_conv_bwd", "fgms_fusion_fwd", "fgms_fwd", "fgms_bwd", "fgms_dgrad",
     "fgms_wgrad", "fgms_wgrad_static", "fgms_set_kernel_policy", "fgms_profile_enable", "fgms_profile_read",
     "fgms_profile_reset", "fgms_probe_gather", "fgms_build_kernel_map", "fgms_allocation_count",
     "fgms_weights_pin", "fgms_weights_unpin", "fgms_relaid_weights_hits",
@@ -60,6 +60,8 @@ def lib():
     L.fgms_dgrad.argtypes = [vp, vp, vp, vp, vp, vp, i64, i64, i32, i32, i32, i64, i32, vp, vp]
     L.fgms_wgrad.argtypes = [vp, vp, vp, vp, vp, vp, i64, i64, i32, i32, i32, i64, i32, vp, vp]
     L.fgms_wgrad_static.argtypes = L.fgms_wgrad.argtypes
+    L.fgms_conv_fwd.argtypes = [vp, vp, vp, vp, vp, vp, i32, i64, i64, i32, i32, i32, i64, i32, vp, vp]
+    L.fgms_conv_bwd.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, i32, i64, i64, i32, i32, i32, i64, i32, vp, vp]
     L.fgms_build_kernel_map.argtypes = [vp, i64, vp, i64, vp, i32, i32, i32, vp, vp, i64, vp, vp,
                                         ctypes.POINTER(ctypes.c_int64), vp]
     L.fgms_build_kernel_map.restype = i32
@@ -268,6 +270,30 @@ def bwd(out_grad, in_feats, kernel, sum_nnz, in_grad, kernel_grad, kpos, qkpos, 
         _p(out_grad), _p(in_feats), _p(kernel), int(sum_nnz), _p(in_grad), _p(kernel_grad),
         _p(kpos), _p(qkpos), _p(in_map), _p(out_map), int(separate_mid), int(arch80),
         in_feats.shape[0], out_grad.shape[0], kernel.shape[1], kernel.shape[2], kernel.shape[0],
+        in_map.numel(), _dtype(in_feats), _ph(plan), _stream()))
+
+
+def conv_fwd(in_feats, kernel, out_feats, kpos, in_map, out_map, arch80=False, plan=None):
+    """``fgms_conv_fwd``: out_feats is written, whatever it holds."""
+    _check_feats(in_feats, kernel)
+    for t, n in ((in_feats, "in_feats"), (kernel, "kernel"), (out_feats, "out_feats")):
+        _need(t, n, in_feats.dtype)
+    _check(lib().fgms_conv_fwd(
+        _p(in_feats), _p(kernel), _p(out_feats), _p(kpos), _p(in_map), _p(out_map), int(arch80), in_feats.shape[0],
+        out_feats.shape[0], kernel.shape[1], kernel.shape[2], kernel.shape[0], in_map.numel(), _dtype(in_feats),
+        _ph(plan), _stream()))
+
+
+def conv_bwd(out_grad, in_feats, kernel, in_grad, kernel_grad, kpos, in_map, out_map, arch80=False, plan=None):
+    """``fgms_conv_bwd``: the gradients are written; None: not computed."""
+    _check_feats(in_feats, kernel)
+    for t, n in ((out_grad, "out_feats_grad"), (in_feats, "in_feats"), (kernel, "kernel"),
+                 (in_grad, "in_feats_grad"), (kernel_grad, "kernel_grad")):
+        if t is not None:
+            _need(t, n, in_feats.dtype)
+    _check(lib().fgms_conv_bwd(
+        _p(out_grad), _p(in_feats), _p(kernel), _p(in_grad), _p(kernel_grad), _p(kpos), _p(in_map), _p(out_map),
+        int(arch80), in_feats.shape[0], out_grad.shape[0], kernel.shape[1], kernel.shape[2], kernel.shape[0],
         in_map.numel(), _dtype(in_feats), _ph(plan), _stream()))
 
 

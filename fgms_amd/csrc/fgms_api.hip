@@ -553,6 +553,7 @@ int run_gms(GmsArgs a, const Plan *plan) {
     ga.w = (const char *)a.w + (size_t)k0 * a.c_in * a.c_out * esz;
     ga.kpos = a.kpos + k0;
     ga.k_vol = g->k_vol;
+    ga.overwrite = a.overwrite && k0 == 0;      // (the later groups add to the first one's sums)
     int rc = run_gms_one(ga, g);
     if (rc != FGMS_OK) return rc;
     k0 += g->k_vol;
@@ -563,8 +564,19 @@ int run_gms(GmsArgs a, const Plan *plan) {
 int run_gms_one(GmsArgs a, const Plan *plan) {
   if (plan) plan_touch(plan, a.stream);
   const bool dense = a.dense_k >= 0;
-  if ((!dense && a.n_pairs == 0) || (dense && a.n_dense == 0)) return FGMS_OK;
-  switch (route_of(a, plan)) {
+  auto zero_result = [&]() {
+    return launch_fill_zero(a.dst, (size_t)a.n_dst * (a.transpose_w ? a.c_in : a.c_out) * elem_size(a.dtype), a.stream);
+  };
+  if ((!dense && a.n_pairs == 0) || (dense && a.n_dense == 0)) return a.overwrite ? zero_result() : FGMS_OK;
+  const Route route = route_of(a, plan);
+  // (these kernels add with atomics, several workgroups to a row)
+  if (a.overwrite && (route == Route::kWide || route == Route::kPairs || route == Route::kGeneric)) {
+    const int rc = zero_result();
+    if (rc != FGMS_OK) return rc;
+  }
+  // (a pending fingerprint check of the plan rides along as the launch's side job)
+  if (plan && !a.side.kind && route != Route::kGeneric) (void)plan_take_check(plan, &a.side);
+  switch (route) {
     case Route::kSkinny: return launch_small_gms(a, plan);
     case Route::kRows: return launch_planned_gms(a, plan);
     case Route::kPairView: return launch_pair_view_gms(a, plan);
@@ -596,13 +608,13 @@ int run_gms_padded(const GmsArgs &a, const Plan *plan, int c_in, int c_out, bool
   PadBatch pads{};
   pads.add(a.src, src, (size_t)a.n_src, 1, 1, c_src, p_src, (int)esz);
   pads.add(a.w, w, (size_t)a.k_vol, a.c_in, c_in, a.c_out, c_out, (int)esz);
-  pads.add(nullptr, dst, (size_t)a.n_dst, 1, 1, p_dst, p_dst, (int)esz);
   if ((rc = launch_pad(pads, a.dtype, a.stream))) return rc;
   p.src = src;
   p.w = w;
   p.dst = dst;
+  p.overwrite = true;
   if ((rc = run_gms(p, plan))) return rc;
-  return launch_crop_add(dst, a.dst, (size_t)a.n_dst, c_dst, p_dst, a.dtype, a.stream);
+  return launch_crop(dst, a.dst, (size_t)a.n_dst, c_dst, p_dst, a.overwrite, a.dtype, a.stream);
 }
 
 // Widened channels of a weight gradient no MFMA / skinny kernel takes as it is.
@@ -647,7 +659,8 @@ int run_wgrad_padded(const WgradArgs &a, int c_in, int c_out, bool *done) {
 }
 
 int run_wgrad(const WgradArgs &a) {
-  if (a.n_pairs == 0) return FGMS_OK;
+  const size_t gw_bytes = (size_t)a.k_vol * a.c_in * a.c_out * elem_size(a.dtype);
+  if (a.n_pairs == 0) return a.overwrite ? launch_fill_zero(a.gw, gw_bytes, a.stream) : FGMS_OK;
   if (a.plan) plan_touch(a.plan, a.stream);
   int pi, po;
   if (padded_wgrad_channels(a, &pi, &po)) {
@@ -656,6 +669,10 @@ int run_wgrad(const WgradArgs &a) {
     if (rc != FGMS_OK || done) return rc;
   }
   if (g_policy != 1 && mfma_wgrad_supported(a)) return launch_mfma_wgrad(a);
+  if (a.overwrite) {
+    const int rc = launch_fill_zero(a.gw, gw_bytes, a.stream);
+    if (rc != FGMS_OK) return rc;
+  }
   return launch_generic_wgrad(a);
 }
 
@@ -741,12 +758,12 @@ int run_bwd_padded(const GmsArgs &d, const Plan *p, const WgradArgs &w, int c_in
   const bool crop_result = c_in != d.c_in || reinterpret_cast<uintptr_t>(d.dst) % 16;
   if (crop_result) {
     if ((rc = workspace_get(s, kSlotPadResult, in_bytes, &gin))) return rc;
-    pads.add(nullptr, gin, (size_t)w.n_in, 1, 1, c_in, c_in, (int)esz);
     pd.dst = gin;
+    pd.overwrite = true;
   }
   if ((rc = launch_pad(pads, d.dtype, s))) return rc;
   if ((rc = run_bwd(pd, p, pw))) return rc;
-  return crop_result ? launch_crop_add(gin, d.dst, (size_t)w.n_in, d.c_in, c_in, d.dtype, s) : FGMS_OK;
+  return crop_result ? launch_crop(gin, d.dst, (size_t)w.n_in, d.c_in, c_in, d.overwrite, d.dtype, s) : FGMS_OK;
 }
 
 int mid_of(int k_vol) { return (k_vol % 2 == 1) ? k_vol / 2 : 0; }
@@ -783,6 +800,48 @@ struct CheckFlush {
   hipStream_t s;
   ~CheckFlush() { if (p) (void)plan_flush_check(p, s); }
 };
+
+// One or both gradients, added to what the tensors hold or written over it.
+int backward(const void *out_feats_grad, const void *in_feats, const void *kernel, void *in_feats_grad,
+             void *kernel_grad, const int32_t *kpos, const int32_t *in_map, const int32_t *out_map, int arch80,
+             int64_t n_in, int64_t n_out, int c_in, int c_out, int k_vol, int64_t n_pairs, int dtype,
+             fgms_plan_t *plan, hipStream_t stream, bool want_in, bool want_kernel, bool overwrite) {
+  int rc;
+  if (want_in && (rc = check_common(out_feats_grad, kernel, in_feats_grad, kpos, in_map, out_map, n_in, n_out, c_in, c_out,
+                                    k_vol, n_pairs, dtype)))
+    return rc;
+  if (want_kernel && (rc = check_common(in_feats, out_feats_grad, kernel_grad, kpos, in_map, out_map, n_in, n_out, c_in,
+                                        c_out, k_vol, n_pairs, dtype)))
+    return rc;
+  const Plan *p = plan_resolve(plan, stream, &rc);
+  CheckFlush flush{p, stream};
+  if (rc) return rc;
+  GmsArgs d{};
+  d.src = out_feats_grad; d.w = kernel; d.dst = in_feats_grad; d.kpos = kpos;
+  d.gmap = out_map; d.smap = in_map;   // roles swap, as at backend/spconv.cu:460,559
+  d.n_src = n_out; d.n_dst = n_in; d.c_in = c_in; d.c_out = c_out; d.k_vol = k_vol;
+  d.n_pairs = n_pairs; d.transpose_w = true; d.dense_k = -1; d.n_dense = 0; d.dtype = dtype;
+  d.stream = stream;
+  d.reduced = arch80 != 0 && dtype == FGMS_F32;     // (the reference's backward is tf32 whenever the tensors are fp32)
+  d.overwrite = overwrite;
+  WgradArgs w{};
+  w.in = in_feats; w.gout = out_feats_grad; w.gw = kernel_grad; w.kpos = kpos;
+  w.imap = in_map; w.omap = out_map; w.n_in = n_in; w.n_out = n_out; w.c_in = c_in;
+  w.c_out = c_out; w.k_vol = k_vol; w.n_pairs = n_pairs; w.dtype = dtype;
+  w.stream = stream;
+  w.plan = p;
+  w.reduced = d.reduced;
+  w.overwrite = overwrite;
+  if (!want_kernel) return want_in ? run_gms(d, p) : FGMS_OK;
+  if (!want_in) return run_wgrad(w);
+  int pi, po;
+  if (n_pairs > 0 && padded_bwd_channels(d, p, w, &pi, &po)) {
+    bool done = false;
+    rc = run_bwd_padded(d, p, w, pi, po, &done);
+    if (rc || done) return rc;
+  }
+  return run_bwd(d, p, w);
+}
 }  // namespace
 
 extern "C" {
@@ -954,36 +1013,34 @@ int fgms_bwd(const void *out_feats_grad, const void *in_feats, const void *kerne
              int64_t n_in, int64_t n_out, int c_in, int c_out, int k_vol, int64_t n_pairs,
              int dtype, fgms_plan_t *plan, void *stream) {
   (void)sum_nnz; (void)qkpos; (void)separate_mid;
-  int rc = check_common(out_feats_grad, kernel, in_feats_grad, kpos, in_map, out_map, n_in, n_out,
-                        c_in, c_out, k_vol, n_pairs, dtype);
+  return backward(out_feats_grad, in_feats, kernel, in_feats_grad, kernel_grad, kpos, in_map, out_map, arch80, n_in,
+                  n_out, c_in, c_out, k_vol, n_pairs, dtype, plan, (hipStream_t)stream, true, true, false);
+}
+
+int fgms_conv_fwd(const void *in_feats, const void *kernel, void *out_feats, const int32_t *kpos, const int32_t *in_map,
+                  const int32_t *out_map, int arch80, int64_t n_in, int64_t n_out, int c_in, int c_out, int k_vol,
+                  int64_t n_pairs, int dtype, fgms_plan_t *plan, void *stream) {
+  int rc = check_common(in_feats, kernel, out_feats, kpos, in_map, out_map, n_in, n_out, c_in,
+                        c_out, k_vol, n_pairs, dtype);
   if (rc) return rc;
-  if ((rc = check_common(in_feats, out_feats_grad, kernel_grad, kpos, in_map, out_map, n_in, n_out,
-                         c_in, c_out, k_vol, n_pairs, dtype)))
-    return rc;
-  const Plan *p = plan_resolve(plan, (hipStream_t)stream, &rc);
-  CheckFlush flush{p, (hipStream_t)stream};
+  hipStream_t s = (hipStream_t)stream;
+  GmsArgs a = fwd_args(in_feats, kernel, out_feats, kpos, in_map, out_map, n_in, n_out, c_in,
+                       c_out, k_vol, n_pairs, dtype, s);
+  a.reduced = arch80 != 0 && dtype == FGMS_F32;
+  a.overwrite = true;
+  const Plan *p = plan_resolve(plan, s, &rc);
+  CheckFlush flush{p, s};
   if (rc) return rc;
-  GmsArgs d{};
-  d.src = out_feats_grad; d.w = kernel; d.dst = in_feats_grad; d.kpos = kpos;
-  d.gmap = out_map; d.smap = in_map;   // roles swap, as at backend/spconv.cu:460,559
-  d.n_src = n_out; d.n_dst = n_in; d.c_in = c_in; d.c_out = c_out; d.k_vol = k_vol;
-  d.n_pairs = n_pairs; d.transpose_w = true; d.dense_k = -1; d.n_dense = 0; d.dtype = dtype;
-  d.stream = (hipStream_t)stream;
-  d.reduced = arch80 != 0 && dtype == FGMS_F32;     // (the reference's backward is tf32 whenever the tensors are fp32)
-  WgradArgs w{};
-  w.in = in_feats; w.gout = out_feats_grad; w.gw = kernel_grad; w.kpos = kpos;
-  w.imap = in_map; w.omap = out_map; w.n_in = n_in; w.n_out = n_out; w.c_in = c_in;
-  w.c_out = c_out; w.k_vol = k_vol; w.n_pairs = n_pairs; w.dtype = dtype;
-  w.stream = (hipStream_t)stream;
-  w.plan = p;
-  w.reduced = d.reduced;
-  int pi, po;
-  if (n_pairs > 0 && padded_bwd_channels(d, p, w, &pi, &po)) {
-    bool done = false;
-    rc = run_bwd_padded(d, p, w, pi, po, &done);
-    if (rc || done) return rc;
-  }
-  return run_bwd(d, p, w);
+  return run_gms(a, p);
+}
+
+int fgms_conv_bwd(const void *out_feats_grad, const void *in_feats, const void *kernel, void *in_feats_grad,
+                  void *kernel_grad, const int32_t *kpos, const int32_t *in_map, const int32_t *out_map, int arch80,
+                  int64_t n_in, int64_t n_out, int c_in, int c_out, int k_vol, int64_t n_pairs, int dtype,
+                  fgms_plan_t *plan, void *stream) {
+  return backward(out_feats_grad, in_feats, kernel, in_feats_grad, kernel_grad, kpos, in_map, out_map, arch80, n_in,
+                  n_out, c_in, c_out, k_vol, n_pairs, dtype, plan, (hipStream_t)stream, in_feats_grad != nullptr,
+                  kernel_grad != nullptr, true);
 }
 
 int fgms_build_kernel_map(const int32_t *in_coords, int64_t n_in, const int32_t *out_coords,

@@ -111,10 +111,26 @@ __device__ __forceinline__ void pack_weight_elements(const T *__restrict__ w, T 
 
 // dst[i] += acc[i] rounded once to fp16, and acc[i] is reset: the accumulator is handed
 // back all-zero, which is the state the next weight gradient expects to find it in.
+// (overwrite: dst[i] = acc[i] rounded.)  Four elements a thread where both lie on their boundaries.
 __device__ __forceinline__ void add_and_clear_elements(__half *__restrict__ dst, float *__restrict__ acc,
-                                                       size_t n, size_t first, size_t stride) {
-  for (size_t i = first; i < n; i += stride) {
-    dst[i] = __float2half(__half2float(dst[i]) + acc[i]);
+                                                       size_t n, size_t first, size_t stride, bool overwrite) {
+  typedef _Float16 half4_ __attribute__((ext_vector_type(4)));
+  typedef float float4_ __attribute__((ext_vector_type(4)));
+  size_t done = 0;
+  if (reinterpret_cast<uintptr_t>(dst) % 8 == 0 && reinterpret_cast<uintptr_t>(acc) % 16 == 0) {
+    for (size_t q = first; q < n / 4; q += stride) {
+      float4_ v = reinterpret_cast<const float4_ *>(acc)[q];
+      half4_ out = 0;
+      if (!overwrite) out = reinterpret_cast<const half4_ *>(dst)[q];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) out[e] = (_Float16)((float)out[e] + v[e]);
+      reinterpret_cast<half4_ *>(dst)[q] = out;
+      reinterpret_cast<float4_ *>(acc)[q] = float4_{0.f, 0.f, 0.f, 0.f};
+    }
+    done = n / 4 * 4;
+  }
+  for (size_t i = done + first; i < n; i += stride) {
+    dst[i] = __float2half((overwrite ? 0.f : __half2float(dst[i])) + acc[i]);
     acc[i] = 0.f;
   }
 }
@@ -128,37 +144,41 @@ __device__ __forceinline__ unsigned long long print_hash(unsigned long long a, u
   x ^= x >> 31; x *= 0xBF58476D1CE4E5B9ull; x ^= x >> 29;
   return x;
 }
+// Cut into kPrintParts parts with a sum of their own, one workgroup each: the sampled entries lie a
+// cache line apart at least, and one workgroup alone fetches its 8 192 lines at the few lines in flight
+// a CU allows (11.4 us a launch of its own, eight workgroups 3.3 us).
 constexpr int kPrintSamples = 4096;
 __host__ __device__ inline int print_stride(int n_pairs) { return n_pairs > kPrintSamples ? n_pairs / kPrintSamples : 1; }
 
-// The fingerprint of the lists as they are now, summed by one workgroup (the sample is 4 096
-// pairs); valid in thread 0.
+// One part of the fingerprint of the lists as they are now, summed by one workgroup; valid in thread 0.
 __device__ __forceinline__ unsigned long long plan_print_sum(const int32_t *__restrict__ kpos,
                                                              const int32_t *__restrict__ imap,
-                                                             const int32_t *__restrict__ omap, int k_vol, int n_pairs) {
+                                                             const int32_t *__restrict__ omap, int k_vol, int n_pairs,
+                                                             int print_part) {
   __shared__ unsigned long long part[16];
   const int threads = blockDim.x;
   const int first = kpos[0], total = min(kpos[k_vol], n_pairs);
   const int stride = print_stride(total - first);
   unsigned long long v = 0;
   // (all of a thread's samples are requested before the first is hashed)
-  constexpr int kMine = 16;
-  for (int s0 = threadIdx.x; first + (long long)s0 * stride < total; s0 += threads * kMine) {
+  constexpr int kMine = 2;
+  const int step = threads * kPrintParts;      // (a part takes every kPrintParts-th sample)
+  for (int s0 = print_part + kPrintParts * threadIdx.x; first + (long long)s0 * stride < total; s0 += step * kMine) {
     int a[kMine], b[kMine];
 #pragma unroll
     for (int u = 0; u < kMine; ++u) {
-      const long long j = first + (long long)(s0 + u * threads) * stride;
+      const long long j = first + (long long)(s0 + u * step) * stride;
       const int jj = (int)(j < total ? j : total - 1);
       a[u] = imap[jj];
       b[u] = omap[jj];
     }
 #pragma unroll
     for (int u = 0; u < kMine; ++u) {
-      const long long j = first + (long long)(s0 + u * threads) * stride;
+      const long long j = first + (long long)(s0 + u * step) * stride;
       if (j < total) v += print_hash((unsigned long long)(j - first), (unsigned)a[u], (unsigned)b[u]);
     }
   }
-  for (int rel = threadIdx.x; rel <= k_vol; rel += threads) v += print_hash(0x100000000ull + rel, (unsigned)kpos[rel], 0u);
+  for (int rel = print_part == 0 ? threadIdx.x : k_vol + 1; rel <= k_vol; rel += threads) v += print_hash(0x100000000ull + rel, (unsigned)kpos[rel], 0u);
   for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d);
   if (threadIdx.x % 64 == 0) part[threadIdx.x / 64] = v;
   __syncthreads();
@@ -171,18 +191,18 @@ __device__ __forceinline__ unsigned long long plan_print_sum(const int32_t *__re
 // Build: the fingerprint goes into the plan's flags.
 __device__ __forceinline__ void plan_print_block(const int32_t *__restrict__ kpos, const int32_t *__restrict__ imap,
                                                  const int32_t *__restrict__ omap, int k_vol, int n_pairs,
-                                                 int *__restrict__ flags) {
-  const unsigned long long sum = plan_print_sum(kpos, imap, omap, k_vol, n_pairs);
-  if (threadIdx.x == 0) *reinterpret_cast<unsigned long long *>(flags + kFlagPrint) = sum;
+                                                 int *__restrict__ flags, int print_part) {
+  const unsigned long long sum = plan_print_sum(kpos, imap, omap, k_vol, n_pairs, print_part);
+  if (threadIdx.x == 0) reinterpret_cast<unsigned long long *>(flags + kFlagPrint)[print_part] = sum;
 }
 
 // fgms_plan_check: taken again and compared with the build's; a difference raises the sticky
 // flag, in device memory and in the plan's pinned block.
 __device__ __forceinline__ void plan_check_block(const int32_t *__restrict__ kpos, const int32_t *__restrict__ imap,
                                                  const int32_t *__restrict__ omap, int k_vol, int n_pairs,
-                                                 int *__restrict__ flags, int *__restrict__ host) {
-  const unsigned long long sum = plan_print_sum(kpos, imap, omap, k_vol, n_pairs);
-  if (threadIdx.x == 0 && sum != *reinterpret_cast<const unsigned long long *>(flags + kFlagPrint)) {
+                                                 int *__restrict__ flags, int *__restrict__ host, int print_part) {
+  const unsigned long long sum = plan_print_sum(kpos, imap, omap, k_vol, n_pairs, print_part);
+  if (threadIdx.x == 0 && sum != reinterpret_cast<const unsigned long long *>(flags + kFlagPrint)[print_part]) {
     flags[kFlagStale] = 1;
     if (host) host[kFlagStale] = 1;
   }
@@ -200,11 +220,10 @@ __device__ __forceinline__ void run_side_job(const SideJob &job, int block) {
       pack_weight_elements<float>((const float *)job.src, (float *)job.dst, job.k_vol, job.c_in,
                                   job.c_out, job.S, job.transpose != 0, first, stride);
   } else if (job.kind == 2) {
-    add_and_clear_elements((__half *)job.dst, job.acc, job.n, first, stride);
+    add_and_clear_elements((__half *)job.dst, job.acc, job.n, first, stride, job.overwrite != 0);
   } else if (job.kind == 3) {
-    if (block == 0)
-      plan_check_block((const int32_t *)job.src, (const int32_t *)job.dst, job.omap, job.k_vol, (int)job.n,
-                       job.flags, job.host);
+    plan_check_block((const int32_t *)job.src, (const int32_t *)job.dst, job.omap, job.k_vol, (int)job.n,
+                     job.flags, job.host, block);
   }
 }
 

@@ -154,6 +154,11 @@ __global__ void fill_zero_kernel(uint32_t *__restrict__ p, size_t words) {
   const size_t stride = (size_t)gridDim.x * blockDim.x;
   for (; i < words; i += stride) p[i] = 0u;
 }
+__global__ void fill_zero_two_kernel(uint32_t *__restrict__ p, size_t words, uint32_t *__restrict__ q, size_t q_words) {
+  const size_t first = (size_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (size_t)gridDim.x * blockDim.x;
+  for (size_t i = first; i < words; i += stride) p[i] = 0u;
+  for (size_t i = first; i < q_words; i += stride) q[i] = 0u;
+}
 __global__ void fill_zero_bytes_kernel(uint8_t *__restrict__ p, size_t n) {
   size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0;
@@ -176,6 +181,19 @@ int launch_fill_zero(void *ptr, size_t bytes, hipStream_t stream) {
   }
   size_t tail = bytes - head - words * 4;
   if (tail) fill_zero_bytes_kernel<<<1, 64, 0, stream>>>((uint8_t *)ptr + head + words * 4, tail);
+  FGMS_HIP_TRY(hipGetLastError());
+  return FGMS_OK;
+}
+
+int launch_fill_zero_two(void *p, size_t bytes, void *q, size_t q_bytes, hipStream_t stream) {
+  if ((reinterpret_cast<uintptr_t>(p) | reinterpret_cast<uintptr_t>(q) | bytes | q_bytes) % 4) {
+    const int rc = launch_fill_zero(p, bytes, stream);
+    return rc != FGMS_OK ? rc : launch_fill_zero(q, q_bytes, stream);
+  }
+  size_t blocks = ((bytes > q_bytes ? bytes : q_bytes) / 4 + 256 * 4 - 1) / (256 * 4);
+  if (blocks == 0) return FGMS_OK;
+  if (blocks > 65535) blocks = 65535;
+  fill_zero_two_kernel<<<(unsigned)blocks, 256, 0, stream>>>((uint32_t *)p, bytes / 4, (uint32_t *)q, q_bytes / 4);
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;
 }

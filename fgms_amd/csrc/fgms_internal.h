@@ -38,8 +38,9 @@ void set_error(const char *fmt, ...);
 //           pack_weights_kernel does), for the launch that follows on the stream;
 //   kind 2: dst[i] += acc[i] rounded once to fp16 and acc[i] = 0 (what add_and_clear_kernel
 //           does) for the fp32 accumulator the previous launch on the stream filled;
+//           (overwrite: dst[i] = acc[i] rounded);
 //   kind 3: the plan's fingerprint check (fgms_plan_check): src = kpos, dst = in_map, omap,
-//           n = the pair bound, k_vol; one workgroup works, the others of the job leave.
+//           n = the pair bound, k_vol; kPrintParts workgroups.
 struct SideJob {
   int kind;      // 0: none
   int blocks;
@@ -47,7 +48,7 @@ struct SideJob {
   void *dst;
   float *acc;
   size_t n;      // elements
-  int k_vol, c_in, c_out, S, transpose, dtype;
+  int k_vol, c_in, c_out, S, transpose, dtype, overwrite;
   const int32_t *omap;
   int *flags, *host;
 };
@@ -73,8 +74,9 @@ struct GmsArgs {
   // fp32 tensors in the reference's "tf32" mode: products may be rounded to tf32 precision
   // (10 mantissa bits) or better, sums stay fp32
   bool reduced;
+  bool overwrite;          // dst = the sums instead of dst += (rows without a pair become zero)
   const void *prepacked;   // output-stationary kernel only: the weights are already re-laid here
-  SideJob side;            // ... and this rides along with its launch
+  SideJob side;            // rides along with the launch (not the shape-agnostic kernel's)
 };
 
 struct WgradArgs {
@@ -90,6 +92,7 @@ struct WgradArgs {
   int dtype;
   hipStream_t stream;
   const struct Plan *plan;   // optional
+  bool overwrite;            // gw = the sums instead of gw +=
   bool reduced;              // fp32 tensors: products may be rounded to tf32 precision or better
   SideJob side;              // MFMA kernels only: rides along with the launch
   // MFMA kernels, fp16: do not launch the fp32 -> fp16 flush of the accumulator; describe
@@ -102,9 +105,10 @@ struct WgradArgs {
   int crop_in, crop_out;
 };
 
-constexpr int kPlanFlags = 16;      // ints the plan build reports back (see fgms_plan.hip)
+constexpr int kPlanFlags = 32;      // ints the plan build reports back (see fgms_plan.hip)
 constexpr int kFlagStale = 13;      // flags[13]: a later check found another fingerprint (fgms_plan_check)
-constexpr int kFlagPrint = 14;      // flags[14], flags[15]: fingerprint of the pair lists (one 64-bit word)
+constexpr int kFlagPrint = 16;      // flags[16 .. 31]: fingerprint of the pair lists (kPrintParts 64-bit words)
+constexpr int kPrintParts = 8;      // ... each over an eighth of the sample, so that as many workgroups take it
 
 // Plan: neighbour tables built from the pair lists.
 struct Plan {
@@ -225,8 +229,11 @@ struct PadBatch {
   void add(const void *src, void *dst, size_t outer, int r, int r_to, int c, int c_to, int elem_size);
 };
 int launch_pad(const PadBatch &batch, int dtype, hipStream_t s);
-int launch_crop_add(const void *src, void *dst, size_t rows, int c, int c_from, int dtype, hipStream_t s);
-int launch_crop_sums(float *sums, void *dst, size_t k_vol, int r, int r_from, int c, int c_from, int dtype, hipStream_t s);
+int launch_crop(const void *src, void *dst, size_t rows, int c, int c_from, bool overwrite, int dtype, hipStream_t s);
+int launch_crop_sums(float *sums, void *dst, size_t k_vol, int r, int r_from, int c, int c_from, bool overwrite, int dtype,
+                     hipStream_t s);
+// Zeroes one or two blocks (of whole 4-byte words, 4-byte aligned) in one launch.
+int launch_fill_zero_two(void *p, size_t bytes, void *q, size_t q_bytes, hipStream_t s);
 int launch_generic_gms(const GmsArgs &a);
 int launch_generic_wgrad(const WgradArgs &a);
 bool mfma_gms_supported(const GmsArgs &a);

@@ -425,7 +425,16 @@ __global__ __launch_bounds__(kThreads) void gms_pairs_kernel(
     const T *__restrict__ src, const T *__restrict__ packed, T *__restrict__ dst,
     const int32_t *__restrict__ kpos, const int32_t *__restrict__ gmap,
     const int32_t *__restrict__ smap, int k_vol, int c_src, int c_dst, int tiles_per_wg,
-    int dense_k, int dense_rows) {
+    int dense_k, int dense_rows, SideJob side) {
+  // the leading workgroups of the grid run the side job, if there is one
+  int block_x = blockIdx.x;
+  if (side.blocks) {
+    if (block_x < side.blocks) {
+      if (blockIdx.y == 0) run_side_job(side, block_x);
+      return;
+    }
+    block_x -= side.blocks;
+  }
   constexpr int E = Elem<T>::per_chunk;
   extern __shared__ int4v lds[];
   const int slabs = c_src / (2 * S * E);
@@ -441,7 +450,7 @@ __global__ __launch_bounds__(kThreads) void gms_pairs_kernel(
   const size_t packed_per_k = (size_t)c_src * c_dst / E;  // chunks
 
   int cur_k = -1;
-  const int t_begin = blockIdx.x * tiles_per_wg;
+  const int t_begin = block_x * tiles_per_wg;
   for (int t = t_begin; t < t_begin + tiles_per_wg; ++t) {
     int k, first, count;
     if (dense_k >= 0) {
@@ -521,7 +530,7 @@ __device__ __forceinline__ void gms_rows_body(
     const int32_t *__restrict__ nbr, const unsigned long long *__restrict__ block_masks,
     const int32_t *__restrict__ perm, const int32_t *__restrict__ tile_order, int n_dst, int k_vol,
     int c_src, int c_dst, int part_stages, int block_x, int block_y, int block_z, int grid_z,
-    unsigned src_bytes, int pair_view = 0) {
+    unsigned src_bytes, int pair_view, int overwrite) {
   constexpr int E = Elem<T>::per_chunk;
   constexpr int C = 2 * S;
   // 16-bit matrix instructions (fp16 tensors, fp32 tensors in split bf16): rows and weights come
@@ -589,7 +598,10 @@ __device__ __forceinline__ void gms_rows_body(
   if (lane == 0 && wave_mask) atomicOr(&wg_mask, wave_mask);
   __syncthreads();
   unsigned long long todo = wg_mask;
-  if (!todo) return;
+  if (!todo) {
+    if (overwrite) zero_rows<T, NT, WR>(dst, didx, c_dst, nt0 * 32, lane);
+    return;
+  }
   // The launch lasts as long as its longest tile, and the tiles with the longest
   // offset lists are few: they get the instruction issue priority, so that they run
   // at their own pace while the many short tiles share what is left.
@@ -868,12 +880,14 @@ __device__ __forceinline__ void gms_rows_body(
       active = next_active;
     }
   }
-  if (wave_mask) {
+  if (wave_mask || overwrite) {
     wave_lds_fence();
     if (shared_tile)
-      add_rows_lds<T, NT, S, true>(acc, dst, didx, reinterpret_cast<float *>(a_lds), c_dst, nt0 * 32, lane);
+      add_rows_lds<T, NT, S, true, false>(acc, dst, didx, reinterpret_cast<float *>(a_lds), c_dst, nt0 * 32, lane);
+    else if (overwrite)
+      add_rows_lds<T, NT, S, false, true>(acc, dst, didx, reinterpret_cast<float *>(a_lds), c_dst, nt0 * 32, lane);
     else
-      add_rows_lds<T, NT, S, false>(acc, dst, didx, reinterpret_cast<float *>(a_lds), c_dst, nt0 * 32, lane);
+      add_rows_lds<T, NT, S, false, false>(acc, dst, didx, reinterpret_cast<float *>(a_lds), c_dst, nt0 * 32, lane);
   }
 }
 
@@ -882,7 +896,7 @@ __global__ __launch_bounds__(kThreads, MT == 1 ? 4 : (NT == 4 ? 2 : 3)) void gms
     const T *__restrict__ src, const T *__restrict__ packed, T *__restrict__ dst,
     const int32_t *__restrict__ nbr, const unsigned long long *__restrict__ block_masks,
     const int32_t *__restrict__ perm, const int32_t *__restrict__ tile_order, int n_dst, int k_vol,
-    int c_src, int c_dst, int part_stages, SideJob side, int pair_view, unsigned src_bytes) {
+    int c_src, int c_dst, int part_stages, SideJob side, int pair_view, unsigned src_bytes, int overwrite) {
   // the leading workgroups of the grid run the side job, if there is one
   int block_x = blockIdx.x;
   if (side.blocks) {
@@ -893,7 +907,8 @@ __global__ __launch_bounds__(kThreads, MT == 1 ? 4 : (NT == 4 ? 2 : 3)) void gms
     block_x -= side.blocks;
   }
   gms_rows_body<T, NT, S, RAW, MT>(src, packed, dst, nbr, block_masks, perm, tile_order, n_dst, k_vol, c_src,
-                                   c_dst, part_stages, block_x, blockIdx.y, blockIdx.z, gridDim.z, src_bytes, pair_view);
+                                   c_dst, part_stages, block_x, blockIdx.y, blockIdx.z, gridDim.z, src_bytes, pair_view,
+                                   overwrite);
 }
 
 // ---------------------------------------------------------------------------
@@ -996,9 +1011,9 @@ int launch_pairs(const GmsArgs &a, const Shape &s) {
     ProfileScope prof(split ? (a.transpose_w ? "gms_pairs_kernel(dgrad, bf16x3)" : "gms_pairs_kernel(fwd, bf16x3)")
                             : (a.transpose_w ? "gms_pairs_kernel(dgrad)" : "gms_pairs_kernel(fwd)"),
                       a.stream);
-    kern<<<dim3(gx, (unsigned)(s.c_dst / (32 * NT))), kThreads, s.lds_bytes, a.stream>>>(
+    kern<<<dim3(gx + (unsigned)a.side.blocks, (unsigned)(s.c_dst / (32 * NT))), kThreads, s.lds_bytes, a.stream>>>(
         (const T *)a.src, packed, (T *)a.dst, a.kpos, a.gmap, a.smap, a.k_vol, s.c_src, s.c_dst,
-        tiles_per_wg, a.dense_k, (int)a.n_dense);
+        tiles_per_wg, a.dense_k, (int)a.n_dense, a.side);
   }
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;
@@ -1129,6 +1144,12 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
               : raw == 1 ? gms_rows_kernel<T, NT, S, kCanRaw && sizeof(T) == 2 ? 1 : 0>
                          : gms_rows_kernel<T, NT, S, 0>;
   { const int rc_lds = allow_dynamic_lds(reinterpret_cast<const void *>(kern), lds_rows); if (rc_lds != FGMS_OK) return rc_lds; }
+  // (a tile shared by two workgroups is added up with atomics: its rows start from zero)
+  const bool overwrite = a.overwrite && rg.gz == 1 && !pair_view;
+  if (a.overwrite && !overwrite) {
+    const int rc = launch_fill_zero(a.dst, (size_t)a.n_dst * s.c_dst * sizeof(T), a.stream);
+    if (rc != FGMS_OK) return rc;
+  }
   const int part_stages = rg.gz > 1 ? rg.part_stages : 0;
   const unsigned gz = rg.gz;
   {
@@ -1139,7 +1160,7 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
     kern<<<dim3(gx + (unsigned)a.side.blocks, gy, gz), kThreads, lds_rows, a.stream>>>(
         (const T *)a.src, packed, (T *)a.dst, nbr, masks, perm, tile_order, (int)a.n_dst, a.k_vol,
         s.c_src, s.c_dst, part_stages > 0 ? part_stages : 1, a.side, pair_view ? 1 : 0,
-        (unsigned)((size_t)a.n_src * s.c_src * sizeof(T)));
+        (unsigned)((size_t)a.n_src * s.c_src * sizeof(T)), overwrite ? 1 : 0);
   }
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;
@@ -1168,7 +1189,7 @@ __global__ __launch_bounds__(kThreads, NT == 4 || BI * BJ == 16 ? 2 : 3) void bw
     int c_in, int c_out, int part_stages, const T *__restrict__ in, float *__restrict__ gw32,
     const int32_t *__restrict__ kpos, const int32_t *__restrict__ imap,
     const int32_t *__restrict__ omap, SliceMap smap, int row_x, int row_y, int row_z, int wgrad_x,
-    unsigned gout_bytes, unsigned in_bytes, int wgrad_blocks, SideJob check) {
+    unsigned gout_bytes, unsigned in_bytes, int wgrad_blocks, SideJob check, int overwrite) {
   // grid: row_x * row_y * row_z workgroups of the input gradient (tiles, column tiles,
   // parts of a tile), then wgrad_x * (tiles of dW[k]) of the weight gradient, then those of a
   // side job (the plan's fingerprint check), if there is one
@@ -1180,7 +1201,7 @@ __global__ __launch_bounds__(kThreads, NT == 4 || BI * BJ == 16 ? 2 : 3) void bw
   if ((int)blockIdx.x < rows_total) {
     const int bx = blockIdx.x % row_x, rest = blockIdx.x / row_x;
     gms_rows_body<T, NT, S, RAWD, MT>(gout, w, gin, nbr, block_masks, perm, tile_order, n_in, k_vol, c_out, c_in,
-                                      part_stages, bx, rest % row_y, rest / row_y, row_z, gout_bytes);
+                                      part_stages, bx, rest % row_y, rest / row_y, row_z, gout_bytes, 0, overwrite);
   } else {
     const int j = blockIdx.x - rows_total;
     if constexpr (BI <= 2 && BJ <= 2)
@@ -1212,6 +1233,14 @@ int launch_fused(const GmsArgs &d, const Shape &s, const Plan *p, const WgradArg
   const unsigned row_z = rg.gz;
   size_t lds = g.lds;
   if (lds < s.lds_rows_bytes) lds = s.lds_rows_bytes;
+  // what the launch adds to with atomics starts from zero: shared tiles of the input gradient, a
+  // weight gradient summed in the caller's fp32 tensor
+  const bool zero_gin = d.overwrite && rg.gz > 1, zero_gw = w.overwrite && (void *)acc32 == w.gw;
+  if (zero_gin || zero_gw) {
+    const int rc = launch_fill_zero_two(d.dst, zero_gin ? (size_t)d.n_dst * s.c_dst * sizeof(T) : 0, w.gw,
+                                        zero_gw ? (size_t)w.k_vol * w.c_in * w.c_out * sizeof(float) : 0, d.stream);
+    if (rc != FGMS_OK) return rc;
+  }
   // RAWD: how the input gradient reads the weights (2: as they lie; 4: also split into bf16
   // pairs, for fp32 tensors whose caller allows tf32 precision)
   constexpr bool kCanSplit = sizeof(T) == 4 && S == 4 && NT != 4;
@@ -1231,7 +1260,7 @@ int launch_fused(const GmsArgs &d, const Shape &s, const Plan *p, const WgradArg
         (int)d.n_dst, d.k_vol, d.c_in, d.c_out, part_stages, (const T *)w.in, acc32, w.kpos, w.imap, w.omap,
         g.smap, (int)row_x, (int)row_y, (int)row_z, (int)g.tiles,
         (unsigned)((size_t)d.n_src * s.c_src * sizeof(T)), (unsigned)((size_t)w.n_in * w.c_in * sizeof(T)),
-        (int)(g.tiles * g.ty), check);
+        (int)(g.tiles * g.ty), check, d.overwrite && rg.gz == 1 ? 1 : 0);
   }
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;
@@ -1449,6 +1478,11 @@ int launch_pair_view_gms(const GmsArgs &a, const Plan *p) {
   // choice of the wave tile's width go by their number
   GmsArgs v = a;
   v.n_dst = p->pv_rows;
+  v.overwrite = false;
+  if (a.overwrite) {
+    const int rc = launch_fill_zero(a.dst, (size_t)a.n_dst * (a.transpose_w ? a.c_in : a.c_out) * (a.dtype == FGMS_F16 ? 2 : 4), a.stream);
+    if (rc != FGMS_OK) return rc;
+  }
   const Shape s = shape_of(v);
   const int32_t *nbr = a.transpose_w ? p->pv_out : p->pv_in;
   const int32_t *dest = a.transpose_w ? p->pv_in : p->pv_out;

@@ -58,26 +58,28 @@ __global__ __launch_bounds__(256) void pad_kernel(PadBatch batch) {
   }
 }
 
-// dst[row][0 .. c) += src[row][0 .. c), rows of c_from elements in src.
+// dst[row][0 .. c) += (overwrite: =) src[row][0 .. c), rows of c_from elements in src.
 template <typename T>
-__global__ __launch_bounds__(256) void crop_kernel(const T *__restrict__ src, T *__restrict__ dst, size_t n, int c, int c_from) {
+__global__ __launch_bounds__(256) void crop_kernel(const T *__restrict__ src, T *__restrict__ dst, size_t n, int c, int c_from,
+                                                   bool overwrite) {
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
-    dst[i] = (T)((float)dst[i] + (float)src[i / c * c_from + i % c]);
+    const float v = (float)src[i / c * c_from + i % c];
+    dst[i] = (T)(overwrite ? v : (float)dst[i] + v);
   }
 }
 
-// The weight gradient's fp32 sums [k][r_from][c_from] -> dst[k][r][c] +=, rounded once; the sums
+// The weight gradient's fp32 sums [k][r_from][c_from] -> dst[k][r][c] += (overwrite: =), rounded once; the sums
 // are all zero afterwards, padding included (a product with an infinite operand leaves NaN there).
 template <typename T>
 __global__ __launch_bounds__(256) void crop_sums_kernel(float *__restrict__ sums, T *__restrict__ dst, size_t n, int r,
-                                                        int r_from, int c, int c_from) {
+                                                        int r_from, int c, int c_from, bool overwrite) {
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
     const int cc = (int)(i % c_from);
     const size_t row = i / c_from;
     const int rr = (int)(row % r_from);
     if (cc < c && rr < r) {
       T *d = dst + (row / r_from * r + rr) * c + cc;
-      *d = (T)((float)*d + sums[i]);
+      *d = (T)(overwrite ? sums[i] : (float)*d + sums[i]);
     }
     sums[i] = 0.f;
   }
@@ -114,21 +116,24 @@ int launch_pad(const PadBatch &batch, int dtype, hipStream_t s) {
   return FGMS_OK;
 }
 
-int launch_crop_add(const void *src, void *dst, size_t rows, int c, int c_from, int dtype, hipStream_t s) {
+int launch_crop(const void *src, void *dst, size_t rows, int c, int c_from, bool overwrite, int dtype, hipStream_t s) {
   const size_t n = rows * c;
   if (n == 0) return FGMS_OK;
   if (dtype == FGMS_F16)
-    crop_kernel<_Float16><<<grid_for(n), 256, 0, s>>>((const _Float16 *)src, (_Float16 *)dst, n, c, c_from);
+    crop_kernel<_Float16><<<grid_for(n), 256, 0, s>>>((const _Float16 *)src, (_Float16 *)dst, n, c, c_from, overwrite);
   else
-    crop_kernel<float><<<grid_for(n), 256, 0, s>>>((const float *)src, (float *)dst, n, c, c_from);
+    crop_kernel<float><<<grid_for(n), 256, 0, s>>>((const float *)src, (float *)dst, n, c, c_from, overwrite);
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;
 }
 
-int launch_crop_sums(float *sums, void *dst, size_t k_vol, int r, int r_from, int c, int c_from, int dtype, hipStream_t s) {
+int launch_crop_sums(float *sums, void *dst, size_t k_vol, int r, int r_from, int c, int c_from, bool overwrite, int dtype,
+                     hipStream_t s) {
   const size_t n = k_vol * r_from * c_from;
-  if (dtype == FGMS_F16) crop_sums_kernel<_Float16><<<grid_for(n), 256, 0, s>>>(sums, (_Float16 *)dst, n, r, r_from, c, c_from);
-  else crop_sums_kernel<float><<<grid_for(n), 256, 0, s>>>(sums, (float *)dst, n, r, r_from, c, c_from);
+  if (dtype == FGMS_F16)
+    crop_sums_kernel<_Float16><<<grid_for(n), 256, 0, s>>>(sums, (_Float16 *)dst, n, r, r_from, c, c_from, overwrite);
+  else
+    crop_sums_kernel<float><<<grid_for(n), 256, 0, s>>>(sums, (float *)dst, n, r, r_from, c, c_from, overwrite);
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;
 }

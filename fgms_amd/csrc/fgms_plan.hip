@@ -56,13 +56,13 @@ __global__ void pair_masks_kernel(const int32_t *__restrict__ kpos, const int32_
                                   int n_out, unsigned long long *__restrict__ rmask_out,
                                   unsigned long long *__restrict__ rmask_in, int *__restrict__ flags) {
   const int total = kpos[k_vol];
-  if (blockIdx.x == 0) {
-    // the launch's first workgroup takes the fingerprint of the lists (fgms_plan_check re-takes
-    // it); first, so that its chain of loads runs next to the others' work, not behind it
-    plan_print_block(kpos, imap, omap, k_vol, n_pairs, flags);
+  if (blockIdx.x < kPrintParts) {
+    // the launch's first workgroups take the fingerprint of the lists (fgms_plan_check re-takes
+    // it); first, so that their chain of loads runs next to the others' work, not behind it
+    plan_print_block(kpos, imap, omap, k_vol, n_pairs, flags, blockIdx.x);
     return;
   }
-  const int j = kpos[0] + (blockIdx.x - 1) * blockDim.x + threadIdx.x;      // (kpos[0] > 0: a plan over a slice of the offsets)
+  const int j = kpos[0] + (blockIdx.x - kPrintParts) * blockDim.x + threadIdx.x;      // (kpos[0] > 0: a plan over a slice of the offsets)
   if (j >= total || j >= n_pairs) return;
   int lo = 0, hi = k_vol;          // offset of pair j: the last k with kpos[k] <= j
   while (hi - lo > 1) {
@@ -599,14 +599,14 @@ void pinned_flags_put(int *q) {
   g_pinned_free.push_back(q);
 }
 
-// fgms_plan_check: the fingerprint taken again from the lists as they are now (one workgroup:
-// the sample is 4 096 pairs), compared with the build's; a difference raises the sticky flag,
-// in device memory and in the plan's pinned block.
-__global__ __launch_bounds__(1024) void plan_check_kernel(const int32_t *__restrict__ kpos,
+// fgms_plan_check: the fingerprint taken again from the lists as they are now (a workgroup per
+// part), compared with the build's; a difference raises the sticky flag, in device memory and in
+// the plan's pinned block.
+__global__ __launch_bounds__(256) void plan_check_kernel(const int32_t *__restrict__ kpos,
                                                           const int32_t *__restrict__ imap,
                                                           const int32_t *__restrict__ omap, int k_vol, int n_pairs,
                                                           int *__restrict__ flags, int *__restrict__ host) {
-  plan_check_block(kpos, imap, omap, k_vol, n_pairs, flags, host);
+  plan_check_block(kpos, imap, omap, k_vol, n_pairs, flags, host, blockIdx.x);
 }
 
 // The build's findings -> pinned host memory (mapped into the device's address space).
@@ -783,7 +783,7 @@ int plan_create(fgms_plan_t **plan_out, const int32_t *kpos, const int32_t *in_m
     }
   }
   if (tables && n_pairs > 0) {
-    pair_masks_kernel<<<(unsigned)((n_pairs + 255) / 256) + 1, 256, 0, s>>>(
+    pair_masks_kernel<<<(unsigned)((n_pairs + 255) / 256) + kPrintParts, 256, 0, s>>>(
         kpos, in_map, out_map, k_vol, (int)n_pairs, (int)n_in, (int)n_out, rmask_out, rmask_in, p->flags);
   }
   // row orders (both sides in the same launches)
@@ -939,7 +939,7 @@ bool plan_take_check(const Plan *p, SideJob *job) {
   if (hipHostGetDevicePointer((void **)&host_dev, b->host_flags, 0) != hipSuccess) host_dev = nullptr;
   *job = SideJob{};
   job->kind = 3;
-  job->blocks = 8;                 // (a multiple of 8: the workgroups behind keep their XCDs)
+  job->blocks = kPrintParts;       // (a multiple of 8: the workgroups behind keep their XCDs)
   job->src = b->kpos;
   job->dst = const_cast<int32_t *>(b->in_map);
   job->omap = b->out_map;
@@ -967,7 +967,7 @@ int plan_flush_check(const Plan *p, hipStream_t s) {
   // (a resolved plan's build has finished; no event is queried then, which a stream under
   // capture would not allow)
   if (!b->resolved && s != b->create_stream) FGMS_HIP_TRY(hipStreamWaitEvent(s, b->ready, 0));
-  plan_check_kernel<<<1, 1024, 0, s>>>(b->kpos, b->in_map, b->out_map, b->k_vol, (int)b->n_pairs, b->flags, host_dev);
+  plan_check_kernel<<<kPrintParts, 256, 0, s>>>(b->kpos, b->in_map, b->out_map, b->k_vol, (int)b->n_pairs, b->flags, host_dev);
   FGMS_HIP_TRY(hipGetLastError());
   b->checked = true;
   return FGMS_OK;

@@ -71,9 +71,14 @@ __device__ __forceinline__ void load_row(float (&x)[N], const T *__restrict__ p)
 }
 
 template <typename T, int N>
-__device__ __forceinline__ void add_store_row(T *__restrict__ p, const float (&acc)[N]) {
+__device__ __forceinline__ void add_store_row(T *__restrict__ p, const float (&acc)[N], int overwrite) {
   float old[N];
-  load_row<T, N>(old, p);
+  if (overwrite) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) old[i] = 0.f;
+  } else {
+    load_row<T, N>(old, p);
+  }
   if constexpr (sizeof(T) == 2) {
     __half2 *q = reinterpret_cast<__half2 *>(p);
 #pragma unroll
@@ -108,13 +113,22 @@ template <typename T, int CS, int CD, bool TR>
 __global__ __launch_bounds__(kSmallThreads) void gms_small_kernel(
     const T *__restrict__ src, const uint32_t *__restrict__ w, T *__restrict__ dst,
     const int32_t *__restrict__ nbr, const unsigned long long *__restrict__ block_masks,
-    const int32_t *__restrict__ perm, int n_dst, int parts) {
+    const int32_t *__restrict__ perm, int n_dst, int parts, int overwrite, SideJob side) {
+  // the leading workgroups of the grid run the side job, if there is one
+  int block_x = blockIdx.x;
+  if (side.blocks) {
+    if (block_x < side.blocks) {
+      run_side_job(side, block_x);
+      return;
+    }
+    block_x -= side.blocks;
+  }
   extern __shared__ __align__(16) float partial[];   // [blocks per WG][parts - 1][CD][64]
   constexpr int kWordsPerOffset = CS * CD * (int)sizeof(T) / 4;
   // (the wave number is the same for the 64 lanes: say so, it steers the offset loop)
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   const int part = wave & (parts - 1), block_in_wg = wave / parts;
-  const int block = blockIdx.x * (kSmallThreads / 64 / parts) + block_in_wg;
+  const int block = block_x * (kSmallThreads / 64 / parts) + block_in_wg;
   const int row = block * 64 + lane;
   const bool live = row < n_dst;
   // the mask is the same for the 64 lanes: tell the compiler, so that the offset loop and
@@ -190,7 +204,8 @@ __global__ __launch_bounds__(kSmallThreads) void gms_small_kernel(
     }
   }
   // `row` is a position in the plan's row order; a block no pair touches leaves its rows alone
-  if (live && mask) add_store_row<T, CD>(dst + (size_t)(perm ? perm[row] : row) * CD, acc);
+  // (overwrite: is zeroed)
+  if (live && (mask || overwrite)) add_store_row<T, CD>(dst + (size_t)(perm ? perm[row] : row) * CD, acc, overwrite);
 }
 
 struct Small {
@@ -229,16 +244,16 @@ int launch_small(const GmsArgs &a, const Plan *p) {
     if (v == 1 || v == 2 || v == 4) parts = v;
   }
   const int blocks_per_wg = kSmallThreads / 64 / parts;
-  const unsigned gx = (unsigned)((blocks + blocks_per_wg - 1) / blocks_per_wg);
+  const unsigned gx = (unsigned)((blocks + blocks_per_wg - 1) / blocks_per_wg) + (unsigned)a.side.blocks;
   const size_t lds = parts > 1 ? (size_t)blocks_per_wg * (parts - 1) * CD * 64 * sizeof(float) : 0;
   {
     ProfileScope prof(a.transpose_w ? "gms_small_kernel(dgrad)" : "gms_small_kernel(fwd)", a.stream);
     if (a.transpose_w)
       gms_small_kernel<T, CS, CD, true><<<gx, kSmallThreads, lds, a.stream>>>(
-          (const T *)a.src, (const uint32_t *)a.w, (T *)a.dst, nbr, masks, perm, (int)a.n_dst, parts);
+          (const T *)a.src, (const uint32_t *)a.w, (T *)a.dst, nbr, masks, perm, (int)a.n_dst, parts, a.overwrite ? 1 : 0, a.side);
     else
       gms_small_kernel<T, CS, CD, false><<<gx, kSmallThreads, lds, a.stream>>>(
-          (const T *)a.src, (const uint32_t *)a.w, (T *)a.dst, nbr, masks, perm, (int)a.n_dst, parts);
+          (const T *)a.src, (const uint32_t *)a.w, (T *)a.dst, nbr, masks, perm, (int)a.n_dst, parts, a.overwrite ? 1 : 0, a.side);
   }
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;

@@ -62,6 +62,17 @@ __device__ __forceinline__ int4v raw_weight_frag(const int4v *__restrict__ w_lds
   return __builtin_bit_cast(int4v, v);
 }
 
+// dst[rows[r]][cd0 .. cd0 + NT * 32) = 0 for the WR rows of a wave.
+template <typename T, int NT, int WR>
+__device__ __forceinline__ void zero_rows(T *__restrict__ dst, const int *__restrict__ rows, int c_dst, int cd0, int lane) {
+  constexpr int CH = NT * 32 * (int)sizeof(T) / 8;      // 8-byte pieces per row
+#pragma unroll 1
+  for (int e = lane; e < WR * CH; e += 64) {
+    const int row = rows[e / CH];
+    if (row >= 0) *reinterpret_cast<int2v *>(reinterpret_cast<char *>(dst + (size_t)row * c_dst + cd0) + (e % CH) * 8) = int2v{0, 0};
+  }
+}
+
 // Writes a wave's accumulators.  Accumulator register r of lane l holds row
 // (r / 4) * 8 + (l / 32) * 4 + r % 4 and column l % 32 of its 32x32 tile.  For
 // fp16 two lanes swap one value each so that every lane owns two neighbouring
@@ -175,7 +186,8 @@ __device__ __forceinline__ void add_rows(const float16v (&acc)[MT][NT], T *__res
 // columns of one row and a destination row is read and written as whole
 // 64..256-byte runs by neighbouring lanes instead of 4 bytes per lane.
 // stage: the wave's staging tile, MT * 32 rows of 2*S * 16 bytes.
-template <typename T, int NT, int S, bool ATOMIC, int MT>
+// OVERWRITE (not with ATOMIC): dst[rows[r]] = acc; the old values are not read.
+template <typename T, int NT, int S, bool ATOMIC, bool OVERWRITE, int MT>
 __device__ __forceinline__ void add_rows_lds(const float16v (&acc)[MT][NT], T *__restrict__ dst,
                                              const int *__restrict__ rows, float *__restrict__ stage,
                                              int c_dst, int cd0, int lane) {
@@ -184,7 +196,14 @@ __device__ __forceinline__ void add_rows_lds(const float16v (&acc)[MT][NT], T *_
   constexpr int R = (WR * 2 * S * 16) / (COLS * 4) >= 32 ? 32 : (WR * 2 * S * 16) / (COLS * 4);
   if constexpr (R < 8) {
     if constexpr (ATOMIC) write_tile<T, NT, true>(acc, dst, rows, c_dst, cd0, lane);
-    else add_rows<T, NT>(acc, dst, rows, c_dst, cd0, lane);
+    else {
+      if constexpr (OVERWRITE) {
+        zero_rows<T, NT, WR>(dst, rows, c_dst, cd0, lane);
+        __builtin_amdgcn_s_waitcnt(0x0F70);      // vmcnt(0): the zeros are on their way before the rows are read
+        __threadfence();
+      }
+      add_rows<T, NT>(acc, dst, rows, c_dst, cd0, lane);
+    }
   } else {
     constexpr int CH = COLS / 4;            // 16-byte chunks per staged row
     constexpr int IT = R * CH / 64;         // chunks per lane and pass
@@ -193,7 +212,7 @@ __device__ __forceinline__ void add_rows_lds(const float16v (&acc)[MT][NT], T *_
     // fp16 with up to 64 columns: the old values of ALL passes are fetched up front (the
     // registers of the gathered rows are free by now), so that the passes do not each wait
     // a memory round trip of their own (0.4 - 0.7 us of a launch)
-    constexpr bool kAhead = !ATOMIC && sizeof(T) == 2 && NT <= 2;
+    constexpr bool kAhead = !ATOMIC && !OVERWRITE && sizeof(T) == 2 && NT <= 2;
     typedef _Float16 half4 __attribute__((ext_vector_type(4)));
     half4 ahead[kAhead ? PASSES : 1][kAhead ? IT : 1];
     if constexpr (kAhead) {
@@ -251,10 +270,14 @@ __device__ __forceinline__ void add_rows_lds(const float16v (&acc)[MT][NT], T *_
       if constexpr (sizeof(T) == 4) {
         float4v old[IT];
 #pragma unroll
-        for (int it = 0; it < IT; ++it)
-          old[it] = *reinterpret_cast<const float4v *>(
-              reinterpret_cast<const float *>(dst) + (size_t)max(row[it], 0) * c_dst + cd0 +
-              ((it * 64 + lane) % CH) * 4);
+        for (int it = 0; it < IT; ++it) {
+          if constexpr (OVERWRITE)
+            old[it] = float4v{0.f, 0.f, 0.f, 0.f};
+          else
+            old[it] = *reinterpret_cast<const float4v *>(
+                reinterpret_cast<const float *>(dst) + (size_t)max(row[it], 0) * c_dst + cd0 +
+                ((it * 64 + lane) % CH) * 4);
+        }
 #pragma unroll
         for (int it = 0; it < IT; ++it)
           if (row[it] >= 0)
@@ -266,6 +289,8 @@ __device__ __forceinline__ void add_rows_lds(const float16v (&acc)[MT][NT], T *_
         for (int it = 0; it < IT; ++it) {
           if constexpr (kAhead)
             old[it] = ahead[p][it];
+          else if constexpr (OVERWRITE)
+            old[it] = half4{0, 0, 0, 0};
           else
             old[it] = *reinterpret_cast<const half4 *>(
                 reinterpret_cast<const _Float16 *>(dst) + (size_t)max(row[it], 0) * c_dst + cd0 +

@@ -18,7 +18,15 @@
 //    some kernels read (inference); a forward call that finds the tensor's version counter
 //    moved drops them;
 //  * HIP errors raise RuntimeError instead of passing silently.
+//
+// sparse_conv is FGMS.nn's layer as one native autograd node: a python autograd.Function around the
+// functions above costs 20-40 us of host time per pass on top of the launches (a small layer's
+// kernels take 10), zero-fills outputs that are then read back to be added to, and computes the
+// input gradient of a first layer that nobody asked for.
 #include <torch/extension.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/saved_variable.h>
 
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
@@ -53,14 +61,24 @@ std::list<CacheEntry> g_cache;            // most recently used first
 size_t g_cache_cap = 8;
 bool g_cache_enabled = true;
 
-void drop(std::list<CacheEntry>::iterator it) {
-  fgms_plan_destroy(it->plan);
-  g_cache.erase(it);
+// Entries leave the cache by way of a list that its owner destroys after g_mutex is released: the
+// last reference to a tensor may need the GIL, which another thread can hold while it waits for
+// g_mutex (calls come from python with the GIL and from autograd's threads without).
+struct Dropped {
+  std::list<CacheEntry> entries;
+  ~Dropped() {
+    for (CacheEntry &e : entries) fgms_plan_destroy(e.plan);
+  }
+};
+
+void drop(std::list<CacheEntry>::iterator it, Dropped &dropped) {
+  dropped.entries.splice(dropped.entries.begin(), g_cache, it);
 }
 
 void clear_cache() {
+  Dropped dropped;
   std::lock_guard<std::mutex> lock(g_mutex);
-  while (!g_cache.empty()) drop(g_cache.begin());
+  dropped.entries.splice(dropped.entries.begin(), g_cache);
 }
 
 void set_cache(bool enabled, int64_t capacity) {
@@ -102,6 +120,7 @@ void need_contiguous_cuda(const at::Tensor &t, const char *name) {
 // Finds or builds the plan for this map.  Returns nullptr when caching is off.
 fgms_plan_t *plan_for(const at::Tensor &kpos, const at::Tensor &in_map, const at::Tensor &out_map,
                       int64_t n_in, int64_t n_out, int k_vol, hipStream_t stream) {
+  Dropped dropped;
   std::lock_guard<std::mutex> lock(g_mutex);
   if (!g_cache_enabled) return nullptr;
   const int dev = in_map.get_device();
@@ -116,7 +135,7 @@ fgms_plan_t *plan_for(const at::Tensor &kpos, const at::Tensor &in_map, const at
         // a call later: that call drops the plan and raises.
         const int rc = fgms_plan_check(it->plan, stream, 1);      // (rides along with this call's launch)
         if (rc == FGMS_E_STALE) {
-          drop(it);
+          drop(it, dropped);
           throw std::runtime_error(
               "FGMS: the kernel map tensors were rewritten in place after their plan was cached "
               "(a write through data_ptr() does not bump the version counter); the previous call on this "
@@ -126,7 +145,7 @@ fgms_plan_t *plan_for(const at::Tensor &kpos, const at::Tensor &in_map, const at
         g_cache.splice(g_cache.begin(), g_cache, it);
         return g_cache.front().plan;
       }
-      drop(it);  // modified in place since the plan was built
+      drop(it, dropped);  // modified in place since the plan was built
       break;
     }
   }
@@ -154,7 +173,7 @@ fgms_plan_t *plan_for(const at::Tensor &kpos, const at::Tensor &in_map, const at
                            in_map.numel(), stream));
   g_cache.push_front(CacheEntry{kpos, in_map, out_map, version_of(kpos), version_of(in_map),
                                 version_of(out_map), n_in, n_out, dev, plan, view});
-  while (g_cache.size() > g_cache_cap) drop(std::prev(g_cache.end()));
+  while (g_cache.size() > g_cache_cap) drop(std::prev(g_cache.end()), dropped);
   return plan;
 }
 
@@ -284,7 +303,98 @@ void ConvolutionBackward(const at::Tensor out_feats_grad, const at::Tensor in_fe
                  dtype_of(in_feats), plan, stream));
 }
 
+namespace {
+
+// One kernel map as a layer uses it.
+struct LayerMap {
+  at::Tensor kpos, in_map, out_map;
+  int64_t n_in, n_out;
+};
+
+at::Tensor layer_forward(const at::Tensor &feats, const at::Tensor &weight, const LayerMap &map, bool tf32) {
+  const int k_vol = (int)weight.size(0);
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(feats.device());
+  hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
+  at::Tensor out = at::empty({map.n_out, weight.size(2)}, feats.options().requires_grad(false));
+  refresh_pin(weight);
+  fgms_plan_t *plan = plan_for(map.kpos, map.in_map, map.out_map, map.n_in, map.n_out, k_vol, stream);
+  check(fgms_conv_fwd(feats.data_ptr(), weight.data_ptr(), out.data_ptr(), i32(map.kpos), i32(map.in_map), i32(map.out_map),
+                      tf32, map.n_in, map.n_out, (int)weight.size(1), (int)weight.size(2), k_vol, map.in_map.numel(),
+                      dtype_of(feats), plan, stream));
+  return out;
+}
+
+struct SparseConvBackward final : public torch::autograd::Node {
+  torch::autograd::SavedVariable feats, weight;
+  LayerMap map;
+  bool tf32 = false;
+
+  torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    if (!grads[0].defined()) return {at::Tensor(), at::Tensor()};
+    const at::Tensor x = feats.unpack(shared_from_this()), w = weight.unpack(shared_from_this());
+    at::NoGradGuard no_grad;
+    at::Tensor g = grads[0].contiguous();
+    same_dtype(x, g, "the output gradient");
+    const int k_vol = (int)w.size(0);
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
+    at::Tensor gx, gw;
+    if (task_should_compute_output(0)) gx = at::empty(x.sizes(), x.options().requires_grad(false));
+    if (task_should_compute_output(1)) gw = at::empty(w.sizes(), w.options().requires_grad(false));
+    fgms_plan_t *plan = plan_for(map.kpos, map.in_map, map.out_map, map.n_in, map.n_out, k_vol, stream);
+    check(fgms_conv_bwd(g.data_ptr(), x.data_ptr(), w.data_ptr(), gx.defined() ? gx.data_ptr() : nullptr,
+                        gw.defined() ? gw.data_ptr() : nullptr, i32(map.kpos), i32(map.in_map), i32(map.out_map), tf32,
+                        map.n_in, map.n_out, (int)w.size(1), (int)w.size(2), k_vol, map.in_map.numel(), dtype_of(x), plan,
+                        stream));
+    return {gx, gw};
+  }
+
+  void release_variables() override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    feats.reset_data();
+    weight.reset_data();
+  }
+
+  std::string name() const override { return "SparseConvBackward"; }
+};
+
+// out[out_map[j]] += feats[in_map[j]] @ weight[k] over a zero output; differentiable in feats and weight.
+at::Tensor sparse_conv(const at::Tensor &feats, const at::Tensor &weight, const at::Tensor &kpos, const at::Tensor &in_map,
+                       const at::Tensor &out_map, int64_t n_in, int64_t n_out, bool tf32) {
+  if (feats.dim() != 2 || weight.dim() != 3 || weight.size(0) != kpos.numel() - 1)
+    throw std::invalid_argument("expected feats [N, Cin] and weight [K, Cin, Cout] with K = the map's offsets");
+  if (feats.size(0) != n_in)
+    throw std::invalid_argument("feats has " + std::to_string(feats.size(0)) + " rows, the kernel map expects " +
+                                std::to_string(n_in));
+  check_channels(feats, weight);
+  const LayerMap map{kpos, in_map, out_map, n_in, n_out};
+  at::Tensor x, w, out;
+  {
+    at::AutoGradMode no_grad(false);
+    x = feats.contiguous();
+    w = weight.contiguous();
+    need_contiguous_cuda(x, "in_feats"); need_contiguous_cuda(w, "kernel"); need_contiguous_cuda(kpos, "kpos");
+    need_contiguous_cuda(in_map, "in_map"); need_contiguous_cuda(out_map, "out_map");
+    same_dtype(x, w, "kernel");
+    out = layer_forward(x, w, map, tf32);
+  }
+  if (at::GradMode::is_enabled() && (feats.requires_grad() || weight.requires_grad())) {
+    auto node = std::shared_ptr<SparseConvBackward>(new SparseConvBackward(), torch::autograd::deleteNode);
+    node->set_next_edges(torch::autograd::collect_next_edges(feats, weight));
+    node->feats = torch::autograd::SavedVariable(x, false);
+    node->weight = torch::autograd::SavedVariable(w, false);
+    node->map = map;
+    node->tf32 = tf32;
+    torch::autograd::set_history(out, node);
+  }
+  return out;
+}
+
+}  // namespace
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("sparse_conv", &sparse_conv);
   m.def("fgms_fusion_fwd_cuda", &ConvolutionForwardFused);
   m.def("fgms_fwd_cuda", &ConvolutionForward);
   m.def("fgms_bwd_cuda", &ConvolutionBackward);

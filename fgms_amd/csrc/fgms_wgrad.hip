@@ -116,7 +116,16 @@ template <typename T, int CS, int CD>
 __global__ __launch_bounds__(kSkinnyThreads) void wgrad_skinny_kernel(
     const T *__restrict__ in, const T *__restrict__ gout, float *__restrict__ gw32,
     const int32_t *__restrict__ kpos, const int32_t *__restrict__ imap,
-    const int32_t *__restrict__ omap, int k_vol, SliceMap smap) {
+    const int32_t *__restrict__ omap, int k_vol, SliceMap smap, SideJob side) {
+  // the leading workgroups of the grid run the side job, if there is one
+  int block_x = blockIdx.x;
+  if (side.blocks) {
+    if (block_x < side.blocks) {
+      run_side_job(side, block_x);
+      return;
+    }
+    block_x -= side.blocks;
+  }
   constexpr int KD = 16 / (int)sizeof(T);     // output channels per lane: one 16-byte load
   constexpr int GD = CD / KD;                 // lanes per pair = steps per round
   constexpr int PPS = 64 / GD;                // pairs per step
@@ -125,7 +134,7 @@ __global__ __launch_bounds__(kSkinnyThreads) void wgrad_skinny_kernel(
   extern __shared__ float red[];            // [waves - 1][CS][CD]
   constexpr int kWavesS = kSkinnyThreads / 64;
   int k, first, count;
-  if (!locate_slice(kpos, smap, k_vol, blockIdx.x, k, first, count)) return;
+  if (!locate_slice(kpos, smap, k_vol, block_x, k, first, count)) return;
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int sub = lane / GD, cg = lane % GD;
   const int rounds = (count + kSkinnyThreads - 1) / kSkinnyThreads;
@@ -239,9 +248,9 @@ __global__ __launch_bounds__(kSkinnyThreads) void wgrad_skinny_kernel(
 }
 
 // dst[i] += acc[i] rounded once to fp16 and acc[i] = 0, in a launch of its own.
-__global__ void add_and_clear_kernel(__half *__restrict__ dst, float *__restrict__ acc, size_t n) {
+__global__ void add_and_clear_kernel(__half *__restrict__ dst, float *__restrict__ acc, size_t n, bool overwrite) {
   add_and_clear_elements(dst, acc, n, (size_t)blockIdx.x * blockDim.x + threadIdx.x,
-                         (size_t)gridDim.x * blockDim.x);
+                         (size_t)gridDim.x * blockDim.x, overwrite);
 }
 
 int blocks_of(int c) { return c % 128 == 0 ? 4 : (c % 64 == 0 ? 2 : 1); }
@@ -338,10 +347,6 @@ bool skinny_shape(const WgradArgs &a) {
 
 template <typename T, int CS, int CD>
 int launch_skinny(const WgradArgs &a, float *acc32) {
-  if (a.side.kind != 0) {       // nothing rides along with this launch
-    int rc = launch_side_job(a.side, a.stream);
-    if (rc != FGMS_OK) return rc;
-  }
   // Few, big workgroups (about two to a CU): measured on the 4 -> 32 layer over 2.1 M
   // pairs, 34 us against 40 us with six to a CU, 36-72 us with equal runs of the pair list
   // instead of the plan's (offset, band) cells (workgroups that run at the same time then
@@ -355,8 +360,8 @@ int launch_skinny(const WgradArgs &a, float *acc32) {
   { const int rc_lds = allow_dynamic_lds(reinterpret_cast<const void *>(kern), (size_t)lds); if (rc_lds != FGMS_OK) return rc_lds; }
   {
     ProfileScope prof("wgrad_skinny_kernel", a.stream);
-    kern<<<(unsigned)tiles, kSkinnyThreads, lds, a.stream>>>(
-        (const T *)a.in, (const T *)a.gout, acc32, a.kpos, a.imap, a.omap, a.k_vol, smap);
+    kern<<<(unsigned)tiles + (unsigned)a.side.blocks, kSkinnyThreads, lds, a.stream>>>(
+        (const T *)a.in, (const T *)a.gout, acc32, a.kpos, a.imap, a.omap, a.k_vol, smap, a.side);
   }
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;
@@ -469,18 +474,24 @@ int wgrad_accumulator(const WgradArgs &a, float **acc32) {
 }
 
 int wgrad_finish(const WgradArgs &a, float *acc32) {
-  if (a.crop_in) return launch_crop_sums(acc32, a.gw, (size_t)a.k_vol, a.crop_in, a.c_in, a.crop_out, a.c_out, a.dtype, a.stream);
+  if (a.crop_in) return launch_crop_sums(acc32, a.gw, (size_t)a.k_vol, a.crop_in, a.c_in, a.crop_out, a.c_out, a.overwrite, a.dtype, a.stream);
   if (a.dtype != FGMS_F16) return FGMS_OK;
   const size_t n = (size_t)a.k_vol * a.c_in * a.c_out;
-  add_and_clear_kernel<<<(unsigned)((n + 255) / 256), 256, 0, a.stream>>>((__half *)a.gw, acc32, n);
+  add_and_clear_kernel<<<(unsigned)((n / 4 + 255) / 256 + 1), 256, 0, a.stream>>>((__half *)a.gw, acc32, n, a.overwrite);
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;
 }
 
-int launch_mfma_wgrad(const WgradArgs &a) {
+int launch_mfma_wgrad(const WgradArgs &args) {
+  WgradArgs a = args;
+  // (a pending fingerprint check of the plan rides along as the launch's side job)
+  if (!a.side.kind && a.plan) (void)plan_take_check(a.plan, &a.side);
   float *acc32 = nullptr;
   int rc = wgrad_accumulator(a, &acc32);
   if (rc != FGMS_OK) return rc;
+  if (a.overwrite && (void *)acc32 == a.gw &&
+      (rc = launch_fill_zero(a.gw, (size_t)a.k_vol * a.c_in * a.c_out * sizeof(float), a.stream)))
+    return rc;
   if (a.dtype != FGMS_F16 && !a.crop_in) return dispatch<float>(a, acc32);
   if ((rc = a.dtype == FGMS_F16 ? dispatch<__half>(a, acc32) : dispatch<float>(a, acc32))) {
     const size_t bytes = a.acc_override ? (size_t)a.k_vol * a.c_in * a.c_out * sizeof(float)
@@ -498,6 +509,7 @@ int launch_mfma_wgrad(const WgradArgs &a) {
     f.acc = acc32;
     f.n = n;
     f.dtype = a.dtype;
+    f.overwrite = a.overwrite;
     size_t blocks = ((n + 2047) / 2048 + 7) / 8 * 8;   // about 8 elements per thread
     f.blocks = (int)(blocks > 1024 ? 1024 : blocks);
     return FGMS_OK;

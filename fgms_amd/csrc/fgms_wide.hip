@@ -30,7 +30,16 @@ __global__ __launch_bounds__(kWideThreads) void gms_wide_kernel(
     const __half *__restrict__ src, const int4v *__restrict__ packed, __half *__restrict__ dst,
     const int32_t *__restrict__ kpos, const int32_t *__restrict__ gmap,
     const int32_t *__restrict__ smap, int k_vol, int c_src, int c_dst, int tiles_per_wg,
-    int dense_k, int dense_rows) {
+    int dense_k, int dense_rows, SideJob side) {
+  // the leading workgroups of the grid run the side job, if there is one
+  int block_x = blockIdx.x;
+  if (side.blocks) {
+    if (block_x < side.blocks) {
+      if (blockIdx.y == 0) run_side_job(side, block_x);
+      return;
+    }
+    block_x -= side.blocks;
+  }
   constexpr int S = 4;
   extern __shared__ int4v lds[];
   int4v *a_buf = lds;                              // [2][4 row groups][512]
@@ -97,7 +106,7 @@ __global__ __launch_bounds__(kWideThreads) void gms_wide_kernel(
   };
   clear();
 
-  int t = blockIdx.x * tiles_per_wg;
+  int t = block_x * tiles_per_wg;
   const int t_end = t + tiles_per_wg;
   int k, first, count;
   if (!tile_at(t, k, first, count)) return;
@@ -191,9 +200,9 @@ int launch_wide_gms(const GmsArgs &a) {
   if (rc_lds != FGMS_OK) return rc_lds;
   {
     ProfileScope prof(a.transpose_w ? "gms_wide_kernel(dgrad)" : "gms_wide_kernel(fwd)", a.stream);
-    gms_wide_kernel<<<dim3(gx, (unsigned)(c_dst / kWideCols)), kWideThreads, lds_bytes, a.stream>>>(
+    gms_wide_kernel<<<dim3(gx + (unsigned)a.side.blocks, (unsigned)(c_dst / kWideCols)), kWideThreads, lds_bytes, a.stream>>>(
         (const __half *)a.src, (const int4v *)packed, (__half *)a.dst, a.kpos, a.gmap, a.smap, a.k_vol, c_src,
-        c_dst, tiles_per_wg, a.dense_k, (int)a.n_dense);
+        c_dst, tiles_per_wg, a.dense_k, (int)a.n_dense, a.side);
   }
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;

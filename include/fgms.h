@@ -166,6 +166,22 @@ int fgms_bwd(const void *out_feats_grad, const void *in_feats, const void *kerne
              int64_t n_in, int64_t n_out, int c_in, int c_out, int k_vol,
              int64_t n_pairs, int dtype, fgms_plan_t *plan, void *stream);
 
+/*
+ * fgms_fusion_fwd and fgms_bwd for callers that hold no partial results (an autograd layer): the
+ * outputs are WRITTEN, not added to, so they need not be zeroed first, and a gradient whose pointer
+ * is NULL is not computed (the input gradient of a network's first layer).  No counterpart in the
+ * reference, whose kernels add to caller-zeroed tensors only (cpu-check.py:107-116).
+ */
+int fgms_conv_fwd(const void *in_feats, const void *kernel, void *out_feats,
+                  const int32_t *kpos, const int32_t *in_map, const int32_t *out_map, int arch80,
+                  int64_t n_in, int64_t n_out, int c_in, int c_out, int k_vol,
+                  int64_t n_pairs, int dtype, fgms_plan_t *plan, void *stream);
+int fgms_conv_bwd(const void *out_feats_grad, const void *in_feats, const void *kernel,
+                  void *in_feats_grad, void *kernel_grad,
+                  const int32_t *kpos, const int32_t *in_map, const int32_t *out_map, int arch80,
+                  int64_t n_in, int64_t n_out, int c_in, int c_out, int k_vol,
+                  int64_t n_pairs, int dtype, fgms_plan_t *plan, void *stream);
+
 /* The two halves of fgms_bwd on their own (the reference launches them back to
  * back, backend/spconv.cu:454-461 + 495-548 / 553-569); exposed so each can be
  * timed and tested separately. */

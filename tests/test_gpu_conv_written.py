@@ -1,0 +1,64 @@
+"""fgms_conv_fwd / fgms_conv_bwd write their outputs: buffers full of NaN, rows no pair reaches, one
+gradient without the other -- for every kernel family the dispatch has, against the CPU oracle."""
+import numpy as np
+import pytest
+import torch
+
+from fgms_amd import clouds
+from tests import gpu_util as G
+
+pytestmark = pytest.mark.gpu
+
+
+def holes(n_side, seed):
+    """A map whose last third of output rows and first third of input rows have no pair."""
+    rng = np.random.default_rng(seed)
+    imap, omap, knnz = [], [], []
+    for k in range(27):
+        m = 0 if k in (3, 20) else int(rng.integers(1, n_side // 3))
+        i = n_side // 3 + rng.permutation(n_side - n_side // 3)[:m]
+        o = np.sort(rng.permutation(n_side - n_side // 3)[:m])
+        imap.append(i.astype(np.int32)); omap.append(o.astype(np.int32)); knnz.append(m)
+    kpos = np.concatenate([[0], np.cumsum(knnz)]).astype(np.int32)
+    return np.concatenate(imap), np.concatenate(omap), np.array(knnz, np.int32), kpos
+
+
+@pytest.mark.parametrize("use_plan", [True, False], ids=["plan", "no_plan"])
+@pytest.mark.parametrize("dtype,tf32", [(np.float16, False), (np.float32, False), (np.float32, True)], ids=["fp16", "fp32", "tf32"])
+@pytest.mark.parametrize("n,shape", [(65, (32, 32)), (700, (4, 32)), (700, (64, 20)), (1500, (64, 64)), (1500, (16, 16)),
+                                     (3000, (32, 256)), (20000, (128, 128)), (70001, (64, 64))])
+def test_written_not_added(oracle, n, shape, dtype, tf32, use_plan):
+    from fgms_amd import capi
+    capi.set_kernel_policy(0)
+    maps = holes(n, n + shape[0])
+    L = clouds.make_layer(np.random.default_rng(7), *maps, n, n, *shape, dtype)
+    D = G.to_dev(L)
+    mode = G.mode_of(L["in_feats"].dtype, tf32)
+    args = (L["knnz"], L["imap"], L["omap"])
+    plan = capi.Plan(D["kpos"], D["imap"], D["omap"], n, n) if use_plan else None
+    nan = lambda *s: torch.full(s, float("nan"), dtype=D["in_feats"].dtype, device="cuda")
+    maps = (D["kpos"], D["imap"], D["omap"])
+    out = nan(n, shape[1])
+    capi.conv_fwd(D["in_feats"], D["kernel"], out, *maps, arch80=tf32, plan=plan)
+    G.assert_close(out.cpu().numpy(), oracle.c_fwd(L["in_feats"], L["kernel"], *args, n), mode, "fwd")
+    ref_gi = oracle.c_dgrad(L["out_grad"], L["kernel"], *args, n)
+    ref_gw = oracle.np_wgrad(L["in_feats"], L["out_grad"], *args, 27)
+    for want in ((True, True), (True, False), (False, True)):
+        gi = nan(n, shape[0]) if want[0] else None
+        gw = nan(27, *shape) if want[1] else None
+        capi.conv_bwd(D["out_grad"], D["in_feats"], D["kernel"], gi, gw, *maps, arch80=tf32, plan=plan)
+        if want[0]:
+            G.assert_close(gi.cpu().numpy(), ref_gi, mode, "dgrad")
+        if want[1]:
+            G.assert_close(gw.cpu().numpy(), ref_gw, mode, "wgrad")
+
+
+def test_no_pairs():
+    from fgms_amd import capi
+    x, w = torch.ones(5, 32, device="cuda"), torch.ones(27, 32, 32, device="cuda")
+    kpos = torch.zeros(28, dtype=torch.int32, device="cuda")
+    none = torch.zeros(0, dtype=torch.int32, device="cuda")
+    out, gi, gw = (torch.full_like(t, 3.0) for t in (x, x, w))
+    capi.conv_fwd(x, w, out, kpos, none, none)
+    capi.conv_bwd(x, x, w, gi, gw, kpos, none, none)
+    assert not out.any() and not gi.any() and not gw.any()
