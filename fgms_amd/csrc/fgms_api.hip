@@ -281,7 +281,36 @@ std::vector<PoolBlock> g_pool_free;
 std::map<void *, std::pair<size_t, int>> g_pool_live;   // ptr -> (bytes, device)
 size_t g_pool_cached = 0;
 constexpr size_t kPoolMaxCached = (size_t)2 << 30;
+
+// Events for blocks on their way back, and for plans: kept per device, a few dozen at most.
+std::mutex g_event_mutex;
+std::vector<std::pair<int, hipEvent_t>> g_events;
 }  // namespace
+
+hipEvent_t event_get(int device) {
+  {
+    std::lock_guard<std::mutex> lock(g_event_mutex);
+    for (size_t i = g_events.size(); i-- > 0;)
+      if (g_events[i].first == device) {
+        hipEvent_t ev = g_events[i].second;
+        g_events.erase(g_events.begin() + i);
+        return ev;
+      }
+  }
+  hipEvent_t ev = nullptr;
+  return hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess ? ev : nullptr;
+}
+
+void event_put(hipEvent_t ev, int device) {
+  {
+    std::lock_guard<std::mutex> lock(g_event_mutex);
+    if (g_events.size() < 64) {
+      g_events.emplace_back(device, ev);
+      return;
+    }
+  }
+  (void)hipEventDestroy(ev);
+}
 
 int pool_alloc(void **ptr, size_t bytes, hipStream_t user) {
   *ptr = nullptr;
@@ -308,7 +337,7 @@ int pool_alloc(void **ptr, size_t bytes, hipStream_t user) {
   if (got.ptr) {
     if (got.ready) {
       hipError_t e = hipStreamWaitEvent(user, got.ready, 0);
-      (void)hipEventDestroy(got.ready);
+      event_put(got.ready, got.device);
       if (e != hipSuccess) {
         set_error("pool_alloc: hipStreamWaitEvent: %s", hipGetErrorString(e));
         return FGMS_E_HIP;
@@ -345,9 +374,8 @@ void pool_free(void *ptr, hipStream_t last_user, bool idle) {
   }
   if (!idle) {
     // queued work may still read the block: mark the point after which it is free
-    hipEvent_t ev = nullptr;
-    if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess ||
-        hipEventRecord(ev, last_user) != hipSuccess) {
+    hipEvent_t ev = event_get(b.device);
+    if (!ev || hipEventRecord(ev, last_user) != hipSuccess) {
       if (ev) (void)hipEventDestroy(ev);
       (void)hipFree(ptr);     // synchronises; also the path taken while the runtime shuts down
       return;

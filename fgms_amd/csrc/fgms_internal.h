@@ -141,6 +141,12 @@ struct Plan {
   int32_t *perm_in;   // [n_in]
   int32_t *nbr_out;   // [k_vol, n_out]: input row feeding the output row at position p through offset k, or -1
   int32_t *nbr_in;    // [k_vol, n_in]:  output row fed by the input row at position p through offset k, or -1
+  // entries from one offset's row of a table to the next one's.  A mirrored map (a submanifold map is
+  // its own mirror image: input row r reaches through offset k what output row r is reached by through
+  // k_vol - 1 - k) keeps one table and one order for both sides: nbr_in starts at nbr_out's last offset
+  // and its stride is negative
+  int nbr_stride_out, nbr_stride_in;
+  void *block;        // the pool block all of the plan's tables lie in
   // bit k of mask_out[b] : some row of the 64-row block b has a neighbour through
   // offset k (only built when k_vol <= 64; the output-stationary kernels need it)
   unsigned long long *mask_out;  // [ceil(n_out / 64)]
@@ -243,6 +249,9 @@ bool mfma_gms_supported(const GmsArgs &a);
 int pool_alloc(void **ptr, size_t bytes, hipStream_t user);
 void pool_free(void *ptr, hipStream_t last_user, bool idle);
 void pool_trim(size_t keep_bytes);
+// Events without timing, created on the current device (`device`) or reused.
+hipEvent_t event_get(int device);
+void event_put(hipEvent_t ev, int device);
 // Raises a kernel's dynamic-LDS limit to `bytes` (hipFuncSetAttribute) unless an earlier call
 // on this device already allowed as much: the attribute call costs a microsecond per launch.
 int allow_dynamic_lds(const void *kernel, size_t bytes);

@@ -14,29 +14,20 @@
 
 #include "fgms_device.h"
 #include "fgms_internal.h"
+#include "fgms_plan_build.h"
 
 namespace fgms {
 namespace {
 
-// p[0 .. n) = v; p is 16-byte aligned (pool blocks are), 16 bytes per store.
-__global__ void fill_i32_kernel(int32_t *__restrict__ p, size_t n, int32_t v) {
-  typedef int int4v_ __attribute__((ext_vector_type(4)));
-  size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  const size_t n4 = n / 4;
-  for (size_t q = i; q < n4; q += stride) reinterpret_cast<int4v_ *>(p)[q] = int4v_{v, v, v, v};
-  if (i < n % 4) p[n4 * 4 + i] = v;
-}
-
-// Two fills in one launch (the build is a chain of small launches, each bound by its latency).
-__global__ void fill_two_kernel(int32_t *__restrict__ p1, size_t n1, int32_t v1, int32_t *__restrict__ p2, size_t n2,
-                                int32_t v2) {
+__global__ __launch_bounds__(256) void fills_kernel(FillBatch batch) {
   typedef int int4v_ __attribute__((ext_vector_type(4)));
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (size_t)gridDim.x * blockDim.x;
-  for (size_t q = i; q < n1 / 4; q += stride) reinterpret_cast<int4v_ *>(p1)[q] = int4v_{v1, v1, v1, v1};
-  if (i < n1 % 4) p1[n1 / 4 * 4 + i] = v1;
-  for (size_t q = i; q < n2 / 4; q += stride) reinterpret_cast<int4v_ *>(p2)[q] = int4v_{v2, v2, v2, v2};
-  if (i < n2 % 4) p2[n2 / 4 * 4 + i] = v2;
+  for (int r = 0; r < batch.count; ++r) {
+    const FillRange &f = batch.range[r];       // (16-byte aligned: pool blocks and what an Arena cuts from them)
+    const int32_t v = f.v;
+    for (size_t q = i; q < f.n / 4; q += stride) reinterpret_cast<int4v_ *>(f.p)[q] = int4v_{v, v, v, v};
+    if (i < f.n % 4) f.p[f.n / 4 * 4 + i] = v;
+  }
 }
 
 // flags[0]: an index is out of range; flags[1]: two pairs of one offset share
@@ -93,115 +84,102 @@ __global__ void pair_masks_kernel(const int32_t *__restrict__ kpos, const int32_
 // high offsets, which is what makes neighbours in the order similar; so the sort runs most
 // significant bits first: a counting sort on the top kBinBits bits of the mask over the whole
 // side (histogram per chunk of rows, scan, stable scatter), then a full sort by (mask, row) of
-// every window of kWindow positions in LDS.  Inside a bin only rows of one window are ordered
+// every window of kWindow positions.  Inside a bin only rows of one window are ordered
 // among themselves; measured on the benchmark clouds that costs 1 % more (block, offset) steps
-// than the exact sort, for a third of its time.  Both sides of a plan go through the same
+// than the exact sort, for a third of its time.  (Bins of 16 bits without the windows: 4 % more
+// steps on surfaces, 23 % on scattered clouds.)  Both sides of a plan go through the same
 // launches (blockIdx.y = side).
-constexpr int kBinBits = 11;
-constexpr int kBins = 1 << kBinBits;
-constexpr int kChunk = 2048;       // rows per workgroup of the histogram / scatter kernels
-constexpr int kWindow = 2048;      // positions per workgroup of the window sort
-constexpr int kSortThreads = 1024;
-
-struct SortSide {
-  const unsigned long long *rmask;
-  int32_t *perm_tmp;     // order after the counting sort
-  int32_t *perm;         // final order: position -> row
-  int32_t *inv;          // row -> position
-  int32_t *hist;         // [chunks][kBins] rows per (chunk, bin)
-  int32_t *hist_before;  // [chunks][kBins] rows of the bin in earlier chunks
-  int32_t *bin_start;    // [kBins] rows per bin
-  int n, chunks;
-};
-struct SortArgs {
-  SortSide side[2];
-  int k_vol;
-};
-
-__device__ __forceinline__ int top_bits(unsigned long long m, int k_vol) {
-  const int shift = k_vol > kBinBits ? k_vol - kBinBits : 0;
-  return (int)((m >> shift) & (kBins - 1));
-}
-
 __global__ __launch_bounds__(kSortThreads) void sort_hist_kernel(SortArgs a) {
   const SortSide &sd = a.side[blockIdx.y];
-  const int chunk = blockIdx.x;
-  if (chunk >= sd.chunks) return;
+  if ((int)blockIdx.x >= sd.chunks) return;
   __shared__ int hist[kBins];
-  for (int i = threadIdx.x; i < kBins; i += kSortThreads) hist[i] = 0;
-  __syncthreads();
-  for (int e = threadIdx.x; e < kChunk; e += kSortThreads) {
-    const int row = chunk * kChunk + e;
-    if (row < sd.n) atomicAdd(&hist[top_bits(sd.rmask[row], a.k_vol)], 1);
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < kBins; i += kSortThreads) sd.hist[(size_t)chunk * kBins + i] = hist[i];
+  sort_hist_body(sd, a.k_vol, blockIdx.x, hist, kSortThreads);
 }
 
 // hist[chunk][bin] -> hist_before[chunk][bin] = rows of the bin in earlier chunks, and
-// bin_total[bin].  Bins are independent: 256 of them per workgroup (one workgroup alone reads
-// the 800 KB of counts at 30 GB/s).
-constexpr int kScanBins = 256;
-__global__ __launch_bounds__(kScanBins) void sort_scan_kernel(SortArgs a) {
+// bin_total[bin].  Bins are independent: 64 of them per workgroup of 256 threads, a quarter of the
+// chunks each (one workgroup alone reads the 800 KB of counts at 30 GB/s).
+constexpr int kScanBins = 64;
+__global__ __launch_bounds__(256) void sort_scan_kernel(SortArgs a) {
   const SortSide &sd = a.side[blockIdx.y];
   if (sd.chunks == 0) return;
-  const int bin = blockIdx.x * kScanBins + threadIdx.x;
+  __shared__ int part_sum[4][kScanBins];
+  const int part = threadIdx.x / kScanBins, b = threadIdx.x % kScanBins;
+  const int bin = blockIdx.x * kScanBins + b;
+  const int per = (sd.chunks + 3) / 4, c0 = min(part * per, sd.chunks), c1 = min(c0 + per, sd.chunks);
   const int32_t *__restrict__ h = sd.hist + bin;
   int32_t *__restrict__ hb = sd.hist_before + bin;
-  int run = 0, c = 0;
-  for (; c + 8 <= sd.chunks; c += 8) {
-    int v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = h[(size_t)(c + u) * kBins];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      hb[(size_t)(c + u) * kBins] = run;
-      run += v[u];
-    }
-  }
-  for (; c < sd.chunks; ++c) {
+  int sum = 0;
+#pragma unroll 8
+  for (int c = c0; c < c1; ++c) sum += h[(size_t)c * kBins];
+  part_sum[part][b] = sum;
+  __syncthreads();
+  int run = 0;
+  for (int q = 0; q < part; ++q) run += part_sum[q][b];
+#pragma unroll 8
+  for (int c = c0; c < c1; ++c) {
+    const int v = h[(size_t)c * kBins];
     hb[(size_t)c * kBins] = run;
-    run += h[(size_t)c * kBins];
+    run += v;
   }
-  sd.bin_start[bin] = run;        // (the bin's total; the scatter kernel turns totals into starts)
+  if (part == 3) sd.bin_start[bin] = run;        // (the bin's total; the scatter kernel turns totals into starts)
 }
 
-// Bitonic sort of n2 (a power of two) (key, value) pairs in LDS, ascending, by the `threads`
-// threads of the workgroup.  Wave w owns the elements [w * per, (w + 1) * per), per = n2 / waves:
-// a phase whose partner distance j is below `per` stays inside the wave's own elements and needs
-// no workgroup barrier (a wave's LDS operations complete in order), the few phases with larger
-// j do.
-template <typename K, typename V>
-__device__ __forceinline__ void bitonic_sort(K *key, V *val, int n2, int threads) {
-  const int waves = threads / 64, per = n2 / waves;
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-  bool wide = true;           // was the previous phase a workgroup-wide one (or the start)?
-  for (int k2 = 2; k2 <= n2; k2 <<= 1)
-    for (int j = k2 >> 1; j > 0; j >>= 1) {
-      const bool local = j < per;
-      if (local && wide) __syncthreads();        // the wave's elements as the others left them
-      if (!local) __syncthreads();
-      for (int c = lane; c < per / 2; c += 64) {
-        // comparator c of this wave: elements i and i + j, i without bit j
-        const int cc = wave * (per / 2) + c;
-        const int i = 2 * cc - (cc & (j - 1));
-        const int o = i + j;
-        const bool asc = (i & k2) == 0;
-        const K a = key[i], b = key[o];
-        const V va = val[i], vb = val[o];
-        const bool gt = a > b || (a == b && va > vb);
-        if (gt == asc) {
-          key[i] = b; key[o] = a;
-          val[i] = vb; val[o] = va;
-        }
-      }
-      if (local) {
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-      }
-      wide = !local;
+// Value of the lane whose number differs from this lane's in bit J.
+template <int J>
+__device__ __forceinline__ unsigned lane_xor(unsigned v) {
+  const int x = (int)v;
+  if constexpr (J == 1) return (unsigned)__builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, true);           // quad_perm [1,0,3,2]
+  else if constexpr (J == 2) return (unsigned)__builtin_amdgcn_mov_dpp(x, 0x4E, 0xF, 0xF, true);      // quad_perm [2,3,0,1]
+  else if constexpr (J == 4)                                                                          // row_half_mirror, quad_perm [3,2,1,0]
+    return (unsigned)__builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(x, 0x141, 0xF, 0xF, true), 0x1B, 0xF, 0xF, true);
+  else if constexpr (J == 8) return (unsigned)__builtin_amdgcn_mov_dpp(x, 0x128, 0xF, 0xF, true);     // row_ror:8
+  else return (unsigned)__shfl_xor(x, J);
+}
+template <int J>
+__device__ __forceinline__ unsigned long long lane_xor(unsigned long long v) {
+  return (unsigned long long)lane_xor<J>((unsigned)v) | (unsigned long long)lane_xor<J>((unsigned)(v >> 32)) << 32;
+}
+
+// Bitonic sort of 2048 keys, ascending, by 1024 threads: wave w holds elements w * 128 ... in two
+// registers per lane (element w * 128 + r * 64 + lane in key[r]), so that 56 of the 66 phases are
+// register exchanges inside a wave (most of them on the vector ALUs alone) and only the 10 with
+// partners 128 or more apart go through LDS (`buf`: 2 x 2048 keys).  A bitonic sort with every
+// phase in LDS took 22 us for 2048 32-bit pairs where this takes 5.
+template <typename K, int K2, int J>
+__device__ __forceinline__ void bitonic_phases(K (&key)[2], K *buf, int base, int lane, int &flip) {
+  if constexpr (J >= 128) {
+    K *to = buf + flip * 2048;
+    flip ^= 1;
+    to[base + lane] = key[0];
+    to[base + 64 + lane] = key[1];
+    __syncthreads();
+    const bool low = ((base & J) == 0) == ((base & K2) == 0);      // (J, K2 >= 128: bits of the wave's number)
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      const K o = to[(base ^ J) + r * 64 + lane];
+      key[r] = (o < key[r]) == low ? o : key[r];
     }
-  __syncthreads();
+  } else if constexpr (J == 64) {
+    const bool asc = (base & K2) == 0;
+    const K lo = key[0] < key[1] ? key[0] : key[1], hi = key[0] < key[1] ? key[1] : key[0];
+    key[0] = asc ? lo : hi;
+    key[1] = asc ? hi : lo;
+  } else {
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      const int i = base + r * 64 + lane;
+      const K o = lane_xor<J>(key[r]);
+      const bool low = ((lane & J) == 0) == ((i & K2) == 0);
+      key[r] = (o < key[r]) == low ? o : key[r];
+    }
+  }
+  if constexpr (J > 1) bitonic_phases<K, K2, J / 2>(key, buf, base, lane, flip);
+}
+template <typename K, int K2 = 2>
+__device__ __forceinline__ void bitonic_2048(K (&key)[2], K *buf, int base, int lane, int &flip) {
+  bitonic_phases<K, K2, K2 / 2>(key, buf, base, lane, flip);
+  if constexpr (K2 < 2048) bitonic_2048<K, K2 * 2>(key, buf, base, lane, flip);
 }
 
 // Stable scatter of a chunk's rows into bin order.
@@ -209,16 +187,20 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(SortArgs a) 
   const SortSide &sd = a.side[blockIdx.y];
   const int chunk = blockIdx.x;
   if (chunk >= sd.chunks) return;
-  __shared__ int key[kChunk];          // bin of the element (kBins: padding)
-  __shared__ int val[kChunk];          // its index inside the chunk
-  __shared__ int start[kBins + 1];     // first sorted position of each bin inside the chunk
-  for (int e = threadIdx.x; e < kChunk; e += kSortThreads) {
-    const int row = chunk * kChunk + e;
-    key[e] = row < sd.n ? top_bits(sd.rmask[row], a.k_vol) : kBins;
-    val[e] = e;
+  __shared__ unsigned buf[2 * kChunk];
+  __shared__ int start[kBins];         // first sorted position of each bin inside the chunk
+  const int lane = threadIdx.x % 64, base = threadIdx.x / 64 * 128;
+  unsigned key[2];                     // bin << 11 | index inside the chunk (all ones: padding)
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const int e = base + r * 64 + lane, row = chunk * kChunk + e;
+    key[r] = row < sd.n ? (unsigned)top_bits(sd.rmask[row], a.k_vol) << 11 | (unsigned)e : ~0u;
   }
+  int flip = 0;
+  bitonic_2048(key, buf, base, lane, flip);
   __syncthreads();
-  bitonic_sort(key, val, kChunk, kSortThreads);
+  buf[base + lane] = key[0];
+  buf[base + 64 + lane] = key[1];
   // rows in smaller bins: exclusive scan of the bin totals (2 per thread; thread, wave, workgroup)
   __shared__ int before_bin[kBins];
   __shared__ int part[kSortThreads / 64];
@@ -233,9 +215,9 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(SortArgs a) 
     int incl = local;
     for (int d = 1; d < 64; d <<= 1) {
       const int up = __shfl_up(incl, d);
-      if ((int)(threadIdx.x % 64) >= d) incl += up;
+      if (lane >= d) incl += up;
     }
-    if (threadIdx.x % 64 == 63) part[threadIdx.x / 64] = incl;
+    if (lane == 63) part[threadIdx.x / 64] = incl;
     __syncthreads();
     int before = incl - local;
     for (int wv = 0; wv < (int)threadIdx.x / 64; ++wv) before += part[wv];
@@ -245,114 +227,84 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(SortArgs a) 
       before += mine[q];
     }
   }
-  for (int e = threadIdx.x; e < kChunk; e += kSortThreads)
-    if (e == 0 || key[e - 1] != key[e]) start[key[e]] = e;
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const int e = base + r * 64 + lane;
+    if (key[r] != ~0u && (e == 0 || buf[e - 1] >> 11 != key[r] >> 11)) start[key[r] >> 11] = e;
+  }
   __syncthreads();
-  for (int e = threadIdx.x; e < kChunk; e += kSortThreads) {
-    const int bin = key[e];
-    if (bin < kBins)
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const int e = base + r * 64 + lane;
+    if (key[r] != ~0u) {
+      const int bin = key[r] >> 11;
       sd.perm_tmp[before_bin[bin] + sd.hist_before[(size_t)chunk * kBins + bin] + (e - start[bin])] =
-          chunk * kChunk + val[e];
+          chunk * kChunk + (int)(key[r] & (kChunk - 1));
+    }
   }
 }
 
-// Full sort by (mask, row) of a window of positions; writes the final order and its inverse.
-// perm_tmp == nullptr: the window starts from the identity order (sides of one window).
+// Full sort by (mask, row) of a window of positions (of masks over more than 32 offsets: by the top
+// 32); writes the final order and its inverse, and what the window's blocks of 64 positions use:
+// block_mask = the OR of their rows' masks, flags[4 + side] += (block, offset) combinations in use,
+// flags[10 + side] += offset bits of all rows.  chunks == 0: the window starts from the identity
+// order (sides of one window).
 __global__ __launch_bounds__(kSortThreads) void sort_window_kernel(SortArgs a) {
   const SortSide &sd = a.side[blockIdx.y];
   const int p0 = blockIdx.x * kWindow;
   if (p0 >= sd.n) return;
-  extern __shared__ unsigned long long win_key[];                    // [kWindow]
-  int *win_val = reinterpret_cast<int *>(win_key + kWindow);        // [kWindow]
-  for (int e = threadIdx.x; e < kWindow; e += kSortThreads) {
-    const int p = p0 + e;
-    const int row = p < sd.n ? (sd.perm_tmp ? sd.perm_tmp[p] : p) : INT32_MAX;
-    win_val[e] = row;
-    win_key[e] = p < sd.n ? sd.rmask[row] : ~0ull;
-  }
-  __syncthreads();
-  bitonic_sort(win_key, win_val, kWindow, kSortThreads);
-  for (int e = threadIdx.x; e < kWindow; e += kSortThreads) {
-    const int p = p0 + e;
+  __shared__ unsigned long long buf[2 * kWindow];
+  __shared__ int sums[kSortThreads / 64][2];
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, base = wave * 128;
+  const int shift = a.k_vol > 32 ? a.k_vol - 32 : 0;
+  unsigned long long key[2];
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const int p = p0 + base + r * 64 + lane;
+    key[r] = ~0ull;
     if (p < sd.n) {
-      sd.perm[p] = win_val[e];
-      sd.inv[win_val[e]] = p;
+      const int row = sd.chunks ? sd.perm_tmp[p] : p;
+      key[r] = (a.by_mask ? (sd.rmask[row] >> shift) << 32 : 0ull) | (unsigned)row;
     }
   }
-}
-
-// Step 3: the neighbour tables by POSITION, straight from the pair lists (tables pre-filled
-// with -1): nbr_out[k][position of o] = i, nbr_in[k][position of i] = o.
-__device__ __forceinline__ void tables_body(const int32_t *__restrict__ kpos, const int32_t *__restrict__ imap,
-                                            const int32_t *__restrict__ omap, int k_vol, int n_pairs, int n_in,
-                                            int n_out, const int32_t *__restrict__ inv_out,
-                                            const int32_t *__restrict__ inv_in, int32_t *__restrict__ nbr_out,
-                                            int32_t *__restrict__ nbr_in, int block) {
-  const int total = kpos[k_vol];
-  const int j = kpos[0] + block * blockDim.x + threadIdx.x;
-  if (j >= total || j >= n_pairs) return;
-  int lo = 0, hi = k_vol;
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (kpos[mid] <= j) lo = mid; else hi = mid;
-  }
-  const int i = imap[j], o = omap[j];
-  if (i < 0 || i >= n_in || o < 0 || o >= n_out) return;
-  nbr_out[(size_t)lo * n_out + (inv_out ? inv_out[o] : o)] = i;
-  nbr_in[(size_t)lo * n_in + (inv_in ? inv_in[i] : i)] = o;
-}
-
-// Step 4: which offsets occur in every block of 64 positions (the OR of its rows' masks), and
-// how many (block, offset) combinations that makes in total (flags[4 + side]).
-struct MaskSide {
-  const unsigned long long *rmask;
-  const int32_t *perm;             // nullptr: identity
-  unsigned long long *block_mask;
-  int n;
-};
-struct MaskArgs {
-  MaskSide side[2];
-  int *flags;
-};
-__global__ __launch_bounds__(1024) void block_masks_kernel(MaskArgs a) {
-  const MaskSide &sd = a.side[blockIdx.y];
-  __shared__ int partial[16];
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-  const int block = blockIdx.x * 16 + wave;
-  const int p = block * 64 + lane;
-  __shared__ int partial_rows[16];
+  int flip = 0;
+  bitonic_2048(key, buf, base, lane, flip);
   int bits = 0, row_bits = 0;
-  if (block * 64 < sd.n) {
-    unsigned long long m = p < sd.n ? sd.rmask[sd.perm ? sd.perm[p] : p] : 0ull;
-    row_bits = __popcll(m);
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const int p = p0 + base + r * 64 + lane;
+    unsigned long long m = 0;
+    if (p < sd.n) {
+      const int row = (int)(unsigned)key[r];
+      sd.perm[p] = row;
+      sd.inv[row] = p;
+      m = a.by_mask && shift == 0 ? key[r] >> 32 : sd.rmask[row];
+    }
+    int rb = __popcll(m);
     for (int d = 32; d > 0; d >>= 1) {
       m |= __shfl_xor(m, d);
-      row_bits += __shfl_xor(row_bits, d);
+      rb += __shfl_xor(rb, d);
     }
-    if (lane == 0) sd.block_mask[block] = m;
-    bits = __popcll(m);
+    if (p0 + base + r * 64 < sd.n) {
+      const int block = (p0 + base) / 64 + r;
+      if (lane == 0) {
+        sd.block_mask[block] = m;
+        if (sd.mirror_mask) sd.mirror_mask[block] = __brevll(m) >> (64 - a.k_vol);
+      }
+      bits += __popcll(m);
+      row_bits += rb;
+    }
   }
   if (lane == 0) {
-    partial[wave] = bits;
-    partial_rows[wave] = row_bits;
+    sums[wave][0] = bits;
+    sums[wave][1] = row_bits;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int sum = 0, rows = 0;
-    for (int i = 0; i < 16; ++i) {
-      sum += partial[i];
-      rows += partial_rows[i];
-    }
-    if (sum) atomicAdd(&a.flags[4 + blockIdx.y], sum);
-    if (rows) atomicAdd(&a.flags[10 + blockIdx.y], rows);
+  if (threadIdx.x < 2) {
+    int sum = 0;
+    for (int i = 0; i < kSortThreads / 64; ++i) sum += sums[i][threadIdx.x];
+    if (sum) atomicAdd(&a.flags[(threadIdx.x ? 10 : 4) + blockIdx.y], sum);
   }
-}
-
-__global__ void tables_kernel(const int32_t *__restrict__ kpos, const int32_t *__restrict__ imap,
-                              const int32_t *__restrict__ omap, int k_vol, int n_pairs, int n_in, int n_out,
-                              const int32_t *__restrict__ inv_out, const int32_t *__restrict__ inv_in,
-                              int32_t *__restrict__ nbr_out, int32_t *__restrict__ nbr_in) {
-  tables_body(kpos, imap, omap, k_vol, n_pairs, n_in, n_out, inv_out, inv_in, nbr_out, nbr_in, blockIdx.x);
 }
 
 // Pair view: the pair lists with every offset's run padded to a multiple of 64 rows
@@ -391,27 +343,6 @@ __global__ void pair_view_kernel(const int32_t *__restrict__ kpos, const int32_t
   if ((r & 63) == 0) pv_mask[r >> 6] = 1ull << lo;
 }
 
-// band_start[k][c] = number of pairs of offset k whose output row is below
-// c * band_rows (a lower bound over the offset's pairs, which are ordered by
-// output row when the result is used); c = band_count gives the offset's size.
-__global__ void band_bounds_kernel(const int32_t *__restrict__ kpos, const int32_t *__restrict__ omap,
-                                   int n_pairs, int band_count, int band_rows,
-                                   int32_t *__restrict__ band_start) {
-  const int k = blockIdx.x;
-  const int first = min(max(kpos[k], 0), n_pairs);
-  const int count = min(max(kpos[k + 1], first), n_pairs) - first;   // never reads past the map
-  for (int c = threadIdx.x; c <= band_count; c += blockDim.x) {
-    int lo = 0, hi = count;              // first pair with omap >= c * band_rows
-    if (c == band_count) lo = count;
-    const long long target = (long long)c * band_rows;
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (omap[first + mid] < target) lo = mid + 1; else hi = mid;
-    }
-    band_start[k * (band_count + 1) + c] = lo;
-  }
-}
-
 // Dispatch order of the 256-position tiles of the output-stationary kernel.
 // Workgroup b runs on XCD b % 8 and, inside an XCD, workgroup number q = b / 8
 // lands on CU q % cus_per_xcd (the dispatcher goes round the CUs).
@@ -427,40 +358,25 @@ __global__ void band_bounds_kernel(const int32_t *__restrict__ kpos, const int32
 //    overfull XCD go to the XCDs that have room.
 // order[q * 8 + xcd] = tile | first offset << 24, -1 where no tile lands.  One workgroup; which of two
 // equally heavy tiles comes first depends on timing, the results do not.
-struct TileSide {
-  const int32_t *perm;
-  const unsigned long long *block_masks;
-  int32_t *order;
-  int n_rows, n_tiles, cap;
-};
-struct TileArgs {
-  TileSide side[2];
-  int cus_per_xcd;
-  const int *flags;   // the build's findings and where they go on the host (this is the
-  int *host;          // build's last launch); nullptr: published by a launch of its own
-};
-__global__ __launch_bounds__(1024) void tile_order_kernel(TileArgs ta) {
-  const int32_t *__restrict__ perm = ta.side[blockIdx.x].perm;
-  const unsigned long long *__restrict__ block_masks = ta.side[blockIdx.x].block_masks;
-  int32_t *__restrict__ order = ta.side[blockIdx.x].order;
-  const int n_rows = ta.side[blockIdx.x].n_rows, n_tiles = ta.side[blockIdx.x].n_tiles;
-  const int cap = ta.side[blockIdx.x].cap, cus_per_xcd = ta.cus_per_xcd;
-  if (blockIdx.x == 0 && ta.host && threadIdx.x < kPlanFlags) ta.host[threadIdx.x] = ta.flags[threadIdx.x];
+__device__ __forceinline__ void tile_order_body(const TileSide &sd, int cus_per_xcd, int32_t *__restrict__ spill) {
+  const int32_t *__restrict__ perm = sd.perm;
+  const unsigned long long *__restrict__ block_masks = sd.block_masks;
+  int32_t *__restrict__ order = sd.order;
+  const int n_rows = sd.n_rows, n_tiles = sd.n_tiles, cap = sd.cap;
   if (!order) return;
   constexpr int kPc = 65;                         // popcount classes 0..64
   __shared__ int hist[8][kPc];                    // tiles per (home, popcount), then start ranks
   __shared__ int cursor[8][kPc];
   __shared__ int total[8];
   __shared__ int spill_count;
-  extern __shared__ int32_t spill[];              // [n_tiles]
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, threads = blockDim.x;     // (spill: n_tiles ints of LDS)
   const int n_blocks = (n_rows + 63) / 64;
-  for (int i = tid; i < 8 * kPc; i += 1024) {
+  for (int i = tid; i < 8 * kPc; i += threads) {
     (&hist[0][0])[i] = 0;
     (&cursor[0][0])[i] = 0;
   }
   if (tid == 0) spill_count = 0;
-  for (int i = tid; i < cap * 8; i += 1024) order[i] = -1;     // (slots no tile lands in)
+  for (int i = tid; i < cap * 8; i += threads) order[i] = -1;     // (slots no tile lands in)
   __syncthreads();
   // entry of tile t in the table: t in the low 24 bits, the first offset the tile uses above
   // them (the kernel starts that offset's index load before it has seen the tile's masks)
@@ -472,7 +388,7 @@ __global__ __launch_bounds__(1024) void tile_order_kernel(TileArgs ta) {
     pc = __builtin_popcountll(m);
     entry = t | ((m ? __builtin_ctzll(m) : 0) << 24);
   };
-  for (int t = tid; t < n_tiles; t += 1024) {
+  for (int t = tid; t < n_tiles; t += threads) {
     int home, pc, entry;
     classify(t, home, pc, entry);
     atomicAdd(&hist[home][pc], 1);
@@ -493,7 +409,7 @@ __global__ __launch_bounds__(1024) void tile_order_kernel(TileArgs ta) {
     const int in_round = min(cus_per_xcd, cap - round * cus_per_xcd);
     return round * cus_per_xcd + ((round & 1) ? in_round - 1 - j : j);
   };
-  for (int t = tid; t < n_tiles; t += 1024) {
+  for (int t = tid; t < n_tiles; t += threads) {
     int home, pc, entry;
     classify(t, home, pc, entry);
     const int rank = hist[home][pc] + atomicAdd(&cursor[home][pc], 1);
@@ -501,7 +417,7 @@ __global__ __launch_bounds__(1024) void tile_order_kernel(TileArgs ta) {
     else spill[atomicAdd(&spill_count, 1)] = entry;
   }
   __syncthreads();
-  for (int sidx = tid; sidx < spill_count; sidx += 1024) {
+  for (int sidx = tid; sidx < spill_count; sidx += threads) {
     int left = sidx;
     for (int q = 0; q < 8; ++q) {
       const int filled = min(total[q], cap), room = cap - filled;
@@ -514,64 +430,114 @@ __global__ __launch_bounds__(1024) void tile_order_kernel(TileArgs ta) {
   }
 }
 
-// Dispatch order of the weight gradient's (offset, band) cells, one table per group
-// size g in {1, 2, 4, 8} (blockIdx.z): cells[q * 8 + xcd] is the q-th cell of XCD
-// xcd, cell = offset * 65536 + band.  XCD x owns the bands x, x + 8, ...; they are
-// taken g at a time (g bands x all offsets are in flight together, so g is chosen
-// at launch such that their rows fit the XCD's L2), and inside a group the cells
+// Row bands of the weight gradient and the dispatch order of its (offset, band) cells.
+// band_start[k][c] = number of pairs of offset k whose output row is below c * band_rows (a lower
+// bound over the offset's pairs, which are ordered by output row when the result is used);
+// c = bands gives the offset's size.  Cell orders: one table per group size g in {1, 2, 4, 8}:
+// cells[q * 8 + xcd] is the q-th cell of XCD xcd, cell = offset * 65536 + band.  XCD x owns the
+// bands x, x + 8, ...; they are taken g at a time (g bands x all offsets are in flight together, so
+// g is chosen at launch such that their rows fit the XCD's L2), and inside a group the cells
 // are ranked by pair count, most first (the longest workgroups start first), ties
-// by cell number.  One thread per cell; a cell's rank is found by comparing with
-// the other cells of its XCD (a few hundred).
-__global__ void band_cells_kernel(const int32_t *__restrict__ band_start, int k_vol, int bands,
-                                  int32_t *__restrict__ cells) {
-  // the pair counts of the XCD's cells (and which of its bands a cell lies in) go to LDS
-  // once: every thread compares with all of them, and the integer divisions of the cell
-  // arithmetic would otherwise dominate the loop
-  constexpr int kCached = 2048;
-  __shared__ int count[kCached];
-  __shared__ short band_of[kCached];
+// by cell number.  Workgroup (x, shift) ranks XCD x's cells in groups of 1 << shift bands by
+// comparing each with the others (a few hundred); it finds their bounds itself, so that bands and
+// order need one launch, and the one with shift 0 writes the bounds down.
+__device__ __forceinline__ void bands_body(const TablesArgs &a, int x, int shift, int32_t *__restrict__ lds) {
+  const int k_vol = a.k_vol, bands = a.bands;
   const int per_xcd = (bands / 8) * k_vol;
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;   // cell number inside its XCD: (band / 8) * k_vol + k
-  const int x = blockIdx.y, shift = blockIdx.z;           // groups of 1 << shift bands
-  auto pairs_of = [&](int cell) {
-    const int k = cell % k_vol, band = (cell / k_vol) * 8 + x;
-    return band_start[k * (bands + 1) + band + 1] - band_start[k * (bands + 1) + band];
+  int *count = lds;                       // [per_xcd]
+  int *group = lds + per_xcd;             // [per_xcd]
+  auto below = [&](int first, int n, long long target) {      // first pair with omap >= target
+    int lo = 0, hi = n;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (a.omap[first + mid] < target) lo = mid + 1; else hi = mid;
+    }
+    return lo;
   };
-  for (int o = threadIdx.x; o < per_xcd && o < kCached; o += blockDim.x) {
-    count[o] = pairs_of(o);
-    band_of[o] = (short)(o / k_vol);
+  for (int o = threadIdx.x; o < per_xcd; o += blockDim.x) {     // cell number inside the XCD: (band / 8) * k_vol + k
+    const int k = o % k_vol, q = o / k_vol, band = q * 8 + x;
+    const int first = min(max(a.kpos[k], 0), a.n_pairs);
+    const int n = min(max(a.kpos[k + 1], first), a.n_pairs) - first;   // never reads past the map
+    const int b0 = below(first, n, (long long)band * a.band_rows);
+    const int b1 = band + 1 == bands ? n : below(first, n, (long long)(band + 1) * a.band_rows);
+    count[o] = b1 - b0;
+    group[o] = q >> shift;
+    if (shift == 0) {
+      a.band_start[k * (bands + 1) + band] = b0;
+      if (band + 1 == bands) a.band_start[k * (bands + 1) + bands] = n;
+    }
   }
   __syncthreads();
-  if (c >= per_xcd) return;
-  const int mine = pairs_of(c), my_group = (c / k_vol) >> shift;
-  int rank = 0;
+  for (int c = threadIdx.x; c < per_xcd; c += blockDim.x) {
+    const int mine = count[c], my_group = group[c];
+    int rank = 0;
 #pragma unroll 8      // (independent LDS reads in flight: the loop is bound by their latency)
-  for (int o = 0; o < per_xcd; ++o) {
-    const bool cached = o < kCached;
-    const int theirs = cached ? count[o] : pairs_of(o);
-    const int their_group = (cached ? (int)band_of[o] : o / k_vol) >> shift;
-    const bool before = their_group != my_group ? their_group < my_group
-                                                 : (theirs > mine || (theirs == mine && o < c));
-    rank += before ? 1 : 0;
+    for (int o = 0; o < per_xcd; ++o) {
+      const int theirs = count[o], their_group = group[o];
+      const bool before = their_group != my_group ? their_group < my_group
+                                                   : (theirs > mine || (theirs == mine && o < c));
+      rank += before ? 1 : 0;
+    }
+    a.band_cells[(size_t)shift * bands * k_vol + rank * 8 + x] = (c % k_vol) * 65536 + (c / k_vol) * 8 + x;
   }
-  cells[(size_t)blockIdx.z * bands * k_vol + rank * 8 + x] = (c % k_vol) * 65536 + (c / k_vol) * 8 + x;
 }
 
-// The two directions of a plan (output side, input side) are chains of a dozen small
-// launches each (masks, radix sort, permutation, block masks, tile order) that do not
-// depend on each other; at 200 k rows every launch is bound by its latency, so the input
-// side's chain runs on a stream of the library's own (default priority, one per device,
-// created on first use) next to the caller's.  nullptr: creation failed, one stream is used.
-hipStream_t side_stream(int device) {
-  static std::mutex m;
-  static std::map<int, hipStream_t> streams;
-  std::lock_guard<std::mutex> lock(m);
-  auto it = streams.find(device);
-  if (it != streams.end()) return it->second;
-  hipStream_t st = nullptr;
-  if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess) st = nullptr;
-  streams[device] = st;
-  return st;
+// The last launch of a build.  Step 3, the neighbour tables by POSITION: nbr_out[k][position of o] =
+// i, nbr_in[k][position of i] = o -- scattered from the pair lists (tables pre-filled with -1), or,
+// where the map builder left a table of the output rows, the output side's read from there in
+// position order (whole lines both ways: no pre-fill, no scattered 4-byte stores).  Next to it, as
+// workgroups of the same launch: tile orders, row bands, the fingerprint of the lists, the findings'
+// way to the host.  (Five launches of 3-12 us each and a second stream before.)
+__global__ __launch_bounds__(256) void tables_kernel(TablesArgs a) {
+  extern __shared__ int32_t lds[];
+  int b = blockIdx.x;
+  if (b < a.tile_blocks) {
+    if (b == 0 && threadIdx.x < kPlanFlags) {
+      const int q = threadIdx.x;
+      // (mirrored maps: one side's counts stand for both)
+      const int v = a.flags[a.mirror && (q == 5 || q == 11) ? q - 1 : q];
+      if (a.host && (q < kFlagPrint)) a.host[q] = v;
+    }
+    if (b < 2) tile_order_body(a.tile[b], a.cus_per_xcd, lds);
+    return;
+  }
+  b -= a.tile_blocks;
+  if (b < a.band_blocks) {
+    bands_body(a, b % 8, b / 8, lds);
+    return;
+  }
+  b -= a.band_blocks;
+  if (b < a.print_blocks) {
+    plan_print_block(a.kpos, a.imap, a.omap, a.k_vol, a.n_pairs, a.flags, b);
+    return;
+  }
+  b -= a.print_blocks;
+  if (b < a.row_blocks) {
+    const int p = b * 256 + threadIdx.x;
+    if (p >= a.n_out) return;
+    typedef int int4v_ __attribute__((ext_vector_type(4)));
+    const int4v_ *row = reinterpret_cast<const int4v_ *>(a.rows + (size_t)a.perm_out[p] * a.row_ld);
+    for (int k0 = 0; k0 < a.k_vol; k0 += 4) {
+      const int4v_ v = row[k0 / 4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (k0 + e < a.k_vol) a.nbr_out[(size_t)(k0 + e) * a.n_out + p] = v[e];
+    }
+    return;
+  }
+  b -= a.row_blocks;
+  const int total = a.kpos[a.k_vol];
+  const int j = a.kpos[0] + b * 256 + threadIdx.x;
+  if (j >= total || j >= a.n_pairs) return;
+  int lo = 0, hi = a.k_vol;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (a.kpos[mid] <= j) lo = mid; else hi = mid;
+  }
+  const int i = a.imap[j], o = a.omap[j];
+  if (i < 0 || i >= a.n_in || o < 0 || o >= a.n_out) return;
+  if (a.inv_out) a.nbr_out[(size_t)lo * a.n_out + a.inv_out[o]] = i;
+  if (a.inv_in) a.nbr_in[(size_t)lo * a.n_in + a.inv_in[i]] = o;
 }
 
 // Pinned blocks for the builds' flag read-backs (hipHostMalloc costs as much as the whole
@@ -609,25 +575,6 @@ __global__ __launch_bounds__(256) void plan_check_kernel(const int32_t *__restri
   plan_check_block(kpos, imap, omap, k_vol, n_pairs, flags, host, blockIdx.x);
 }
 
-// The build's findings -> pinned host memory (mapped into the device's address space).
-__global__ void publish_flags_kernel(const int *__restrict__ flags, int *__restrict__ host) {
-  if (threadIdx.x < kPlanFlags) host[threadIdx.x] = flags[threadIdx.x];
-}
-
-int fill_i32(int32_t *p, size_t n, int32_t v, hipStream_t s) {
-  if (n == 0) return FGMS_OK;
-  if (reinterpret_cast<uintptr_t>(p) % 16) {
-    set_error("fill_i32: unaligned block");
-    return FGMS_E_INVALID;
-  }
-  size_t blocks = (n / 4 + 255) / 256;          // one 16-byte store per thread, a few for big blocks
-  if (blocks > 8192) blocks = 8192;
-  if (blocks == 0) blocks = 1;
-  fill_i32_kernel<<<(unsigned)blocks, 256, 0, s>>>(p, n, v);
-  FGMS_HIP_TRY(hipGetLastError());
-  return FGMS_OK;
-}
-
 }  // namespace
 }  // namespace fgms
 
@@ -635,10 +582,146 @@ using namespace fgms;
 
 namespace fgms {
 
-// Builds a plan.  Everything is queued on `stream` (the weight gradient's band tables and the
-// table pre-fill on a stream of the library's own next to it); nothing waits for the GPU.  What
+int launch_fills(const FillBatch &batch, hipStream_t s) {
+  size_t most = 0;
+  for (int r = 0; r < batch.count; ++r)
+    if (batch.range[r].n > most) most = batch.range[r].n;
+  if (most == 0) return FGMS_OK;
+  size_t blocks = (most / 4 + 255) / 256;          // one 16-byte store per thread, a few for big blocks
+  if (blocks > 4096) blocks = 4096;
+  fills_kernel<<<(unsigned)(blocks ? blocks : 1), 256, 0, s>>>(batch);
+  FGMS_HIP_TRY(hipGetLastError());
+  return FGMS_OK;
+}
+
+void sort_side_layout(SortSide &sd, int64_t n, Arena &tmp) {
+  sd.n = (int)n;
+  sd.chunks = n > kWindow ? (int)((n + kChunk - 1) / kChunk) : 0;      // one window: no counting sort
+  tmp.take(sd.inv, (size_t)n);
+  if (sd.chunks) {
+    tmp.take(sd.perm_tmp, (size_t)n);
+    tmp.take(sd.hist, (size_t)kBins * sd.chunks);
+    tmp.take(sd.hist_before, (size_t)kBins * sd.chunks);
+    tmp.take(sd.bin_start, (size_t)kBins);
+  }
+}
+
+int launch_sort(const SortArgs &args, bool hist_done, hipStream_t s) {
+  // FGMS_PLAN_SORT=0 keeps the rows in their natural order (for comparison).
+  static const bool sort_rows = !(getenv("FGMS_PLAN_SORT") && atoi(getenv("FGMS_PLAN_SORT")) == 0);
+  SortArgs a = args;
+  a.by_mask = sort_rows;
+  if (!sort_rows) a.side[0].chunks = a.side[1].chunks = 0;
+  const int most = a.side[0].n > a.side[1].n ? a.side[0].n : a.side[1].n;
+  const int chunks = a.side[0].chunks > a.side[1].chunks ? a.side[0].chunks : a.side[1].chunks;
+  const unsigned sides = a.side[1].n > 0 ? 2 : 1;
+  if (chunks) {
+    if (!hist_done) sort_hist_kernel<<<dim3((unsigned)chunks, sides), kSortThreads, 0, s>>>(a);
+    sort_scan_kernel<<<dim3(kBins / kScanBins, sides), 256, 0, s>>>(a);
+    sort_scatter_kernel<<<dim3((unsigned)chunks, sides), kSortThreads, 0, s>>>(a);
+  }
+  if (most) sort_window_kernel<<<dim3((unsigned)((most + kWindow - 1) / kWindow), sides), kSortThreads, 0, s>>>(a);
+  FGMS_HIP_TRY(hipGetLastError());
+  return FGMS_OK;
+}
+
+int launch_tables(TablesArgs a, hipStream_t s) {
+  const int tiles = a.tile[0].n_tiles > a.tile[1].n_tiles ? a.tile[0].n_tiles : a.tile[1].n_tiles;
+  size_t lds = (size_t)tiles * sizeof(int32_t);
+  a.tile_blocks = 8;                               // (two at work; the parts behind start on a multiple of eight)
+  a.band_blocks = 0;
+  if (a.band_start) {
+    const size_t need = (size_t)2 * (a.bands / 8) * a.k_vol * sizeof(int32_t);
+    if (need > lds) lds = need;
+    a.band_blocks = 32;
+  }
+  a.print_blocks = a.take_print ? kPrintParts : 0;
+  a.row_blocks = a.rows ? (a.n_out + 255) / 256 : 0;
+  a.pair_blocks = a.inv_out || a.inv_in ? (a.n_pairs + 255) / 256 : 0;
+  a.cus_per_xcd = num_cus() >= 8 ? num_cus() / 8 : 1;
+  if (lds > 48 * 1024) {
+    const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(tables_kernel), lds);
+    if (rc != FGMS_OK) return rc;
+  }
+  tables_kernel<<<(unsigned)(a.tile_blocks + a.band_blocks + a.print_blocks + a.row_blocks + a.pair_blocks), 256, lds, s>>>(a);
+  FGMS_HIP_TRY(hipGetLastError());
+  return FGMS_OK;
+}
+
+Plan *plan_alloc(int k_vol, int64_t n_in, int64_t n_out, int64_t n_pairs, hipStream_t s) {
+  Plan *p = new Plan();          // (value-initialised: every field starts out zero)
+  p->k_vol = k_vol; p->n_in = n_in; p->n_out = n_out; p->n_pairs = n_pairs;
+  p->last_stream = s;
+  p->create_stream = s;
+  p->nbr_stride_out = (int)n_out;
+  p->nbr_stride_in = (int)n_in;
+  if (hipGetDevice(&p->device) == hipSuccess && (p->host_flags = pinned_flags_get()) &&
+      (p->ready = event_get(p->device))) {
+    p->host_flags[kFlagStale] = 0;     // (a recycled block: the flag is read before the build has run)
+    return p;
+  }
+  set_error("plan: pinned flag block / event creation failed");
+  fgms_plan_destroy((fgms_plan_t *)p);
+  return nullptr;
+}
+
+// Weight-gradient row bands: 8, 16, 32 or 64 (the XCDs take them in groups of 1, 2, 4 or 8;
+// other counts measured worse), the fewest that leave an (offset, band) cell at most ~1 900
+// pairs -- a workgroup's fixed costs (first loads, the four waves' partial tiles summed through
+// LDS, 16 KB of atomic updates) are those of ~600 pairs, and with bigger cells the chip waits
+// for the last ones -- then more while the cells are fewer than 1.5 per CU and keep ~400 pairs.
+// 64 -> 64 fp16 backward launch with 64 bands throughout / with this rule: 50 k voxels 35.5 /
+// 29.8 us, 80 k 55.6 / 45.2, 100 k 59.1 / 46.2, 120 k 61.5 / 55.6, 140 k 67.7 / 65.3 (32 bands
+// each), 170 k and 200 k voxels 64 bands either way.
+void plan_bands(Plan *p) {
+  constexpr int kMaxBands = 64;
+  int bands = 8;
+  while (bands < kMaxBands && p->n_pairs / ((int64_t)p->k_vol * bands) > 1900) bands *= 2;
+  while (bands < kMaxBands && (int64_t)bands * p->k_vol * 2 < 3 * (int64_t)num_cus() &&
+         p->n_pairs / ((int64_t)p->k_vol * bands * 2) >= 384)
+    bands *= 2;
+  p->band_count = bands;
+  p->band_rows = (int)((p->n_out + bands - 1) / bands);
+}
+
+// Tile -> XCD homes pay off once every XCD has a few dozen tiles of its own.
+int tile_table(int64_t n, int *cap) {
+  static const bool xcd_homes = !(getenv("FGMS_XCD_HOME") && atoi(getenv("FGMS_XCD_HOME")) == 0);
+  const int64_t n_tiles = (n + 255) / 256;
+  *cap = (int)((n_tiles + 7) / 8);
+  return xcd_homes && n_tiles >= 256 && n_tiles * sizeof(int32_t) <= 60000 ? (int)n_tiles : 0;
+}
+
+void plan_fill_tables_args(const Plan *p, TablesArgs *t) {
+  t->kpos = p->kpos; t->imap = p->in_map; t->omap = p->out_map;
+  t->k_vol = p->k_vol; t->n_pairs = (int)p->n_pairs; t->n_in = (int)p->n_in; t->n_out = (int)p->n_out;
+  t->band_start = p->band_start; t->band_cells = p->band_cells;
+  t->bands = p->band_count;
+  t->band_rows = p->band_rows > 0 ? p->band_rows : 1;
+  for (int d = 0; d < 2; ++d) {
+    int32_t *order = d ? p->tile_in : p->tile_out;
+    if (!order) continue;
+    int cap;
+    const int64_t n = d ? p->n_in : p->n_out;
+    const int n_tiles = tile_table(n, &cap);
+    t->tile[d] = TileSide{d ? p->perm_in : p->perm_out, d ? p->mask_in : p->mask_out, order, (int)n, n_tiles, cap};
+  }
+  t->flags = p->flags;
+  if (hipHostGetDevicePointer((void **)&t->host, p->host_flags, 0) != hipSuccess) t->host = nullptr;
+}
+
+int plan_publish(Plan *p, bool written, hipStream_t s) {
+  if ((!written && hipMemcpyAsync(p->host_flags, p->flags, kPlanFlags * sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess) ||
+      hipEventRecord(p->ready, s) != hipSuccess) {
+    set_error("plan: queuing the flag read-back failed");
+    return FGMS_E_HIP;
+  }
+  return FGMS_OK;
+}
+
+// Builds a plan.  Everything is queued on `stream`; nothing waits for the GPU.  What
 // the build finds out about the map (index out of range, rows shared inside an offset, pair
-// order, block counts) travels to pinned host memory behind the last kernel and is read by
+// order, block counts) travels to pinned host memory with the last kernel and is read by
 // plan_resolve when the plan is first used.
 int plan_create(fgms_plan_t **plan_out, const int32_t *kpos, const int32_t *in_map,
                 const int32_t *out_map, int64_t n_in, int64_t n_out, int k_vol, int64_t n_pairs, void *stream,
@@ -662,240 +745,83 @@ int plan_create(fgms_plan_t **plan_out, const int32_t *kpos, const int32_t *in_m
       return FGMS_E_INVALID;
     }
   }
-  Plan *p = new Plan();          // (value-initialised: every field starts out zero)
-  p->k_vol = k_vol; p->n_in = n_in; p->n_out = n_out; p->n_pairs = n_pairs;
-  p->last_stream = s;
-  p->create_stream = s;
+  Plan *p = plan_alloc(k_vol, n_in, n_out, n_pairs, s);
+  if (!p) return FGMS_E_NOMEM;
   p->kpos = kpos; p->in_map = in_map; p->out_map = out_map;
+  plan_bands(p);
+  const bool tables = k_vol <= 64;      // (64-bit offset masks; beyond that the plan is bands only)
+  if (k_vol > 1500) want_bands = false;   // (the cell orders are ranked in LDS)
+  p->has_tables = tables;
+  p->has_bands = want_bands;
+  const size_t so = tables ? (size_t)n_out * k_vol : 0, si = tables ? (size_t)n_in * k_vol : 0;
+  const size_t bo = (size_t)(n_out + 63) / 64, bi = (size_t)(n_in + 63) / 64;
+  SortArgs sa{};
+  sa.k_vol = k_vol;
+  unsigned long long *rmask = nullptr;          // [n_out] then [n_in]
+  int cap_out = 0, cap_in = 0;
+  const int tiles_out = tables ? tile_table(n_out, &cap_out) : 0, tiles_in = tables ? tile_table(n_in, &cap_in) : 0;
+  void *scratch = nullptr;
+  auto layout = [&](Arena &keep, Arena &tmp) {
+    keep.take(p->flags, kPlanFlags);
+    if (want_bands) {
+      keep.take(p->band_start, (size_t)k_vol * (p->band_count + 1));
+      keep.take(p->band_cells, (size_t)4 * k_vol * p->band_count);
+    }
+    if (!tables) return;
+    keep.take(p->nbr_out, so + si);             // (nbr_in right behind: one fill)
+    keep.take(p->mask_out, bo);
+    keep.take(p->mask_in, bi);
+    keep.take(p->perm_out, (size_t)n_out);
+    keep.take(p->perm_in, (size_t)n_in);
+    if (tiles_out) keep.take(p->tile_out, (size_t)cap_out * 8);
+    if (tiles_in) keep.take(p->tile_in, (size_t)cap_in * 8);
+    tmp.take(rmask, (size_t)(n_out + n_in));
+    sort_side_layout(sa.side[0], n_out, tmp);
+    sort_side_layout(sa.side[1], n_in, tmp);
+  };
   int rc = FGMS_OK;
-  std::vector<void *> tmp;          // temporaries: handed back to the pool behind the last kernel
-  hipStream_t side_in_use = nullptr;     // the library's own stream, once work of this build is queued on it
   auto fail = [&](int code) {
-    // (blocks are handed back behind `s` alone: the side stream's work must have finished)
-    if (side_in_use) (void)hipStreamSynchronize(side_in_use);
-    for (void *q : tmp) pool_free(q, s, false);
+    if (scratch) pool_free(scratch, s, false);
     fgms_plan_destroy((fgms_plan_t *)p);
     return code;
   };
-  auto take = [&](void **q, size_t bytes, bool temporary) {
-    if (pool_alloc(q, bytes ? bytes : 256, s) != FGMS_OK) return false;
-    if (temporary) tmp.push_back(*q);
-    return true;
-  };
-  if (hipGetDevice(&p->device) != hipSuccess) return fail(FGMS_E_HIP);
-  if ((p->host_flags = pinned_flags_get())) p->host_flags[kFlagStale] = 0;     // (a recycled block: the flag is read before the build has run)
-  if (!p->host_flags ||
-      hipEventCreateWithFlags(&p->ready, hipEventDisableTiming) != hipSuccess) {
-    set_error("fgms_plan_create: pinned flag block / event creation failed");
-    return fail(FGMS_E_NOMEM);
-  }
-  // weight-gradient row bands: 8, 16, 32 or 64 (the XCDs take them in groups of 1, 2, 4 or 8;
-  // other counts measured worse), the fewest that leave an (offset, band) cell at most ~1 900
-  // pairs -- a workgroup's fixed costs (first loads, the four waves' partial tiles summed through
-  // LDS, 16 KB of atomic updates) are those of ~600 pairs, and with bigger cells the chip waits
-  // for the last ones -- then more while the cells are fewer than 1.5 per CU and keep ~400 pairs.
-  // 64 -> 64 fp16 backward launch with 64 bands throughout / with this rule: 50 k voxels 35.5 /
-  // 29.8 us, 80 k 55.6 / 45.2, 100 k 59.1 / 46.2, 120 k 61.5 / 55.6, 140 k 67.7 / 65.3 (32 bands
-  // each), 170 k and 200 k voxels 64 bands either way.
   {
-    constexpr int kMaxBands = 64;
-    int bands = 8;
-    while (bands < kMaxBands && n_pairs / ((int64_t)k_vol * bands) > 1900) bands *= 2;
-    while (bands < kMaxBands && (int64_t)bands * k_vol * 2 < 3 * (int64_t)num_cus() &&
-           n_pairs / ((int64_t)k_vol * bands * 2) >= 384)
-      bands *= 2;
-    p->band_count = bands;
-  }
-  const int band_rows = (int)((n_out + p->band_count - 1) / p->band_count);
-  p->band_rows = band_rows;
-  const bool tables = k_vol <= 64;      // (64-bit offset masks; beyond that the plan is bands only)
-  const size_t so = tables ? (size_t)n_out * k_vol : 0, si = tables ? (size_t)n_in * k_vol : 0;
-  const size_t bo = (size_t)(n_out + 63) / 64, bi = (size_t)(n_in + 63) / 64;
-  unsigned long long *rmask = nullptr;          // [n_out] then [n_in]
-  if ((want_bands && (!take((void **)&p->band_start, (size_t)k_vol * (p->band_count + 1) * sizeof(int32_t), false) ||
-                      !take((void **)&p->band_cells, (size_t)4 * k_vol * p->band_count * sizeof(int32_t), false))) ||
-      !take((void **)&p->flags, kPlanFlags * sizeof(int), false) ||
-      (tables && (!take((void **)&p->nbr_out, (so + si) * sizeof(int32_t), false) ||
-                  !take((void **)&p->mask_out, (bo + bi) * sizeof(unsigned long long), false) ||
-                  !take((void **)&rmask, (size_t)(n_out + n_in) * sizeof(unsigned long long), true)))) {
-    set_error("fgms_plan_create: table allocation failed");
-    return fail(FGMS_E_NOMEM);
+    Arena keep, tmp;
+    layout(keep, tmp);
+    if ((rc = pool_alloc(&p->block, keep.used, s)) || (tmp.used && (rc = pool_alloc(&scratch, tmp.used, s)))) return fail(rc);
+    Arena keep_at, tmp_at;
+    keep_at.base = (char *)p->block;
+    tmp_at.base = (char *)scratch;
+    layout(keep_at, tmp_at);
   }
   if (tables) {
     p->nbr_in = p->nbr_out + so;
-    p->mask_in = p->mask_out + bo;
+    p->tile_grid_out = p->tile_out ? cap_out * 8 : 0;
+    p->tile_grid_in = p->tile_in ? cap_in * 8 : 0;
+    sa.flags = p->flags;
+    sa.side[0].rmask = rmask; sa.side[0].perm = p->perm_out; sa.side[0].block_mask = p->mask_out;
+    sa.side[1].rmask = rmask + n_out; sa.side[1].perm = p->perm_in; sa.side[1].block_mask = p->mask_in;
   }
-  unsigned long long *rmask_out = rmask, *rmask_in = rmask ? rmask + n_out : nullptr;
-  // (the flags are cleared together with the row masks below; without tables, here)
-  if (!tables && (rc = fill_i32(p->flags, kPlanFlags, 0, s))) return fail(rc);
-  p->has_tables = tables;
-  p->has_bands = want_bands;
-
-  // fork: the band tables and the pre-fill of the neighbour tables do not depend on the rest
-  static const bool two_streams = !(getenv("FGMS_PLAN_STREAMS") && atoi(getenv("FGMS_PLAN_STREAMS")) == 1);
-  hipStream_t s2 = two_streams ? side_stream(p->device) : nullptr;
-  hipEvent_t forked = nullptr, joined = nullptr;
-  if (s2) {
-    if (hipEventCreateWithFlags(&forked, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&joined, hipEventDisableTiming) != hipSuccess ||
-        hipEventRecord(forked, s) != hipSuccess || hipStreamWaitEvent(s2, forked, 0) != hipSuccess) {
-      if (forked) (void)hipEventDestroy(forked);
-      if (joined) (void)hipEventDestroy(joined);
-      forked = joined = nullptr;
-      s2 = nullptr;      // (nothing was queued on it)
-    }
-  }
-  auto drop_events = [&]() {
-    if (forked) (void)hipEventDestroy(forked);
-    if (joined) (void)hipEventDestroy(joined);
-    forked = joined = nullptr;
-  };
-  {
-    hipStream_t sb = s2 ? s2 : s;
-    side_in_use = s2;
-    if (want_bands) {
-      band_bounds_kernel<<<(unsigned)k_vol, 128, 0, sb>>>(kpos, out_map, (int)n_pairs, p->band_count,
-                                                          band_rows > 0 ? band_rows : 1, p->band_start);
-      const int per_xcd = (p->band_count / 8) * k_vol;
-      band_cells_kernel<<<dim3((unsigned)((per_xcd + 255) / 256), 8, 4), 256, 0, sb>>>(
-          p->band_start, k_vol, p->band_count, p->band_cells);
-    }
-    if (tables && (rc = fill_i32(p->nbr_out, so + si, -1, sb))) {
-      drop_events();
-      return fail(rc);
-    }
-    if (s2 && (hipEventRecord(joined, s2) != hipSuccess)) {
-      (void)hipStreamSynchronize(s2);
-      drop_events();
-      set_error("fgms_plan_create: recording on the side stream failed");
-      return fail(FGMS_E_HIP);
-    }
-  }
+  FillBatch fills{};
+  fills.add(p->flags, kPlanFlags * sizeof(int), 0);
   if (tables) {
-    const size_t n_mask = (size_t)(n_out + n_in) * 2;
-    size_t blocks = (n_mask / 4 + 255) / 256;
-    fill_two_kernel<<<(unsigned)(blocks > 8192 ? 8192 : (blocks ? blocks : 1)), 256, 0, s>>>(
-        (int32_t *)rmask, n_mask, 0, p->flags, (size_t)kPlanFlags, 0);
-    if (hipGetLastError() != hipSuccess) {
-      drop_events();
-      set_error("fgms_plan_create: a build launch failed");
-      return fail(FGMS_E_HIP);
-    }
+    fills.add(rmask, (size_t)(n_out + n_in) * sizeof(unsigned long long), 0);
+    fills.add(p->nbr_out, (so + si) * sizeof(int32_t), -1);
   }
-  if (tables && n_pairs > 0) {
-    pair_masks_kernel<<<(unsigned)((n_pairs + 255) / 256) + kPrintParts, 256, 0, s>>>(
-        kpos, in_map, out_map, k_vol, (int)n_pairs, (int)n_in, (int)n_out, rmask_out, rmask_in, p->flags);
-  }
-  // row orders (both sides in the same launches)
-  static const bool sort_rows = !(getenv("FGMS_PLAN_SORT") && atoi(getenv("FGMS_PLAN_SORT")) == 0);
-  int32_t *inv[2] = {nullptr, nullptr};
-  bool published = false;      // the flags reach the host with the tile-order launch
+  if ((rc = launch_fills(fills, s))) return fail(rc);
+  TablesArgs ta{};
+  plan_fill_tables_args(p, &ta);
   if (tables) {
-    SortArgs sa{};
-    sa.k_vol = k_vol;
-    bool any_sort = false, any_count = false;
-    int max_chunks = 0, max_windows = 0;
-    for (int d = 0; d < 2; ++d) {
-      const int64_t n = d ? n_in : n_out;
-      SortSide &sd = sa.side[d];
-      sd.rmask = d ? rmask_in : rmask_out;
-      sd.n = 0;
-      sd.chunks = 0;
-      if (!sort_rows || n <= 64) continue;
-      int32_t *&perm = d ? p->perm_in : p->perm_out;
-      if (!take((void **)&perm, (size_t)n * sizeof(int32_t), false) ||
-          !take((void **)&inv[d], (size_t)n * sizeof(int32_t), true)) {
-        drop_events();
-        set_error("fgms_plan_create: reorder allocation failed");
-        return fail(FGMS_E_NOMEM);
-      }
-      sd.perm = perm;
-      sd.inv = inv[d];
-      sd.n = (int)n;
-      any_sort = true;
-      const int windows = (int)((n + kWindow - 1) / kWindow);
-      if (windows > max_windows) max_windows = windows;
-      if (n > kWindow) {            // more than one window: counting sort on the top bits first
-        sd.chunks = (int)((n + kChunk - 1) / kChunk);
-        if (!take((void **)&sd.perm_tmp, (size_t)n * sizeof(int32_t), true) ||
-            !take((void **)&sd.hist, (size_t)kBins * sd.chunks * sizeof(int32_t), true) ||
-            !take((void **)&sd.hist_before, (size_t)kBins * sd.chunks * sizeof(int32_t), true) ||
-            !take((void **)&sd.bin_start, (size_t)kBins * sizeof(int32_t), true)) {
-          drop_events();
-          set_error("fgms_plan_create: sort allocation failed");
-          return fail(FGMS_E_NOMEM);
-        }
-        any_count = true;
-        if (sd.chunks > max_chunks) max_chunks = sd.chunks;
-      }
-    }
-    if (any_count) {
-      sort_hist_kernel<<<dim3((unsigned)max_chunks, 2), kSortThreads, 0, s>>>(sa);
-      sort_scan_kernel<<<dim3(kBins / kScanBins, 2), kScanBins, 0, s>>>(sa);
-      sort_scatter_kernel<<<dim3((unsigned)max_chunks, 2), kSortThreads, 0, s>>>(sa);
-    }
-    if (any_sort)
-      sort_window_kernel<<<dim3((unsigned)max_windows, 2), kSortThreads,
-                           kWindow * (sizeof(unsigned long long) + sizeof(int)), s>>>(sa);
-  }
-  // join: the tables are pre-filled
-  if (s2 && hipStreamWaitEvent(s, joined, 0) != hipSuccess) {
-    (void)hipStreamSynchronize(s2);
-    drop_events();
-    set_error("fgms_plan_create: joining the side stream failed");
-    return fail(FGMS_E_HIP);
-  }
-  drop_events();
-  if (tables) {
-    MaskArgs ma{};
-    ma.flags = p->flags;
-    ma.side[0] = MaskSide{rmask_out, p->perm_out, p->mask_out, (int)n_out};
-    ma.side[1] = MaskSide{rmask_in, p->perm_in, p->mask_in, (int)n_in};
-    const size_t most = bo > bi ? bo : bi;
     if (n_pairs > 0)
-      tables_kernel<<<(unsigned)((n_pairs + 255) / 256), 256, 0, s>>>(
-          kpos, in_map, out_map, k_vol, (int)n_pairs, (int)n_in, (int)n_out, inv[0], inv[1], p->nbr_out, p->nbr_in);
-    if (most > 0) block_masks_kernel<<<dim3((unsigned)((most + 15) / 16), 2), 1024, 0, s>>>(ma);
-    // tile -> XCD homes pay off once every XCD has a few dozen tiles of its own
-    static const bool xcd_homes = !(getenv("FGMS_XCD_HOME") && atoi(getenv("FGMS_XCD_HOME")) == 0);
-    TileArgs ta{};
-    ta.cus_per_xcd = num_cus() >= 8 ? num_cus() / 8 : 1;
-    int most_tiles = 0;
-    for (int d = 0; d < 2; ++d) {
-      const int64_t n = d ? n_in : n_out;
-      const int n_tiles = (int)((n + 255) / 256);
-      if (!xcd_homes || n_tiles < 256 || (size_t)n_tiles * sizeof(int32_t) > 60000) continue;
-      int32_t *&order = d ? p->tile_in : p->tile_out;
-      const int cap = (n_tiles + 7) / 8;
-      if (!take((void **)&order, (size_t)cap * 8 * sizeof(int32_t), false)) {
-        order = nullptr;       // (the kernels then take the tiles in plain order)
-        continue;
-      }
-      (d ? p->tile_grid_in : p->tile_grid_out) = cap * 8;
-      ta.side[d] = TileSide{d ? p->perm_in : p->perm_out, d ? p->mask_in : p->mask_out, order, (int)n, n_tiles, cap};
-      if (n_tiles > most_tiles) most_tiles = n_tiles;
-    }
-    if (most_tiles > 0) {
-      if (hipHostGetDevicePointer((void **)&ta.host, p->host_flags, 0) != hipSuccess) ta.host = nullptr;
-      ta.flags = p->flags;
-      tile_order_kernel<<<2, 1024, (size_t)most_tiles * sizeof(int32_t), s>>>(ta);
-      published = ta.host != nullptr;
-    }
+      pair_masks_kernel<<<(unsigned)((n_pairs + 255) / 256) + kPrintParts, 256, 0, s>>>(
+          kpos, in_map, out_map, k_vol, (int)n_pairs, (int)n_in, (int)n_out, rmask, rmask + n_out, p->flags);
+    if ((rc = launch_sort(sa, false, s))) return fail(rc);
+    ta.inv_out = sa.side[0].inv; ta.inv_in = sa.side[1].inv;
+    ta.nbr_out = p->nbr_out; ta.nbr_in = p->nbr_in;
   }
-  if (hipGetLastError() != hipSuccess) {
-    set_error("fgms_plan_create: a build launch failed");
-    return fail(FGMS_E_HIP);
-  }
-  int *host_dev = nullptr;
-  if (hipHostGetDevicePointer((void **)&host_dev, p->host_flags, 0) != hipSuccess) host_dev = nullptr;
-  if (host_dev && !published) publish_flags_kernel<<<1, 64, 0, s>>>(p->flags, host_dev);
-  if ((!host_dev && hipMemcpyAsync(p->host_flags, p->flags, kPlanFlags * sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess) ||
-      hipEventRecord(p->ready, s) != hipSuccess) {
-    set_error("fgms_plan_create: queuing the flag read-back failed");
-    return fail(FGMS_E_HIP);
-  }
-  for (void *q : tmp) pool_free(q, s, false);
-  tmp.clear();
+  if ((rc = launch_tables(ta, s)) || (rc = plan_publish(p, ta.host != nullptr, s))) return fail(rc);
+  if (scratch) pool_free(scratch, s, false);
+  scratch = nullptr;
   // More than 64 offsets: the tables and masks hold 64 offsets each, so the offsets are cut
   // into groups of 64, every group with tables of its own (the pairs of a group are one
   // contiguous run of the lists); the entry points walk the groups, the weight gradient uses
@@ -982,6 +908,14 @@ static bool plan_is_stale(const Plan *p) {
   return false;
 }
 
+static int fill_pair_view(const Plan *p, int64_t rows, hipStream_t s) {
+  FillBatch fills{};
+  fills.add(p->pv_in, (size_t)rows * sizeof(int32_t), -1);
+  fills.add(p->pv_out, (size_t)rows * sizeof(int32_t), -1);
+  fills.add(p->pv_mask, (size_t)(rows / 64) * sizeof(unsigned long long), 0);
+  return launch_fills(fills, s);
+}
+
 const Plan *plan_resolve(fgms_plan_t *plan, hipStream_t stream, int *rc) {
   *rc = FGMS_OK;
   Plan *p = (Plan *)plan;
@@ -998,6 +932,7 @@ const Plan *plan_resolve(fgms_plan_t *plan, hipStream_t stream, int *rc) {
     std::lock_guard<std::mutex> lock(p->mutex);
     if (!p->resolved) {
       p->nbr_out = b->nbr_in; p->nbr_in = b->nbr_out;
+      p->nbr_stride_out = b->nbr_stride_in; p->nbr_stride_in = b->nbr_stride_out;
       p->perm_out = b->perm_in; p->perm_in = b->perm_out;
       p->mask_out = b->mask_in; p->mask_in = b->mask_out;
       p->tile_out = b->tile_in; p->tile_in = b->tile_out;
@@ -1056,8 +991,7 @@ const Plan *plan_resolve(fgms_plan_t *plan, hipStream_t stream, int *rc) {
             pool_alloc((void **)&p->pv_in, (size_t)rows * sizeof(int32_t), s) == FGMS_OK &&
             pool_alloc((void **)&p->pv_out, (size_t)rows * sizeof(int32_t), s) == FGMS_OK &&
             pool_alloc((void **)&p->pv_mask, (size_t)(rows / 64) * sizeof(unsigned long long), s) == FGMS_OK &&
-            fill_i32(p->pv_in, (size_t)rows, -1, s) == FGMS_OK && fill_i32(p->pv_out, (size_t)rows, -1, s) == FGMS_OK &&
-            fill_i32((int32_t *)p->pv_mask, (size_t)(rows / 64) * 2, 0, s) == FGMS_OK) {
+            fill_pair_view(p, rows, s) == FGMS_OK) {
           pair_view_kernel<<<(unsigned)((p->n_pairs + 255) / 256), 256, 0, s>>>(
               p->kpos, p->in_map, p->out_map, p->k_vol, (int)p->n_pairs, (long long)rows, p->pv_in, p->pv_out,
               p->pv_mask);
@@ -1164,14 +1098,7 @@ void fgms_plan_destroy(fgms_plan_t *plan) {
   }
   p->groups.clear();
   if (p->many_streams) (void)hipDeviceSynchronize();     // (blocks are handed back behind ONE stream's work)
-  if (p->nbr_out) pool_free(p->nbr_out, p->last_stream, false);      // (nbr_in is the same block)
-  if (p->mask_out) pool_free(p->mask_out, p->last_stream, false);    // (mask_in likewise)
-  if (p->perm_out) pool_free(p->perm_out, p->last_stream, false);
-  if (p->perm_in) pool_free(p->perm_in, p->last_stream, false);
-  if (p->band_start) pool_free(p->band_start, p->last_stream, false);
-  if (p->band_cells) pool_free(p->band_cells, p->last_stream, false);
-  if (p->tile_out) pool_free(p->tile_out, p->last_stream, false);
-  if (p->tile_in) pool_free(p->tile_in, p->last_stream, false);
+  if (p->block) pool_free(p->block, p->last_stream, false);
   if (p->pv_ready) {
     // the view may have been built on another stream than the one the blocks are handed back behind
     if (p->pv_stream != p->last_stream) (void)hipStreamWaitEvent(p->last_stream, p->pv_ready, 0);
@@ -1183,9 +1110,8 @@ void fgms_plan_destroy(fgms_plan_t *plan) {
   if (p->ready) {
     // the flag read-back must not land in freed host memory
     (void)hipEventSynchronize(p->ready);
-    (void)hipEventDestroy(p->ready);
+    event_put(p->ready, p->device);
   }
-  if (p->flags) pool_free(p->flags, p->last_stream, false);
   if (p->host_flags) pinned_flags_put(p->host_flags);
   delete p;
 }

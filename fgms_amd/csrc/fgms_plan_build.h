@@ -1,0 +1,122 @@
+// What the two ways to a plan share: from a caller's pair lists (fgms_plan.hip) and together with
+// the map itself from voxel coordinates (fgms_kmap.hip).  Both end in the same row masks; from
+// there on the row order, the tables and the dispatch orders are built by the launches declared here.
+#pragma once
+
+#include "fgms_device.h"
+#include "fgms_internal.h"
+
+namespace fgms {
+
+// Blocks of one pool allocation, laid out by running the same `take` calls twice: without a base
+// to add the sizes up, then with it.  (One block per build: a pool block costs two runtime calls
+// on its way out and two on its way back.)
+struct Arena {
+  char *base = nullptr;
+  size_t used = 0;
+  template <typename T>
+  void take(T *&p, size_t count) {
+    p = base ? reinterpret_cast<T *>(base + used) : nullptr;
+    used += (count * sizeof(T) + 255) & ~(size_t)255;
+  }
+};
+
+// ---- fills of a build, all in one launch
+struct FillRange {
+  int32_t *p;
+  size_t n;
+  int32_t v;
+};
+struct FillBatch {
+  FillRange range[6];
+  int count;
+  void add(void *p, size_t bytes, int32_t v) {
+    if (bytes) range[count++] = FillRange{(int32_t *)p, bytes / 4, v};
+  }
+};
+int launch_fills(const FillBatch &batch, hipStream_t s);
+
+// ---- row order (see fgms_plan.hip)
+struct SortSide {
+  const unsigned long long *rmask;   // per row: the offsets it has a pair in
+  int32_t *perm_tmp;                 // order after the counting sort
+  int32_t *perm;                     // final order: position -> row
+  int32_t *inv;                      // row -> position
+  int32_t *hist;                     // [chunks][kBins] rows per (chunk, bin)
+  int32_t *hist_before;              // [chunks][kBins] rows of the bin in earlier chunks
+  int32_t *bin_start;                // [kBins] rows per bin
+  unsigned long long *block_mask;    // OR of the masks of every 64 positions
+  unsigned long long *mirror_mask;   // the same with bit k at k_vol - 1 - k, or nullptr
+  int n, chunks;                     // chunks == 0: one window, no counting sort
+};
+struct SortArgs {
+  SortSide side[2];                  // output side, input side (n == 0: none)
+  int k_vol;
+  int *flags;
+  bool by_mask;                      // false: natural order
+};
+constexpr int kBinBits = 11;
+constexpr int kBins = 1 << kBinBits;
+constexpr int kChunk = 2048;         // rows per workgroup of the histogram / scatter kernels
+constexpr int kWindow = 2048;        // positions per workgroup of the window sort
+constexpr int kSortThreads = 1024;
+
+__device__ __forceinline__ int top_bits(unsigned long long m, int k_vol) {
+  const int shift = k_vol > kBinBits ? k_vol - kBinBits : 0;
+  return (int)((m >> shift) & (kBins - 1));
+}
+
+// Rows per bin of one chunk; `hist`: kBins ints of LDS, `threads` threads.
+__device__ __forceinline__ void sort_hist_body(const SortSide &sd, int k_vol, int chunk, int *hist, int threads) {
+  for (int i = threadIdx.x; i < kBins; i += threads) hist[i] = 0;
+  __syncthreads();
+  for (int e = threadIdx.x; e < kChunk; e += threads) {
+    const int row = chunk * kChunk + e;
+    if (row < sd.n) atomicAdd(&hist[top_bits(sd.rmask[row], k_vol)], 1);
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < kBins; i += threads) sd.hist[(size_t)chunk * kBins + i] = hist[i];
+}
+
+// Lays out a side's temporaries.
+void sort_side_layout(SortSide &sd, int64_t n, Arena &tmp);
+// Histogram (unless the caller's own launch took it), scan, scatter, window sort.
+int launch_sort(const SortArgs &a, bool hist_done, hipStream_t s);
+
+// ---- the last launch of a build: tables by position, row bands, tile order, findings
+struct TileSide {
+  const int32_t *perm;
+  const unsigned long long *block_masks;
+  int32_t *order;                    // nullptr: none
+  int n_rows, n_tiles, cap;
+};
+struct TablesArgs {
+  const int32_t *kpos, *imap, *omap;
+  int k_vol, n_pairs, n_in, n_out;
+  // from the pair lists: position -> neighbour through offset k (tables pre-filled with -1; nullptr: not this one)
+  const int32_t *inv_out, *inv_in;
+  int32_t *nbr_out, *nbr_in;
+  // from a table of the output rows, [n_out][row_ld]: nbr_out only
+  const int32_t *rows;
+  const int32_t *perm_out;
+  int row_ld;
+  // bands
+  int32_t *band_start, *band_cells;
+  int bands, band_rows;
+  TileSide tile[2];
+  int cus_per_xcd;
+  int *flags, *host;                 // findings and where they go on the host (nullptr: a copy follows)
+  bool mirror, take_print;           // one side's counts stand for both; fingerprint of the lists
+  // workgroups of each part, in this order
+  int tile_blocks, band_blocks, print_blocks, row_blocks, pair_blocks;
+};
+int launch_tables(TablesArgs a, hipStream_t s);
+
+// Plan objects without their tables.
+Plan *plan_alloc(int k_vol, int64_t n_in, int64_t n_out, int64_t n_pairs, hipStream_t s);
+void plan_bands(Plan *p);                                // band_count / band_rows from the sizes
+int tile_table(int64_t n, int *cap);                     // tiles of a side that gets a table, else 0
+void plan_fill_tables_args(const Plan *p, TablesArgs *t);
+int plan_publish(Plan *p, bool written, hipStream_t s);  // findings on their way to the host, `ready` recorded
+
+}  // namespace fgms

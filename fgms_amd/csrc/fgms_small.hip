@@ -113,7 +113,7 @@ template <typename T, int CS, int CD, bool TR>
 __global__ __launch_bounds__(kSmallThreads) void gms_small_kernel(
     const T *__restrict__ src, const uint32_t *__restrict__ w, T *__restrict__ dst,
     const int32_t *__restrict__ nbr, const unsigned long long *__restrict__ block_masks,
-    const int32_t *__restrict__ perm, int n_dst, int parts, int overwrite, SideJob side) {
+    const int32_t *__restrict__ perm, int n_dst, int parts, int overwrite, SideJob side, int nbr_stride) {
   // the leading workgroups of the grid run the side job, if there is one
   int block_x = blockIdx.x;
   if (side.blocks) {
@@ -162,7 +162,7 @@ __global__ __launch_bounds__(kSmallThreads) void gms_small_kernel(
   // lanes past the last row shadow it and skip the final store; an index asked for past
   // the last offset (k < 0) is read from offset 0 and never used
   const int row_c = live ? row : n_dst - 1;
-  auto index_of = [&](int k) { return nbr[(size_t)(k < 0 ? 0 : k) * n_dst + row_c]; };
+  auto index_of = [&](int k) { return nbr[(ptrdiff_t)(k < 0 ? 0 : k) * nbr_stride + row_c]; };
   auto gather = [&](float (&x)[CS], int g) { load_row<T, CS>(x, src + (size_t)(g < 0 ? 0 : g) * CS); };
   int k0 = next_k();
   if (k0 >= 0) {
@@ -250,10 +250,12 @@ int launch_small(const GmsArgs &a, const Plan *p) {
     ProfileScope prof(a.transpose_w ? "gms_small_kernel(dgrad)" : "gms_small_kernel(fwd)", a.stream);
     if (a.transpose_w)
       gms_small_kernel<T, CS, CD, true><<<gx, kSmallThreads, lds, a.stream>>>(
-          (const T *)a.src, (const uint32_t *)a.w, (T *)a.dst, nbr, masks, perm, (int)a.n_dst, parts, a.overwrite ? 1 : 0, a.side);
+          (const T *)a.src, (const uint32_t *)a.w, (T *)a.dst, nbr, masks, perm, (int)a.n_dst, parts, a.overwrite ? 1 : 0, a.side,
+          a.transpose_w ? p->nbr_stride_in : p->nbr_stride_out);
     else
       gms_small_kernel<T, CS, CD, false><<<gx, kSmallThreads, lds, a.stream>>>(
-          (const T *)a.src, (const uint32_t *)a.w, (T *)a.dst, nbr, masks, perm, (int)a.n_dst, parts, a.overwrite ? 1 : 0, a.side);
+          (const T *)a.src, (const uint32_t *)a.w, (T *)a.dst, nbr, masks, perm, (int)a.n_dst, parts, a.overwrite ? 1 : 0, a.side,
+          a.transpose_w ? p->nbr_stride_in : p->nbr_stride_out);
   }
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;
