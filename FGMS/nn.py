@@ -13,7 +13,9 @@ layer, pass and iteration that shares a map shares its plan through ``FGMS.backe
 cache, which is keyed on these tensors.
 """
 import math
+import threading
 
+import numpy as np
 import torch
 
 from . import backend
@@ -43,10 +45,30 @@ class KernelMap:
     @classmethod
     def from_coords(cls, in_coords, out_coords, offsets, stride=1):
         """Builds the map on the device from int32 voxel coordinates ``[N, 3]``: pairs
-        (i, o) with ``in_coords[i] == out_coords[o] * stride + offsets[k]``."""
-        from fgms_amd import capi
-        in_map, out_map, knnz, _ = capi.build_kernel_map(in_coords, out_coords, offsets, stride)
-        return cls(in_map, out_map, knnz, in_coords.shape[0], out_coords.shape[0])
+        (i, o) with ``in_coords[i] == out_coords[o] * stride + offsets[k]``, and the plan along
+        with it.  Everything is queued on the stream; the first use of the map waits for it."""
+        offs = torch.from_numpy(np.ascontiguousarray(np.asarray(offsets, dtype=np.int32).reshape(-1, 3)))
+        m = cls.__new__(cls)
+        m._on_its_way = backend.MapOnItsWay(in_coords, out_coords, offs, int(stride))
+        m._lock = threading.Lock()
+        m.k_vol, m.n_in, m.n_out = offs.shape[0], in_coords.shape[0], out_coords.shape[0]
+        return m
+
+    def __getattr__(self, name):
+        # a map from coordinates is waited for when something first needs it
+        if name in ("in_map", "out_map", "kernel_nnz", "kpos", "qkpos", "qsum") and "_lock" in self.__dict__:
+            with self._lock:
+                if "_on_its_way" in self.__dict__:
+                    parts = self._on_its_way.finish()
+                    del self._on_its_way
+                    self.in_map, self.out_map, self.kernel_nnz, self.kpos, self.qkpos, self.qsum = parts
+            if name in self.__dict__:
+                return self.__dict__[name]
+        raise AttributeError(name)
+
+    def __getstate__(self):
+        self.kpos                                                   # (copies are taken of a finished map)
+        return {k: v for k, v in self.__dict__.items() if k != "_lock"}
 
     def transposed(self):
         """The map of the transposed convolution: the same pairs, roles swapped.  It keeps

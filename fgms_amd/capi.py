@@ -17,7 +17,7 @@ SYMBOLS = [
     "fgms_version", "fgms_last_error", "fgms_plan_create", "fgms_plan_check", "fgms_plan_transposed", "fgms_plan_destroy",
     "fgms_plan_usable", "fgms_plan_stats", "fgms_conv_fwd", "fgms_conv_bwd", "fgms_fusion_fwd", "fgms_fwd", "fgms_bwd", "fgms_dgrad",
     "fgms_wgrad", "fgms_wgrad_static", "fgms_set_kernel_policy", "fgms_profile_enable", "fgms_profile_read",
-    "fgms_profile_reset", "fgms_probe_gather", "fgms_build_kernel_map", "fgms_allocation_count",
+    "fgms_profile_reset", "fgms_probe_gather", "fgms_build_kernel_map", "fgms_build_map_begin", "fgms_build_map_end", "fgms_allocation_count",
     "fgms_weights_pin", "fgms_weights_unpin", "fgms_relaid_weights_hits",
 ]
 
@@ -65,6 +65,9 @@ def lib():
     L.fgms_build_kernel_map.argtypes = [vp, i64, vp, i64, vp, i32, i32, i32, vp, vp, i64, vp, vp,
                                         ctypes.POINTER(ctypes.c_int64), vp]
     L.fgms_build_kernel_map.restype = i32
+    L.fgms_build_map_begin.argtypes = [ctypes.POINTER(vp), vp, i64, vp, i64, vp, i32, i32, i32, vp, vp, i64, vp, vp, vp,
+                                       i32, vp]
+    L.fgms_build_map_end.argtypes = [vp, vp, ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(vp)]
     L.fgms_probe_gather.argtypes = [vp, i32, i32, i32, vp, vp]
     L.fgms_probe_gather.restype = i32
     L.fgms_set_kernel_policy.argtypes = [i32]

@@ -1075,15 +1075,37 @@ int fgms_build_kernel_map(const int32_t *in_coords, int64_t n_in, const int32_t 
                           int64_t n_out, const int32_t *offsets, int k_vol, int stride,
                           int skip_offset, int32_t *in_map, int32_t *out_map, int64_t capacity,
                           int32_t *kernel_nnz, int32_t *kpos, int64_t *n_pairs, void *stream) {
-  if (n_in < 0 || n_out < 0 || k_vol <= 0 || stride <= 0 || capacity < 0 || !offsets || !kernel_nnz ||
-      !kpos || !n_pairs || (n_in > 0 && !in_coords) || (n_out > 0 && !out_coords) ||
+  if (!n_pairs) {
+    set_error("fgms_build_kernel_map: bad argument");
+    return FGMS_E_INVALID;
+  }
+  fgms_map_build_t *build = nullptr;
+  const int rc = fgms_build_map_begin(&build, in_coords, n_in, out_coords, n_out, offsets, k_vol, stride, skip_offset, in_map,
+                                      out_map, capacity, kernel_nnz, kpos, nullptr, 0, stream);
+  return rc != FGMS_OK ? rc : fgms_build_map_end(build, nullptr, n_pairs, nullptr);
+}
+
+int fgms_build_map_begin(fgms_map_build_t **build, const int32_t *in_coords, int64_t n_in, const int32_t *out_coords,
+                         int64_t n_out, const int32_t *offsets, int k_vol, int stride, int skip_offset, int32_t *in_map,
+                         int32_t *out_map, int64_t capacity, int32_t *kernel_nnz, int32_t *kpos, int32_t *qkpos,
+                         int want_plan, void *stream) {
+  if (!build || n_in < 0 || n_out < 0 || k_vol <= 0 || stride <= 0 || capacity < 0 || !offsets || !kernel_nnz ||
+      !kpos || (n_in > 0 && !in_coords) || (n_out > 0 && !out_coords) ||
       (capacity > 0 && (!in_map || !out_map)) || n_in > INT32_MAX ||
       (int64_t)k_vol * n_out > INT32_MAX - 65536) {
     set_error("fgms_build_kernel_map: bad argument");
     return FGMS_E_INVALID;
   }
-  return build_kernel_map(in_coords, n_in, out_coords, n_out, offsets, k_vol, stride, skip_offset,
-                          in_map, out_map, capacity, kernel_nnz, kpos, n_pairs, (hipStream_t)stream);
+  return map_build_begin((MapBuild **)build, in_coords, n_in, out_coords, n_out, offsets, k_vol, stride, skip_offset, in_map,
+                         out_map, capacity, kernel_nnz, kpos, qkpos, want_plan != 0, true, (hipStream_t)stream);
+}
+
+int fgms_build_map_end(fgms_map_build_t *build, int32_t *host_nnz, int64_t *n_pairs, fgms_plan_t **plan) {
+  if (!build || !n_pairs) {
+    set_error("fgms_build_map_end: bad argument");
+    return FGMS_E_INVALID;
+  }
+  return map_build_end((MapBuild *)build, host_nnz, n_pairs, plan);
 }
 
 int fgms_probe_gather(const void *feats, int c_src, int dtype, int for_dgrad, fgms_plan_t *plan,

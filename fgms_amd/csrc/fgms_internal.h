@@ -141,11 +141,11 @@ struct Plan {
   int32_t *perm_in;   // [n_in]
   int32_t *nbr_out;   // [k_vol, n_out]: input row feeding the output row at position p through offset k, or -1
   int32_t *nbr_in;    // [k_vol, n_in]:  output row fed by the input row at position p through offset k, or -1
-  // entries from one offset's row of a table to the next one's.  A mirrored map (a submanifold map is
-  // its own mirror image: input row r reaches through offset k what output row r is reached by through
-  // k_vol - 1 - k) keeps one table and one order for both sides: nbr_in starts at nbr_out's last offset
-  // and its stride is negative
-  int nbr_stride_out, nbr_stride_in;
+  // A submanifold map is its own mirror image: input row r reaches through offset k what output row r
+  // is reached by through k_vol - 1 - k.  Where the builder knows that, both sides share one set of
+  // tables, in the output side's numbering: what the input side's kernels read as offset k stands for
+  // the weights of k_vol - 1 - k.  flip = k_vol - 1 says so (0: offsets are what they are).
+  int flip_out, flip_in;
   void *block;        // the pool block all of the plan's tables lie in
   // bit k of mask_out[b] : some row of the 64-row block b has a neighbour through
   // offset k (only built when k_vol <= 64; the output-stationary kernels need it)
@@ -296,10 +296,13 @@ const Plan *plan_if_resolved(fgms_plan_t *plan);
 bool plan_take_check(const Plan *p, SideJob *job);
 int plan_flush_check(const Plan *p, hipStream_t stream);
 void note_allocation();      // counts a hipMalloc / hipHostMalloc of the library (fgms_allocation_count)
-int build_kernel_map(const int32_t *in_coords, int64_t n_in, const int32_t *out_coords, int64_t n_out,
-                     const int32_t *offsets_host, int k_vol, int stride, int skip_offset,
-                     int32_t *in_map, int32_t *out_map, int64_t capacity, int32_t *kernel_nnz,
-                     int32_t *kpos, int64_t *n_pairs, hipStream_t stream);
+// fgms_build_map_begin / fgms_build_map_end (fgms_kmap.hip).
+struct MapBuild;
+int map_build_begin(MapBuild **build, const int32_t *in_coords, int64_t n_in, const int32_t *out_coords, int64_t n_out,
+                    const int32_t *offsets_host, int k_vol, int stride, int skip_offset,
+                    int32_t *in_map, int32_t *out_map, int64_t capacity, int32_t *kernel_nnz,
+                    int32_t *kpos, int32_t *qkpos, bool want_plan, bool allow_mirror, hipStream_t s);
+int map_build_end(MapBuild *b, int32_t *host_nnz, int64_t *n_pairs, fgms_plan_t **plan_out);
 int launch_gather_probe(const Plan *p, const void *src, int c_src, int dtype, bool for_dgrad,
                         void *sink, hipStream_t stream);
 

@@ -1,341 +1,740 @@
 // Kernel-map builder on the device: from voxel coordinates to the pair lists the
-// convolution kernels consume.  The reference has no builder (its scripts load
-// in_map / out_map / kernel_nnz / kernel_pos from files, cpu-check.py:89-94,
-// spconv-test.py:64-73); this is the step right before the path.
+// convolution kernels consume, and, if asked for, to the plan of the map as well.  The reference has
+// no builder (its scripts load in_map / out_map / kernel_nnz / kernel_pos from files,
+// cpu-check.py:89-94, spconv-test.py:64-73); this is the step right before the path.
 //
 // Pairs (i, o) with  in_coords[i] == out_coords[o] * stride + offsets[k],
 // grouped by offset k, ascending o inside a group; when several input rows share
 // a coordinate the smallest row index wins.  The result is a pure function of
 // the inputs (no dependence on thread timing).
 //
-//   1. insert   every input coordinate, packed into 63 bits, goes into an open-
-//               addressing hash table (linear probing, load <= 0.5); the slot
-//               keeps the smallest row index (atomicMin)
-//   2. lookup   one thread per (offset, output row): probe, write the hit (or
-//               -1) into a [k_vol][n_out] table, count hits per 256-row block
-//   3. scan     exclusive prefix sum over the (offset, block) counts (one workgroup)
-//   4. write    hits are compacted in (offset, row) order: block base from the
-//               scan, rank inside the block from wave ballots
+//   1. fill     everything that has to start from a value
+//   2. insert   every input row enters its block of 2 x 2 x 4 voxels; the blocks are found through
+//               an open-addressing hash table (linear probing, load <= 0.5); equal coordinates keep the
+//               smallest row
+//   3. lookup   a table of the output rows, [n_out][offsets] -> input row or -1, the
+//               set of offsets every row has a pair through, hits per (offset, 256 rows)
+//   4. scan     prefix sum over those counts
+//   5. lists    hits compacted in (offset, row) order; next to it the histogram of the plan's sort
+//   6. plan     row order and tables (fgms_plan.hip), from the table of step 3: no atomics per
+//               pair, no second pass over the lists.  A submanifold map (one coordinate list on
+//               both sides, mirrored offsets) is its own mirror image, so one order and one table
+//               serve both directions.
+// At 100 k voxels x 27 offsets the whole build takes 110 us of the stream; lists alone and a plan from
+// them afterwards took 140 and 195 us, each behind a wait of the host for the one before.
+#include <immintrin.h>
 #include <stdlib.h>
 #include <string.h>
 
+#include <atomic>
+#include <mutex>
 #include <vector>
 
 #include "fgms_device.h"
 #include "fgms_internal.h"
+#include "fgms_plan_build.h"
 
 namespace fgms {
 namespace {
 
-constexpr unsigned long long kEmptyKey = ~0ull;
-constexpr int kCoordBits = 21;
-constexpr long long kCoordBias = 1ll << (kCoordBits - 1);   // coordinates in [-2^20, 2^20)
-constexpr int kBlock = 256;
+typedef int int4v_ __attribute__((ext_vector_type(4)));
 
-// Exclusive prefix sum of n ints by one workgroup of 1024 threads, 4096 values a round: every
-// thread takes four neighbouring values (the loads of a wave are contiguous), the waves scan
-// their threads' sums with lane shuffles, the 16 wave totals go through LDS, and the sum of the
-// rounds so far is carried in a register.  The counts are few (offsets x 256-row blocks: 21 k
-// for 200 k voxels), so one workgroup is enough.
-__global__ __launch_bounds__(1024) void kmap_scan_kernel(const int32_t *__restrict__ in, int32_t *__restrict__ out,
-                                                         size_t n) {
-  __shared__ int wave_totals[2][16];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  int carry = 0, round = 0;
-  for (size_t base = 0; base < n; base += 4096, round ^= 1) {
-    const size_t i = base + (size_t)tid * 4;
-    int v[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = i + j < n ? in[i + j] : 0;
-    const int mine = v[0] + v[1] + v[2] + v[3];
-    int incl = mine;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int up = __shfl_up(incl, d, 64);
-      if (lane >= d) incl += up;
-    }
-    if (lane == 63) wave_totals[round][wave] = incl;
-    __syncthreads();      // the other buffer is written next round, after every wave has passed this barrier
-    int before = 0, total = 0;
-#pragma unroll
-    for (int w = 0; w < 16; ++w) {
-      const int t = wave_totals[round][w];
-      before += w < wave ? t : 0;
-      total += t;
-    }
-    int run = carry + before + incl - mine;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (i + j < n) out[i + j] = run;
-      run += v[j];
-    }
-    carry += total;
-  }
+constexpr int kCoordLimit = 1 << 20;        // coordinates in [-2^20, 2^20)
+constexpr int kListRows = 256;              // output rows per count
+constexpr int kKernargOffsets = 128;        // offsets that travel as a kernel argument
+// pinned read-back: [0] coordinates looked at, [1] bad one among them, [2] shared ones; [3] sizes there, [4] pairs, [16 ...] sizes
+constexpr int kHostInts = 16 + 1024;
+
+struct Offsets {
+  int xyz[kKernargOffsets * 3];
+};
+
+// Voxels are found by blocks of 2 x 2 x 4: the hash table holds one row number per block in use (its
+// representative: the row that got there first), and a block's 16 voxels lie in one 64-byte piece of
+// `cells`, at the representative's number.  The 27 neighbours of a voxel lie in 8 blocks, and
+// neighbouring rows share them: an eighth of the random accesses that a table of voxels costs, which
+// is what such a table is bound by (100 k rows x 27 offsets: 2.7 M probes of a line each).
+constexpr int kBlockX = 1, kBlockY = 1, kBlockZ = 2;      // bits of a coordinate inside its block
+constexpr int kCells = 1 << (kBlockX + kBlockY + kBlockZ);
+constexpr int kNoRow = INT32_MAX;
+
+__device__ __forceinline__ unsigned slot_of(int bx, int by, int bz, unsigned mask) {
+  unsigned h = (unsigned)bx * 0x9E3779B1u ^ (unsigned)by * 0x85EBCA77u ^ (unsigned)bz * 0xC2B2AE3Du;
+  h ^= h >> 15; h *= 0x2C1B3C6Du;
+  h ^= h >> 12; h *= 0x297A2D39u;
+  h ^= h >> 15;
+  return h & mask;
+}
+__device__ __forceinline__ int cell_of(int x, int y, int z) { return (x & 1) << 3 | (y & 1) << 2 | (z & 3); }
+__device__ __forceinline__ bool same_block(const int32_t *__restrict__ coords, int row, int bx, int by, int bz) {
+  return coords[3 * row] >> kBlockX == bx && coords[3 * row + 1] >> kBlockY == by && coords[3 * row + 2] >> kBlockZ == bz;
 }
 
-__device__ __forceinline__ bool pack_key(long long x, long long y, long long z, unsigned long long &key) {
-  x += kCoordBias; y += kCoordBias; z += kCoordBias;
-  if ((x | y | z) < 0 || ((x | y | z) >> kCoordBits) != 0) return false;
-  key = ((unsigned long long)x << (2 * kCoordBits)) | ((unsigned long long)y << kCoordBits) |
-        (unsigned long long)z;
-  return true;
-}
-
-__device__ __forceinline__ unsigned long long mix(unsigned long long h) {   // splitmix64 finaliser
-  h ^= h >> 30; h *= 0xbf58476d1ce4e5b9ull;
-  h ^= h >> 27; h *= 0x94d049bb133111ebull;
-  return h ^ (h >> 31);
-}
-
-__global__ void kmap_fill_kernel(unsigned long long *__restrict__ keys, int32_t *__restrict__ vals,
-                                 size_t slots) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < slots) {
-    keys[i] = kEmptyKey;
-    vals[i] = INT32_MAX;
-  }
-}
-
-__global__ void kmap_fill_none_kernel(int32_t *__restrict__ p, size_t n) {
-  size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (; i < n; i += stride) p[i] = -1;
-}
-
-// flags[0]: an input coordinate is outside the packable range; flags[2]: two input rows share
-// their coordinates
-__global__ void kmap_insert_kernel(const int32_t *__restrict__ coords, int n,
-                                   unsigned long long *__restrict__ keys, int32_t *__restrict__ vals,
-                                   unsigned long long mask, int *__restrict__ flags) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+// flags[0]: an input coordinate is outside the range; flags[1]: two input rows share their coordinates
+__global__ __launch_bounds__(256) void kmap_insert_kernel(const int32_t *__restrict__ coords, int n, int32_t *__restrict__ slots,
+                                                          unsigned mask, int32_t *__restrict__ cells, int *__restrict__ flags) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
-  unsigned long long key;
-  if (!pack_key(coords[3 * i], coords[3 * i + 1], coords[3 * i + 2], key)) {
+  const int x = coords[3 * i], y = coords[3 * i + 1], z = coords[3 * i + 2];
+  if (x < -kCoordLimit || x >= kCoordLimit || y < -kCoordLimit || y >= kCoordLimit || z < -kCoordLimit || z >= kCoordLimit) {
     flags[0] = 1;
     return;
   }
-  unsigned long long slot = mix(key) & mask;
-  while (true) {                       // ends: load <= 0.5, a free or equal slot exists
-    const unsigned long long prev = atomicCAS(&keys[slot], kEmptyKey, key);
-    if (prev == kEmptyKey || prev == key) {
-      if (prev == key) flags[2] = 1;
-      atomicMin(&vals[slot], i);
-      return;
+  const int bx = x >> kBlockX, by = y >> kBlockY, bz = z >> kBlockZ;
+  unsigned slot = slot_of(bx, by, bz, mask);
+  int rep = i;
+  while (true) {                       // ends: the table has two slots per row and more
+    const int prev = atomicCAS(&slots[slot], -1, i);
+    if (prev < 0) break;
+    if (same_block(coords, prev, bx, by, bz)) {
+      rep = prev;
+      break;
     }
     slot = (slot + 1) & mask;
   }
+  if (atomicMin(&cells[(size_t)rep * kCells + cell_of(x, y, z)], i) != kNoRow) flags[1] = 1;
 }
 
-// grid (blocks of 256 output rows, k_vol).  table[k][o] = input row or -1;
-// counts[k * n_blocks + block] = hits of the block.
-// mirror_k > 0 (= k_vol, odd): the map is its own mirror image -- one coordinate list on
-// both sides, unique coordinates, offsets[k_vol - 1 - k] = -offsets[k] -- so a hit (k, o) -> i
-// is also the hit (k_vol - 1 - k, i) -> o.  The grid then covers the offsets up to the centre
-// only and fills the other half of the table (pre-filled with -1) from its hits: half the
-// hash lookups.  kmap_count_kernel then counts that half's hits per block.
-__global__ __launch_bounds__(kBlock) void kmap_lookup_kernel(
-    const int32_t *__restrict__ out_coords, int n_out, const int32_t *__restrict__ offsets,
-    int stride, int skip_offset, const unsigned long long *__restrict__ keys,
-    const int32_t *__restrict__ vals, unsigned long long mask, int32_t *__restrict__ table,
-    int32_t *__restrict__ counts, int mirror_k) {
-  __shared__ int block_hits;
-  const int k = blockIdx.y, o = blockIdx.x * kBlock + threadIdx.x;
-  if (threadIdx.x == 0) block_hits = 0;
-  __syncthreads();
-  int hit = -1;
-  if (o < n_out && k != skip_offset) {
-    unsigned long long key;
-    if (pack_key((long long)out_coords[3 * o] * stride + offsets[3 * k],
-                 (long long)out_coords[3 * o + 1] * stride + offsets[3 * k + 1],
-                 (long long)out_coords[3 * o + 2] * stride + offsets[3 * k + 2], key)) {
-      unsigned long long slot = mix(key) & mask;
-      while (true) {
-        const unsigned long long at = keys[slot];
-        if (at == key) { hit = vals[slot]; break; }
-        if (at == kEmptyKey) break;
-        slot = (slot + 1) & mask;
+struct LookupArgs {
+  const int32_t *in_coords, *out_coords;
+  int n_out, k_vol, stride, skip_offset, row_ld;
+  const int32_t *slots, *cells;
+  unsigned mask;
+  const int32_t *offsets;                      // device; nullptr: `offs`
+  int32_t *rows;                               // [n_out][row_ld]
+  int32_t *counts;                             // [k_vol][blocks of kListRows rows]
+  int blocks;
+  unsigned long long *rmask_out, *rmask_in;    // nullptr: no plan / a mirrored one
+  const int *flags;
+  int *host;                                   // pinned
+};
+
+// What the insertion found out, to the host.
+__device__ __forceinline__ void publish_coordinates(const int *__restrict__ flags, int *__restrict__ host) {
+  if (threadIdx.x != 0) return;
+  host[1] = flags[0];
+  host[2] = flags[1];
+  __threadfence_system();
+  __hip_atomic_store(&host[0], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// The representatives of N blocks (-1: not in use; want = false: not asked for), all probed together.
+template <int N>
+__device__ __forceinline__ void find_blocks(const LookupArgs &a, const int (&bx)[N], const int (&by)[N], const int (&bz)[N],
+                                            const bool (&want)[N], int (&rep)[N]) {
+  unsigned slot[N];
+  bool open[N], any = false;
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    rep[u] = -1;
+    open[u] = want[u];
+    any = any || open[u];
+    slot[u] = slot_of(bx[u], by[u], bz[u], a.mask);
+  }
+  while (any) {                        // ends: every chain meets its block or an empty slot
+    int cand[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) cand[u] = open[u] ? a.slots[slot[u]] : -1;
+    int cx[N], cy[N], cz[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      const int c = cand[u] < 0 ? 0 : cand[u];
+      cx[u] = a.in_coords[3 * c]; cy[u] = a.in_coords[3 * c + 1]; cz[u] = a.in_coords[3 * c + 2];
+    }
+    any = false;
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      if (cand[u] < 0) {
+        open[u] = false;
+      } else if (cx[u] >> kBlockX == bx[u] && cy[u] >> kBlockY == by[u] && cz[u] >> kBlockZ == bz[u]) {
+        rep[u] = cand[u];
+        open[u] = false;
+      } else if (open[u]) {
+        slot[u] = (slot[u] + 1) & a.mask;
+        any = true;
       }
     }
   }
-  if (o < n_out) table[(size_t)k * n_out + o] = hit;
-  if (mirror_k > 0 && hit >= 0 && 2 * k + 1 < mirror_k) {
-    const int km = mirror_k - 1 - k;
-    table[(size_t)km * n_out + hit] = o;      // (counted by kmap_count_kernel afterwards)
+}
+
+// The last workgroup sends the insertion's findings to the host.  The others take 64 output rows
+// each.  NEAR (every offset within one voxel): its four waves find two of
+// each row's eight blocks each, then every wave reads every fourth offset's cell from them.  Else
+// (wider kernels) a lane finds the blocks of up to seven offsets at a time for itself.
+// Bound by latency -- slot, representative's coordinates, cell: three dependent loads, with two to
+// seven of each in flight per lane.  17 us at 100 k rows x 27 offsets; one probe chain per thread in a
+// table of voxels took 14.5 us for half of the offsets, a table of voxels probed like this 116 us.
+constexpr int kLookupRows = 64, kLookupChunk = 28;
+template <bool NEAR>
+__global__ __launch_bounds__(256) void kmap_lookup_kernel(LookupArgs a, Offsets offs) {
+  constexpr int kMine = kLookupChunk / 4;
+  __shared__ int32_t found[kLookupRows][kLookupChunk + 1];
+  __shared__ unsigned long long wave_mask[4][kLookupRows];
+  __shared__ int32_t near_rep[8][kLookupRows];
+  if (blockIdx.x == gridDim.x - 1) {
+    publish_coordinates(a.flags, a.host);
+    return;
   }
-  const unsigned long long b = __ballot(hit >= 0);
-  if (threadIdx.x % 64 == 0 && b) atomicAdd(&block_hits, __builtin_popcountll(b));
-  __syncthreads();
-  if (threadIdx.x == 0) counts[(size_t)k * gridDim.x + blockIdx.x] = block_hits;
-}
-
-// grid (blocks of 256 output rows, offsets from k_first on): counts[k * n_blocks + block] =
-// entries >= 0 of the block.
-__global__ __launch_bounds__(kBlock) void kmap_count_kernel(const int32_t *__restrict__ table, int n_out,
-                                                            int k_first, int32_t *__restrict__ counts) {
-  __shared__ int block_hits;
-  const int k = k_first + blockIdx.y, o = blockIdx.x * kBlock + threadIdx.x;
-  if (threadIdx.x == 0) block_hits = 0;
-  __syncthreads();
-  const bool hit = o < n_out && table[(size_t)k * n_out + o] >= 0;
-  const unsigned long long b = __ballot(hit);
-  if (threadIdx.x % 64 == 0 && b) atomicAdd(&block_hits, __builtin_popcountll(b));
-  __syncthreads();
-  if (threadIdx.x == 0) counts[(size_t)k * gridDim.x + blockIdx.x] = block_hits;
-}
-
-__global__ __launch_bounds__(kBlock) void kmap_write_kernel(
-    const int32_t *__restrict__ table, int n_out, const int32_t *__restrict__ bases,
-    int32_t *__restrict__ in_map, int32_t *__restrict__ out_map, long long capacity) {
-  __shared__ int wave_hits[kBlock / 64];
-  const int k = blockIdx.y, o = blockIdx.x * kBlock + threadIdx.x;
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-  const int hit = o < n_out ? table[(size_t)k * n_out + o] : -1;
-  const unsigned long long b = __ballot(hit >= 0);
-  if (lane == 0) wave_hits[wave] = __builtin_popcountll(b);
+  const int o = blockIdx.x * kLookupRows + lane;
+  const bool live = o < a.n_out;
+  const int oc = live ? o : a.n_out - 1;
+  const long long lx = (long long)a.out_coords[3 * oc] * a.stride, ly = (long long)a.out_coords[3 * oc + 1] * a.stride,
+                  lz = (long long)a.out_coords[3 * oc + 2] * a.stride;
+  constexpr long long kFar = 1 << 30;          // (offsets are below it as well: sums stay in 32 bits)
+  const bool sane = live && lx > -kFar && lx < kFar && ly > -kFar && ly < kFar && lz > -kFar && lz < kFar;
+  const int x0 = sane ? (int)lx : 0, y0 = sane ? (int)ly : 0, z0 = sane ? (int)lz : 0;
+  const int block = blockIdx.x * kLookupRows / kListRows;
+  if constexpr (NEAR) {
+    // block j of a row: the row's own (bits 0) or the nearer neighbour along x (bit 2), y (bit 1), z (bit 0)
+    int bx[2], by[2], bz[2], rep[2];
+    bool want[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int j = wave * 2 + u;
+      const int zi = z0 & 3, dz = zi == 0 ? -1 : zi == 3 ? 1 : 0;
+      bx[u] = (x0 >> kBlockX) + (j & 4 ? ((x0 & 1) ? 1 : -1) : 0);
+      by[u] = (y0 >> kBlockY) + (j & 2 ? ((y0 & 1) ? 1 : -1) : 0);
+      bz[u] = (z0 >> kBlockZ) + (j & 1 ? dz : 0);
+      want[u] = sane && !((j & 1) && dz == 0);
+    }
+    find_blocks<2>(a, bx, by, bz, want, rep);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) near_rep[wave * 2 + u][lane] = rep[u];
+    __syncthreads();
+  }
+  unsigned long long mine = 0;
+  for (int k0 = 0; k0 < a.k_vol; k0 += kLookupChunk) {
+    int hit[kMine], rep[kMine], cell[kMine];
+    if constexpr (NEAR) {
+#pragma unroll
+      for (int u = 0; u < kMine; ++u) {
+        const int k = k0 + u * 4 + wave;
+        rep[u] = -1;
+        cell[u] = 0;
+        if (k < a.k_vol && k != a.skip_offset) {
+          const int *d = a.offsets ? a.offsets + 3 * k : offs.xyz + 3 * k;
+          const int x = x0 + d[0], y = y0 + d[1], z = z0 + d[2];
+          const int j = (x >> kBlockX != x0 >> kBlockX) << 2 | (y >> kBlockY != y0 >> kBlockY) << 1 | (z >> kBlockZ != z0 >> kBlockZ);
+          rep[u] = near_rep[j][lane];
+          cell[u] = cell_of(x, y, z);
+        }
+      }
+    } else {
+      int bx[kMine], by[kMine], bz[kMine];
+      bool want[kMine];
+#pragma unroll
+      for (int u = 0; u < kMine; ++u) {
+        const int k = k0 + u * 4 + wave;
+        want[u] = false;
+        bx[u] = by[u] = bz[u] = 0;
+        cell[u] = 0;
+        if (k < a.k_vol && k != a.skip_offset) {
+          const int *d = a.offsets ? a.offsets + 3 * k : offs.xyz + 3 * k;
+          const long long x = (long long)x0 + d[0], y = (long long)y0 + d[1], z = (long long)z0 + d[2];
+          want[u] = sane && x == (int)x && y == (int)y && z == (int)z;
+          bx[u] = (int)x >> kBlockX; by[u] = (int)y >> kBlockY; bz[u] = (int)z >> kBlockZ;
+          cell[u] = cell_of((int)x, (int)y, (int)z);
+        }
+      }
+      find_blocks<kMine>(a, bx, by, bz, want, rep);
+    }
+#pragma unroll
+    for (int u = 0; u < kMine; ++u) hit[u] = a.cells[(size_t)(rep[u] < 0 ? 0 : rep[u]) * kCells + cell[u]];
+#pragma unroll
+    for (int u = 0; u < kMine; ++u) {
+      const int k = k0 + u * 4 + wave;
+      if (k >= a.k_vol) break;
+      if (rep[u] < 0 || hit[u] == kNoRow) hit[u] = -1;
+      found[lane][k - k0] = hit[u];
+      const unsigned long long b = __ballot(hit[u] >= 0);
+      if (lane == 0 && b) atomicAdd(&a.counts[(size_t)k * a.blocks + block], __builtin_popcountll(b));
+      if (a.rmask_out && hit[u] >= 0) {
+        mine |= 1ull << k;
+        if (a.rmask_in)
+          (void)__hip_atomic_fetch_or(reinterpret_cast<unsigned *>(a.rmask_in + hit[u]) + (k >> 5), 1u << (k & 31),
+                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    __syncthreads();
+    // the chunk's part of every row, 16 bytes a thread
+    const int width = min(kLookupChunk, a.row_ld - k0) / 4;
+    for (int e = threadIdx.x; e < kLookupRows * width; e += 256) {
+      const int r = e / width, c = e % width * 4, row = blockIdx.x * kLookupRows + r;
+      if (row < a.n_out) {
+        int4v_ v;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = k0 + c + q < a.k_vol ? found[r][c + q] : -1;
+        *reinterpret_cast<int4v_ *>(a.rows + (size_t)row * a.row_ld + k0 + c) = v;
+      }
+    }
+    __syncthreads();
+  }
+  if (!a.rmask_out) return;
+  wave_mask[wave][lane] = mine;
   __syncthreads();
-  if (hit < 0) return;
-  long long pos = bases[(size_t)k * gridDim.x + blockIdx.x];
-  for (int w = 0; w < wave; ++w) pos += wave_hits[w];
-  pos += __builtin_popcountll(b & ((1ull << lane) - 1));
-  if (pos < capacity) {
-    in_map[pos] = hit;
-    out_map[pos] = o;
+  if (wave == 0 && live) a.rmask_out[o] = wave_mask[0][lane] | wave_mask[1][lane] | wave_mask[2][lane] | wave_mask[3][lane];
+}
+
+struct ScanArgs {
+  const int32_t *counts;      // [k_vol][blocks]
+  int32_t *bases;             // pairs before each of them, and the total behind
+  int k_vol, blocks;
+  int32_t *kernel_nnz, *kpos, *qkpos;      // (qkpos: nullptr: not wanted)
+  int *plan_flags;            // flags[12] of the plan: its pair count
+};
+
+// Exclusive prefix sum by one workgroup, 4096 values a round: every thread takes four neighbouring
+// values (the loads of a wave are contiguous; those of eight rounds are in flight together), the waves
+// scan their threads' sums with lane shuffles, the 16 wave totals go through LDS, and the sum of the
+// rounds so far is carried in a register.  The counts are few (offsets x 256-row blocks: 21 k for
+// 200 k voxels), so one workgroup is enough; its first wave then writes the per-offset tables.
+__global__ __launch_bounds__(1024) void kmap_scan_kernel(ScanArgs a) {
+  __shared__ int wave_totals[2][16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const size_t n = (size_t)a.k_vol * a.blocks;
+  constexpr int kAhead = 8;
+  int carry = 0, round = 0;
+  for (size_t base0 = 0; base0 < n; base0 += 4096 * kAhead) {
+    int v[kAhead][4];
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const size_t i = base0 + (size_t)q * 4096 + (size_t)tid * 4 + j;
+        v[q][j] = i < n ? a.counts[i] : 0;
+      }
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) {
+      const size_t i = base0 + (size_t)q * 4096 + (size_t)tid * 4;
+      if (base0 + (size_t)q * 4096 >= n) break;
+      const int mine = v[q][0] + v[q][1] + v[q][2] + v[q][3];
+      int incl = mine;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const int up = __shfl_up(incl, d, 64);
+        if (lane >= d) incl += up;
+      }
+      if (lane == 63) wave_totals[round][wave] = incl;
+      __syncthreads();      // the other buffer is written next round, after every wave has passed this barrier
+      int before = 0, total = 0;
+#pragma unroll
+      for (int w = 0; w < 16; ++w) {
+        const int t = wave_totals[round][w];
+        before += w < wave ? t : 0;
+        total += t;
+      }
+      int run = carry + before + incl - mine;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (i + j < n) a.bases[i + j] = run;
+        run += v[q][j];
+      }
+      carry += total;
+      round ^= 1;
+    }
+  }
+  if (tid == 0) a.bases[n] = carry;
+  __threadfence_block();
+  __syncthreads();
+  if (wave != 0) return;
+  int padded_before = 0;                       // (256-padded sizes of the offsets so far)
+  for (int k0 = 0; k0 < a.k_vol; k0 += 64) {
+    const int k = k0 + lane;
+    int size = 0;
+    if (k < a.k_vol) {
+      const int first = a.bases[(size_t)k * a.blocks];
+      size = a.bases[(size_t)(k + 1) * a.blocks] - first;
+      a.kpos[k] = first;
+      a.kernel_nnz[k] = size;
+    }
+    int padded = (size + 255) / 256 * 256;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int up = __shfl_up(padded, d, 64);
+      if (lane >= d) padded += up;
+    }
+    if (a.qkpos && k < a.k_vol) a.qkpos[k + 1] = padded_before + padded;
+    padded_before += __shfl(padded, 63, 64);
+  }
+  if (lane == 0) {
+    a.kpos[a.k_vol] = carry;
+    if (a.qkpos) a.qkpos[0] = 0;
+    if (a.plan_flags) a.plan_flags[12] = carry;
   }
 }
 
-// kpos[k] = first pair of offset k, kernel_nnz[k] = its size; total -> result[0]
-__global__ void kmap_finish_kernel(const int32_t *__restrict__ bases, int k_vol, int n_blocks,
-                                   int32_t *__restrict__ kernel_nnz, int32_t *__restrict__ kpos,
-                                   int32_t *__restrict__ result) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k > k_vol) return;
-  const int here = bases[(size_t)k * n_blocks];        // bases has k_vol * n_blocks + 1 entries
-  kpos[k] = here;
-  if (k < k_vol) kernel_nnz[k] = bases[(size_t)(k + 1) * n_blocks] - here;
-  if (k == k_vol) result[0] = here;
+struct ListArgs {
+  const int32_t *rows;
+  int n_out, k_vol, row_ld, blocks;
+  const int32_t *bases;
+  int32_t *in_map, *out_map;
+  long long capacity;
+  int32_t *band_start;        // of the plan, or nullptr
+  int cus;
+  const int32_t *kernel_nnz, *kpos;
+  const int *flags;           // nullptr: the lookup's launch has sent them
+  int *host;                  // pinned
+};
+
+// Workgroup 0 sends the sizes to the host.  Workgroups [1, list_blocks]: 256 output rows each, 28 offsets at a time through LDS; a wave takes
+// every fourth offset and ranks its hits with ballots.  The rest: the histogram of the plan's sort,
+// which needs the row masks only.
+__global__ __launch_bounds__(256) void kmap_lists_kernel(ListArgs a, SortArgs sort, int list_blocks) {
+  constexpr int kWidth = 28;
+  __shared__ int32_t tile[kListRows * (kWidth + 1) > kBins ? kListRows * (kWidth + 1) : kBins];
+  if (blockIdx.x == 0) {
+    if (threadIdx.x >= 64) return;
+    for (int k = threadIdx.x; k < min(a.k_vol, kHostInts - 16); k += 64) a.host[16 + k] = a.kernel_nnz[k];
+    if (threadIdx.x == 0) a.host[4] = a.kpos[a.k_vol];
+    __threadfence_system();
+    if (threadIdx.x == 0) __hip_atomic_store(&a.host[3], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (a.flags) publish_coordinates(a.flags, a.host);
+    return;
+  }
+  const int list_block = blockIdx.x - 1;
+  if (list_block >= list_blocks) {
+    const int b = list_block - list_blocks;
+    const int side = b < sort.side[0].chunks ? 0 : 1;
+    sort_hist_body(sort.side[side], sort.k_vol, side ? b - sort.side[0].chunks : b, tile, 256);
+    return;
+  }
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+  const int row0 = list_block * kListRows;
+  // bounds of the plan's row bands that fall into this block of rows (the last block has those behind
+  // it, too): what lies below them inside the block is in the ballots anyway
+  int bands = 0, band_rows = 1, c_first = 1, c_last = 0;
+  if (a.band_start) {
+    bands = band_count_of(a.kpos[a.k_vol], a.k_vol, a.cus);
+    band_rows = (a.n_out + bands - 1) / bands;
+    c_first = (row0 + band_rows - 1) / band_rows;
+    c_last = list_block + 1 == list_blocks ? bands : min(bands, (row0 + kListRows - 1) / band_rows);
+  }
+  for (int k0 = 0; k0 < a.k_vol; k0 += kWidth) {
+    const int width = min(kWidth, a.row_ld - k0) / 4;
+    for (int e = threadIdx.x; e < kListRows * width; e += 256) {
+      const int r = e / width, c = e % width * 4;
+      int4v_ v = {-1, -1, -1, -1};
+      if (row0 + r < a.n_out) v = *reinterpret_cast<const int4v_ *>(a.rows + (size_t)(row0 + r) * a.row_ld + k0 + c);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) tile[r * (kWidth + 1) + c + q] = v[q];
+    }
+    __syncthreads();
+    for (int k = k0 + wave; k < min(k0 + kWidth, a.k_vol); k += 4) {
+      const int block_first = a.bases[(size_t)k * a.blocks + list_block];
+      const int before = block_first - a.bases[(size_t)k * a.blocks];
+      long long pos = block_first;
+      unsigned long long hits[kListRows / 64];
+#pragma unroll
+      for (int q = 0; q < kListRows / 64; ++q) {
+        const int r = q * 64 + lane, hit = tile[r * (kWidth + 1) + k - k0];
+        const unsigned long long b = __ballot(hit >= 0);
+        if (hit >= 0) {
+          const long long at = pos + __builtin_popcountll(b & ((1ull << lane) - 1));
+          if (at < a.capacity) {
+            a.in_map[at] = hit;
+            a.out_map[at] = row0 + r;
+          }
+        }
+        pos += __builtin_popcountll(b);
+        hits[q] = b;
+      }
+      for (int c = c_first + lane; c <= c_last; c += 64) {
+        const long long end = (long long)c * band_rows - row0;      // rows of the block below the bound
+        int below = before;
+#pragma unroll
+        for (int q = 0; q < kListRows / 64; ++q) {
+          const long long r = end - q * 64;
+          below += __builtin_popcountll(r >= 64 ? hits[q] : r > 0 ? hits[q] & ((1ull << r) - 1) : 0ull);
+        }
+        a.band_start[k * (bands + 1) + c] = below;
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// Pinned read-back blocks, kept.
+std::mutex g_host_mutex;
+std::vector<int *> g_host_free;
+
+int *host_block_get() {
+  {
+    std::lock_guard<std::mutex> lock(g_host_mutex);
+    if (!g_host_free.empty()) {
+      int *q = g_host_free.back();
+      g_host_free.pop_back();
+      return q;
+    }
+  }
+  int *q = nullptr;
+  note_allocation();
+  if (hipHostMalloc((void **)&q, kHostInts * sizeof(int), hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) return nullptr;
+  return q;
+}
+
+void host_block_put(int *q) {
+  std::lock_guard<std::mutex> lock(g_host_mutex);
+  g_host_free.push_back(q);
+}
+
+// Waits for a kernel's word, or, if that takes long, for everything queued so far.
+int wait_for(volatile int *done, hipStream_t s) {
+  for (int spins = 0; !*done; ++spins) {
+    _mm_pause();
+    if (spins > (1 << 20)) {
+      FGMS_HIP_TRY(hipStreamSynchronize(s));
+      if (*done) break;
+      set_error("fgms_build_kernel_map: the build's kernels did not run");
+      return FGMS_E_HIP;
+    }
+  }
+  std::atomic_thread_fence(std::memory_order_acquire);
+  return FGMS_OK;
 }
 
 }  // namespace
 
-namespace {
-int build_kernel_map_impl(const int32_t *in_coords, int64_t n_in, const int32_t *out_coords, int64_t n_out,
-                          const int32_t *offsets_host, int k_vol, int stride, int skip_offset,
-                          int32_t *in_map, int32_t *out_map, int64_t capacity, int32_t *kernel_nnz,
-                          int32_t *kpos, int64_t *n_pairs, hipStream_t s, bool allow_mirror, bool *retry) {
-  *retry = false;
-  // A submanifold map (one coordinate list on both sides, symmetric offsets) is its own
-  // mirror image: half of the lookups give the other half (see kmap_lookup_kernel).
-  // FGMS_KMAP_MIRROR=0 looks every offset up.
-  static const bool mirror_on = !(getenv("FGMS_KMAP_MIRROR") && atoi(getenv("FGMS_KMAP_MIRROR")) == 0);
-  bool mirror = allow_mirror && mirror_on && in_coords == out_coords && n_in == n_out && stride == 1 &&
-                k_vol >= 3 && k_vol % 2 == 1 && (skip_offset < 0 || skip_offset == k_vol / 2);
+// A build whose sizes have not been asked for yet.
+struct MapBuild {
+  int *host;
+  hipStream_t stream;
+  int k_vol;
+  int64_t capacity, n_in, n_out;
+  const int32_t *kernel_nnz, *kpos, *in_map, *out_map;
+  Plan *plan;
+  bool plan_from_lists;       // more offsets than one plan's tables hold
+};
+
+int map_build_begin(MapBuild **build, const int32_t *in_coords, int64_t n_in, const int32_t *out_coords, int64_t n_out,
+                    const int32_t *offsets_host, int k_vol, int stride, int skip_offset,
+                    int32_t *in_map, int32_t *out_map, int64_t capacity, int32_t *kernel_nnz,
+                    int32_t *kpos, int32_t *qkpos, bool want_plan, bool allow_mirror, hipStream_t s) {
+  *build = nullptr;
+  {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (s && hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone) {
+      set_error("fgms_build_kernel_map: the stream is being captured (the build waits for its sizes)");
+      return FGMS_E_INVALID;
+    }
+  }
+  // the plan comes out of the same launches where its tables hold all offsets
+  const bool with_plan = want_plan && k_vol <= 64 && n_in > 0 && n_out > 0;
+  bool mirror = with_plan && allow_mirror && in_coords == out_coords && n_in == n_out && stride == 1 && k_vol % 2 == 1 &&
+                (skip_offset < 0 || skip_offset == k_vol / 2);
   for (int k = 0; mirror && k < k_vol; ++k)
     for (int c = 0; c < 3; ++c)
       if (offsets_host[3 * (k_vol - 1 - k) + c] != -offsets_host[3 * k + c]) mirror = false;
-  size_t slots = 64;
-  while (slots < 2 * (size_t)n_in) slots <<= 1;
-  const int n_blocks = (int)((n_out + kBlock - 1) / kBlock);
-  const size_t n_counts = (size_t)k_vol * n_blocks + 1;     // + one zero, so the scan ends with the total
 
-  std::vector<void *> tmp;
-  bool synced = false;      // true once the stream has drained
-  auto release = [&]() { for (void *q : tmp) pool_free(q, s, synced); tmp.clear(); };
-  auto alloc = [&](size_t bytes) -> void * {
-    void *q = nullptr;
-    if (pool_alloc(&q, bytes, s) != FGMS_OK) return nullptr;
-    tmp.push_back(q);
-    return q;
-  };
-  auto *keys = (unsigned long long *)alloc(slots * sizeof(unsigned long long));
-  auto *vals = (int32_t *)alloc(slots * sizeof(int32_t));
-  auto *table = (int32_t *)alloc((size_t)k_vol * (n_out ? n_out : 1) * sizeof(int32_t));
-  auto *counts = (int32_t *)alloc(n_counts * sizeof(int32_t));
-  auto *bases = (int32_t *)alloc(n_counts * sizeof(int32_t));
-  auto *offs = (int32_t *)alloc((size_t)k_vol * 3 * sizeof(int32_t));
-  auto *flags = (int32_t *)alloc(4 * sizeof(int32_t));      // [0] bad coordinate, [1] total
-  const bool ok = keys && vals && table && counts && bases && offs && flags;
-  if (!ok) {
-    release();
-    set_error("fgms_build_kernel_map: temporary allocation failed");
-    return FGMS_E_NOMEM;
-  }
-  const unsigned long long mask = slots - 1;
+  size_t slots = 256;
+  while (slots < 2 * (size_t)n_in) slots <<= 1;
+  const int blocks = (int)((n_out + kListRows - 1) / kListRows);
+  const int row_ld = (k_vol + 3) / 4 * 4;
+  const size_t n_counts = (size_t)k_vol * blocks;
+
   int rc = FGMS_OK;
-  auto fail = [&](const char *what) {
-    synced = hipStreamSynchronize(s) == hipSuccess;
-    release();
-    set_error("fgms_build_kernel_map: %s", what);
-    return FGMS_E_HIP;
+  Plan *p = with_plan ? plan_alloc(k_vol, n_in, n_out, 0, s) : nullptr;
+  if (with_plan && !p) return FGMS_E_NOMEM;
+  SortArgs sort{};
+  sort.k_vol = k_vol;
+  int cap_out = 0, cap_in = 0;
+  const int tiles_out = with_plan ? tile_table(n_out, &cap_out) : 0, tiles_in = with_plan ? tile_table(n_in, &cap_in) : 0;
+  const size_t so = (size_t)n_out * k_vol, si = mirror ? 0 : (size_t)n_in * k_vol;
+  int32_t *slot_table = nullptr, *cells = nullptr, *rows = nullptr, *counts = nullptr, *bases = nullptr, *offs_dev = nullptr, *flags = nullptr;
+  unsigned long long *rmask_out = nullptr, *rmask_in = nullptr;
+  void *scratch = nullptr;
+  auto layout = [&](Arena &keep, Arena &tmp) {
+    tmp.take(slot_table, slots);
+    tmp.take(cells, (size_t)n_in * kCells);
+    tmp.take(rows, (size_t)n_out * row_ld);
+    tmp.take(flags, 64);
+    tmp.take(counts, n_counts);                     // (behind the flags: one fill)
+    tmp.take(bases, n_counts + 1);
+    if (k_vol > kKernargOffsets) tmp.take(offs_dev, (size_t)k_vol * 3);
+    if (!with_plan) return;
+    tmp.take(rmask_out, (size_t)n_out);
+    if (!mirror) tmp.take(rmask_in, (size_t)n_in);
+    sort_side_layout(sort.side[0], n_out, tmp);
+    if (!mirror) sort_side_layout(sort.side[1], n_in, tmp);
+    keep.take(p->flags, kPlanFlags);
+    keep.take(p->band_start, (size_t)k_vol * (64 + 1));          // (the band count follows from the pair count)
+    keep.take(p->band_cells, (size_t)4 * k_vol * 64);
+    keep.take(p->nbr_out, so);
+    if (!mirror) keep.take(p->nbr_in, si);
+    keep.take(p->mask_out, (size_t)(n_out + 63) / 64);
+    keep.take(p->perm_out, (size_t)n_out);
+    if (!mirror) keep.take(p->mask_in, (size_t)(n_in + 63) / 64);
+    if (!mirror) keep.take(p->perm_in, (size_t)n_in);
+    if (tiles_out) keep.take(p->tile_out, (size_t)cap_out * 8);
+    if (tiles_in && !mirror) keep.take(p->tile_in, (size_t)cap_in * 8);
   };
-  if (hipMemcpyAsync(offs, offsets_host, (size_t)k_vol * 3 * sizeof(int32_t), hipMemcpyHostToDevice, s) != hipSuccess)
-    return fail("copying the offsets failed");
-  if ((rc = launch_fill_zero(flags, 4 * sizeof(int32_t), s)) || (rc = launch_fill_zero(counts, n_counts * sizeof(int32_t), s))) {
-    synced = hipStreamSynchronize(s) == hipSuccess;
-    release();
-    return rc;
+  int *host = host_block_get(), *host_dev = nullptr;
+  auto fail = [&](int code) {
+    (void)hipStreamSynchronize(s);
+    if (scratch) pool_free(scratch, s, true);
+    if (p) fgms_plan_destroy((fgms_plan_t *)p);
+    if (host) host_block_put(host);
+    return code;
+  };
+  if (!host || hipHostGetDevicePointer((void **)&host_dev, host, 0) != hipSuccess) {
+    set_error("fgms_build_kernel_map: pinned allocation failed");
+    return fail(FGMS_E_NOMEM);
   }
-  kmap_fill_kernel<<<(unsigned)((slots + 255) / 256), 256, 0, s>>>(keys, vals, slots);
-  if (n_in > 0) {
-    ProfileScope prof("kmap_insert_kernel", s);
-    kmap_insert_kernel<<<(unsigned)((n_in + 255) / 256), 256, 0, s>>>(in_coords, (int)n_in, keys, vals, mask, flags);
+  host[0] = host[3] = 0;
+  {
+    Arena keep, tmp;
+    layout(keep, tmp);
+    if ((rc = pool_alloc(&scratch, tmp.used, s)) || (p && (rc = pool_alloc(&p->block, keep.used, s)))) return fail(rc);
+    Arena keep_at, tmp_at;
+    keep_at.base = p ? (char *)p->block : nullptr;
+    tmp_at.base = (char *)scratch;
+    layout(keep_at, tmp_at);
   }
-  if (n_out > 0) {
-    {
-      ProfileScope prof("kmap_lookup_kernel", s);
-      if (mirror) {
-        const size_t half = (size_t)(k_vol / 2) * n_out;     // the offsets after the centre
-        size_t blocks = (half + 1023) / 1024;
-        kmap_fill_none_kernel<<<(unsigned)(blocks > 65535 ? 65535 : blocks), 256, 0, s>>>(
-            table + (size_t)(k_vol / 2 + 1) * n_out, half);
-      }
-      kmap_lookup_kernel<<<dim3((unsigned)n_blocks, (unsigned)(mirror ? k_vol / 2 + 1 : k_vol)), kBlock, 0, s>>>(
-          out_coords, (int)n_out, offs, stride, skip_offset, keys, vals, mask, table, counts, mirror ? k_vol : 0);
-      if (mirror)
-        kmap_count_kernel<<<dim3((unsigned)n_blocks, (unsigned)(k_vol / 2)), kBlock, 0, s>>>(table, (int)n_out,
-                                                                                            k_vol / 2 + 1, counts);
+  if (p) {
+    p->kpos = kpos; p->in_map = in_map; p->out_map = out_map;
+    p->has_tables = true;
+    p->has_bands = true;
+    if (mirror) {
+      p->perm_in = p->perm_out;
+      p->nbr_in = p->nbr_out;
+      p->mask_in = p->mask_out;
+      p->tile_in = p->tile_out;
+      p->flip_in = k_vol - 1;
+    }
+    p->tile_grid_out = p->tile_out ? cap_out * 8 : 0;
+    p->tile_grid_in = p->tile_in ? cap_in * 8 : 0;
+    sort.flags = p->flags;
+    sort.side[0].rmask = rmask_out; sort.side[0].perm = p->perm_out; sort.side[0].block_mask = p->mask_out;
+    if (!mirror) {
+      sort.side[1].rmask = rmask_in; sort.side[1].perm = p->perm_in; sort.side[1].block_mask = p->mask_in;
     }
   }
-  kmap_scan_kernel<<<1, 1024, 0, s>>>(counts, bases, n_counts);
-  if (n_out > 0) {
+  FillBatch fills{};
+  fills.add(slot_table, slots * sizeof(int32_t), -1);
+  fills.add(cells, (size_t)n_in * kCells * sizeof(int32_t), kNoRow);
+  fills.add(flags, (size_t)((char *)(counts + n_counts) - (char *)flags), 0);
+  if (p) {
+    fills.add(p->flags, kPlanFlags * sizeof(int), 0);
+    if (!mirror) {
+      fills.add(rmask_in, (size_t)n_in * sizeof(unsigned long long), 0);
+      fills.add(p->nbr_in, si * sizeof(int32_t), -1);
+    }
+  }
+  Offsets offs;
+  if (offs_dev) {
+    if (hipMemcpyAsync(offs_dev, offsets_host, (size_t)k_vol * 3 * sizeof(int32_t), hipMemcpyHostToDevice, s) != hipSuccess) {
+      set_error("fgms_build_kernel_map: copying the offsets failed");
+      return fail(FGMS_E_HIP);
+    }
+  } else {
+    memcpy(offs.xyz, offsets_host, (size_t)k_vol * 3 * sizeof(int32_t));
+  }
+  if ((rc = launch_fills(fills, s))) return fail(rc);
+  const unsigned mask = (unsigned)(slots - 1);
+  if (n_in > 0) {
+    ProfileScope prof("kmap_insert_kernel", s);
+    kmap_insert_kernel<<<(unsigned)((n_in + 255) / 256), 256, 0, s>>>(in_coords, (int)n_in, slot_table, mask, cells, flags);
+  }
+  if (n_out > 0 && n_in > 0) {
+    ProfileScope prof("kmap_lookup_kernel", s);
+    LookupArgs la{in_coords, out_coords, (int)n_out, k_vol, stride, skip_offset, row_ld, slot_table, cells, mask, offs_dev,
+                  rows, counts, blocks, rmask_out, rmask_in, flags, host_dev};
+    bool near = true;
+    for (int q = 0; q < 3 * k_vol; ++q) near = near && offsets_host[q] >= -1 && offsets_host[q] <= 1;
+    auto kern = near ? kmap_lookup_kernel<true> : kmap_lookup_kernel<false>;
+    kern<<<(unsigned)((n_out + kLookupRows - 1) / kLookupRows) + 1, 256, 0, s>>>(la, offs);
+  }
+  {
+    ScanArgs sc{counts, bases, k_vol, blocks, kernel_nnz, kpos, qkpos, p ? p->flags : nullptr};
+    kmap_scan_kernel<<<1, 1024, 0, s>>>(sc);
+  }
+  {
     ProfileScope prof("kmap_write_kernel", s);
-    kmap_write_kernel<<<dim3((unsigned)n_blocks, (unsigned)k_vol), kBlock, 0, s>>>(
-        table, (int)n_out, bases, in_map, out_map, (long long)capacity);
+    ListArgs la{rows, (int)n_out, k_vol, row_ld, blocks, bases, in_map, out_map, (long long)capacity, p ? p->band_start : nullptr, num_cus(),
+                kernel_nnz, kpos, n_out > 0 && n_in > 0 ? nullptr : flags, host_dev};
+    const int hist_blocks = p ? sort.side[0].chunks + sort.side[1].chunks : 0;
+    const int list_blocks = n_in > 0 ? blocks : 0;
+    kmap_lists_kernel<<<(unsigned)(1 + list_blocks + hist_blocks), 256, 0, s>>>(la, sort, list_blocks);
   }
-  kmap_finish_kernel<<<(unsigned)((k_vol + 1 + 255) / 256), 256, 0, s>>>(bases, k_vol, n_blocks, kernel_nnz, kpos, flags + 1);
-  if (hipGetLastError() != hipSuccess) return fail("kernel launch failed");
-  int32_t h[3] = {0, 0, 0};
-  if (hipMemcpyAsync(h, flags, sizeof(h), hipMemcpyDeviceToHost, s) != hipSuccess ||
-      hipStreamSynchronize(s) != hipSuccess)
-    return fail("reading the result size failed");
-  synced = true;
-  release();
-  if (mirror && h[2] && !h[0]) {       // rows that share coordinates: every offset has to be looked up
-    *retry = true;
-    return FGMS_OK;
+  if (hipGetLastError() != hipSuccess) {
+    set_error("fgms_build_kernel_map: a kernel launch failed");
+    return fail(FGMS_E_HIP);
   }
-  if (h[0]) {
+  if (p && (rc = launch_sort(sort, true, s))) return fail(rc);
+  if (p) {
+    TablesArgs ta{};
+    p->n_pairs = (int64_t)k_vol * n_out;         // (a bound; the count is known to the device only)
+    plan_fill_tables_args(p, &ta);
+    ta.rows = rows;
+    ta.bands = 0;
+    ta.bands_known = true;
+    ta.row_ld = row_ld;
+    ta.perm_out = p->perm_out;
+    ta.nbr_out = p->nbr_out;
+    if (!mirror) {
+      ta.nbr_in = p->nbr_in;
+      ta.inv_in = sort.side[1].inv;
+    }
+    ta.mirror = mirror;
+    ta.take_print = true;
+    if ((rc = launch_tables(ta, s)) || (rc = plan_publish(p, ta.host != nullptr, s))) return fail(rc);
+  }
+  // (the launches above are the longer way: the insertion's findings have arrived by now)
+  if ((rc = wait_for(host, s))) return fail(rc);
+  if (host[1]) {
     set_error("fgms_build_kernel_map: an input coordinate is outside [-2^20, 2^20)");
-    return FGMS_E_INVALID;
+    return fail(FGMS_E_INVALID);
   }
-  *n_pairs = h[1];
-  if (h[1] > capacity) {
-    set_error("fgms_build_kernel_map: %d pairs do not fit the capacity of %lld", h[1], (long long)capacity);
-    return FGMS_E_INVALID;
+  if (mirror && host[2]) {         // rows that share coordinates: the map is not its own mirror image
+    (void)fail(FGMS_OK);
+    return map_build_begin(build, in_coords, n_in, out_coords, n_out, offsets_host, k_vol, stride, skip_offset, in_map, out_map,
+                           capacity, kernel_nnz, kpos, qkpos, want_plan, false, s);
   }
+  pool_free(scratch, s, false);
+  *build = new MapBuild{host, s, k_vol, capacity, n_in, n_out, kernel_nnz, kpos, in_map, out_map, p,
+                        want_plan && !p && n_in > 0 && n_out > 0};
   return FGMS_OK;
 }
-}  // namespace
 
-int build_kernel_map(const int32_t *in_coords, int64_t n_in, const int32_t *out_coords, int64_t n_out,
-                     const int32_t *offsets_host, int k_vol, int stride, int skip_offset,
-                     int32_t *in_map, int32_t *out_map, int64_t capacity, int32_t *kernel_nnz,
-                     int32_t *kpos, int64_t *n_pairs, hipStream_t s) {
-  bool retry = false;
-  int rc = build_kernel_map_impl(in_coords, n_in, out_coords, n_out, offsets_host, k_vol, stride, skip_offset,
-                                 in_map, out_map, capacity, kernel_nnz, kpos, n_pairs, s, true, &retry);
-  if (rc == FGMS_OK && retry)
-    rc = build_kernel_map_impl(in_coords, n_in, out_coords, n_out, offsets_host, k_vol, stride, skip_offset,
-                               in_map, out_map, capacity, kernel_nnz, kpos, n_pairs, s, false, &retry);
+// Waits for the build and takes it apart.
+int map_build_end(MapBuild *b, int32_t *host_nnz, int64_t *n_pairs, fgms_plan_t **plan_out) {
+  if (plan_out) *plan_out = nullptr;
+  // (for the whole build: lists and tables can then be read on any stream)
+  int rc = FGMS_OK;
+  if ((b->plan ? hipEventSynchronize(b->plan->ready) : hipStreamSynchronize(b->stream)) != hipSuccess || !*(volatile int *)(b->host + 3)) {
+    set_error("fgms_build_kernel_map: the build failed");
+    rc = FGMS_E_HIP;
+  }
+  const int pairs = rc == FGMS_OK ? b->host[4] : 0;
+  if (rc == FGMS_OK) {
+    *n_pairs = pairs;
+    if (host_nnz) {
+      if (b->k_vol <= kHostInts - 16) {
+        memcpy(host_nnz, b->host + 16, (size_t)b->k_vol * sizeof(int));
+      } else if (hipMemcpyAsync(host_nnz, b->kernel_nnz, (size_t)b->k_vol * sizeof(int), hipMemcpyDeviceToHost, b->stream) != hipSuccess ||
+                 hipStreamSynchronize(b->stream) != hipSuccess) {
+        set_error("fgms_build_kernel_map: reading the sizes failed");
+        rc = FGMS_E_HIP;
+      }
+    }
+    if (pairs > b->capacity) {
+      set_error("fgms_build_kernel_map: %d pairs do not fit the capacity of %lld", pairs, (long long)b->capacity);
+      rc = FGMS_E_INVALID;
+    }
+  }
+  if (rc == FGMS_OK && b->plan) {
+    b->plan->n_pairs = pairs;
+    plan_bands(b->plan);
+    if (plan_out) {
+      *plan_out = (fgms_plan_t *)b->plan;
+      b->plan = nullptr;
+    }
+  } else if (rc == FGMS_OK && b->plan_from_lists && plan_out) {
+    rc = plan_create(plan_out, b->kpos, b->in_map, b->out_map, b->n_in, b->n_out, b->k_vol, pairs, b->stream, true);
+  }
+  if (b->plan) fgms_plan_destroy((fgms_plan_t *)b->plan);
+  host_block_put(b->host);
+  delete b;
   return rc;
 }
 

@@ -530,7 +530,7 @@ __device__ __forceinline__ void gms_rows_body(
     const int32_t *__restrict__ nbr, const unsigned long long *__restrict__ block_masks,
     const int32_t *__restrict__ perm, const int32_t *__restrict__ tile_order, int n_dst, int k_vol,
     int c_src, int c_dst, int part_stages, int block_x, int block_y, int block_z, int grid_z,
-    unsigned src_bytes, int pair_view, int overwrite, int nbr_stride) {
+    unsigned src_bytes, int pair_view, int overwrite, int flip) {
   constexpr int E = Elem<T>::per_chunk;
   constexpr int C = 2 * S;
   // 16-bit matrix instructions (fp16 tensors, fp32 tensors in split bf16): rows and weights come
@@ -543,7 +543,7 @@ __device__ __forceinline__ void gms_rows_body(
   auto row_offset = [&](int g) { return !kBuf ? (unsigned)g : g < 0 ? kAbsentRow : (unsigned)g * row_bytes; };
   // pair view: `nbr` is one list of source rows for all offsets (a 64-row block belongs to
   // the one offset its mask names), `perm` the destination rows; results are added atomically
-  // (nbr_stride: entries from one offset's row of the table to the next one's; 0 for a pair view)
+  const size_t nbr_stride = pair_view ? 0 : (size_t)n_dst;
   constexpr int WCH = S * NT * 64;                        // 16-byte chunks of one stage's weights
   constexpr int NW = (WCH + kThreads - 1) / kThreads;     // ... per thread
   extern __shared__ int4v lds[];
@@ -584,7 +584,7 @@ __device__ __forceinline__ void gms_rows_body(
   // start of a launch every workgroup walks this chain of dependent loads at the same time
   // and nothing else covers it (0.4 us of a 46 us launch)
   int g_first = -1;
-  if (k_first >= 0 && in_range) g_first = nbr[(ptrdiff_t)k_first * nbr_stride + my_row];
+  if (k_first >= 0 && in_range) g_first = nbr[(size_t)k_first * nbr_stride + my_row];
   if (owns_row) didx[lane] = in_range ? (perm ? perm[my_row] : my_row) : -1;   // my_row is a position in the plan's row order
 
   // which offsets touch this wave's rows / this workgroup's rows (from the plan)
@@ -660,7 +660,9 @@ __device__ __forceinline__ void gms_rows_body(
     else if constexpr (RAW == 3) wvoff[i] = (unsigned)(((e / (NT * 128)) * nts * 128 + e % (NT * 128)) * 16);
     else wvoff[i] = (unsigned)(((e / (NT * 64)) * nts * 64 + e % (NT * 64)) * 16);
   }
-  auto weights_issue = [&](int4v (&wreg)[NW], int k, int slab) {
+  // (flip: the tables number the offsets from the other end, see Plan)
+  auto weights_issue = [&](int4v (&wreg)[NW], int k_, int slab) {
+    const int k = flip ? flip - k_ : k_;
     if constexpr (!kBuf) {
 #pragma unroll
       for (int i = 0; i < NW; ++i) {
@@ -730,8 +732,8 @@ __device__ __forceinline__ void gms_rows_body(
   };
 
   // prologue: stage 0 goes straight to LDS
-  if (owns_row) goff[lane] = row_offset(k_first >= 0 ? g_first : (in_range ? nbr[(ptrdiff_t)k * nbr_stride + my_row] : -1));
-  int g_nxt = (k_nxt >= 0 && in_range) ? nbr[(ptrdiff_t)k_nxt * nbr_stride + my_row] : -1;
+  if (owns_row) goff[lane] = row_offset(k_first >= 0 ? g_first : (in_range ? nbr[(size_t)k * nbr_stride + my_row] : -1));
+  int g_nxt = (k_nxt >= 0 && in_range) ? nbr[(size_t)k_nxt * nbr_stride + my_row] : -1;
   wave_lds_fence();
   weights_issue(wreg, k, 0);
   if (active) rows_issue(0);
@@ -771,7 +773,7 @@ __device__ __forceinline__ void gms_rows_body(
     // (nothing of the prologue is in flight any more; said explicitly, because the compiler
     // cannot tell from the prologue's branches and would wait for loads that never were issued)
     __builtin_amdgcn_s_waitcnt(0x0F70);      // vmcnt(0)
-    if (k2 >= 0) g_nxt = nbr[(ptrdiff_t)k2 * nbr_stride + safe_row];
+    if (k2 >= 0) g_nxt = nbr[(size_t)k2 * nbr_stride + safe_row];
     int slot = 0;
     // One pass of the loop per stage that has a successor: request the successor's weights and
     // rows, multiply this stage, move the successor to LDS; the last stage's products follow
@@ -792,7 +794,7 @@ __device__ __forceinline__ void gms_rows_body(
         wave_lds_fence();
         k3 = todo ? __builtin_ctzll(todo) : -1;
         if (todo) todo &= todo - 1;
-        if (k3 >= 0) g_nxt = nbr[(ptrdiff_t)k3 * nbr_stride + safe_row];
+        if (k3 >= 0) g_nxt = nbr[(size_t)k3 * nbr_stride + safe_row];
       }
       if (active) mma_stage();
       wave_lds_fence();
@@ -871,7 +873,7 @@ __device__ __forceinline__ void gms_rows_body(
       if (nk != k) {
         k_nxt = todo ? __builtin_ctzll(todo) : -1;
         if (todo) todo &= todo - 1;
-        g_nxt = (k_nxt >= 0 && in_range) ? nbr[(ptrdiff_t)k_nxt * nbr_stride + my_row] : -1;
+        g_nxt = (k_nxt >= 0 && in_range) ? nbr[(size_t)k_nxt * nbr_stride + my_row] : -1;
       }
       __syncthreads();
       buf ^= 1;
@@ -897,7 +899,7 @@ __global__ __launch_bounds__(kThreads, MT == 1 ? 4 : (NT == 4 ? 2 : 3)) void gms
     const int32_t *__restrict__ nbr, const unsigned long long *__restrict__ block_masks,
     const int32_t *__restrict__ perm, const int32_t *__restrict__ tile_order, int n_dst, int k_vol,
     int c_src, int c_dst, int part_stages, SideJob side, int pair_view, unsigned src_bytes, int overwrite,
-    int nbr_stride) {
+    int flip) {
   // the leading workgroups of the grid run the side job, if there is one
   int block_x = blockIdx.x;
   if (side.blocks) {
@@ -909,7 +911,7 @@ __global__ __launch_bounds__(kThreads, MT == 1 ? 4 : (NT == 4 ? 2 : 3)) void gms
   }
   gms_rows_body<T, NT, S, RAW, MT>(src, packed, dst, nbr, block_masks, perm, tile_order, n_dst, k_vol, c_src,
                                    c_dst, part_stages, block_x, blockIdx.y, blockIdx.z, gridDim.z, src_bytes, pair_view,
-                                   overwrite, nbr_stride);
+                                   overwrite, flip);
 }
 
 // ---------------------------------------------------------------------------
@@ -1087,7 +1089,7 @@ bool raw_weights_enabled() {
 template <typename T, int NT, int S>
 int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
                 const unsigned long long *masks, const int32_t *perm, const int32_t *tile_order,
-                int tile_grid, int nbr_stride, bool pair_view = false) {
+                int tile_grid, int flip, bool pair_view = false) {
   // With 64-column wave tiles the input gradient and the fp16 forward pass read the weight
   // tensor as it is (16-byte aligned rows of the tile) when the caller brings no re-laid
   // copy; the rest gets one, made here.  Measured: 64 -> 64 over 200k voxels, input gradient
@@ -1161,7 +1163,7 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
     kern<<<dim3(gx + (unsigned)a.side.blocks, gy, gz), kThreads, lds_rows, a.stream>>>(
         (const T *)a.src, packed, (T *)a.dst, nbr, masks, perm, tile_order, (int)a.n_dst, a.k_vol,
         s.c_src, s.c_dst, part_stages > 0 ? part_stages : 1, a.side, pair_view ? 1 : 0,
-        (unsigned)((size_t)a.n_src * s.c_src * sizeof(T)), overwrite ? 1 : 0, nbr_stride);
+        (unsigned)((size_t)a.n_src * s.c_src * sizeof(T)), overwrite ? 1 : 0, flip);
   }
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;
@@ -1190,7 +1192,7 @@ __global__ __launch_bounds__(kThreads, NT == 4 || BI * BJ == 16 ? 2 : 3) void bw
     int c_in, int c_out, int part_stages, const T *__restrict__ in, float *__restrict__ gw32,
     const int32_t *__restrict__ kpos, const int32_t *__restrict__ imap,
     const int32_t *__restrict__ omap, SliceMap smap, int row_x, int row_y, int row_z, int wgrad_x,
-    unsigned gout_bytes, unsigned in_bytes, int wgrad_blocks, SideJob check, int overwrite, int nbr_stride) {
+    unsigned gout_bytes, unsigned in_bytes, int wgrad_blocks, SideJob check, int overwrite, int flip) {
   // grid: row_x * row_y * row_z workgroups of the input gradient (tiles, column tiles,
   // parts of a tile), then wgrad_x * (tiles of dW[k]) of the weight gradient, then those of a
   // side job (the plan's fingerprint check), if there is one
@@ -1202,7 +1204,7 @@ __global__ __launch_bounds__(kThreads, NT == 4 || BI * BJ == 16 ? 2 : 3) void bw
   if ((int)blockIdx.x < rows_total) {
     const int bx = blockIdx.x % row_x, rest = blockIdx.x / row_x;
     gms_rows_body<T, NT, S, RAWD, MT>(gout, w, gin, nbr, block_masks, perm, tile_order, n_in, k_vol, c_out, c_in,
-                                      part_stages, bx, rest % row_y, rest / row_y, row_z, gout_bytes, 0, overwrite, nbr_stride);
+                                      part_stages, bx, rest % row_y, rest / row_y, row_z, gout_bytes, 0, overwrite, flip);
   } else {
     const int j = blockIdx.x - rows_total;
     if constexpr (BI <= 2 && BJ <= 2)
@@ -1261,7 +1263,7 @@ int launch_fused(const GmsArgs &d, const Shape &s, const Plan *p, const WgradArg
         (int)d.n_dst, d.k_vol, d.c_in, d.c_out, part_stages, (const T *)w.in, acc32, w.kpos, w.imap, w.omap,
         g.smap, (int)row_x, (int)row_y, (int)row_z, (int)g.tiles,
         (unsigned)((size_t)d.n_src * s.c_src * sizeof(T)), (unsigned)((size_t)w.n_in * w.c_in * sizeof(T)),
-        (int)(g.tiles * g.ty), check, d.overwrite && rg.gz == 1 ? 1 : 0, p->nbr_stride_in);
+        (int)(g.tiles * g.ty), check, d.overwrite && rg.gz == 1 ? 1 : 0, p->flip_in);
   }
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;
@@ -1447,7 +1449,7 @@ int launch_planned_gms(const GmsArgs &a, const Plan *p) {
   const int32_t *perm = a.transpose_w ? p->perm_in : p->perm_out;
   const int32_t *tile_order = a.transpose_w ? p->tile_in : p->tile_out;
   const int tile_grid = a.transpose_w ? p->tile_grid_in : p->tile_grid_out;
-  const int nbr_stride = a.transpose_w ? p->nbr_stride_in : p->nbr_stride_out;
+  const int flip = a.transpose_w ? p->flip_in : p->flip_out;
   // (a pending fingerprint check of the plan rides along as the launch's side job)
   GmsArgs with_check = a;
   if (!with_check.side.kind) (void)plan_take_check(p, &with_check.side);
@@ -1455,11 +1457,11 @@ int launch_planned_gms(const GmsArgs &a, const Plan *p) {
   if (a.dtype == FGMS_F16)
     return dispatch_rows_shape<__half>(s, [&](auto nt, auto sv) {
       return launch_rows<__half, decltype(nt)::value, decltype(sv)::value>(a_, s, nbr, masks, perm, tile_order, tile_grid,
-                                                                              nbr_stride);
+                                                                              flip);
     });
   return dispatch_rows_shape<float>(s, [&](auto nt, auto sv) {
     return launch_rows<float, decltype(nt)::value, decltype(sv)::value>(a_, s, nbr, masks, perm, tile_order, tile_grid,
-                                                                              nbr_stride);
+                                                                              flip);
   });
 }
 

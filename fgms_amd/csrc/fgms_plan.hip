@@ -45,7 +45,8 @@ __global__ __launch_bounds__(256) void fills_kernel(FillBatch batch) {
 __global__ void pair_masks_kernel(const int32_t *__restrict__ kpos, const int32_t *__restrict__ imap,
                                   const int32_t *__restrict__ omap, int k_vol, int n_pairs, int n_in,
                                   int n_out, unsigned long long *__restrict__ rmask_out,
-                                  unsigned long long *__restrict__ rmask_in, int *__restrict__ flags) {
+                                  unsigned long long *__restrict__ rmask_in, int *__restrict__ flags,
+                                  int32_t *__restrict__ band_start, int bands, int band_rows) {
   const int total = kpos[k_vol];
   if (blockIdx.x < kPrintParts) {
     // the launch's first workgroups take the fingerprint of the lists (fgms_plan_check re-takes
@@ -67,7 +68,17 @@ __global__ void pair_masks_kernel(const int32_t *__restrict__ kpos, const int32_
     flags[0] = 1;
     return;
   }
-  if (j > kpos[k] && omap[j - 1] > o) flags[3] = 1;
+  const int before = j > kpos[k] ? omap[j - 1] : -1;
+  if (before > o) flags[3] = 1;
+  // the bounds of the weight gradient's row bands that fall between this pair and the one before it
+  // (pre-set to 0; meaningful where the pairs are ordered by output row, in bounds always)
+  if (band_start) {
+    int32_t *row = band_start + k * (bands + 1);
+    const int here = o / band_rows;
+    for (int c = before < 0 ? 0 : before / band_rows + 1; c <= here; ++c) row[c] = j - kpos[k];
+    if (j + 1 == min(min(kpos[k + 1], total), n_pairs))
+      for (int c = here + 1; c <= bands; ++c) row[c] = j + 1 - kpos[k];
+  }
   // the 32-bit half of the mask that holds bit k (little-endian words); the old value is not
   // asked for, so the atomics need no reply
   const unsigned bit = 1u << (k & 31);
@@ -87,7 +98,8 @@ __global__ void pair_masks_kernel(const int32_t *__restrict__ kpos, const int32_
 // every window of kWindow positions.  Inside a bin only rows of one window are ordered
 // among themselves; measured on the benchmark clouds that costs 1 % more (block, offset) steps
 // than the exact sort, for a third of its time.  (Bins of 16 bits without the windows: 4 % more
-// steps on surfaces, 23 % on scattered clouds.)  Both sides of a plan go through the same
+// steps on surfaces, 23 % on scattered clouds; windows of 2048: 0.3 % fewer steps on surfaces, 3 % on
+// scattered clouds, for twice the sort.)  Both sides of a plan go through the same
 // launches (blockIdx.y = side).
 __global__ __launch_bounds__(kSortThreads) void sort_hist_kernel(SortArgs a) {
   const SortSide &sd = a.side[blockIdx.y];
@@ -141,15 +153,15 @@ __device__ __forceinline__ unsigned long long lane_xor(unsigned long long v) {
   return (unsigned long long)lane_xor<J>((unsigned)v) | (unsigned long long)lane_xor<J>((unsigned)(v >> 32)) << 32;
 }
 
-// Bitonic sort of 2048 keys, ascending, by 1024 threads: wave w holds elements w * 128 ... in two
-// registers per lane (element w * 128 + r * 64 + lane in key[r]), so that 56 of the 66 phases are
-// register exchanges inside a wave (most of them on the vector ALUs alone) and only the 10 with
-// partners 128 or more apart go through LDS (`buf`: 2 x 2048 keys).  A bitonic sort with every
-// phase in LDS took 22 us for 2048 32-bit pairs where this takes 5.
+// Bitonic sort of kWindow keys, ascending, by kWindowThreads threads: wave w holds elements w * 128 ...
+// in two registers per lane (element w * 128 + r * 64 + lane in key[r]), so that 49 of the 55 phases
+// are register exchanges inside a wave (most of them on the vector ALUs alone) and only the 6 with
+// partners 128 or more apart go through LDS (`buf`: 2 x kWindow keys).  The vector ALUs are its
+// limit, hence small windows on many CUs: 2048 keys by 1024 threads took 13 us, with every phase in LDS 25.
 template <typename K, int K2, int J>
 __device__ __forceinline__ void bitonic_phases(K (&key)[2], K *buf, int base, int lane, int &flip) {
   if constexpr (J >= 128) {
-    K *to = buf + flip * 2048;
+    K *to = buf + flip * kWindow;
     flip ^= 1;
     to[base + lane] = key[0];
     to[base + 64 + lane] = key[1];
@@ -177,33 +189,42 @@ __device__ __forceinline__ void bitonic_phases(K (&key)[2], K *buf, int base, in
   if constexpr (J > 1) bitonic_phases<K, K2, J / 2>(key, buf, base, lane, flip);
 }
 template <typename K, int K2 = 2>
-__device__ __forceinline__ void bitonic_2048(K (&key)[2], K *buf, int base, int lane, int &flip) {
+__device__ __forceinline__ void bitonic_window(K (&key)[2], K *buf, int base, int lane, int &flip) {
   bitonic_phases<K, K2, K2 / 2>(key, buf, base, lane, flip);
-  if constexpr (K2 < 2048) bitonic_2048<K, K2 * 2>(key, buf, base, lane, flip);
+  if constexpr (K2 < kWindow) bitonic_window<K, K2 * 2>(key, buf, base, lane, flip);
 }
 
-// Stable scatter of a chunk's rows into bin order.
+// Stable scatter of a chunk's rows into bin order.  Lanes of a wave that share a bin find each other
+// with one ballot per bit of the bin; the waves then take their bins' counters in turn, the rows of a
+// wave as one addition per bin.  (Sorting the chunk instead, in registers as above: 9 us.)
 __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(SortArgs a) {
   const SortSide &sd = a.side[blockIdx.y];
   const int chunk = blockIdx.x;
   if (chunk >= sd.chunks) return;
-  __shared__ unsigned buf[2 * kChunk];
-  __shared__ int start[kBins];         // first sorted position of each bin inside the chunk
-  const int lane = threadIdx.x % 64, base = threadIdx.x / 64 * 128;
-  unsigned key[2];                     // bin << 11 | index inside the chunk (all ones: padding)
-#pragma unroll
-  for (int r = 0; r < 2; ++r) {
-    const int e = base + r * 64 + lane, row = chunk * kChunk + e;
-    key[r] = row < sd.n ? (unsigned)top_bits(sd.rmask[row], a.k_vol) << 11 | (unsigned)e : ~0u;
-  }
-  int flip = 0;
-  bitonic_2048(key, buf, base, lane, flip);
-  __syncthreads();
-  buf[base + lane] = key[0];
-  buf[base + 64 + lane] = key[1];
-  // rows in smaller bins: exclusive scan of the bin totals (2 per thread; thread, wave, workgroup)
-  __shared__ int before_bin[kBins];
+  __shared__ int next[kBins];          // where the bin's next row goes
   __shared__ int part[kSortThreads / 64];
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+  constexpr int kBatches = kChunk / kSortThreads;
+  int bin[kBatches], rank[kBatches], peers[kBatches];
+  bool first[kBatches];
+#pragma unroll
+  for (int r = 0; r < kBatches; ++r) {
+    const int row = chunk * kChunk + (wave * kBatches + r) * 64 + lane;
+    const bool live = row < sd.n;
+    bin[r] = live ? top_bits(sd.rmask[row], a.k_vol) : -1;
+    unsigned long long same = __ballot(live);
+#pragma unroll
+    for (int bit = 0; bit < kBinBits; ++bit) {
+      const bool set = bin[r] >> bit & 1;
+      const unsigned long long b = __ballot(set);
+      same &= set ? b : ~b;
+    }
+    const unsigned long long below = same & ((1ull << lane) - 1);
+    rank[r] = __builtin_popcountll(below);
+    peers[r] = __builtin_popcountll(same);
+    first[r] = live && below == 0;
+  }
+  // rows in smaller bins: exclusive scan of the bin totals (thread, wave, workgroup)
   {
     constexpr int kPer = kBins / kSortThreads;
     int mine[kPer], local = 0;
@@ -217,31 +238,36 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(SortArgs a) 
       const int up = __shfl_up(incl, d);
       if (lane >= d) incl += up;
     }
-    if (lane == 63) part[threadIdx.x / 64] = incl;
+    if (lane == 63) part[wave] = incl;
     __syncthreads();
     int before = incl - local;
-    for (int wv = 0; wv < (int)threadIdx.x / 64; ++wv) before += part[wv];
+    for (int wv = 0; wv < wave; ++wv) before += part[wv];
 #pragma unroll
     for (int q = 0; q < kPer; ++q) {
-      before_bin[threadIdx.x * kPer + q] = before;
+      const int b = threadIdx.x * kPer + q;
+      next[b] = before + sd.hist_before[(size_t)chunk * kBins + b];
       before += mine[q];
     }
   }
-#pragma unroll
-  for (int r = 0; r < 2; ++r) {
-    const int e = base + r * 64 + lane;
-    if (key[r] != ~0u && (e == 0 || buf[e - 1] >> 11 != key[r] >> 11)) start[key[r] >> 11] = e;
-  }
   __syncthreads();
+  int at[kBatches];
+  for (int turn = 0; turn < kSortThreads / 64; ++turn) {
+    if (wave == turn) {
 #pragma unroll
-  for (int r = 0; r < 2; ++r) {
-    const int e = base + r * 64 + lane;
-    if (key[r] != ~0u) {
-      const int bin = key[r] >> 11;
-      sd.perm_tmp[before_bin[bin] + sd.hist_before[(size_t)chunk * kBins + bin] + (e - start[bin])] =
-          chunk * kChunk + (int)(key[r] & (kChunk - 1));
+      for (int r = 0; r < kBatches; ++r) {
+        at[r] = bin[r] >= 0 ? next[bin[r]] : 0;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (first[r]) next[bin[r]] = at[r] + peers[r];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+      }
     }
+    __syncthreads();
   }
+#pragma unroll
+  for (int r = 0; r < kBatches; ++r)
+    if (bin[r] >= 0) sd.perm_tmp[at[r] + rank[r]] = chunk * kChunk + (wave * kBatches + r) * 64 + lane;
 }
 
 // Full sort by (mask, row) of a window of positions (of masks over more than 32 offsets: by the top
@@ -249,12 +275,12 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(SortArgs a) 
 // block_mask = the OR of their rows' masks, flags[4 + side] += (block, offset) combinations in use,
 // flags[10 + side] += offset bits of all rows.  chunks == 0: the window starts from the identity
 // order (sides of one window).
-__global__ __launch_bounds__(kSortThreads) void sort_window_kernel(SortArgs a) {
+__global__ __launch_bounds__(kWindowThreads) void sort_window_kernel(SortArgs a) {
   const SortSide &sd = a.side[blockIdx.y];
   const int p0 = blockIdx.x * kWindow;
   if (p0 >= sd.n) return;
   __shared__ unsigned long long buf[2 * kWindow];
-  __shared__ int sums[kSortThreads / 64][2];
+  __shared__ int sums[kWindowThreads / 64][2];
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, base = wave * 128;
   const int shift = a.k_vol > 32 ? a.k_vol - 32 : 0;
   unsigned long long key[2];
@@ -268,7 +294,7 @@ __global__ __launch_bounds__(kSortThreads) void sort_window_kernel(SortArgs a) {
     }
   }
   int flip = 0;
-  bitonic_2048(key, buf, base, lane, flip);
+  bitonic_window(key, buf, base, lane, flip);
   int bits = 0, row_bits = 0;
 #pragma unroll
   for (int r = 0; r < 2; ++r) {
@@ -287,10 +313,7 @@ __global__ __launch_bounds__(kSortThreads) void sort_window_kernel(SortArgs a) {
     }
     if (p0 + base + r * 64 < sd.n) {
       const int block = (p0 + base) / 64 + r;
-      if (lane == 0) {
-        sd.block_mask[block] = m;
-        if (sd.mirror_mask) sd.mirror_mask[block] = __brevll(m) >> (64 - a.k_vol);
-      }
+      if (lane == 0) sd.block_mask[block] = m;
       bits += __popcll(m);
       row_bits += rb;
     }
@@ -302,7 +325,7 @@ __global__ __launch_bounds__(kSortThreads) void sort_window_kernel(SortArgs a) {
   __syncthreads();
   if (threadIdx.x < 2) {
     int sum = 0;
-    for (int i = 0; i < kSortThreads / 64; ++i) sum += sums[i][threadIdx.x];
+    for (int i = 0; i < kWindowThreads / 64; ++i) sum += sums[i][threadIdx.x];
     if (sum) atomicAdd(&a.flags[(threadIdx.x ? 10 : 4) + blockIdx.y], sum);
   }
 }
@@ -384,7 +407,8 @@ __device__ __forceinline__ void tile_order_body(const TileSide &sd, int cus_per_
     const int mid = min(t * 256 + 128, n_rows - 1);
     home = (int)((long long)(perm ? perm[mid] : mid) * 8 / n_rows);
     unsigned long long m = 0;
-    for (int b = 4 * t; b < min(4 * t + 4, n_blocks); ++b) m |= block_masks[b];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) m |= block_masks[min(4 * t + q, n_blocks - 1)];
     pc = __builtin_popcountll(m);
     entry = t | ((m ? __builtin_ctzll(m) : 0) << 24);
   };
@@ -394,14 +418,21 @@ __device__ __forceinline__ void tile_order_body(const TileSide &sd, int cus_per_
     atomicAdd(&hist[home][pc], 1);
   }
   __syncthreads();
-  if (tid < 8) {                                  // start rank of each class, heaviest first
-    int run = 0;
-    for (int pc = kPc - 1; pc >= 0; --pc) {
-      const int n = hist[tid][pc];
-      hist[tid][pc] = run;
-      run += n;
+  // start rank of each class, heaviest first: a wave per home, lane l takes class 64 - l
+  for (int home = tid / 64; home < 8; home += threads / 64) {
+    const int lane = tid % 64, pc = 64 - lane;
+    const int n = hist[home][pc];
+    int incl = n;
+    for (int d = 1; d < 64; d <<= 1) {
+      const int up = __shfl_up(incl, d);
+      if (lane >= d) incl += up;
     }
-    total[tid] = run;
+    hist[home][pc] = incl - n;
+    if (lane == 63) {
+      const int n0 = hist[home][0];
+      hist[home][0] = incl;
+      total[home] = incl + n0;
+    }
   }
   __syncthreads();
   auto position = [&](int rank) {                 // snake over the CUs
@@ -439,10 +470,11 @@ __device__ __forceinline__ void tile_order_body(const TileSide &sd, int cus_per_
 // g is chosen at launch such that their rows fit the XCD's L2), and inside a group the cells
 // are ranked by pair count, most first (the longest workgroups start first), ties
 // by cell number.  Workgroup (x, shift) ranks XCD x's cells in groups of 1 << shift bands by
-// comparing each with the others (a few hundred); it finds their bounds itself, so that bands and
-// order need one launch, and the one with shift 0 writes the bounds down.
+// comparing each with the others (a few hundred).  The bounds are there already (`bands_known`: the
+// mask pass over the lists or the map builder left them), or -- plans over more than 64 offsets -- the
+// workgroup finds them by bisection and the one with shift 0 writes them down.
 __device__ __forceinline__ void bands_body(const TablesArgs &a, int x, int shift, int32_t *__restrict__ lds) {
-  const int k_vol = a.k_vol, bands = a.bands;
+  const int k_vol = a.k_vol, bands = a.bands ? a.bands : band_count_of(a.kpos[a.k_vol], a.k_vol, a.cus_per_xcd * 8);
   const int per_xcd = (bands / 8) * k_vol;
   int *count = lds;                       // [per_xcd]
   int *group = lds + per_xcd;             // [per_xcd]
@@ -458,11 +490,17 @@ __device__ __forceinline__ void bands_body(const TablesArgs &a, int x, int shift
     const int k = o % k_vol, q = o / k_vol, band = q * 8 + x;
     const int first = min(max(a.kpos[k], 0), a.n_pairs);
     const int n = min(max(a.kpos[k + 1], first), a.n_pairs) - first;   // never reads past the map
-    const int b0 = below(first, n, (long long)band * a.band_rows);
-    const int b1 = band + 1 == bands ? n : below(first, n, (long long)(band + 1) * a.band_rows);
+    int b0, b1;
+    if (a.bands_known) {
+      b0 = a.band_start[k * (bands + 1) + band];
+      b1 = a.band_start[k * (bands + 1) + band + 1];
+    } else {
+      b0 = below(first, n, (long long)band * a.band_rows);
+      b1 = band + 1 == bands ? n : below(first, n, (long long)(band + 1) * a.band_rows);
+    }
     count[o] = b1 - b0;
     group[o] = q >> shift;
-    if (shift == 0) {
+    if (shift == 0 && !a.bands_known) {
       a.band_start[k * (bands + 1) + band] = b0;
       if (band + 1 == bands) a.band_start[k * (bands + 1) + bands] = n;
     }
@@ -484,8 +522,8 @@ __device__ __forceinline__ void bands_body(const TablesArgs &a, int x, int shift
 
 // The last launch of a build.  Step 3, the neighbour tables by POSITION: nbr_out[k][position of o] =
 // i, nbr_in[k][position of i] = o -- scattered from the pair lists (tables pre-filled with -1), or,
-// where the map builder left a table of the output rows, the output side's read from there in
-// position order (whole lines both ways: no pre-fill, no scattered 4-byte stores).  Next to it, as
+// where the map builder left a table of the output rows, read from there in the output side's
+// position order (whole lines both ways: no pre-fill, no scattered 4-byte stores on that side).  Next to it, as
 // workgroups of the same launch: tile orders, row bands, the fingerprint of the lists, the findings'
 // way to the host.  (Five launches of 3-12 us each and a second stream before.)
 __global__ __launch_bounds__(256) void tables_kernel(TablesArgs a) {
@@ -513,15 +551,27 @@ __global__ __launch_bounds__(256) void tables_kernel(TablesArgs a) {
   }
   b -= a.print_blocks;
   if (b < a.row_blocks) {
-    const int p = b * 256 + threadIdx.x;
-    if (p >= a.n_out) return;
+    // 64 positions, transposed in LDS: rows come in as whole 16-byte pieces of neighbouring lanes
+    // (a lane that reads its own row alone fetches every line as often as it has pieces)
     typedef int int4v_ __attribute__((ext_vector_type(4)));
-    const int4v_ *row = reinterpret_cast<const int4v_ *>(a.rows + (size_t)a.perm_out[p] * a.row_ld);
-    for (int k0 = 0; k0 < a.k_vol; k0 += 4) {
-      const int4v_ v = row[k0 / 4];
+    const int p0 = b * 64, lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    const int per_row = a.row_ld / 4, ld = a.row_ld + 1;
+    for (int e = threadIdx.x; e < 64 * per_row; e += 256) {
+      const int r = e / per_row, c = e % per_row, p = p0 + r;
+      if (p < a.n_out) {
+        const int4v_ v = *reinterpret_cast<const int4v_ *>(a.rows + (size_t)a.perm_out[p] * a.row_ld + c * 4);
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (k0 + e < a.k_vol) a.nbr_out[(size_t)(k0 + e) * a.n_out + p] = v[e];
+        for (int q = 0; q < 4; ++q) lds[r * ld + c * 4 + q] = v[q];
+      }
+    }
+    __syncthreads();
+    if (p0 + lane < a.n_out) {
+      const int o = a.inv_in ? a.perm_out[p0 + lane] : 0;
+      for (int k = wave; k < a.k_vol; k += 4) {
+        const int i = lds[lane * ld + k];
+        a.nbr_out[(size_t)k * a.n_out + p0 + lane] = i;
+        if (a.inv_in && i >= 0) a.nbr_in[(size_t)k * a.n_in + a.inv_in[i]] = o;
+      }
     }
     return;
   }
@@ -620,7 +670,7 @@ int launch_sort(const SortArgs &args, bool hist_done, hipStream_t s) {
     sort_scan_kernel<<<dim3(kBins / kScanBins, sides), 256, 0, s>>>(a);
     sort_scatter_kernel<<<dim3((unsigned)chunks, sides), kSortThreads, 0, s>>>(a);
   }
-  if (most) sort_window_kernel<<<dim3((unsigned)((most + kWindow - 1) / kWindow), sides), kSortThreads, 0, s>>>(a);
+  if (most) sort_window_kernel<<<dim3((unsigned)((most + kWindow - 1) / kWindow), sides), kWindowThreads, 0, s>>>(a);
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;
 }
@@ -631,13 +681,14 @@ int launch_tables(TablesArgs a, hipStream_t s) {
   a.tile_blocks = 8;                               // (two at work; the parts behind start on a multiple of eight)
   a.band_blocks = 0;
   if (a.band_start) {
-    const size_t need = (size_t)2 * (a.bands / 8) * a.k_vol * sizeof(int32_t);
+    const size_t need = (size_t)2 * ((a.bands ? a.bands : 64) / 8) * a.k_vol * sizeof(int32_t);
     if (need > lds) lds = need;
     a.band_blocks = 32;
   }
   a.print_blocks = a.take_print ? kPrintParts : 0;
-  a.row_blocks = a.rows ? (a.n_out + 255) / 256 : 0;
-  a.pair_blocks = a.inv_out || a.inv_in ? (a.n_pairs + 255) / 256 : 0;
+  a.row_blocks = a.rows ? (a.n_out + 63) / 64 : 0;
+  if (a.rows && (size_t)64 * (a.row_ld + 1) * sizeof(int32_t) > lds) lds = (size_t)64 * (a.row_ld + 1) * sizeof(int32_t);
+  a.pair_blocks = !a.rows && (a.inv_out || a.inv_in) ? (a.n_pairs + 255) / 256 : 0;
   a.cus_per_xcd = num_cus() >= 8 ? num_cus() / 8 : 1;
   if (lds > 48 * 1024) {
     const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(tables_kernel), lds);
@@ -653,8 +704,6 @@ Plan *plan_alloc(int k_vol, int64_t n_in, int64_t n_out, int64_t n_pairs, hipStr
   p->k_vol = k_vol; p->n_in = n_in; p->n_out = n_out; p->n_pairs = n_pairs;
   p->last_stream = s;
   p->create_stream = s;
-  p->nbr_stride_out = (int)n_out;
-  p->nbr_stride_in = (int)n_in;
   if (hipGetDevice(&p->device) == hipSuccess && (p->host_flags = pinned_flags_get()) &&
       (p->ready = event_get(p->device))) {
     p->host_flags[kFlagStale] = 0;     // (a recycled block: the flag is read before the build has run)
@@ -665,23 +714,9 @@ Plan *plan_alloc(int k_vol, int64_t n_in, int64_t n_out, int64_t n_pairs, hipStr
   return nullptr;
 }
 
-// Weight-gradient row bands: 8, 16, 32 or 64 (the XCDs take them in groups of 1, 2, 4 or 8;
-// other counts measured worse), the fewest that leave an (offset, band) cell at most ~1 900
-// pairs -- a workgroup's fixed costs (first loads, the four waves' partial tiles summed through
-// LDS, 16 KB of atomic updates) are those of ~600 pairs, and with bigger cells the chip waits
-// for the last ones -- then more while the cells are fewer than 1.5 per CU and keep ~400 pairs.
-// 64 -> 64 fp16 backward launch with 64 bands throughout / with this rule: 50 k voxels 35.5 /
-// 29.8 us, 80 k 55.6 / 45.2, 100 k 59.1 / 46.2, 120 k 61.5 / 55.6, 140 k 67.7 / 65.3 (32 bands
-// each), 170 k and 200 k voxels 64 bands either way.
 void plan_bands(Plan *p) {
-  constexpr int kMaxBands = 64;
-  int bands = 8;
-  while (bands < kMaxBands && p->n_pairs / ((int64_t)p->k_vol * bands) > 1900) bands *= 2;
-  while (bands < kMaxBands && (int64_t)bands * p->k_vol * 2 < 3 * (int64_t)num_cus() &&
-         p->n_pairs / ((int64_t)p->k_vol * bands * 2) >= 384)
-    bands *= 2;
-  p->band_count = bands;
-  p->band_rows = (int)((p->n_out + bands - 1) / bands);
+  p->band_count = band_count_of(p->n_pairs, p->k_vol, num_cus());
+  p->band_rows = (int)((p->n_out + p->band_count - 1) / p->band_count);
 }
 
 // Tile -> XCD homes pay off once every XCD has a few dozen tiles of its own.
@@ -700,7 +735,7 @@ void plan_fill_tables_args(const Plan *p, TablesArgs *t) {
   t->band_rows = p->band_rows > 0 ? p->band_rows : 1;
   for (int d = 0; d < 2; ++d) {
     int32_t *order = d ? p->tile_in : p->tile_out;
-    if (!order) continue;
+    if (!order || (d && order == p->tile_out)) continue;
     int cap;
     const int64_t n = d ? p->n_in : p->n_out;
     const int n_tiles = tile_table(n, &cap);
@@ -807,6 +842,7 @@ int plan_create(fgms_plan_t **plan_out, const int32_t *kpos, const int32_t *in_m
   if (tables) {
     fills.add(rmask, (size_t)(n_out + n_in) * sizeof(unsigned long long), 0);
     fills.add(p->nbr_out, (so + si) * sizeof(int32_t), -1);
+    if (want_bands) fills.add(p->band_start, (size_t)k_vol * (p->band_count + 1) * sizeof(int32_t), 0);
   }
   if ((rc = launch_fills(fills, s))) return fail(rc);
   TablesArgs ta{};
@@ -814,10 +850,12 @@ int plan_create(fgms_plan_t **plan_out, const int32_t *kpos, const int32_t *in_m
   if (tables) {
     if (n_pairs > 0)
       pair_masks_kernel<<<(unsigned)((n_pairs + 255) / 256) + kPrintParts, 256, 0, s>>>(
-          kpos, in_map, out_map, k_vol, (int)n_pairs, (int)n_in, (int)n_out, rmask, rmask + n_out, p->flags);
+          kpos, in_map, out_map, k_vol, (int)n_pairs, (int)n_in, (int)n_out, rmask, rmask + n_out, p->flags,
+          want_bands ? p->band_start : nullptr, p->band_count, p->band_rows > 0 ? p->band_rows : 1);
     if ((rc = launch_sort(sa, false, s))) return fail(rc);
     ta.inv_out = sa.side[0].inv; ta.inv_in = sa.side[1].inv;
     ta.nbr_out = p->nbr_out; ta.nbr_in = p->nbr_in;
+    ta.bands_known = true;
   }
   if ((rc = launch_tables(ta, s)) || (rc = plan_publish(p, ta.host != nullptr, s))) return fail(rc);
   if (scratch) pool_free(scratch, s, false);
@@ -932,7 +970,7 @@ const Plan *plan_resolve(fgms_plan_t *plan, hipStream_t stream, int *rc) {
     std::lock_guard<std::mutex> lock(p->mutex);
     if (!p->resolved) {
       p->nbr_out = b->nbr_in; p->nbr_in = b->nbr_out;
-      p->nbr_stride_out = b->nbr_stride_in; p->nbr_stride_in = b->nbr_stride_out;
+      p->flip_out = b->flip_in; p->flip_in = b->flip_out;
       p->perm_out = b->perm_in; p->perm_in = b->perm_out;
       p->mask_out = b->mask_in; p->mask_in = b->mask_out;
       p->tile_out = b->tile_in; p->tile_in = b->tile_out;

@@ -46,7 +46,6 @@ struct SortSide {
   int32_t *hist_before;              // [chunks][kBins] rows of the bin in earlier chunks
   int32_t *bin_start;                // [kBins] rows per bin
   unsigned long long *block_mask;    // OR of the masks of every 64 positions
-  unsigned long long *mirror_mask;   // the same with bit k at k_vol - 1 - k, or nullptr
   int n, chunks;                     // chunks == 0: one window, no counting sort
 };
 struct SortArgs {
@@ -55,11 +54,12 @@ struct SortArgs {
   int *flags;
   bool by_mask;                      // false: natural order
 };
-constexpr int kBinBits = 11;
+constexpr int kBinBits = 12;
 constexpr int kBins = 1 << kBinBits;
 constexpr int kChunk = 2048;         // rows per workgroup of the histogram / scatter kernels
-constexpr int kWindow = 2048;        // positions per workgroup of the window sort
+constexpr int kWindow = 1024;        // positions per workgroup of the window sort
 constexpr int kSortThreads = 1024;
+constexpr int kWindowThreads = kWindow / 2;
 
 __device__ __forceinline__ int top_bits(unsigned long long m, int k_vol) {
   const int shift = k_vol > kBinBits ? k_vol - kBinBits : 0;
@@ -83,6 +83,23 @@ void sort_side_layout(SortSide &sd, int64_t n, Arena &tmp);
 // Histogram (unless the caller's own launch took it), scan, scatter, window sort.
 int launch_sort(const SortArgs &a, bool hist_done, hipStream_t s);
 
+// Weight-gradient row bands: 8, 16, 32 or 64 (the XCDs take them in groups of 1, 2, 4 or 8;
+// other counts measured worse), the fewest that leave an (offset, band) cell at most ~1 900
+// pairs -- a workgroup's fixed costs (first loads, the four waves' partial tiles summed through
+// LDS, 16 KB of atomic updates) are those of ~600 pairs, and with bigger cells the chip waits
+// for the last ones -- then more while the cells are fewer than 1.5 per CU and keep ~400 pairs.
+// 64 -> 64 fp16 backward launch with 64 bands throughout / with this rule: 50 k voxels 35.5 /
+// 29.8 us, 80 k 55.6 / 45.2, 100 k 59.1 / 46.2, 120 k 61.5 / 55.6, 140 k 67.7 / 65.3 (32 bands
+// each), 170 k and 200 k voxels 64 bands either way.
+__host__ __device__ inline int band_count_of(int64_t n_pairs, int k_vol, int cus) {
+  constexpr int kMaxBands = 64;
+  int bands = 8;
+  while (bands < kMaxBands && n_pairs / ((int64_t)k_vol * bands) > 1900) bands *= 2;
+  while (bands < kMaxBands && (int64_t)bands * k_vol * 2 < 3 * (int64_t)cus && n_pairs / ((int64_t)k_vol * bands * 2) >= 384)
+    bands *= 2;
+  return bands;
+}
+
 // ---- the last launch of a build: tables by position, row bands, tile order, findings
 struct TileSide {
   const int32_t *perm;
@@ -96,13 +113,14 @@ struct TablesArgs {
   // from the pair lists: position -> neighbour through offset k (tables pre-filled with -1; nullptr: not this one)
   const int32_t *inv_out, *inv_in;
   int32_t *nbr_out, *nbr_in;
-  // from a table of the output rows, [n_out][row_ld]: nbr_out only
+  // from a table of the output rows, [n_out][row_ld] (nbr_in: where inv_in is given)
   const int32_t *rows;
   const int32_t *perm_out;
   int row_ld;
   // bands
   int32_t *band_start, *band_cells;
-  int bands, band_rows;
+  int bands, band_rows;              // (bands == 0: as many as the pairs in kpos ask for)
+  bool bands_known;                  // band_start is filled in already
   TileSide tile[2];
   int cus_per_xcd;
   int *flags, *host;                 // findings and where they go on the host (nullptr: a copy follows)
@@ -112,6 +130,9 @@ struct TablesArgs {
 };
 int launch_tables(TablesArgs a, hipStream_t s);
 
+// A plan from pair lists (fgms_plan_create; want_bands: with the weight gradient's row bands).
+int plan_create(fgms_plan_t **plan, const int32_t *kpos, const int32_t *in_map, const int32_t *out_map, int64_t n_in,
+                int64_t n_out, int k_vol, int64_t n_pairs, void *stream, bool want_bands);
 // Plan objects without their tables.
 Plan *plan_alloc(int k_vol, int64_t n_in, int64_t n_out, int64_t n_pairs, hipStream_t s);
 void plan_bands(Plan *p);                                // band_count / band_rows from the sizes

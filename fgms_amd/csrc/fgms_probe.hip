@@ -20,7 +20,7 @@ typedef int int4v __attribute__((ext_vector_type(4)));
 template <int CR>
 __global__ __launch_bounds__(256) void gather_probe_kernel(
     const int4v *__restrict__ src, const int32_t *__restrict__ nbr,
-    const unsigned long long *__restrict__ block_masks, int n_dst, int *__restrict__ sink, int nbr_stride) {
+    const unsigned long long *__restrict__ block_masks, int n_dst, int *__restrict__ sink) {
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int row0 = (blockIdx.x * 4 + wave) * 64;
   if (row0 >= n_dst) return;
@@ -29,11 +29,11 @@ __global__ __launch_bounds__(256) void gather_probe_kernel(
   const bool live = row0 + lane < n_dst;
   int4v acc = {0, 0, 0, 0};
   int g_next = -1;
-  if (todo) g_next = nbr[(ptrdiff_t)__builtin_ctzll(todo) * nbr_stride + my];
+  if (todo) g_next = nbr[(size_t)__builtin_ctzll(todo) * n_dst + my];
   while (todo) {
     todo &= todo - 1;
     const int g = live ? g_next : -1;
-    if (todo) g_next = nbr[(ptrdiff_t)__builtin_ctzll(todo) * nbr_stride + my];   // next offset's line in flight
+    if (todo) g_next = nbr[(size_t)__builtin_ctzll(todo) * n_dst + my];   // next offset's line in flight
     // 64 rows x CR pieces, 64 pieces per load instruction, consecutive lanes on one row
     constexpr int kBatch = CR < 8 ? CR : 8;
 #pragma unroll 1
@@ -67,7 +67,7 @@ int launch_gather_probe(const Plan *p, const void *src, int c_src, int dtype, bo
   if (n_dst == 0) return FGMS_OK;
   const unsigned gx = (unsigned)((n_dst + 255) / 256);
   const int cr = (int)(row_bytes / 16);
-  void (*kern)(const int4v *, const int32_t *, const unsigned long long *, int, int *, int) = nullptr;
+  void (*kern)(const int4v *, const int32_t *, const unsigned long long *, int, int *) = nullptr;
   switch (cr) {
     case 1: kern = gather_probe_kernel<1>; break;
     case 2: kern = gather_probe_kernel<2>; break;
@@ -83,8 +83,7 @@ int launch_gather_probe(const Plan *p, const void *src, int c_src, int dtype, bo
   {
     ProfileScope prof(for_dgrad ? "gather_probe_kernel(dgrad)" : "gather_probe_kernel(fwd)", stream);
     kern<<<gx, 256, 0, stream>>>((const int4v *)src, for_dgrad ? p->nbr_in : p->nbr_out,
-                                 for_dgrad ? p->mask_in : p->mask_out, (int)n_dst, (int *)sink,
-                                 for_dgrad ? p->nbr_stride_in : p->nbr_stride_out);
+                                 for_dgrad ? p->mask_in : p->mask_out, (int)n_dst, (int *)sink);
   }
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;

@@ -113,7 +113,7 @@ template <typename T, int CS, int CD, bool TR>
 __global__ __launch_bounds__(kSmallThreads) void gms_small_kernel(
     const T *__restrict__ src, const uint32_t *__restrict__ w, T *__restrict__ dst,
     const int32_t *__restrict__ nbr, const unsigned long long *__restrict__ block_masks,
-    const int32_t *__restrict__ perm, int n_dst, int parts, int overwrite, SideJob side, int nbr_stride) {
+    const int32_t *__restrict__ perm, int n_dst, int parts, int overwrite, SideJob side, int flip) {
   // the leading workgroups of the grid run the side job, if there is one
   int block_x = blockIdx.x;
   if (side.blocks) {
@@ -162,7 +162,7 @@ __global__ __launch_bounds__(kSmallThreads) void gms_small_kernel(
   // lanes past the last row shadow it and skip the final store; an index asked for past
   // the last offset (k < 0) is read from offset 0 and never used
   const int row_c = live ? row : n_dst - 1;
-  auto index_of = [&](int k) { return nbr[(ptrdiff_t)(k < 0 ? 0 : k) * nbr_stride + row_c]; };
+  auto index_of = [&](int k) { return nbr[(size_t)(k < 0 ? 0 : k) * n_dst + row_c]; };
   auto gather = [&](float (&x)[CS], int g) { load_row<T, CS>(x, src + (size_t)(g < 0 ? 0 : g) * CS); };
   int k0 = next_k();
   if (k0 >= 0) {
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(kSmallThreads) void gms_small_kernel(
       gather(x1, g1);                                             // next offset's row
       const int k3 = next_k();
       const int g3 = index_of(k3);                                // index two offsets ahead
-      const uint32_t *wk = w + (size_t)k0 * kWordsPerOffset;
+      const uint32_t *wk = w + (size_t)(flip ? flip - k0 : k0) * kWordsPerOffset;      // (flip: see Plan)
       if (g0 >= 0) {                                              // rows without a pair here sit out
 #pragma unroll
         for (int cs = 0; cs < CS; ++cs)
@@ -251,11 +251,11 @@ int launch_small(const GmsArgs &a, const Plan *p) {
     if (a.transpose_w)
       gms_small_kernel<T, CS, CD, true><<<gx, kSmallThreads, lds, a.stream>>>(
           (const T *)a.src, (const uint32_t *)a.w, (T *)a.dst, nbr, masks, perm, (int)a.n_dst, parts, a.overwrite ? 1 : 0, a.side,
-          a.transpose_w ? p->nbr_stride_in : p->nbr_stride_out);
+          a.transpose_w ? p->flip_in : p->flip_out);
     else
       gms_small_kernel<T, CS, CD, false><<<gx, kSmallThreads, lds, a.stream>>>(
           (const T *)a.src, (const uint32_t *)a.w, (T *)a.dst, nbr, masks, perm, (int)a.n_dst, parts, a.overwrite ? 1 : 0, a.side,
-          a.transpose_w ? p->nbr_stride_in : p->nbr_stride_out);
+          a.transpose_w ? p->flip_in : p->flip_out);
   }
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;

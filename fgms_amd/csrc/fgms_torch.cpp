@@ -35,6 +35,7 @@
 #include <list>
 #include <mutex>
 #include <stdexcept>
+#include <utility>
 #include <vector>
 
 #include "fgms.h"
@@ -393,7 +394,84 @@ at::Tensor sparse_conv(const at::Tensor &feats, const at::Tensor &weight, const 
 
 }  // namespace
 
+namespace {
+
+void need_coords(const at::Tensor &t, const char *name) {
+  if (t.scalar_type() != at::ScalarType::Int || !t.is_cuda() || !t.is_contiguous() || t.dim() != 2 || t.size(1) != 3)
+    throw std::invalid_argument(std::string(name) + " must be a contiguous int32 [N, 3] tensor on the GPU");
+}
+
+// A kernel map from voxel coordinates on its way: everything is queued, the sizes are not known yet.
+struct MapOnItsWay {
+  at::Tensor in_coords, out_coords;        // (read by the queued build: kept until its sizes are there)
+  at::Tensor in_map, out_map, sizes, nnz;
+  int64_t n_in = 0, n_out = 0, k_vol = 0;
+  fgms_map_build_t *build = nullptr;
+  hipStream_t stream = nullptr;
+
+  MapOnItsWay(const at::Tensor &in_coords_, const at::Tensor &out_coords_, const at::Tensor &offsets, int64_t stride)
+      : in_coords(in_coords_), out_coords(out_coords_) {
+    need_coords(in_coords, "in_coords");
+    need_coords(out_coords, "out_coords");
+    if (offsets.scalar_type() != at::ScalarType::Int || offsets.is_cuda() || !offsets.is_contiguous() || offsets.dim() != 2 ||
+        offsets.size(1) != 3)
+      throw std::invalid_argument("offsets must be a contiguous int32 [K, 3] tensor on the host");
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(in_coords.device());
+    stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
+    k_vol = offsets.size(0), n_in = in_coords.size(0), n_out = out_coords.size(0);
+    const int64_t capacity = std::max<int64_t>(k_vol * n_out, 1);
+    const auto opts = in_coords.options().requires_grad(false);
+    in_map = at::empty({capacity}, opts);
+    out_map = at::empty({capacity}, opts);
+    sizes = at::empty({3 * k_vol + 2}, opts);         // kernel_nnz, kpos, qkpos
+    nnz = at::empty({k_vol}, offsets.options());
+    int *base = sizes.data_ptr<int>();
+    bool want_plan;
+    {
+      std::lock_guard<std::mutex> lock(g_mutex);
+      want_plan = g_cache_enabled;
+    }
+    check(fgms_build_map_begin(&build, i32(in_coords), n_in, i32(out_coords), n_out, offsets.data_ptr<int>(), (int)k_vol,
+                               (int)stride, -1, in_map.data_ptr<int>(), out_map.data_ptr<int>(), k_vol * n_out, base,
+                               base + k_vol, base + 2 * k_vol + 1, want_plan, stream));
+  }
+
+  ~MapOnItsWay() {
+    if (!build) return;
+    int64_t pairs;
+    (void)fgms_build_map_end(build, nullptr, &pairs, nullptr);
+  }
+
+  // (in_map, out_map, kernel_nnz on the host, kpos, qkpos, sum of the padded sizes); its plan goes to the cache.
+  std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor, int64_t> finish() {
+    fgms_map_build_t *b = std::exchange(build, nullptr);
+    if (!b) throw std::runtime_error("FGMS: this kernel map has been taken already");
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(in_coords.device());
+    int64_t pairs = 0;
+    fgms_plan_t *plan = nullptr;
+    check(fgms_build_map_end(b, nnz.data_ptr<int>(), &pairs, &plan));
+    at::Tensor im = in_map.narrow(0, 0, pairs), om = out_map.narrow(0, 0, pairs);
+    at::Tensor kpos = sizes.narrow(0, k_vol, k_vol + 1), qkpos = sizes.narrow(0, 2 * k_vol + 1, k_vol + 1);
+    int64_t qsum = 0;
+    for (int64_t k = 0; k < k_vol; ++k) qsum += (nnz.data_ptr<int>()[k] + 255) / 256 * 256;
+    if (plan) {
+      Dropped dropped;
+      std::lock_guard<std::mutex> lock(g_mutex);
+      g_cache.push_front(CacheEntry{kpos, im, om, version_of(kpos), version_of(im), version_of(om), n_in, n_out,
+                                    (int)in_coords.get_device(), plan, false});
+      while (g_cache.size() > (g_cache_enabled ? g_cache_cap : 0)) drop(std::prev(g_cache.end()), dropped);
+    }
+    return {im, om, nnz, kpos, qkpos, qsum};
+  }
+};
+
+}  // namespace
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  pybind11::class_<MapOnItsWay>(m, "MapOnItsWay")
+      .def(pybind11::init<const at::Tensor &, const at::Tensor &, const at::Tensor &, int64_t>(),
+           pybind11::call_guard<pybind11::gil_scoped_release>())
+      .def("finish", &MapOnItsWay::finish, pybind11::call_guard<pybind11::gil_scoped_release>());
   m.def("sparse_conv", &sparse_conv);
   m.def("fgms_fusion_fwd_cuda", &ConvolutionForwardFused);
   m.def("fgms_fwd_cuda", &ConvolutionForward);

@@ -243,7 +243,7 @@ int fgms_weights_unpin(const void *kernel);
  * in_coords / out_coords: device int32 [n][3], every component in
  * [-2^20, 2^20); offsets: HOST int32 [k_vol][3]; skip_offset: an offset to
  * leave empty (the centre, for callers that use separate_mid), or -1.
- * Synchronises the stream once.  FGMS_E_INVALID if a coordinate is out of
+ * Waits for the sizes once.  FGMS_E_INVALID if a coordinate is out of
  * range or the pairs do not fit `capacity` (*n_pairs is set, the lists hold
  * the first `capacity` pairs).
  */
@@ -252,6 +252,23 @@ int fgms_build_kernel_map(const int32_t *in_coords, int64_t n_in,
                           const int32_t *offsets, int k_vol, int stride, int skip_offset,
                           int32_t *in_map, int32_t *out_map, int64_t capacity,
                           int32_t *kernel_nnz, int32_t *kpos, int64_t *n_pairs, void *stream);
+
+/*
+ * The same in two calls and together with what a caller makes of the map next.  `begin` queues the
+ * whole build -- the lists, qkpos[k_vol + 1] (device, may be NULL: the 256-padded prefix sum of the
+ * sizes, cpu-check.py:6-14) and, with want_plan, the map's plan (fgms_plan_create), made from the
+ * lookups instead of from the lists -- and waits for the check of the coordinates only.  `end`
+ * waits for the build: host_nnz[k_vol] (HOST, may be NULL), *n_pairs, *plan (NULL where one side is
+ * empty).  Maps that are begun one after the other are built one behind the other without a gap.
+ * Every build that begins has to end, on any thread; the arrays stay valid until then.
+ */
+typedef struct fgms_map_build fgms_map_build_t;
+int fgms_build_map_begin(fgms_map_build_t **build, const int32_t *in_coords, int64_t n_in,
+                         const int32_t *out_coords, int64_t n_out,
+                         const int32_t *offsets, int k_vol, int stride, int skip_offset,
+                         int32_t *in_map, int32_t *out_map, int64_t capacity,
+                         int32_t *kernel_nnz, int32_t *kpos, int32_t *qkpos, int want_plan, void *stream);
+int fgms_build_map_end(fgms_map_build_t *build, int32_t *host_nnz, int64_t *n_pairs, fgms_plan_t **plan);
 
 #ifdef __cplusplus
 }
