@@ -524,7 +524,17 @@ __global__ __launch_bounds__(kThreads) void gms_pairs_kernel(
 // MT: 32-row MFMA tiles per wave.  2 (a workgroup tile of 256 rows) is the layout every plan
 // table is made for; 1 (tiles of 128 rows, half the work per wave and stage) serves launches
 // too small to fill the chip, where a tile's chain of stages is all there is to the duration.
-template <typename T, int NT, int S, int RAW, int MT = 2>
+// KG > 1 (MT = 1): the workgroup is KG groups of four waves, every group walks its share of the
+// tile's offsets with LDS of its own, and the groups' sums meet in LDS behind the last stage: the chain
+// is a KG-th as long, without the atomics (and the zeroed result rows) that workgroups sharing a tile need.
+template <typename T, int NT, int S, int MT>
+constexpr int rows_group_chunks() {      // 16-byte chunks of LDS per group: two stages of weights, row tiles, indices
+  return 2 * S * NT * 64 + kWaves * MT * 32 * 2 * S + kWaves * 3 * MT * 32 / 4;
+}
+template <int NT, int MT>
+constexpr int rows_sum_chunks() { return kWaves * MT * NT * 4 * 64; }      // ... of a group's sums
+
+template <typename T, int NT, int S, int RAW, int MT = 2, int KG = 1>
 __device__ __forceinline__ void gms_rows_body(
     const T *__restrict__ src, const T *__restrict__ packed, T *__restrict__ dst,
     const int32_t *__restrict__ nbr, const unsigned long long *__restrict__ block_masks,
@@ -546,15 +556,18 @@ __device__ __forceinline__ void gms_rows_body(
   const size_t nbr_stride = pair_view ? 0 : (size_t)n_dst;
   constexpr int WCH = S * NT * 64;                        // 16-byte chunks of one stage's weights
   constexpr int NW = (WCH + kThreads - 1) / kThreads;     // ... per thread
-  extern __shared__ int4v lds[];
+  extern __shared__ int4v lds_all[];
   __shared__ unsigned long long wg_mask;
+  const int group = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / kThreads);
+  const int tid = KG == 1 ? threadIdx.x : threadIdx.x % kThreads;
+  int4v *const lds = KG == 1 ? lds_all : lds_all + group * rows_group_chunks<T, NT, S, MT>();
   // fp32 only: its MFMA phase is long enough (4 k clocks a stage) to absorb the loads'
   // issue waits; for fp16 the interleaved stage measured 2 us slower per launch
   constexpr bool kInterleave = sizeof(T) == 4 && RAW != 3 && RAW != 4;
   const int slabs = c_src / (C * E);
   const int nts = c_dst / 32;
   int4v *w_lds = lds;                                     // [2][WCH]
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+  const int wave = tid / 64, lane = tid % 64;
   constexpr int WR = MT * 32;                             // rows per wave
   constexpr int TR = kWaves * WR;                         // rows per workgroup tile
   int4v *a_lds = lds + 2 * WCH + wave * (WR * C);
@@ -599,7 +612,7 @@ __device__ __forceinline__ void gms_rows_body(
   __syncthreads();
   unsigned long long todo = wg_mask;
   if (!todo) {
-    if (overwrite) zero_rows<T, NT, WR>(dst, didx, c_dst, nt0 * 32, lane);
+    if (overwrite && group == 0) zero_rows<T, NT, WR>(dst, didx, c_dst, nt0 * 32, lane);
     return;
   }
   // The launch lasts as long as its longest tile, and the tiles with the longest
@@ -632,6 +645,27 @@ __device__ __forceinline__ void gms_rows_body(
     }
   }
 
+  if constexpr (KG > 1) {
+    // this group's run of the tile's offsets; a group with fewer than the others also walks some of
+    // theirs, for which its rows count as absent, so that all groups meet at the same barriers
+    const int per = (__builtin_popcountll(todo) + KG - 1) / KG;
+    unsigned long long rest = todo, mine = 0;
+    for (int i = 0; i < group * per; ++i) rest &= rest - 1;
+    int count = 0;
+    for (; count < per && rest; ++count) {
+      mine |= rest & (0 - rest);
+      rest &= rest - 1;
+    }
+    unsigned long long others = todo & ~mine;
+    todo = mine;
+    for (; count < per; ++count) {
+      todo |= others & (0 - others);
+      others &= others - 1;
+    }
+    wave_mask &= mine;
+    k_first = -1;
+  }
+
   float16v acc[MT][NT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
@@ -654,7 +688,7 @@ __device__ __forceinline__ void gms_rows_body(
   unsigned wvoff[NW];
 #pragma unroll
   for (int i = 0; i < NW; ++i) {
-    const int e = threadIdx.x + kThreads * i;
+    const int e = tid + kThreads * i;
     if constexpr (RAW == 1) wvoff[i] = (unsigned)(((e / (NT * 4)) * c_dst + (e % (NT * 4)) * E) * (int)sizeof(T));
     else if constexpr (RAW == 2 || RAW == 4) wvoff[i] = (unsigned)(((e / C) * c_src + (e % C) * E) * (int)sizeof(T));
     else if constexpr (RAW == 3) wvoff[i] = (unsigned)(((e / (NT * 128)) * nts * 128 + e % (NT * 128)) * 16);
@@ -666,7 +700,7 @@ __device__ __forceinline__ void gms_rows_body(
     if constexpr (!kBuf) {
 #pragma unroll
       for (int i = 0; i < NW; ++i) {
-        const int e = threadIdx.x + kThreads * i;
+        const int e = tid + kThreads * i;
         if (NW * kThreads == WCH || e < WCH) {
           if constexpr (RAW == 2) {
             const int row = e / C, c = e % C;
@@ -687,7 +721,7 @@ __device__ __forceinline__ void gms_rows_body(
     else soff = (unsigned)(((int)packed_per_k * k + ((slab * S) * nts + nt0) * 64) * 16);
 #pragma unroll
     for (int i = 0; i < NW; ++i) {
-      const int e = threadIdx.x + kThreads * i;
+      const int e = tid + kThreads * i;
       if (NW * kThreads == WCH || e < WCH)
         wreg[i] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(wrsrc, wvoff[i], soff, 0));
     }
@@ -695,7 +729,7 @@ __device__ __forceinline__ void gms_rows_body(
   auto weights_commit = [&](const int4v (&wreg)[NW], int buf) {
 #pragma unroll
     for (int i = 0; i < NW; ++i) {
-      const int e = threadIdx.x + kThreads * i;
+      const int e = tid + kThreads * i;
       if (NW * kThreads == WCH || e < WCH) {
         if constexpr (RAW == 1) {
           const int row = e / (NT * 4), c = e % (NT * 4);
@@ -732,7 +766,8 @@ __device__ __forceinline__ void gms_rows_body(
   };
 
   // prologue: stage 0 goes straight to LDS
-  if (owns_row) goff[lane] = row_offset(k_first >= 0 ? g_first : (in_range ? nbr[(size_t)k * nbr_stride + my_row] : -1));
+  if (owns_row)
+    goff[lane] = row_offset(k_first >= 0 ? g_first : (in_range && (KG == 1 || active) ? nbr[(size_t)k * nbr_stride + my_row] : -1));
   int g_nxt = (k_nxt >= 0 && in_range) ? nbr[(size_t)k_nxt * nbr_stride + my_row] : -1;
   wave_lds_fence();
   weights_issue(wreg, k, 0);
@@ -882,7 +917,32 @@ __device__ __forceinline__ void gms_rows_body(
       active = next_active;
     }
   }
-  if (wave_mask || overwrite) {
+  if constexpr (KG > 1) {
+    // the groups' sums meet in the LDS behind the first group's
+    float4v *const sums = reinterpret_cast<float4v *>(lds_all + rows_group_chunks<T, NT, S, MT>());
+    constexpr int per_group = rows_sum_chunks<NT, MT>();
+    __syncthreads();                   // every group is through with its row tiles and weights
+    if (group > 0) {
+#pragma unroll
+      for (int q = 0; q < MT * NT * 4; ++q) {
+        float4v v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = acc[q / 4 / NT][q / 4 % NT][q % 4 * 4 + e];
+        sums[(group - 1) * per_group + (wave * (MT * NT * 4) + q) * 64 + lane] = v;
+      }
+    }
+    __syncthreads();
+    if (group > 0) return;
+#pragma unroll
+    for (int g = 0; g < KG - 1; ++g)
+#pragma unroll
+      for (int q = 0; q < MT * NT * 4; ++q) {
+        const float4v v = sums[g * per_group + (wave * (MT * NT * 4) + q) * 64 + lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[q / 4 / NT][q / 4 % NT][q % 4 * 4 + e] += v[e];
+      }
+  }
+  if (wave_mask || overwrite || KG > 1) {
     wave_lds_fence();
     if (shared_tile)
       add_rows_lds<T, NT, S, true, false>(acc, dst, didx, reinterpret_cast<float *>(a_lds), c_dst, nt0 * 32, lane);
@@ -893,8 +953,8 @@ __device__ __forceinline__ void gms_rows_body(
   }
 }
 
-template <typename T, int NT, int S, int RAW, int MT = 2>
-__global__ __launch_bounds__(kThreads, MT == 1 ? 4 : (NT == 4 ? 2 : 3)) void gms_rows_kernel(
+template <typename T, int NT, int S, int RAW, int MT = 2, int KG = 1>
+__global__ __launch_bounds__(kThreads * KG, MT == 1 ? 4 : (NT == 4 ? 2 : 3)) void gms_rows_kernel(
     const T *__restrict__ src, const T *__restrict__ packed, T *__restrict__ dst,
     const int32_t *__restrict__ nbr, const unsigned long long *__restrict__ block_masks,
     const int32_t *__restrict__ perm, const int32_t *__restrict__ tile_order, int n_dst, int k_vol,
@@ -909,7 +969,7 @@ __global__ __launch_bounds__(kThreads, MT == 1 ? 4 : (NT == 4 ? 2 : 3)) void gms
     }
     block_x -= side.blocks;
   }
-  gms_rows_body<T, NT, S, RAW, MT>(src, packed, dst, nbr, block_masks, perm, tile_order, n_dst, k_vol, c_src,
+  gms_rows_body<T, NT, S, RAW, MT, KG>(src, packed, dst, nbr, block_masks, perm, tile_order, n_dst, k_vol, c_src,
                                    c_dst, part_stages, block_x, blockIdx.y, blockIdx.z, gridDim.z, src_bytes, pair_view,
                                    overwrite, flip);
 }
@@ -1047,11 +1107,12 @@ bool half_tiles_enabled() {
 struct RowsGrid {
   bool half_tiles;
   bool drop_table;      // the launch does better on plain 128-row tiles than on the plan's tile table
+  int groups;           // groups of four waves per workgroup (KG), 128-row tiles only
   unsigned gx, gz;
   int part_stages;
 };
 RowsGrid rows_grid(int64_t n_dst, unsigned gy, int stages, bool can_half, bool has_table, int table_grid,
-                   bool pair_view, int wgs_per_cu, bool input_gradient) {
+                   bool pair_view, int wgs_per_cu, bool input_gradient, bool can_group) {
   RowsGrid g{};
   const int64_t small_tiles = (int64_t)((n_dst + 127) / 128) * gy;
   // A forward launch too big to share its 256-row tiles between two workgroups (below) and
@@ -1073,6 +1134,11 @@ RowsGrid rows_grid(int64_t n_dst, unsigned gy, int stages, bool can_half, bool h
                         : input_gradient ? (int64_t)num_cus() * 9 / 4 : (int64_t)num_cus() * wgs_per_cu;
   g.gz = 1;
   g.part_stages = 1;
+  g.groups = 1;
+  if (g.half_tiles && can_group && stages >= 4 && (int64_t)g.gx * gy <= (int64_t)num_cus() * 2) {
+    g.groups = (int64_t)g.gx * gy <= num_cus() ? 4 : 2;
+    return g;
+  }
   if (!pair_view && (int64_t)g.gx * gy * 2 <= slots && stages >= 8) {
     g.part_stages = (stages + 1) / 2;
     g.gz = 2;
@@ -1127,25 +1193,30 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
   const unsigned gy = (unsigned)(s.c_dst / (32 * NT));
   constexpr bool kCanHalf = NT != 4;
   const RowsGrid rg = rows_grid(a.n_dst, gy, a.k_vol * slabs, kCanHalf, tile_order != nullptr, tile_grid, pair_view,
-                                NT == 4 ? 2 : 3, a.transpose_w);
+                                NT == 4 ? 2 : 3, a.transpose_w, kCanHalf && !a.transpose_w);
   const bool half_tiles = rg.half_tiles;
   if (rg.drop_table) tile_order = nullptr;
-  const size_t lds_rows = half_tiles ? s.lds_rows_bytes - (size_t)kWaves * 32 * (2 * S * 16 + 3 * sizeof(int))
-                                     : s.lds_rows_bytes;
+  constexpr int kHalfMT = kCanHalf ? 1 : 2;
+  constexpr size_t kGroup = rows_group_chunks<T, NT, S, kHalfMT>() * 16, kSums = rows_sum_chunks<NT, kHalfMT>() * 16;
+  const int kg = half_tiles ? rg.groups : 1;
+  size_t lds_rows = half_tiles ? kGroup * kg : s.lds_rows_bytes;
+  if (kg > 1 && lds_rows < kGroup + kSums * (kg - 1)) lds_rows = kGroup + kSums * (kg - 1);
   const unsigned gx = rg.gx;
   if (gx == 0) return a.side.kind ? launch_side_job(a.side, a.stream) : FGMS_OK;
   constexpr bool kCanRaw = NT != 4;
-  constexpr int kHalfMT = kCanHalf ? 1 : 2;
-  auto kern = half_tiles ? (raw == 4   ? gms_rows_kernel<T, NT, S, kCanSplit ? 4 : 0, kHalfMT>
-                            : raw == 3 ? gms_rows_kernel<T, NT, S, kCanSplit ? 3 : 0, kHalfMT>
-                            : raw == 2 ? gms_rows_kernel<T, NT, S, kCanRaw ? 2 : 0, kHalfMT>
-                            : raw == 1 ? gms_rows_kernel<T, NT, S, kCanRaw && sizeof(T) == 2 ? 1 : 0, kHalfMT>
-                                       : gms_rows_kernel<T, NT, S, 0, kHalfMT>)
-              : raw == 4 ? gms_rows_kernel<T, NT, S, kCanSplit ? 4 : 0>
-              : raw == 3 ? gms_rows_kernel<T, NT, S, kCanSplit ? 3 : 0>
-              : raw == 2 ? gms_rows_kernel<T, NT, S, kCanRaw ? 2 : 0>
-              : raw == 1 ? gms_rows_kernel<T, NT, S, kCanRaw && sizeof(T) == 2 ? 1 : 0>
-                         : gms_rows_kernel<T, NT, S, 0>;
+  constexpr int kRaw4 = kCanSplit ? 4 : 0, kRaw3 = kCanSplit ? 3 : 0, kRaw2 = kCanRaw ? 2 : 0, kRaw1 = kCanRaw && sizeof(T) == 2 ? 1 : 0;
+  // (raw is one of the five the type and the tile allow)
+#define FGMS_BY_RAW(MTv, KGv)                                                                                       \
+  (raw == 4   ? gms_rows_kernel<T, NT, S, kRaw4, MTv, KGv>                                                          \
+   : raw == 3 ? gms_rows_kernel<T, NT, S, kRaw3, MTv, KGv>                                                          \
+   : raw == 2 ? gms_rows_kernel<T, NT, S, kRaw2, MTv, KGv>                                                          \
+   : raw == 1 ? gms_rows_kernel<T, NT, S, kRaw1, MTv, KGv>                                                          \
+              : gms_rows_kernel<T, NT, S, 0, MTv, KGv>)
+  auto kern = FGMS_BY_RAW(2, 1);
+  if constexpr (kCanHalf) {
+    if (half_tiles) kern = kg == 4 ? FGMS_BY_RAW(1, 4) : kg == 2 ? FGMS_BY_RAW(1, 2) : FGMS_BY_RAW(1, 1);
+  }
+#undef FGMS_BY_RAW
   { const int rc_lds = allow_dynamic_lds(reinterpret_cast<const void *>(kern), lds_rows); if (rc_lds != FGMS_OK) return rc_lds; }
   // (a tile shared by two workgroups is added up with atomics: its rows start from zero)
   const bool overwrite = a.overwrite && rg.gz == 1 && !pair_view;
@@ -1160,7 +1231,7 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
                       : raw == 3 ? "gms_rows_kernel(fwd, bf16x3)"
                       : a.transpose_w ? "gms_rows_kernel(dgrad)" : "gms_rows_kernel(fwd)",
                       a.stream);
-    kern<<<dim3(gx + (unsigned)a.side.blocks, gy, gz), kThreads, lds_rows, a.stream>>>(
+    kern<<<dim3(gx + (unsigned)a.side.blocks, gy, gz), kThreads * kg, lds_rows, a.stream>>>(
         (const T *)a.src, packed, (T *)a.dst, nbr, masks, perm, tile_order, (int)a.n_dst, a.k_vol,
         s.c_src, s.c_dst, part_stages > 0 ? part_stages : 1, a.side, pair_view ? 1 : 0,
         (unsigned)((size_t)a.n_src * s.c_src * sizeof(T)), overwrite ? 1 : 0, flip);
@@ -1230,7 +1301,7 @@ int launch_fused(const GmsArgs &d, const Shape &s, const Plan *p, const WgradArg
   const unsigned row_y = (unsigned)(s.c_dst / (32 * NT));
   constexpr bool kCanHalf = NT != 4;
   const RowsGrid rg = rows_grid(d.n_dst, row_y, d.k_vol * slabs, kCanHalf, p->tile_in != nullptr, p->tile_grid_in,
-                                false, NT == 4 ? 2 : 3, true);
+                                false, NT == 4 ? 2 : 3, true, false);
   const unsigned row_x = (rg.gx + 7) / 8 * 8;
   const int part_stages = rg.part_stages;
   const unsigned row_z = rg.gz;
