@@ -1135,6 +1135,11 @@ RowsGrid rows_grid(int64_t n_dst, unsigned gy, int stages, bool can_half, bool h
   g.gz = 1;
   g.part_stages = 1;
   g.groups = 1;
+  // Forward: no sharing between workgroups but groups of waves inside them, four where every CU has at
+  // most one workgroup, two up to two of them (64 -> 64 fp16 over 20 k / 32 k / 45 k / 64 k voxels of
+  // the indoor cloud, a whole call: 17.8 -> 15.8, 19.1 -> 17.2, 21.0 -> 19.8, 25.4 -> 22.3 us).  Four
+  // waves already keep a CU's matrix cores busy, so groups hide latency but do not make the products
+  // of one CU faster: launch_rows therefore takes 32-column tiles while these leave CUs idle.
   if (g.half_tiles && can_group && stages >= 4 && (int64_t)g.gx * gy <= (int64_t)num_cus() * 2) {
     g.groups = (int64_t)g.gx * gy <= num_cus() ? 4 : 2;
     return g;
@@ -1156,6 +1161,20 @@ template <typename T, int NT, int S>
 int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
                 const unsigned long long *masks, const int32_t *perm, const int32_t *tile_order,
                 int tile_grid, int flip, bool pair_view = false) {
+  const int slabs = s.c_src / (2 * S * s.E);
+  const unsigned gy = (unsigned)(s.c_dst / (32 * NT));
+  constexpr bool kCanHalf = NT != 4;
+  const RowsGrid rg = rows_grid(a.n_dst, gy, a.k_vol * slabs, kCanHalf, tile_order != nullptr, tile_grid, pair_view,
+                                NT == 4 ? 2 : 3, a.transpose_w, kCanHalf && !a.transpose_w);
+  // Few tiles: column tiles of 32 put them on twice the CUs, as long as each still has one to itself.
+  // A tile's rows are then gathered twice, by CUs that had nothing to do.  Against two workgroups
+  // per 64-column tile and atomics / 64-column tiles with four groups: 64 -> 64 fp16 over 1 k voxels
+  // 14.3 / 15.3 -> 12.4 us, 5 k 14.4 / 15.0 -> 12.2, 12 k 15.3 / 15.4 -> 13.1; fp32 over 2 k
+  // 47.2 / 66.4 -> 40.9; tf32 mode over 5 k 35.2 / 31.6 -> 27.4; 128 -> 128 fp16 over 2 k 21.8 / 24.1 -> 19.5.
+  if constexpr (NT == 2) {
+    if (rg.groups == 4 && (int64_t)rg.gx * gy * 2 <= num_cus())
+      return launch_rows<T, 1, S>(a, s, nbr, masks, perm, tile_order, tile_grid, flip, pair_view);
+  }
   // With 64-column wave tiles the input gradient and the fp16 forward pass read the weight
   // tensor as it is (16-byte aligned rows of the tile) when the caller brings no re-laid
   // copy; the rest gets one, made here.  Measured: 64 -> 64 over 200k voxels, input gradient
@@ -1189,11 +1208,6 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
     int rc = pack_weights<T>(a, s, &packed);
     if (rc != FGMS_OK) return rc;
   }
-  const int slabs = s.c_src / (2 * S * s.E);
-  const unsigned gy = (unsigned)(s.c_dst / (32 * NT));
-  constexpr bool kCanHalf = NT != 4;
-  const RowsGrid rg = rows_grid(a.n_dst, gy, a.k_vol * slabs, kCanHalf, tile_order != nullptr, tile_grid, pair_view,
-                                NT == 4 ? 2 : 3, a.transpose_w, kCanHalf && !a.transpose_w);
   const bool half_tiles = rg.half_tiles;
   if (rg.drop_table) tile_order = nullptr;
   constexpr int kHalfMT = kCanHalf ? 1 : 2;

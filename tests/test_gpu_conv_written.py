@@ -62,3 +62,21 @@ def test_no_pairs():
     capi.conv_fwd(x, w, out, kpos, none, none)
     capi.conv_bwd(x, x, w, gi, gw, kpos, none, none)
     assert not out.any() and not gi.any() and not gw.any()
+
+
+@pytest.mark.parametrize("dtype,tf32", [(np.float16, False), (np.float32, False), (np.float32, True)], ids=["fp16", "fp32", "tf32"])
+@pytest.mark.parametrize("n", [1, 127, 129, 16384, 16385, 32768, 32769, 65536, 65537])
+def test_small_forward_launches(oracle, n, dtype, tf32):
+    """The edges of the choice of column tiles and groups of waves (128-row tiles against 256 CUs)."""
+    from fgms_amd import capi
+    rng = np.random.default_rng(n)
+    knnz = np.array([0 if k == 4 else min(n, 1 + 40 * k) for k in range(27)], np.int32)
+    side = lambda: np.concatenate([np.sort(rng.permutation(n)[:m]) for m in knnz]).astype(np.int32)
+    kpos = np.concatenate([[0], np.cumsum(knnz)]).astype(np.int32)
+    L = clouds.make_layer(rng, side(), side(), knnz, kpos, n, n, 64, 64, dtype)
+    D = G.to_dev(L)
+    plan = capi.Plan(D["kpos"], D["imap"], D["omap"], n, n)
+    out = torch.full((n, 64), float("nan"), dtype=D["in_feats"].dtype, device="cuda")
+    capi.conv_fwd(D["in_feats"], D["kernel"], out, D["kpos"], D["imap"], D["omap"], arch80=tf32, plan=plan)
+    ref = oracle.c_fwd(L["in_feats"], L["kernel"], L["knnz"], L["imap"], L["omap"], n)
+    G.assert_close(out.cpu().numpy(), ref, G.mode_of(L["in_feats"].dtype, tf32), "fwd")
