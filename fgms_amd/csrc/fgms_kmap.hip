@@ -396,7 +396,7 @@ __global__ __launch_bounds__(256) void kmap_lists_kernel(ListArgs a, SortArgs so
   if (list_block >= list_blocks) {
     const int b = list_block - list_blocks;
     const int side = b < sort.side[0].chunks ? 0 : 1;
-    sort_hist_body(sort.side[side], sort.k_vol, side ? b - sort.side[0].chunks : b, tile, 256);
+    sort_hist_body(sort.side[side], sort, side ? b - sort.side[0].chunks : b, tile, 256);
     return;
   }
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
@@ -604,6 +604,7 @@ int map_build_begin(MapBuild **build, const int32_t *in_coords, int64_t n_in, co
     p->tile_grid_out = p->tile_out ? cap_out * 8 : 0;
     p->tile_grid_in = p->tile_in ? cap_in * 8 : 0;
     sort.flags = p->flags;
+    sort.kpos = kpos;
     sort.side[0].rmask = rmask_out; sort.side[0].perm = p->perm_out; sort.side[0].block_mask = p->mask_out;
     if (!mirror) {
       sort.side[1].rmask = rmask_in; sort.side[1].perm = p->perm_in; sort.side[1].block_mask = p->mask_in;

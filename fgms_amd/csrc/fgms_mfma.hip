@@ -1115,13 +1115,14 @@ RowsGrid rows_grid(int64_t n_dst, unsigned gy, int stages, bool can_half, bool h
                    bool pair_view, int wgs_per_cu, bool input_gradient, bool can_group) {
   RowsGrid g{};
   const int64_t small_tiles = (int64_t)((n_dst + 127) / 128) * gy;
+  const int64_t tiles = (n_dst + kTileRows - 1) / kTileRows;      // (the table has more entries than tiles)
   // A forward launch too big to share its 256-row tiles between two workgroups (below) and
   // not yet a full round of them is neither short-chained nor busy: 128-row tiles in plain order
   // then beat the table's XCD-aware 256-row tiles (64 -> 64 fp16 over 100 k / 130 k voxels:
   // 40.9 -> 34.4, 41.2 -> 36.9 us; 70 k / 80 k voxels with shared 256-row tiles: 28.1 / 29.1 us).
   g.drop_table = can_half && half_tiles_enabled() && has_table && !pair_view && !input_gradient &&
                  small_tiles <= (int64_t)num_cus() * 4 &&
-                 ((int64_t)table_grid * gy * 2 > (int64_t)num_cus() * wgs_per_cu || stages < 8);
+                 (tiles * gy * 2 > (int64_t)num_cus() * wgs_per_cu || stages < 8);
   if (g.drop_table) has_table = false;
   g.half_tiles = can_half && half_tiles_enabled() && !has_table && !pair_view &&
                  (input_gradient ? small_tiles * 4 <= (int64_t)num_cus() * 3 : small_tiles <= (int64_t)num_cus() * 4);
@@ -1144,7 +1145,7 @@ RowsGrid rows_grid(int64_t n_dst, unsigned gy, int stages, bool can_half, bool h
     g.groups = (int64_t)g.gx * gy <= num_cus() ? 4 : 2;
     return g;
   }
-  if (!pair_view && (int64_t)g.gx * gy * 2 <= slots && stages >= 8) {
+  if (!pair_view && (has_table ? tiles : (int64_t)g.gx) * gy * 2 <= slots && stages >= 8) {
     g.part_stages = (stages + 1) / 2;
     g.gz = 2;
   }

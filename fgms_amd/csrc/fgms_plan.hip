@@ -88,24 +88,23 @@ __global__ void pair_masks_kernel(const int32_t *__restrict__ kpos, const int32_
                               __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Step 2: the order in which a side's rows are visited.  Rows are sorted by their offset mask
-// (as a number), so that the 64 rows of a wave use nearly the same offsets and whole (block,
-// offset) steps can be skipped: on a surface-like cloud of 200 k voxels the number of such
-// steps drops from 68.6 k to 37 k (33 k would be perfect).  Numerically close masks share their
-// high offsets, which is what makes neighbours in the order similar; so the sort runs most
-// significant bits first: a counting sort on the top kBinBits bits of the mask over the whole
-// side (histogram per chunk of rows, scan, stable scatter), then a full sort by (mask, row) of
+// Step 2: the order in which a side's rows are visited.  Rows are sorted by the set of their offsets
+// (sort_key), so that the 64 rows of a wave and the 256 of a workgroup use nearly the same offsets and
+// whole (block, offset) steps can be skipped: on a surface-like cloud of 200 k voxels the number of
+// such steps drops from 68.6 k to 36.3 k (33 k would be perfect).  Close keys share their high bits,
+// which is what makes neighbours in the order similar; so the sort runs most
+// significant bits first: a counting sort on the top kBinBits bits of the key over the whole
+// side (histogram per chunk of rows, scan, stable scatter), then a full sort by (key, row) of
 // every window of kWindow positions.  Inside a bin only rows of one window are ordered
-// among themselves; measured on the benchmark clouds that costs 1 % more (block, offset) steps
-// than the exact sort, for a third of its time.  (Bins of 16 bits without the windows: 4 % more
-// steps on surfaces, 23 % on scattered clouds; windows of 2048: 0.3 % fewer steps on surfaces, 3 % on
-// scattered clouds, for twice the sort.)  Both sides of a plan go through the same
+// among themselves; that costs 1.5 % more (block, offset) steps than the exact sort on 200 k indoor
+// voxels, 2 % on 120 k LiDAR voxels and 28 % on 50 k scattered ones (windows of 2048: 0.5 %, 0.7 % and
+// 7 % fewer steps).  Both sides of a plan go through the same
 // launches (blockIdx.y = side).
 __global__ __launch_bounds__(kSortThreads) void sort_hist_kernel(SortArgs a) {
   const SortSide &sd = a.side[blockIdx.y];
   if ((int)blockIdx.x >= sd.chunks) return;
   __shared__ int hist[kBins];
-  sort_hist_body(sd, a.k_vol, blockIdx.x, hist, kSortThreads);
+  sort_hist_body(sd, a, blockIdx.x, hist, kSortThreads);
 }
 
 // hist[chunk][bin] -> hist_before[chunk][bin] = rows of the bin in earlier chunks, and
@@ -211,7 +210,7 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(SortArgs a) 
   for (int r = 0; r < kBatches; ++r) {
     const int row = chunk * kChunk + (wave * kBatches + r) * 64 + lane;
     const bool live = row < sd.n;
-    bin[r] = live ? top_bits(sd.rmask[row], a.k_vol) : -1;
+    bin[r] = live ? top_bits(sd.key[row], a.k_vol) : -1;
     unsigned long long same = __ballot(live);
 #pragma unroll
     for (int bit = 0; bit < kBinBits; ++bit) {
@@ -270,8 +269,8 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(SortArgs a) 
     if (bin[r] >= 0) sd.perm_tmp[at[r] + rank[r]] = chunk * kChunk + (wave * kBatches + r) * 64 + lane;
 }
 
-// Full sort by (mask, row) of a window of positions (of masks over more than 32 offsets: by the top
-// 32); writes the final order and its inverse, and what the window's blocks of 64 positions use:
+// Full sort by (key, row) of a window of positions (of keys over more than 32 offsets: by the top
+// 32 bits); writes the final order and its inverse, and what the window's blocks of 64 positions use:
 // block_mask = the OR of their rows' masks, flags[4 + side] += (block, offset) combinations in use,
 // flags[10 + side] += offset bits of all rows.  chunks == 0: the window starts from the identity
 // order (sides of one window).
@@ -284,13 +283,19 @@ __global__ __launch_bounds__(kWindowThreads) void sort_window_kernel(SortArgs a)
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, base = wave * 128;
   const int shift = a.k_vol > 32 ? a.k_vol - 32 : 0;
   unsigned long long key[2];
+  __shared__ unsigned char order[64];
+  if (a.by_mask && sd.chunks == 0) {           // (no histogram has left keys)
+    sort_offset_order(a.kpos, a.k_vol, order);
+    __syncthreads();
+  }
 #pragma unroll
   for (int r = 0; r < 2; ++r) {
     const int p = p0 + base + r * 64 + lane;
     key[r] = ~0ull;
     if (p < sd.n) {
       const int row = sd.chunks ? sd.perm_tmp[p] : p;
-      key[r] = (a.by_mask ? (sd.rmask[row] >> shift) << 32 : 0ull) | (unsigned)row;
+      const unsigned long long full = !a.by_mask ? 0ull : sd.chunks ? sd.key[row] : sort_key(sd.rmask[row], a.k_vol, order);
+      key[r] = (full >> shift) << 32 | (unsigned)row;
     }
   }
   int flip = 0;
@@ -304,7 +309,7 @@ __global__ __launch_bounds__(kWindowThreads) void sort_window_kernel(SortArgs a)
       const int row = (int)(unsigned)key[r];
       sd.perm[p] = row;
       sd.inv[row] = p;
-      m = a.by_mask && shift == 0 ? key[r] >> 32 : sd.rmask[row];
+      m = sd.rmask[row];
     }
     int rb = __popcll(m);
     for (int d = 32; d > 0; d >>= 1) {
@@ -369,94 +374,156 @@ __global__ void pair_view_kernel(const int32_t *__restrict__ kpos, const int32_t
 // Dispatch order of the 256-position tiles of the output-stationary kernel.
 // Workgroup b runs on XCD b % 8 and, inside an XCD, workgroup number q = b / 8
 // lands on CU q % cus_per_xcd (the dispatcher goes round the CUs).
-//  * A tile's home XCD is the eighth of the cloud its middle row lies in
+//  * A tile's weight is the number of offsets it uses and a little for its start and end.
+//  * A tile's home XCD is the eighth of the cloud's weight its middle row lies in
 //    (original row numbers follow the voxel order, i.e. space), so that
-//    neighbouring rows meet in one L2.
-//  * Inside an XCD the tiles are ranked by the number of offsets they use, most
-//    first: the launch lasts as long as its longest tile, so those must start
-//    first.  Ranks are laid over the CUs in a snake (first sweep forwards, second
-//    backwards, ...), so every CU gets a mix of long and short tiles instead of
-//    three long ones competing for the same SIMDs.
-//  * Every XCD takes at most cap = ceil(tiles / 8) tiles; the lightest tiles of an
+//    neighbouring rows meet in one L2 and the XCDs get equal work.
+//  * Inside an XCD the tiles are ranked by weight, heaviest first: those must start first.  The
+//    first kHeadRounds tiles of a CU are resident together, so the launch lasts as long as the
+//    heaviest such sum: in every round the heaviest tile goes to the CU with the least so far.
+//    Tiles behind those go to whichever CU has room.
+//  * Every XCD takes at most cap tiles (tile_table); the lightest tiles of an
 //    overfull XCD go to the XCDs that have room.
+// Counted on 200 k indoor / 120 k LiDAR voxels, offsets of the busiest CU (the mean is 40 / 31): with
+// eighths of the rows and a snake over the CUs 60 / 43, like this 48 / 37; 64 -> 64 over the former fp16
+// forward 41.2 -> 40.1 us, in tf32 mode 110.7 -> 104.7, 128 -> 128 fp16 over the latter 82.0 -> 79.9.
 // order[q * 8 + xcd] = tile | first offset << 24, -1 where no tile lands.  One workgroup; which of two
 // equally heavy tiles comes first depends on timing, the results do not.
-__device__ __forceinline__ void tile_order_body(const TileSide &sd, int cus_per_xcd, int32_t *__restrict__ spill) {
+constexpr int kHeadRounds = 3, kHeadCus = 32, kHomeBuckets = 512;
+__device__ __forceinline__ void tile_order_body(const TileSide &sd, int cus_per_xcd, int32_t *__restrict__ tiles) {
   const int32_t *__restrict__ perm = sd.perm;
   const unsigned long long *__restrict__ block_masks = sd.block_masks;
   int32_t *__restrict__ order = sd.order;
   const int n_rows = sd.n_rows, n_tiles = sd.n_tiles, cap = sd.cap;
   if (!order) return;
   constexpr int kPc = 65;                         // popcount classes 0..64
-  __shared__ int hist[8][kPc];                    // tiles per (home, popcount), then start ranks
-  __shared__ int cursor[8][kPc];
+  __shared__ int rank_of[8][kPc];                 // tiles per (home, popcount), then the next rank of each
   __shared__ int total[8];
+  __shared__ int before[kHomeBuckets];            // weight by middle row, then that in front of it
+  __shared__ unsigned short head[8][kHeadRounds * kHeadCus];     // the first tiles by rank
+  __shared__ int wave_sum[4];
   __shared__ int spill_count;
-  const int tid = threadIdx.x, threads = blockDim.x;     // (spill: n_tiles ints of LDS)
+  const int tid = threadIdx.x, threads = blockDim.x;     // (256 threads)
   const int n_blocks = (n_rows + 63) / 64;
-  for (int i = tid; i < 8 * kPc; i += threads) {
-    (&hist[0][0])[i] = 0;
-    (&cursor[0][0])[i] = 0;
-  }
+  const int head_ranks = cus_per_xcd <= kHeadCus ? min(kHeadRounds * cus_per_xcd, cap) : 0;
+  constexpr unsigned short kNoTile = 0xffff;             // (tile_table: at most 15000 tiles)
+  for (int i = tid; i < 8 * kPc; i += threads) (&rank_of[0][0])[i] = 0;
+  for (int i = tid; i < kHomeBuckets; i += threads) before[i] = 0;
+  for (int i = tid; i < 8 * kHeadRounds * kHeadCus; i += threads) (&head[0][0])[i] = kNoTile;
   if (tid == 0) spill_count = 0;
   for (int i = tid; i < cap * 8; i += threads) order[i] = -1;     // (slots no tile lands in)
   __syncthreads();
+  // tiles[t] (n_tiles ints of LDS): number of offsets, first offset << 7, bucket or home << 13
+  auto count_of = [](int info) { return info & 127; };
+  auto weight_of = [](int info) { return (info & 127) + 2; };
   // entry of tile t in the table: t in the low 24 bits, the first offset the tile uses above
   // them (the kernel starts that offset's index load before it has seen the tile's masks)
-  auto classify = [&](int t, int &home, int &pc, int &entry) {
+  auto entry_of = [](int t, int info) { return t | (info >> 7 & 63) << 24; };
+  for (int t = tid; t < n_tiles; t += threads) {
     const int mid = min(t * 256 + 128, n_rows - 1);
-    home = (int)((long long)(perm ? perm[mid] : mid) * 8 / n_rows);
+    const int bucket = (int)((long long)(perm ? perm[mid] : mid) * kHomeBuckets / n_rows);
     unsigned long long m = 0;
 #pragma unroll
     for (int q = 0; q < 4; ++q) m |= block_masks[min(4 * t + q, n_blocks - 1)];
-    pc = __builtin_popcountll(m);
-    entry = t | ((m ? __builtin_ctzll(m) : 0) << 24);
-  };
+    const int info = __builtin_popcountll(m) | (m ? __builtin_ctzll(m) : 0) << 7 | bucket << 13;
+    tiles[t] = info;
+    atomicAdd(&before[bucket], weight_of(info));
+  }
+  __syncthreads();
+  // weight in front of the middle of each bucket
+  int all = 0;
+  {
+    constexpr int kPer = kHomeBuckets / 256;
+    int w[kPer], sum = 0;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) { w[i] = before[tid * kPer + i]; sum += w[i]; }
+    int incl = sum;
+    for (int d = 1; d < 64; d <<= 1) {
+      const int up = __shfl_up(incl, d);
+      if (tid % 64 >= d) incl += up;
+    }
+    if (tid % 64 == 63) wave_sum[tid / 64] = incl;
+    __syncthreads();
+    int run = incl - sum;
+    for (int q = 0; q < 4; ++q) {
+      if (q < tid / 64) run += wave_sum[q];
+      all += wave_sum[q];
+    }
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      before[tid * kPer + i] = run + w[i] / 2;
+      run += w[i];
+    }
+  }
+  __syncthreads();
   for (int t = tid; t < n_tiles; t += threads) {
-    int home, pc, entry;
-    classify(t, home, pc, entry);
-    atomicAdd(&hist[home][pc], 1);
+    const int info = tiles[t];
+    const int home = min(7, before[info >> 13] * 8 / max(all, 1));
+    tiles[t] = (info & 0x1fff) | home << 13;
+    atomicAdd(&rank_of[home][count_of(info)], 1);
   }
   __syncthreads();
   // start rank of each class, heaviest first: a wave per home, lane l takes class 64 - l
   for (int home = tid / 64; home < 8; home += threads / 64) {
     const int lane = tid % 64, pc = 64 - lane;
-    const int n = hist[home][pc];
+    const int n = rank_of[home][pc];
     int incl = n;
     for (int d = 1; d < 64; d <<= 1) {
       const int up = __shfl_up(incl, d);
       if (lane >= d) incl += up;
     }
-    hist[home][pc] = incl - n;
+    rank_of[home][pc] = incl - n;
     if (lane == 63) {
-      const int n0 = hist[home][0];
-      hist[home][0] = incl;
+      const int n0 = rank_of[home][0];
+      rank_of[home][0] = incl;
       total[home] = incl + n0;
     }
   }
   __syncthreads();
-  auto position = [&](int rank) {                 // snake over the CUs
-    const int round = rank / cus_per_xcd, j = rank % cus_per_xcd;
-    const int in_round = min(cus_per_xcd, cap - round * cus_per_xcd);
-    return round * cus_per_xcd + ((round & 1) ? in_round - 1 - j : j);
+  auto place = [&](int home, int rank, int t, int info) {
+    if (rank < head_ranks) head[home][rank] = (unsigned short)t;
+    else order[rank * 8 + home] = entry_of(t, info);
   };
+  constexpr int kSpilled = 1 << 16;
   for (int t = tid; t < n_tiles; t += threads) {
-    int home, pc, entry;
-    classify(t, home, pc, entry);
-    const int rank = hist[home][pc] + atomicAdd(&cursor[home][pc], 1);
-    if (rank < cap) order[position(rank) * 8 + home] = entry;
-    else spill[atomicAdd(&spill_count, 1)] = entry;
+    const int info = tiles[t], home = info >> 13;
+    const int rank = atomicAdd(&rank_of[home][count_of(info)], 1);
+    if (rank < cap) place(home, rank, t, info);
+    else tiles[t] = info | kSpilled;
   }
   __syncthreads();
-  for (int sidx = tid; sidx < spill_count; sidx += threads) {
-    int left = sidx;
+  for (int t = tid; t < n_tiles; t += threads) {
+    const int info = tiles[t];
+    if (!(info & kSpilled)) continue;
+    int left = atomicAdd(&spill_count, 1);
     for (int q = 0; q < 8; ++q) {
       const int filled = min(total[q], cap), room = cap - filled;
       if (left < room) {
-        order[position(filled + left) * 8 + q] = spill[sidx];
+        place(q, filled + left, t, info);
         break;
       }
       left -= room;
+    }
+  }
+  __syncthreads();
+  // the head: half a wave per home, a lane per CU
+  {
+    const int home = tid / 32, lane = tid % 32;
+    int sum = 0;
+    for (int first = 0; first < head_ranks; first += cus_per_xcd) {
+      const int n = min(cus_per_xcd, head_ranks - first);
+      int nth = 0;                                   // CUs of this round with less so far
+      for (int o = 0; o < n; ++o) {
+        const int theirs = __shfl(sum, o, 32);
+        nth += theirs < sum || (theirs == sum && o < lane) ? 1 : 0;
+      }
+      if (lane < n) {
+        const int t = head[home][first + nth];
+        if (t != kNoTile) {
+          order[(first + lane) * 8 + home] = entry_of(t, tiles[t]);
+          sum += weight_of(tiles[t]);
+        }
+      }
     }
   }
 }
@@ -653,6 +720,7 @@ void sort_side_layout(SortSide &sd, int64_t n, Arena &tmp) {
     tmp.take(sd.hist, (size_t)kBins * sd.chunks);
     tmp.take(sd.hist_before, (size_t)kBins * sd.chunks);
     tmp.take(sd.bin_start, (size_t)kBins);
+    tmp.take(sd.key, (size_t)n);
   }
 }
 
@@ -720,10 +788,11 @@ void plan_bands(Plan *p) {
 }
 
 // Tile -> XCD homes pay off once every XCD has a few dozen tiles of its own.
+// (cap: an eighth more than an eighth of them, for an XCD with many light tiles)
 int tile_table(int64_t n, int *cap) {
   static const bool xcd_homes = !(getenv("FGMS_XCD_HOME") && atoi(getenv("FGMS_XCD_HOME")) == 0);
   const int64_t n_tiles = (n + 255) / 256;
-  *cap = (int)((n_tiles + 7) / 8);
+  *cap = (int)((n_tiles * 9 / 8 + 7) / 8);
   return xcd_homes && n_tiles >= 256 && n_tiles * sizeof(int32_t) <= 60000 ? (int)n_tiles : 0;
 }
 
@@ -834,6 +903,7 @@ int plan_create(fgms_plan_t **plan_out, const int32_t *kpos, const int32_t *in_m
     p->tile_grid_out = p->tile_out ? cap_out * 8 : 0;
     p->tile_grid_in = p->tile_in ? cap_in * 8 : 0;
     sa.flags = p->flags;
+    sa.kpos = kpos;
     sa.side[0].rmask = rmask; sa.side[0].perm = p->perm_out; sa.side[0].block_mask = p->mask_out;
     sa.side[1].rmask = rmask + n_out; sa.side[1].perm = p->perm_in; sa.side[1].block_mask = p->mask_in;
   }

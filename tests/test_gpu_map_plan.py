@@ -100,3 +100,14 @@ def test_maps_begun_together_and_used_elsewhere(oracle):
         torch.cuda.synchronize()
         assert np.array_equal(im.cpu().numpy(), imap)
         G.assert_close(y.cpu().numpy(), oracle.c_fwd(x.cpu().numpy(), w.cpu().numpy(), knnz, imap, omap, len(v)), "fp32", "fwd")
+
+
+def test_tiles_of_very_different_weight(oracle):
+    """Most voxels alone, the rest in one solid block: equal work per XCD then means very unequal numbers
+    of tiles, more than the tile table has room for in one of them."""
+    grid = np.stack(np.meshgrid(*[np.arange(38)] * 3, indexing="ij"), -1).reshape(-1, 3)[:50000] * 3
+    solid = np.stack(np.meshgrid(*[np.arange(27)] * 3, indexing="ij"), -1).reshape(-1, 3) + [200, 0, 0]
+    vox = np.concatenate([grid, solid]).astype(np.int32)
+    vox = vox[np.lexsort(vox.T[::-1])]
+    vox = np.concatenate([np.zeros((len(vox), cloud(1).shape[1] - 3), np.int32), vox], 1) if cloud(1).shape[1] > 3 else vox
+    check(oracle, vox, vox, clouds.offsets_cube(3), 1, 64, 64)
