@@ -274,6 +274,11 @@ int planned_pack_job(const GmsArgs &a, SideJob *job, const void **packed);
 int launch_fused_bwd(const GmsArgs &d, const struct Plan *p, const WgradArgs &w, bool *done);
 // Runs a side job in a launch of its own.
 int launch_side_job(const SideJob &job, hipStream_t stream);
+// Tiles 96 columns wide save repeated gathers of rows, at the price of waves: for maps with several pairs to
+// a row.  (96 <-> 128 fp16 down and up over 100 k voxels, one pair a row: backward launches 52.8 us with
+// 32-wide tiles, 53.9 with 96; 96 -> 96 over 40 k scattered ones, 3.3 pairs a row, forward and backward 100 us
+// against 108; the submanifold maps that gain by it have 10.)
+inline bool worth_96_columns(int64_t n_pairs, int64_t n_a, int64_t n_b) { return n_pairs >= 5 * (n_a > n_b ? n_a : n_b); }
 bool split_bf16_enabled();   // products of fp32 tensors in split bf16 where the caller allows tf32 precision
 bool small_gms_supported(const GmsArgs &a, const Plan *p);
 int launch_small_gms(const GmsArgs &a, const Plan *p);

@@ -381,7 +381,7 @@ __device__ __forceinline__ void gather_issue_buf(int4v (&v)[N], const unsigned *
   constexpr int C = 2 * S;
   unsigned off[N];
 #pragma unroll
-  for (int it = 0; it < N; ++it) off[it] = offs[(it * 64 + lane) / C] + (unsigned)((lane % C) * 16);
+  for (int it = 0; it < N; ++it) off[it] = offs[(it * 64 + lane) / C] + (unsigned)(((it * 64 + lane) % C) * 16);
 #pragma unroll
   for (int it = 0; it < N; ++it)
     v[it] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off[it], slab * (C * 16), 0));
@@ -954,7 +954,7 @@ __device__ __forceinline__ void gms_rows_body(
 }
 
 template <typename T, int NT, int S, int RAW, int MT = 2, int KG = 1>
-__global__ __launch_bounds__(kThreads * KG, MT == 1 ? 4 : (NT == 4 ? 2 : 3)) void gms_rows_kernel(
+__global__ __launch_bounds__(kThreads * KG, MT == 1 ? (NT == 3 ? 3 : 4) : (NT >= 3 ? 2 : 3)) void gms_rows_kernel(
     const T *__restrict__ src, const T *__restrict__ packed, T *__restrict__ dst,
     const int32_t *__restrict__ nbr, const unsigned long long *__restrict__ block_masks,
     const int32_t *__restrict__ perm, const int32_t *__restrict__ tile_order, int n_dst, int k_vol,
@@ -977,7 +977,7 @@ __global__ __launch_bounds__(kThreads * KG, MT == 1 ? 4 : (NT == 4 ? 2 : 3)) voi
 // ---------------------------------------------------------------------------
 struct Shape {
   int c_src, c_dst, S, NT, E;
-  int NTR;                // 32-column tiles per wave in the output-stationary kernel
+  int NTR, SR;            // 32-column tiles per wave and k-steps per slab in the output-stationary kernel
   size_t lds_bytes;       // pair-stationary kernel
   size_t lds_rows_bytes;  // output-stationary kernel
   bool ok;
@@ -1004,25 +1004,35 @@ Shape shape_of(const GmsArgs &a) {
   // fill the chip; fp32 has 8x the MFMA time per gathered byte and gains nothing.
   const int64_t wide_wgs = (a.n_dst + kTileRows - 1) / kTileRows * (s.c_dst / 128);
   const bool wide = kernel_policy() == 3 || (a.dtype == FGMS_F16 && wide_wgs * 2 >= 3 * (int64_t)num_cus());
-  s.NTR = (s.c_dst % 128 == 0 && wide) ? 4 : s.NT;
-  s.lds_rows_bytes = 2 * (size_t)s.S * s.NTR * 64 * 16 + tiles;  // + two stages of weights
+  // 96 columns: a row is gathered once for all of them, not once per 32; 48 channels (fp16; 24 fp32):
+  // one slab, not three of 16.  96 -> 96 fp16 over 80 k voxels forward 57.5 -> 45.8 us, 48 -> 96 48.5 -> 26.5,
+  // 24 -> 32 fp32 over 40 k 39.6 -> 27.1.  fp32 products keep 32 columns: they take 16 times the matrix
+  // time, so that more waves are worth more than fewer gathers (96 -> 96 over 40 k: 127.5 us against 184.8
+  // with 96); in tf32 mode the forward pass takes 96 once there are tiles enough (over 150 k 243.9 ->
+  // 166.2 us, over 40 k the same).
+  const bool cols96 = s.c_dst % 96 == 0 && worth_96_columns(a.n_pairs, a.n_src, a.n_dst) && (a.dtype == FGMS_F16 || (a.reduced && !a.transpose_w && s.S == 4 && split_bf16_enabled() &&
+                      (a.n_dst + kTileRows - 1) / kTileRows * (s.c_dst / 96) * 2 >= 3 * (int64_t)num_cus()));
+  s.NTR = (s.c_dst % 128 == 0 && wide) ? 4 : s.c_dst % 64 == 0 ? 2 : cols96 ? 3 : 1;
+  s.SR = s.S < 4 && s.c_src % (6 * s.E) == 0 ? 3 : s.S;
+  s.lds_rows_bytes = 2 * (size_t)s.SR * s.NTR * 64 * 16          // two stages of weights
+                     + (size_t)kWaves * kWaveRows * 2 * s.SR * 16 + (size_t)kWaves * 3 * kWaveRows * sizeof(int);
   s.ok = s.lds_bytes <= 128 * 1024;
   return s;
 }
 
 template <typename T>
-int pack_weights(const GmsArgs &a, const Shape &s, const T **packed) {
+int pack_weights(const GmsArgs &a, int S, const T **packed) {
   void *ws = nullptr;
   const size_t n = (size_t)a.k_vol * a.c_in * a.c_out;
   bool fill = true;
-  int rc = relaid_weights_buffer(a, (unsigned)s.S << 8 | (a.transpose_w ? 2u : 0u), n * sizeof(T), &ws, &fill);
+  int rc = relaid_weights_buffer(a, (unsigned)S << 8 | (a.transpose_w ? 2u : 0u), n * sizeof(T), &ws, &fill);
   if (rc != FGMS_OK) return rc;
   *packed = (const T *)ws;
   if (!fill) return FGMS_OK;
   unsigned blocks = (unsigned)((n + 255) / 256);
   if (blocks > 4096) blocks = 4096;
   pack_weights_kernel<T><<<blocks, 256, 0, a.stream>>>((const T *)a.w, (T *)ws, a.k_vol, a.c_in,
-                                                       a.c_out, s.S, a.transpose_w);
+                                                       a.c_out, S, a.transpose_w);
   FGMS_HIP_TRY(hipGetLastError());
   relaid_weights_filled(a, ws);
   return FGMS_OK;
@@ -1058,7 +1068,7 @@ int launch_pairs(const GmsArgs &a, const Shape &s) {
     if (rc != FGMS_OK) return rc;
     packed = (const T *)ws;
   } else {
-    int rc = pack_weights<T>(a, s, &packed);
+    int rc = pack_weights<T>(a, S, &packed);
     if (rc != FGMS_OK) return rc;
   }
   const bool dense = a.dense_k >= 0;
@@ -1166,14 +1176,14 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
   const unsigned gy = (unsigned)(s.c_dst / (32 * NT));
   constexpr bool kCanHalf = NT != 4;
   const RowsGrid rg = rows_grid(a.n_dst, gy, a.k_vol * slabs, kCanHalf, tile_order != nullptr, tile_grid, pair_view,
-                                NT == 4 ? 2 : 3, a.transpose_w, kCanHalf && !a.transpose_w);
+                                NT >= 3 ? 2 : 3, a.transpose_w, kCanHalf && !a.transpose_w);
   // Few tiles: column tiles of 32 put them on twice the CUs, as long as each still has one to itself.
   // A tile's rows are then gathered twice, by CUs that had nothing to do.  Against two workgroups
   // per 64-column tile and atomics / 64-column tiles with four groups: 64 -> 64 fp16 over 1 k voxels
   // 14.3 / 15.3 -> 12.4 us, 5 k 14.4 / 15.0 -> 12.2, 12 k 15.3 / 15.4 -> 13.1; fp32 over 2 k
   // 47.2 / 66.4 -> 40.9; tf32 mode over 5 k 35.2 / 31.6 -> 27.4; 128 -> 128 fp16 over 2 k 21.8 / 24.1 -> 19.5.
-  if constexpr (NT == 2) {
-    if (rg.groups == 4 && (int64_t)rg.gx * gy * 2 <= num_cus())
+  if constexpr (NT == 2 || NT == 3) {
+    if (rg.groups == 4 && (int64_t)rg.gx * gy * NT <= num_cus())
       return launch_rows<T, 1, S>(a, s, nbr, masks, perm, tile_order, tile_grid, flip, pair_view);
   }
   // With 64-column wave tiles the input gradient and the fp16 forward pass read the weight
@@ -1206,14 +1216,15 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
     packed = (const T *)ws;
     raw = 3;
   } else if (!packed) {
-    int rc = pack_weights<T>(a, s, &packed);
+    int rc = pack_weights<T>(a, S, &packed);
     if (rc != FGMS_OK) return rc;
   }
   const bool half_tiles = rg.half_tiles;
   if (rg.drop_table) tile_order = nullptr;
   constexpr int kHalfMT = kCanHalf ? 1 : 2;
   constexpr size_t kGroup = rows_group_chunks<T, NT, S, kHalfMT>() * 16, kSums = rows_sum_chunks<NT, kHalfMT>() * 16;
-  const int kg = half_tiles ? rg.groups : 1;
+  constexpr int kMaxGroups = NT == 3 ? 2 : 4;          // (four groups' sums of 96 columns do not fit LDS)
+  const int kg = !half_tiles ? 1 : rg.groups < kMaxGroups ? rg.groups : kMaxGroups;
   size_t lds_rows = half_tiles ? kGroup * kg : s.lds_rows_bytes;
   if (kg > 1 && lds_rows < kGroup + kSums * (kg - 1)) lds_rows = kGroup + kSums * (kg - 1);
   const unsigned gx = rg.gx;
@@ -1229,7 +1240,7 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
               : gms_rows_kernel<T, NT, S, 0, MTv, KGv>)
   auto kern = FGMS_BY_RAW(2, 1);
   if constexpr (kCanHalf) {
-    if (half_tiles) kern = kg == 4 ? FGMS_BY_RAW(1, 4) : kg == 2 ? FGMS_BY_RAW(1, 2) : FGMS_BY_RAW(1, 1);
+    if (half_tiles) kern = kg == 4 ? FGMS_BY_RAW(1, kMaxGroups) : kg == 2 ? FGMS_BY_RAW(1, 2) : FGMS_BY_RAW(1, 1);
   }
 #undef FGMS_BY_RAW
   { const int rc_lds = allow_dynamic_lds(reinterpret_cast<const void *>(kern), lds_rows); if (rc_lds != FGMS_OK) return rc_lds; }
@@ -1271,7 +1282,7 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
 // (2 waves per SIMD where the weight gradient's tile is 128 x 128: its 64 accumulators per lane and
 // the rows in flight spill at 3.  128 -> 128 over 40k voxels, forward and backward: tf32 mode 477 -> 327 us.)
 template <typename T, int NT, int S, int BI, int BJ, int RAWD, int MT = 2>
-__global__ __launch_bounds__(kThreads, NT == 4 || BI * BJ == 16 ? 2 : 3) void bwd_fused_kernel(
+__global__ __launch_bounds__(kThreads, NT >= 3 || BI * BJ == 16 || ((BI == 3 || BJ == 3) && BI * BJ >= 6) ? 2 : 3) void bwd_fused_kernel(
     const T *__restrict__ gout, const T *__restrict__ w, T *__restrict__ gin,
     const int32_t *__restrict__ nbr, const unsigned long long *__restrict__ block_masks,
     const int32_t *__restrict__ perm, const int32_t *__restrict__ tile_order, int n_in, int k_vol,
@@ -1293,7 +1304,7 @@ __global__ __launch_bounds__(kThreads, NT == 4 || BI * BJ == 16 ? 2 : 3) void bw
                                       part_stages, bx, rest % row_y, rest / row_y, row_z, gout_bytes, 0, overwrite, flip);
   } else {
     const int j = blockIdx.x - rows_total;
-    if constexpr (BI <= 2 && BJ <= 2)
+    if constexpr (BI <= 3 && BJ <= 3)
       wgrad_wave_body<T, BI, BJ, RAWD == 4>(in, gout, gw32, kpos, imap, omap, k_vol, c_in, c_out, smap,
                                             j % wgrad_x, j / wgrad_x, in_bytes, gout_bytes);
     else
@@ -1316,7 +1327,7 @@ int launch_fused(const GmsArgs &d, const Shape &s, const Plan *p, const WgradArg
   const unsigned row_y = (unsigned)(s.c_dst / (32 * NT));
   constexpr bool kCanHalf = NT != 4;
   const RowsGrid rg = rows_grid(d.n_dst, row_y, d.k_vol * slabs, kCanHalf, p->tile_in != nullptr, p->tile_grid_in,
-                                false, NT == 4 ? 2 : 3, true, false);
+                                false, NT >= 3 ? 2 : 3, true, false);
   const unsigned row_x = (rg.gx + 7) / 8 * 8;
   const int part_stages = rg.part_stages;
   const unsigned row_z = rg.gz;
@@ -1358,14 +1369,20 @@ int launch_fused(const GmsArgs &d, const Shape &s, const Plan *p, const WgradArg
 template <typename T, typename F>
 int dispatch_shape(const Shape &s, F &&f);
 
+template <int NT, typename F>
+int dispatch_rows_slab(const Shape &s, F &&f) {
+  if (s.SR == 4) return f(std::integral_constant<int, NT>{}, std::integral_constant<int, 4>{});
+  if (s.SR == 3) return f(std::integral_constant<int, NT>{}, std::integral_constant<int, 3>{});
+  if (s.SR == 2) return f(std::integral_constant<int, NT>{}, std::integral_constant<int, 2>{});
+  return f(std::integral_constant<int, NT>{}, std::integral_constant<int, 1>{});
+}
+
 template <typename T, typename F>
 int dispatch_rows_shape(const Shape &s, F &&f) {
-  if (s.NTR == 4) {
-    if (s.S == 4) return f(std::integral_constant<int, 4>{}, std::integral_constant<int, 4>{});
-    if (s.S == 2) return f(std::integral_constant<int, 4>{}, std::integral_constant<int, 2>{});
-    return f(std::integral_constant<int, 4>{}, std::integral_constant<int, 1>{});
-  }
-  return dispatch_shape<T>(s, f);
+  if (s.NTR == 4) return dispatch_rows_slab<4>(s, f);
+  if (s.NTR == 3) return dispatch_rows_slab<3>(s, f);
+  if (s.NTR == 2) return dispatch_rows_slab<2>(s, f);
+  return dispatch_rows_slab<1>(s, f);
 }
 
 template <typename T, typename F>
@@ -1395,16 +1412,14 @@ int num_cus() {
 }
 
 int pack_weights_any(const GmsArgs &a, int S, const void **packed) {
-  Shape s{};
-  s.S = S;
   if (a.dtype == FGMS_F16) {
     const __half *p = nullptr;
-    int rc = pack_weights<__half>(a, s, &p);
+    int rc = pack_weights<__half>(a, S, &p);
     *packed = p;
     return rc;
   }
   const float *p = nullptr;
-  int rc = pack_weights<float>(a, s, &p);
+  int rc = pack_weights<float>(a, S, &p);
   *packed = p;
   return rc;
 }
@@ -1428,7 +1443,7 @@ int launch_fused_bwd(const GmsArgs &d, const Plan *p, const WgradArgs &w, bool *
   // (wave tile columns NT of the input gradient, MFMA steps per slab S) follow from c_in and
   // c_out, and so do the block counts (BI, BJ) of the weight gradient's tile
 #define FGMS_FB(TT, NTv, Sv, BIv, BJv)                                             \
-  if (!found && s.NTR == NTv && s.S == Sv && g.bi == BIv && g.bj == BJv) {          \
+  if (!found && s.NTR == NTv && s.SR == Sv && g.bi == BIv && g.bj == BJv) {          \
     found = true;                                                                    \
     rc = launch_fused<TT, NTv, Sv, BIv, BJv>(d, s, p, w, g, acc32);                 \
   }
@@ -1437,6 +1452,9 @@ int launch_fused_bwd(const GmsArgs &d, const Plan *p, const WgradArgs &w, bool *
     FGMS_FB(__half, 2, 2, 2, 1) FGMS_FB(__half, 2, 4, 2, 2) FGMS_FB(__half, 2, 4, 2, 4)
     FGMS_FB(__half, 2, 2, 4, 1) FGMS_FB(__half, 2, 4, 4, 2) FGMS_FB(__half, 2, 4, 4, 4)
     FGMS_FB(__half, 4, 2, 4, 1) FGMS_FB(__half, 4, 4, 4, 2) FGMS_FB(__half, 4, 4, 4, 4)
+    FGMS_FB(__half, 3, 2, 3, 1) FGMS_FB(__half, 3, 4, 3, 2) FGMS_FB(__half, 3, 3, 3, 3)
+    FGMS_FB(__half, 1, 3, 1, 3) FGMS_FB(__half, 2, 3, 2, 3) FGMS_FB(__half, 4, 3, 2, 3)
+    FGMS_FB(__half, 1, 3, 1, 1) FGMS_FB(__half, 2, 3, 2, 1) FGMS_FB(__half, 2, 3, 4, 1) FGMS_FB(__half, 4, 3, 4, 1)
   } else {
     FGMS_FB(float, 1, 4, 1, 1) FGMS_FB(float, 1, 4, 1, 2) FGMS_FB(float, 1, 4, 1, 4)
     FGMS_FB(float, 2, 4, 2, 1) FGMS_FB(float, 2, 4, 2, 2) FGMS_FB(float, 2, 4, 2, 4)
@@ -1466,7 +1484,7 @@ int planned_pack_job(const GmsArgs &a, SideJob *job, const void **packed) {
   job->dst = ws;
   job->n = n;
   job->k_vol = a.k_vol; job->c_in = a.c_in; job->c_out = a.c_out;
-  job->S = s.S; job->transpose = a.transpose_w; job->dtype = a.dtype;
+  job->S = s.SR; job->transpose = a.transpose_w; job->dtype = a.dtype;
   // about 8 elements per thread of 256-thread workgroups
   size_t blocks = ((n + 2047) / 2048 + 7) / 8 * 8;
   job->blocks = (int)(blocks > 1024 ? 1024 : blocks);

@@ -22,11 +22,14 @@ __device__ __forceinline__ void wave_lds_fence() {
 // halves of a span, and the eight row pairs of a pass land on eight different slots of their
 // half.  (XOR by row % 8 had rows r and r + 8 collide: measured 137 against 255 bytes per
 // clock and CU for this read.)  The writes of a staged gather (8 lanes per row, 2 rows per
-// pass) are conflict-free either way.
+// pass) are conflict-free either way.  With 96-byte rows (S = 3) eight consecutive rows start in
+// eight different 32-byte pieces of the banks, and rows r and r + 8 in the same one: these two take
+// its two halves.
 template <int S>
 __device__ __forceinline__ int a_slot(int row, int c) {
   constexpr int C = 2 * S;
   if constexpr (C == 8) return row * C + (c ^ ((row >> 1) & 7));
+  else if constexpr (C == 6) return row * C + (c ^ ((row >> 3) & 1));
   else return row * C + (c ^ ((row / (8 / C)) % C));
 }
 
@@ -41,7 +44,7 @@ template <int NT>
 __device__ __forceinline__ int raw_swizzle(int row) {
   if constexpr (NT == 4) return (row & 3) << 2;          // 256-byte rows
   else if constexpr (NT == 2) return ((row >> 1) & 1) << 2;   // 128-byte rows
-  else return 0;                                          // 64-byte rows
+  else return 0;                        // 64- and 192-byte rows: four of them cover all banks as they lie
 }
 
 // B fragment of MFMA step s, 32-column tile nt: the 8 values W[(h*S + s)*8 + 0..7][nt*32 + lane%32].
@@ -193,7 +196,8 @@ __device__ __forceinline__ void add_rows_lds(const float16v (&acc)[MT][NT], T *_
                                              int c_dst, int cd0, int lane) {
   constexpr int COLS = NT * 32;
   constexpr int WR = MT * 32;             // the wave's rows
-  constexpr int R = (WR * 2 * S * 16) / (COLS * 4) >= 32 ? 32 : (WR * 2 * S * 16) / (COLS * 4);
+  constexpr int FIT = (WR * 2 * S * 16) / (COLS * 4);
+  constexpr int R = FIT >= 32 ? 32 : FIT >= 16 ? 16 : FIT >= 8 ? 8 : 0;
   if constexpr (R < 8) {
     if constexpr (ATOMIC) write_tile<T, NT, true>(acc, dst, rows, c_dst, cd0, lane);
     else {

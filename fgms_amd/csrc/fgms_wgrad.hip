@@ -54,7 +54,7 @@ __global__ __launch_bounds__(kThreads) void wgrad_kernel(
 
 // The per-wave variant (wgrad_wave_body) in a launch of its own.
 template <typename T, int BI, int BJ, bool SPLIT>
-__global__ __launch_bounds__(kThreads, 3) void wgrad_wave_kernel(
+__global__ __launch_bounds__(kThreads, BI * BJ >= 6 ? 2 : 3) void wgrad_wave_kernel(
     const T *__restrict__ in, const T *__restrict__ gout, float *__restrict__ gw32,
     const int32_t *__restrict__ kpos, const int32_t *__restrict__ imap,
     const int32_t *__restrict__ omap, int k_vol, int c_in, int c_out, SliceMap smap, SideJob side,
@@ -253,16 +253,22 @@ __global__ void add_and_clear_kernel(__half *__restrict__ dst, float *__restrict
                          (size_t)gridDim.x * blockDim.x, overwrite);
 }
 
-int blocks_of(int c) { return c % 128 == 0 ? 4 : (c % 64 == 0 ? 2 : 1); }
+int blocks_of(int c, bool three) { return c % 128 == 0 ? 4 : c % 64 == 0 ? 2 : three && c % 96 == 0 ? 3 : 1; }
 
 // 32-column blocks (BI x BJ) of the tile a wave or workgroup holds of dW[k].  A 128 x 128 fp16 tile
 // in a launch of its own is cut into four 64 x 64 tiles for the per-wave body (rows gathered twice,
 // twelve independent waves per CU instead of two workgroups of four: 110 -> 100 us at 128 -> 128
 // over 120k voxels); in the backward launch, next to the input gradient's workgroups, the
-// workgroup-level body stays ahead (163 against 166 us).
+// workgroup-level body stays ahead (163 against 166 us).  fp16 channel counts of 96 take tiles 96 wide in
+// the per-wave body, so that both rows of a pair are gathered once and not three times: 96 -> 96
+// over 80 k voxels, forward and backward, 194.6 -> 112.4 us (in tf32 mode the split tiles spill at that size,
+// fp32 loses by it: 351 -> 420 us over 40 k).
 void tile_blocks(const WgradArgs &a, bool shares_grid, int *bi, int *bj) {
-  *bi = blocks_of(a.c_in);
-  *bj = blocks_of(a.c_out);
+  const bool three = a.dtype == FGMS_F16 && worth_96_columns(a.n_pairs, a.n_in, a.n_out);
+  *bi = blocks_of(a.c_in, three);
+  *bj = blocks_of(a.c_out, three);
+  if (*bi == 3 && *bj == 4) *bj = 2;     // (96 channels: the per-wave body)
+  if (*bj == 3 && *bi == 4) *bi = 2;
   if (!shares_grid && a.dtype == FGMS_F16 && *bi * *bj == 16) {
     *bi = 2;
     *bj = 2;
@@ -380,6 +386,7 @@ int dispatch(const WgradArgs &a, float *acc32) {
   tile_blocks(a, false, &bi, &bj);
 #define FGMS_WW(I, J) if (bi == I && bj == J) return launch_wave<T, I, J>(a, acc32);
   FGMS_WW(1, 1) FGMS_WW(1, 2) FGMS_WW(2, 1) FGMS_WW(2, 2)
+  if constexpr (sizeof(T) == 2) { FGMS_WW(1, 3) FGMS_WW(3, 1) FGMS_WW(2, 3) FGMS_WW(3, 2) FGMS_WW(3, 3) }
 #undef FGMS_WW
 #define FGMS_WG(I, J) if (bi == I && bj == J) return launch<T, I, J>(a, acc32);
   FGMS_WG(1, 4) FGMS_WG(2, 4)
@@ -415,7 +422,7 @@ int wgrad_geometry(const WgradArgs &a, WgradGeometry *g, bool shares_grid) {
   g->bi = bi;
   g->bj = bj;
   g->ty = (a.c_in / (32 * bi)) * (a.c_out / (32 * bj));
-  g->wave = bi <= 2 && bj <= 2;
+  g->wave = bi <= 3 && bj <= 3;
   if (g->wave) {
     const int sp = f16 ? WTW<__half>::stage_pairs : WTW<float>::stage_pairs;
     g->smap = choose_slices(a, g->ty, sp, (int64_t)num_cus() * 6);
@@ -425,7 +432,7 @@ int wgrad_geometry(const WgradArgs &a, WgradGeometry *g, bool shares_grid) {
     const size_t lds = (g->split ? 4 * (size_t)sp * 2 * ((bi * 32 + 16) + (bj * 32 + 16)) * 2
                                  : 4 * (size_t)sp * ((bi * 32 + (f16 ? 0 : pad)) + (bj * 32 + (f16 ? 0 : pad))) * esz)
                        + 4 * 64 * sizeof(int);                           // + the waves' index exchange
-    const size_t red = 3 * (size_t)bi * bj * 16 * 64 * sizeof(float);     // the partial tiles' exchange
+    const size_t red = 3 * (size_t)(bi * bj > 4 ? 1 : bi) * bj * 16 * 64 * sizeof(float);     // the partial tiles' exchange
     g->lds = lds < red ? red : lds;
     return FGMS_OK;
   }

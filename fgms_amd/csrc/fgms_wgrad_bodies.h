@@ -38,13 +38,13 @@ __device__ __forceinline__ half8 tr_frag(const __half *tile, int ld, int p0, int
   return __builtin_bit_cast(half8, v);
 }
 
-// The same from a tile without row padding (rows of exactly `ld` = 32 or 64 halfs).  One
+// The same from a tile without row padding (rows of exactly `ld` = 32, 64 or 96 halfs).  One
 // transposing read touches rows p .. p + 3 and p + 8 .. p + 11, 64 bytes of each; with 128-byte
 // rows, rows p and p + 2 would meet in the same banks, so the writer exchanges the two 64-byte
 // halves of every row whose (row >> 1) is odd (wave tile below) and the read does the same.
 template <int LD>
 __device__ __forceinline__ half8 tr_frag_dense(const __half *tile, int p0, int c0, int lane) {
-  static_assert(LD == 32 || LD == 64, "dense tile: 32 or 64 channels a row");
+  static_assert(LD == 32 || LD == 64 || LD == 96, "dense tile: 32, 64 or 96 channels a row");
   const int b = lane >> 4, i = lane & 15, h = lane >> 5;
   const int sw = LD == 64 ? ((lane >> 3) & 1) * 32 : 0;
   const __half *base = tile + (size_t)(p0 + h * 8 + (i >> 2)) * LD + (c0 ^ sw) + (b & 1) * 16 + (i & 3) * 4;
@@ -186,13 +186,16 @@ __device__ __forceinline__ void wgrad_wave_body(
   // indices, lanes 32.. the output rows') and are handed round through 256 bytes of LDS behind
   // the staging tiles, instead of one load instruction per row instruction: a lane's chunks then
   // belong to NX (NG) consecutive pairs, whose indices it reads back with one LDS read each.
-  static_assert(!kBufW || (SP == 32 && (NX == 2 || NX == 4) && (NG == 2 || NG == 4)), "index exchange: 32 pairs a stage");
+  // (96 channels: four lanes to a pair, three of its chunks each, then the pair sixteen further on)
+  static_assert(!kBufW || (SP == 32 && (NX == 2 || NX == 4 || NX == 6) && (NG == 2 || NG == 4 || NG == 6)), "index exchange: 32 pairs a stage");
   int *ibuf = reinterpret_cast<int *>(reinterpret_cast<T *>(lds) + (size_t)4 * SP * (LDI + LDO)) + wave * 64;
   const int32_t *const my_map = lane < 32 ? imap : omap;
   int idx_raw = 0;
   // chunk i of this lane: pair `row`, 16-byte piece `cc` of its row
-  auto x_row = [&](int i) { return kBufW ? (lane / NCI) * NX + i : (lane + 64 * i) / NCI; };
-  auto g_row = [&](int i) { return kBufW ? (lane / NCO) * NG + i : (lane + 64 * i) / NCO; };
+  auto x_row = [&](int i) { return !kBufW ? (lane + 64 * i) / NCI : NX == 6 ? lane / 4 + 16 * (i / 3) : (lane / NCI) * NX + i; };
+  auto g_row = [&](int i) { return !kBufW ? (lane + 64 * i) / NCO : NG == 6 ? lane / 4 + 16 * (i / 3) : (lane / NCO) * NG + i; };
+  auto x_chunk = [&](int i) { return !kBufW ? (lane + 64 * i) % NCI : NX == 6 ? lane % 4 + 4 * (i % 3) : lane % NCI; };
+  auto g_chunk = [&](int i) { return !kBufW ? (lane + 64 * i) % NCO : NG == 6 ? lane % 4 + 4 * (i % 3) : lane % NCO; };
 
   // Everything is issued unconditionally and nothing touches a loaded register before
   // its consumer: an index or a row that is selected, copied or loaded under a branch
@@ -219,6 +222,9 @@ __device__ __forceinline__ void wgrad_wave_body(
     if constexpr (NX == 4) {
       const int4v v = *reinterpret_cast<const int4v *>(ibuf + (lane / NCI) * 4);
       xi[0] = v[0]; xi[1] = v[1]; xi[2] = v[2]; xi[3] = v[3];
+    } else if constexpr (NX == 6) {
+      xi[0] = xi[1] = xi[2] = ibuf[lane / 4];
+      xi[3] = xi[4] = xi[5] = ibuf[lane / 4 + 16];
     } else {
       const int2v v = *reinterpret_cast<const int2v *>(ibuf + (lane / NCI) * 2);
       xi[0] = v[0]; xi[1] = v[1];
@@ -226,6 +232,9 @@ __device__ __forceinline__ void wgrad_wave_body(
     if constexpr (NG == 4) {
       const int4v v = *reinterpret_cast<const int4v *>(ibuf + 32 + (lane / NCO) * 4);
       gi[0] = v[0]; gi[1] = v[1]; gi[2] = v[2]; gi[3] = v[3];
+    } else if constexpr (NG == 6) {
+      gi[0] = gi[1] = gi[2] = ibuf[32 + lane / 4];
+      gi[3] = gi[4] = gi[5] = ibuf[32 + lane / 4 + 16];
     } else {
       const int2v v = *reinterpret_cast<const int2v *>(ibuf + 32 + (lane / NCO) * 2);
       gi[0] = v[0]; gi[1] = v[1];
@@ -234,7 +243,7 @@ __device__ __forceinline__ void wgrad_wave_body(
   auto load_rows = [&](int st_) {      // st_: the stage the indices in xi / gi belong to
 #pragma unroll
     for (int i = 0; i < NX; ++i) {
-      const int cc = kBufW ? lane % NCI : (lane + 64 * i) % NCI;
+      const int cc = x_chunk(i);
       if constexpr (kBufW) {
         const bool live = st_ * SP + x_row(i) < count;
         const unsigned off = live ? (unsigned)xi[i] * (unsigned)(c_in * (int)sizeof(T)) : kAbsentRow;
@@ -246,7 +255,7 @@ __device__ __forceinline__ void wgrad_wave_body(
     }
 #pragma unroll
     for (int i = 0; i < NG; ++i) {
-      const int cc = kBufW ? lane % NCO : (lane + 64 * i) % NCO;
+      const int cc = g_chunk(i);
       if constexpr (kBufW) {
         const bool live = st_ * SP + g_row(i) < count;
         const unsigned off = live ? (unsigned)gi[i] * (unsigned)(c_out * (int)sizeof(T)) : kAbsentRow;
@@ -264,7 +273,7 @@ __device__ __forceinline__ void wgrad_wave_body(
       if constexpr (SPLIT)
         store_split_chunk(xh, xl, LDIh, e / NCI, e % NCI, xr[i], st * SP + e / NCI < count, lane);
       else if constexpr (kBufW)
-        *reinterpret_cast<int4v *>(x + x_row(i) * LDI + (((lane % NCI) ^ (CI == 64 ? ((x_row(i) >> 1) & 1) * 4 : 0)) * E)) = xr[i];
+        *reinterpret_cast<int4v *>(x + x_row(i) * LDI + ((x_chunk(i) ^ (CI == 64 ? ((x_row(i) >> 1) & 1) * 4 : 0)) * E)) = xr[i];
       else
         *reinterpret_cast<int4v *>(x + (e / NCI) * LDI + (e % NCI) * E) =
             st * SP + e / NCI < count ? xr[i] : int4v{0, 0, 0, 0};
@@ -275,7 +284,7 @@ __device__ __forceinline__ void wgrad_wave_body(
       if constexpr (SPLIT)
         store_split_chunk(gh, gl, LDOh, e / NCO, e % NCO, gr[i], st * SP + e / NCO < count, lane);
       else if constexpr (kBufW)
-        *reinterpret_cast<int4v *>(g + g_row(i) * LDO + (((lane % NCO) ^ (CO == 64 ? ((g_row(i) >> 1) & 1) * 4 : 0)) * E)) = gr[i];
+        *reinterpret_cast<int4v *>(g + g_row(i) * LDO + ((g_chunk(i) ^ (CO == 64 ? ((g_row(i) >> 1) & 1) * 4 : 0)) * E)) = gr[i];
       else
         *reinterpret_cast<int4v *>(g + (e / NCO) * LDO + (e % NCO) * E) =
             st * SP + e / NCO < count ? gr[i] : int4v{0, 0, 0, 0};
@@ -320,23 +329,27 @@ __device__ __forceinline__ void wgrad_wave_body(
           acc[ti][tj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[ti], bh[tj], acc[ti][tj], 0, 0, 0);
         }
     } else if constexpr (kBufW) {
-      constexpr int KS = SP / KP;
-      half8 a[KS][BI], b[KS][BJ];
+      // (tiles of more than 64 x 64: one k-step's fragments at a time, for want of registers)
+      constexpr int KS = SP / KP, KF = BI * BJ > 4 ? 1 : KS;
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
+      for (int k0 = 0; k0 < KS; k0 += KF) {
+        half8 a[KF][BI], b[KF][BJ];
 #pragma unroll
-        for (int ti = 0; ti < BI; ++ti) a[ks][ti] = tr_frag_dense<CI>(x, ks * KP, ti * 32, lane);
+        for (int ks = 0; ks < KF; ++ks) {
 #pragma unroll
-        for (int tj = 0; tj < BJ; ++tj) b[ks][tj] = tr_frag_dense<CO>(g, ks * KP, tj * 32, lane);
+          for (int ti = 0; ti < BI; ++ti) a[ks][ti] = tr_frag_dense<CI>(x, (k0 + ks) * KP, ti * 32, lane);
+#pragma unroll
+          for (int tj = 0; tj < BJ; ++tj) b[ks][tj] = tr_frag_dense<CO>(g, (k0 + ks) * KP, tj * 32, lane);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int ks = 0; ks < KF; ++ks)
+#pragma unroll
+          for (int ti = 0; ti < BI; ++ti)
+#pragma unroll
+            for (int tj = 0; tj < BJ; ++tj)
+              acc[ti][tj] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[ks][ti], b[ks][tj], acc[ti][tj], 0, 0, 0);
       }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-        for (int ti = 0; ti < BI; ++ti)
-#pragma unroll
-          for (int tj = 0; tj < BJ; ++tj)
-            acc[ti][tj] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[ks][ti], b[ks][tj], acc[ti][tj], 0, 0, 0);
     } else {
 #pragma unroll
     for (int ks = 0; ks < SP / KP; ++ks) {
@@ -375,35 +388,40 @@ __device__ __forceinline__ void wgrad_wave_body(
   }
 
   // Sum the four waves' tiles through LDS and flush.  Every wave ends up with a quarter of the
-  // summed tile (accumulator registers q * R / 4 ... of the R = BI * BJ * 16 a lane holds) and
+  // summed tile (accumulator registers q * R / 4 ... of the R a lane holds) and
   // flushes that: one barrier, and the atomic updates of the tile issued by four waves instead
-  // of one.  red: [quarter][contribution 0..2][register of the quarter][lane].
+  // of one.  red: [quarter][contribution 0..2][register of the quarter][lane].  (Tiles of more than
+  // 64 x 64 a row of blocks at a time: LDS for the whole would leave one workgroup to a CU.)
   float *red = reinterpret_cast<float *>(lds);
-  constexpr int R = BI * BJ * 16, RQ = R / 4;
-  __syncthreads();                  // every wave is done with its staging tiles
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    if (q == wave) continue;
-    const int slot = wave < q ? wave : wave - 1;
-#pragma unroll
-    for (int j = 0; j < RQ; ++j) {
-      const int idx = q * RQ + j, t = idx / 16;
-      red[(size_t)((q * 3 + slot) * RQ + j) * 64 + lane] = acc[t / BJ][t % BJ][idx % 16];
-    }
-  }
-  __syncthreads();
+  constexpr int PB = BI * BJ > 4 ? 1 : BI;       // block rows per pass
+  constexpr int R = PB * BJ * 16, RQ = R / 4;
   const int h = lane >> 5, c = lane & 31;
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    if (q != wave) continue;
+  for (int ti0 = 0; ti0 < BI; ti0 += PB) {
+    __syncthreads();                // every wave is done with its staging tiles (the sums of the last pass)
 #pragma unroll
-    for (int j = 0; j < RQ; ++j) {
-      const int idx = q * RQ + j, t = idx / 16, r = idx % 16, ti = t / BJ, tj = t % BJ;
-      float v = acc[ti][tj][r];
+    for (int q = 0; q < 4; ++q) {
+      if (q == wave) continue;
+      const int slot = wave < q ? wave : wave - 1;
 #pragma unroll
-      for (int slot = 0; slot < 3; ++slot) v += red[(size_t)((q * 3 + slot) * RQ + j) * 64 + lane];
-      // accumulator register r of lane l is row (r/4)*8 + (l/32)*4 + r%4, column l%32 of its 32 x 32 tile
-      atomic_add(gw32 + ((size_t)k * c_in + ci0 + ti * 32 + (r / 4) * 8 + h * 4 + (r % 4)) * c_out + co0 + tj * 32 + c, v);
+      for (int j = 0; j < RQ; ++j) {
+        const int idx = q * RQ + j, t = idx / 16;
+        red[(size_t)((q * 3 + slot) * RQ + j) * 64 + lane] = acc[ti0 + t / BJ][t % BJ][idx % 16];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (q != wave) continue;
+#pragma unroll
+      for (int j = 0; j < RQ; ++j) {
+        const int idx = q * RQ + j, t = idx / 16, r = idx % 16, ti = ti0 + t / BJ, tj = t % BJ;
+        float v = acc[ti][tj][r];
+#pragma unroll
+        for (int slot = 0; slot < 3; ++slot) v += red[(size_t)((q * 3 + slot) * RQ + j) * 64 + lane];
+        // accumulator register r of lane l is row (r/4)*8 + (l/32)*4 + r%4, column l%32 of its 32 x 32 tile
+        atomic_add(gw32 + ((size_t)k * c_in + ci0 + ti * 32 + (r / 4) * 8 + h * 4 + (r % 4)) * c_out + co0 + tj * 32 + c, v);
+      }
     }
   }
 }

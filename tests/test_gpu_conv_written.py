@@ -80,3 +80,11 @@ def test_small_forward_launches(oracle, n, dtype, tf32):
     capi.conv_fwd(D["in_feats"], D["kernel"], out, D["kpos"], D["imap"], D["omap"], arch80=tf32, plan=plan)
     ref = oracle.c_fwd(L["in_feats"], L["kernel"], L["knnz"], L["imap"], L["omap"], n)
     G.assert_close(out.cpu().numpy(), ref, G.mode_of(L["in_feats"].dtype, tf32), "fwd")
+
+
+@pytest.mark.parametrize("use_plan", [True, False], ids=["plan", "no_plan"])
+@pytest.mark.parametrize("dtype,tf32", [(np.float16, False), (np.float32, False), (np.float32, True)], ids=["fp16", "fp32", "tf32"])
+@pytest.mark.parametrize("n,shape", [(65, (96, 96)), (900, (48, 96)), (900, (96, 48)), (900, (96, 32)), (900, (32, 96)), (900, (96, 64)),
+                                     (900, (64, 96)), (900, (96, 128)), (900, (128, 96)), (900, (24, 96)), (900, (48, 160)), (70001, (96, 96))])
+def test_96_and_48_channels(oracle, n, shape, dtype, tf32, use_plan):
+    test_written_not_added(oracle, n, shape, dtype, tf32, use_plan)
