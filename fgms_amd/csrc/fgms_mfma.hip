@@ -381,7 +381,7 @@ __device__ __forceinline__ void gather_issue_buf(int4v (&v)[N], const unsigned *
   constexpr int C = 2 * S;
   unsigned off[N];
 #pragma unroll
-  for (int it = 0; it < N; ++it) off[it] = offs[(it * 64 + lane) / C] + (unsigned)(((it * 64 + lane) % C) * 16);
+  for (int it = 0; it < N; ++it) off[it] = offs[(it * 64 + lane) / C] + (unsigned)((64 % C == 0 ? lane % C : (it * 64 + lane) % C) * 16);
 #pragma unroll
   for (int it = 0; it < N; ++it)
     v[it] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off[it], slab * (C * 16), 0));
