@@ -561,12 +561,22 @@ bool padded_gms_channels(const GmsArgs &a, const Plan *plan, int *c_in, int *c_o
   return tuned_gms(with_channels(a, *c_in, *c_out), plan);
 }
 
+// fp16 layers whose channels fill no whole tile go straight to kernels that mask the rest, where the map
+// is dense enough for the output-stationary kernel (else the pair-stationary kernels over padded copies).
+bool takes_ragged(const GmsArgs &a, const Plan *plan) {
+  return g_policy == 0 && plan && a.n_pairs > 0 && a.dense_k < 0 && !small_gms_supported(a, plan) && !sparse_rows(a, plan);
+}
+
 // A pass over all offsets: one walk for plans of up to 64 offsets (or none), one per group of 64
 // offsets for larger kernels (the groups' results add up in the destination rows).
 int run_gms_padded(const GmsArgs &a, const Plan *plan, int c_in, int c_out, bool *done);
 
 int run_gms(GmsArgs a, const Plan *plan) {
   int pi, po;
+  if (takes_ragged(a, plan) && ragged_gms_supported(a, plan)) {
+    plan_touch(plan, a.stream);
+    return launch_ragged_gms(a, plan);
+  }
   if ((a.dense_k >= 0 ? a.n_dense : a.n_pairs) > 0 && padded_gms_channels(a, plan, &pi, &po)) {
     bool done = false;
     const int rc = run_gms_padded(a, plan, pi, po, &done);
@@ -863,6 +873,12 @@ int backward(const void *out_feats_grad, const void *in_feats, const void *kerne
   if (!want_kernel) return want_in ? run_gms(d, p) : FGMS_OK;
   if (!want_in) return run_wgrad(w);
   int pi, po;
+  if (takes_ragged(d, p)) {
+    bool done = false;
+    plan_touch(p, stream);
+    rc = launch_ragged_bwd(d, p, w, &done);
+    if (rc || done) return rc;
+  }
   if (n_pairs > 0 && padded_bwd_channels(d, p, w, &pi, &po)) {
     bool done = false;
     rc = run_bwd_padded(d, p, w, pi, po, &done);

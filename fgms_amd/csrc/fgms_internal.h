@@ -271,6 +271,10 @@ int wgrad_static(WgradArgs a);
 // (nothing is launched) and returns where the packed weights will be.
 int planned_pack_job(const GmsArgs &a, SideJob *job, const void **packed);
 // Both gradients of a layer in one launch where that is supported (*done says whether).
+// fp16 channel counts that fill no whole tile, through plan p: the forward pass, and both gradients in one launch.
+bool ragged_gms_supported(const GmsArgs &a, const Plan *p);
+int launch_ragged_gms(const GmsArgs &a, const Plan *p);
+int launch_ragged_bwd(const GmsArgs &d, const Plan *p, const WgradArgs &w, bool *done);
 int launch_fused_bwd(const GmsArgs &d, const struct Plan *p, const WgradArgs &w, bool *done);
 // Runs a side job in a launch of its own.
 int launch_side_job(const SideJob &job, hipStream_t stream);

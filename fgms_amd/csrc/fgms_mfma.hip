@@ -375,13 +375,19 @@ __device__ __forceinline__ void gather_commit(int4v *__restrict__ a_lds, int4v (
 // `offs` holds a byte offset per row of the wave's tile, kAbsentRow for a row that has no
 // neighbour through this offset, which then arrives as zeros by itself: no select on the way
 // to LDS, no row index kept per load, 32-bit address arithmetic.
-template <int S, int N>
+// (RAGGED: the slab's chunks from row_bytes on do not exist either)
+template <int S, bool RAGGED = false, int N>
 __device__ __forceinline__ void gather_issue_buf(int4v (&v)[N], const unsigned *__restrict__ offs,
-                                                 __amdgpu_buffer_rsrc_t rsrc, int slab, int lane) {
+                                                 __amdgpu_buffer_rsrc_t rsrc, int slab, int lane, unsigned row_bytes = 0) {
   constexpr int C = 2 * S;
   unsigned off[N];
 #pragma unroll
   for (int it = 0; it < N; ++it) off[it] = offs[(it * 64 + lane) / C] + (unsigned)((64 % C == 0 ? lane % C : (it * 64 + lane) % C) * 16);
+  if constexpr (RAGGED) {
+#pragma unroll
+    for (int it = 0; it < N; ++it)
+      if ((unsigned)((slab * C + (it * 64 + lane) % C) * 16) >= row_bytes) off[it] = kAbsentRow;
+  }
 #pragma unroll
   for (int it = 0; it < N; ++it)
     v[it] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off[it], slab * (C * 16), 0));
@@ -534,7 +540,10 @@ constexpr int rows_group_chunks() {      // 16-byte chunks of LDS per group: two
 template <int NT, int MT>
 constexpr int rows_sum_chunks() { return kWaves * MT * NT * 4 * 64; }      // ... of a group's sums
 
-template <typename T, int NT, int S, int RAW, int MT = 2, int KG = 1>
+// RAGGED (fp16, RAW 1 and 2): channel counts that fill no whole tile.  Chunks of rows and weights from c_src
+// on, and of weights from c_dst on, are loaded from outside their buffers and arrive as zeros; columns from
+// c_dst on are not written.
+template <typename T, int NT, int S, int RAW, int MT = 2, int KG = 1, bool RAGGED = false>
 __device__ __forceinline__ void gms_rows_body(
     const T *__restrict__ src, const T *__restrict__ packed, T *__restrict__ dst,
     const int32_t *__restrict__ nbr, const unsigned long long *__restrict__ block_masks,
@@ -564,7 +573,8 @@ __device__ __forceinline__ void gms_rows_body(
   // fp32 only: its MFMA phase is long enough (4 k clocks a stage) to absorb the loads'
   // issue waits; for fp16 the interleaved stage measured 2 us slower per launch
   constexpr bool kInterleave = sizeof(T) == 4 && RAW != 3 && RAW != 4;
-  const int slabs = c_src / (C * E);
+  static_assert(!RAGGED || (sizeof(T) == 2 && (RAW == 1 || RAW == 2)), "ragged: fp16 weights as they lie");
+  const int slabs = RAGGED ? (c_src + C * E - 1) / (C * E) : c_src / (C * E);
   const int nts = c_dst / 32;
   int4v *w_lds = lds;                                     // [2][WCH]
   const int wave = tid / 64, lane = tid % 64;
@@ -612,7 +622,7 @@ __device__ __forceinline__ void gms_rows_body(
   __syncthreads();
   unsigned long long todo = wg_mask;
   if (!todo) {
-    if (overwrite && group == 0) zero_rows<T, NT, WR>(dst, didx, c_dst, nt0 * 32, lane);
+    if (overwrite && group == 0) zero_rows<T, NT, WR, RAGGED>(dst, didx, c_dst, nt0 * 32, lane);
     return;
   }
   // The launch lasts as long as its longest tile, and the tiles with the longest
@@ -722,8 +732,15 @@ __device__ __forceinline__ void gms_rows_body(
 #pragma unroll
     for (int i = 0; i < NW; ++i) {
       const int e = tid + kThreads * i;
-      if (NW * kThreads == WCH || e < WCH)
-        wreg[i] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(wrsrc, wvoff[i], soff, 0));
+      if (NW * kThreads == WCH || e < WCH) {
+        unsigned off = wvoff[i];
+        if constexpr (RAGGED) {
+          const int from = slab * (C * E) + (RAW == 1 ? e / (NT * 4) : e % C * E);
+          const int to = nt0 * 32 + (RAW == 1 ? e % (NT * 4) * E : e / C);
+          if (from >= c_src || to >= c_dst) off = kAbsentRow;
+        }
+        wreg[i] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(wrsrc, off, soff, 0));
+      }
     }
   };
   auto weights_commit = [&](const int4v (&wreg)[NW], int buf) {
@@ -756,7 +773,7 @@ __device__ __forceinline__ void gms_rows_body(
   int4v v[NV];
   int gsel[kBuf ? 1 : NV];
   auto rows_issue = [&](int slab_, int slot_ = 0) {
-    if constexpr (kBuf) gather_issue_buf<S>(v, goff + slot_ * WR, rsrc, slab_, lane);
+    if constexpr (kBuf) gather_issue_buf<S, RAGGED>(v, goff + slot_ * WR, rsrc, slab_, lane, row_bytes);
     else gather_issue<T, S>(v, gsel, gidx, src, c_src, slab_, lane);
   };
   auto rows_commit = [&]() {
@@ -945,15 +962,15 @@ __device__ __forceinline__ void gms_rows_body(
   if (wave_mask || overwrite || KG > 1) {
     wave_lds_fence();
     if (shared_tile)
-      add_rows_lds<T, NT, S, true, false>(acc, dst, didx, reinterpret_cast<float *>(a_lds), c_dst, nt0 * 32, lane);
+      add_rows_lds<T, NT, S, true, false, RAGGED>(acc, dst, didx, reinterpret_cast<float *>(a_lds), c_dst, nt0 * 32, lane);
     else if (overwrite)
-      add_rows_lds<T, NT, S, false, true>(acc, dst, didx, reinterpret_cast<float *>(a_lds), c_dst, nt0 * 32, lane);
+      add_rows_lds<T, NT, S, false, true, RAGGED>(acc, dst, didx, reinterpret_cast<float *>(a_lds), c_dst, nt0 * 32, lane);
     else
-      add_rows_lds<T, NT, S, false, false>(acc, dst, didx, reinterpret_cast<float *>(a_lds), c_dst, nt0 * 32, lane);
+      add_rows_lds<T, NT, S, false, false, RAGGED>(acc, dst, didx, reinterpret_cast<float *>(a_lds), c_dst, nt0 * 32, lane);
   }
 }
 
-template <typename T, int NT, int S, int RAW, int MT = 2, int KG = 1>
+template <typename T, int NT, int S, int RAW, int MT = 2, int KG = 1, bool RAGGED = false>
 __global__ __launch_bounds__(kThreads * KG, MT == 1 ? (NT == 3 ? 3 : 4) : (NT >= 3 ? 2 : 3)) void gms_rows_kernel(
     const T *__restrict__ src, const T *__restrict__ packed, T *__restrict__ dst,
     const int32_t *__restrict__ nbr, const unsigned long long *__restrict__ block_masks,
@@ -969,7 +986,7 @@ __global__ __launch_bounds__(kThreads * KG, MT == 1 ? (NT == 3 ? 3 : 4) : (NT >=
     }
     block_x -= side.blocks;
   }
-  gms_rows_body<T, NT, S, RAW, MT, KG>(src, packed, dst, nbr, block_masks, perm, tile_order, n_dst, k_vol, c_src,
+  gms_rows_body<T, NT, S, RAW, MT, KG, RAGGED>(src, packed, dst, nbr, block_masks, perm, tile_order, n_dst, k_vol, c_src,
                                    c_dst, part_stages, block_x, blockIdx.y, blockIdx.z, gridDim.z, src_bytes, pair_view,
                                    overwrite, flip);
 }
@@ -1017,6 +1034,56 @@ Shape shape_of(const GmsArgs &a) {
   s.lds_rows_bytes = 2 * (size_t)s.SR * s.NTR * 64 * 16          // two stages of weights
                      + (size_t)kWaves * kWaveRows * 2 * s.SR * 16 + (size_t)kWaves * 3 * kWaveRows * sizeof(int);
   s.ok = s.lds_bytes <= 128 * 1024;
+  return s;
+}
+
+// FGMS_RAW_WEIGHTS=0 keeps the forward pass on re-laid weights (for comparison).
+bool raw_weights_enabled() {
+  static const bool on = !(getenv("FGMS_RAW_WEIGHTS") && atoi(getenv("FGMS_RAW_WEIGHTS")) == 0);
+  return on;
+}
+
+// --- fp16 channel counts that fill no whole tile (RAGGED) --------------------------------------
+// 32-column tiles per wave (and blocks of a weight-gradient tile) for c columns, 0: not served.
+int ragged_tiles(int c, bool three) {
+  const int t = (c + 31) / 32;
+  if (t <= 2) return t;
+  if (t % 3 == 0 && three) return 3;
+  if (t % 2 == 0) return 2;
+  return three ? 3 : 0;
+}
+// k-steps of a slab: a stage costs about two k-steps however few it has.  (160 channels: three slabs of 64, the
+// last one half empty, not five of 32.)
+int ragged_steps(int c) {
+  int best = 4, least = 1 << 30;
+  for (int S = 4; S >= 2; --S) {
+    const int cost = (c + 16 * S - 1) / (16 * S) * (S + 2);
+    if (cost < least) { least = cost; best = S; }
+  }
+  return best;
+}
+// The shapes that take it: multiples of 8 channels (16-byte chunks) that no whole tile fits -- a source of a pass
+// that is no multiple of 16, anything else that is none of 32 -- or an odd number of 32s from five
+// on (160), which whole tiles take 32 columns at a time.  Kernels on the vector ALUs keep the narrow ones.
+bool ragged_channels(int c_in, int c_out, bool forward) {
+  if (c_in % 8 || c_out % 8 || c_in < 16 || c_out < 16 || c_in * c_out <= 256) return false;
+  auto odd = [](int c, int whole) { return c % whole != 0 || (c % 32 == 0 && c / 32 % 2 == 1 && c / 32 >= 5 && c / 32 % 3 != 0); };
+  return odd(c_in, forward ? 16 : 32) || odd(c_out, 32);
+}
+Shape ragged_shape(const GmsArgs &a) {
+  Shape s{};
+  s.c_src = a.transpose_w ? a.c_out : a.c_in;
+  s.c_dst = a.transpose_w ? a.c_in : a.c_out;
+  s.E = 8;
+  if (a.dtype != FGMS_F16 || !ragged_channels(a.c_in, a.c_out, !a.transpose_w)) return s;
+  if (reinterpret_cast<uintptr_t>(a.src) % 16 || reinterpret_cast<uintptr_t>(a.dst) % 16 ||
+      reinterpret_cast<uintptr_t>(a.w) % 16 || !raw_weights_enabled())
+    return s;
+  s.NTR = ragged_tiles(s.c_dst, worth_96_columns(a.n_pairs, a.n_src, a.n_dst));
+  s.SR = ragged_steps(s.c_src);
+  s.lds_rows_bytes = 2 * (size_t)s.SR * s.NTR * 64 * 16 + (size_t)kWaves * kWaveRows * 2 * s.SR * 16 +
+                     (size_t)kWaves * 3 * kWaveRows * sizeof(int);
+  s.ok = s.NTR > 0;
   return s;
 }
 
@@ -1162,18 +1229,12 @@ RowsGrid rows_grid(int64_t n_dst, unsigned gy, int stages, bool can_half, bool h
   return g;
 }
 
-// FGMS_RAW_WEIGHTS=0 keeps the forward pass on re-laid weights (for comparison).
-bool raw_weights_enabled() {
-  static const bool on = !(getenv("FGMS_RAW_WEIGHTS") && atoi(getenv("FGMS_RAW_WEIGHTS")) == 0);
-  return on;
-}
-
-template <typename T, int NT, int S>
+template <typename T, int NT, int S, bool RAGGED = false>
 int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
                 const unsigned long long *masks, const int32_t *perm, const int32_t *tile_order,
                 int tile_grid, int flip, bool pair_view = false) {
-  const int slabs = s.c_src / (2 * S * s.E);
-  const unsigned gy = (unsigned)(s.c_dst / (32 * NT));
+  const int slabs = (s.c_src + 2 * S * s.E - 1) / (2 * S * s.E);
+  const unsigned gy = (unsigned)((s.c_dst + 32 * NT - 1) / (32 * NT));
   constexpr bool kCanHalf = NT != 4;
   const RowsGrid rg = rows_grid(a.n_dst, gy, a.k_vol * slabs, kCanHalf, tile_order != nullptr, tile_grid, pair_view,
                                 NT >= 3 ? 2 : 3, a.transpose_w, kCanHalf && !a.transpose_w);
@@ -1184,7 +1245,15 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
   // 47.2 / 66.4 -> 40.9; tf32 mode over 5 k 35.2 / 31.6 -> 27.4; 128 -> 128 fp16 over 2 k 21.8 / 24.1 -> 19.5.
   if constexpr (NT == 2 || NT == 3) {
     if (rg.groups == 4 && (int64_t)rg.gx * gy * NT <= num_cus())
-      return launch_rows<T, 1, S>(a, s, nbr, masks, perm, tile_order, tile_grid, flip, pair_view);
+      return launch_rows<T, 1, S, RAGGED>(a, s, nbr, masks, perm, tile_order, tile_grid, flip, pair_view);
+    // ... and where 96-column tiles would be partly empty and 32-column ones fit the chip in one round
+    // (128 -> 160 fp16 over 20 k voxels 48.6 -> 37.5 us)
+    if (RAGGED && NT == 3 && (s.c_dst + 31) / 32 % 3 != 0 &&
+        (a.n_dst + 127) / 128 * ((s.c_dst + 31) / 32) <= (int64_t)num_cus() * 4) {
+      if (s.c_dst % 32 == 0 && s.c_src % (2 * S * s.E) == 0)      // (nothing left to mask)
+        return launch_rows<T, 1, S>(a, s, nbr, masks, perm, tile_order, tile_grid, flip, pair_view);
+      return launch_rows<T, 1, S, RAGGED>(a, s, nbr, masks, perm, tile_order, tile_grid, flip, pair_view);
+    }
   }
   // With 64-column wave tiles the input gradient and the fp16 forward pass read the weight
   // tensor as it is (16-byte aligned rows of the tile) when the caller brings no re-laid
@@ -1199,7 +1268,7 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
     raw = a.transpose_w ? 2 : (sizeof(T) == 2 ? 1 : 0);
   // pinned weights: their re-laid copy is made once, and its plain fragment reads beat the
   // transposing ones of the raw tile (64 -> 64 fp16 forward over 200k voxels 41.9 -> 41.3 us)
-  if (raw == 1 && weights_pinned(a.w)) {
+  if (!RAGGED && raw == 1 && weights_pinned(a.w)) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (!(a.stream && hipStreamIsCapturing(a.stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone)) raw = 0;
   }
@@ -1233,7 +1302,8 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
   constexpr int kRaw4 = kCanSplit ? 4 : 0, kRaw3 = kCanSplit ? 3 : 0, kRaw2 = kCanRaw ? 2 : 0, kRaw1 = kCanRaw && sizeof(T) == 2 ? 1 : 0;
   // (raw is one of the five the type and the tile allow)
 #define FGMS_BY_RAW(MTv, KGv)                                                                                       \
-  (raw == 4   ? gms_rows_kernel<T, NT, S, kRaw4, MTv, KGv>                                                          \
+  (RAGGED     ? gms_rows_kernel<T, NT, S, RAGGED ? kRaw1 : 0, MTv, KGv, RAGGED>                                     \
+   : raw == 4   ? gms_rows_kernel<T, NT, S, kRaw4, MTv, KGv>                                                          \
    : raw == 3 ? gms_rows_kernel<T, NT, S, kRaw3, MTv, KGv>                                                          \
    : raw == 2 ? gms_rows_kernel<T, NT, S, kRaw2, MTv, KGv>                                                          \
    : raw == 1 ? gms_rows_kernel<T, NT, S, kRaw1, MTv, KGv>                                                          \
@@ -1281,7 +1351,7 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
 // plan's XCD-aware orders of either kind assume.
 // (2 waves per SIMD where the weight gradient's tile is 128 x 128: its 64 accumulators per lane and
 // the rows in flight spill at 3.  128 -> 128 over 40k voxels, forward and backward: tf32 mode 477 -> 327 us.)
-template <typename T, int NT, int S, int BI, int BJ, int RAWD, int MT = 2>
+template <typename T, int NT, int S, int BI, int BJ, int RAWD, int MT = 2, bool RAGGED = false>
 __global__ __launch_bounds__(kThreads, NT >= 3 || BI * BJ == 16 || ((BI == 3 || BJ == 3) && BI * BJ >= 6) ? 2 : 3) void bwd_fused_kernel(
     const T *__restrict__ gout, const T *__restrict__ w, T *__restrict__ gin,
     const int32_t *__restrict__ nbr, const unsigned long long *__restrict__ block_masks,
@@ -1300,12 +1370,12 @@ __global__ __launch_bounds__(kThreads, NT >= 3 || BI * BJ == 16 || ((BI == 3 || 
   }
   if ((int)blockIdx.x < rows_total) {
     const int bx = blockIdx.x % row_x, rest = blockIdx.x / row_x;
-    gms_rows_body<T, NT, S, RAWD, MT>(gout, w, gin, nbr, block_masks, perm, tile_order, n_in, k_vol, c_out, c_in,
+    gms_rows_body<T, NT, S, RAWD, MT, 1, RAGGED>(gout, w, gin, nbr, block_masks, perm, tile_order, n_in, k_vol, c_out, c_in,
                                       part_stages, bx, rest % row_y, rest / row_y, row_z, gout_bytes, 0, overwrite, flip);
   } else {
     const int j = blockIdx.x - rows_total;
     if constexpr (BI <= 3 && BJ <= 3)
-      wgrad_wave_body<T, BI, BJ, RAWD == 4>(in, gout, gw32, kpos, imap, omap, k_vol, c_in, c_out, smap,
+      wgrad_wave_body<T, BI, BJ, RAWD == 4, RAGGED>(in, gout, gw32, kpos, imap, omap, k_vol, c_in, c_out, smap,
                                             j % wgrad_x, j / wgrad_x, in_bytes, gout_bytes);
     else
       wgrad_wg_body<T, BI, BJ, RAWD == 4>(in, gout, gw32, kpos, imap, omap, k_vol, c_in, c_out, smap,
@@ -1319,12 +1389,12 @@ bool fused_bwd_enabled() {
   return on;
 }
 
-template <typename T, int NT, int S, int BI, int BJ>
+template <typename T, int NT, int S, int BI, int BJ, bool RAGGED = false>
 int launch_fused(const GmsArgs &d, const Shape &s, const Plan *p, const WgradArgs &w, const WgradGeometry &g,
                  float *acc32) {
   // the input gradient's grid, as launch_rows lays it out (tiles padded to a multiple of 8)
-  const int slabs = s.c_src / (2 * S * s.E);
-  const unsigned row_y = (unsigned)(s.c_dst / (32 * NT));
+  const int slabs = (s.c_src + 2 * S * s.E - 1) / (2 * S * s.E);
+  const unsigned row_y = (unsigned)((s.c_dst + 32 * NT - 1) / (32 * NT));
   constexpr bool kCanHalf = NT != 4;
   const RowsGrid rg = rows_grid(d.n_dst, row_y, d.k_vol * slabs, kCanHalf, p->tile_in != nullptr, p->tile_grid_in,
                                 false, NT >= 3 ? 2 : 3, true, false);
@@ -1346,10 +1416,10 @@ int launch_fused(const GmsArgs &d, const Shape &s, const Plan *p, const WgradArg
   constexpr bool kCanSplit = sizeof(T) == 4 && S == 4 && NT != 4;
   const bool split = kCanSplit && d.reduced && split_bf16_enabled() && g.split;
   constexpr int kHalfMT = kCanHalf ? 1 : 2;
-  auto kern = rg.half_tiles ? (split ? bwd_fused_kernel<T, NT, S, BI, BJ, kCanSplit ? 4 : 2, kHalfMT>
-                                     : bwd_fused_kernel<T, NT, S, BI, BJ, 2, kHalfMT>)
-              : split       ? bwd_fused_kernel<T, NT, S, BI, BJ, kCanSplit ? 4 : 2>
-                            : bwd_fused_kernel<T, NT, S, BI, BJ, 2>;
+  auto kern = rg.half_tiles ? (split ? bwd_fused_kernel<T, NT, S, BI, BJ, kCanSplit ? 4 : 2, kHalfMT, RAGGED>
+                                     : bwd_fused_kernel<T, NT, S, BI, BJ, 2, kHalfMT, RAGGED>)
+              : split       ? bwd_fused_kernel<T, NT, S, BI, BJ, kCanSplit ? 4 : 2, 2, RAGGED>
+                            : bwd_fused_kernel<T, NT, S, BI, BJ, 2, 2, RAGGED>;
   { const int rc_lds = allow_dynamic_lds(reinterpret_cast<const void *>(kern), (size_t)lds); if (rc_lds != FGMS_OK) return rc_lds; }
   {
     ProfileScope prof(split ? "bwd_fused_kernel(bf16x3)" : "bwd_fused_kernel", d.stream);
@@ -1467,6 +1537,43 @@ int launch_fused_bwd(const GmsArgs &d, const Plan *p, const WgradArgs &w, bool *
   return wgrad_finish(w, acc32);
 }
 
+// The output-stationary kernel gathers through a buffer resource: 32-bit byte offsets, and
+// offsets at or above 2^31 stand for "no row" (gather_issue_buf).
+static bool rows_fit_buffer(const GmsArgs &a) {
+  const size_t c_src = a.transpose_w ? a.c_out : a.c_in;
+  return (size_t)a.n_src * c_src * (a.dtype == FGMS_F16 ? 2 : 4) <= kMaxBufferBytes;
+}
+
+// The same for channel counts that fill no whole tile (fp16).
+int launch_ragged_bwd(const GmsArgs &d, const Plan *p, const WgradArgs &w, bool *done) {
+  *done = false;
+  if (!fused_bwd_enabled() || !p || !p->groups.empty() || d.k_vol > 64 || d.k_vol != p->k_vol || !p->dgrad_ok ||
+      d.n_dst != p->n_in || d.n_src != p->n_out || !rows_fit_buffer(d))
+    return FGMS_OK;
+  const Shape s = ragged_shape(d);
+  WgradGeometry g;
+  if (!s.ok || !ragged_wgrad_geometry(w, ragged_tiles(w.c_in, worth_96_columns(w.n_pairs, w.n_in, w.n_out)),
+                                      ragged_tiles(w.c_out, worth_96_columns(w.n_pairs, w.n_in, w.n_out)), &g))
+    return FGMS_OK;
+  bool found = false;
+  int rc = FGMS_OK;
+  float *acc32 = nullptr;
+#define FGMS_FR(NTv, Sv, BJv)                                                                                     \
+  if (!found && s.NTR == NTv && s.SR == Sv && g.bi == NTv && g.bj == BJv) {                                       \
+    found = true;                                                                                                 \
+    if ((rc = wgrad_accumulator(w, &acc32)) == FGMS_OK)                                                           \
+      rc = launch_fused<__half, NTv, Sv, NTv, BJv, true>(d, s, p, w, g, acc32);                                   \
+  }
+  FGMS_FR(1, 2, 1) FGMS_FR(1, 3, 2) FGMS_FR(1, 4, 2) FGMS_FR(1, 3, 3) FGMS_FR(1, 2, 3) FGMS_FR(1, 4, 3)
+  FGMS_FR(2, 2, 1) FGMS_FR(2, 3, 2) FGMS_FR(2, 4, 2) FGMS_FR(2, 3, 3) FGMS_FR(2, 2, 3) FGMS_FR(2, 4, 3)
+  FGMS_FR(3, 2, 1) FGMS_FR(3, 3, 2) FGMS_FR(3, 4, 2) FGMS_FR(3, 3, 3) FGMS_FR(3, 2, 3) FGMS_FR(3, 4, 3)
+#undef FGMS_FR
+  if (!found) return FGMS_OK;
+  if (rc != FGMS_OK) return rc;
+  *done = true;
+  return wgrad_finish(w, acc32);
+}
+
 int planned_pack_job(const GmsArgs &a, SideJob *job, const void **packed) {
   const Shape s = shape_of(a);
   if (!s.ok) {
@@ -1522,13 +1629,6 @@ int launch_mfma_gms(const GmsArgs &a) {
   });
 }
 
-// The output-stationary kernel gathers through a buffer resource: 32-bit byte offsets, and
-// offsets at or above 2^31 stand for "no row" (gather_issue_buf).
-static bool rows_fit_buffer(const GmsArgs &a) {
-  const size_t c_src = a.transpose_w ? a.c_out : a.c_in;
-  return (size_t)a.n_src * c_src * (a.dtype == FGMS_F16 ? 2 : 4) <= kMaxBufferBytes;
-}
-
 bool planned_gms_supported(const GmsArgs &a, const Plan *p) {
   if (!p || a.dense_k >= 0 || a.k_vol > 64 || a.k_vol != p->k_vol) return false;
   if (a.transpose_w) {
@@ -1567,6 +1667,28 @@ int launch_planned_gms(const GmsArgs &a, const Plan *p) {
     return launch_rows<float, decltype(nt)::value, decltype(sv)::value>(a_, s, nbr, masks, perm, tile_order, tile_grid,
                                                                               flip);
   });
+}
+
+bool ragged_gms_supported(const GmsArgs &a, const Plan *p) {
+  if (!p || !p->groups.empty() || a.dense_k >= 0 || a.transpose_w || a.k_vol > 64 || a.k_vol != p->k_vol) return false;
+  return p->fwd_ok && a.n_dst == p->n_out && a.n_src == p->n_in && rows_fit_buffer(a) && ragged_shape(a).ok;
+}
+
+int launch_ragged_gms(const GmsArgs &a, const Plan *p) {
+  const Shape s = ragged_shape(a);
+  if (!ragged_gms_supported(a, p)) {
+    set_error("launch_ragged_gms: unsupported shape or plan");
+    return FGMS_E_INVALID;
+  }
+  GmsArgs a_ = a;
+  if (!a_.side.kind) (void)plan_take_check(p, &a_.side);
+#define FGMS_RG(NTv, Sv)                   \
+  if (s.NTR == NTv && s.SR == Sv)          \
+    return launch_rows<__half, NTv, Sv, true>(a_, s, p->nbr_out, p->mask_out, p->perm_out, p->tile_out, p->tile_grid_out, p->flip_out);
+  FGMS_RG(1, 2) FGMS_RG(1, 3) FGMS_RG(1, 4) FGMS_RG(2, 2) FGMS_RG(2, 3) FGMS_RG(2, 4) FGMS_RG(3, 2) FGMS_RG(3, 3) FGMS_RG(3, 4)
+#undef FGMS_RG
+  set_error("launch_ragged_gms: no such tile");
+  return FGMS_E_INVALID;
 }
 
 bool pair_view_gms_supported(const GmsArgs &a, const Plan *p) {

@@ -3,6 +3,9 @@
 // and of the weights, results cropped on their way back.  The padding channels are zero in both
 // operands of every product, so the results are those of the original shape.
 //
+// (fp16 counts that are multiples of 8 do without on dense maps: there the MFMA kernels mask the rest of
+// a tile themselves.  48 -> 48 over 80 k voxels, forward and backward, 100.7 us over copies, 64.6 without.)
+//
 // Bound by memory: a copy reads n * c and writes n * c_padded elements once, 16 bytes per thread,
 // where the shape-agnostic kernels spend a scalar atomic per result element: 96 -> 20 fp16 over
 // 60 k voxels, forward and backward, 2378 us without and 95 us with the copies; 3 -> 32 over 125

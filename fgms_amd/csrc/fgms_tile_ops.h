@@ -66,12 +66,14 @@ __device__ __forceinline__ int4v raw_weight_frag(const int4v *__restrict__ w_lds
 }
 
 // dst[rows[r]][cd0 .. cd0 + NT * 32) = 0 for the WR rows of a wave.
-template <typename T, int NT, int WR>
+// (RAGGED, here and below: the tile's columns from c_dst on do not exist.)
+template <typename T, int NT, int WR, bool RAGGED = false>
 __device__ __forceinline__ void zero_rows(T *__restrict__ dst, const int *__restrict__ rows, int c_dst, int cd0, int lane) {
   constexpr int CH = NT * 32 * (int)sizeof(T) / 8;      // 8-byte pieces per row
 #pragma unroll 1
   for (int e = lane; e < WR * CH; e += 64) {
     const int row = rows[e / CH];
+    if (RAGGED && cd0 + (e % CH) * 8 / (int)sizeof(T) >= c_dst) continue;
     if (row >= 0) *reinterpret_cast<int2v *>(reinterpret_cast<char *>(dst + (size_t)row * c_dst + cd0) + (e % CH) * 8) = int2v{0, 0};
   }
 }
@@ -80,7 +82,7 @@ __device__ __forceinline__ void zero_rows(T *__restrict__ dst, const int *__rest
 // (r / 4) * 8 + (l / 32) * 4 + r % 4 and column l % 32 of its 32x32 tile.  For
 // fp16 two lanes swap one value each so that every lane owns two neighbouring
 // columns of one row and can issue a packed 4-byte update.
-template <typename T, int NT, bool ATOMIC, int MT>
+template <typename T, int NT, bool ATOMIC, bool RAGGED = false, int MT>
 __device__ __forceinline__ void write_tile(const float16v (&acc)[MT][NT], T *__restrict__ dst,
                                            const int *__restrict__ rows, int c_dst, int cd0,
                                            int lane) {
@@ -89,11 +91,12 @@ __device__ __forceinline__ void write_tile(const float16v (&acc)[MT][NT], T *__r
   for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
+      const bool column = !RAGGED || cd0 + nt * 32 + col < c_dst;
       if constexpr (sizeof(T) == 4) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int row = rows[mt * 32 + (r / 4) * 8 + h * 4 + (r % 4)];
-          if (row >= 0) {
+          if (row >= 0 && column) {
             float *p = reinterpret_cast<float *>(dst) + (size_t)row * c_dst + cd0 + nt * 32 + col;
             if constexpr (ATOMIC) atomic_add(p, acc[mt][nt][r]);
             else *p += acc[mt][nt][r];
@@ -108,7 +111,7 @@ __device__ __forceinline__ void write_tile(const float16v (&acc)[MT][NT], T *__r
           const float lo = odd ? got : v0, hi = odd ? v1 : got;
           const int r = 2 * rp + (odd ? 1 : 0);
           const int row = rows[mt * 32 + (r / 4) * 8 + h * 4 + (r % 4)];
-          if (row >= 0) {
+          if (row >= 0 && column) {
             __half *p = reinterpret_cast<__half *>(dst) + (size_t)row * c_dst + cd0 + nt * 32 + (col & ~1);
             if constexpr (ATOMIC) {
               atomic_add_pk(p, lo, hi);
@@ -127,7 +130,7 @@ __device__ __forceinline__ void write_tile(const float16v (&acc)[MT][NT], T *__r
 // dst[rows[r]] += acc for the MT * 32 rows of a wave (rows[] in LDS, -1 = none; no
 // atomics: the caller owns these rows).  All reads of the old values are issued
 // before the first add so that they overlap.
-template <typename T, int NT, int MT>
+template <typename T, int NT, bool RAGGED = false, int MT>
 __device__ __forceinline__ void add_rows(const float16v (&acc)[MT][NT], T *__restrict__ dst,
                                          const int *__restrict__ rows, int c_dst, int cd0,
                                          int lane) {
@@ -140,6 +143,7 @@ __device__ __forceinline__ void add_rows(const float16v (&acc)[MT][NT], T *__res
       for (int r = 0; r < 16; ++r) row[r] = rows[mt * 32 + (r / 4) * 8 + h * 4 + (r % 4)];
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
+        if (RAGGED && cd0 + nt * 32 + col >= c_dst) continue;
         float old[16];
 #pragma unroll
         for (int r = 0; r < 16; ++r)
@@ -161,10 +165,11 @@ __device__ __forceinline__ void add_rows(const float16v (&acc)[MT][NT], T *__res
       }
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
+        const bool column = !RAGGED || cd0 + nt * 32 + col < c_dst;
         __half2 old[8];
 #pragma unroll
         for (int rp = 0; rp < 8; ++rp)
-          old[rp] = *reinterpret_cast<const __half2 *>(
+          old[rp] = !column ? __half2{} : *reinterpret_cast<const __half2 *>(
               reinterpret_cast<const __half *>(dst) + (size_t)max(row[rp], 0) * c_dst + cd0 +
               nt * 32 + (col & ~1));
 #pragma unroll
@@ -173,7 +178,7 @@ __device__ __forceinline__ void add_rows(const float16v (&acc)[MT][NT], T *__res
           const float got = swap_with_neighbour(odd ? v0 : v1);
           const float lo = odd ? got : v0, hi = odd ? v1 : got;
           const float2 o = __half22float2(old[rp]);
-          if (row[rp] >= 0)
+          if (row[rp] >= 0 && column)
             *reinterpret_cast<__half2 *>(reinterpret_cast<__half *>(dst) + (size_t)row[rp] * c_dst +
                                          cd0 + nt * 32 + (col & ~1)) =
                 __floats2half2_rn(o.x + lo, o.y + hi);
@@ -190,7 +195,7 @@ __device__ __forceinline__ void add_rows(const float16v (&acc)[MT][NT], T *__res
 // 64..256-byte runs by neighbouring lanes instead of 4 bytes per lane.
 // stage: the wave's staging tile, MT * 32 rows of 2*S * 16 bytes.
 // OVERWRITE (not with ATOMIC): dst[rows[r]] = acc; the old values are not read.
-template <typename T, int NT, int S, bool ATOMIC, bool OVERWRITE, int MT>
+template <typename T, int NT, int S, bool ATOMIC, bool OVERWRITE, bool RAGGED = false, int MT>
 __device__ __forceinline__ void add_rows_lds(const float16v (&acc)[MT][NT], T *__restrict__ dst,
                                              const int *__restrict__ rows, float *__restrict__ stage,
                                              int c_dst, int cd0, int lane) {
@@ -199,14 +204,14 @@ __device__ __forceinline__ void add_rows_lds(const float16v (&acc)[MT][NT], T *_
   constexpr int FIT = (WR * 2 * S * 16) / (COLS * 4);
   constexpr int R = FIT >= 32 ? 32 : FIT >= 16 ? 16 : FIT >= 8 ? 8 : 0;
   if constexpr (R < 8) {
-    if constexpr (ATOMIC) write_tile<T, NT, true>(acc, dst, rows, c_dst, cd0, lane);
+    if constexpr (ATOMIC) write_tile<T, NT, true, RAGGED>(acc, dst, rows, c_dst, cd0, lane);
     else {
       if constexpr (OVERWRITE) {
-        zero_rows<T, NT, WR>(dst, rows, c_dst, cd0, lane);
+        zero_rows<T, NT, WR, RAGGED>(dst, rows, c_dst, cd0, lane);
         __builtin_amdgcn_s_waitcnt(0x0F70);      // vmcnt(0): the zeros are on their way before the rows are read
         __threadfence();
       }
-      add_rows<T, NT>(acc, dst, rows, c_dst, cd0, lane);
+      add_rows<T, NT, RAGGED>(acc, dst, rows, c_dst, cd0, lane);
     }
   } else {
     constexpr int CH = COLS / 4;            // 16-byte chunks per staged row
@@ -225,7 +230,8 @@ __device__ __forceinline__ void add_rows_lds(const float16v (&acc)[MT][NT], T *_
 #pragma unroll
         for (int it = 0; it < IT; ++it) {
           const int e = it * 64 + lane;
-          ahead[p][it] = *reinterpret_cast<const half4 *>(
+          if (RAGGED && cd0 + (e % CH) * 4 >= c_dst) ahead[p][it] = half4{0, 0, 0, 0};
+          else ahead[p][it] = *reinterpret_cast<const half4 *>(
               reinterpret_cast<const _Float16 *>(dst) + (size_t)max(rows[p * R + e / CH], 0) * c_dst + cd0 +
               (e % CH) * 4);
         }
@@ -250,7 +256,7 @@ __device__ __forceinline__ void add_rows_lds(const float16v (&acc)[MT][NT], T *_
         for (int q = 0; q < R * WORDS / 64; ++q) {
           const int e = q * 64 + lane;
           const int r = e / WORDS, c = e % WORDS;
-          const int row = rows[p * R + r];
+          const int row = RAGGED && cd0 + c * (4 / (int)sizeof(T)) >= c_dst ? -1 : rows[p * R + r];
           if constexpr (sizeof(T) == 4) {
             const float v = stage[r * COLS + c];
             if (row >= 0) atomic_add(reinterpret_cast<float *>(dst) + (size_t)row * c_dst + cd0 + c, v);
@@ -269,7 +275,7 @@ __device__ __forceinline__ void add_rows_lds(const float16v (&acc)[MT][NT], T *_
       for (int it = 0; it < IT; ++it) {
         const int e = it * 64 + lane;
         part[it] = *reinterpret_cast<const float4v *>(stage + (e / CH) * COLS + (e % CH) * 4);
-        row[it] = rows[p * R + e / CH];
+        row[it] = RAGGED && cd0 + (e % CH) * 4 >= c_dst ? -1 : rows[p * R + e / CH];
       }
       if constexpr (sizeof(T) == 4) {
         float4v old[IT];
@@ -294,6 +300,8 @@ __device__ __forceinline__ void add_rows_lds(const float16v (&acc)[MT][NT], T *_
           if constexpr (kAhead)
             old[it] = ahead[p][it];
           else if constexpr (OVERWRITE)
+            old[it] = half4{0, 0, 0, 0};
+          else if (RAGGED && row[it] < 0)
             old[it] = half4{0, 0, 0, 0};
           else
             old[it] = *reinterpret_cast<const half4 *>(

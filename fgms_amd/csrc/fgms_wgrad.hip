@@ -408,6 +408,23 @@ bool mfma_wgrad_supported(const WgradArgs &a) {
   return true;
 }
 
+// Grid and LDS of the per-wave body for g's tile.
+static void wave_geometry(const WgradArgs &a, WgradGeometry *g) {
+  const bool f16 = a.dtype == FGMS_F16;
+  const int bi = g->bi, bj = g->bj, pad = f16 ? 0 : WT<float>::pad;
+  const int sp = f16 ? WTW<__half>::stage_pairs : WTW<float>::stage_pairs;
+  g->wave = true;
+  g->smap = choose_slices(a, g->ty, sp, (int64_t)num_cus() * 6);
+  g->tiles = (int64_t)g->smap.slices * a.k_vol;
+  // fp32 tensors whose caller allows tf32 precision: four 16-bit tiles per wave instead
+  g->split = !f16 && a.reduced && split_bf16_enabled();
+  const size_t lds = (g->split ? 4 * (size_t)sp * 2 * ((bi * 32 + 16) + (bj * 32 + 16)) * 2
+                               : 4 * (size_t)sp * ((bi * 32 + pad) + (bj * 32 + pad)) * (f16 ? 2 : 4))
+                     + 4 * 64 * sizeof(int);                           // + the waves' index exchange
+  const size_t red = 3 * (size_t)(bi * bj > 4 ? 1 : bi) * bj * 16 * 64 * sizeof(float);     // the partial tiles' exchange
+  g->lds = lds < red ? red : lds;
+}
+
 int wgrad_geometry(const WgradArgs &a, WgradGeometry *g, bool shares_grid) {
   if (skinny_shape(a) || !mfma_wgrad_supported(a)) {
     set_error("wgrad_geometry: not a shape of the MFMA weight-gradient kernels");
@@ -422,18 +439,8 @@ int wgrad_geometry(const WgradArgs &a, WgradGeometry *g, bool shares_grid) {
   g->bi = bi;
   g->bj = bj;
   g->ty = (a.c_in / (32 * bi)) * (a.c_out / (32 * bj));
-  g->wave = bi <= 3 && bj <= 3;
-  if (g->wave) {
-    const int sp = f16 ? WTW<__half>::stage_pairs : WTW<float>::stage_pairs;
-    g->smap = choose_slices(a, g->ty, sp, (int64_t)num_cus() * 6);
-    g->tiles = (int64_t)g->smap.slices * a.k_vol;
-    // fp32 tensors whose caller allows tf32 precision: four 16-bit tiles per wave instead
-    g->split = !f16 && a.reduced && split_bf16_enabled();
-    const size_t lds = (g->split ? 4 * (size_t)sp * 2 * ((bi * 32 + 16) + (bj * 32 + 16)) * 2
-                                 : 4 * (size_t)sp * ((bi * 32 + (f16 ? 0 : pad)) + (bj * 32 + (f16 ? 0 : pad))) * esz)
-                       + 4 * 64 * sizeof(int);                           // + the waves' index exchange
-    const size_t red = 3 * (size_t)(bi * bj > 4 ? 1 : bi) * bj * 16 * 64 * sizeof(float);     // the partial tiles' exchange
-    g->lds = lds < red ? red : lds;
+  if (bi <= 3 && bj <= 3) {
+    wave_geometry(a, g);
     return FGMS_OK;
   }
   const int sp = f16 ? WT<__half>::stage_pairs : WT<float>::stage_pairs;
@@ -456,6 +463,18 @@ int wgrad_geometry(const WgradArgs &a, WgradGeometry *g, bool shares_grid) {
   g->lds = g->split ? 2 * (size_t)sp * 2 * ((bi * 32 + 16) + (bj * 32 + 16)) * 2
                     : 2 * (size_t)sp * ((bi * 32 + pad) + (bj * 32 + pad)) * esz;
   return FGMS_OK;
+}
+
+bool ragged_wgrad_geometry(const WgradArgs &a, int bi, int bj, WgradGeometry *g) {
+  if (a.dtype != FGMS_F16 || bi < 1 || bj < 1 || a.side.kind || a.crop_in) return false;
+  if (reinterpret_cast<uintptr_t>(a.in) % 16 || reinterpret_cast<uintptr_t>(a.gout) % 16) return false;
+  if ((size_t)a.n_in * a.c_in * 2 > kMaxBufferBytes || (size_t)a.n_out * a.c_out * 2 > kMaxBufferBytes) return false;
+  *g = WgradGeometry{};
+  g->bi = bi;
+  g->bj = bj;
+  g->ty = ((a.c_in + 32 * bi - 1) / (32 * bi)) * ((a.c_out + 32 * bj - 1) / (32 * bj));
+  wave_geometry(a, g);
+  return true;
 }
 
 int wgrad_accumulator(const WgradArgs &a, float **acc32) {

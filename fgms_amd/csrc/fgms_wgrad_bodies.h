@@ -137,7 +137,9 @@ template <> struct WTW<float> { static constexpr int stage_pairs = 16; };
 // bf16 pairs, x = hi + lo, on their way to LDS -- four 16-bit tiles per wave, laid out like
 // the fp16 path's two -- and a product is three bf16 MFMAs, hi*hi + hi*lo + lo*hi, fed
 // through the same transposing LDS reads as fp16.
-template <typename T, int BI, int BJ, bool SPLIT = false>
+// RAGGED (fp16): the tile's channels from c_in / c_out on do not exist; they are loaded from outside the
+// buffers, as zeros, and not flushed.
+template <typename T, int BI, int BJ, bool SPLIT = false, bool RAGGED = false>
 __device__ __forceinline__ void wgrad_wave_body(
     const T *__restrict__ in, const T *__restrict__ gout, float *__restrict__ gw32,
     const int32_t *__restrict__ kpos, const int32_t *__restrict__ imap,
@@ -155,11 +157,12 @@ __device__ __forceinline__ void wgrad_wave_body(
   constexpr int LDI = CI + (kBufW ? 0 : W::pad), LDO = CO + (kBufW ? 0 : W::pad);
   constexpr int NCI = CI / E, NCO = CO / E;
   constexpr int NX = SP * NCI / 64, NG = SP * NCO / 64;   // chunks per lane and stage
+  static_assert(!RAGGED || kBufW, "ragged: fp16");
   static_assert(NX >= 1 && NG >= 1, "stage too small");
   extern __shared__ int4v lds[];
   int k, first, count;
   if (!locate_slice(kpos, smap, k_vol, block_x, k, first, count)) return;
-  const int tiles_co = c_out / CO;
+  const int tiles_co = RAGGED ? (c_out + CO - 1) / CO : c_out / CO;
   const int ci0 = (block_y / tiles_co) * CI;
   const int co0 = (block_y % tiles_co) * CO;
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
@@ -245,7 +248,7 @@ __device__ __forceinline__ void wgrad_wave_body(
     for (int i = 0; i < NX; ++i) {
       const int cc = x_chunk(i);
       if constexpr (kBufW) {
-        const bool live = st_ * SP + x_row(i) < count;
+        const bool live = st_ * SP + x_row(i) < count && (!RAGGED || ci0 + cc * E < c_in);
         const unsigned off = live ? (unsigned)xi[i] * (unsigned)(c_in * (int)sizeof(T)) : kAbsentRow;
         xr[i] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(
                                               in_rsrc, off + (unsigned)((ci0 + cc * E) * (int)sizeof(T)), 0, 0));
@@ -257,7 +260,7 @@ __device__ __forceinline__ void wgrad_wave_body(
     for (int i = 0; i < NG; ++i) {
       const int cc = g_chunk(i);
       if constexpr (kBufW) {
-        const bool live = st_ * SP + g_row(i) < count;
+        const bool live = st_ * SP + g_row(i) < count && (!RAGGED || co0 + cc * E < c_out);
         const unsigned off = live ? (unsigned)gi[i] * (unsigned)(c_out * (int)sizeof(T)) : kAbsentRow;
         gr[i] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(
                                               gout_rsrc, off + (unsigned)((co0 + cc * E) * (int)sizeof(T)), 0, 0));
@@ -420,6 +423,7 @@ __device__ __forceinline__ void wgrad_wave_body(
 #pragma unroll
         for (int slot = 0; slot < 3; ++slot) v += red[(size_t)((q * 3 + slot) * RQ + j) * 64 + lane];
         // accumulator register r of lane l is row (r/4)*8 + (l/32)*4 + r%4, column l%32 of its 32 x 32 tile
+        if (RAGGED && (ci0 + ti * 32 + (r / 4) * 8 + h * 4 + (r % 4) >= c_in || co0 + tj * 32 + c >= c_out)) continue;
         atomic_add(gw32 + ((size_t)k * c_in + ci0 + ti * 32 + (r / 4) * 8 + h * 4 + (r % 4)) * c_out + co0 + tj * 32 + c, v);
       }
     }
@@ -675,6 +679,8 @@ struct WgradGeometry {
 };
 // shares_grid: the launch also holds the input gradient's workgroups.
 int wgrad_geometry(const WgradArgs &a, WgradGeometry *g, bool shares_grid = false);
+// For a tile of bi x bj blocks whose last channels need not exist (false: not fp16, or not that size).
+bool ragged_wgrad_geometry(const WgradArgs &a, int bi, int bj, WgradGeometry *g);
 // Where the kernels accumulate: the caller's fp32 tensor, or for fp16 the stream's fp32
 // scratch (zero between calls), which wgrad_finish rounds into the caller's tensor and
 // clears again in a launch of its own.

@@ -88,3 +88,11 @@ def test_small_forward_launches(oracle, n, dtype, tf32):
                                      (900, (64, 96)), (900, (96, 128)), (900, (128, 96)), (900, (24, 96)), (900, (48, 160)), (70001, (96, 96))])
 def test_96_and_48_channels(oracle, n, shape, dtype, tf32, use_plan):
     test_written_not_added(oracle, n, shape, dtype, tf32, use_plan)
+
+
+@pytest.mark.parametrize("n,shape", [(65, (48, 48)), (900, (24, 24)), (900, (16, 32)), (900, (24, 48)), (900, (48, 24)), (900, (40, 56)),
+                                     (900, (96, 48)), (900, (80, 72)), (900, (160, 160)), (900, (128, 24)), (900, (104, 136)), (3000, (56, 88)),
+                                     (40000, (48, 48)), (70001, (24, 48)), (70001, (48, 160))])
+def test_channels_that_fill_no_tile(oracle, n, shape):
+    """Masked columns and channels (fp16), at the edges of 16-byte chunks, slabs and 32-column tiles."""
+    test_written_not_added(oracle, n, shape, np.float16, False, True)
