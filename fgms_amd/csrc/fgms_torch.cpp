@@ -306,6 +306,14 @@ void ConvolutionBackward(const at::Tensor out_feats_grad, const at::Tensor in_fe
 
 namespace {
 
+// The layer has no formula for tangents: an input that carries one is refused, as torch refuses it for a
+// python autograd.Function without jvp (the kernels read the primal values alone, and an output without a
+// tangent stands for a derivative of zero).
+void refuse_tangent(const at::Tensor &t, const char *name) {
+  TORCH_CHECK_NOT_IMPLEMENTED(!torch::autograd::isFwGradDefined(t), "sparse_conv has no forward-mode derivative, but ",
+                              name, " carries a tangent");
+}
+
 // One kernel map as a layer uses it.
 struct LayerMap {
   at::Tensor kpos, in_map, out_map;
@@ -334,6 +342,9 @@ struct SparseConvBackward final : public torch::autograd::Node {
     std::lock_guard<std::mutex> lock(mutex_);
     if (!grads[0].defined()) return {at::Tensor(), at::Tensor()};
     const at::Tensor x = feats.unpack(shared_from_this()), w = weight.unpack(shared_from_this());
+    refuse_tangent(x, "feats");
+    refuse_tangent(w, "weight");
+    refuse_tangent(grads[0], "the output gradient");
     at::NoGradGuard no_grad;
     at::Tensor g = grads[0].contiguous();
     same_dtype(x, g, "the output gradient");
@@ -369,6 +380,8 @@ at::Tensor sparse_conv(const at::Tensor &feats, const at::Tensor &weight, const 
     throw std::invalid_argument("feats has " + std::to_string(feats.size(0)) + " rows, the kernel map expects " +
                                 std::to_string(n_in));
   check_channels(feats, weight);
+  refuse_tangent(feats, "feats");
+  refuse_tangent(weight, "weight");
   const LayerMap map{kpos, in_map, out_map, n_in, n_out};
   at::Tensor x, w, out;
   {

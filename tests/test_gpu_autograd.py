@@ -102,3 +102,31 @@ def test_kernel_map_checks_its_sizes():
     kmap = fnn.KernelMap(e, e, [2, 3], 10, 10)
     with pytest.raises(ValueError):
         fnn.sparse_conv(torch.zeros(9, 4, device="cuda"), torch.zeros(2, 4, 4, device="cuda"), kmap)
+
+
+@pytest.fixture
+def one_layer():
+    from FGMS import nn as fnn
+    L = small_layer(44, 32, 48, np.float32)
+    D = G.to_dev(L)
+    kmap = fnn.KernelMap(D["imap"], D["omap"], L["knnz"], L["n_in"], L["n_out"])
+    return D["in_feats"], D["kernel"], D["out_grad"], kmap
+
+
+def test_tangents_are_refused(one_layer):
+    """No forward-mode derivative exists: an input with a tangent must not come out as one without."""
+    import torch.autograd.forward_ad as fwd
+    from FGMS import nn as fnn
+    x, w, g, kmap = one_layer
+    with fwd.dual_level():
+        for feats, weight in ((fwd.make_dual(x, x), w), (x, fwd.make_dual(w, w))):
+            with pytest.raises(NotImplementedError, match="tangent"):
+                fnn.sparse_conv(feats, weight, kmap)
+        leaf = x.clone().requires_grad_(True)
+        y = fnn.sparse_conv(leaf, w, kmap)
+        with pytest.raises(NotImplementedError, match="tangent"):
+            torch.autograd.grad(y, leaf, fwd.make_dual(g, g))
+        assert fwd.unpack_dual(fnn.sparse_conv(x, w, kmap)).tangent is None
+    for transform in (torch.func.vmap, lambda f: torch.func.grad(lambda t: f(t).sum()), lambda f: lambda t: torch.func.jvp(f, (t,), (t,))):
+        with pytest.raises(RuntimeError):
+            transform(lambda t: fnn.sparse_conv(t, w, kmap))(x[None] if transform is torch.func.vmap else x)
