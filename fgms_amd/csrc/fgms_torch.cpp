@@ -335,17 +335,29 @@ at::Tensor layer_forward(const at::Tensor &feats, const at::Tensor &weight, cons
 
 struct SparseConvBackward final : public torch::autograd::Node {
   torch::autograd::SavedVariable feats, weight;
+  std::vector<int64_t> feats_shape, weight_shape;
+  at::TensorOptions options;               // dtype and device of both
   LayerMap map;
   bool tf32 = false;
+
+  // A saved tensor as the forward pass had it.  Saved-tensor hooks (offloading, compression) may hand back
+  // any tensor for it, and the kernels go by its pointer and the forward pass's sizes.
+  at::Tensor unpacked(torch::autograd::SavedVariable &saved, const std::vector<int64_t> &shape, const char *name) {
+    const at::Tensor t = saved.unpack(shared_from_this());
+    TORCH_CHECK_VALUE(t.sizes() == at::IntArrayRef(shape) && t.dtype() == options.dtype() && t.device() == options.device(),
+                      "sparse_conv: the saved ", name, " came back with another shape, dtype or device than it was saved with");
+    refuse_tangent(t, name);
+    return t;
+  }
 
   torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
     if (!grads[0].defined()) return {at::Tensor(), at::Tensor()};
-    const at::Tensor x = feats.unpack(shared_from_this()), w = weight.unpack(shared_from_this());
-    refuse_tangent(x, "feats");
-    refuse_tangent(w, "weight");
+    at::Tensor x = unpacked(feats, feats_shape, "feats"), w = unpacked(weight, weight_shape, "weight");
     refuse_tangent(grads[0], "the output gradient");
     at::NoGradGuard no_grad;
+    x = x.contiguous();
+    w = w.contiguous();
     at::Tensor g = grads[0].contiguous();
     same_dtype(x, g, "the output gradient");
     const int k_vol = (int)w.size(0);
@@ -398,6 +410,9 @@ at::Tensor sparse_conv(const at::Tensor &feats, const at::Tensor &weight, const 
     node->set_next_edges(torch::autograd::collect_next_edges(feats, weight));
     node->feats = torch::autograd::SavedVariable(x, false);
     node->weight = torch::autograd::SavedVariable(w, false);
+    node->feats_shape = x.sizes().vec();
+    node->weight_shape = w.sizes().vec();
+    node->options = x.options();
     node->map = map;
     node->tf32 = tf32;
     torch::autograd::set_history(out, node);

@@ -130,3 +130,35 @@ def test_tangents_are_refused(one_layer):
     for transform in (torch.func.vmap, lambda f: torch.func.grad(lambda t: f(t).sum()), lambda f: lambda t: torch.func.jvp(f, (t,), (t,))):
         with pytest.raises(RuntimeError):
             transform(lambda t: fnn.sparse_conv(t, w, kmap))(x[None] if transform is torch.func.vmap else x)
+
+
+def test_saved_tensor_hooks(one_layer):
+    """Offloading hooks and checkpointing give the plain gradients; a hook that hands back something other
+    than what was saved is an error, not a read past its end."""
+    from torch.utils.checkpoint import checkpoint
+    from FGMS import nn as fnn
+    x0, w0, g, kmap = one_layer
+
+    def grads(layer, unpack=None, offload=False):
+        x, w = x0.clone().requires_grad_(True), w0.clone().requires_grad_(True)
+        if offload:
+            with torch.autograd.graph.save_on_cpu():
+                y = layer(x, w)
+        elif unpack:
+            with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+                y = layer(x, w)
+        else:
+            y = layer(x, w)
+        return torch.autograd.grad(y, (x, w), g)
+
+    conv = lambda x, w: fnn.sparse_conv(x, w, kmap)
+    want = grads(conv)
+    strided = lambda t: t.detach().transpose(0, 1).contiguous().transpose(0, 1)
+    for got in (grads(conv, offload=True), grads(conv, unpack=strided),
+                grads(lambda x, w: checkpoint(conv, x, w, use_reentrant=False))):
+        for a, b in zip(got, want):          # (sums of atomics: equal up to their order)
+            G.assert_close(a.cpu().numpy(), b.cpu().numpy(), "fp32")
+    for wrong in (lambda t: t.detach().half(), lambda t: t.detach().cpu(), lambda t: t.detach()[:-1], lambda t: t.detach()[..., :4],
+                  lambda t: t.detach().reshape(-1)):
+        with pytest.raises(ValueError, match="came back"):
+            grads(conv, unpack=wrong)
