@@ -27,6 +27,8 @@
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
+#include <torch/library.h>
 
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
@@ -384,7 +386,7 @@ struct SparseConvBackward final : public torch::autograd::Node {
 };
 
 // out[out_map[j]] += feats[in_map[j]] @ weight[k] over a zero output; differentiable in feats and weight.
-at::Tensor sparse_conv(const at::Tensor &feats, const at::Tensor &weight, const at::Tensor &kpos, const at::Tensor &in_map,
+at::Tensor sparse_conv_node(const at::Tensor &feats, const at::Tensor &weight, const at::Tensor &kpos, const at::Tensor &in_map,
                        const at::Tensor &out_map, int64_t n_in, int64_t n_out, bool tf32) {
   if (feats.dim() != 2 || weight.dim() != 3 || weight.size(0) != kpos.numel() - 1)
     throw std::invalid_argument("expected feats [N, Cin] and weight [K, Cin, Cout] with K = the map's offsets");
@@ -420,7 +422,23 @@ at::Tensor sparse_conv(const at::Tensor &feats, const at::Tensor &weight, const 
   return out;
 }
 
+// Under torch.jit.trace the layer goes through torch's dispatcher, as operator fgms::sparse_conv, whose
+// calls the tracer records; a plain function's result would stand in the graph as a constant.  (Only there:
+// the dispatcher costs a small layer host time and gives it nothing.)
+at::Tensor sparse_conv(const at::Tensor &feats, const at::Tensor &weight, const at::Tensor &kpos, const at::Tensor &in_map,
+                       const at::Tensor &out_map, int64_t n_in, int64_t n_out, bool tf32) {
+  if (!torch::jit::tracer::isTracing()) return sparse_conv_node(feats, weight, kpos, in_map, out_map, n_in, n_out, tf32);
+  static const auto op =
+      c10::Dispatcher::singleton().findSchemaOrThrow("fgms::sparse_conv", "").typed<decltype(sparse_conv)>();
+  return op.call(feats, weight, kpos, in_map, out_map, n_in, n_out, tf32);
+}
+
 }  // namespace
+
+TORCH_LIBRARY(fgms, m) {
+  m.def("sparse_conv(Tensor feats, Tensor weight, Tensor kpos, Tensor in_map, Tensor out_map, int n_in, int n_out, bool tf32) -> Tensor",
+        &sparse_conv_node);
+}
 
 namespace {
 

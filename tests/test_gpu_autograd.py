@@ -162,3 +162,30 @@ def test_saved_tensor_hooks(one_layer):
                   lambda t: t.detach().reshape(-1)):
         with pytest.raises(ValueError, match="came back"):
             grads(conv, unpack=wrong)
+
+
+def test_traced_layer_is_recorded(one_layer, tmp_path):
+    """torch.jit.trace records the call, not its result: other inputs give other outputs, gradients included."""
+    from FGMS import nn as fnn
+    x, w, g, kmap = one_layer
+
+    class Net(torch.nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.conv = fnn.SparseConv(w.shape[1], w.shape[2], 27, device="cuda")
+
+        def forward(self, t):
+            return torch.relu(self.conv(t, kmap))
+
+    net = Net()
+    traced = torch.jit.trace(net, x, check_trace=False)
+    torch.jit.save(traced, str(tmp_path / "net.pt"))
+    other = torch.randn_like(x)
+    with torch.no_grad():
+        net.conv.weight.mul_(-0.5)             # (the trace shares the module's parameter)
+    for run, scale in ((traced, 1.0), (torch.jit.load(str(tmp_path / "net.pt")), -2.0)):
+        a, b = other.clone().requires_grad_(True), other.clone().requires_grad_(True)
+        y = run(a)
+        z = torch.relu(fnn.sparse_conv(b, net.conv.weight.detach() * scale, kmap))
+        G.assert_close(y.detach().cpu().numpy(), z.detach().cpu().numpy(), "fp32")
+        G.assert_close(torch.autograd.grad(y, a, g)[0].cpu().numpy(), torch.autograd.grad(z, b, g)[0].cpu().numpy(), "fp32")
