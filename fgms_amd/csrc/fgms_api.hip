@@ -42,10 +42,16 @@ struct WsKey {
 struct WsBuf {
   void *ptr = nullptr;
   size_t bytes = 0;
+  bool captured = false;      // a call under stream capture was given it: a graph points at it
 };
 std::mutex g_ws_mutex;
 std::map<WsKey, WsBuf> g_ws;
 }  // namespace
+
+bool is_capturing(hipStream_t stream) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return stream && hipStreamIsCapturing(stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+}
 
 size_t workspace_bytes(hipStream_t stream, int slot) {
   int dev = 0;
@@ -65,31 +71,27 @@ int workspace_get(hipStream_t stream, int slot, size_t bytes, void **ptr, bool *
   FGMS_HIP_TRY(hipGetDevice(&dev));
   std::lock_guard<std::mutex> lock(g_ws_mutex);
   WsBuf &b = g_ws[WsKey{dev, stream, slot}];
+  const bool capturing = is_capturing(stream);
   if (b.bytes < bytes) {
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (stream && hipStreamIsCapturing(stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone) {
-      // growing would free a buffer that recorded kernels point at, and allocate under capture
+    if (capturing) {
+      // (an allocation cannot be recorded)
       set_error("a workspace of %zu bytes is needed while the stream is being captured: run the call once "
                 "outside the capture first", bytes);
       return FGMS_E_INVALID;
     }
-    if (b.ptr) {
-      // the old buffer may still be in use by work queued on this stream
-      FGMS_HIP_TRY(hipStreamSynchronize(stream));
-      FGMS_HIP_TRY(hipFree(b.ptr));
-      b.ptr = nullptr;
-      b.bytes = 0;
-    }
-    size_t want = bytes + bytes / 4 + 4096;
-    note_allocation();
-    if (hipMalloc(&b.ptr, want) != hipSuccess) {
-      b.ptr = nullptr;
-      set_error("workspace allocation of %zu bytes failed", want);
-      return FGMS_E_NOMEM;
-    }
-    b.bytes = want;
+    const size_t want = bytes + bytes / 4 + 4096;
+    void *p = nullptr;
+    const int rc = pool_alloc(&p, want, stream);
+    if (rc != FGMS_OK) return rc;
+    // The old buffer goes back to the pool, to be handed out again behind the work queued on this stream;
+    // one that a capture was given is kept for good: a replay of the graph may come at any time, and nothing
+    // says when the graph is gone.  (Buffers grow by a quarter and more, so all that is kept of one is less
+    // than four times its latest size.)
+    if (b.ptr && !b.captured) pool_free(b.ptr, stream, false);
+    b = WsBuf{p, want, false};
     if (fresh) *fresh = true;
   }
+  b.captured |= capturing;
   *ptr = b.ptr;
   return FGMS_OK;
 }
@@ -161,8 +163,7 @@ int relaid_weights_buffer(const GmsArgs &a, unsigned layout, size_t bytes, void 
   if (g_pinned_count.load(std::memory_order_relaxed) > 0) {
     int dev = 0;
     FGMS_HIP_TRY(hipGetDevice(&dev));
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    const bool capturing = a.stream && hipStreamIsCapturing(a.stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+    const bool capturing = is_capturing(a.stream);
     std::lock_guard<std::mutex> lock(g_pin_mutex);
     if (!capturing && is_pinned_locked(dev, a.w)) {
       for (RelaidCopy &c : g_relaid) {
@@ -513,8 +514,7 @@ constexpr int kSlotPadIn = 4, kSlotPadOut = 5, kSlotPadWeights = 6, kSlotPadResu
 // May the call grow the stream's workspaces?  (Not under stream capture: the shape-agnostic
 // kernels, which need none, then serve it unless an earlier call has left them big enough.)
 bool workspaces_fit(hipStream_t s, std::initializer_list<std::pair<int, size_t>> wanted) {
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (!s || hipStreamIsCapturing(s, &st) != hipSuccess || st == hipStreamCaptureStatusNone) return true;
+  if (!is_capturing(s)) return true;
   for (const auto &w : wanted)
     if (workspace_bytes(s, w.first) < w.second) return false;
   return true;

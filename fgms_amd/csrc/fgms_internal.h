@@ -194,7 +194,9 @@ struct Plan {
   bool dgrad_ok;      // no offset maps two pairs from one input row
 };
 
-// Fp32 scratch that outlives a call (per device and stream, grown on demand).
+bool is_capturing(hipStream_t stream);   // into a HIP graph
+
+// Scratch that outlives a call (per device and stream, grown on demand; a block of the pool below).
 // slot 0: packed weights, slot 1: fp32 weight-gradient accumulator of the MFMA kernels (kept
 // all-zero between calls), slot 2: the generic kernel's accumulator, slot 3: the gather probe's sink,
 // slots 4 .. 7: padded copies of input rows, output rows, weights and a result (fgms_pad.hip).
