@@ -35,6 +35,7 @@
 
 #include <cstdlib>
 #include <list>
+#include <memory>
 #include <mutex>
 #include <stdexcept>
 #include <utility>
@@ -45,12 +46,17 @@
 
 namespace {
 
+// A call holds the plan it was given until its launches are queued: another thread's call may drop the
+// entry from the cache meanwhile (autograd's threads run without the GIL).
+using PlanRef = std::shared_ptr<fgms_plan_t>;
+PlanRef own(fgms_plan_t *plan) { return PlanRef(plan, fgms_plan_destroy); }
+
 struct CacheEntry {
   at::Tensor kpos, in_map, out_map;       // keeps the storage alive
   int64_t v_kpos, v_in, v_out;            // version counters at build time
   int64_t n_in, n_out;
   int device;
-  fgms_plan_t *plan;
+  PlanRef plan;
   bool view;                              // a transposed view of another entry's plan
 };
 
@@ -69,9 +75,6 @@ bool g_cache_enabled = true;
 // g_mutex (calls come from python with the GIL and from autograd's threads without).
 struct Dropped {
   std::list<CacheEntry> entries;
-  ~Dropped() {
-    for (CacheEntry &e : entries) fgms_plan_destroy(e.plan);
-  }
 };
 
 void drop(std::list<CacheEntry>::iterator it, Dropped &dropped) {
@@ -121,8 +124,8 @@ void need_contiguous_cuda(const at::Tensor &t, const char *name) {
 }
 
 // Finds or builds the plan for this map.  Returns nullptr when caching is off.
-fgms_plan_t *plan_for(const at::Tensor &kpos, const at::Tensor &in_map, const at::Tensor &out_map,
-                      int64_t n_in, int64_t n_out, int k_vol, hipStream_t stream) {
+PlanRef plan_for(const at::Tensor &kpos, const at::Tensor &in_map, const at::Tensor &out_map,
+                 int64_t n_in, int64_t n_out, int k_vol, hipStream_t stream) {
   Dropped dropped;
   std::lock_guard<std::mutex> lock(g_mutex);
   if (!g_cache_enabled) return nullptr;
@@ -136,7 +139,7 @@ fgms_plan_t *plan_for(const at::Tensor &kpos, const at::Tensor &in_map, const at
         // pre-allocated tensor, this library's own included).  Every hit queues a check of the
         // lists against the fingerprint the plan was built with; what it finds reaches the host
         // a call later: that call drops the plan and raises.
-        const int rc = fgms_plan_check(it->plan, stream, 1);      // (rides along with this call's launch)
+        const int rc = fgms_plan_check(it->plan.get(), stream, 1);      // (rides along with this call's launch)
         if (rc == FGMS_E_STALE) {
           drop(it, dropped);
           throw std::runtime_error(
@@ -158,22 +161,23 @@ fgms_plan_t *plan_for(const at::Tensor &kpos, const at::Tensor &in_map, const at
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone) return nullptr;
   }
-  fgms_plan_t *plan = nullptr;
+  fgms_plan_t *made = nullptr;
   bool view = false;
   // the same pairs with the sides exchanged: share that plan's tables
   for (auto it = g_cache.begin(); it != g_cache.end(); ++it) {
     if (!it->view && it->in_map.is_same(out_map) && it->out_map.is_same(in_map) && it->kpos.is_same(kpos) &&
         it->n_in == n_out && it->n_out == n_in && it->device == dev && it->v_in == version_of(out_map) &&
         it->v_out == version_of(in_map) && it->v_kpos == version_of(kpos)) {
-      check(fgms_plan_transposed(&plan, it->plan));
+      check(fgms_plan_transposed(&made, it->plan.get()));
       view = true;
       ++g_views_made;
       break;
     }
   }
-  if (!plan)
-    check(fgms_plan_create(&plan, i32(kpos), i32(in_map), i32(out_map), n_in, n_out, k_vol,
+  if (!made)
+    check(fgms_plan_create(&made, i32(kpos), i32(in_map), i32(out_map), n_in, n_out, k_vol,
                            in_map.numel(), stream));
+  PlanRef plan = own(made);
   g_cache.push_front(CacheEntry{kpos, in_map, out_map, version_of(kpos), version_of(in_map),
                                 version_of(out_map), n_in, n_out, dev, plan, view});
   while (g_cache.size() > g_cache_cap) drop(std::prev(g_cache.end()), dropped);
@@ -250,12 +254,12 @@ void ConvolutionForwardFused(const at::Tensor in_feats, const at::Tensor kernel,
   hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
   const int k_vol = (int)kernel.size(0);
   refresh_pin(kernel);
-  fgms_plan_t *plan = plan_for(kpos, in_map, out_map, in_feats.size(0), out_feats.size(0), k_vol, stream);
+  const PlanRef plan = plan_for(kpos, in_map, out_map, in_feats.size(0), out_feats.size(0), k_vol, stream);
   check(fgms_fusion_fwd(in_feats.data_ptr(), kernel.data_ptr(), sum_nnz, out_feats.data_ptr(),
                         i32(kpos), qkpos.defined() && qkpos.numel() ? i32(qkpos) : nullptr,
                         i32(in_map), i32(out_map), separate_mid, arch80, in_feats.size(0),
                         out_feats.size(0), (int)kernel.size(1), (int)kernel.size(2), k_vol,
-                        in_map.numel(), dtype_of(in_feats), plan, stream));
+                        in_map.numel(), dtype_of(in_feats), plan.get(), stream));
 }
 
 void ConvolutionForward(const at::Tensor in_feats, const at::Tensor kernel, const int sum_nnz,
@@ -275,11 +279,11 @@ void ConvolutionForward(const at::Tensor in_feats, const at::Tensor kernel, cons
   c10::hip::HIPGuardMasqueradingAsCUDA guard(in_feats.device());
   hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
   refresh_pin(kernel);
-  fgms_plan_t *plan = plan_for(kernel_pos, in_map, out_map, in_feats.size(0), out_feats.size(0), k_vol, stream);
+  const PlanRef plan = plan_for(kernel_pos, in_map, out_map, in_feats.size(0), out_feats.size(0), k_vol, stream);
   check(fgms_fwd(in_feats.data_ptr(), kernel.data_ptr(), sum_nnz, out_feats.data_ptr(),
                  knnz.data_ptr<int>(), i32(kernel_pos), i32(in_map), i32(out_map), separate_mid,
                  arch80, in_feats.size(0), out_feats.size(0), (int)kernel.size(1),
-                 (int)kernel.size(2), k_vol, in_map.numel(), dtype_of(in_feats), plan, stream));
+                 (int)kernel.size(2), k_vol, in_map.numel(), dtype_of(in_feats), plan.get(), stream));
 }
 
 void ConvolutionBackward(const at::Tensor out_feats_grad, const at::Tensor in_feats,
@@ -297,13 +301,13 @@ void ConvolutionBackward(const at::Tensor out_feats_grad, const at::Tensor in_fe
   c10::hip::HIPGuardMasqueradingAsCUDA guard(in_feats.device());
   hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
   const int k_vol = (int)kernel.size(0);
-  fgms_plan_t *plan = plan_for(kpos, in_map, out_map, in_feats.size(0), out_feats_grad.size(0), k_vol, stream);
+  const PlanRef plan = plan_for(kpos, in_map, out_map, in_feats.size(0), out_feats_grad.size(0), k_vol, stream);
   check(fgms_bwd(out_feats_grad.data_ptr(), in_feats.data_ptr(), kernel.data_ptr(), sum_nnz,
                  in_feats_grad.data_ptr(), kernel_grad.data_ptr(), i32(kpos),
                  qkpos.defined() && qkpos.numel() ? i32(qkpos) : nullptr, i32(in_map),
                  i32(out_map), separate_mid, arch80, in_feats.size(0), out_feats_grad.size(0),
                  (int)kernel.size(1), (int)kernel.size(2), k_vol, in_map.numel(),
-                 dtype_of(in_feats), plan, stream));
+                 dtype_of(in_feats), plan.get(), stream));
 }
 
 namespace {
@@ -328,10 +332,10 @@ at::Tensor layer_forward(const at::Tensor &feats, const at::Tensor &weight, cons
   hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
   at::Tensor out = at::empty({map.n_out, weight.size(2)}, feats.options().requires_grad(false));
   refresh_pin(weight);
-  fgms_plan_t *plan = plan_for(map.kpos, map.in_map, map.out_map, map.n_in, map.n_out, k_vol, stream);
+  const PlanRef plan = plan_for(map.kpos, map.in_map, map.out_map, map.n_in, map.n_out, k_vol, stream);
   check(fgms_conv_fwd(feats.data_ptr(), weight.data_ptr(), out.data_ptr(), i32(map.kpos), i32(map.in_map), i32(map.out_map),
                       tf32, map.n_in, map.n_out, (int)weight.size(1), (int)weight.size(2), k_vol, map.in_map.numel(),
-                      dtype_of(feats), plan, stream));
+                      dtype_of(feats), plan.get(), stream));
   return out;
 }
 
@@ -368,10 +372,10 @@ struct SparseConvBackward final : public torch::autograd::Node {
     at::Tensor gx, gw;
     if (task_should_compute_output(0)) gx = at::empty(x.sizes(), x.options().requires_grad(false));
     if (task_should_compute_output(1)) gw = at::empty(w.sizes(), w.options().requires_grad(false));
-    fgms_plan_t *plan = plan_for(map.kpos, map.in_map, map.out_map, map.n_in, map.n_out, k_vol, stream);
+    const PlanRef plan = plan_for(map.kpos, map.in_map, map.out_map, map.n_in, map.n_out, k_vol, stream);
     check(fgms_conv_bwd(g.data_ptr(), x.data_ptr(), w.data_ptr(), gx.defined() ? gx.data_ptr() : nullptr,
                         gw.defined() ? gw.data_ptr() : nullptr, i32(map.kpos), i32(map.in_map), i32(map.out_map), tf32,
-                        map.n_in, map.n_out, (int)w.size(1), (int)w.size(2), k_vol, map.in_map.numel(), dtype_of(x), plan,
+                        map.n_in, map.n_out, (int)w.size(1), (int)w.size(2), k_vol, map.in_map.numel(), dtype_of(x), plan.get(),
                         stream));
     return {gx, gw};
   }
@@ -504,7 +508,7 @@ struct MapOnItsWay {
       Dropped dropped;
       std::lock_guard<std::mutex> lock(g_mutex);
       g_cache.push_front(CacheEntry{kpos, im, om, version_of(kpos), version_of(im), version_of(om), n_in, n_out,
-                                    (int)in_coords.get_device(), plan, false});
+                                    (int)in_coords.get_device(), own(plan), false});
       while (g_cache.size() > (g_cache_enabled ? g_cache_cap : 0)) drop(std::prev(g_cache.end()), dropped);
     }
     return {im, om, nnz, kpos, qkpos, qsum};

@@ -189,3 +189,36 @@ def test_traced_layer_is_recorded(one_layer, tmp_path):
         z = torch.relu(fnn.sparse_conv(b, net.conv.weight.detach() * scale, kmap))
         G.assert_close(y.detach().cpu().numpy(), z.detach().cpu().numpy(), "fp32")
         G.assert_close(torch.autograd.grad(y, a, g)[0].cpu().numpy(), torch.autograd.grad(z, b, g)[0].cpu().numpy(), "fp32")
+
+
+def test_threads_drop_each_others_plans():
+    """Forward and backward passes of several threads over more maps than the plan cache holds."""
+    import threading
+    from FGMS import backend, nn as fnn
+    backend.fgms_plan_cache(True, 1)
+    failures = []
+
+    def work(seed):
+        try:
+            L = small_layer(seed, 32, 32, np.float16)
+            with torch.cuda.stream(torch.cuda.Stream()):
+                D = G.to_dev(L)
+                kmap = fnn.KernelMap(D["imap"], D["omap"], L["knnz"], L["n_in"], L["n_out"])
+                x, w = D["in_feats"].clone().requires_grad_(True), D["kernel"].clone().requires_grad_(True)
+                passes = [torch.autograd.grad(fnn.sparse_conv(x, w, kmap), (x, w), D["out_grad"]) for _ in range(25)]
+                torch.cuda.current_stream().synchronize()
+            for got in passes:
+                for a, b in zip(got, passes[0]):
+                    G.assert_close(a.cpu().numpy(), b.cpu().numpy(), "fp16")
+        except Exception as e:          # noqa: BLE001 (reported by the main thread)
+            failures.append(e)
+
+    try:
+        threads = [threading.Thread(target=work, args=(60 + i,)) for i in range(4)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    finally:
+        backend.fgms_plan_cache(True, 8)
+    assert not failures, failures[0]
