@@ -58,6 +58,7 @@ struct CacheEntry {
   int device;
   PlanRef plan;
   bool view;                              // a transposed view of another entry's plan
+  bool captured = false;                  // a call under stream capture used it
 };
 
 // Inference tensors track no version.
@@ -70,6 +71,16 @@ std::list<CacheEntry> g_cache;            // most recently used first
 size_t g_cache_cap = 8;
 bool g_cache_enabled = true;
 
+// Kernels recorded into a HIP graph point at a plan's tables and at the lists they were made from, and
+// nothing says when the graph is gone: an entry that a capture used does not count towards the cache's
+// capacity, and once it has to leave (its map was rewritten, the cache cleared) it is kept here for good.
+std::list<CacheEntry> g_captured;
+
+bool is_capturing(hipStream_t stream) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return stream && hipStreamIsCapturing(stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+}
+
 // Entries leave the cache by way of a list that its owner destroys after g_mutex is released: the
 // last reference to a tensor may need the GIL, which another thread can hold while it waits for
 // g_mutex (calls come from python with the GIL and from autograd's threads without).
@@ -78,13 +89,23 @@ struct Dropped {
 };
 
 void drop(std::list<CacheEntry>::iterator it, Dropped &dropped) {
-  dropped.entries.splice(dropped.entries.begin(), g_cache, it);
+  std::list<CacheEntry> &to = it->captured ? g_captured : dropped.entries;
+  to.splice(to.begin(), g_cache, it);
+}
+
+// Leaves the `capacity` entries used last, and those of captures.
+void shrink_cache(size_t capacity, Dropped &dropped) {
+  size_t seen = 0;
+  for (auto it = g_cache.begin(); it != g_cache.end();) {
+    const auto entry = it++;
+    if (!entry->captured && ++seen > capacity) drop(entry, dropped);
+  }
 }
 
 void clear_cache() {
   Dropped dropped;
   std::lock_guard<std::mutex> lock(g_mutex);
-  dropped.entries.splice(dropped.entries.begin(), g_cache);
+  while (!g_cache.empty()) drop(g_cache.begin(), dropped);
 }
 
 void set_cache(bool enabled, int64_t capacity) {
@@ -148,6 +169,7 @@ PlanRef plan_for(const at::Tensor &kpos, const at::Tensor &in_map, const at::Ten
               "map used the old neighbour tables.  Call fgms_plan_cache_clear() after rewriting a map.");
         }
         check(rc);
+        if (is_capturing(stream)) it->captured = true;
         g_cache.splice(g_cache.begin(), g_cache, it);
         return g_cache.front().plan;
       }
@@ -157,10 +179,7 @@ PlanRef plan_for(const at::Tensor &kpos, const at::Tensor &in_map, const at::Ten
   }
   // a map first seen while the stream is being captured into a graph: no plan is built (the build
   // allocates, and its kernels would be recorded); the call records the kernels that need none
-  {
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone) return nullptr;
-  }
+  if (is_capturing(stream)) return nullptr;
   fgms_plan_t *made = nullptr;
   bool view = false;
   // the same pairs with the sides exchanged: share that plan's tables
@@ -180,7 +199,7 @@ PlanRef plan_for(const at::Tensor &kpos, const at::Tensor &in_map, const at::Ten
   PlanRef plan = own(made);
   g_cache.push_front(CacheEntry{kpos, in_map, out_map, version_of(kpos), version_of(in_map),
                                 version_of(out_map), n_in, n_out, dev, plan, view});
-  while (g_cache.size() > g_cache_cap) drop(std::prev(g_cache.end()), dropped);
+  shrink_cache(g_cache_cap, dropped);
   return plan;
 }
 
@@ -509,7 +528,7 @@ struct MapOnItsWay {
       std::lock_guard<std::mutex> lock(g_mutex);
       g_cache.push_front(CacheEntry{kpos, im, om, version_of(kpos), version_of(im), version_of(om), n_in, n_out,
                                     (int)in_coords.get_device(), own(plan), false});
-      while (g_cache.size() > (g_cache_enabled ? g_cache_cap : 0)) drop(std::prev(g_cache.end()), dropped);
+      shrink_cache(g_cache_enabled ? g_cache_cap : 0, dropped);
     }
     return {im, om, nnz, kpos, qkpos, qsum};
   }

@@ -1,5 +1,5 @@
-"""A captured graph keeps the workspaces it points at: later eager calls that need bigger ones get new
-buffers, and replays still give the eager results."""
+"""A captured graph keeps what it points at: later eager calls that need bigger workspaces get new
+buffers, the plan cache does not give its plans back, and replays still give the eager results."""
 import numpy as np
 import pytest
 import torch
@@ -76,3 +76,38 @@ def test_replays_after_bigger_calls(shape, dtype, policy):
         capi.set_kernel_policy(0)
         for layer in layers:
             layer[3].close()
+
+
+def test_replays_after_the_plan_cache_moved_on():
+    """A layer recorded through FGMS.nn, then more maps than the cache holds, then an emptied cache."""
+    from FGMS import backend, nn as fnn
+    backend.fgms_plan_cache(True, 2)
+    layers = []
+    for n in (2500, 2600, 2700, 2800, 2900):
+        L = cloud_layer(n, 64, 64, np.float16)
+        D = G.to_dev(L)
+        layers.append((D["in_feats"], D["kernel"], fnn.KernelMap(D["imap"], D["omap"], L["knnz"], L["n_in"], L["n_out"])))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    x, w, kmap = layers[0]
+    try:
+        with torch.cuda.stream(side):
+            want = fnn.sparse_conv(x, w, kmap)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            out = fnn.sparse_conv(x, w, kmap)
+        for step in range(3):
+            for other in layers[1:]:
+                fnn.sparse_conv(*other)
+            assert backend.fgms_plan_cache_size() == (3 if step == 0 else 2)   # (the captured map's, and two)
+            backend.fgms_plan_cache_clear()
+            for other in layers[1:]:                    # (builds that would take the blocks given back)
+                fnn.sparse_conv(*other)
+            torch.cuda.synchronize()
+            out.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            G.assert_close(out.cpu().numpy(), want.cpu().numpy(), "fp16", "replay")
+    finally:
+        backend.fgms_plan_cache(True, 8)
