@@ -541,7 +541,7 @@ __device__ __forceinline__ void tile_order_body(const TileSide &sd, int cus_per_
 // mask pass over the lists or the map builder left them), or -- plans over more than 64 offsets -- the
 // workgroup finds them by bisection and the one with shift 0 writes them down.
 __device__ __forceinline__ void bands_body(const TablesArgs &a, int x, int shift, int32_t *__restrict__ lds) {
-  const int k_vol = a.k_vol, bands = a.bands ? a.bands : band_count_of(a.kpos[a.k_vol], a.k_vol, a.cus_per_xcd * 8);
+  const int k_vol = a.k_vol, bands = a.bands ? a.bands : band_count_of(a.kpos[a.k_vol], a.k_vol, a.cus);
   const int per_xcd = (bands / 8) * k_vol;
   int *count = lds;                       // [per_xcd]
   int *group = lds + per_xcd;             // [per_xcd]
@@ -603,7 +603,7 @@ __global__ __launch_bounds__(256) void tables_kernel(TablesArgs a) {
       const int v = a.flags[a.mirror && (q == 5 || q == 11) ? q - 1 : q];
       if (a.host && (q < kFlagPrint)) a.host[q] = v;
     }
-    if (b < 2) tile_order_body(a.tile[b], a.cus_per_xcd, lds);
+    if (b < 2) tile_order_body(a.tile[b], a.cus >= 8 ? a.cus / 8 : 1, lds);
     return;
   }
   b -= a.tile_blocks;
@@ -757,7 +757,7 @@ int launch_tables(TablesArgs a, hipStream_t s) {
   a.row_blocks = a.rows ? (a.n_out + 63) / 64 : 0;
   if (a.rows && (size_t)64 * (a.row_ld + 1) * sizeof(int32_t) > lds) lds = (size_t)64 * (a.row_ld + 1) * sizeof(int32_t);
   a.pair_blocks = !a.rows && (a.inv_out || a.inv_in) ? (a.n_pairs + 255) / 256 : 0;
-  a.cus_per_xcd = num_cus() >= 8 ? num_cus() / 8 : 1;
+  a.cus = num_cus();
   if (lds > 48 * 1024) {
     const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(tables_kernel), lds);
     if (rc != FGMS_OK) return rc;

@@ -155,10 +155,10 @@ struct TablesArgs {
   int row_ld;
   // bands
   int32_t *band_start, *band_cells;
-  int bands, band_rows;              // (bands == 0: as many as the pairs in kpos ask for)
+  int bands, band_rows;              // (bands == 0: as many as the pairs in kpos ask for, on `cus` compute units)
   bool bands_known;                  // band_start is filled in already
   TileSide tile[2];
-  int cus_per_xcd;
+  int cus;
   int *flags, *host;                 // findings and where they go on the host (nullptr: a copy follows)
   bool mirror, take_print;           // one side's counts stand for both; fingerprint of the lists
   // workgroups of each part, in this order
