@@ -538,13 +538,58 @@ GmsArgs with_channels(GmsArgs a, int c_in, int c_out) {
   return a;
 }
 
-bool tuned_gms(const GmsArgs &a, const Plan *plan) {
+// Route of a pass over all offsets (of its first group, for plans over more than 64).
+Route first_route(const GmsArgs &a, const Plan *plan) {
   if (plan && !plan->groups.empty() && a.dense_k < 0) {
     GmsArgs g = a;
     g.k_vol = plan->groups.front()->k_vol;
-    return route_of(g, plan->groups.front()) != Route::kGeneric;
+    return route_of(g, plan->groups.front());
   }
-  return route_of(a, plan) != Route::kGeneric;
+  return route_of(a, plan);
+}
+bool tuned_gms(const GmsArgs &a, const Plan *plan) { return first_route(a, plan) != Route::kGeneric; }
+
+// fp32 passes: padded copies, or the vector ALUs' kernel on the channels as they are.  The copies are two
+// more launches in front (three where the weights are re-laid) and one behind, and on small clouds a tile's
+// chain of fp32 products is all there is to the main launch, where the shape-agnostic kernel spreads single
+// 32-pair pieces over the chip.  The functions below estimate either side in microseconds, fitted to 22 channel
+// counts from 3 x 32 to 96 x 100 and 48 x 200 over 500 .. 60 k voxels, dense, LiDAR and thinned clouds, with and without a
+// plan (4 500 pairs of times; half of the estimates are within 8 % and nine in ten within 20 %).  Forward,
+// copies / vector ALUs: 32 -> 20 over 2 k dense voxels 32 / 16 us, 10 k 32 / 25, 14 k 32 / 31, 40 k 42 / 72;
+// 48 -> 48 over 2 k 49 / 18, 20 k 76 / 64, 40 k 98 / 120; over 20 k thinned ones (pair view, atomics) 44 / 30.
+double pairs_of(const GmsArgs &a, const Plan *plan) {
+  return (double)(a.dense_k >= 0 ? a.n_dense : plan && plan->pairs_counted > 0 ? plan->pairs_counted : a.n_pairs);
+}
+int group_count(const GmsArgs &a, const Plan *plan) {
+  return plan && !plan->groups.empty() && a.dense_k < 0 ? (int)plan->groups.size() : 1;
+}
+// Products (pieces of 32 source and 64 destination channels), atomics, gathered channels.
+double vector_alu_us(const GmsArgs &a, const Plan *plan) {
+  const int c_src = a.transpose_w ? a.c_out : a.c_in, c_dst = a.transpose_w ? a.c_in : a.c_out;
+  const double base = (a.overwrite ? 13 : 11) * group_count(a, plan);       // (fill and) launch
+  return base + 1e-6 * pairs_of(a, plan) * (0.043 * up_to_32(c_src) * ((c_dst + 63) / 64 * 64) + 1.4 * c_dst + c_src);
+}
+// `p`: the pass over the copies.  What a small launch takes is its launches and a tile's chain of (offset,
+// 32-channel slab) stages, more of it once there is more than a tile to a CU; the routes with atomics add what these cost.
+double padded_us(const GmsArgs &p, const Plan *plan) {
+  const int c_src = p.transpose_w ? p.c_out : p.c_in, c_dst = p.transpose_w ? p.c_in : p.c_out;
+  const double slabs = (c_src + 31) / 32, wide = c_dst % 64 == 0 ? 1 : 0;
+  switch (first_route(p, plan)) {
+    case Route::kSkinny: return 17 * group_count(p, plan) + (p.transpose_w ? 1.5 : c_src * c_dst / 45.0);
+    case Route::kRows: {
+      const bool split = p.reduced && split_bf16_enabled();
+      const double tiles_per_cu = (double)((p.n_dst + 127) / 128 * (c_dst / 32)) / num_cus(), stages = p.k_vol * slabs;
+      if (p.transpose_w) return 15 + 3 * wide + (split ? 0.42 : 0.5) * stages * (1 + 1.45 * std::max(0.0, tiles_per_cu - 0.43));
+      return 14 + (split ? 0.41 : 0.65) * stages * (tiles_per_cu <= 1 ? 1 : 1.25 + 0.25 * tiles_per_cu);
+    }
+    default:
+      return 20 + 1.5 * slabs * (1 + wide) + 1e-6 * pairs_of(p, plan) * (p.dense_k >= 0 ? 2.0 * c_dst : 3.4 * c_dst + 0.4 * c_src);
+  }
+}
+bool padding_pays(const GmsArgs &a, const Plan *plan, int c_in, int c_out) {
+  // (fp16 adds on the vector ALUs cost ten times as much: 32 -> 20 over 500 voxels 17 us over copies, 24 without.
+  // The copies' fp32 kernels mostly do without atomics: a near tie goes to them.)
+  return a.dtype == FGMS_F16 || padded_us(with_channels(a, c_in, c_out), plan) < 1.05 * vector_alu_us(a, plan);
 }
 
 // Widened channels of a forward / input-gradient pass that no tuned kernel takes as it is: the
@@ -555,10 +600,11 @@ bool padded_gms_channels(const GmsArgs &a, const Plan *plan, int *c_in, int *c_o
   const int si = up_to_power_of_two(a.c_in, 4), so = up_to_power_of_two(a.c_out, 4);
   if (si * so <= 256 && tuned_gms(with_channels(a, si, so), plan)) {
     *c_in = si; *c_out = so;
-    return true;
+  } else {
+    *c_in = up_to_32(a.c_in); *c_out = up_to_32(a.c_out);
+    if (!tuned_gms(with_channels(a, *c_in, *c_out), plan)) return false;
   }
-  *c_in = up_to_32(a.c_in); *c_out = up_to_32(a.c_out);
-  return tuned_gms(with_channels(a, *c_in, *c_out), plan);
+  return padding_pays(a, plan, *c_in, *c_out);
 }
 
 // fp16 layers whose channels fill no whole tile go straight to kernels that mask the rest, where the map
@@ -668,7 +714,7 @@ bool padded_wgrad_channels(const WgradArgs &a, int *c_in, int *c_out) {
     p.c_out = up_to_32(a.c_out);
   }
   *c_in = p.c_in; *c_out = p.c_out;
-  return mfma_wgrad_supported(p);
+  return mfma_wgrad_supported(p) && (a.dtype == FGMS_F16 || padded_wgrad_us(p) < vector_alu_wgrad_us(a));
 }
 
 // The weight gradient over padded copies of the rows (as above); its fp32 sums are cropped when
@@ -746,6 +792,15 @@ int run_bwd(GmsArgs d, const Plan *p, WgradArgs w) {
   return run_wgrad(w);
 }
 
+// fp32: both gradients over shared copies in one grid (`pd`, `pw`), or each on its better side in a call of its own?
+// The grid overlaps the shorter of the two with the longer.  (48 -> 48 over 2 k voxels: 55 us together, 19 and 20
+// apart; 20 -> 128 over 10 k: 69 together, 69 and 50 apart.)
+bool together_pays(const GmsArgs &d, const Plan *p, const WgradArgs &w, const GmsArgs &pd, const WgradArgs &pw) {
+  const double in_us = padded_us(pd, p), w_us = padded_wgrad_us(pw);
+  const double in_alone = tuned_gms(d, p) ? padded_us(d, p) : std::min(in_us, vector_alu_us(d, p));
+  return std::max(in_us, w_us) + 0.4 * std::min(in_us, w_us) < 1.1 * (in_alone + std::min(w_us, vector_alu_wgrad_us(w)));
+}
+
 // Widened channels for a backward pass one of whose gradients no tuned kernel takes as it is: the
 // narrow layers' kernels up to 16 x 64, else multiples of 32 for both, which the one-grid launch takes.
 bool padded_bwd_channels(const GmsArgs &d, const Plan *p, const WgradArgs &w, int *c_in, int *c_out) {
@@ -757,7 +812,8 @@ bool padded_bwd_channels(const GmsArgs &d, const Plan *p, const WgradArgs &w, in
     pw.in = pw.gout = (const void *)4096;
     pw.c_in = *c_in;
     pw.c_out = *c_out;
-    if (tuned_gms(with_channels(d, *c_in, *c_out), p) && mfma_wgrad_supported(pw)) return true;
+    if (!tuned_gms(with_channels(d, *c_in, *c_out), p) || !mfma_wgrad_supported(pw)) continue;
+    return d.dtype == FGMS_F16 || together_pays(d, p, w, with_channels(d, *c_in, *c_out), pw);
   }
   return false;
 }

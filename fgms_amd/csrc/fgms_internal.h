@@ -266,6 +266,9 @@ bool wide_gms_supported(const GmsArgs &a);
 int launch_wide_gms(const GmsArgs &a);
 bool mfma_wgrad_supported(const WgradArgs &a);
 int launch_mfma_wgrad(const WgradArgs &a);
+// fp32 estimates in microseconds: the weight gradient over padded copies (the call over them), and on the vector ALUs.
+double padded_wgrad_us(const WgradArgs &p);
+double vector_alu_wgrad_us(const WgradArgs &a);
 // The MFMA / skinny weight gradient with its fp32 accumulator in a static device array: no
 // allocation of any kind.
 int wgrad_static(WgradArgs a);

@@ -408,6 +408,32 @@ bool mfma_wgrad_supported(const WgradArgs &a) {
   return true;
 }
 
+// One cell's walk waits for the rows it meets -- 3.3 times the cloud's rows to a cell, or its pairs where these
+// are fewer, by what a row of the tile costs -- and the chip multiplies 40 pairs x 32 x 32 channels a nanosecond.  On dense maps the copies always pay, twice over; on thin ones there are too few pairs to cut more
+// cells, where the vector ALUs take pieces of 512 pairs x 32 x 32 channels.  Thinned clouds, fp32, copies / vector ALUs:
+// 48 x 48 over 10 k voxels 39 / 42 us, 20 k 67 / 68, 40 k 122 / 88; 128 x 20 over 5 k 30 / 39, 40 k 171 / 90;
+// 32 x 20 over 40 k 49 / 60 (tf32 mode 69 / 61).
+double padded_wgrad_us(const WgradArgs &p) {
+  double per_row = 0, cells = 1;
+  WgradGeometry g;
+  if (skinny_shape(p)) {
+    per_row = 0.076 / 512 * p.c_in * p.c_out;
+    cells = (double)choose_slices(p, 1, 64, (int64_t)num_cus() * 2).slices * p.k_vol;
+  } else if (wgrad_geometry(p, &g) == FGMS_OK) {
+    const int blocks = g.bi * g.bj;
+    per_row = blocks == 1 ? (g.split ? 0.083 : 0.05) : blocks == 2 ? (g.split ? 0.122 : 0.095)
+              : g.bi == 2 && g.bj == 2 ? (g.split ? 0.147 : 0.172) : 0.06 * blocks;
+    cells = (double)g.tiles;
+  }
+  const double rows = 3.3 * (double)(p.n_in > p.n_out ? p.n_in : p.n_out), pairs = (double)p.n_pairs;
+  const double us = 14 + per_row * (rows < pairs ? rows : pairs) / cells + 25e-6 * pairs * ((p.c_in + 31) / 32) * ((p.c_out + 31) / 32);
+  return us < 19 ? 19 : us;
+}
+double vector_alu_wgrad_us(const WgradArgs &a) {
+  const double tiles = (double)((a.c_in + 31) / 32) * ((a.c_out + 31) / 32), us = 35 + 1e-5 * (double)a.n_pairs * (4 + 9.6 * tiles);
+  return us < 39 ? 39 : us;
+}
+
 // Grid and LDS of the per-wave body for g's tile.
 static void wave_geometry(const WgradArgs &a, WgradGeometry *g) {
   const bool f16 = a.dtype == FGMS_F16;
