@@ -76,7 +76,8 @@ const char *fgms_last_error(void);
  * given a plan whose map has an out-of-range index returns FGMS_E_INVALID.  Exception:
  * a first use recorded into a HIP graph (stream capture) cannot wait and records the
  * kernels that need no plan.  The map arrays must stay valid and unchanged while the plan
- * lives.  Not to be called on a stream that is being captured.
+ * lives, and the plan while a HIP graph that recorded a call with it may be replayed.  Not to be
+ * called on a stream that is being captured.
  */
 int fgms_plan_create(fgms_plan_t **plan, const int32_t *kpos,
                      const int32_t *in_map, const int32_t *out_map,
