@@ -58,6 +58,8 @@ constexpr int kBlockX = 1, kBlockY = 1, kBlockZ = 2;      // bits of a coordinat
 constexpr int kCells = 1 << (kBlockX + kBlockY + kBlockZ);
 constexpr int kNoRow = INT32_MAX;
 
+// (Factors: the first three 32-bit primes of xxHash, Y. Collet; finaliser: prospector32, C. Wellons, "Prospecting for
+// hash functions", 2018.)
 __device__ __forceinline__ unsigned slot_of(int bx, int by, int bz, unsigned mask) {
   unsigned h = (unsigned)bx * 0x9E3779B1u ^ (unsigned)by * 0x85EBCA77u ^ (unsigned)bz * 0xC2B2AE3Du;
   h ^= h >> 15; h *= 0x2C1B3C6Du;

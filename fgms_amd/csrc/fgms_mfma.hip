@@ -1166,10 +1166,12 @@ bool half_tiles_enabled() {
 }
 
 // Grid of an output-stationary launch over n_dst destination rows: tiles of 256 rows from the
-// plan's tile table where there is one (`table_grid` entries), else plain tiles of 256 or --
+// plan's tile table where there is one (65 k rows and more, `table_grid` entries), else plain tiles of 256 or --
 // where those still fit the chip's workgroup slots in one round -- of 128 rows (32 per wave:
 // twice the waves, half the work per wave and stage; such a launch lasts as long as one
-// tile's chain of stages).  A launch that then fills less than half of the slots shares every
+// tile's chain of stages).  A small forward launch on 128-row tiles shortens the chain with groups of waves
+// inside a workgroup (can_group, below).  Where there are no groups -- an input gradient, a forward launch on the
+// plan's table or with 128-column wave tiles -- a launch that fills less than half of the slots shares every
 // tile between two workgroups, each taking half of the tile's stages and adding its part with
 // atomics: twice the workgroups, half the critical path.  (Two parts only: the sum of two
 // partial results does not depend on their order.  On launches that fill the chip the atomics
@@ -1178,9 +1180,8 @@ bool half_tiles_enabled() {
 // tiles only where they (times two, for the shared tiles) fill at most half of the slots, since
 // in the backward launch its workgroups share the chip with the weight gradient's and more of
 // them delay those.  Measured (MI355X, 64 -> 64 fp16 over 10 k / 20 k / 50 k / 60 k voxels of the
-// indoor cloud): forward 23.5 -> 16.9, 23.3 -> 18.3, 26.5 -> 22.8, 28.5 -> 25.7 us; backward
-// launch 22.5 -> 17.0, 26.1 -> 20.9, 35.6 -> 36.0, 43.2 -> 47.8 us (128 -> 128 over 28 k voxels:
-// 53.2 -> 63.0 us), hence the rule; 32 -> 32 fp32 over 20 k voxels, whole step: 64.0 -> 56.6 us.
+// indoor cloud, without / with the small tiles): backward launch 22.5 -> 17.0, 26.1 -> 20.9, 35.6 -> 36.0,
+// 43.2 -> 47.8 us (128 -> 128 over 28 k voxels: 53.2 -> 63.0 us), hence the rule.
 struct RowsGrid {
   bool half_tiles;
   bool drop_table;      // the launch does better on plain 128-row tiles than on the plan's tile table
@@ -1511,7 +1512,10 @@ int launch_fused_bwd(const GmsArgs &d, const Plan *p, const WgradArgs &w, bool *
   if (rc != FGMS_OK) return rc;
   bool found = false;
   // (wave tile columns NT of the input gradient, MFMA steps per slab S) follow from c_in and
-  // c_out, and so do the block counts (BI, BJ) of the weight gradient's tile
+  // c_out, and so do the block counts (BI, BJ) of the weight gradient's tile.  Input channels: NT 1, BI 1 for
+  // odd numbers of 32s; 2, 2 for 64 and odd multiples; 2 or (launches that fill the chip) 4, BI 4 for multiples of 128; 3, 3
+  // for odd multiples of 96 over dense maps.  Output channels: S 2, BJ 1 for 32 and other odd numbers of 32s; 4, 2
+  // for 64 and odd multiples; 4, 4 for multiples of 128; 3, 3 for odd multiples of 96 over dense maps, 3, 1 over thin ones.
 #define FGMS_FB(TT, NTv, Sv, BIv, BJv)                                             \
   if (!found && s.NTR == NTv && s.SR == Sv && g.bi == BIv && g.bj == BJv) {          \
     found = true;                                                                    \
@@ -1558,15 +1562,19 @@ int launch_ragged_bwd(const GmsArgs &d, const Plan *p, const WgradArgs &w, bool 
   bool found = false;
   int rc = FGMS_OK;
   float *acc32 = nullptr;
+  // (column tiles NT of the input gradient, k-steps S of its slab, blocks BJ of the weight gradient's tile; BI = NT.
+  // NT: 1 up to 32 input channels, 2 up to 64 and for an even number of 32s, 3 for 72 .. 96, 136 .. 160 and the like.
+  // S, BJ by output channels: 2, 1 up to 32; 3, 2 for 40 and 48; 4, 2 for 56, 64 and an even number of 32s; 3, 3 for
+  // 72 .. 96; 4, 3 for 136 .. 160 and other odd numbers of 32s.)
 #define FGMS_FR(NTv, Sv, BJv)                                                                                     \
   if (!found && s.NTR == NTv && s.SR == Sv && g.bi == NTv && g.bj == BJv) {                                       \
     found = true;                                                                                                 \
     if ((rc = wgrad_accumulator(w, &acc32)) == FGMS_OK)                                                           \
       rc = launch_fused<__half, NTv, Sv, NTv, BJv, true>(d, s, p, w, g, acc32);                                   \
   }
-  FGMS_FR(1, 2, 1) FGMS_FR(1, 3, 2) FGMS_FR(1, 4, 2) FGMS_FR(1, 3, 3) FGMS_FR(1, 2, 3) FGMS_FR(1, 4, 3)
-  FGMS_FR(2, 2, 1) FGMS_FR(2, 3, 2) FGMS_FR(2, 4, 2) FGMS_FR(2, 3, 3) FGMS_FR(2, 2, 3) FGMS_FR(2, 4, 3)
-  FGMS_FR(3, 2, 1) FGMS_FR(3, 3, 2) FGMS_FR(3, 4, 2) FGMS_FR(3, 3, 3) FGMS_FR(3, 2, 3) FGMS_FR(3, 4, 3)
+  FGMS_FR(1, 2, 1) FGMS_FR(1, 3, 2) FGMS_FR(1, 4, 2) FGMS_FR(1, 3, 3) FGMS_FR(1, 4, 3)
+  FGMS_FR(2, 2, 1) FGMS_FR(2, 3, 2) FGMS_FR(2, 4, 2) FGMS_FR(2, 3, 3) FGMS_FR(2, 4, 3)
+  FGMS_FR(3, 2, 1) FGMS_FR(3, 3, 2) FGMS_FR(3, 4, 2) FGMS_FR(3, 3, 3) FGMS_FR(3, 4, 3)
 #undef FGMS_FR
   if (!found) return FGMS_OK;
   if (rc != FGMS_OK) return rc;
