@@ -1,6 +1,7 @@
-"""Channel counts that run over padded copies: one off the kernels' multiples on either side, one
+"""Channel counts that no tuned kernel takes: one off the kernels' multiples on either side, one
 channel, a kernel of more than 64 offsets, with and without a plan, results added to what the
-buffers hold -- against the CPU oracle."""
+buffers hold -- against the CPU oracle.  fp16 runs over padded copies (or masked), small fp32 calls on
+the vector ALUs, bigger ones over copies: the last tests stand on both sides of that rule."""
 import numpy as np
 import pytest
 import torch
@@ -98,3 +99,26 @@ def test_fp32_side_of_the_rule(oracle, shape, tf32):
         for got, want, what in zip((out, gi, gw) + both, ref + ref[1:], ("fwd", "dgrad", "wgrad", "dgrad of both", "wgrad of both")):
             G.assert_close(got.cpu().numpy(), want, mode, "%s %d" % (what, n))
         plan.close()
+
+
+@pytest.mark.parametrize("c_in", [3, 5])
+def test_wide_kernel_fp32_over_copies(oracle, c_in):
+    """125 offsets over a cloud big enough for the copies: one copy, two groups of offsets."""
+    from fgms_amd import capi
+    capi.set_kernel_policy(0)
+    rng = np.random.default_rng(6)
+    vox = clouds.cloud_indoor(clouds.rng_for(2), target=20000)
+    imap, omap, knnz, kpos = clouds.build_kernel_map(vox, vox, clouds.offsets_cube(5))
+    L = clouds.make_layer(rng, imap, omap, knnz, kpos, len(vox), len(vox), c_in, 32, np.float32)
+    D = G.to_dev(L)
+    plan = capi.Plan(D["kpos"], D["imap"], D["omap"], D["n_in"], D["n_out"])
+    init = torch.randn(D["n_out"], 32, device="cuda")
+    G.run_fwd(capi, D, plan=plan)
+    capi.profile_reset()
+    capi.profile_enable(True)
+    out = G.run_fwd(capi, D, plan=plan, out_init=init)
+    capi.profile_enable(False)
+    names = [r[0] for r in capi.profile_records()]
+    capi.profile_reset()
+    assert len(names) == 2 and not any("generic" in n for n in names), names
+    G.assert_close(out - init.cpu().numpy(), oracle.c_fwd(L["in_feats"], L["kernel"], L["knnz"], L["imap"], L["omap"], L["n_out"]), "fp32", "fwd")
