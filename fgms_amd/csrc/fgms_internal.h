@@ -199,7 +199,8 @@ bool is_capturing(hipStream_t stream);   // into a HIP graph
 // Scratch that outlives a call (per device and stream, grown on demand; a block of the pool below).
 // slot 0: packed weights, slot 1: fp32 weight-gradient accumulator of the MFMA kernels (kept
 // all-zero between calls), slot 2: the generic kernel's accumulator, slot 3: the gather probe's sink,
-// slots 4 .. 7: padded copies of input rows, output rows, weights and a result (fgms_pad.hip).
+// slots 4 .. 7: padded copies of input rows, output rows, weights and a result (fgms_pad.hip), slot 8: the
+// workgroups' sums of a narrow layer's weight gradient (fgms_narrow.hip).
 // *fresh (optional) is set when the buffer was (re)allocated by this call.
 int workspace_get(hipStream_t stream, int slot, size_t bytes, void **ptr, bool *fresh = nullptr);
 // Buffer for a re-laid copy of a.w in `layout` (any number that tells the layouts of one weight
@@ -291,6 +292,11 @@ inline bool worth_96_columns(int64_t n_pairs, int64_t n_a, int64_t n_b) { return
 bool split_bf16_enabled();   // products of fp32 tensors in split bf16 where the caller allows tf32 precision
 bool small_gms_supported(const GmsArgs &a, const Plan *p);
 int launch_small_gms(const GmsArgs &a, const Plan *p);
+// Narrow input sides on the matrix cores (fgms_narrow.hip): the forward pass, and the weight gradient.
+bool narrow_gms_supported(const GmsArgs &a, const Plan *p);
+int launch_narrow_gms(const GmsArgs &a, const Plan *p);
+bool narrow_wgrad_supported(const WgradArgs &a, const Plan *p);
+int launch_narrow_wgrad(const WgradArgs &a, const Plan *p);
 bool planned_gms_supported(const GmsArgs &a, const Plan *p);
 int launch_planned_gms(const GmsArgs &a, const Plan *p);
 // The same kernel over the plan's pair view (no wasted row slots, atomic adds).

@@ -373,6 +373,11 @@ int launch_skinny(const WgradArgs &a, float *acc32) {
   return FGMS_OK;
 }
 
+// Narrow layers through the plan's tables.
+bool takes_narrow(const WgradArgs &a) {
+  return (kernel_policy() == 0 || kernel_policy() == 4) && narrow_wgrad_supported(a, a.plan);
+}
+
 template <typename T>
 int dispatch(const WgradArgs &a, float *acc32) {
   if (skinny_shape(a)) {
@@ -398,7 +403,7 @@ int dispatch(const WgradArgs &a, float *acc32) {
 
 }  // namespace
 
-bool mfma_wgrad_supported(const WgradArgs &a) {
+static bool mfma_wgrad_shape(const WgradArgs &a) {
   if (skinny_shape(a)) return true;     // (no MFMA there: the skinny kernel shares this path's accumulator)
   if (a.c_in % 32 != 0 || a.c_out % 32 != 0) return false;
   if (reinterpret_cast<uintptr_t>(a.in) % 16 || reinterpret_cast<uintptr_t>(a.gout) % 16) return false;
@@ -408,6 +413,8 @@ bool mfma_wgrad_supported(const WgradArgs &a) {
   return true;
 }
 
+bool mfma_wgrad_supported(const WgradArgs &a) { return takes_narrow(a) || mfma_wgrad_shape(a); }
+
 // One cell's walk waits for the rows it meets -- 3.3 times the cloud's rows to a cell, or its pairs where these
 // are fewer, by what a row of the tile costs -- and the chip multiplies 40 pairs x 32 x 32 channels a nanosecond.  On dense maps the copies always pay, twice over; on thin ones there are too few pairs to cut more
 // cells, where the vector ALUs take pieces of 512 pairs x 32 x 32 channels.  Thinned clouds, fp32, copies / vector ALUs:
@@ -416,7 +423,9 @@ bool mfma_wgrad_supported(const WgradArgs &a) {
 double padded_wgrad_us(const WgradArgs &p) {
   double per_row = 0, cells = 1;
   WgradGeometry g;
-  if (skinny_shape(p)) {
+  if (takes_narrow(p)) {
+    return 19;
+  } else if (skinny_shape(p)) {
     per_row = 0.076 / 512 * p.c_in * p.c_out;
     cells = (double)choose_slices(p, 1, 64, (int64_t)num_cus() * 2).slices * p.k_vol;
   } else if (wgrad_geometry(p, &g) == FGMS_OK) {
@@ -452,7 +461,7 @@ static void wave_geometry(const WgradArgs &a, WgradGeometry *g) {
 }
 
 int wgrad_geometry(const WgradArgs &a, WgradGeometry *g, bool shares_grid) {
-  if (skinny_shape(a) || !mfma_wgrad_supported(a)) {
+  if (skinny_shape(a) || !mfma_wgrad_shape(a)) {
     set_error("wgrad_geometry: not a shape of the MFMA weight-gradient kernels");
     return FGMS_E_INVALID;
   }
@@ -538,6 +547,7 @@ int launch_mfma_wgrad(const WgradArgs &args) {
   WgradArgs a = args;
   // (a pending fingerprint check of the plan rides along as the launch's side job)
   if (!a.side.kind && a.plan) (void)plan_take_check(a.plan, &a.side);
+  if (takes_narrow(a)) return launch_narrow_wgrad(a, a.plan);
   float *acc32 = nullptr;
   int rc = wgrad_accumulator(a, &acc32);
   if (rc != FGMS_OK) return rc;
@@ -602,7 +612,7 @@ int scratch_address(float **ptr) {
 
 int wgrad_static(WgradArgs a) {
   if (a.n_pairs == 0) return FGMS_OK;
-  if (kernel_policy() == 1 || !mfma_wgrad_supported(a)) {
+  if (kernel_policy() == 1 || !mfma_wgrad_shape(a)) {
     set_error("fgms_wgrad_static: only the shapes of the MFMA / skinny weight-gradient kernels "
               "(channel counts that are multiples of 32, or 4/8/16 -> 16/32/64; 16-byte aligned rows)");
     return FGMS_E_INVALID;
