@@ -68,6 +68,7 @@ struct GmsArgs {
   int64_t n_pairs;    // upper bound on kpos[k_vol]
   bool transpose_w;   // dgrad
   int dense_k;        // >= 0: identity map over n_dense rows with W[dense_k]
+  int centre;         // k + 1: the lists without offset k, and the identity map over all rows with W[k]; 0: none
   int64_t n_dense;
   int dtype;
   hipStream_t stream;
@@ -107,6 +108,7 @@ struct WgradArgs {
 
 constexpr int kPlanFlags = 32;      // ints the plan build reports back (see fgms_plan.hip)
 constexpr int kFlagStale = 13;      // flags[13]: a later check found another fingerprint (fgms_plan_check)
+constexpr int kFlagCentre = 14;     // flags[14]: see Plan::centre_line
 constexpr int kFlagPrint = 16;      // flags[16 .. 31]: fingerprint of the pair lists (kPrintParts 64-bit words)
 constexpr int kPrintParts = 8;      // ... each over an eighth of the sample, so that as many workgroups take it
 
@@ -190,6 +192,10 @@ struct Plan {
   int32_t *pv_in, *pv_out;        // [pv_rows]
   unsigned long long *pv_mask;    // [pv_rows / 64]
   int64_t pv_rows;                // a multiple of 256
+  // The middle offset of an odd number of them has no pairs (the caller keeps it out of the lists): its lines
+  // of the tables then hold the row order, through which every row is its own neighbour.  No mask names
+  // the offset, so that only a launch that asks for it (GmsArgs::centre) sees them.
+  bool centre_line;
   bool fwd_ok;        // no offset maps two pairs onto one output row
   bool dgrad_ok;      // no offset maps two pairs from one input row
 };

@@ -607,9 +607,9 @@ int map_build_begin(MapBuild **build, const int32_t *in_coords, int64_t n_in, co
     p->tile_grid_in = p->tile_in ? cap_in * 8 : 0;
     sort.flags = p->flags;
     sort.kpos = kpos;
-    sort.side[0].rmask = rmask_out; sort.side[0].perm = p->perm_out; sort.side[0].block_mask = p->mask_out;
+    sort.side[0].rmask = rmask_out; sort.side[0].perm = p->perm_out; sort.side[0].block_mask = p->mask_out; sort.side[0].nbr = p->nbr_out;
     if (!mirror) {
-      sort.side[1].rmask = rmask_in; sort.side[1].perm = p->perm_in; sort.side[1].block_mask = p->mask_in;
+      sort.side[1].rmask = rmask_in; sort.side[1].perm = p->perm_in; sort.side[1].block_mask = p->mask_in; sort.side[1].nbr = p->nbr_in;
     }
   }
   FillBatch fills{};

@@ -540,6 +540,9 @@ constexpr int rows_group_chunks() {      // 16-byte chunks of LDS per group: two
 template <int NT, int MT>
 constexpr int rows_sum_chunks() { return kWaves * MT * NT * 4 * 64; }      // ... of a group's sums
 
+// centre (forward only; 0: none): the bit of an offset through which every row is its own neighbour, and which the caller
+// keeps out of its lists; the offset's line of the table says so, the masks do not (see Plan::centre_line).
+
 // RAGGED (fp16, RAW 1 and 2): channel counts that fill no whole tile.  Chunks of rows and weights from c_src
 // on, and of weights from c_dst on, are loaded from outside their buffers and arrive as zeros; columns from
 // c_dst on are not written.
@@ -549,7 +552,7 @@ __device__ __forceinline__ void gms_rows_body(
     const int32_t *__restrict__ nbr, const unsigned long long *__restrict__ block_masks,
     const int32_t *__restrict__ perm, const int32_t *__restrict__ tile_order, int n_dst, int k_vol,
     int c_src, int c_dst, int part_stages, int block_x, int block_y, int block_z, int grid_z,
-    unsigned src_bytes, int pair_view, int overwrite, int flip) {
+    unsigned src_bytes, int pair_view, int overwrite, int flip, unsigned long long centre) {
   constexpr int E = Elem<T>::per_chunk;
   constexpr int C = 2 * S;
   // 16-bit matrix instructions (fp16 tensors, fp32 tensors in split bf16): rows and weights come
@@ -597,7 +600,7 @@ __device__ __forceinline__ void gms_rows_body(
     const int entry = tile_order[block_x];
     if (entry < 0) return;
     tile = entry & 0xFFFFFF;
-    if (grid_z == 1) k_first = entry >> 24;
+    if (grid_z == 1 && !centre) k_first = entry >> 24;
   }
   const int row0 = tile * TR + wave * WR;
   const int my_row = row0 + lane;
@@ -611,7 +614,7 @@ __device__ __forceinline__ void gms_rows_body(
   if (owns_row) didx[lane] = in_range ? (perm ? perm[my_row] : my_row) : -1;   // my_row is a position in the plan's row order
 
   // which offsets touch this wave's rows / this workgroup's rows (from the plan)
-  unsigned long long wave_mask = row0 < n_dst ? block_masks[row0 / 64] : 0ull;
+  unsigned long long wave_mask = row0 < n_dst ? block_masks[row0 / 64] | centre : 0ull;
   // (one value for the whole wave: in scalar registers where vector registers are short)
   if constexpr (sizeof(T) == 2 || RAW == 3 || RAW == 4)
     wave_mask = (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(wave_mask & 0xffffffffu)) |
@@ -976,7 +979,7 @@ __global__ __launch_bounds__(kThreads * KG, MT == 1 ? (NT == 3 ? 3 : 4) : (NT >=
     const int32_t *__restrict__ nbr, const unsigned long long *__restrict__ block_masks,
     const int32_t *__restrict__ perm, const int32_t *__restrict__ tile_order, int n_dst, int k_vol,
     int c_src, int c_dst, int part_stages, SideJob side, int pair_view, unsigned src_bytes, int overwrite,
-    int flip) {
+    int flip, unsigned long long centre) {
   // the leading workgroups of the grid run the side job, if there is one
   int block_x = blockIdx.x;
   if (side.blocks) {
@@ -988,7 +991,7 @@ __global__ __launch_bounds__(kThreads * KG, MT == 1 ? (NT == 3 ? 3 : 4) : (NT >=
   }
   gms_rows_body<T, NT, S, RAW, MT, KG, RAGGED>(src, packed, dst, nbr, block_masks, perm, tile_order, n_dst, k_vol, c_src,
                                    c_dst, part_stages, block_x, blockIdx.y, blockIdx.z, gridDim.z, src_bytes, pair_view,
-                                   overwrite, flip);
+                                   overwrite, flip, centre);
 }
 
 // ---------------------------------------------------------------------------
@@ -1331,7 +1334,7 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
     kern<<<dim3(gx + (unsigned)a.side.blocks, gy, gz), kThreads * kg, lds_rows, a.stream>>>(
         (const T *)a.src, packed, (T *)a.dst, nbr, masks, perm, tile_order, (int)a.n_dst, a.k_vol,
         s.c_src, s.c_dst, part_stages > 0 ? part_stages : 1, a.side, pair_view ? 1 : 0,
-        (unsigned)((size_t)a.n_src * s.c_src * sizeof(T)), overwrite ? 1 : 0, flip);
+        (unsigned)((size_t)a.n_src * s.c_src * sizeof(T)), overwrite ? 1 : 0, flip, a.centre ? 1ull << (a.centre - 1) : 0ull);
   }
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;
@@ -1372,7 +1375,7 @@ __global__ __launch_bounds__(kThreads, NT >= 3 || BI * BJ == 16 || ((BI == 3 || 
   if ((int)blockIdx.x < rows_total) {
     const int bx = blockIdx.x % row_x, rest = blockIdx.x / row_x;
     gms_rows_body<T, NT, S, RAWD, MT, 1, RAGGED>(gout, w, gin, nbr, block_masks, perm, tile_order, n_in, k_vol, c_out, c_in,
-                                      part_stages, bx, rest % row_y, rest / row_y, row_z, gout_bytes, 0, overwrite, flip);
+                                      part_stages, bx, rest % row_y, rest / row_y, row_z, gout_bytes, 0, overwrite, flip, 0);
   } else {
     const int j = blockIdx.x - rows_total;
     if constexpr (BI <= 3 && BJ <= 3)

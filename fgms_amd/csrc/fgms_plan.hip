@@ -301,6 +301,8 @@ __global__ __launch_bounds__(kWindowThreads) void sort_window_kernel(SortArgs a)
   int flip = 0;
   bitonic_window(key, buf, base, lane, flip);
   int bits = 0, row_bits = 0;
+  const int centre = empty_centre(a.kpos, a.k_vol);
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) a.flags[kFlagCentre] = centre >= 0;
 #pragma unroll
   for (int r = 0; r < 2; ++r) {
     const int p = p0 + base + r * 64 + lane;
@@ -308,6 +310,7 @@ __global__ __launch_bounds__(kWindowThreads) void sort_window_kernel(SortArgs a)
     if (p < sd.n) {
       const int row = (int)(unsigned)key[r];
       sd.perm[p] = row;
+      if (centre >= 0) sd.nbr[(size_t)centre * sd.n + p] = row;
       sd.inv[row] = p;
       m = sd.rmask[row];
     }
@@ -632,9 +635,14 @@ __global__ __launch_bounds__(256) void tables_kernel(TablesArgs a) {
       }
     }
     __syncthreads();
+    const int centre = empty_centre(a.kpos, a.k_vol);
     if (p0 + lane < a.n_out) {
-      const int o = a.inv_in ? a.perm_out[p0 + lane] : 0;
+      const int o = a.inv_in || centre >= 0 ? a.perm_out[p0 + lane] : 0;
       for (int k = wave; k < a.k_vol; k += 4) {
+        if (k == centre) {
+          a.nbr_out[(size_t)k * a.n_out + p0 + lane] = o;
+          continue;
+        }
         const int i = lds[lane * ld + k];
         a.nbr_out[(size_t)k * a.n_out + p0 + lane] = i;
         if (a.inv_in && i >= 0) a.nbr_in[(size_t)k * a.n_in + a.inv_in[i]] = o;
@@ -904,8 +912,8 @@ int plan_create(fgms_plan_t **plan_out, const int32_t *kpos, const int32_t *in_m
     p->tile_grid_in = p->tile_in ? cap_in * 8 : 0;
     sa.flags = p->flags;
     sa.kpos = kpos;
-    sa.side[0].rmask = rmask; sa.side[0].perm = p->perm_out; sa.side[0].block_mask = p->mask_out;
-    sa.side[1].rmask = rmask + n_out; sa.side[1].perm = p->perm_in; sa.side[1].block_mask = p->mask_in;
+    sa.side[0].rmask = rmask; sa.side[0].perm = p->perm_out; sa.side[0].block_mask = p->mask_out; sa.side[0].nbr = p->nbr_out;
+    sa.side[1].rmask = rmask + n_out; sa.side[1].perm = p->perm_in; sa.side[1].block_mask = p->mask_in; sa.side[1].nbr = p->nbr_in;
   }
   FillBatch fills{};
   fills.add(p->flags, kPlanFlags * sizeof(int), 0);
@@ -1050,6 +1058,7 @@ const Plan *plan_resolve(fgms_plan_t *plan, hipStream_t stream, int *rc) {
       p->pv_in = b->pv_out; p->pv_out = b->pv_in; p->pv_mask = b->pv_mask; p->pv_rows = b->pv_rows;
       p->pv_ready = b->pv_ready; p->pv_stream = b->pv_stream;
       p->has_tables = b->has_tables;
+      p->centre_line = b->centre_line;
       p->pairs_counted = b->pairs_counted;
       p->ordered = false;
       // (the weight gradient's row bands follow the base's output rows: not valid for the swapped lists)
@@ -1078,6 +1087,7 @@ const Plan *plan_resolve(fgms_plan_t *plan, hipStream_t stream, int *rc) {
       p->dgrad_ok = p->has_tables && !h[0] && !h[2] && h[11] == h[12];
       p->ordered = !h[0] && !h[3];
       p->bands_ok = p->has_bands && p->ordered;
+      p->centre_line = p->has_tables && h[kFlagCentre];
       p->stages_out = h[4];
       p->stages_in = h[5];
       p->pairs_counted = p->has_tables ? h[12] : p->n_pairs;

@@ -47,6 +47,7 @@ struct SortSide {
   int32_t *hist_before;              // [chunks][kBins] rows of the bin in earlier chunks
   int32_t *bin_start;                // [kBins] rows per bin
   unsigned long long *block_mask;    // OR of the masks of every 64 positions
+  int32_t *nbr;                      // the side's table (the middle offset's line, see Plan::centre_line)
   int n, chunks;                     // chunks == 0: one window, no counting sort
 };
 struct SortArgs {
@@ -62,6 +63,12 @@ constexpr int kChunk = 2048;         // rows per workgroup of the histogram / sc
 constexpr int kWindow = 1024;        // positions per workgroup of the window sort
 constexpr int kSortThreads = 1024;
 constexpr int kWindowThreads = kWindow / 2;
+
+// An odd number of offsets without pairs in the middle one (-1: otherwise).
+__device__ __forceinline__ int empty_centre(const int32_t *__restrict__ kpos, int k_vol) {
+  const int mid = k_vol / 2;
+  return k_vol % 2 == 1 && kpos[mid] == kpos[mid + 1] ? mid : -1;
+}
 
 // Bin of a key.
 __device__ __forceinline__ int top_bits(unsigned long long key, int k_vol) {
