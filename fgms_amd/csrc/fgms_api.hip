@@ -719,25 +719,31 @@ int run_gms_padded(const GmsArgs &a, const Plan *plan, int c_in, int c_out, bool
   const size_t src_bytes = (size_t)a.n_src * p_src * esz, w_bytes = (size_t)a.k_vol * c_in * c_out * esz,
                dst_bytes = (size_t)a.n_dst * p_dst * esz;
   const int src_slot = a.transpose_w ? kSlotPadOut : kSlotPadIn;
-  *done = workspaces_fit(a.stream, {{src_slot, src_bytes}, {kSlotPadWeights, w_bytes}, {kSlotPadResult, dst_bytes}});
+  // (rows that fill whole tiles as they are need no copy, nor do results)
+  const bool copy_src = p_src != c_src || reinterpret_cast<uintptr_t>(a.src) % 16, crop = p_dst != c_dst || reinterpret_cast<uintptr_t>(a.dst) % 16;
+  *done = workspaces_fit(a.stream, {{src_slot, copy_src ? src_bytes : 0}, {kSlotPadWeights, w_bytes}, {kSlotPadResult, crop ? dst_bytes : 0}});
   if (!*done) return FGMS_OK;
   GmsArgs p = a;
   p.c_in = c_in;
   p.c_out = c_out;
   void *src = nullptr, *w = nullptr, *dst = nullptr;
   int rc;
-  if ((rc = workspace_get(a.stream, src_slot, src_bytes, &src)) || (rc = workspace_get(a.stream, kSlotPadWeights, w_bytes, &w)) ||
-      (rc = workspace_get(a.stream, kSlotPadResult, dst_bytes, &dst)))
+  if ((copy_src && (rc = workspace_get(a.stream, src_slot, src_bytes, &src))) || (rc = workspace_get(a.stream, kSlotPadWeights, w_bytes, &w)) ||
+      (crop && (rc = workspace_get(a.stream, kSlotPadResult, dst_bytes, &dst))))
     return rc;
   PadBatch pads{};
-  pads.add(a.src, src, (size_t)a.n_src, 1, 1, c_src, p_src, (int)esz);
+  if (copy_src) {
+    pads.add(a.src, src, (size_t)a.n_src, 1, 1, c_src, p_src, (int)esz);
+    p.src = src;
+  }
   pads.add(a.w, w, (size_t)a.k_vol, a.c_in, c_in, a.c_out, c_out, (int)esz);
   if ((rc = launch_pad(pads, a.dtype, a.stream))) return rc;
-  p.src = src;
   p.w = w;
-  p.dst = dst;
-  p.overwrite = true;
-  if ((rc = run_gms(p, plan))) return rc;
+  if (crop) {
+    p.dst = dst;
+    p.overwrite = true;
+  }
+  if ((rc = run_gms(p, plan)) || !crop) return rc;
   return launch_crop(dst, a.dst, (size_t)a.n_dst, c_dst, p_dst, a.overwrite, a.dtype, a.stream);
 }
 
@@ -761,20 +767,26 @@ bool padded_wgrad_channels(const WgradArgs &a, int *c_in, int *c_out) {
 // they are added to the caller's tensor.
 int run_wgrad_padded(const WgradArgs &a, int c_in, int c_out, bool *done) {
   const size_t esz = elem_size(a.dtype);
-  const size_t in_bytes = (size_t)a.n_in * c_in * esz, gout_bytes = (size_t)a.n_out * c_out * esz;
+  const bool copy_in = c_in != a.c_in || reinterpret_cast<uintptr_t>(a.in) % 16, copy_gout = c_out != a.c_out || reinterpret_cast<uintptr_t>(a.gout) % 16;
+  const size_t in_bytes = copy_in ? (size_t)a.n_in * c_in * esz : 0, gout_bytes = copy_gout ? (size_t)a.n_out * c_out * esz : 0;
   *done = workspaces_fit(a.stream, {{kSlotPadIn, in_bytes}, {kSlotPadOut, gout_bytes}, {1, (size_t)a.k_vol * c_in * c_out * sizeof(float)}});
   if (!*done) return FGMS_OK;
   void *in = nullptr, *gout = nullptr;
   int rc;
-  if ((rc = workspace_get(a.stream, kSlotPadIn, in_bytes, &in)) || (rc = workspace_get(a.stream, kSlotPadOut, gout_bytes, &gout)))
+  if ((copy_in && (rc = workspace_get(a.stream, kSlotPadIn, in_bytes, &in))) ||
+      (copy_gout && (rc = workspace_get(a.stream, kSlotPadOut, gout_bytes, &gout))))
     return rc;
-  PadBatch pads{};
-  pads.add(a.in, in, (size_t)a.n_in, 1, 1, a.c_in, c_in, (int)esz);
-  pads.add(a.gout, gout, (size_t)a.n_out, 1, 1, a.c_out, c_out, (int)esz);
-  if ((rc = launch_pad(pads, a.dtype, a.stream))) return rc;
   WgradArgs p = a;
-  p.in = in;
-  p.gout = gout;
+  PadBatch pads{};
+  if (copy_in) {
+    pads.add(a.in, in, (size_t)a.n_in, 1, 1, a.c_in, c_in, (int)esz);
+    p.in = in;
+  }
+  if (copy_gout) {
+    pads.add(a.gout, gout, (size_t)a.n_out, 1, 1, a.c_out, c_out, (int)esz);
+    p.gout = gout;
+  }
+  if ((rc = launch_pad(pads, a.dtype, a.stream))) return rc;
   p.c_in = c_in;
   p.c_out = c_out;
   p.crop_in = a.c_in;
