@@ -441,9 +441,12 @@ def main():
             # the backward call's single launch computes both gradients
             parts = ("dgrad", "wgrad") if dom.startswith("bwd_fused") else \
                 (("dgrad",) if "dgrad" in dom else (("wgrad",) if "wgrad" in dom else ("fwd",)))
-            # fp32 tensors in tf32 mode: every product is three bf16 MFMAs (hi*hi + hi*lo + lo*hi),
-            # so the matrix pipes do three times the algorithmic flop, at the 16-bit rate
-            factor, peak = (3, PEAK_TFLOPS["f16"]) if "bf16x3" in dom else (1, PEAK_TFLOPS[arith])
+            # fp32 tensors: every product is several bf16 MFMAs of the values' parts (three in tf32 mode, six in
+            # fp32 mode), so the matrix pipes do that many times the algorithmic flop, at the 16-bit rate
+            six = (arith == "f32" and not arch80 and dom.startswith(("gms_rows", "bwd_fused", "wgrad_wave")) and
+                   L["c_in"] % 32 == 0 and L["c_out"] % 32 == 0 and os.environ.get("FGMS_SPLIT_BF16") != "0")
+            factor = 3 if "bf16x3" in dom else 6 if six else 1
+            peak = PEAK_TFLOPS["f16" if factor > 1 else arith]
             ach = factor * len(parts) * flops_pass / avg_s / 1e12
             flow = sum(dataflow_bytes(L, w_) for w_ in parts)
             traffic = measured_traffic(args.workload, dom)
@@ -451,7 +454,7 @@ def main():
                         "unit": "TFLOP/s", "frac": ach / peak, "traffic": traffic,
                         "traffic_source": TRAFFIC_SOURCE if traffic is not None else None,
                         "mfma_flop_per_algorithmic_flop": factor,
-                        # `frac` prices the matrix pipes' work (for split bf16: three MFMA flop per
+                        # `frac` prices the matrix pipes' work (for bf16 parts: three or six MFMA flop per
                         # algorithmic flop); frac_algorithmic prices the useful work alone, against
                         # the same 16-bit peak and against the fp32 MFMA peak the tensors' type has
                         "frac_algorithmic": len(parts) * flops_pass / avg_s / 1e12 / peak,

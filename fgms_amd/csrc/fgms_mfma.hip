@@ -67,9 +67,9 @@ __device__ __forceinline__ void load_weights(int4v *__restrict__ w_lds,
   }
 }
 
-// The same for split weights (pack_weights_bf3_kernel): per (slab, k-step) NT * 128 chunks.
+// The same for split weights (pack_weights_parts_kernel): per (slab, k-step) NT * 128 chunks.
 template <int NT>
-__device__ __forceinline__ void load_weights_bf3(int4v *__restrict__ w_lds,
+__device__ __forceinline__ void load_weights_split(int4v *__restrict__ w_lds,
                                                  const int4v *__restrict__ packed_k, int slabs, int nts,
                                                  int nt0) {
   const int n = slabs * 2 * NT * 128;
@@ -210,108 +210,76 @@ __device__ __forceinline__ void mma_slab_rawt(float16v (&acc)[MT][NT], const int
 // is below 2^-16 of the product, so this is more exact than tf32, at 3/16 of the fp32 matrix
 // time.  Rows are split when they go from registers to LDS, the weights by their re-layout
 // kernel.
-// Slot (16 bytes = 8 bf16) of a wave's split staging tile: row-major, a row holds its 32
-// values of the slab as 4 chunks of hi followed by 4 chunks of lo (128 bytes, as the fp32
-// row did); the XOR spreads the 8 rows one b128 read pass touches over all banks.
-__device__ __forceinline__ int a_bf_slot(int row, int part, int j) {
-  return row * 8 + part * 4 + (j ^ ((row >> 1) & 3));
+//
+// The same for fp32 tensors in full precision, with three parts and six products (RAW = 5 and 6): x = h + m + l holds
+// all 24 bits, and what is dropped of a product (m*l, l*m, l*l) is below 2^-23 of it and of either sign, less than the fp32
+// sum around it rounds off (mma_parts has the errors).  Six 16-bit matrix steps take 6/16 of the fp32 ones' time; a
+// tile of rows takes half as much LDS again, which leaves two workgroups to a CU.  fp32 MFMAs / this: 64 -> 64 forward over
+// 40 k voxels 88 / 63 us, 150 k 172 / 111; backward 123 / 77, 342 / 232; 128 -> 128 over 40 k 231 / 133 and 360 / 238;
+// 32 -> 32 over 4 k 25 / 21 and 20 / 18.5.  (A value below 2^-110 or so loses the last bits of its small parts, and an
+// infinite one makes NaN of what it reaches.)
+//
+// Slot (16 bytes = 8 bf16) of a split tile of P parts: row-major, a row holds its 32 values of the slab
+// as 4 chunks of each part; the XOR spreads the rows one b128 read pass (16 lanes) touches over all banks: rows of
+// 128 bytes go by pairs, of 192 bytes by fours.
+template <int P>
+__device__ __forceinline__ int part_slot(int row, int part, int j) {
+  return row * (4 * P) + part * 4 + (j ^ ((row >> (P == 3 ? 2 : 1)) & 3));
 }
 
-// One fp32 chunk (4 values; chunk c of its row's slab) split and written to a split tile.
-// Lane pairs hold the two fp32 chunks that make one bf16 chunk; they exchange halves, so the
-// even lane ends up with the 8 hi values and the odd one with the 8 lo values and each
-// still writes one 16-byte chunk.
-__device__ __forceinline__ void split_and_store(int4v *__restrict__ tile, const float4v &x, int row, int c,
-                                                int lane) {
-  const bool odd = lane & 1;
-  bf16x4 hi, lo;
+// One fp32 chunk (4 values; chunk c of its row's slab) split and written to a split tile: 8 bytes of each part.
+template <int P>
+__device__ __forceinline__ void split_and_store(int4v *__restrict__ tile, const float4v &x, int row, int c) {
+  int2v part[P];
+  split_parts<P>(x, part);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    __bf16 h, l;
-    split_bf16(x[i], h, l);
-    hi[i] = h;
-    lo[i] = l;
-  }
-  const int2v h2 = __builtin_bit_cast(int2v, hi), l2 = __builtin_bit_cast(int2v, lo);
-  // the even lane hands over its lo half and takes the odd lane's hi half
-  const int got0 = __builtin_bit_cast(int, swap_with_neighbour(__builtin_bit_cast(float, odd ? h2[0] : l2[0])));
-  const int got1 = __builtin_bit_cast(int, swap_with_neighbour(__builtin_bit_cast(float, odd ? h2[1] : l2[1])));
-  tile[a_bf_slot(row, odd ? 1 : 0, c / 2)] = odd ? int4v{got0, got1, l2[0], l2[1]} : int4v{h2[0], h2[1], got0, got1};
+  for (int q = 0; q < P; ++q) reinterpret_cast<int2v *>(tile)[part_slot<P>(row, q, c / 2) * 2 + (c & 1)] = part[q];
 }
 
 // registers -> LDS for the split tile of gathered rows (absent rows as zeros).
-template <int N>
-__device__ __forceinline__ void gather_commit_bf3(int4v *__restrict__ a_lds, int4v (&v)[N],
-                                                  const int (&g)[N], int lane) {
+template <int P, int N>
+__device__ __forceinline__ void gather_commit_parts(int4v *__restrict__ a_lds, int4v (&v)[N],
+                                                    const int (&g)[N], int lane) {
 #pragma unroll
   for (int it = 0; it < N; ++it) {
     const int slot = it * 64 + lane;
     const float4v x = g[it] < 0 ? float4v{0.f, 0.f, 0.f, 0.f} : __builtin_bit_cast(float4v, v[it]);
-    split_and_store(a_lds, x, slot / 8, slot % 8, lane);
+    split_and_store<P>(a_lds, x, slot / 8, slot % 8);
   }
 }
 
-// acc[mt][nt] += A(slab) x W(slab), both split; weights in LDS as [k-step][nt][hi, lo][lane].
-template <int NT, int MT>
-__device__ __forceinline__ void mma_slab_bf3(float16v (&acc)[MT][NT], const int4v *__restrict__ a_lds,
-                                             const int4v *__restrict__ w_lds, int lane) {
+// acc[mt][nt] += A(slab) x W(slab), both split.  Weights in LDS as [k-step][nt][part][lane], or (AS_ROWS: the input
+// gradient) as a split tile of the NT*32 rows of W[k], the slab's 32 columns.
+template <int P, bool AS_ROWS, int NT, int MT>
+__device__ __forceinline__ void mma_slab_parts(float16v (&acc)[MT][NT], float16v (&low)[P == 3 ? MT : 1][P == 3 ? NT : 1], const int4v *__restrict__ a_lds,
+                                               const int4v *__restrict__ w_lds, int lane) {
   const int h = lane / 32, r = lane % 32;
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
-    bf16x8 bh[NT], bl[NT];
+    bf16x8 b[NT][P];
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      bh[nt] = __builtin_bit_cast(bf16x8, w_lds[((s * NT + nt) * 2 + 0) * 64 + lane]);
-      bl[nt] = __builtin_bit_cast(bf16x8, w_lds[((s * NT + nt) * 2 + 1) * 64 + lane]);
-    }
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int q = 0; q < P; ++q)
+        b[nt][q] = __builtin_bit_cast(bf16x8, w_lds[AS_ROWS ? part_slot<P>(nt * 32 + r, q, s * 2 + h) : ((s * NT + nt) * P + q) * 64 + lane]);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
-      const bf16x8 ah = __builtin_bit_cast(bf16x8, a_lds[a_bf_slot(mt * 32 + r, 0, s * 2 + h)]);
-      const bf16x8 al = __builtin_bit_cast(bf16x8, a_lds[a_bf_slot(mt * 32 + r, 1, s * 2 + h)]);
+      bf16x8 a[P];
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bh[nt], acc[mt][nt], 0, 0, 0);
-        acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bl[nt], acc[mt][nt], 0, 0, 0);
-        acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bh[nt], acc[mt][nt], 0, 0, 0);
-      }
+      for (int q = 0; q < P; ++q) a[q] = __builtin_bit_cast(bf16x8, a_lds[part_slot<P>(mt * 32 + r, q, s * 2 + h)]);
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) mma_parts<P>(acc[mt][nt], low[P == 3 ? mt : 0][P == 3 ? nt : 0], a, b[nt]);
     }
   }
 }
 
-// The same for the input gradient: the weight tile (NT*32 rows of W[k], the slab's 32 columns)
-// was split on its way to LDS like a tile of gathered rows (RAW = 4).
-template <int NT, int MT>
-__device__ __forceinline__ void mma_slab_bf3t(float16v (&acc)[MT][NT], const int4v *__restrict__ a_lds,
-                                              const int4v *__restrict__ w_lds, int lane) {
-  const int h = lane / 32, r = lane % 32;
-#pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    bf16x8 bh[NT], bl[NT];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      bh[nt] = __builtin_bit_cast(bf16x8, w_lds[a_bf_slot(nt * 32 + r, 0, s * 2 + h)]);
-      bl[nt] = __builtin_bit_cast(bf16x8, w_lds[a_bf_slot(nt * 32 + r, 1, s * 2 + h)]);
-    }
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const bf16x8 ah = __builtin_bit_cast(bf16x8, a_lds[a_bf_slot(mt * 32 + r, 0, s * 2 + h)]);
-      const bf16x8 al = __builtin_bit_cast(bf16x8, a_lds[a_bf_slot(mt * 32 + r, 1, s * 2 + h)]);
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bh[nt], acc[mt][nt], 0, 0, 0);
-        acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bl[nt], acc[mt][nt], 0, 0, 0);
-        acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bh[nt], acc[mt][nt], 0, 0, 0);
-      }
-    }
-  }
-}
-
-// Split weights in the order mma_slab_bf3 reads them: chunk
-//   ((((k * slabs + slab) * 2 + s) * nts + nt) * 2 + part) * 64 + lane
-// holds the 8 values op(W[k])[slab*32 + s*16 + (lane/32)*8 + 0..7][nt*32 + lane%32], hi (part 0)
-// or lo (part 1).  One thread per chunk pair.
-__global__ void pack_weights_bf3_kernel(const float *__restrict__ w, int4v *__restrict__ packed,
-                                        int k_vol, int c_in, int c_out, bool transpose) {
+// Split weights in the order mma_slab_parts reads them: chunk
+//   ((((k * slabs + slab) * 2 + s) * nts + nt) * P + part) * 64 + lane
+// holds the 8 values op(W[k])[slab*32 + s*16 + (lane/32)*8 + 0..7][nt*32 + lane%32] of that part.
+// One thread per P chunks.
+template <int P>
+__global__ void pack_weights_parts_kernel(const float *__restrict__ w, int4v *__restrict__ packed,
+                                          int k_vol, int c_in, int c_out, bool transpose) {
   // (transpose: the input gradient's view, W[k]^T -- source channels are the columns of W[k])
   const int slabs = (transpose ? c_out : c_in) / 32, nts = (transpose ? c_in : c_out) / 32;
   const size_t total = (size_t)k_vol * slabs * 2 * nts * 64;
@@ -324,17 +292,16 @@ __global__ void pack_weights_bf3_kernel(const float *__restrict__ w, int4v *__re
     const int slab = (int)(q % slabs);
     const int k = (int)(q / slabs);
     const int cs0 = slab * 32 + s * 16 + (lane / 32) * 8, cd = nt * 32 + lane % 32;
-    bf16x8 hi, lo;
+    float4v x[2];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      __bf16 h, l;
-      split_bf16(transpose ? w[((size_t)k * c_in + cd) * c_out + cs0 + e] : w[((size_t)k * c_in + cs0 + e) * c_out + cd], h, l);
-      hi[e] = h;
-      lo[e] = l;
-    }
-    const size_t base = (t / 64) * 128 + lane;
-    packed[base] = __builtin_bit_cast(int4v, hi);
-    packed[base + 64] = __builtin_bit_cast(int4v, lo);
+    for (int e = 0; e < 8; ++e)
+      x[e / 4][e % 4] = transpose ? w[((size_t)k * c_in + cd) * c_out + cs0 + e] : w[((size_t)k * c_in + cs0 + e) * c_out + cd];
+    int2v lo[P], hi[P];
+    split_parts<P>(x[0], lo);
+    split_parts<P>(x[1], hi);
+    const size_t base = (t / 64) * (64 * P) + lane;
+#pragma unroll
+    for (int part = 0; part < P; ++part) packed[base + part * 64] = int4v{lo[part][0], lo[part][1], hi[part][0], hi[part][1]};
   }
 }
 
@@ -413,19 +380,19 @@ __device__ __forceinline__ void gather_commit_buf(int4v *__restrict__ a_lds, con
   }
 }
 
-template <int N>
-__device__ __forceinline__ void gather_commit_bf3_buf(int4v *__restrict__ a_lds, const int4v (&v)[N], int lane) {
+template <int P, int N>
+__device__ __forceinline__ void gather_commit_parts_buf(int4v *__restrict__ a_lds, const int4v (&v)[N], int lane) {
 #pragma unroll
   for (int it = 0; it < N; ++it) {
     const int slot = it * 64 + lane;
-    split_and_store(a_lds, __builtin_bit_cast(float4v, v[it]), slot / 8, slot % 8, lane);
+    split_and_store<P>(a_lds, __builtin_bit_cast(float4v, v[it]), slot / 8, slot % 8);
   }
 }
 
 // ---------------------------------------------------------------------------
 // Pair-stationary kernel.
 // SPLIT: fp32 tensors whose caller allows tf32 precision, products in split bf16 (see
-// mma_slab_bf3); `packed` from pack_weights_bf3_kernel.
+// mma_slab_parts); `packed` from pack_weights_parts_kernel.
 template <typename T, int NT, int S, bool SPLIT>
 __global__ __launch_bounds__(kThreads) void gms_pairs_kernel(
     const T *__restrict__ src, const T *__restrict__ packed, T *__restrict__ dst,
@@ -470,7 +437,7 @@ __global__ __launch_bounds__(kThreads) void gms_pairs_kernel(
     if (k != cur_k) {  // uniform over the workgroup
       __syncthreads();
       if constexpr (SPLIT)
-        load_weights_bf3<NT>(w_lds, reinterpret_cast<const int4v *>(packed) + packed_per_k * k, slabs, nts, nt0);
+        load_weights_split<NT>(w_lds, reinterpret_cast<const int4v *>(packed) + packed_per_k * k, slabs, nts, nt0);
       else
         load_weights<NT>(w_lds, reinterpret_cast<const int4v *>(packed) + packed_per_k * k, qs, nts, nt0);
       __syncthreads();
@@ -493,15 +460,16 @@ __global__ __launch_bounds__(kThreads) void gms_pairs_kernel(
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[mt][nt][r] = 0.f;
 
+    float16v low[1][1];      // (two parts: not used)
     int4v v[2 * S];
     int gsel[2 * S];
     gather_issue<T, S>(v, gsel, gidx, src, c_src, 0, lane);
     for (int slab = 0; slab < slabs; ++slab) {
-      if constexpr (SPLIT) gather_commit_bf3(a_lds, v, gsel, lane);
+      if constexpr (SPLIT) gather_commit_parts<2>(a_lds, v, gsel, lane);
       else gather_commit<S>(a_lds, v, gsel, lane);
       wave_lds_fence();
       if (slab + 1 < slabs) gather_issue<T, S>(v, gsel, gidx, src, c_src, slab + 1, lane);   // under the MFMAs
-      if constexpr (SPLIT) mma_slab_bf3<NT>(acc, a_lds, w_lds + slab * (2 * NT * 128), lane);
+      if constexpr (SPLIT) mma_slab_parts<2, false>(acc, low, a_lds, w_lds + slab * (2 * NT * 128), lane);
       else mma_slab<T, NT, S>(acc, a_lds, w_lds, slab, lane);
       wave_lds_fence();
     }
@@ -523,8 +491,9 @@ __global__ __launch_bounds__(kThreads) void gms_pairs_kernel(
 // wave reads it).
 // RAW = 1: `packed` is the caller's weight tensor itself, forward (fp16: see raw_weight_frag);
 // RAW = 2: the same for the input gradient (see mma_slab_rawt); RAW = 3: fp32 tensors with
-// products in split bf16 (see mma_slab_bf3), `packed` from pack_weights_bf3_kernel; RAW = 4:
+// products in split bf16 (see mma_slab_parts), `packed` from pack_weights_parts_kernel; RAW = 4:
 // the input gradient in split bf16, weights read as they lie and split on their way to LDS;
+// RAW = 5 and 6: as 3 and 4 with three parts to a value, for fp32 tensors in full precision;
 // RAW = 0: the re-laid copy pack_weight_elements makes.
 // (block_x, block_y, block_z) of a grid (tiles, column tiles, grid_z parts of a tile).
 // MT: 32-row MFMA tiles per wave.  2 (a workgroup tile of 256 rows) is the layout every plan
@@ -533,9 +502,12 @@ __global__ __launch_bounds__(kThreads) void gms_pairs_kernel(
 // KG > 1 (MT = 1): the workgroup is KG groups of four waves, every group walks its share of the
 // tile's offsets with LDS of its own, and the groups' sums meet in LDS behind the last stage: the chain
 // is a KG-th as long, without the atomics (and the zeroed result rows) that workgroups sharing a tile need.
+constexpr int split_parts_of(int raw) { return raw == 3 || raw == 4 ? 2 : raw == 5 || raw == 6 ? 3 : 0; }
+// 16-byte chunks of LDS per group: two stages of weights, row tiles, indices.  (Three bf16 parts take half as much
+// again as the fp32 value.)
 template <typename T, int NT, int S, int MT>
-constexpr int rows_group_chunks() {      // 16-byte chunks of LDS per group: two stages of weights, row tiles, indices
-  return 2 * S * NT * 64 + kWaves * MT * 32 * 2 * S + kWaves * 3 * MT * 32 / 4;
+constexpr int rows_group_chunks(int raw) {
+  return (2 * S * NT * 64 + kWaves * MT * 32 * 2 * S) * (split_parts_of(raw) == 3 ? 3 : 2) / 2 + kWaves * 3 * MT * 32 / 4;
 }
 template <int NT, int MT>
 constexpr int rows_sum_chunks() { return kWaves * MT * NT * 4 * 64; }      // ... of a group's sums
@@ -558,7 +530,8 @@ __device__ __forceinline__ void gms_rows_body(
   // 16-bit matrix instructions (fp16 tensors, fp32 tensors in split bf16): rows and weights come
   // through buffer loads and the MFMA phase is pipelined by hand; plain fp32, whose MFMA phase is
   // eight times as long, keeps pointer loads and interleaves them with its MFMAs instead
-  constexpr bool kBuf = sizeof(T) == 2 || RAW == 3 || RAW == 4;
+  constexpr int P = split_parts_of(RAW);
+  constexpr bool kBuf = sizeof(T) == 2 || P > 0;
   const __amdgpu_buffer_rsrc_t rsrc = rows_resource(src, src_bytes);
   const unsigned row_bytes = (unsigned)c_src * (unsigned)sizeof(T);
   // byte offset of source row g in the buffer (kAbsentRow: no neighbour, the loads return zeros)
@@ -566,16 +539,19 @@ __device__ __forceinline__ void gms_rows_body(
   // pair view: `nbr` is one list of source rows for all offsets (a 64-row block belongs to
   // the one offset its mask names), `perm` the destination rows; results are added atomically
   const size_t nbr_stride = pair_view ? 0 : (size_t)n_dst;
-  constexpr int WCH = S * NT * 64;                        // 16-byte chunks of one stage's weights
-  constexpr int NW = (WCH + kThreads - 1) / kThreads;     // ... per thread
+  constexpr int kGrow = P == 3 ? 3 : 2;                   // (three parts: halves again)
+  constexpr int WCH = S * NT * 64 * kGrow / 2;            // 16-byte chunks of one stage's weights in LDS
+  constexpr int WLD = RAW == 6 ? S * NT * 64 : WCH;       // ... as they are read
+  constexpr int NW = (WLD + kThreads - 1) / kThreads;     // ... per thread
+  constexpr int CL = C * kGrow / 2;                       // chunks of a row of the wave's tile in LDS
   extern __shared__ int4v lds_all[];
   __shared__ unsigned long long wg_mask;
   const int group = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / kThreads);
   const int tid = KG == 1 ? threadIdx.x : threadIdx.x % kThreads;
-  int4v *const lds = KG == 1 ? lds_all : lds_all + group * rows_group_chunks<T, NT, S, MT>();
+  int4v *const lds = KG == 1 ? lds_all : lds_all + group * rows_group_chunks<T, NT, S, MT>(RAW);
   // fp32 only: its MFMA phase is long enough (4 k clocks a stage) to absorb the loads'
   // issue waits; for fp16 the interleaved stage measured 2 us slower per launch
-  constexpr bool kInterleave = sizeof(T) == 4 && RAW != 3 && RAW != 4;
+  constexpr bool kInterleave = sizeof(T) == 4 && P == 0;
   static_assert(!RAGGED || (sizeof(T) == 2 && (RAW == 1 || RAW == 2)), "ragged: fp16 weights as they lie");
   const int slabs = RAGGED ? (c_src + C * E - 1) / (C * E) : c_src / (C * E);
   const int nts = c_dst / 32;
@@ -583,8 +559,8 @@ __device__ __forceinline__ void gms_rows_body(
   const int wave = tid / 64, lane = tid % 64;
   constexpr int WR = MT * 32;                             // rows per wave
   constexpr int TR = kWaves * WR;                         // rows per workgroup tile
-  int4v *a_lds = lds + 2 * WCH + wave * (WR * C);
-  int *idx_all = reinterpret_cast<int *>(lds + 2 * WCH + kWaves * (WR * C));
+  int4v *a_lds = lds + 2 * WCH + wave * (WR * CL);
+  int *idx_all = reinterpret_cast<int *>(lds + 2 * WCH + kWaves * (WR * CL));
   // per wave: the rows to gather -- byte offsets, two sets (this offset's and the next one's), or
   // plain indices (!kBuf, one set) -- and the destination rows
   unsigned *goff = reinterpret_cast<unsigned *>(idx_all + wave * 3 * WR);
@@ -592,7 +568,7 @@ __device__ __forceinline__ void gms_rows_body(
   int *didx = idx_all + wave * 3 * WR + 2 * WR;
   const int nt0 = block_y * NT;
   const int4v *packed4 = reinterpret_cast<const int4v *>(packed);
-  const size_t packed_per_k = (size_t)c_src * c_dst / E;  // chunks
+  const size_t packed_per_k = (size_t)c_src * c_dst / E * (RAW == 5 ? 3 : 2) / 2;  // chunks
 
   // the plan's table gives the tile and the first offset it uses
   int tile = block_x, k_first = -1;
@@ -616,7 +592,7 @@ __device__ __forceinline__ void gms_rows_body(
   // which offsets touch this wave's rows / this workgroup's rows (from the plan)
   unsigned long long wave_mask = row0 < n_dst ? block_masks[row0 / 64] | centre : 0ull;
   // (one value for the whole wave: in scalar registers where vector registers are short)
-  if constexpr (sizeof(T) == 2 || RAW == 3 || RAW == 4)
+  if constexpr (kBuf)
     wave_mask = (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(wave_mask & 0xffffffffu)) |
               ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(wave_mask >> 32)) << 32);
   if (threadIdx.x == 0) wg_mask = 0;
@@ -687,24 +663,32 @@ __device__ __forceinline__ void gms_rows_body(
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[mt][nt][r] = 0.f;
 
+  float16v low[P == 3 ? MT : 1][P == 3 ? NT : 1];         // three parts: the small products (mma_parts)
+  if constexpr (P == 3) {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) low[mt][nt] = acc[mt][nt];
+  }
+
   // Weights of stage (k, slab), 16-byte chunk e = threadIdx.x + kThreads * i of the stage's tile,
   // through a buffer resource over the weight tensor: the part of a chunk's address that depends
   // on the thread is a per-lane constant (wvoff), the part that depends on the stage is scalar.
   //   RAW = 1: row e / (NT*4) of the slab's 2*S*8 rows of W[k], 16-byte piece e % (NT*4) of the
   //            NT*32 columns from nt0*32 on
-  //   RAW = 2, 4: row e / C of the NT*32 rows of W[k] from nt0*32 on (c_dst rows of c_src
+  //   RAW = 2, 4, 6: row e / C of the NT*32 rows of W[k] from nt0*32 on (c_dst rows of c_src
   //            elements here), 16-byte piece e % C of the slab
-  //   RAW = 3: k-step e / (NT*128) of the stage, then [nt][hi, lo][lane]
+  //   RAW = 3, 5: k-step e / (NT*64*P) of the stage, then [nt][part][lane]
   //   RAW = 0: chunks [(slab*S + s) * nts + nt0 + nt] * 64 + lane of the re-laid copy
   const __amdgpu_buffer_rsrc_t wrsrc =
-      rows_resource(packed, (unsigned)k_vol * (unsigned)c_src * (unsigned)c_dst * (unsigned)sizeof(T));
+      rows_resource(packed, (unsigned)k_vol * (unsigned)c_src * (unsigned)c_dst * (RAW == 5 ? 6u : (unsigned)sizeof(T)));
   unsigned wvoff[NW];
 #pragma unroll
   for (int i = 0; i < NW; ++i) {
     const int e = tid + kThreads * i;
     if constexpr (RAW == 1) wvoff[i] = (unsigned)(((e / (NT * 4)) * c_dst + (e % (NT * 4)) * E) * (int)sizeof(T));
-    else if constexpr (RAW == 2 || RAW == 4) wvoff[i] = (unsigned)(((e / C) * c_src + (e % C) * E) * (int)sizeof(T));
-    else if constexpr (RAW == 3) wvoff[i] = (unsigned)(((e / (NT * 128)) * nts * 128 + e % (NT * 128)) * 16);
+    else if constexpr (RAW == 2 || RAW == 4 || RAW == 6) wvoff[i] = (unsigned)(((e / C) * c_src + (e % C) * E) * (int)sizeof(T));
+    else if constexpr (P > 0) wvoff[i] = (unsigned)(((e / (NT * 64 * P)) * nts * 64 * P + e % (NT * 64 * P)) * 16);
     else wvoff[i] = (unsigned)(((e / (NT * 64)) * nts * 64 + e % (NT * 64)) * 16);
   }
   // (flip: the tables number the offsets from the other end, see Plan)
@@ -714,7 +698,7 @@ __device__ __forceinline__ void gms_rows_body(
 #pragma unroll
       for (int i = 0; i < NW; ++i) {
         const int e = tid + kThreads * i;
-        if (NW * kThreads == WCH || e < WCH) {
+        if (NW * kThreads == WLD || e < WLD) {
           if constexpr (RAW == 2) {
             const int row = e / C, c = e % C;
             wreg[i] = *reinterpret_cast<const int4v *>(
@@ -729,13 +713,13 @@ __device__ __forceinline__ void gms_rows_body(
     }
     unsigned soff;                                       // (wave-uniform: goes to the scalar offset)
     if constexpr (RAW == 1) soff = (unsigned)(((k * c_src + slab * (C * E)) * c_dst + nt0 * 32) * (int)sizeof(T));
-    else if constexpr (RAW == 2 || RAW == 4) soff = (unsigned)(((k * c_dst + nt0 * 32) * c_src + slab * (C * E)) * (int)sizeof(T));
-    else if constexpr (RAW == 3) soff = (unsigned)(((int)packed_per_k * k + ((slab * 2) * nts + nt0) * 128) * 16);
+    else if constexpr (RAW == 2 || RAW == 4 || RAW == 6) soff = (unsigned)(((k * c_dst + nt0 * 32) * c_src + slab * (C * E)) * (int)sizeof(T));
+    else if constexpr (P > 0) soff = (unsigned)(((int)packed_per_k * k + ((slab * 2) * nts + nt0) * 64 * P) * 16);
     else soff = (unsigned)(((int)packed_per_k * k + ((slab * S) * nts + nt0) * 64) * 16);
 #pragma unroll
     for (int i = 0; i < NW; ++i) {
       const int e = tid + kThreads * i;
-      if (NW * kThreads == WCH || e < WCH) {
+      if (NW * kThreads == WLD || e < WLD) {
         unsigned off = wvoff[i];
         if constexpr (RAGGED) {
           const int from = slab * (C * E) + (RAW == 1 ? e / (NT * 4) : e % C * E);
@@ -750,14 +734,14 @@ __device__ __forceinline__ void gms_rows_body(
 #pragma unroll
     for (int i = 0; i < NW; ++i) {
       const int e = tid + kThreads * i;
-      if (NW * kThreads == WCH || e < WCH) {
+      if (NW * kThreads == WLD || e < WLD) {
         if constexpr (RAW == 1) {
           const int row = e / (NT * 4), c = e % (NT * 4);
           w_lds[buf * WCH + row * (NT * 4) + (c ^ raw_swizzle<NT>(row))] = wreg[i];
         } else if constexpr (RAW == 2) {
           w_lds[buf * WCH + a_slot<S>(e / C, e % C)] = wreg[i];
-        } else if constexpr (RAW == 4) {
-          split_and_store(w_lds + buf * WCH, __builtin_bit_cast(float4v, wreg[i]), e / C, e % C, lane);
+        } else if constexpr (RAW == 4 || RAW == 6) {
+          split_and_store<P>(w_lds + buf * WCH, __builtin_bit_cast(float4v, wreg[i]), e / C, e % C);
         } else {
           w_lds[buf * WCH + e] = wreg[i];
         }
@@ -780,7 +764,7 @@ __device__ __forceinline__ void gms_rows_body(
     else gather_issue<T, S>(v, gsel, gidx, src, c_src, slab_, lane);
   };
   auto rows_commit = [&]() {
-    if constexpr (RAW == 3 || RAW == 4) gather_commit_bf3_buf(a_lds, v, lane);
+    if constexpr (P > 0) gather_commit_parts_buf<P>(a_lds, v, lane);
     else if constexpr (kBuf) gather_commit_buf<S>(a_lds, v, lane);
     else gather_commit<S>(a_lds, v, gsel, lane);
   };
@@ -808,8 +792,7 @@ __device__ __forceinline__ void gms_rows_body(
     auto mma_stage = [&]() {
       if constexpr (RAW == 1) mma_slab_raw<T, NT, S>(acc, a_lds, w_lds + buf * WCH, lane);
       else if constexpr (RAW == 2) mma_slab_rawt<T, NT, S>(acc, a_lds, w_lds + buf * WCH, lane);
-      else if constexpr (RAW == 3) mma_slab_bf3<NT>(acc, a_lds, w_lds + buf * WCH, lane);
-      else if constexpr (RAW == 4) mma_slab_bf3t<NT>(acc, a_lds, w_lds + buf * WCH, lane);
+      else if constexpr (P > 0) mma_slab_parts<P, RAW == 4 || RAW == 6>(acc, low, a_lds, w_lds + buf * WCH, lane);
       else mma_slab<T, NT, S>(acc, a_lds, w_lds + buf * WCH, 0, lane);
     };
     // Offsets are numbered in the order the tile walks them; offset j gathers through the index
@@ -916,8 +899,6 @@ __device__ __forceinline__ void gms_rows_body(
         if (active) {
           if constexpr (RAW == 1) mma_slab_raw<T, NT, S>(acc, a_lds, w_lds + buf * WCH, lane);
           else if constexpr (RAW == 2) mma_slab_rawt<T, NT, S>(acc, a_lds, w_lds + buf * WCH, lane);
-          else if constexpr (RAW == 3) mma_slab_bf3<NT>(acc, a_lds, w_lds + buf * WCH, lane);
-          else if constexpr (RAW == 4) mma_slab_bf3t<NT>(acc, a_lds, w_lds + buf * WCH, lane);
           else mma_slab<T, NT, S>(acc, a_lds, w_lds + buf * WCH, 0, lane);
         }
       }
@@ -937,9 +918,17 @@ __device__ __forceinline__ void gms_rows_body(
       active = next_active;
     }
   }
+  if constexpr (P == 3) {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[mt][nt][r] += low[mt][nt][r];
+  }
   if constexpr (KG > 1) {
     // the groups' sums meet in the LDS behind the first group's
-    float4v *const sums = reinterpret_cast<float4v *>(lds_all + rows_group_chunks<T, NT, S, MT>());
+    float4v *const sums = reinterpret_cast<float4v *>(lds_all + rows_group_chunks<T, NT, S, MT>(RAW));
     constexpr int per_group = rows_sum_chunks<NT, MT>();
     __syncthreads();                   // every group is through with its row tiles and weights
     if (group > 0) {
@@ -974,7 +963,8 @@ __device__ __forceinline__ void gms_rows_body(
 }
 
 template <typename T, int NT, int S, int RAW, int MT = 2, int KG = 1, bool RAGGED = false>
-__global__ __launch_bounds__(kThreads * KG, MT == 1 ? (NT == 3 ? 3 : 4) : (NT >= 3 ? 2 : 3)) void gms_rows_kernel(
+__global__ __launch_bounds__(kThreads * KG, RAW >= 5 ? (MT == 2 || KG == 2 ? 2 : KG == 4 ? 4 : 3)
+                                                      : MT == 1 ? (NT == 3 ? 3 : 4) : (NT >= 3 ? 2 : 3)) void gms_rows_kernel(
     const T *__restrict__ src, const T *__restrict__ packed, T *__restrict__ dst,
     const int32_t *__restrict__ nbr, const unsigned long long *__restrict__ block_masks,
     const int32_t *__restrict__ perm, const int32_t *__restrict__ tile_order, int n_dst, int k_vol,
@@ -1108,17 +1098,18 @@ int pack_weights(const GmsArgs &a, int S, const T **packed) {
   return FGMS_OK;
 }
 
-// The same for the split-bf16 layout of fp32 weights (pack_weights_bf3_kernel).
-int pack_weights_bf3(const GmsArgs &a, bool transpose, const void **packed) {
+// The same for fp32 weights in bf16 parts (pack_weights_parts_kernel).
+template <int P>
+int pack_weights_parts(const GmsArgs &a, bool transpose, const void **packed) {
   void *ws = nullptr;
   const size_t n = (size_t)a.k_vol * a.c_in * a.c_out;
   bool fill = true;
-  int rc = relaid_weights_buffer(a, 1u | (transpose ? 2u : 0u), n * sizeof(float), &ws, &fill);
+  int rc = relaid_weights_buffer(a, 1u | (transpose ? 2u : 0u) | (P == 3 ? 4u : 0u), n * 2 * P, &ws, &fill);
   if (rc != FGMS_OK) return rc;
   *packed = ws;
   if (!fill) return FGMS_OK;
   size_t blocks = (n / 8 + 255) / 256;
-  pack_weights_bf3_kernel<<<(unsigned)(blocks > 4096 ? 4096 : blocks), 256, 0, a.stream>>>(
+  pack_weights_parts_kernel<P><<<(unsigned)(blocks > 4096 ? 4096 : blocks), 256, 0, a.stream>>>(
       (const float *)a.w, (int4v *)ws, a.k_vol, a.c_in, a.c_out, transpose);
   FGMS_HIP_TRY(hipGetLastError());
   relaid_weights_filled(a, ws);
@@ -1134,7 +1125,7 @@ int launch_pairs(const GmsArgs &a, const Shape &s) {
   const bool split = kCanSplit && a.reduced && split_bf16_enabled();
   if (split) {
     const void *ws = nullptr;
-    int rc = pack_weights_bf3(a, a.transpose_w, &ws);
+    int rc = pack_weights_parts<2>(a, a.transpose_w, &ws);
     if (rc != FGMS_OK) return rc;
     packed = (const T *)ws;
   } else {
@@ -1241,7 +1232,8 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
   const unsigned gy = (unsigned)((s.c_dst + 32 * NT - 1) / (32 * NT));
   constexpr bool kCanHalf = NT != 4;
   const RowsGrid rg = rows_grid(a.n_dst, gy, a.k_vol * slabs, kCanHalf, tile_order != nullptr, tile_grid, pair_view,
-                                NT >= 3 ? 2 : 3, a.transpose_w, kCanHalf && !a.transpose_w);
+                                NT >= 3 || (sizeof(T) == 4 && S == 4 && !a.reduced && split_bf16_enabled()) ? 2 : 3, a.transpose_w,
+                                kCanHalf && !a.transpose_w);
   // Few tiles: column tiles of 32 put them on twice the CUs, as long as each still has one to itself.
   // A tile's rows are then gathered twice, by CUs that had nothing to do.  Against two workgroups
   // per 64-column tile and atomics / 64-column tiles with four groups: 64 -> 64 fp16 over 1 k voxels
@@ -1276,18 +1268,18 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (!(a.stream && hipStreamIsCapturing(a.stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone)) raw = 0;
   }
-  // fp32 forward in "tf32" mode: products in split bf16 (three 16-bit MFMAs instead of
-  // sixteen fp32 ones per product tile); needs whole 32-channel slabs
+  // fp32 tensors: products of bf16 parts, two to a value in "tf32" mode, else three (three or six 16-bit MFMAs instead
+  // of sixteen fp32 ones per product tile); needs whole 32-channel slabs
   constexpr bool kCanSplit = sizeof(T) == 4 && S == 4 && NT != 4;
-  const bool split = kCanSplit && a.reduced && !a.transpose_w && !a.prepacked && split_bf16_enabled();
-  if (kCanSplit && a.reduced && raw == 2 && split_bf16_enabled()) raw = 4;   // (the input gradient splits as it reads)
+  const bool split = kCanSplit && !a.transpose_w && !a.prepacked && split_bf16_enabled() && (a.reduced || NT != 3);
+  if (kCanSplit && raw == 2 && split_bf16_enabled()) raw = a.reduced ? 4 : NT != 3 ? 6 : 2;   // (the input gradient splits as it reads)
   const T *packed = raw ? (const T *)a.w : (const T *)a.prepacked;
   if (split) {
     const void *ws = nullptr;
-    int rc = pack_weights_bf3(a, false, &ws);
+    int rc = a.reduced ? pack_weights_parts<2>(a, false, &ws) : pack_weights_parts<3>(a, false, &ws);
     if (rc != FGMS_OK) return rc;
     packed = (const T *)ws;
-    raw = 3;
+    raw = a.reduced ? 3 : 5;
   } else if (!packed) {
     int rc = pack_weights<T>(a, S, &packed);
     if (rc != FGMS_OK) return rc;
@@ -1295,19 +1287,22 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
   const bool half_tiles = rg.half_tiles;
   if (rg.drop_table) tile_order = nullptr;
   constexpr int kHalfMT = kCanHalf ? 1 : 2;
-  constexpr size_t kGroup = rows_group_chunks<T, NT, S, kHalfMT>() * 16, kSums = rows_sum_chunks<NT, kHalfMT>() * 16;
+  const size_t kGroup = rows_group_chunks<T, NT, S, kHalfMT>(raw) * 16, kSums = rows_sum_chunks<NT, kHalfMT>() * 16;
   constexpr int kMaxGroups = NT == 3 ? 2 : 4;          // (four groups' sums of 96 columns do not fit LDS)
-  const int kg = !half_tiles ? 1 : rg.groups < kMaxGroups ? rg.groups : kMaxGroups;
-  size_t lds_rows = half_tiles ? kGroup * kg : s.lds_rows_bytes;
+  // (three parts and 64 columns: 50 KB a group, half of the groups)
+  const int kg = !half_tiles ? 1 : raw == 5 && NT == 2 ? (rg.groups + 1) / 2 : rg.groups < kMaxGroups ? rg.groups : kMaxGroups;
+  size_t lds_rows = half_tiles ? kGroup * kg : rows_group_chunks<T, NT, S, 2>(raw) * 16;
   if (kg > 1 && lds_rows < kGroup + kSums * (kg - 1)) lds_rows = kGroup + kSums * (kg - 1);
   const unsigned gx = rg.gx;
   if (gx == 0) return a.side.kind ? launch_side_job(a.side, a.stream) : FGMS_OK;
   constexpr bool kCanRaw = NT != 4;
-  constexpr int kRaw4 = kCanSplit ? 4 : 0, kRaw3 = kCanSplit ? 3 : 0, kRaw2 = kCanRaw ? 2 : 0, kRaw1 = kCanRaw && sizeof(T) == 2 ? 1 : 0;
-  // (raw is one of the five the type and the tile allow)
+  constexpr int kRaw6 = kCanSplit && NT != 3 ? 6 : 0, kRaw5 = kCanSplit && NT != 3 ? 5 : 0, kRaw4 = kCanSplit ? 4 : 0, kRaw3 = kCanSplit ? 3 : 0, kRaw2 = kCanRaw ? 2 : 0, kRaw1 = kCanRaw && sizeof(T) == 2 ? 1 : 0;
+  // (raw is one of those the type and the tile allow)
 #define FGMS_BY_RAW(MTv, KGv)                                                                                       \
   (RAGGED     ? gms_rows_kernel<T, NT, S, RAGGED ? kRaw1 : 0, MTv, KGv, RAGGED>                                     \
-   : raw == 4   ? gms_rows_kernel<T, NT, S, kRaw4, MTv, KGv>                                                          \
+   : raw == 6 ? gms_rows_kernel<T, NT, S, kRaw6, MTv, 1>                                                            \
+   : raw == 5 ? gms_rows_kernel<T, NT, S, kRaw5, MTv, KGv == 4 && NT == 2 ? 2 : KGv>                                \
+   : raw == 4 ? gms_rows_kernel<T, NT, S, kRaw4, MTv, KGv>                                                          \
    : raw == 3 ? gms_rows_kernel<T, NT, S, kRaw3, MTv, KGv>                                                          \
    : raw == 2 ? gms_rows_kernel<T, NT, S, kRaw2, MTv, KGv>                                                          \
    : raw == 1 ? gms_rows_kernel<T, NT, S, kRaw1, MTv, KGv>                                                          \
@@ -1327,7 +1322,7 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
   const int part_stages = rg.gz > 1 ? rg.part_stages : 0;
   const unsigned gz = rg.gz;
   {
-    ProfileScope prof(pair_view ? (a.transpose_w ? "gms_rows_kernel(dgrad, pair view)" : "gms_rows_kernel(fwd, pair view)") :raw == 4   ? "gms_rows_kernel(dgrad, bf16x3)"
+    ProfileScope prof(pair_view ? (a.transpose_w ? "gms_rows_kernel(dgrad, pair view)" : "gms_rows_kernel(fwd, pair view)") : raw == 4 ? "gms_rows_kernel(dgrad, bf16x3)"
                       : raw == 3 ? "gms_rows_kernel(fwd, bf16x3)"
                       : a.transpose_w ? "gms_rows_kernel(dgrad)" : "gms_rows_kernel(fwd)",
                       a.stream);
@@ -1356,7 +1351,7 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
 // (2 waves per SIMD where the weight gradient's tile is 128 x 128: its 64 accumulators per lane and
 // the rows in flight spill at 3.  128 -> 128 over 40k voxels, forward and backward: tf32 mode 477 -> 327 us.)
 template <typename T, int NT, int S, int BI, int BJ, int RAWD, int MT = 2, bool RAGGED = false>
-__global__ __launch_bounds__(kThreads, NT >= 3 || BI * BJ == 16 || ((BI == 3 || BJ == 3) && BI * BJ >= 6) ? 2 : 3) void bwd_fused_kernel(
+__global__ __launch_bounds__(kThreads, NT >= 3 || RAWD == 6 || BI * BJ == 16 || ((BI == 3 || BJ == 3) && BI * BJ >= 6) ? 2 : 3) void bwd_fused_kernel(
     const T *__restrict__ gout, const T *__restrict__ w, T *__restrict__ gin,
     const int32_t *__restrict__ nbr, const unsigned long long *__restrict__ block_masks,
     const int32_t *__restrict__ perm, const int32_t *__restrict__ tile_order, int n_in, int k_vol,
@@ -1379,7 +1374,7 @@ __global__ __launch_bounds__(kThreads, NT >= 3 || BI * BJ == 16 || ((BI == 3 || 
   } else {
     const int j = blockIdx.x - rows_total;
     if constexpr (BI <= 3 && BJ <= 3)
-      wgrad_wave_body<T, BI, BJ, RAWD == 4, RAGGED>(in, gout, gw32, kpos, imap, omap, k_vol, c_in, c_out, smap,
+      wgrad_wave_body<T, BI, BJ, split_parts_of(RAWD), RAGGED>(in, gout, gw32, kpos, imap, omap, k_vol, c_in, c_out, smap,
                                             j % wgrad_x, j / wgrad_x, in_bytes, gout_bytes);
     else
       wgrad_wg_body<T, BI, BJ, RAWD == 4>(in, gout, gw32, kpos, imap, omap, k_vol, c_in, c_out, smap,
@@ -1401,12 +1396,10 @@ int launch_fused(const GmsArgs &d, const Shape &s, const Plan *p, const WgradArg
   const unsigned row_y = (unsigned)((s.c_dst + 32 * NT - 1) / (32 * NT));
   constexpr bool kCanHalf = NT != 4;
   const RowsGrid rg = rows_grid(d.n_dst, row_y, d.k_vol * slabs, kCanHalf, p->tile_in != nullptr, p->tile_grid_in,
-                                false, NT >= 3 ? 2 : 3, true, false);
+                                false, NT >= 3 || g.split == 3 ? 2 : 3, true, false);
   const unsigned row_x = (rg.gx + 7) / 8 * 8;
   const int part_stages = rg.part_stages;
   const unsigned row_z = rg.gz;
-  size_t lds = g.lds;
-  if (lds < s.lds_rows_bytes) lds = s.lds_rows_bytes;
   // what the launch adds to with atomics starts from zero: shared tiles of the input gradient, a
   // weight gradient summed in the caller's fp32 tensor
   const bool zero_gin = d.overwrite && rg.gz > 1, zero_gw = w.overwrite && (void *)acc32 == w.gw;
@@ -1415,18 +1408,24 @@ int launch_fused(const GmsArgs &d, const Shape &s, const Plan *p, const WgradArg
                                         zero_gw ? (size_t)w.k_vol * w.c_in * w.c_out * sizeof(float) : 0, d.stream);
     if (rc != FGMS_OK) return rc;
   }
-  // RAWD: how the input gradient reads the weights (2: as they lie; 4: also split into bf16
-  // pairs, for fp32 tensors whose caller allows tf32 precision)
-  constexpr bool kCanSplit = sizeof(T) == 4 && S == 4 && NT != 4;
-  const bool split = kCanSplit && d.reduced && split_bf16_enabled() && g.split;
+  // RAWD: how the input gradient reads the weights (2: as they lie; 4, 6: also split into bf16
+  // parts, for fp32 tensors)
+  constexpr bool kCanSplit = sizeof(T) == 4 && S == 4 && NT != 4, kCan3 = kCanSplit && BI <= 2 && BJ <= 2;
+  const int raw = kCan3 && g.split == 3 ? 6 : kCanSplit && g.split == 2 ? 4 : 2;
   constexpr int kHalfMT = kCanHalf ? 1 : 2;
-  auto kern = rg.half_tiles ? (split ? bwd_fused_kernel<T, NT, S, BI, BJ, kCanSplit ? 4 : 2, kHalfMT, RAGGED>
-                                     : bwd_fused_kernel<T, NT, S, BI, BJ, 2, kHalfMT, RAGGED>)
-              : split       ? bwd_fused_kernel<T, NT, S, BI, BJ, kCanSplit ? 4 : 2, 2, RAGGED>
+  constexpr int kRaw4 = kCanSplit ? 4 : 2, kRaw6 = kCan3 ? 6 : 2;
+  auto kern = rg.half_tiles ? (raw == 6 ? bwd_fused_kernel<T, NT, S, BI, BJ, kRaw6, kHalfMT, RAGGED>
+                               : raw == 4 ? bwd_fused_kernel<T, NT, S, BI, BJ, kRaw4, kHalfMT, RAGGED>
+                                          : bwd_fused_kernel<T, NT, S, BI, BJ, 2, kHalfMT, RAGGED>)
+              : raw == 6    ? bwd_fused_kernel<T, NT, S, BI, BJ, kRaw6, 2, RAGGED>
+              : raw == 4    ? bwd_fused_kernel<T, NT, S, BI, BJ, kRaw4, 2, RAGGED>
                             : bwd_fused_kernel<T, NT, S, BI, BJ, 2, 2, RAGGED>;
+  size_t lds = g.lds;
+  const size_t lds_rows = rg.half_tiles ? rows_group_chunks<T, NT, S, kHalfMT>(raw) * 16 : rows_group_chunks<T, NT, S, 2>(raw) * 16;
+  if (lds < lds_rows) lds = lds_rows;
   { const int rc_lds = allow_dynamic_lds(reinterpret_cast<const void *>(kern), (size_t)lds); if (rc_lds != FGMS_OK) return rc_lds; }
   {
-    ProfileScope prof(split ? "bwd_fused_kernel(bf16x3)" : "bwd_fused_kernel", d.stream);
+    ProfileScope prof(raw == 4 ? "bwd_fused_kernel(bf16x3)" : "bwd_fused_kernel", d.stream);
     SideJob check{};
     (void)plan_take_check(p, &check);
     kern<<<row_x * row_y * row_z + (unsigned)(g.tiles * g.ty) + (unsigned)check.blocks, kThreads, lds, d.stream>>>(

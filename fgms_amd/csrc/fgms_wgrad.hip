@@ -53,8 +53,8 @@ __global__ __launch_bounds__(kThreads) void wgrad_kernel(
 }
 
 // The per-wave variant (wgrad_wave_body) in a launch of its own.
-template <typename T, int BI, int BJ, bool SPLIT>
-__global__ __launch_bounds__(kThreads, BI * BJ >= 6 ? 2 : 3) void wgrad_wave_kernel(
+template <typename T, int BI, int BJ, int SPLIT>
+__global__ __launch_bounds__(kThreads, BI * BJ >= 6 || SPLIT == 3 ? 2 : 3) void wgrad_wave_kernel(
     const T *__restrict__ in, const T *__restrict__ gout, float *__restrict__ gw32,
     const int32_t *__restrict__ kpos, const int32_t *__restrict__ imap,
     const int32_t *__restrict__ omap, int k_vol, int c_in, int c_out, SliceMap smap, SideJob side,
@@ -269,6 +269,11 @@ void tile_blocks(const WgradArgs &a, bool shares_grid, int *bi, int *bj) {
   *bj = blocks_of(a.c_out, three);
   if (*bi == 3 && *bj == 4) *bj = 2;     // (96 channels: the per-wave body)
   if (*bj == 3 && *bi == 4) *bi = 2;
+  // (fp32 in three parts: the per-wave body only)
+  if (a.dtype != FGMS_F16 && !a.reduced && split_bf16_enabled()) {
+    if (*bi > 2) *bi = 2;
+    if (*bj > 2) *bj = 2;
+  }
   if (!shares_grid && a.dtype == FGMS_F16 && *bi * *bj == 16) {
     *bi = 2;
     *bj = 2;
@@ -331,10 +336,12 @@ int launch_wave(const WgradArgs &a, float *acc32) {
   int rc = wgrad_geometry(a, &g);
   if (rc != FGMS_OK) return rc;
   constexpr bool kCanSplit = sizeof(T) == 4;
-  auto kern = g.split ? wgrad_wave_kernel<T, BI, BJ, kCanSplit> : wgrad_wave_kernel<T, BI, BJ, false>;
+  auto kern = g.split == 3   ? wgrad_wave_kernel<T, BI, BJ, kCanSplit ? 3 : 0>
+              : g.split == 2 ? wgrad_wave_kernel<T, BI, BJ, kCanSplit ? 2 : 0>
+                             : wgrad_wave_kernel<T, BI, BJ, 0>;
   { const int rc_lds = allow_dynamic_lds(reinterpret_cast<const void *>(kern), (size_t)g.lds); if (rc_lds != FGMS_OK) return rc_lds; }
   {
-    ProfileScope prof(g.split ? "wgrad_wave_kernel(bf16x3)" : "wgrad_wave_kernel", a.stream);
+    ProfileScope prof(g.split == 2 ? "wgrad_wave_kernel(bf16x3)" : "wgrad_wave_kernel", a.stream);
     kern<<<dim3((unsigned)g.tiles + (unsigned)a.side.blocks, (unsigned)g.ty), kThreads, g.lds, a.stream>>>(
         (const T *)a.in, (const T *)a.gout, acc32, a.kpos, a.imap, a.omap, a.k_vol, a.c_in,
         a.c_out, g.smap, a.side, (unsigned)((size_t)a.n_in * a.c_in * sizeof(T)),
@@ -451,9 +458,9 @@ static void wave_geometry(const WgradArgs &a, WgradGeometry *g) {
   g->wave = true;
   g->smap = choose_slices(a, g->ty, sp, (int64_t)num_cus() * 6);
   g->tiles = (int64_t)g->smap.slices * a.k_vol;
-  // fp32 tensors whose caller allows tf32 precision: four 16-bit tiles per wave instead
-  g->split = !f16 && a.reduced && split_bf16_enabled();
-  const size_t lds = (g->split ? 4 * (size_t)sp * 2 * ((bi * 32 + 16) + (bj * 32 + 16)) * 2
+  // fp32 tensors: 16-bit tiles of every part instead
+  g->split = f16 || !split_bf16_enabled() ? 0 : a.reduced ? 2 : 3;
+  const size_t lds = (g->split ? 4 * (size_t)sp * g->split * ((bi * 32 + 16) + (bj * 32 + 16)) * 2
                                : 4 * (size_t)sp * ((bi * 32 + pad) + (bj * 32 + pad)) * (f16 ? 2 : 4))
                      + 4 * 64 * sizeof(int);                           // + the waves' index exchange
   const size_t red = 3 * (size_t)(bi * bj > 4 ? 1 : bi) * bj * 16 * 64 * sizeof(float);     // the partial tiles' exchange
@@ -494,7 +501,7 @@ int wgrad_geometry(const WgradArgs &a, WgradGeometry *g, bool shares_grid) {
     g->smap = choose_slices(a, g->ty, sp, (int64_t)num_cus() * 4);
     g->tiles = (int64_t)g->smap.slices * a.k_vol;
   }
-  g->split = !f16 && a.reduced && split_bf16_enabled();
+  g->split = !f16 && a.reduced && split_bf16_enabled() ? 2 : 0;
   g->lds = g->split ? 2 * (size_t)sp * 2 * ((bi * 32 + 16) + (bj * 32 + 16)) * 2
                     : 2 * (size_t)sp * ((bi * 32 + pad) + (bj * 32 + pad)) * esz;
   return FGMS_OK;

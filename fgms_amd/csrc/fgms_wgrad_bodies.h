@@ -99,27 +99,14 @@ __device__ __forceinline__ bool locate_slice(const int32_t *__restrict__ kpos, c
   return count > 0;
 }
 
-// Split staging (fp32 rows whose caller allows tf32 precision): chunk c (4 fp32 values) of a
-// staged row becomes 4 hi and 4 lo bf16 values in two 16-bit tiles laid out like the fp16
-// path's.  Lane pairs hold neighbouring chunks and exchange halves, so the even lane writes
-// 8 hi values and the odd one 8 lo values, 16 bytes each.
-__device__ __forceinline__ void store_split_chunk(__half *hi_tile, __half *lo_tile, int ld, int row, int c,
-                                                  const int4v &raw, bool valid, int lane) {
-  const bool odd = lane & 1;
-  const float4v v = valid ? __builtin_bit_cast(float4v, raw) : float4v{0.f, 0.f, 0.f, 0.f};
-  bf16x4 hi, lo;
+// Split staging (fp32 rows): chunk c (4 fp32 values) of a staged row becomes 4 bf16 values in each of P
+// 16-bit tiles laid out like the fp16 path's, `stride` halfs apart.
+template <int P>
+__device__ __forceinline__ void store_split_chunk(__half *tiles, int stride, int ld, int row, int c, const int4v &raw, bool valid) {
+  int2v part[P];
+  split_parts<P>(valid ? __builtin_bit_cast(float4v, raw) : float4v{0.f, 0.f, 0.f, 0.f}, part);
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    __bf16 h, l;
-    split_bf16(v[q], h, l);
-    hi[q] = h;
-    lo[q] = l;
-  }
-  const int2v h2 = __builtin_bit_cast(int2v, hi), l2 = __builtin_bit_cast(int2v, lo);
-  const int got0 = __builtin_bit_cast(int, swap_with_neighbour(__builtin_bit_cast(float, odd ? h2[0] : l2[0])));
-  const int got1 = __builtin_bit_cast(int, swap_with_neighbour(__builtin_bit_cast(float, odd ? h2[1] : l2[1])));
-  if (odd) *reinterpret_cast<int4v *>(lo_tile + row * ld + (c - 1) * 4) = int4v{got0, got1, l2[0], l2[1]};
-  else *reinterpret_cast<int4v *>(hi_tile + row * ld + c * 4) = int4v{h2[0], h2[1], got0, got1};
+  for (int q = 0; q < P; ++q) *reinterpret_cast<int2v *>(tiles + q * stride + row * ld + c * 4) = part[q];
 }
 
 // Variant for dW tiles up to 64 x 64: every wave stages its own pairs in its own
@@ -133,13 +120,12 @@ template <> struct WTW<__half> { static constexpr int stage_pairs = 32; };
 template <> struct WTW<float> { static constexpr int stage_pairs = 16; };
 
 // (block_x, block_y): the workgroup's place in a grid of cells x tiles of dW[k]; 256 threads.
-// SPLIT (fp32 tensors whose caller allows tf32 precision): the staged rows are split into
-// bf16 pairs, x = hi + lo, on their way to LDS -- four 16-bit tiles per wave, laid out like
-// the fp16 path's two -- and a product is three bf16 MFMAs, hi*hi + hi*lo + lo*hi, fed
-// through the same transposing LDS reads as fp16.
+// SPLIT (fp32 tensors): the staged rows are split into so many bf16 parts on their way to LDS -- 16-bit tiles
+// of every part per wave, laid out like the fp16 path's two -- and a product is three (two parts, where the
+// caller allows tf32 precision) or six bf16 MFMAs, fed through the same transposing LDS reads as fp16.
 // RAGGED (fp16): the tile's channels from c_in / c_out on do not exist; they are loaded from outside the
 // buffers, as zeros, and not flushed.
-template <typename T, int BI, int BJ, bool SPLIT = false, bool RAGGED = false>
+template <typename T, int BI, int BJ, int SPLIT = 0, bool RAGGED = false>
 __device__ __forceinline__ void wgrad_wave_body(
     const T *__restrict__ in, const T *__restrict__ gout, float *__restrict__ gw32,
     const int32_t *__restrict__ kpos, const int32_t *__restrict__ imap,
@@ -170,8 +156,8 @@ __device__ __forceinline__ void wgrad_wave_body(
   T *g = x + SP * LDI;
   // SPLIT: 16-bit tiles with the fp16 path's row padding (32 bytes)
   constexpr int LDIh = CI + 16, LDOh = CO + 16;
-  __half *xh = reinterpret_cast<__half *>(lds) + (size_t)wave * SP * 2 * (LDIh + LDOh);
-  __half *xl = xh + SP * LDIh, *gh = xl + SP * LDIh, *gl = gh + SP * LDOh;
+  constexpr int P = SPLIT ? SPLIT : 1;
+  __half *xs = reinterpret_cast<__half *>(lds) + (size_t)wave * SP * P * (LDIh + LDOh), *gs = xs + P * SP * LDIh;
   static_assert(!SPLIT || (sizeof(T) == 4 && SP == 16), "split tiles: fp32 rows, one 16-pair MFMA step a stage");
 
   float16v acc[BI][BJ];
@@ -181,6 +167,13 @@ __device__ __forceinline__ void wgrad_wave_body(
     for (int b = 0; b < BJ; ++b)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
+  float16v low[P == 3 ? BI : 1][P == 3 ? BJ : 1];      // three parts: the small products (mma_parts)
+  if constexpr (P == 3) {
+#pragma unroll
+    for (int a = 0; a < BI; ++a)
+#pragma unroll
+      for (int b = 0; b < BJ; ++b) low[a][b] = acc[a][b];
+  }
 
   const int nstages = (count + SP - 1) / SP;
   int xi[NX], gi[NG];        // gather rows of the next stage to load
@@ -274,7 +267,7 @@ __device__ __forceinline__ void wgrad_wave_body(
     for (int i = 0; i < NX; ++i) {
       const int e = lane + 64 * i;
       if constexpr (SPLIT)
-        store_split_chunk(xh, xl, LDIh, e / NCI, e % NCI, xr[i], st * SP + e / NCI < count, lane);
+        store_split_chunk<P>(xs, SP * LDIh, LDIh, e / NCI, e % NCI, xr[i], st * SP + e / NCI < count);
       else if constexpr (kBufW)
         *reinterpret_cast<int4v *>(x + x_row(i) * LDI + ((x_chunk(i) ^ (CI == 64 ? ((x_row(i) >> 1) & 1) * 4 : 0)) * E)) = xr[i];
       else
@@ -285,7 +278,7 @@ __device__ __forceinline__ void wgrad_wave_body(
     for (int i = 0; i < NG; ++i) {
       const int e = lane + 64 * i;
       if constexpr (SPLIT)
-        store_split_chunk(gh, gl, LDOh, e / NCO, e % NCO, gr[i], st * SP + e / NCO < count, lane);
+        store_split_chunk<P>(gs, SP * LDOh, LDOh, e / NCO, e % NCO, gr[i], st * SP + e / NCO < count);
       else if constexpr (kBufW)
         *reinterpret_cast<int4v *>(g + g_row(i) * LDO + ((g_chunk(i) ^ (CO == 64 ? ((g_row(i) >> 1) & 1) * 4 : 0)) * E)) = gr[i];
       else
@@ -312,25 +305,18 @@ __device__ __forceinline__ void wgrad_wave_body(
     load_idx(st + 8);                    //  the wait for the rows then leaves the indices in flight)
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (SPLIT) {
-      bf16x8 ah[BI], al[BI], bh[BJ], bl[BJ];
+      bf16x8 a[BI][P], b[BJ][P];
 #pragma unroll
-      for (int ti = 0; ti < BI; ++ti) {
-        ah[ti] = __builtin_bit_cast(bf16x8, tr_frag(xh, LDIh, 0, ti * 32, lane));
-        al[ti] = __builtin_bit_cast(bf16x8, tr_frag(xl, LDIh, 0, ti * 32, lane));
-      }
+      for (int q = 0; q < P; ++q) {
 #pragma unroll
-      for (int tj = 0; tj < BJ; ++tj) {
-        bh[tj] = __builtin_bit_cast(bf16x8, tr_frag(gh, LDOh, 0, tj * 32, lane));
-        bl[tj] = __builtin_bit_cast(bf16x8, tr_frag(gl, LDOh, 0, tj * 32, lane));
+        for (int ti = 0; ti < BI; ++ti) a[ti][q] = __builtin_bit_cast(bf16x8, tr_frag(xs + q * SP * LDIh, LDIh, 0, ti * 32, lane));
+#pragma unroll
+        for (int tj = 0; tj < BJ; ++tj) b[tj][q] = __builtin_bit_cast(bf16x8, tr_frag(gs + q * SP * LDOh, LDOh, 0, tj * 32, lane));
       }
 #pragma unroll
       for (int ti = 0; ti < BI; ++ti)
 #pragma unroll
-        for (int tj = 0; tj < BJ; ++tj) {
-          acc[ti][tj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[ti], bh[tj], acc[ti][tj], 0, 0, 0);
-          acc[ti][tj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[ti], bl[tj], acc[ti][tj], 0, 0, 0);
-          acc[ti][tj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[ti], bh[tj], acc[ti][tj], 0, 0, 0);
-        }
+        for (int tj = 0; tj < BJ; ++tj) mma_parts<P>(acc[ti][tj], low[P == 3 ? ti : 0][P == 3 ? tj : 0], a[ti], b[tj]);
     } else if constexpr (kBufW) {
       // (tiles of more than 64 x 64: one k-step's fragments at a time, for want of registers)
       constexpr int KS = SP / KP, KF = BI * BJ > 4 ? 1 : KS;
@@ -390,6 +376,14 @@ __device__ __forceinline__ void wgrad_wave_body(
     st += 4;
   }
 
+  if constexpr (P == 3) {
+#pragma unroll
+    for (int a = 0; a < BI; ++a)
+#pragma unroll
+      for (int b = 0; b < BJ; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[a][b][r] += low[a][b][r];
+  }
   // Sum the four waves' tiles through LDS and flush.  Every wave ends up with a quarter of the
   // summed tile (accumulator registers q * R / 4 ... of the R a lane holds) and
   // flushes that: one barrier, and the atomic updates of the tile issued by four waves instead
@@ -443,7 +437,7 @@ template <int BI, int BJ> struct WaveGrid {
 // The workgroup-level weight-gradient kernel body (dW tiles wider than 64 x 64): the four
 // waves share the staged pairs and split the tile.  (block_x, block_y): the workgroup's
 // place in a grid of cells x tiles of dW[k]; 256 threads.
-// SPLIT: as in wgrad_wave_body (fp32 rows staged as hi / lo bf16 tiles, three bf16 MFMAs a product).
+// SPLIT: as in wgrad_wave_body with two parts.
 template <typename T, int BI, int BJ, bool SPLIT = false>
 __device__ __forceinline__ void wgrad_wg_body(
     const T *__restrict__ in, const T *__restrict__ gout, float *__restrict__ gw32,
@@ -525,7 +519,7 @@ __device__ __forceinline__ void wgrad_wg_body(
       const int e = tid + kThreads * i;
       if constexpr (SPLIT) {
         __half *xh = stage0h + buf * kBufHalfs;
-        store_split_chunk(xh, xh + SP * LDIh, LDIh, e / NCI, e % NCI, xr[i], st * SP + e / NCI < count, lane);
+        store_split_chunk<2>(xh, SP * LDIh, LDIh, e / NCI, e % NCI, xr[i], st * SP + e / NCI < count);
       } else {
         *reinterpret_cast<int4v *>(stage0 + buf * kBufElems + (e / NCI) * LDI + (e % NCI) * E) =
             st * SP + e / NCI < count ? xr[i] : int4v{0, 0, 0, 0};
@@ -536,7 +530,7 @@ __device__ __forceinline__ void wgrad_wg_body(
       const int e = tid + kThreads * i;
       if constexpr (SPLIT) {
         __half *gh = stage0h + buf * kBufHalfs + SP * 2 * LDIh;
-        store_split_chunk(gh, gh + SP * LDOh, LDOh, e / NCO, e % NCO, gr[i], st * SP + e / NCO < count, lane);
+        store_split_chunk<2>(gh, SP * LDOh, LDOh, e / NCO, e % NCO, gr[i], st * SP + e / NCO < count);
       } else {
         *reinterpret_cast<int4v *>(stage0 + buf * kBufElems + SP * LDI + (e / NCO) * LDO + (e % NCO) * E) =
             st * SP + e / NCO < count ? gr[i] : int4v{0, 0, 0, 0};
@@ -674,7 +668,7 @@ struct WgradGeometry {
   int ty;          // grid y: BI*32 x BJ*32 tiles of dW[k]
   int bi, bj;
   bool wave;       // wgrad_wave_body, else wgrad_wg_body
-  bool split;      // wgrad_wave_body in split bf16
+  int split;       // bf16 parts of an fp32 value (0: fp32 MFMAs)
   size_t lds;      // dynamic LDS
 };
 // shares_grid: the launch also holds the input gradient's workgroups.
