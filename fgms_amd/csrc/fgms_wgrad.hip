@@ -451,7 +451,7 @@ double vector_alu_wgrad_us(const WgradArgs &a) {
 }
 
 // Grid and LDS of the per-wave body for g's tile.
-static void wave_geometry(const WgradArgs &a, WgradGeometry *g) {
+static void wave_geometry(const WgradArgs &a, WgradGeometry *g, bool shares_grid) {
   const bool f16 = a.dtype == FGMS_F16;
   const int bi = g->bi, bj = g->bj, pad = f16 ? 0 : WT<float>::pad;
   const int sp = f16 ? WTW<__half>::stage_pairs : WTW<float>::stage_pairs;
@@ -459,7 +459,12 @@ static void wave_geometry(const WgradArgs &a, WgradGeometry *g) {
   g->smap = choose_slices(a, g->ty, sp, (int64_t)num_cus() * 6);
   g->tiles = (int64_t)g->smap.slices * a.k_vol;
   // fp32 tensors: 16-bit tiles of every part instead
-  g->split = f16 || !split_bf16_enabled() ? 0 : a.reduced ? 2 : 3;
+  // (Three parts in a launch of tiles of one or two blocks only where each cell walks many pairs: a walk of few is mostly
+  // the splits and the wait for its first rows.  fp32 MFMAs / three parts: 32 x 32 over 20 k scattered voxels 22.8 / 25.2 us,
+  // 60 k LiDAR ones 35.8 / 37.7, indoor 100 k 41.6 / 39.3; 32 x 64 over 10 k LiDAR voxels 20.8 / 22.3, 60 k 59.5 / 58.4,
+  // indoor 30 k 35.4 / 33.1, 100 k 79.8 / 68.3; 96 x 64 over 164 k pairs 47 / 40.)
+  const bool few = !shares_grid && bi * bj <= 2 && (double)a.n_pairs * g->ty * (bi * bj * bi * bj) < 8e5;
+  g->split = f16 || !split_bf16_enabled() ? 0 : a.reduced ? 2 : few ? 0 : 3;
   const size_t lds = (g->split ? 4 * (size_t)sp * g->split * ((bi * 32 + 16) + (bj * 32 + 16)) * 2
                                : 4 * (size_t)sp * ((bi * 32 + pad) + (bj * 32 + pad)) * (f16 ? 2 : 4))
                      + 4 * 64 * sizeof(int);                           // + the waves' index exchange
@@ -482,7 +487,7 @@ int wgrad_geometry(const WgradArgs &a, WgradGeometry *g, bool shares_grid) {
   g->bj = bj;
   g->ty = (a.c_in / (32 * bi)) * (a.c_out / (32 * bj));
   if (bi <= 3 && bj <= 3) {
-    wave_geometry(a, g);
+    wave_geometry(a, g, shares_grid);
     return FGMS_OK;
   }
   const int sp = f16 ? WT<__half>::stage_pairs : WT<float>::stage_pairs;
@@ -515,7 +520,7 @@ bool ragged_wgrad_geometry(const WgradArgs &a, int bi, int bj, WgradGeometry *g)
   g->bi = bi;
   g->bj = bj;
   g->ty = ((a.c_in + 32 * bi - 1) / (32 * bi)) * ((a.c_out + 32 * bj - 1) / (32 * bj));
-  wave_geometry(a, g);
+  wave_geometry(a, g, true);
   return true;
 }
 
