@@ -593,7 +593,23 @@ double padded_us(const GmsArgs &p, const Plan *plan) {
       return 20 + 1.5 * slabs * (1 + wide) + 1e-6 * pairs_of(p, plan) * (p.dense_k >= 0 ? 2.0 * c_dst : 3.4 * c_dst + 0.4 * c_src);
   }
 }
+// The same over the masked tiles (fp32: no copies, nothing to crop).  Forward over 4 k dense voxels, measured (estimated):
+// 24 -> 32 21.0 us (20.4), tf32 mode 18.1 (17.4); 48 -> 48 33.2 (32.3) and 27.2 (26.3); 96 -> 24 44.1 (44.1) and 35.8 (35.2);
+// 48 -> 48 over 30 k 49.5 (49).  On the vector ALUs 48 -> 48 over 4 k 21 us, 96 -> 24 27.  Both gradients, the weights'
+// hidden behind the tiles: 24 -> 32 19.5 us (19.3), 48 -> 48 39 (39.8), 48 -> 96 56 (55); tf32 mode 18.7, 35.2, 46.5 (18.7, 36.2, 49.8).
+double masked_us(const GmsArgs &a) {
+  const int c_src = a.transpose_w ? a.c_out : a.c_in, c_dst = a.transpose_w ? a.c_in : a.c_out;
+  const double stages = (double)a.k_vol * ((c_src + 31) / 32), tiles_per_cu = (double)((a.n_dst + 127) / 128 * ((c_dst + 31) / 32)) / num_cus();
+  if (a.transpose_w) {
+    const bool pairs_of_tiles = (c_dst + 31) / 32 % 2 == 0;     // (two column tiles to a workgroup)
+    const double stage = (a.reduced ? 0.36 : 0.38) * (!pairs_of_tiles ? 1 : a.reduced ? 1.4 : 1.5), per_cu = tiles_per_cu / (pairs_of_tiles ? 2 : 1);
+    return 9 + stage * stages * (1 + 1.45 * std::max(0.0, per_cu - 0.43));
+  }
+  return 8.5 + (a.reduced ? 0.33 : 0.44) * stages * (tiles_per_cu <= 1 ? 1 : 1.25 + 0.25 * tiles_per_cu);
+}
+bool takes_ragged(const GmsArgs &a, const Plan *plan);
 bool padding_pays(const GmsArgs &a, const Plan *plan, int c_in, int c_out) {
+  if (a.dtype != FGMS_F16 && takes_ragged(a, plan) && ragged_gms_supported(a, plan)) return masked_us(a) < vector_alu_us(a, plan);
   // (fp16 adds on the vector ALUs cost ten times as much: 32 -> 20 over 500 voxels 17 us over copies, 24 without.
   // The copies' fp32 kernels mostly do without atomics: a near tie goes to them.)
   return a.dtype == FGMS_F16 || padded_us(with_channels(a, c_in, c_out), plan) < 1.05 * vector_alu_us(a, plan);
@@ -620,6 +636,18 @@ bool takes_ragged(const GmsArgs &a, const Plan *plan) {
   return g_policy == 0 && plan && a.n_pairs > 0 && a.dense_k < 0 && !narrow_gms_supported(a, plan) && !small_gms_supported(a, plan) && !sparse_rows(a, plan);
 }
 
+// fp32 counts that are no multiple of 32: over the masked tiles where another matrix kernel takes them as they are or the
+// vector ALUs are slower.  (Not for 16 channels forward in fp32: half of every slab of 32 is empty, and six products
+// each make it 61 us for 16 -> 64 over 120 k voxels where slabs of 16 on fp32 MFMAs took 47; in tf32 mode 36.)
+bool ragged_pays(const GmsArgs &a, const Plan *plan) {
+  int pi, po;
+  if (a.dtype == FGMS_F16) return true;
+  const size_t parts = (size_t)a.k_vol * up_to_32(a.c_in) * up_to_32(a.c_out) * (a.reduced ? 4 : 6);
+  if (parts > 0xfffffff0u || !workspaces_fit(a.stream, {{0, parts}})) return false;     // (the re-laid weights)
+  if (tuned_gms(a, plan)) return a.reduced || a.transpose_w || a.c_in > 16;
+  return padded_gms_channels(a, plan, &pi, &po);
+}
+
 // A pass over all offsets: one walk for plans of up to 64 offsets (or none), one per group of 64
 // offsets for larger kernels (the groups' results add up in the destination rows).
 int run_gms_padded(const GmsArgs &a, const Plan *plan, int c_in, int c_out, bool *done);
@@ -629,7 +657,7 @@ int run_gms_padded(const GmsArgs &a, const Plan *plan, int c_in, int c_out, bool
 // a forward and a backward call, 125 -> 98 us.)
 bool centre_rides(const GmsArgs &a, const Plan *plan) {
   if (!plan || a.n_pairs == 0 || !plan->groups.empty() || !plan->centre_line || a.centre - 1 != a.k_vol / 2 || a.n_src != a.n_dst) return false;
-  if (takes_ragged(a, plan) && ragged_gms_supported(a, plan)) return true;
+  if (takes_ragged(a, plan) && ragged_gms_supported(a, plan) && ragged_pays(a, plan)) return true;
   int pi, po;
   return route_of(padded_gms_channels(a, plan, &pi, &po) ? with_channels(a, pi, po) : a, plan) == Route::kRows;
 }
@@ -652,7 +680,7 @@ int run_gms(GmsArgs a, const Plan *plan) {
     a.overwrite = false;
   }
   int pi, po;
-  if (takes_ragged(a, plan) && ragged_gms_supported(a, plan)) {
+  if (takes_ragged(a, plan) && ragged_gms_supported(a, plan) && ragged_pays(a, plan)) {
     plan_touch(plan, a.stream);
     return launch_ragged_gms(a, plan);
   }
@@ -853,6 +881,19 @@ bool together_pays(const GmsArgs &d, const Plan *p, const WgradArgs &w, const Gm
   return std::max(in_us, w_us) + 0.4 * std::min(in_us, w_us) < 1.1 * (in_alone + std::min(w_us, vector_alu_wgrad_us(w)));
 }
 
+// fp32: both gradients over the masked tiles, or each on its better side?  The weights' hide behind the tiles; on their own they
+// take three launches and what the copies' kernel adds (48 x 48: 15 us over 9 k pairs, 23 over 39 k).  Masked / apart:
+// 48 -> 48 over 2 k voxels 41 / 32 us, 3 k 41 / 37, 4 k 39 / 44; 48 -> 96 over 4 k 56 / 50; 24 -> 32 over 1 k 19.5 / 28.  Maps too thin
+// for the output-stationary kernel at the copies' channel counts stay with the copies (64 -> 48 over 1 k 40 / 32).
+bool masked_bwd_pays(const GmsArgs &d, const Plan *p, const WgradArgs &w) {
+  if (d.dtype == FGMS_F16 || (tuned_gms(d, p) && mfma_wgrad_supported(w))) return true;
+  const GmsArgs pd = with_channels(d, up_to_32(d.c_in), up_to_32(d.c_out));
+  if (sparse_rows(pd, p)) return false;
+  const double in_alone = tuned_gms(d, p) ? padded_us(d, p) : std::min(padded_us(pd, p), vector_alu_us(d, p));
+  const double cells = (double)(pd.c_in / 32) * (pd.c_out / 32), w_alone = 12.3 + 1e-3 * (double)w.n_pairs * (0.045 + 0.05 * std::min(cells, 4.0));
+  return masked_us(d) < 0.88 * (in_alone + w_alone);     // (vector_alu_us is a sixth high on maps this small)
+}
+
 // Widened channels for a backward pass one of whose gradients no tuned kernel takes as it is: the
 // narrow layers' kernels up to 16 x 64, else multiples of 32 for both, which the one-grid launch takes.
 bool padded_bwd_channels(const GmsArgs &d, const Plan *p, const WgradArgs &w, int *c_in, int *c_out) {
@@ -981,7 +1022,7 @@ int backward(const void *out_feats_grad, const void *in_feats, const void *kerne
   if (!want_kernel) return want_in ? run_gms(d, p) : FGMS_OK;
   if (!want_in) return run_wgrad(w);
   int pi, po;
-  if (takes_ragged(d, p)) {
+  if (takes_ragged(d, p) && masked_bwd_pays(d, p, w)) {
     bool done = false;
     plan_touch(p, stream);
     rc = launch_ragged_bwd(d, p, w, &done);

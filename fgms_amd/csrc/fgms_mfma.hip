@@ -277,11 +277,12 @@ __device__ __forceinline__ void mma_slab_parts(float16v (&acc)[MT][NT], float16v
 //   ((((k * slabs + slab) * 2 + s) * nts + nt) * P + part) * 64 + lane
 // holds the 8 values op(W[k])[slab*32 + s*16 + (lane/32)*8 + 0..7][nt*32 + lane%32] of that part.
 // One thread per P chunks.
+// (Channels that fill no whole tile: zeros behind them.)
 template <int P>
 __global__ void pack_weights_parts_kernel(const float *__restrict__ w, int4v *__restrict__ packed,
                                           int k_vol, int c_in, int c_out, bool transpose) {
   // (transpose: the input gradient's view, W[k]^T -- source channels are the columns of W[k])
-  const int slabs = (transpose ? c_out : c_in) / 32, nts = (transpose ? c_in : c_out) / 32;
+  const int c_src = transpose ? c_out : c_in, c_dst = transpose ? c_in : c_out, slabs = (c_src + 31) / 32, nts = (c_dst + 31) / 32;
   const size_t total = (size_t)k_vol * slabs * 2 * nts * 64;
   for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < total;
        t += (size_t)gridDim.x * blockDim.x) {
@@ -295,7 +296,8 @@ __global__ void pack_weights_parts_kernel(const float *__restrict__ w, int4v *__
     float4v x[2];
 #pragma unroll
     for (int e = 0; e < 8; ++e)
-      x[e / 4][e % 4] = transpose ? w[((size_t)k * c_in + cd) * c_out + cs0 + e] : w[((size_t)k * c_in + cs0 + e) * c_out + cd];
+      x[e / 4][e % 4] = cs0 + e >= c_src || cd >= c_dst ? 0.f
+                        : transpose ? w[((size_t)k * c_in + cd) * c_out + cs0 + e] : w[((size_t)k * c_in + cs0 + e) * c_out + cd];
     int2v lo[P], hi[P];
     split_parts<P>(x[0], lo);
     split_parts<P>(x[1], hi);
@@ -515,9 +517,9 @@ constexpr int rows_sum_chunks() { return kWaves * MT * NT * 4 * 64; }      // ..
 // centre (forward only; 0: none): the bit of an offset through which every row is its own neighbour, and which the caller
 // keeps out of its lists; the offset's line of the table says so, the masks do not (see Plan::centre_line).
 
-// RAGGED (fp16, RAW 1 and 2): channel counts that fill no whole tile.  Chunks of rows and weights from c_src
-// on, and of weights from c_dst on, are loaded from outside their buffers and arrive as zeros; columns from
-// c_dst on are not written.
+// RAGGED (fp16, RAW 1 and 2; fp32, RAW 3 to 6): channel counts that fill no whole tile.  Chunks of rows and weights from
+// c_src on, and of weights from c_dst on, are loaded from outside their buffers and arrive as zeros (re-laid weights hold
+// zeros there); columns from c_dst on are not written.
 template <typename T, int NT, int S, int RAW, int MT = 2, int KG = 1, bool RAGGED = false>
 __device__ __forceinline__ void gms_rows_body(
     const T *__restrict__ src, const T *__restrict__ packed, T *__restrict__ dst,
@@ -552,9 +554,9 @@ __device__ __forceinline__ void gms_rows_body(
   // fp32 only: its MFMA phase is long enough (4 k clocks a stage) to absorb the loads'
   // issue waits; for fp16 the interleaved stage measured 2 us slower per launch
   constexpr bool kInterleave = sizeof(T) == 4 && P == 0;
-  static_assert(!RAGGED || (sizeof(T) == 2 && (RAW == 1 || RAW == 2)), "ragged: fp16 weights as they lie");
+  static_assert(!RAGGED || (sizeof(T) == 2 ? RAW == 1 || RAW == 2 : P > 0), "ragged: fp16 weights as they lie, fp32 in parts");
   const int slabs = RAGGED ? (c_src + C * E - 1) / (C * E) : c_src / (C * E);
-  const int nts = c_dst / 32;
+  const int nts = RAGGED ? (c_dst + 31) / 32 : c_dst / 32;
   int4v *w_lds = lds;                                     // [2][WCH]
   const int wave = tid / 64, lane = tid % 64;
   constexpr int WR = MT * 32;                             // rows per wave
@@ -568,7 +570,8 @@ __device__ __forceinline__ void gms_rows_body(
   int *didx = idx_all + wave * 3 * WR + 2 * WR;
   const int nt0 = block_y * NT;
   const int4v *packed4 = reinterpret_cast<const int4v *>(packed);
-  const size_t packed_per_k = (size_t)c_src * c_dst / E * (RAW == 5 ? 3 : 2) / 2;  // chunks
+  // chunks of an offset's weights
+  const size_t packed_per_k = RAW == 3 || RAW == 5 ? (size_t)slabs * nts * 128 * P : (size_t)c_src * c_dst / E;
 
   // the plan's table gives the tile and the first offset it uses
   int tile = block_x, k_first = -1;
@@ -681,7 +684,8 @@ __device__ __forceinline__ void gms_rows_body(
   //   RAW = 3, 5: k-step e / (NT*64*P) of the stage, then [nt][part][lane]
   //   RAW = 0: chunks [(slab*S + s) * nts + nt0 + nt] * 64 + lane of the re-laid copy
   const __amdgpu_buffer_rsrc_t wrsrc =
-      rows_resource(packed, (unsigned)k_vol * (unsigned)c_src * (unsigned)c_dst * (RAW == 5 ? 6u : (unsigned)sizeof(T)));
+      rows_resource(packed, RAW == 3 || RAW == 5 ? (unsigned)k_vol * (unsigned)packed_per_k * 16u
+                                                   : (unsigned)k_vol * (unsigned)c_src * (unsigned)c_dst * (unsigned)sizeof(T));
   unsigned wvoff[NW];
 #pragma unroll
   for (int i = 0; i < NW; ++i) {
@@ -721,7 +725,7 @@ __device__ __forceinline__ void gms_rows_body(
       const int e = tid + kThreads * i;
       if (NW * kThreads == WLD || e < WLD) {
         unsigned off = wvoff[i];
-        if constexpr (RAGGED) {
+        if constexpr (RAGGED && RAW != 3 && RAW != 5) {
           const int from = slab * (C * E) + (RAW == 1 ? e / (NT * 4) : e % C * E);
           const int to = nt0 * 32 + (RAW == 1 ? e % (NT * 4) * E : e / C);
           if (from >= c_src || to >= c_dst) off = kAbsentRow;
@@ -1058,8 +1062,12 @@ int ragged_steps(int c) {
 // The shapes that take it: multiples of 8 channels (16-byte chunks) that no whole tile fits -- a source of a pass
 // that is no multiple of 16, anything else that is none of 32 -- or an odd number of 32s from five
 // on (160), which whole tiles take 32 columns at a time.  Kernels on the vector ALUs keep the narrow ones.
-bool ragged_channels(int c_in, int c_out, bool forward) {
+// fp32 (in bf16 parts): what is no multiple of 32 on either side.  Without (fp32 MFMAs, padded copies) / with masks:
+// 48 -> 48 over 30 k voxels forward 83 / 50 us, both gradients 123 / 65; 48 -> 64 over 120 k 121 / 108 and 303 / 189, in
+// tf32 mode 121 / 65 and 180 / 131.
+bool ragged_channels(int c_in, int c_out, bool forward, bool f16) {
   if (c_in % 8 || c_out % 8 || c_in < 16 || c_out < 16 || c_in * c_out <= 256) return false;
+  if (!f16) return c_in % 32 != 0 || c_out % 32 != 0;
   auto odd = [](int c, int whole) { return c % whole != 0 || (c % 32 == 0 && c / 32 % 2 == 1 && c / 32 >= 5 && c / 32 % 3 != 0); };
   return odd(c_in, forward ? 16 : 32) || odd(c_out, 32);
 }
@@ -1067,13 +1075,14 @@ Shape ragged_shape(const GmsArgs &a) {
   Shape s{};
   s.c_src = a.transpose_w ? a.c_out : a.c_in;
   s.c_dst = a.transpose_w ? a.c_in : a.c_out;
-  s.E = 8;
-  if (a.dtype != FGMS_F16 || !ragged_channels(a.c_in, a.c_out, !a.transpose_w)) return s;
+  const bool f16 = a.dtype == FGMS_F16;
+  s.E = f16 ? 8 : 4;
+  if ((!f16 && !split_bf16_enabled()) || !ragged_channels(a.c_in, a.c_out, !a.transpose_w, f16)) return s;
   if (reinterpret_cast<uintptr_t>(a.src) % 16 || reinterpret_cast<uintptr_t>(a.dst) % 16 ||
       reinterpret_cast<uintptr_t>(a.w) % 16 || !raw_weights_enabled())
     return s;
-  s.NTR = ragged_tiles(s.c_dst, worth_96_columns(a.n_pairs, a.n_src, a.n_dst));
-  s.SR = ragged_steps(s.c_src);
+  s.NTR = f16 ? ragged_tiles(s.c_dst, worth_96_columns(a.n_pairs, a.n_src, a.n_dst)) : (s.c_dst + 31) / 32 % 2 ? 1 : 2;
+  s.SR = f16 ? ragged_steps(s.c_src) : 4;
   s.lds_rows_bytes = 2 * (size_t)s.SR * s.NTR * 64 * 16 + (size_t)kWaves * kWaveRows * 2 * s.SR * 16 +
                      (size_t)kWaves * 3 * kWaveRows * sizeof(int);
   s.ok = s.NTR > 0;
@@ -1102,7 +1111,7 @@ int pack_weights(const GmsArgs &a, int S, const T **packed) {
 template <int P>
 int pack_weights_parts(const GmsArgs &a, bool transpose, const void **packed) {
   void *ws = nullptr;
-  const size_t n = (size_t)a.k_vol * a.c_in * a.c_out;
+  const size_t n = (size_t)a.k_vol * ((a.c_in + 31) / 32 * 32) * ((a.c_out + 31) / 32 * 32);
   bool fill = true;
   int rc = relaid_weights_buffer(a, 1u | (transpose ? 2u : 0u) | (P == 3 ? 4u : 0u), n * 2 * P, &ws, &fill);
   if (rc != FGMS_OK) return rc;
@@ -1271,7 +1280,8 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
   // fp32 tensors: products of bf16 parts, two to a value in "tf32" mode, else three (three or six 16-bit MFMAs instead
   // of sixteen fp32 ones per product tile); needs whole 32-channel slabs
   constexpr bool kCanSplit = sizeof(T) == 4 && S == 4 && NT != 4;
-  const bool split = kCanSplit && !a.transpose_w && !a.prepacked && split_bf16_enabled() && (a.reduced || NT != 3);
+  const bool split = kCanSplit && !a.transpose_w && !a.prepacked && split_bf16_enabled() &&
+                     (a.reduced || (NT != 3 && (size_t)a.k_vol * a.c_in * a.c_out <= 0xfffffff0u / 6));     // (32-bit offsets)
   if (kCanSplit && raw == 2 && split_bf16_enabled()) raw = a.reduced ? 4 : NT != 3 ? 6 : 2;   // (the input gradient splits as it reads)
   const T *packed = raw ? (const T *)a.w : (const T *)a.prepacked;
   if (split) {
@@ -1297,9 +1307,11 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
   if (gx == 0) return a.side.kind ? launch_side_job(a.side, a.stream) : FGMS_OK;
   constexpr bool kCanRaw = NT != 4;
   constexpr int kRaw6 = kCanSplit && NT != 3 ? 6 : 0, kRaw5 = kCanSplit && NT != 3 ? 5 : 0, kRaw4 = kCanSplit ? 4 : 0, kRaw3 = kCanSplit ? 3 : 0, kRaw2 = kCanRaw ? 2 : 0, kRaw1 = kCanRaw && sizeof(T) == 2 ? 1 : 0;
+  constexpr int kRagRaw = !RAGGED ? 0 : sizeof(T) == 2 ? kRaw1 : kRaw3, kRagRaw5 = !RAGGED ? 0 : sizeof(T) == 2 ? kRaw1 : kRaw5;
   // (raw is one of those the type and the tile allow)
 #define FGMS_BY_RAW(MTv, KGv)                                                                                       \
-  (RAGGED     ? gms_rows_kernel<T, NT, S, RAGGED ? kRaw1 : 0, MTv, KGv, RAGGED>                                     \
+  (RAGGED && raw == 5 ? gms_rows_kernel<T, NT, S, kRagRaw5, MTv, KGv == 4 && NT == 2 && sizeof(T) == 4 ? 2 : KGv, RAGGED> \
+   : RAGGED   ? gms_rows_kernel<T, NT, S, kRagRaw, MTv, KGv, RAGGED>                                                \
    : raw == 6 ? gms_rows_kernel<T, NT, S, kRaw6, MTv, 1>                                                            \
    : raw == 5 ? gms_rows_kernel<T, NT, S, kRaw5, MTv, KGv == 4 && NT == 2 ? 2 : KGv>                                \
    : raw == 4 ? gms_rows_kernel<T, NT, S, kRaw4, MTv, KGv>                                                          \
@@ -1412,14 +1424,15 @@ int launch_fused(const GmsArgs &d, const Shape &s, const Plan *p, const WgradArg
   // parts, for fp32 tensors)
   constexpr bool kCanSplit = sizeof(T) == 4 && S == 4 && NT != 4, kCan3 = kCanSplit && BI <= 2 && BJ <= 2;
   const int raw = kCan3 && g.split == 3 ? 6 : kCanSplit && g.split == 2 ? 4 : 2;
+  constexpr int kRaw2 = RAGGED && sizeof(T) == 4 ? 4 : 2;        // (masked fp32 shapes come in parts only)
   constexpr int kHalfMT = kCanHalf ? 1 : 2;
   constexpr int kRaw4 = kCanSplit ? 4 : 2, kRaw6 = kCan3 ? 6 : 2;
   auto kern = rg.half_tiles ? (raw == 6 ? bwd_fused_kernel<T, NT, S, BI, BJ, kRaw6, kHalfMT, RAGGED>
                                : raw == 4 ? bwd_fused_kernel<T, NT, S, BI, BJ, kRaw4, kHalfMT, RAGGED>
-                                          : bwd_fused_kernel<T, NT, S, BI, BJ, 2, kHalfMT, RAGGED>)
+                                          : bwd_fused_kernel<T, NT, S, BI, BJ, kRaw2, kHalfMT, RAGGED>)
               : raw == 6    ? bwd_fused_kernel<T, NT, S, BI, BJ, kRaw6, 2, RAGGED>
               : raw == 4    ? bwd_fused_kernel<T, NT, S, BI, BJ, kRaw4, 2, RAGGED>
-                            : bwd_fused_kernel<T, NT, S, BI, BJ, 2, 2, RAGGED>;
+                            : bwd_fused_kernel<T, NT, S, BI, BJ, kRaw2, 2, RAGGED>;
   size_t lds = g.lds;
   const size_t lds_rows = rg.half_tiles ? rows_group_chunks<T, NT, S, kHalfMT>(raw) * 16 : rows_group_chunks<T, NT, S, 2>(raw) * 16;
   if (lds < lds_rows) lds = lds_rows;
@@ -1558,9 +1571,9 @@ int launch_ragged_bwd(const GmsArgs &d, const Plan *p, const WgradArgs &w, bool 
     return FGMS_OK;
   const Shape s = ragged_shape(d);
   WgradGeometry g;
-  if (!s.ok || !ragged_wgrad_geometry(w, ragged_tiles(w.c_in, worth_96_columns(w.n_pairs, w.n_in, w.n_out)),
-                                      ragged_tiles(w.c_out, worth_96_columns(w.n_pairs, w.n_in, w.n_out)), &g))
-    return FGMS_OK;
+  const bool f16 = d.dtype == FGMS_F16;
+  auto tiles = [&](int c) { return f16 ? ragged_tiles(c, worth_96_columns(w.n_pairs, w.n_in, w.n_out)) : (c + 31) / 32 % 2 ? 1 : 2; };
+  if (!s.ok || !ragged_wgrad_geometry(w, tiles(w.c_in), tiles(w.c_out), &g)) return FGMS_OK;
   bool found = false;
   int rc = FGMS_OK;
   float *acc32 = nullptr;
@@ -1568,8 +1581,16 @@ int launch_ragged_bwd(const GmsArgs &d, const Plan *p, const WgradArgs &w, bool 
   // NT: 1 up to 32 input channels, 2 up to 64 and for an even number of 32s, 3 for 72 .. 96, 136 .. 160 and the like.
   // S, BJ by output channels: 2, 1 up to 32; 3, 2 for 40 and 48; 4, 2 for 56, 64 and an even number of 32s; 3, 3 for
   // 72 .. 96; 4, 3 for 136 .. 160 and other odd numbers of 32s.)
+#define FGMS_FRF(NTv, BJv)                                                                                        \
+  if (!found && !f16 && s.NTR == NTv && g.bi == NTv && g.bj == BJv) {                                             \
+    found = true;                                                                                                 \
+    if ((rc = wgrad_accumulator(w, &acc32)) == FGMS_OK)                                                           \
+      rc = launch_fused<float, NTv, 4, NTv, BJv, true>(d, s, p, w, g, acc32);                                     \
+  }
+  FGMS_FRF(1, 1) FGMS_FRF(1, 2) FGMS_FRF(2, 1) FGMS_FRF(2, 2)
+#undef FGMS_FRF
 #define FGMS_FR(NTv, Sv, BJv)                                                                                     \
-  if (!found && s.NTR == NTv && s.SR == Sv && g.bi == NTv && g.bj == BJv) {                                       \
+  if (!found && f16 && s.NTR == NTv && s.SR == Sv && g.bi == NTv && g.bj == BJv) {                                \
     found = true;                                                                                                 \
     if ((rc = wgrad_accumulator(w, &acc32)) == FGMS_OK)                                                           \
       rc = launch_fused<__half, NTv, Sv, NTv, BJv, true>(d, s, p, w, g, acc32);                                   \
@@ -1692,6 +1713,11 @@ int launch_ragged_gms(const GmsArgs &a, const Plan *p) {
   }
   GmsArgs a_ = a;
   if (!a_.side.kind) (void)plan_take_check(p, &a_.side);
+  if (a.dtype != FGMS_F16) {
+    if (s.NTR == 2)
+      return launch_rows<float, 2, 4, true>(a_, s, p->nbr_out, p->mask_out, p->perm_out, p->tile_out, p->tile_grid_out, p->flip_out);
+    return launch_rows<float, 1, 4, true>(a_, s, p->nbr_out, p->mask_out, p->perm_out, p->tile_out, p->tile_grid_out, p->flip_out);
+  }
 #define FGMS_RG(NTv, Sv)                   \
   if (s.NTR == NTv && s.SR == Sv)          \
     return launch_rows<__half, NTv, Sv, true>(a_, s, p->nbr_out, p->mask_out, p->perm_out, p->tile_out, p->tile_grid_out, p->flip_out);

@@ -283,6 +283,8 @@ __device__ __forceinline__ void add_rows_lds(const float16v (&acc)[MT][NT], T *_
         for (int it = 0; it < IT; ++it) {
           if constexpr (OVERWRITE)
             old[it] = float4v{0.f, 0.f, 0.f, 0.f};
+          else if (RAGGED && row[it] < 0)
+            old[it] = float4v{0.f, 0.f, 0.f, 0.f};
           else
             old[it] = *reinterpret_cast<const float4v *>(
                 reinterpret_cast<const float *>(dst) + (size_t)max(row[it], 0) * c_dst + cd0 +

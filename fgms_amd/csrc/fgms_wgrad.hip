@@ -513,9 +513,10 @@ int wgrad_geometry(const WgradArgs &a, WgradGeometry *g, bool shares_grid) {
 }
 
 bool ragged_wgrad_geometry(const WgradArgs &a, int bi, int bj, WgradGeometry *g) {
-  if (a.dtype != FGMS_F16 || bi < 1 || bj < 1 || a.side.kind || a.crop_in) return false;
+  const size_t esz = a.dtype == FGMS_F16 ? 2 : 4;
+  if ((a.dtype != FGMS_F16 && !split_bf16_enabled()) || bi < 1 || bj < 1 || a.side.kind || a.crop_in) return false;
   if (reinterpret_cast<uintptr_t>(a.in) % 16 || reinterpret_cast<uintptr_t>(a.gout) % 16) return false;
-  if ((size_t)a.n_in * a.c_in * 2 > kMaxBufferBytes || (size_t)a.n_out * a.c_out * 2 > kMaxBufferBytes) return false;
+  if ((size_t)a.n_in * a.c_in * esz > kMaxBufferBytes || (size_t)a.n_out * a.c_out * esz > kMaxBufferBytes) return false;
   *g = WgradGeometry{};
   g->bi = bi;
   g->bj = bj;

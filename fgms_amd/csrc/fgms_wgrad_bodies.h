@@ -143,7 +143,7 @@ __device__ __forceinline__ void wgrad_wave_body(
   constexpr int LDI = CI + (kBufW ? 0 : W::pad), LDO = CO + (kBufW ? 0 : W::pad);
   constexpr int NCI = CI / E, NCO = CO / E;
   constexpr int NX = SP * NCI / 64, NG = SP * NCO / 64;   // chunks per lane and stage
-  static_assert(!RAGGED || kBufW, "ragged: fp16");
+  static_assert(!RAGGED || kBufW || SPLIT, "ragged: fp16, or fp32 in parts");
   static_assert(NX >= 1 && NG >= 1, "stage too small");
   extern __shared__ int4v lds[];
   int k, first, count;
@@ -246,7 +246,8 @@ __device__ __forceinline__ void wgrad_wave_body(
         xr[i] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(
                                               in_rsrc, off + (unsigned)((ci0 + cc * E) * (int)sizeof(T)), 0, 0));
       } else {
-        xr[i] = *reinterpret_cast<const int4v *>(in + (size_t)xi[i] * c_in + ci0 + cc * E);
+        // (RAGGED: a chunk that does not exist is read from the row's last one, and stored as zeros)
+        xr[i] = *reinterpret_cast<const int4v *>(in + (size_t)xi[i] * c_in + (RAGGED ? min(ci0 + cc * E, c_in - E) : ci0 + cc * E));
       }
     }
 #pragma unroll
@@ -258,7 +259,7 @@ __device__ __forceinline__ void wgrad_wave_body(
         gr[i] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(
                                               gout_rsrc, off + (unsigned)((co0 + cc * E) * (int)sizeof(T)), 0, 0));
       } else {
-        gr[i] = *reinterpret_cast<const int4v *>(gout + (size_t)gi[i] * c_out + co0 + cc * E);
+        gr[i] = *reinterpret_cast<const int4v *>(gout + (size_t)gi[i] * c_out + (RAGGED ? min(co0 + cc * E, c_out - E) : co0 + cc * E));
       }
     }
   };
@@ -267,7 +268,8 @@ __device__ __forceinline__ void wgrad_wave_body(
     for (int i = 0; i < NX; ++i) {
       const int e = lane + 64 * i;
       if constexpr (SPLIT)
-        store_split_chunk<P>(xs, SP * LDIh, LDIh, e / NCI, e % NCI, xr[i], st * SP + e / NCI < count);
+        store_split_chunk<P>(xs, SP * LDIh, LDIh, e / NCI, e % NCI, xr[i],
+                             st * SP + e / NCI < count && (!RAGGED || ci0 + e % NCI * E < c_in));
       else if constexpr (kBufW)
         *reinterpret_cast<int4v *>(x + x_row(i) * LDI + ((x_chunk(i) ^ (CI == 64 ? ((x_row(i) >> 1) & 1) * 4 : 0)) * E)) = xr[i];
       else
@@ -278,7 +280,8 @@ __device__ __forceinline__ void wgrad_wave_body(
     for (int i = 0; i < NG; ++i) {
       const int e = lane + 64 * i;
       if constexpr (SPLIT)
-        store_split_chunk<P>(gs, SP * LDOh, LDOh, e / NCO, e % NCO, gr[i], st * SP + e / NCO < count);
+        store_split_chunk<P>(gs, SP * LDOh, LDOh, e / NCO, e % NCO, gr[i],
+                             st * SP + e / NCO < count && (!RAGGED || co0 + e % NCO * E < c_out));
       else if constexpr (kBufW)
         *reinterpret_cast<int4v *>(g + g_row(i) * LDO + ((g_chunk(i) ^ (CO == 64 ? ((g_row(i) >> 1) & 1) * 4 : 0)) * E)) = gr[i];
       else
