@@ -398,11 +398,12 @@ __global__ __launch_bounds__(256) void kmap_lists_kernel(ListArgs a, SortArgs so
   if (list_block >= list_blocks) {
     const int b = list_block - list_blocks;
     const int side = b < sort.side[0].chunks ? 0 : 1;
-    sort_hist_body(sort.side[side], sort, side ? b - sort.side[0].chunks : b, tile, 256);
+    sort_hist_body<256>(sort.side[side], sort, side ? b - sort.side[0].chunks : b, tile);
     return;
   }
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
   const int row0 = list_block * kListRows;
+  constexpr int kTurns = kWidth / 4;      // 16-byte chunks of a row per thread, and offsets per wave
   // bounds of the plan's row bands that fall into this block of rows (the last block has those behind
   // it, too): what lies below them inside the block is in the ballots anyway
   int bands = 0, band_rows = 1, c_first = 1, c_last = 0;
@@ -413,19 +414,36 @@ __global__ __launch_bounds__(256) void kmap_lists_kernel(ListArgs a, SortArgs so
     c_last = list_block + 1 == list_blocks ? bands : min(bands, (row0 + kListRows - 1) / band_rows);
   }
   for (int k0 = 0; k0 < a.k_vol; k0 += kWidth) {
-    const int width = min(kWidth, a.row_ld - k0) / 4;
-    for (int e = threadIdx.x; e < kListRows * width; e += 256) {
-      const int r = e / width, c = e % width * 4;
-      int4v_ v = {-1, -1, -1, -1};
-      if (row0 + r < a.n_out) v = *reinterpret_cast<const int4v_ *>(a.rows + (size_t)(row0 + r) * a.row_ld + k0 + c);
+    const int width = min(kWidth, a.row_ld - k0) / 4, k_end = min(k0 + kWidth, a.k_vol);
+    // (all of a part's loads in flight together)
+    int4v_ v[kTurns];
+    int block_first[kTurns], first[kTurns];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) tile[r * (kWidth + 1) + c + q] = v[q];
+    for (int i = 0; i < kTurns; ++i) {
+      const int e = threadIdx.x + 256 * i, row = row0 + e / width;
+      v[i] = int4v_{-1, -1, -1, -1};
+      if (i < width && row < a.n_out) v[i] = *reinterpret_cast<const int4v_ *>(a.rows + (size_t)row * a.row_ld + k0 + e % width * 4);
+    }
+#pragma unroll
+    for (int i = 0; i < kTurns; ++i) {
+      const size_t line = (size_t)min(k0 + wave + 4 * i, a.k_vol - 1) * a.blocks;
+      block_first[i] = a.bases[line + list_block];
+      first[i] = a.bases[line];
+    }
+#pragma unroll
+    for (int i = 0; i < kTurns; ++i) {
+      if (i >= width) break;
+      const int e = threadIdx.x + 256 * i;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) tile[e / width * (kWidth + 1) + e % width * 4 + q] = v[i][q];
     }
     __syncthreads();
-    for (int k = k0 + wave; k < min(k0 + kWidth, a.k_vol); k += 4) {
-      const int block_first = a.bases[(size_t)k * a.blocks + list_block];
-      const int before = block_first - a.bases[(size_t)k * a.blocks];
-      long long pos = block_first;
+#pragma unroll
+    for (int i = 0; i < kTurns; ++i) {
+      const int k = k0 + wave + 4 * i;
+      if (k >= k_end) break;
+      const int before = block_first[i] - first[i];
+      long long pos = block_first[i];
       unsigned long long hits[kListRows / 64];
 #pragma unroll
       for (int q = 0; q < kListRows / 64; ++q) {

@@ -104,7 +104,7 @@ __global__ __launch_bounds__(kSortThreads) void sort_hist_kernel(SortArgs a) {
   const SortSide &sd = a.side[blockIdx.y];
   if ((int)blockIdx.x >= sd.chunks) return;
   __shared__ int hist[kBins];
-  sort_hist_body(sd, a, blockIdx.x, hist, kSortThreads);
+  sort_hist_body<kSortThreads>(sd, a, blockIdx.x, hist);
 }
 
 // hist[chunk][bin] -> hist_before[chunk][bin] = rows of the bin in earlier chunks, and
