@@ -68,12 +68,50 @@ struct SliceMap {
   const int32_t *cells;        // the plan's dispatch order of the (offset, band) cells, or nullptr
   int bands, stride;           // slice sl = bands [sl * stride, (sl + 1) * stride)
   int slices;
-  int chunk;                   // > 0: plain tiles of `chunk` pairs in pair-list order instead
+  int chunk;                   // > 0: plain tiles of `chunk` pairs instead, in pair-list order ...
+  bool by_xcd;                 // ... or the same part of every list on the same XCD (locate_tile_by_xcd)
 };
+
+// Tiles of `chunk` pairs: XCD x takes the tiles of every offset's list from x eighths of it to x + 1 (the cut shifted
+// from offset to offset, so that an XCD does not get the longer part of each).  Lists that are ordered by output row then meet
+// the same rows in the same L2 at about the same time.  (Tiles in list
+// order, round the XCDs / so: 128 -> 128 fp16 backward launch over 120 k LiDAR voxels sorted 168 / 151 us, as scanned 166 / 158,
+// indoor 160 / 151; 256 -> 256 over 40 k 230 / 216.  Three tiles per CU instead of two: 120 k indoor 146, 20 k 65 for 56.)
+// A lane per offset.
+__device__ __forceinline__ bool locate_tile_by_xcd(const int32_t *__restrict__ kpos, int k_vol, int chunk, int block,
+                                                   int &k, int &first, int &count) {
+  const int xcd = block % 8, lane = threadIdx.x % 64;
+  int j = block / 8;
+  for (int k0 = 0; k0 < k_vol; k0 += 64) {
+    const int kk = k0 + lane, start = kk < k_vol ? kpos[kk] : 0, n = kk < k_vol ? kpos[kk + 1] - start : 0;
+    const int tiles = (n + chunk - 1) / chunk, shift = 7 - (5 * kk & 7);
+    const int c0 = (tiles * xcd + shift) >> 3, mine = ((tiles * (xcd + 1) + shift) >> 3) - c0;
+    int upto = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d *= 2) {
+      const int other = __shfl_up(upto, d);
+      if (lane >= d) upto += other;
+    }
+    const unsigned long long past = __ballot(upto > j);
+    if (past) {
+      const int at = __builtin_ctzll(past);
+      const int c = j + __builtin_amdgcn_readlane(c0 - (upto - mine), at);
+      k = k0 + at;
+      first = __builtin_amdgcn_readlane(start, at) + c * chunk;
+      count = min(chunk, __builtin_amdgcn_readlane(n, at) - c * chunk);
+      return true;
+    }
+    j -= __builtin_amdgcn_readlane(upto, 63);
+  }
+  return false;
+}
+// Workgroups that takes, at most: an XCD's share of the tiles, and one more of every offset's.
+inline int64_t tiles_by_xcd(int64_t n_pairs, int64_t chunk, int k_vol) { return 8 * (((n_pairs + chunk - 1) / chunk + k_vol + 7) / 8 + k_vol); }
 
 __device__ __forceinline__ bool locate_slice(const int32_t *__restrict__ kpos, const SliceMap &m,
                                              int k_vol, int block, int &k, int &first, int &count) {
-  if (m.chunk > 0) return locate_tile(kpos, k_vol, m.chunk, block, k, first, count);
+  if (m.chunk > 0)
+    return m.by_xcd ? locate_tile_by_xcd(kpos, k_vol, m.chunk, block, k, first, count) : locate_tile(kpos, k_vol, m.chunk, block, k, first, count);
   int sl;
   if (m.cells) {                    // biggest cells of this XCD first
     const int cell = m.cells[block];
