@@ -630,7 +630,7 @@ bool padded_gms_channels(const GmsArgs &a, const Plan *plan, int *c_in, int *c_o
   return padding_pays(a, plan, *c_in, *c_out);
 }
 
-// fp16 layers whose channels fill no whole tile go straight to kernels that mask the rest, where the map
+// Layers whose channels fill no whole tile go straight to kernels that mask the rest, where the map
 // is dense enough for the output-stationary kernel (else the pair-stationary kernels over padded copies).
 bool takes_ragged(const GmsArgs &a, const Plan *plan) {
   return g_policy == 0 && plan && a.n_pairs > 0 && a.dense_k < 0 && !narrow_gms_supported(a, plan) && !small_gms_supported(a, plan) && !sparse_rows(a, plan);

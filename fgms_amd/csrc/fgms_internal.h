@@ -283,7 +283,7 @@ int wgrad_static(WgradArgs a);
 // (nothing is launched) and returns where the packed weights will be.
 int planned_pack_job(const GmsArgs &a, SideJob *job, const void **packed);
 // Both gradients of a layer in one launch where that is supported (*done says whether).
-// fp16 channel counts that fill no whole tile, through plan p: the forward pass, and both gradients in one launch.
+// Channel counts that fill no whole tile, through plan p: the forward pass, and both gradients in one launch.
 bool ragged_gms_supported(const GmsArgs &a, const Plan *p);
 int launch_ragged_gms(const GmsArgs &a, const Plan *p);
 int launch_ragged_bwd(const GmsArgs &d, const Plan *p, const WgradArgs &w, bool *done);

@@ -1040,7 +1040,7 @@ bool raw_weights_enabled() {
   return on;
 }
 
-// --- fp16 channel counts that fill no whole tile (RAGGED) --------------------------------------
+// --- channel counts that fill no whole tile (RAGGED) --------------------------------------
 // 32-column tiles per wave (and blocks of a weight-gradient tile) for c columns, 0: not served.
 int ragged_tiles(int c, bool three) {
   const int t = (c + 31) / 32;
@@ -1563,7 +1563,7 @@ static bool rows_fit_buffer(const GmsArgs &a) {
   return (size_t)a.n_src * c_src * (a.dtype == FGMS_F16 ? 2 : 4) <= kMaxBufferBytes;
 }
 
-// The same for channel counts that fill no whole tile (fp16).
+// The same for channel counts that fill no whole tile.
 int launch_ragged_bwd(const GmsArgs &d, const Plan *p, const WgradArgs &w, bool *done) {
   *done = false;
   if (!fused_bwd_enabled() || !p || !p->groups.empty() || d.k_vol > 64 || d.k_vol != p->k_vol || !p->dgrad_ok ||

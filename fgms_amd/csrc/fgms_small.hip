@@ -1,5 +1,5 @@
 // Skinny-channel gather-GEMM kernel (no MFMA): layers whose narrow side is at
-// most 16 channels, e.g. the 4 -> 32 first layer of a voxel network.  Such a
+// most 16 channels (fp16 forward passes from a narrow input side: fgms_narrow.hip).  Such a
 // layer moves ~10x more bytes than it has flops for the matrix cores to matter
 // (a 4-channel fp16 row is 8 bytes), so the kernel is organised around memory:
 //
