@@ -466,10 +466,25 @@ int check_common(const void *a, const void *b, const void *c, const int32_t *kpo
 // density, 2 .. 3 for random subsamples of them) and on the channel count.  Measured on
 // MI355X over subsamples of a 200 k-voxel indoor-like cloud (35 k .. 200 k voxels, 32 .. 256
 // channels), the slots per pair at which both take the same time:
-//   fp32: 2.35 / 1.76 / 1.3 at 32 / 64 / 128 channels, i.e. about 1 + 45 / c (the MFMA time
-//         of the empty slots against a fixed cost per atomic);
-//   fp16: 2.25 .. 2.5 at every channel count (2.2 + 16 / c).
+//   fp16: 2.25 .. 2.5 at every channel count (2.2 + 16 / c);
+//   fp32 MFMAs: 2.35 / 1.76 / 1.3 at 32 / 64 / 128 channels, about 1 + 45 / c.
 // The kernel without atomics, whose results do not depend on the run, gets 5 % on top.
+// fp32 tensors in bf16 parts, beyond that line: products cost so little that the output-stationary kernel's chain of stages (small maps)
+// or rounds of tiles (large ones) counts, and not the empty slots; estimated for either side, fitted to thinned clouds of
+// 10 k .. 60 k voxels.  Pair view / output-stationary, fp32 and tf32 mode, over thinned clouds: 64 -> 64 forward 20 k voxels of
+// 60 k 32.4 / 48.6 and 31.1 / 32.9 us, 60 k of 100 k 113.9 / 71.1 and 103.7 / 45.1, 60 k of 200 k 72.2 / 67.6 and
+// 66.1 / 43.3; 128 -> 128 60 k of 150 k 168 / 202 and 149 / 119.  Both gradients, in one grid where the output-stationary
+// kernel takes the input's (beside_us): 64 -> 64 20 k of 60 k 85.7 / 61.6 and 74.9 / 52.2, 256 -> 256 295 / 419 and 278 / 326.
+double stages_us(const GmsArgs &a) {
+  const int c_src = a.transpose_w ? a.c_out : a.c_in, c_dst = a.transpose_w ? a.c_in : a.c_out, slabs = (c_src + 31) / 32;
+  const double tiles_per_cu = (double)((a.n_dst + 127) / 128 * ((c_dst + 31) / 32)) / num_cus();
+  const double stage = a.transpose_w ? (a.reduced ? 0.36 + 0.02 * slabs : 0.45 + 0.0035 * slabs * slabs) : (a.reduced ? 0.33 : 0.55);
+  return 8.5 + stage * a.k_vol * slabs * (tiles_per_cu <= 1 ? 1 : 1.25 + 0.25 * tiles_per_cu);
+}
+double pair_view_us(const GmsArgs &a, double pairs) {
+  const int c_src = a.transpose_w ? a.c_out : a.c_in, c_dst = a.transpose_w ? a.c_in : a.c_out;
+  return 9 + 6e-4 * c_src * c_dst + (a.reduced ? 0.8e-6 : 1e-6) * pairs * c_dst * (3.6 + 0.0042 * c_src);
+}
 bool sparse_rows(const GmsArgs &a, const Plan *plan) {
   const int stages = a.transpose_w ? plan->stages_in : plan->stages_out;
   if (stages <= 0 || plan->pairs_counted <= 0) return false;   // (the plan's own pair count: a.n_pairs is a bound)
@@ -478,7 +493,9 @@ bool sparse_rows(const GmsArgs &a, const Plan *plan) {
   const double even = a.dtype == FGMS_F16 ? 2.2 + 16.0 / c_src : 1.0 + 45.0 / c_src;
   // (no break-even point was measured below 1.3: denser maps stay output-stationary)
   const double need = 1.05 * even;
-  return slots_per_pair > (need > 1.4 ? need : 1.4);
+  if (slots_per_pair <= (need > 1.4 ? need : 1.4)) return false;
+  return a.dtype == FGMS_F16 || !split_bf16_enabled() ||
+         stages_us(a) > 1.08 * (pair_view_us(a, (double)plan->pairs_counted) + a.beside_us);
 }
 
 enum class Route { kNarrow, kSkinny, kRows, kPairView, kWide, kPairs, kGeneric };
@@ -1021,6 +1038,10 @@ int backward(const void *out_feats_grad, const void *in_feats, const void *kerne
   w.overwrite = overwrite;
   if (!want_kernel) return want_in ? run_gms(d, p) : FGMS_OK;
   if (!want_in) return run_wgrad(w);
+  // (a weight gradient of its own: 64 x 64 over 20 k thinned voxels 53 us, 128 x 128 60 .. 68, 256 x 256 120 .. 170; three
+  // quarters of it vanish in the other's grid)
+  if (dtype != FGMS_F16)
+    d.beside_us = 0.74 * (d.reduced ? 0.75 : 1) * (25 + 1e-3 * (double)n_out + 18e-6 * pairs_of(d, p) * up_to_32(c_in) / 32 * (up_to_32(c_out) / 32));
   int pi, po;
   if (takes_ragged(d, p) && masked_bwd_pays(d, p, w)) {
     bool done = false;

@@ -76,6 +76,7 @@ struct GmsArgs {
   // (10 mantissa bits) or better, sums stay fp32
   bool reduced;
   bool overwrite;          // dst = the sums instead of dst += (rows without a pair become zero)
+  double beside_us;        // input gradient of fp32 tensors: what the output-stationary grid hides of the weight gradient's time
   const void *prepacked;   // output-stationary kernel only: the weights are already re-laid here
   SideJob side;            // rides along with the launch (not the shape-agnostic kernel's)
 };

@@ -1092,7 +1092,7 @@ const Plan *plan_resolve(fgms_plan_t *plan, hipStream_t stream, int *rc) {
       p->stages_in = h[5];
       p->pairs_counted = p->has_tables ? h[12] : p->n_pairs;
       // The pair view, for maps sparse enough that some layer would take it (fp32 layers prefer
-      // it from about 1 + 45 / channels row slots per pair on, never below 1.4): built now that
+      // it from about 1 + 45 / channels row slots per pair on, never below 1.4, where the products are many): built now that
       // the counts are known, so that dense maps pay nothing.
       static const bool pair_view = !(getenv("FGMS_PAIR_VIEW") && atoi(getenv("FGMS_PAIR_VIEW")) == 0);
       const int most = p->stages_out > p->stages_in ? p->stages_out : p->stages_in;
