@@ -154,6 +154,32 @@ __device__ __forceinline__ void mma_slab_raw(float16v (&acc)[MT][NT], const int4
   }
 }
 
+// The same for fp32 (forward): the stage's 2*S*4 rows of W[k] as they lie, NT*32 columns each; a lane's four values of a
+// k-step are four reads down a column.
+template <int NT, int S, int MT>
+__device__ __forceinline__ void mma_slab_raw32(float16v (&acc)[MT][NT], const int4v *__restrict__ a_lds,
+                                               const int4v *__restrict__ w_lds, int lane) {
+  const int h = lane / 32, r = lane % 32;
+  const float *w = reinterpret_cast<const float *>(w_lds) + h * S * 4 * (NT * 32) + r;
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    int4v b[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      float4v f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) f[j] = w[(s * 4 + j) * (NT * 32) + nt * 32];
+      b[nt] = __builtin_bit_cast(int4v, f);
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const int4v a = a_lds[a_slot<S>(mt * 32 + r, h * S + s)];
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) mma<float>(acc[mt][nt], a, b[nt]);
+    }
+  }
+}
+
 // --- input-gradient weights straight from the caller's tensor --------------------------
 // The input gradient contracts over the COLUMNS of W[k] (dIn[ci] = sum over co of
 // dOut[co] * W[k][ci][co]), and those are contiguous in memory: the 8 halfs (4 floats) an
@@ -216,8 +242,10 @@ __device__ __forceinline__ void mma_slab_rawt(float16v (&acc)[MT][NT], const int
 // sum around it rounds off (mma_parts has the errors).  Six 16-bit matrix steps take 6/16 of the fp32 ones' time; a
 // tile of rows takes half as much LDS again, which leaves two workgroups to a CU.  fp32 MFMAs / this: 64 -> 64 forward over
 // 40 k voxels 88 / 63 us, 150 k 172 / 111; backward 123 / 77, 342 / 232; 128 -> 128 over 40 k 231 / 133 and 360 / 238;
-// 32 -> 32 over 4 k 25 / 21 and 20 / 18.5.  (A value below 2^-110 or so loses the last bits of its small parts, and an
-// infinite one makes NaN of what it reaches.)
+// 32 -> 32 over 4 k 25 / 21 and 20 / 18.5.  (A value below 2^-110 or so loses the last bits of its small parts.)
+// The parts of an infinite value are no numbers, so sums that reach one come out as NaN or infinite whatever else is in
+// them, and a workgroup that ends up with such a sum does its work again with fp32 MFMAs (RAW = 7 and 8; the tile is
+// written only then): what an infinity reaches is what fp32 arithmetic makes of it, in that tile at the price of both.
 //
 // Slot (16 bytes = 8 bf16) of a split tile of P parts: row-major, a row holds its 32 values of the slab
 // as 4 chunks of each part; the XOR spreads the rows one b128 read pass (16 lanes) touches over all banks: rows of
@@ -496,7 +524,8 @@ __global__ __launch_bounds__(kThreads) void gms_pairs_kernel(
 // products in split bf16 (see mma_slab_parts), `packed` from pack_weights_parts_kernel; RAW = 4:
 // the input gradient in split bf16, weights read as they lie and split on their way to LDS;
 // RAW = 5 and 6: as 3 and 4 with three parts to a value, for fp32 tensors in full precision;
-// RAW = 0: the re-laid copy pack_weight_elements makes.
+// RAW = 7 and 8: what a workgroup of those does where a sum is not finite, the same tile on fp32 MFMAs with the
+// weights as they lie, forward (mma_slab_raw32) and input gradient; RAW = 0: the re-laid copy pack_weight_elements makes.
 // (block_x, block_y, block_z) of a grid (tiles, column tiles, grid_z parts of a tile).
 // MT: 32-row MFMA tiles per wave.  2 (a workgroup tile of 256 rows) is the layout every plan
 // table is made for; 1 (tiles of 128 rows, half the work per wave and stage) serves launches
@@ -526,14 +555,17 @@ __device__ __forceinline__ void gms_rows_body(
     const int32_t *__restrict__ nbr, const unsigned long long *__restrict__ block_masks,
     const int32_t *__restrict__ perm, const int32_t *__restrict__ tile_order, int n_dst, int k_vol,
     int c_src, int c_dst, int part_stages, int block_x, int block_y, int block_z, int grid_z,
-    unsigned src_bytes, int pair_view, int overwrite, int flip, unsigned long long centre) {
+    unsigned src_bytes, int pair_view, int overwrite, int flip, unsigned long long centre, const T *__restrict__ w_raw) {
   constexpr int E = Elem<T>::per_chunk;
   constexpr int C = 2 * S;
+  constexpr bool kAsRows = RAW == 2 || RAW == 4 || RAW == 6 || RAW == 8;      // weights as they lie, input gradient
+  constexpr bool kAsLies = RAW == 1 || RAW == 7;                              // ... forward
+  constexpr int WP = NT * 32 / E;                                             // 16-byte pieces of a weight row of the tile
   // 16-bit matrix instructions (fp16 tensors, fp32 tensors in split bf16): rows and weights come
   // through buffer loads and the MFMA phase is pipelined by hand; plain fp32, whose MFMA phase is
   // eight times as long, keeps pointer loads and interleaves them with its MFMAs instead
   constexpr int P = split_parts_of(RAW);
-  constexpr bool kBuf = sizeof(T) == 2 || P > 0;
+  constexpr bool kBuf = sizeof(T) == 2 || P > 0 || RAW >= 7;
   const __amdgpu_buffer_rsrc_t rsrc = rows_resource(src, src_bytes);
   const unsigned row_bytes = (unsigned)c_src * (unsigned)sizeof(T);
   // byte offset of source row g in the buffer (kAbsentRow: no neighbour, the loads return zeros)
@@ -553,8 +585,9 @@ __device__ __forceinline__ void gms_rows_body(
   int4v *const lds = KG == 1 ? lds_all : lds_all + group * rows_group_chunks<T, NT, S, MT>(RAW);
   // fp32 only: its MFMA phase is long enough (4 k clocks a stage) to absorb the loads'
   // issue waits; for fp16 the interleaved stage measured 2 us slower per launch
-  constexpr bool kInterleave = sizeof(T) == 4 && P == 0;
-  static_assert(!RAGGED || (sizeof(T) == 2 ? RAW == 1 || RAW == 2 : P > 0), "ragged: fp16 weights as they lie, fp32 in parts");
+  constexpr bool kInterleave = !kBuf;
+  static_assert(!RAGGED || (sizeof(T) == 2 ? RAW == 1 || RAW == 2 : P > 0 || RAW >= 7), "ragged: fp16 weights as they lie, fp32 in parts");
+  static_assert(RAW < 7 || (sizeof(T) == 4 && S == 4), "the tiles of RAW 5 and 6");
   const int slabs = RAGGED ? (c_src + C * E - 1) / (C * E) : c_src / (C * E);
   const int nts = RAGGED ? (c_dst + 31) / 32 : c_dst / 32;
   int4v *w_lds = lds;                                     // [2][WCH]
@@ -677,9 +710,9 @@ __device__ __forceinline__ void gms_rows_body(
   // Weights of stage (k, slab), 16-byte chunk e = threadIdx.x + kThreads * i of the stage's tile,
   // through a buffer resource over the weight tensor: the part of a chunk's address that depends
   // on the thread is a per-lane constant (wvoff), the part that depends on the stage is scalar.
-  //   RAW = 1: row e / (NT*4) of the slab's 2*S*8 rows of W[k], 16-byte piece e % (NT*4) of the
+  //   RAW = 1, 7: row e / WP of the slab's C*E rows of W[k], 16-byte piece e % WP of the
   //            NT*32 columns from nt0*32 on
-  //   RAW = 2, 4, 6: row e / C of the NT*32 rows of W[k] from nt0*32 on (c_dst rows of c_src
+  //   RAW = 2, 4, 6, 8: row e / C of the NT*32 rows of W[k] from nt0*32 on (c_dst rows of c_src
   //            elements here), 16-byte piece e % C of the slab
   //   RAW = 3, 5: k-step e / (NT*64*P) of the stage, then [nt][part][lane]
   //   RAW = 0: chunks [(slab*S + s) * nts + nt0 + nt] * 64 + lane of the re-laid copy
@@ -690,8 +723,8 @@ __device__ __forceinline__ void gms_rows_body(
 #pragma unroll
   for (int i = 0; i < NW; ++i) {
     const int e = tid + kThreads * i;
-    if constexpr (RAW == 1) wvoff[i] = (unsigned)(((e / (NT * 4)) * c_dst + (e % (NT * 4)) * E) * (int)sizeof(T));
-    else if constexpr (RAW == 2 || RAW == 4 || RAW == 6) wvoff[i] = (unsigned)(((e / C) * c_src + (e % C) * E) * (int)sizeof(T));
+    if constexpr (kAsLies) wvoff[i] = (unsigned)(((e / WP) * c_dst + (e % WP) * E) * (int)sizeof(T));
+    else if constexpr (kAsRows) wvoff[i] = (unsigned)(((e / C) * c_src + (e % C) * E) * (int)sizeof(T));
     else if constexpr (P > 0) wvoff[i] = (unsigned)(((e / (NT * 64 * P)) * nts * 64 * P + e % (NT * 64 * P)) * 16);
     else wvoff[i] = (unsigned)(((e / (NT * 64)) * nts * 64 + e % (NT * 64)) * 16);
   }
@@ -716,8 +749,8 @@ __device__ __forceinline__ void gms_rows_body(
       return;
     }
     unsigned soff;                                       // (wave-uniform: goes to the scalar offset)
-    if constexpr (RAW == 1) soff = (unsigned)(((k * c_src + slab * (C * E)) * c_dst + nt0 * 32) * (int)sizeof(T));
-    else if constexpr (RAW == 2 || RAW == 4 || RAW == 6) soff = (unsigned)(((k * c_dst + nt0 * 32) * c_src + slab * (C * E)) * (int)sizeof(T));
+    if constexpr (kAsLies) soff = (unsigned)(((k * c_src + slab * (C * E)) * c_dst + nt0 * 32) * (int)sizeof(T));
+    else if constexpr (kAsRows) soff = (unsigned)(((k * c_dst + nt0 * 32) * c_src + slab * (C * E)) * (int)sizeof(T));
     else if constexpr (P > 0) soff = (unsigned)(((int)packed_per_k * k + ((slab * 2) * nts + nt0) * 64 * P) * 16);
     else soff = (unsigned)(((int)packed_per_k * k + ((slab * S) * nts + nt0) * 64) * 16);
 #pragma unroll
@@ -726,8 +759,8 @@ __device__ __forceinline__ void gms_rows_body(
       if (NW * kThreads == WLD || e < WLD) {
         unsigned off = wvoff[i];
         if constexpr (RAGGED && RAW != 3 && RAW != 5) {
-          const int from = slab * (C * E) + (RAW == 1 ? e / (NT * 4) : e % C * E);
-          const int to = nt0 * 32 + (RAW == 1 ? e % (NT * 4) * E : e / C);
+          const int from = slab * (C * E) + (kAsLies ? e / WP : e % C * E);
+          const int to = nt0 * 32 + (kAsLies ? e % WP * E : e / C);
           if (from >= c_src || to >= c_dst) off = kAbsentRow;
         }
         wreg[i] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(wrsrc, off, soff, 0));
@@ -742,7 +775,7 @@ __device__ __forceinline__ void gms_rows_body(
         if constexpr (RAW == 1) {
           const int row = e / (NT * 4), c = e % (NT * 4);
           w_lds[buf * WCH + row * (NT * 4) + (c ^ raw_swizzle<NT>(row))] = wreg[i];
-        } else if constexpr (RAW == 2) {
+        } else if constexpr (RAW == 2 || RAW == 8) {
           w_lds[buf * WCH + a_slot<S>(e / C, e % C)] = wreg[i];
         } else if constexpr (RAW == 4 || RAW == 6) {
           split_and_store<P>(w_lds + buf * WCH, __builtin_bit_cast(float4v, wreg[i]), e / C, e % C);
@@ -795,7 +828,8 @@ __device__ __forceinline__ void gms_rows_body(
     const int safe_row = min(my_row, n_dst - 1);
     auto mma_stage = [&]() {
       if constexpr (RAW == 1) mma_slab_raw<T, NT, S>(acc, a_lds, w_lds + buf * WCH, lane);
-      else if constexpr (RAW == 2) mma_slab_rawt<T, NT, S>(acc, a_lds, w_lds + buf * WCH, lane);
+      else if constexpr (RAW == 7) mma_slab_raw32<NT, S>(acc, a_lds, w_lds + buf * WCH, lane);
+      else if constexpr (RAW == 2 || RAW == 8) mma_slab_rawt<T, NT, S>(acc, a_lds, w_lds + buf * WCH, lane);
       else if constexpr (P > 0) mma_slab_parts<P, RAW == 4 || RAW == 6>(acc, low, a_lds, w_lds + buf * WCH, lane);
       else mma_slab<T, NT, S>(acc, a_lds, w_lds + buf * WCH, 0, lane);
     };
@@ -923,12 +957,22 @@ __device__ __forceinline__ void gms_rows_body(
     }
   }
   if constexpr (P == 3) {
+    float beyond = 0.f;                                      // (NaN where a sum is not finite)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[mt][nt][r] += low[mt][nt][r];
+        for (int r = 0; r < 16; ++r) {
+          acc[mt][nt][r] += low[mt][nt][r];
+          beyond = __builtin_fmaf(acc[mt][nt][r], 0.f, beyond);
+        }
+    if (__syncthreads_or(beyond != 0.f)) {                   // (also: every wave is through with LDS)
+      gms_rows_body<T, NT, S, RAW + 2, MT, KG, RAGGED>(src, RAW == 5 ? w_raw : packed, dst, nbr, block_masks, perm, tile_order, n_dst, k_vol,
+                                                       c_src, c_dst, part_stages, block_x, block_y, block_z, grid_z, src_bytes,
+                                                       pair_view, overwrite, flip, centre, nullptr);
+      return;
+    }
   }
   if constexpr (KG > 1) {
     // the groups' sums meet in the LDS behind the first group's
@@ -973,7 +1017,7 @@ __global__ __launch_bounds__(kThreads * KG, RAW >= 5 ? (MT == 2 || KG == 2 ? 2 :
     const int32_t *__restrict__ nbr, const unsigned long long *__restrict__ block_masks,
     const int32_t *__restrict__ perm, const int32_t *__restrict__ tile_order, int n_dst, int k_vol,
     int c_src, int c_dst, int part_stages, SideJob side, int pair_view, unsigned src_bytes, int overwrite,
-    int flip, unsigned long long centre) {
+    int flip, unsigned long long centre, const T *__restrict__ w_raw) {
   // the leading workgroups of the grid run the side job, if there is one
   int block_x = blockIdx.x;
   if (side.blocks) {
@@ -985,7 +1029,7 @@ __global__ __launch_bounds__(kThreads * KG, RAW >= 5 ? (MT == 2 || KG == 2 ? 2 :
   }
   gms_rows_body<T, NT, S, RAW, MT, KG, RAGGED>(src, packed, dst, nbr, block_masks, perm, tile_order, n_dst, k_vol, c_src,
                                    c_dst, part_stages, block_x, blockIdx.y, blockIdx.z, gridDim.z, src_bytes, pair_view,
-                                   overwrite, flip, centre);
+                                   overwrite, flip, centre, w_raw);
 }
 
 // ---------------------------------------------------------------------------
@@ -1341,7 +1385,7 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
     kern<<<dim3(gx + (unsigned)a.side.blocks, gy, gz), kThreads * kg, lds_rows, a.stream>>>(
         (const T *)a.src, packed, (T *)a.dst, nbr, masks, perm, tile_order, (int)a.n_dst, a.k_vol,
         s.c_src, s.c_dst, part_stages > 0 ? part_stages : 1, a.side, pair_view ? 1 : 0,
-        (unsigned)((size_t)a.n_src * s.c_src * sizeof(T)), overwrite ? 1 : 0, flip, a.centre ? 1ull << (a.centre - 1) : 0ull);
+        (unsigned)((size_t)a.n_src * s.c_src * sizeof(T)), overwrite ? 1 : 0, flip, a.centre ? 1ull << (a.centre - 1) : 0ull, (const T *)a.w);
   }
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;
@@ -1382,7 +1426,7 @@ __global__ __launch_bounds__(kThreads, NT >= 3 || RAWD == 6 || BI * BJ == 16 || 
   if ((int)blockIdx.x < rows_total) {
     const int bx = blockIdx.x % row_x, rest = blockIdx.x / row_x;
     gms_rows_body<T, NT, S, RAWD, MT, 1, RAGGED>(gout, w, gin, nbr, block_masks, perm, tile_order, n_in, k_vol, c_out, c_in,
-                                      part_stages, bx, rest % row_y, rest / row_y, row_z, gout_bytes, 0, overwrite, flip, 0);
+                                      part_stages, bx, rest % row_y, rest / row_y, row_z, gout_bytes, 0, overwrite, flip, 0, nullptr);
   } else {
     const int j = blockIdx.x - rows_total;
     if constexpr (BI <= 3 && BJ <= 3)

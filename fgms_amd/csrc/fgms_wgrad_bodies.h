@@ -161,8 +161,10 @@ template <> struct WTW<float> { static constexpr int stage_pairs = 16; };
 // SPLIT (fp32 tensors): the staged rows are split into so many bf16 parts on their way to LDS -- 16-bit tiles
 // of every part per wave, laid out like the fp16 path's two -- and a product is three (two parts, where the
 // caller allows tf32 precision) or six bf16 MFMAs, fed through the same transposing LDS reads as fp16.
-// RAGGED (fp16): the tile's channels from c_in / c_out on do not exist; they are loaded from outside the
-// buffers, as zeros, and not flushed.
+// Three parts: a workgroup whose sums are not all finite does its work again on fp32 MFMAs before anything is flushed (an
+// infinite value has no parts).
+// RAGGED (not fp32 MFMAs alone): the tile's channels from c_in / c_out on do not exist; they are loaded from outside the
+// buffers, or another chunk in their place, and count as zeros, and are not flushed.
 template <typename T, int BI, int BJ, int SPLIT = 0, bool RAGGED = false>
 __device__ __forceinline__ void wgrad_wave_body(
     const T *__restrict__ in, const T *__restrict__ gout, float *__restrict__ gw32,
@@ -181,7 +183,6 @@ __device__ __forceinline__ void wgrad_wave_body(
   constexpr int LDI = CI + (kBufW ? 0 : W::pad), LDO = CO + (kBufW ? 0 : W::pad);
   constexpr int NCI = CI / E, NCO = CO / E;
   constexpr int NX = SP * NCI / 64, NG = SP * NCO / 64;   // chunks per lane and stage
-  static_assert(!RAGGED || kBufW || SPLIT, "ragged: fp16, or fp32 in parts");
   static_assert(NX >= 1 && NG >= 1, "stage too small");
   extern __shared__ int4v lds[];
   int k, first, count;
@@ -312,7 +313,7 @@ __device__ __forceinline__ void wgrad_wave_body(
         *reinterpret_cast<int4v *>(x + x_row(i) * LDI + ((x_chunk(i) ^ (CI == 64 ? ((x_row(i) >> 1) & 1) * 4 : 0)) * E)) = xr[i];
       else
         *reinterpret_cast<int4v *>(x + (e / NCI) * LDI + (e % NCI) * E) =
-            st * SP + e / NCI < count ? xr[i] : int4v{0, 0, 0, 0};
+            st * SP + e / NCI < count && (!RAGGED || ci0 + e % NCI * E < c_in) ? xr[i] : int4v{0, 0, 0, 0};
     }
 #pragma unroll
     for (int i = 0; i < NG; ++i) {
@@ -324,7 +325,7 @@ __device__ __forceinline__ void wgrad_wave_body(
         *reinterpret_cast<int4v *>(g + g_row(i) * LDO + ((g_chunk(i) ^ (CO == 64 ? ((g_row(i) >> 1) & 1) * 4 : 0)) * E)) = gr[i];
       else
         *reinterpret_cast<int4v *>(g + (e / NCO) * LDO + (e % NCO) * E) =
-            st * SP + e / NCO < count ? gr[i] : int4v{0, 0, 0, 0};
+            st * SP + e / NCO < count && (!RAGGED || co0 + e % NCO * E < c_out) ? gr[i] : int4v{0, 0, 0, 0};
     }
   };
   auto wave_fence = [] {
@@ -418,12 +419,20 @@ __device__ __forceinline__ void wgrad_wave_body(
   }
 
   if constexpr (P == 3) {
+    float beyond = 0.f;                                  // (NaN where a sum is not finite)
 #pragma unroll
     for (int a = 0; a < BI; ++a)
 #pragma unroll
       for (int b = 0; b < BJ; ++b)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[a][b][r] += low[a][b][r];
+        for (int r = 0; r < 16; ++r) {
+          acc[a][b][r] += low[a][b][r];
+          beyond = __builtin_fmaf(acc[a][b][r], 0.f, beyond);
+        }
+    if (__syncthreads_or(beyond != 0.f)) {
+      wgrad_wave_body<T, BI, BJ, 0, RAGGED>(in, gout, gw32, kpos, imap, omap, k_vol, c_in, c_out, smap, block_x, block_y, in_bytes, gout_bytes);
+      return;
+    }
   }
   // Sum the four waves' tiles through LDS and flush.  Every wave ends up with a quarter of the
   // summed tile (accumulator registers q * R / 4 ... of the R a lane holds) and
