@@ -103,6 +103,7 @@ struct WgradArgs {
   // MFMA kernels, fp16: use this fp32 accumulator (k_vol * c_in * c_out floats, all zero)
   // instead of the stream's workspace; nothing is allocated then
   float *acc_override;
+  bool no_alloc;             // the caller cannot allocate: only kernels that take no workspace
   // the rows are padded copies: the caller's tensor is [k_vol, crop_in, crop_out] (0: [k_vol, c_in, c_out])
   int crop_in, crop_out;
 };

@@ -593,7 +593,7 @@ int launch_narrow_gms(const GmsArgs &a, const Plan *p) {
 }
 
 bool narrow_wgrad_supported(const WgradArgs &a, const Plan *p) {
-  if (!p || a.k_vol != p->k_vol || a.crop_in || a.acc_override) return false;
+  if (!p || a.k_vol != p->k_vol || a.crop_in || a.no_alloc) return false;
   auto tables = [&](const Plan *q) {
     return q->has_tables && q->nbr_out && q->fwd_ok && a.n_out == q->n_out && a.n_in == q->n_in && a.n_out > 0 && a.n_in > 0;
   };

@@ -650,6 +650,7 @@ int wgrad_static(WgradArgs a) {
   }
   a.side = SideJob{};
   a.deferred_flush = nullptr;
+  a.no_alloc = true;
   if (a.plan) plan_touch(a.plan, a.stream);
   return launch_mfma_wgrad(a);
 }

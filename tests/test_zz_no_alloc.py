@@ -98,3 +98,32 @@ def test_static_weight_gradient_allocates_nothing(capi):
     torch.cuda.synchronize()
     G.assert_close(got.cpu().numpy(), want.cpu().numpy(), "fp16", "static (fresh plan of a strided map) vs fgms_wgrad")
     plan.close()
+
+
+@pytest.mark.parametrize("dtype", [np.float16, np.float32], ids=["fp16", "fp32"])
+@pytest.mark.parametrize("c_in,c_out", [(4, 32), (8, 64)])
+def test_static_weight_gradient_of_narrow_layers_allocates_nothing(capi, oracle, c_in, c_out, dtype):
+    """A plan whose build results are known, clouds big enough for the kernel that leaves its workgroups' sums in a
+    workspace (fgms_wgrad's choice), on a stream that has none."""
+    L = layer(40000, c_in, c_out, dtype, 7)
+    D = G.to_dev(L)
+    maps = (D["kpos"], D["imap"], D["omap"])
+    plan = capi.Plan(*maps, D["n_in"], D["n_out"])
+    want = torch.zeros_like(D["kernel"])
+    capi.wgrad(D["in_feats"], D["out_grad"], want, *maps, plan=plan)
+    got = torch.zeros_like(D["kernel"])
+    capi.wgrad_static(D["in_feats"], D["out_grad"], got, *maps, plan=plan)      # (symbol address, LDS limits)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        got.zero_()
+    torch.cuda.synchronize()
+    before, free_before = capi.allocation_count(), torch.cuda.mem_get_info()[0]
+    with torch.cuda.stream(side):
+        capi.wgrad_static(D["in_feats"], D["out_grad"], got, *maps, plan=plan)
+    torch.cuda.synchronize()
+    assert capi.allocation_count() == before
+    assert torch.cuda.mem_get_info()[0] == free_before
+    G.assert_close(got.cpu().numpy(), want.cpu().numpy(), G.mode_of(dtype), "static vs fgms_wgrad")
+    ref = oracle.np_wgrad(L["in_feats"], L["out_grad"], L["knnz"], L["imap"], L["omap"], L["k_vol"])
+    G.assert_close(got.cpu().numpy(), ref, G.mode_of(dtype), "static vs oracle")
+    plan.close()
