@@ -805,6 +805,7 @@ bool padded_wgrad_channels(const WgradArgs &a, int *c_in, int *c_out) {
     p.c_out = up_to_32(a.c_out);
   }
   *c_in = p.c_in; *c_out = p.c_out;
+  p.crop_in = a.c_in; p.crop_out = a.c_out;      // (what will run, and at what price)
   return mfma_wgrad_supported(p) && (a.dtype == FGMS_F16 || padded_wgrad_us(p) < vector_alu_wgrad_us(a));
 }
 
@@ -922,6 +923,8 @@ bool padded_bwd_channels(const GmsArgs &d, const Plan *p, const WgradArgs &w, in
     pw.in = pw.gout = (const void *)4096;
     pw.c_in = *c_in;
     pw.c_out = *c_out;
+    pw.crop_in = w.c_in;
+    pw.crop_out = w.c_out;
     if (!tuned_gms(with_channels(d, *c_in, *c_out), p) || !mfma_wgrad_supported(pw)) continue;
     return d.dtype == FGMS_F16 || together_pays(d, p, w, with_channels(d, *c_in, *c_out), pw);
   }

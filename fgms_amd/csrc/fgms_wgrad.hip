@@ -430,9 +430,7 @@ bool mfma_wgrad_supported(const WgradArgs &a) { return takes_narrow(a) || mfma_w
 double padded_wgrad_us(const WgradArgs &p) {
   double per_row = 0, cells = 1;
   WgradGeometry g;
-  if (takes_narrow(p)) {
-    return 19;
-  } else if (skinny_shape(p)) {
+  if (skinny_shape(p)) {
     per_row = 0.076 / 512 * p.c_in * p.c_out;
     cells = (double)choose_slices(p, 1, 64, (int64_t)num_cus() * 2).slices * p.k_vol;
   } else if (wgrad_geometry(p, &g) == FGMS_OK) {
