@@ -1324,8 +1324,11 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
   // fp32 tensors: products of bf16 parts, two to a value in "tf32" mode, else three (three or six 16-bit MFMAs instead
   // of sixteen fp32 ones per product tile); needs whole 32-channel slabs
   constexpr bool kCanSplit = sizeof(T) == 4 && S == 4 && NT != 4;
+  // (Three parts take 6 bytes a weight, at 32-bit offsets: a stream under capture whose workspace holds only the 4 of the other
+  // layouts stays on fp32 MFMAs.  Masked channel counts come here with room for them.)
+  const size_t three = (size_t)a.k_vol * a.c_in * a.c_out * 6;
   const bool split = kCanSplit && !a.transpose_w && !a.prepacked && split_bf16_enabled() &&
-                     (a.reduced || (NT != 3 && (size_t)a.k_vol * a.c_in * a.c_out <= 0xfffffff0u / 6));     // (32-bit offsets)
+                     (a.reduced || RAGGED || (NT != 3 && three <= 0xfffffff0u && (!is_capturing(a.stream) || workspace_bytes(a.stream, 0) >= three)));
   if (kCanSplit && raw == 2 && split_bf16_enabled()) raw = a.reduced ? 4 : NT != 3 ? 6 : 2;   // (the input gradient splits as it reads)
   const T *packed = raw ? (const T *)a.w : (const T *)a.prepacked;
   if (split) {

@@ -111,3 +111,33 @@ def test_replays_after_the_plan_cache_moved_on():
             G.assert_close(out.cpu().numpy(), want.cpu().numpy(), "fp16", "replay")
     finally:
         backend.fgms_plan_cache(True, 8)
+
+
+def test_fp32_capture_in_the_workspace_of_another_mode():
+    """A stream that has run a layer in tf32 mode holds 4 bytes a weight: a capture of the layer in fp32 finds a kernel that
+    needs no more, and its replays give the eager results."""
+    from fgms_amd import capi
+    capi.set_kernel_policy(0)
+    D = G.to_dev(cloud_layer(9000, 64, 64, np.float32))
+    maps = (D["kpos"], D["imap"], D["omap"])
+    plan = capi.Plan(*maps, D["n_in"], D["n_out"])
+    side, out = torch.cuda.Stream(), torch.empty_like(D["out_grad"])
+    want = torch.empty_like(out)
+    capi.conv_fwd(D["in_feats"], D["kernel"], want, *maps, plan=plan)
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        capi.conv_fwd(D["in_feats"], D["kernel"], out, *maps, arch80=True, plan=plan)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side, capture_error_mode="thread_local"):
+        capi.conv_fwd(D["in_feats"], D["kernel"], out, *maps, plan=plan)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        G.assert_close(out.cpu().numpy(), want.cpu().numpy(), "fp32", "replay")
+        with torch.cuda.stream(side):                  # (the buffer grows: the graph keeps the one it points at)
+            capi.conv_fwd(D["in_feats"], D["kernel"], out, *maps, plan=plan)
+        torch.cuda.synchronize()
+        G.assert_close(out.cpu().numpy(), want.cpu().numpy(), "fp32", "eager")
+    plan.close()
