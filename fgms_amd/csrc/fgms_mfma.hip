@@ -237,12 +237,11 @@ __device__ __forceinline__ void mma_slab_rawt(float16v (&acc)[MT][NT], const int
 // time.  Rows are split when they go from registers to LDS, the weights by their re-layout
 // kernel.
 //
-// The same for fp32 tensors in full precision, with three parts and six products (RAW = 5 and 6): x = h + m + l holds
-// all 24 bits, and what is dropped of a product (m*l, l*m, l*l) is below 2^-23 of it and of either sign, less than the fp32
-// sum around it rounds off (mma_parts has the errors).  Six 16-bit matrix steps take 6/16 of the fp32 ones' time; a
-// tile of rows takes half as much LDS again, which leaves two workgroups to a CU.  fp32 MFMAs / this: 64 -> 64 forward over
-// 40 k voxels 88 / 63 us, 150 k 172 / 111; backward 123 / 77, 342 / 232; 128 -> 128 over 40 k 231 / 133 and 360 / 238;
-// 32 -> 32 over 4 k 25 / 21 and 20 / 18.5.  (A value below 2^-110 or so loses the last bits of its small parts.)
+// The same for fp32 tensors in full precision, with three parts and eight products (RAW = 5 and 6): x = h + m + l holds
+// all 24 bits, and a product is rounded once, as by fp32 arithmetic (mma_parts).  Eight 16-bit matrix steps take half of the
+// fp32 ones' time; a tile of rows takes half as much LDS again, which leaves two workgroups to a CU.  fp32 MFMAs / this:
+// 64 -> 64 forward over 40 k voxels 88 / 73 us, 200 k 227 / 164; backward 116 / 87, 398 / 312; 128 -> 128 over 40 k 249 / 161
+// and 349 / 257; 32 -> 32 over 2 k 24.3 / 21.6 and 20.0 / 19.5.  (A value below 2^-110 or so loses the last bits of its small parts.)
 // The parts of an infinite value are no numbers, so sums that reach one come out as NaN or infinite whatever else is in
 // them, and a workgroup that ends up with such a sum does its work again with fp32 MFMAs (RAW = 7 and 8; the tile is
 // written only then): what an infinity reaches is what fp32 arithmetic makes of it, in that tile at the price of both.
@@ -1321,7 +1320,7 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (!(a.stream && hipStreamIsCapturing(a.stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone)) raw = 0;
   }
-  // fp32 tensors: products of bf16 parts, two to a value in "tf32" mode, else three (three or six 16-bit MFMAs instead
+  // fp32 tensors: products of bf16 parts, two to a value in "tf32" mode, else three (three or eight 16-bit MFMAs instead
   // of sixteen fp32 ones per product tile); needs whole 32-channel slabs
   constexpr bool kCanSplit = sizeof(T) == 4 && S == 4 && NT != 4;
   // (Three parts take 6 bytes a weight, at 32-bit offsets: a stream under capture whose workspace holds only the 4 of the other

@@ -74,17 +74,17 @@ __device__ __forceinline__ void split_parts(const float4v &x, int2v (&part)[P]) 
   }
 }
 
-// acc += a x b for operands of P parts: the products whose parts' ranks add up to less than P, the small ones first.
-// P = 3: the small ones have an accumulator of their own, `low`, to be added at the end: the big one is then rounded once
-// per 16 products (a chain of fp32 MFMAs: eight times), and the sums come out closer to the exact ones than those of
-// fp32 arithmetic: 64 -> 64 over 100 k voxels, relative error (2-norm) of forward pass / weight gradient against
-// float64 1.5e-7 / 1.7e-7, with fp32 MFMAs 4.8e-7 / 4.0e-7, with one accumulator for all six products 4.0e-7 / 4.4e-7.
+// acc += a x b for operands of P parts, the small products first.  P = 2: all but lo x lo.  P = 3: all but l x l, which is
+// below 2^-30 of the product, so that a single product is rounded once, as by fp32 arithmetic (without m x l and l x m, which
+// reach 1.7 x 2^-23 of it, its error was up to 3.9 x 2^-24).  The small ones have an accumulator of their own, `low`, to be added
+// at the end: the big one is then rounded once per 16 products.
 template <int P>
 __device__ __forceinline__ void mma_parts(float16v &acc, float16v &low, const bf16x8 (&a)[P], const bf16x8 (&b)[P]) {
 #pragma unroll
-  for (int rank = P - 1; rank >= 0; --rank)
+  for (int rank = P == 3 ? 3 : 1; rank >= 0; --rank)
 #pragma unroll
-    for (int i = rank; i >= 0; --i) {
+    for (int i = P - 1; i >= 0; --i) {
+      if (i > rank || rank - i >= P) continue;
       float16v &to = P == 3 && rank > 0 ? low : acc;
       to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[rank - i], to, 0, 0, 0);
     }

@@ -160,7 +160,7 @@ template <> struct WTW<float> { static constexpr int stage_pairs = 16; };
 // (block_x, block_y): the workgroup's place in a grid of cells x tiles of dW[k]; 256 threads.
 // SPLIT (fp32 tensors): the staged rows are split into so many bf16 parts on their way to LDS -- 16-bit tiles
 // of every part per wave, laid out like the fp16 path's two -- and a product is three (two parts, where the
-// caller allows tf32 precision) or six bf16 MFMAs, fed through the same transposing LDS reads as fp16.
+// caller allows tf32 precision) or eight bf16 MFMAs, fed through the same transposing LDS reads as fp16.
 // Three parts: a workgroup whose sums are not all finite does its work again on fp32 MFMAs before anything is flushed (an
 // infinite value has no parts).
 // RAGGED (not fp32 MFMAs alone): the tile's channels from c_in / c_out on do not exist; they are loaded from outside the
