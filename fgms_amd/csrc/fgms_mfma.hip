@@ -240,11 +240,11 @@ __device__ __forceinline__ void mma_slab_rawt(float16v (&acc)[MT][NT], const int
 // The same for fp32 tensors in full precision, with three parts and eight products (RAW = 5 and 6): x = h + m + l holds
 // all 24 bits, and a product is rounded once, as by fp32 arithmetic (mma_parts).  Eight 16-bit matrix steps take half of the
 // fp32 ones' time; a tile of rows takes half as much LDS again, which leaves two workgroups to a CU.  fp32 MFMAs / this:
-// 64 -> 64 forward over 40 k voxels 88 / 73 us, 200 k 227 / 164; backward 116 / 87, 398 / 312; 128 -> 128 over 40 k 249 / 161
-// and 349 / 257; 32 -> 32 over 2 k 24.3 / 21.6 and 20.0 / 19.5.  (A value below 2^-110 or so loses the last bits of its small parts.)
-// The parts of an infinite value are no numbers, so sums that reach one come out as NaN or infinite whatever else is in
-// them, and a workgroup that ends up with such a sum does its work again with fp32 MFMAs (RAW = 7 and 8; the tile is
-// written only then): what an infinity reaches is what fp32 arithmetic makes of it, in that tile at the price of both.
+// 64 -> 64 forward over 40 k voxels 88 / 76 us, 200 k 227 / 165; backward 116 / 91, 398 / 319; 128 -> 128 over 40 k 249 / 161
+// and 349 / 271; 32 -> 32 over 20 k 25.4 / 23.2 and 25.6 / 24.0.
+// What the parts cannot hold goes to fp32 MFMAs (RAW = 7 and 8): sums that an infinite value reaches come out as NaN or infinite
+// whatever else is in them, and a value too small for them (below 2^-102 at most) is noted when it is split, so that a workgroup that has met either does its
+// work again before it writes its tile, in that tile at the price of both.
 //
 // Slot (16 bytes = 8 bf16) of a split tile of P parts: row-major, a row holds its 32 values of the slab
 // as 4 chunks of each part; the XOR spreads the rows one b128 read pass (16 lanes) touches over all banks: rows of
@@ -256,9 +256,9 @@ __device__ __forceinline__ int part_slot(int row, int part, int j) {
 
 // One fp32 chunk (4 values; chunk c of its row's slab) split and written to a split tile: 8 bytes of each part.
 template <int P>
-__device__ __forceinline__ void split_and_store(int4v *__restrict__ tile, const float4v &x, int row, int c) {
+__device__ __forceinline__ void split_and_store(int4v *__restrict__ tile, const float4v &x, int row, int c, bool &lost) {
   int2v part[P];
-  split_parts<P>(x, part);
+  split_parts<P>(x, part, lost);
 #pragma unroll
   for (int q = 0; q < P; ++q) reinterpret_cast<int2v *>(tile)[part_slot<P>(row, q, c / 2) * 2 + (c & 1)] = part[q];
 }
@@ -271,7 +271,8 @@ __device__ __forceinline__ void gather_commit_parts(int4v *__restrict__ a_lds, i
   for (int it = 0; it < N; ++it) {
     const int slot = it * 64 + lane;
     const float4v x = g[it] < 0 ? float4v{0.f, 0.f, 0.f, 0.f} : __builtin_bit_cast(float4v, v[it]);
-    split_and_store<P>(a_lds, x, slot / 8, slot % 8);
+    bool lost = false;      // (two parts: not used)
+    split_and_store<P>(a_lds, x, slot / 8, slot % 8, lost);
   }
 }
 
@@ -305,6 +306,7 @@ __device__ __forceinline__ void mma_slab_parts(float16v (&acc)[MT][NT], float16v
 // holds the 8 values op(W[k])[slab*32 + s*16 + (lane/32)*8 + 0..7][nt*32 + lane%32] of that part.
 // One thread per P chunks.
 // (Channels that fill no whole tile: zeros behind them.)
+// A chunk with a weight that three parts do not hold is marked with a NaN, which takes every tile that meets it to fp32 MFMAs and the weights as they are.
 template <int P>
 __global__ void pack_weights_parts_kernel(const float *__restrict__ w, int4v *__restrict__ packed,
                                           int k_vol, int c_in, int c_out, bool transpose) {
@@ -326,8 +328,10 @@ __global__ void pack_weights_parts_kernel(const float *__restrict__ w, int4v *__
       x[e / 4][e % 4] = cs0 + e >= c_src || cd >= c_dst ? 0.f
                         : transpose ? w[((size_t)k * c_in + cd) * c_out + cs0 + e] : w[((size_t)k * c_in + cs0 + e) * c_out + cd];
     int2v lo[P], hi[P];
-    split_parts<P>(x[0], lo);
-    split_parts<P>(x[1], hi);
+    bool lost = false;
+    split_parts<P>(x[0], lo, lost);
+    split_parts<P>(x[1], hi, lost);
+    if (P == 3 && lost) lo[0][0] = 0x7fc07fc0;
     const size_t base = (t / 64) * (64 * P) + lane;
 #pragma unroll
     for (int part = 0; part < P; ++part) packed[base + part * 64] = int4v{lo[part][0], lo[part][1], hi[part][0], hi[part][1]};
@@ -410,11 +414,11 @@ __device__ __forceinline__ void gather_commit_buf(int4v *__restrict__ a_lds, con
 }
 
 template <int P, int N>
-__device__ __forceinline__ void gather_commit_parts_buf(int4v *__restrict__ a_lds, const int4v (&v)[N], int lane) {
+__device__ __forceinline__ void gather_commit_parts_buf(int4v *__restrict__ a_lds, const int4v (&v)[N], int lane, bool &lost) {
 #pragma unroll
   for (int it = 0; it < N; ++it) {
     const int slot = it * 64 + lane;
-    split_and_store<P>(a_lds, __builtin_bit_cast(float4v, v[it]), slot / 8, slot % 8);
+    split_and_store<P>(a_lds, __builtin_bit_cast(float4v, v[it]), slot / 8, slot % 8, lost);
   }
 }
 
@@ -706,6 +710,8 @@ __device__ __forceinline__ void gms_rows_body(
       for (int nt = 0; nt < NT; ++nt) low[mt][nt] = acc[mt][nt];
   }
 
+  bool lost = false;                                      // ... met a value they do not hold (split_parts)
+
   // Weights of stage (k, slab), 16-byte chunk e = threadIdx.x + kThreads * i of the stage's tile,
   // through a buffer resource over the weight tensor: the part of a chunk's address that depends
   // on the thread is a per-lane constant (wvoff), the part that depends on the stage is scalar.
@@ -777,7 +783,7 @@ __device__ __forceinline__ void gms_rows_body(
         } else if constexpr (RAW == 2 || RAW == 8) {
           w_lds[buf * WCH + a_slot<S>(e / C, e % C)] = wreg[i];
         } else if constexpr (RAW == 4 || RAW == 6) {
-          split_and_store<P>(w_lds + buf * WCH, __builtin_bit_cast(float4v, wreg[i]), e / C, e % C);
+          split_and_store<P>(w_lds + buf * WCH, __builtin_bit_cast(float4v, wreg[i]), e / C, e % C, lost);
         } else {
           w_lds[buf * WCH + e] = wreg[i];
         }
@@ -800,7 +806,7 @@ __device__ __forceinline__ void gms_rows_body(
     else gather_issue<T, S>(v, gsel, gidx, src, c_src, slab_, lane);
   };
   auto rows_commit = [&]() {
-    if constexpr (P > 0) gather_commit_parts_buf<P>(a_lds, v, lane);
+    if constexpr (P > 0) gather_commit_parts_buf<P>(a_lds, v, lane, lost);
     else if constexpr (kBuf) gather_commit_buf<S>(a_lds, v, lane);
     else gather_commit<S>(a_lds, v, gsel, lane);
   };
@@ -956,7 +962,7 @@ __device__ __forceinline__ void gms_rows_body(
     }
   }
   if constexpr (P == 3) {
-    float beyond = 0.f;                                      // (NaN where a sum is not finite)
+    float beyond = 0.f;                                      // (NaN where a sum is not finite: an infinity, a weight that is marked)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -966,7 +972,7 @@ __device__ __forceinline__ void gms_rows_body(
           acc[mt][nt][r] += low[mt][nt][r];
           beyond = __builtin_fmaf(acc[mt][nt][r], 0.f, beyond);
         }
-    if (__syncthreads_or(beyond != 0.f)) {                   // (also: every wave is through with LDS)
+    if (__syncthreads_or(beyond != 0.f || lost)) {          // (also: every wave is through with LDS)
       gms_rows_body<T, NT, S, RAW + 2, MT, KG, RAGGED>(src, RAW == 5 ? w_raw : packed, dst, nbr, block_masks, perm, tile_order, n_dst, k_vol,
                                                        c_src, c_dst, part_stages, block_x, block_y, block_z, grid_z, src_bytes,
                                                        pair_view, overwrite, flip, centre, nullptr);

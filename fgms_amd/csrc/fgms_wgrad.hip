@@ -54,7 +54,7 @@ __global__ __launch_bounds__(kThreads) void wgrad_kernel(
 
 // The per-wave variant (wgrad_wave_body) in a launch of its own.
 template <typename T, int BI, int BJ, int SPLIT>
-__global__ __launch_bounds__(kThreads, BI * BJ >= 6 || SPLIT == 3 ? 2 : 3) void wgrad_wave_kernel(
+__global__ __launch_bounds__(kThreads, BI * BJ >= 6 || (SPLIT == 3 && BI * BJ == 4) ? 2 : 3) void wgrad_wave_kernel(
     const T *__restrict__ in, const T *__restrict__ gout, float *__restrict__ gw32,
     const int32_t *__restrict__ kpos, const int32_t *__restrict__ imap,
     const int32_t *__restrict__ omap, int k_vol, int c_in, int c_out, SliceMap smap, SideJob side,

@@ -140,9 +140,11 @@ __device__ __forceinline__ bool locate_slice(const int32_t *__restrict__ kpos, c
 // Split staging (fp32 rows): chunk c (4 fp32 values) of a staged row becomes 4 bf16 values in each of P
 // 16-bit tiles laid out like the fp16 path's, `stride` halfs apart.
 template <int P>
-__device__ __forceinline__ void store_split_chunk(__half *tiles, int stride, int ld, int row, int c, const int4v &raw, bool valid) {
+__device__ __forceinline__ void store_split_chunk(__half *tiles, int stride, int ld, int row, int c, const int4v &raw, bool valid,
+                                                  bool &lost) {
   int2v part[P];
-  split_parts<P>(valid ? __builtin_bit_cast(float4v, raw) : float4v{0.f, 0.f, 0.f, 0.f}, part);
+  const float4v x = valid ? __builtin_bit_cast(float4v, raw) : float4v{0.f, 0.f, 0.f, 0.f};
+  split_parts<P>(x, part, lost);
 #pragma unroll
   for (int q = 0; q < P; ++q) *reinterpret_cast<int2v *>(tiles + q * stride + row * ld + c * 4) = part[q];
 }
@@ -161,8 +163,8 @@ template <> struct WTW<float> { static constexpr int stage_pairs = 16; };
 // SPLIT (fp32 tensors): the staged rows are split into so many bf16 parts on their way to LDS -- 16-bit tiles
 // of every part per wave, laid out like the fp16 path's two -- and a product is three (two parts, where the
 // caller allows tf32 precision) or eight bf16 MFMAs, fed through the same transposing LDS reads as fp16.
-// Three parts: a workgroup whose sums are not all finite does its work again on fp32 MFMAs before anything is flushed (an
-// infinite value has no parts).
+// Three parts: a workgroup whose sums are not all finite (an infinite value has no parts), or that has met a value too small for
+// them, does its work again on fp32 MFMAs before anything is flushed.
 // RAGGED (not fp32 MFMAs alone): the tile's channels from c_in / c_out on do not exist; they are loaded from outside the
 // buffers, or another chunk in their place, and count as zeros, and are not flushed.
 template <typename T, int BI, int BJ, int SPLIT = 0, bool RAGGED = false>
@@ -213,6 +215,7 @@ __device__ __forceinline__ void wgrad_wave_body(
 #pragma unroll
       for (int b = 0; b < BJ; ++b) low[a][b] = acc[a][b];
   }
+  bool lost = false;                                   // ... met a value they do not hold (split_parts)
 
   const int nstages = (count + SP - 1) / SP;
   int xi[NX], gi[NG];        // gather rows of the next stage to load
@@ -308,7 +311,7 @@ __device__ __forceinline__ void wgrad_wave_body(
       const int e = lane + 64 * i;
       if constexpr (SPLIT)
         store_split_chunk<P>(xs, SP * LDIh, LDIh, e / NCI, e % NCI, xr[i],
-                             st * SP + e / NCI < count && (!RAGGED || ci0 + e % NCI * E < c_in));
+                             st * SP + e / NCI < count && (!RAGGED || ci0 + e % NCI * E < c_in), lost);
       else if constexpr (kBufW)
         *reinterpret_cast<int4v *>(x + x_row(i) * LDI + ((x_chunk(i) ^ (CI == 64 ? ((x_row(i) >> 1) & 1) * 4 : 0)) * E)) = xr[i];
       else
@@ -320,7 +323,7 @@ __device__ __forceinline__ void wgrad_wave_body(
       const int e = lane + 64 * i;
       if constexpr (SPLIT)
         store_split_chunk<P>(gs, SP * LDOh, LDOh, e / NCO, e % NCO, gr[i],
-                             st * SP + e / NCO < count && (!RAGGED || co0 + e % NCO * E < c_out));
+                             st * SP + e / NCO < count && (!RAGGED || co0 + e % NCO * E < c_out), lost);
       else if constexpr (kBufW)
         *reinterpret_cast<int4v *>(g + g_row(i) * LDO + ((g_chunk(i) ^ (CO == 64 ? ((g_row(i) >> 1) & 1) * 4 : 0)) * E)) = gr[i];
       else
@@ -429,7 +432,7 @@ __device__ __forceinline__ void wgrad_wave_body(
           acc[a][b][r] += low[a][b][r];
           beyond = __builtin_fmaf(acc[a][b][r], 0.f, beyond);
         }
-    if (__syncthreads_or(beyond != 0.f)) {
+    if (__syncthreads_or(beyond != 0.f || lost)) {
       wgrad_wave_body<T, BI, BJ, 0, RAGGED>(in, gout, gw32, kpos, imap, omap, k_vol, c_in, c_out, smap, block_x, block_y, in_bytes, gout_bytes);
       return;
     }
@@ -564,12 +567,13 @@ __device__ __forceinline__ void wgrad_wg_body(
     }
   };
   auto store_rows = [&](int buf, int st, const int4v (&xr)[NX], const int4v (&gr)[NG]) {
+    bool lost = false;      // (two parts: not used)
 #pragma unroll
     for (int i = 0; i < NX; ++i) {
       const int e = tid + kThreads * i;
       if constexpr (SPLIT) {
         __half *xh = stage0h + buf * kBufHalfs;
-        store_split_chunk<2>(xh, SP * LDIh, LDIh, e / NCI, e % NCI, xr[i], st * SP + e / NCI < count);
+        store_split_chunk<2>(xh, SP * LDIh, LDIh, e / NCI, e % NCI, xr[i], st * SP + e / NCI < count, lost);
       } else {
         *reinterpret_cast<int4v *>(stage0 + buf * kBufElems + (e / NCI) * LDI + (e % NCI) * E) =
             st * SP + e / NCI < count ? xr[i] : int4v{0, 0, 0, 0};
@@ -580,7 +584,7 @@ __device__ __forceinline__ void wgrad_wg_body(
       const int e = tid + kThreads * i;
       if constexpr (SPLIT) {
         __half *gh = stage0h + buf * kBufHalfs + SP * 2 * LDIh;
-        store_split_chunk<2>(gh, SP * LDOh, LDOh, e / NCO, e % NCO, gr[i], st * SP + e / NCO < count);
+        store_split_chunk<2>(gh, SP * LDOh, LDOh, e / NCO, e % NCO, gr[i], st * SP + e / NCO < count, lost);
       } else {
         *reinterpret_cast<int4v *>(stage0 + buf * kBufElems + SP * LDI + (e / NCO) * LDO + (e % NCO) * E) =
             st * SP + e / NCO < count ? gr[i] : int4v{0, 0, 0, 0};

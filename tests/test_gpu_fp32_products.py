@@ -1,4 +1,5 @@
-"""fp32 layers in full precision whose results are one product each: rounded once, as by fp32 arithmetic, on every route."""
+"""fp32 layers in full precision whose results are one product each: rounded once, as by fp32 arithmetic, on every route, also where
+a factor is far below the ordinary range (down to subnormal numbers) and the other as far above it."""
 import pytest
 import torch
 
@@ -7,7 +8,7 @@ from tests.test_gpu_fp32_special import CASES, Layer
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("small", ["none"])
+@pytest.mark.parametrize("small", ["none", "rows", "weights", "gradients"])
 @pytest.mark.parametrize("n,shape,cloud", CASES)
 def test_single_products(n, shape, cloud, small):
     layer = Layer(n, shape, cloud)
@@ -15,6 +16,16 @@ def test_single_products(n, shape, cloud, small):
     k = int(torch.bincount(layer.offset[layer.offset != 13], minlength=27).argmax())
     pair = layer.offset == k
     row = int(layer.om[pair][n // 50])
+
+    if small != "none":
+        down, up = 2.0 ** -125, 2.0 ** 58
+        tiny = torch.tensor([0, n // 3, row, int(layer.im[pair][n // 50]), layer.n - 1], device="cuda")
+        x, w, g = (t * up for t in (x, w, g))
+        for t, name in ((x, "rows"), (g, "gradients")):
+            if small == name:
+                t[tiny] = t[tiny] / up * down
+        if small == "weights":
+            w[k, 5:] = w[k, 5:] / up * down
 
     # one weight to a column and to a row, at one offset; one row of output gradients
     c = min(shape)
