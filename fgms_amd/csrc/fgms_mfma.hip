@@ -1329,12 +1329,16 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
   // fp32 tensors: products of bf16 parts, two to a value in "tf32" mode, else three (three or eight 16-bit MFMAs instead
   // of sixteen fp32 ones per product tile); needs whole 32-channel slabs
   constexpr bool kCanSplit = sizeof(T) == 4 && S == 4 && NT != 4;
+  // (The pair view at 32 columns gathers as much for half the products, and its atomics bound it: fp32 MFMAs / three parts
+  // 32 -> 32 over 5 k scattered voxels 16 / 18 us, 96 -> 96 over 60 k LiDAR ones 144 / 162; at 64 columns 64 -> 64 over 60 k 97 / 97,
+  // 256 -> 256 over 5 k scattered ones 84 / 63.)
+  const bool three_parts = NT != 3 && !(pair_view && NT == 1);
   // (Three parts take 6 bytes a weight, at 32-bit offsets: a stream under capture whose workspace holds only the 4 of the other
   // layouts stays on fp32 MFMAs.  Masked channel counts come here with room for them.)
-  const size_t three = (size_t)a.k_vol * a.c_in * a.c_out * 6;
+  const size_t bytes = (size_t)a.k_vol * a.c_in * a.c_out * 6;
   const bool split = kCanSplit && !a.transpose_w && !a.prepacked && split_bf16_enabled() &&
-                     (a.reduced || RAGGED || (NT != 3 && three <= 0xfffffff0u && (!is_capturing(a.stream) || workspace_bytes(a.stream, 0) >= three)));
-  if (kCanSplit && raw == 2 && split_bf16_enabled()) raw = a.reduced ? 4 : NT != 3 ? 6 : 2;   // (the input gradient splits as it reads)
+                     (a.reduced || RAGGED || (three_parts && bytes <= 0xfffffff0u && (!is_capturing(a.stream) || workspace_bytes(a.stream, 0) >= bytes)));
+  if (kCanSplit && raw == 2 && split_bf16_enabled()) raw = a.reduced ? 4 : three_parts ? 6 : 2;   // (the input gradient splits as it reads)
   const T *packed = raw ? (const T *)a.w : (const T *)a.prepacked;
   if (split) {
     const void *ws = nullptr;
@@ -1438,7 +1442,7 @@ __global__ __launch_bounds__(kThreads, NT >= 3 || RAWD == 6 || BI * BJ == 16 || 
   } else {
     const int j = blockIdx.x - rows_total;
     if constexpr (BI <= 3 && BJ <= 3)
-      wgrad_wave_body<T, BI, BJ, split_parts_of(RAWD), RAGGED>(in, gout, gw32, kpos, imap, omap, k_vol, c_in, c_out, smap,
+      wgrad_wave_body<T, BI, BJ, RAWD == 6 && BI * BJ == 1 ? 0 : split_parts_of(RAWD), RAGGED>(in, gout, gw32, kpos, imap, omap, k_vol, c_in, c_out, smap,
                                             j % wgrad_x, j / wgrad_x, in_bytes, gout_bytes);
     else
       wgrad_wg_body<T, BI, BJ, RAWD == 4>(in, gout, gw32, kpos, imap, omap, k_vol, c_in, c_out, smap,
@@ -1459,8 +1463,12 @@ int launch_fused(const GmsArgs &d, const Shape &s, const Plan *p, const WgradArg
   const int slabs = (s.c_src + 2 * S * s.E - 1) / (2 * S * s.E);
   const unsigned row_y = (unsigned)((s.c_dst + 32 * NT - 1) / (32 * NT));
   constexpr bool kCanHalf = NT != 4;
+  // RAWD: how the input gradient reads the weights (2: as they lie; 4, 6: also split into bf16
+  // parts, for fp32 tensors)
+  constexpr bool kCanSplit = sizeof(T) == 4 && S == 4 && NT != 4, kCan3 = kCanSplit && BI <= 2 && BJ <= 2;
+  const int raw = !kCanSplit || !split_bf16_enabled() ? 2 : d.reduced ? 4 : kCan3 ? 6 : 2;
   const RowsGrid rg = rows_grid(d.n_dst, row_y, d.k_vol * slabs, kCanHalf, p->tile_in != nullptr, p->tile_grid_in,
-                                false, NT >= 3 || g.split == 3 ? 2 : 3, true, false);
+                                false, NT >= 3 || raw == 6 ? 2 : 3, true, false);
   const unsigned row_x = (rg.gx + 7) / 8 * 8;
   const int part_stages = rg.part_stages;
   const unsigned row_z = rg.gz;
@@ -1472,10 +1480,6 @@ int launch_fused(const GmsArgs &d, const Shape &s, const Plan *p, const WgradArg
                                         zero_gw ? (size_t)w.k_vol * w.c_in * w.c_out * sizeof(float) : 0, d.stream);
     if (rc != FGMS_OK) return rc;
   }
-  // RAWD: how the input gradient reads the weights (2: as they lie; 4, 6: also split into bf16
-  // parts, for fp32 tensors)
-  constexpr bool kCanSplit = sizeof(T) == 4 && S == 4 && NT != 4, kCan3 = kCanSplit && BI <= 2 && BJ <= 2;
-  const int raw = kCan3 && g.split == 3 ? 6 : kCanSplit && g.split == 2 ? 4 : 2;
   constexpr int kRaw2 = RAGGED && sizeof(T) == 4 ? 4 : 2;        // (masked fp32 shapes come in parts only)
   constexpr int kHalfMT = kCanHalf ? 1 : 2;
   constexpr int kRaw4 = kCanSplit ? 4 : 2, kRaw6 = kCan3 ? 6 : 2;

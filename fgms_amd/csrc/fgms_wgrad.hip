@@ -269,10 +269,15 @@ void tile_blocks(const WgradArgs &a, bool shares_grid, int *bi, int *bj) {
   *bj = blocks_of(a.c_out, three);
   if (*bi == 3 && *bj == 4) *bj = 2;     // (96 channels: the per-wave body)
   if (*bj == 3 && *bi == 4) *bi = 2;
-  // (fp32 in three parts: the per-wave body only)
+  // (fp32 in three parts: the per-wave body only.  A launch of 128 x 128 tiles whose gathers count stays on fp32 MFMAs, which read a
+  // row once per 128 channels: thin maps, and few pairs of many tiles.  fp32 MFMAs / three parts: 128 x 128 over 50 k
+  // scattered voxels, 3.5 pairs a row, 95 / 119 us, over 60 k LiDAR ones, 5.7, 147 / 168, indoor 20 k, 10.5, 110 / 83; 256 x 256 over
+  // 500 voxels 25 / 54, 2 k 61 / 60, scattered 20 k 181 / 150.)
   if (a.dtype != FGMS_F16 && !a.reduced && split_bf16_enabled()) {
-    if (*bi > 2) *bi = 2;
-    if (*bj > 2) *bj = 2;
+    const int64_t tiles = (int64_t)(a.c_in / 128) * (a.c_out / 128), rows = a.n_in > a.n_out ? a.n_in : a.n_out;
+    const bool whole = !shares_grid && *bi * *bj == 16 && ((tiles <= 2 && a.n_pairs < 7 * rows) || (tiles >= 2 && a.n_pairs * tiles < 70000));
+    if (*bi > 2 && !whole) *bi = 2;
+    if (*bj > 2 && !whole) *bj = 2;
   }
   if (!shares_grid && a.dtype == FGMS_F16 && *bi * *bj == 16) {
     *bi = 2;
@@ -457,11 +462,11 @@ static void wave_geometry(const WgradArgs &a, WgradGeometry *g, bool shares_grid
   g->smap = choose_slices(a, g->ty, sp, (int64_t)num_cus() * 6);
   g->tiles = (int64_t)g->smap.slices * a.k_vol;
   // fp32 tensors: 16-bit tiles of every part instead
-  // (Three parts in a launch of tiles of one or two blocks only where each cell walks many pairs: a walk of few is mostly
-  // the splits and the wait for its first rows.  fp32 MFMAs / three parts: 32 x 32 over 20 k scattered voxels 22.8 / 25.2 us,
-  // 60 k LiDAR ones 35.8 / 37.7, indoor 100 k 41.6 / 39.3; 32 x 64 over 10 k LiDAR voxels 20.8 / 22.3, 60 k 59.5 / 58.4,
-  // indoor 30 k 35.4 / 33.1, 100 k 79.8 / 68.3; 96 x 64 over 164 k pairs 47 / 40.)
-  const bool few = !shares_grid && bi * bj <= 2 && (double)a.n_pairs * g->ty * (bi * bj * bi * bj) < 8e5;
+  // (Three parts split every value once per 32 x 32 products at one block, as much work as they save: fp32 MFMAs there.  Two blocks in a
+  // launch of their own: where each cell walks many pairs, a walk of few being mostly the wait for its first rows.  fp32
+  // MFMAs / three parts: 32 x 32 over 60 k LiDAR voxels 35 / 35 us, 120 k 53 / 57, 96 x 96 over 60 k 141 / 162; 32 x 64 over 20 k indoor
+  // voxels 26 / 28, 60 k 61 / 66, 150 k 117 / 106.)
+  const bool few = bi * bj == 1 || (!shares_grid && bi * bj == 2 && (double)a.n_pairs * g->ty < 9e5);
   g->split = f16 || !split_bf16_enabled() ? 0 : a.reduced ? 2 : few ? 0 : 3;
   const size_t lds = (g->split ? 4 * (size_t)sp * g->split * ((bi * 32 + 16) + (bj * 32 + 16)) * 2
                                : 4 * (size_t)sp * ((bi * 32 + pad) + (bj * 32 + pad)) * (f16 ? 2 : 4))
