@@ -469,23 +469,27 @@ int check_common(const void *a, const void *b, const void *c, const int32_t *kpo
 //   fp16: 2.25 .. 2.5 at every channel count (2.2 + 16 / c);
 //   fp32 MFMAs: 2.35 / 1.76 / 1.3 at 32 / 64 / 128 channels, about 1 + 45 / c.
 // The kernel without atomics, whose results do not depend on the run, gets 5 % on top.
-// fp32 tensors in bf16 parts, beyond that line: products cost so little that the output-stationary kernel's chain of stages (small maps)
-// or rounds of tiles (large ones) counts, and not the empty slots; estimated for either side, fitted to thinned clouds of
-// 10 k .. 60 k voxels.  Pair view / output-stationary, fp32 and tf32 mode, over thinned clouds: 64 -> 64 forward 20 k voxels of
-// 60 k 32.4 / 48.6 and 31.1 / 32.9 us, 60 k of 100 k 113.9 / 71.1 and 103.7 / 45.1, 60 k of 200 k 72.2 / 67.6 and
-// 66.1 / 43.3; 128 -> 128 60 k of 150 k 168 / 202 and 149 / 119.  Both gradients, in one grid where the output-stationary
-// kernel takes the input's (beside_us): 64 -> 64 20 k of 60 k 85.7 / 61.6 and 74.9 / 52.2, 256 -> 256 295 / 419 and 278 / 326.
-double stages_us(const GmsArgs &a) {
-  const int c_src = a.transpose_w ? a.c_out : a.c_in, c_dst = a.transpose_w ? a.c_in : a.c_out, slabs = (c_src + 31) / 32;
-  const double tiles_per_cu = (double)((a.n_dst + 127) / 128 * ((c_dst + 31) / 32)) / num_cus();
-  const double stage = a.transpose_w ? (a.reduced ? 0.36 + 0.02 * slabs : 0.45 + 0.0035 * slabs * slabs) : (a.reduced ? 0.33 : 0.55);
-  return 8.5 + stage * a.k_vol * slabs * (tiles_per_cu <= 1 ? 1 : 1.25 + 0.25 * tiles_per_cu);
+// fp32 tensors in bf16 parts, beyond that line: products cost so little that the output-stationary kernel's chain of stages counts (a
+// stage: an offset and a slab of 32 channels; a tile waits for one after the other), and what the (64-row block, offset)
+// combinations of all its tiles come to, against the pair view's atomics and gathers.  Fitted to either kernel over 17 channel counts from
+// 32 x 32 to 256 x 256 on indoor, LiDAR and scattered clouds of 500 .. 150 k voxels, sorted and in scan order (half of the
+// estimates are within 9 %, nine in ten within 25 .. 30 %; the choice costs 0.4 .. 1.7 % over the better of the two in the mean).
+// Pair view / output-stationary, fp32: 64 -> 64 forward over 20 k scattered voxels 32 / 55 us, LiDAR 60 k 97 / 74; 96 -> 96 over that
+// 140 / 207; 128 -> 128 input gradient over 50 k scattered 117 / 239; with its weight gradient, which the output-stationary
+// kernel's grid hides, 64 -> 64 over 50 k 130 / 101, 128 -> 128 225 / 253.
+double rows_us(const GmsArgs &a, const Plan *plan) {
+  const int c_src = a.transpose_w ? a.c_out : a.c_in, c_dst = a.transpose_w ? a.c_in : a.c_out, slabs = (c_src + 31) / 32, cols = (c_dst + 31) / 32;
+  const double blocks = (double)(a.transpose_w ? plan->stages_in : plan->stages_out) * cols / num_cus();
+  const double chain = a.k_vol * (a.transpose_w && cols % 2 == 0 ? 1.23 : 1.0);      // (64 columns a tile; small forward launches: 32)
+  return 9.5 + slabs * (a.reduced ? 0.30 * chain + 0.155 * blocks : 0.41 * chain + 0.293 * blocks);
 }
 double pair_view_us(const GmsArgs &a, double pairs) {
   const int c_src = a.transpose_w ? a.c_out : a.c_in, c_dst = a.transpose_w ? a.c_in : a.c_out;
-  return 9 + 6e-4 * c_src * c_dst + (a.reduced ? 0.8e-6 : 1e-6) * pairs * c_dst * (3.6 + 0.0042 * c_src);
+  return a.reduced ? 14.1 + 3.4e-4 * c_src * c_dst + 1e-6 * pairs * c_dst * (2.8 + 0.0046 * c_src)
+                   : 14.6 + 6.1e-4 * c_src * c_dst + 1e-6 * pairs * c_dst * (2.7 + 0.0104 * c_src);
 }
-bool sparse_rows(const GmsArgs &a, const Plan *plan) {
+// `masked`: the channels' rest would be masked (else counts that are no multiple of 32 stay on fp32 MFMAs, which the first rule is for).
+bool sparse_rows(const GmsArgs &a, const Plan *plan, bool masked = false) {
   const int stages = a.transpose_w ? plan->stages_in : plan->stages_out;
   if (stages <= 0 || plan->pairs_counted <= 0) return false;   // (the plan's own pair count: a.n_pairs is a bound)
   const double slots_per_pair = (double)stages * 64.0 / (double)plan->pairs_counted;
@@ -494,8 +498,8 @@ bool sparse_rows(const GmsArgs &a, const Plan *plan) {
   // (no break-even point was measured below 1.3: denser maps stay output-stationary)
   const double need = 1.05 * even;
   if (slots_per_pair <= (need > 1.4 ? need : 1.4)) return false;
-  return a.dtype == FGMS_F16 || !split_bf16_enabled() ||
-         stages_us(a) > 1.08 * (pair_view_us(a, (double)plan->pairs_counted) + a.beside_us);
+  return a.dtype == FGMS_F16 || !split_bf16_enabled() || ((int)c_src % 32 != 0 && !masked) ||
+         rows_us(a, plan) > pair_view_us(a, (double)plan->pairs_counted) + a.beside_us;
 }
 
 enum class Route { kNarrow, kSkinny, kRows, kPairView, kWide, kPairs, kGeneric };
@@ -600,33 +604,21 @@ double padded_us(const GmsArgs &p, const Plan *plan) {
   switch (first_route(p, plan)) {
     case Route::kNarrow:
     case Route::kSkinny: return 17 * group_count(p, plan) + (p.transpose_w ? 1.5 : c_src * c_dst / 45.0);
-    case Route::kRows: {
-      const bool split = p.reduced && split_bf16_enabled();
-      const double tiles_per_cu = (double)((p.n_dst + 127) / 128 * (c_dst / 32)) / num_cus(), stages = p.k_vol * slabs;
-      if (p.transpose_w) return 15 + 3 * wide + (split ? 0.42 : 0.5) * stages * (1 + 1.45 * std::max(0.0, tiles_per_cu - 0.43));
-      return 14 + (split ? 0.41 : 0.65) * stages * (tiles_per_cu <= 1 ? 1 : 1.25 + 0.25 * tiles_per_cu);
-    }
+    case Route::kRows: return 6 + rows_us(p, plan);      // (copies in front, crop behind)
     default:
       return 20 + 1.5 * slabs * (1 + wide) + 1e-6 * pairs_of(p, plan) * (p.dense_k >= 0 ? 2.0 * c_dst : 3.4 * c_dst + 0.4 * c_src);
   }
 }
-// The same over the masked tiles (fp32: no copies, nothing to crop).  Forward over 4 k dense voxels, measured (estimated):
-// 24 -> 32 21.0 us (20.4), tf32 mode 18.1 (17.4); 48 -> 48 33.2 (32.3) and 27.2 (26.3); 96 -> 24 44.1 (44.1) and 35.8 (35.2);
-// 48 -> 48 over 30 k 49.5 (49).  On the vector ALUs 48 -> 48 over 4 k 21 us, 96 -> 24 27.  Both gradients, the weights'
-// hidden behind the tiles: 24 -> 32 19.5 us (19.3), 48 -> 48 39 (39.8), 48 -> 96 56 (55); tf32 mode 18.7, 35.2, 46.5 (18.7, 36.2, 49.8).
-double masked_us(const GmsArgs &a) {
-  const int c_src = a.transpose_w ? a.c_out : a.c_in, c_dst = a.transpose_w ? a.c_in : a.c_out;
-  const double stages = (double)a.k_vol * ((c_src + 31) / 32), tiles_per_cu = (double)((a.n_dst + 127) / 128 * ((c_dst + 31) / 32)) / num_cus();
-  if (a.transpose_w) {
-    const bool pairs_of_tiles = (c_dst + 31) / 32 % 2 == 0;     // (two column tiles to a workgroup)
-    const double stage = (a.reduced ? 0.36 : 0.38) * (!pairs_of_tiles ? 1 : a.reduced ? 1.4 : 1.5), per_cu = tiles_per_cu / (pairs_of_tiles ? 2 : 1);
-    return 9 + stage * stages * (1 + 1.45 * std::max(0.0, per_cu - 0.43));
-  }
-  return 8.5 + (a.reduced ? 0.33 : 0.44) * stages * (tiles_per_cu <= 1 ? 1 : 1.25 + 0.25 * tiles_per_cu);
+// The same over the masked tiles (fp32: no copies, nothing to crop), with the weight gradient beside the input's if there is one.
+// Forward, measured (estimated), fp32 and tf32 mode: 24 -> 32 over 4 k dense voxels 24.1 us (21.7) and 18.6 (18.2), 48 -> 48 over 30 k
+// 56 (58) and 34 (39), LiDAR 60 k 77 (76) and 42 (49).  On the vector ALUs 24 -> 32 over 4 k 15, 48 -> 48 over 30 k 93.  Both gradients:
+// 24 -> 32 over 4 k 22.6 (22.4) and 19.6 (18.9), 48 -> 48 45 (44) and 34 (35), over 60 k 127 (129) and 86 (98).
+double masked_us(const GmsArgs &a, const Plan *plan) {
+  return rows_us(a, plan) + (a.transpose_w ? 16e-6 * pairs_of(a, plan) * (up_to_32(a.c_in) / 32) * (up_to_32(a.c_out) / 32) : 0);
 }
 bool takes_ragged(const GmsArgs &a, const Plan *plan);
 bool padding_pays(const GmsArgs &a, const Plan *plan, int c_in, int c_out) {
-  if (a.dtype != FGMS_F16 && takes_ragged(a, plan) && ragged_gms_supported(a, plan)) return masked_us(a) < vector_alu_us(a, plan);
+  if (a.dtype != FGMS_F16 && takes_ragged(a, plan) && ragged_gms_supported(a, plan)) return masked_us(a, plan) < vector_alu_us(a, plan);
   // (fp16 adds on the vector ALUs cost ten times as much: 32 -> 20 over 500 voxels 17 us over copies, 24 without.
   // The copies' fp32 kernels mostly do without atomics: a near tie goes to them.)
   return a.dtype == FGMS_F16 || padded_us(with_channels(a, c_in, c_out), plan) < 1.05 * vector_alu_us(a, plan);
@@ -650,12 +642,12 @@ bool padded_gms_channels(const GmsArgs &a, const Plan *plan, int *c_in, int *c_o
 // Layers whose channels fill no whole tile go straight to kernels that mask the rest, where the map
 // is dense enough for the output-stationary kernel (else the pair-stationary kernels over padded copies).
 bool takes_ragged(const GmsArgs &a, const Plan *plan) {
-  return g_policy == 0 && plan && a.n_pairs > 0 && a.dense_k < 0 && !narrow_gms_supported(a, plan) && !small_gms_supported(a, plan) && !sparse_rows(a, plan);
+  return g_policy == 0 && plan && a.n_pairs > 0 && a.dense_k < 0 && !narrow_gms_supported(a, plan) && !small_gms_supported(a, plan) && !sparse_rows(a, plan, true);
 }
 
 // fp32 counts that are no multiple of 32: over the masked tiles where another matrix kernel takes them as they are or the
-// vector ALUs are slower.  (Not for 16 channels forward in fp32: half of every slab of 32 is empty, and six products
-// each make it 61 us for 16 -> 64 over 120 k voxels where slabs of 16 on fp32 MFMAs took 47; in tf32 mode 36.)
+// vector ALUs are slower.  (Not for 16 channels forward in fp32: half of every slab of 32 is empty, and eight products (then six)
+// each make it more than 61 us for 16 -> 64 over 120 k voxels where slabs of 16 on fp32 MFMAs took 47; in tf32 mode 36.)
 bool ragged_pays(const GmsArgs &a, const Plan *plan) {
   int pi, po;
   if (a.dtype == FGMS_F16) return true;
@@ -900,16 +892,16 @@ bool together_pays(const GmsArgs &d, const Plan *p, const WgradArgs &w, const Gm
 }
 
 // fp32: both gradients over the masked tiles, or each on its better side?  The weights' hide behind the tiles; on their own they
-// take three launches and what the copies' kernel adds (48 x 48: 15 us over 9 k pairs, 23 over 39 k).  Masked / apart:
-// 48 -> 48 over 2 k voxels 41 / 32 us, 3 k 41 / 37, 4 k 39 / 44; 48 -> 96 over 4 k 56 / 50; 24 -> 32 over 1 k 19.5 / 28.  Maps too thin
-// for the output-stationary kernel at the copies' channel counts stay with the copies (64 -> 48 over 1 k 40 / 32).
+// take three launches and what the copies' kernel adds (48 x 48: 15 us over 9 k pairs, 23 over 39 k, 74 over 69 k of 20 k scattered
+// voxels, whose cells wait for more rows).  Masked / apart: 48 -> 48 over 4 k voxels 45 / 44 us, 20 k scattered ones 72 / 104; 24 -> 32
+// over 1 k 22 / 28.  Maps too thin for the output-stationary kernel at the copies' channel counts stay with the copies.
 bool masked_bwd_pays(const GmsArgs &d, const Plan *p, const WgradArgs &w) {
   if (d.dtype == FGMS_F16 || (tuned_gms(d, p) && mfma_wgrad_supported(w))) return true;
   const GmsArgs pd = with_channels(d, up_to_32(d.c_in), up_to_32(d.c_out));
   if (sparse_rows(pd, p)) return false;
   const double in_alone = tuned_gms(d, p) ? padded_us(d, p) : std::min(padded_us(pd, p), vector_alu_us(d, p));
-  const double cells = (double)(pd.c_in / 32) * (pd.c_out / 32), w_alone = 12.3 + 1e-3 * (double)w.n_pairs * (0.045 + 0.05 * std::min(cells, 4.0));
-  return masked_us(d) < 0.88 * (in_alone + w_alone);     // (vector_alu_us is a sixth high on maps this small)
+  const double cells = (double)(pd.c_in / 32) * (pd.c_out / 32), w_alone = 12.3 + 6e-4 * (double)w.n_out + 1e-3 * (double)w.n_pairs * (0.045 + 0.05 * std::min(cells, 4.0));
+  return masked_us(d, p) < 0.95 * (in_alone + w_alone);
 }
 
 // Widened channels for a backward pass one of whose gradients no tuned kernel takes as it is: the
@@ -1041,10 +1033,11 @@ int backward(const void *out_feats_grad, const void *in_feats, const void *kerne
   w.overwrite = overwrite;
   if (!want_kernel) return want_in ? run_gms(d, p) : FGMS_OK;
   if (!want_in) return run_wgrad(w);
-  // (a weight gradient of its own: 64 x 64 over 20 k thinned voxels 53 us, 128 x 128 60 .. 68, 256 x 256 120 .. 170; three
-  // quarters of it vanish in the other's grid)
+  // (a weight gradient of its own: 64 x 64 over 20 k scattered voxels 60 us, 128 x 128 66; half of it vanishes in the other's
+  // grid.  Next to masked tiles more: on its own it needs padded copies.  48 x 48 over 20 k: masked tiles 60 us, copies and pair view 104.)
   if (dtype != FGMS_F16)
-    d.beside_us = 0.74 * (d.reduced ? 0.75 : 1) * (25 + 1e-3 * (double)n_out + 18e-6 * pairs_of(d, p) * up_to_32(c_in) / 32 * (up_to_32(c_out) / 32));
+    d.beside_us = (c_in % 32 || c_out % 32 ? 0.8 : 0.5) * (d.reduced ? 0.75 : 1) *
+                  (25 + 1e-3 * (double)n_out + 18e-6 * pairs_of(d, p) * (up_to_32(c_in) / 32) * (up_to_32(c_out) / 32));
   int pi, po;
   if (takes_ragged(d, p) && masked_bwd_pays(d, p, w)) {
     bool done = false;
