@@ -473,15 +473,16 @@ int check_common(const void *a, const void *b, const void *c, const int32_t *kpo
 // stage: an offset and a slab of 32 channels; a tile waits for one after the other), and what the (64-row block, offset)
 // combinations of all its tiles come to, against the pair view's atomics and gathers.  Fitted to either kernel over 17 channel counts from
 // 32 x 32 to 256 x 256 on indoor, LiDAR and scattered clouds of 500 .. 150 k voxels, sorted and in scan order (half of the
-// estimates are within 9 %, nine in ten within 25 .. 30 %; the choice costs 0.4 .. 1.7 % over the better of the two in the mean).
+// estimates are within 9 %, nine in ten within 21 .. 32 %; the choice costs 0.3 .. 1.4 % over the better of the two in the mean).
 // Pair view / output-stationary, fp32: 64 -> 64 forward over 20 k scattered voxels 32 / 55 us, LiDAR 60 k 97 / 74; 96 -> 96 over that
 // 140 / 207; 128 -> 128 input gradient over 50 k scattered 117 / 239; with its weight gradient, which the output-stationary
 // kernel's grid hides, 64 -> 64 over 50 k 130 / 101, 128 -> 128 225 / 253.
 double rows_us(const GmsArgs &a, const Plan *plan) {
   const int c_src = a.transpose_w ? a.c_out : a.c_in, c_dst = a.transpose_w ? a.c_in : a.c_out, slabs = (c_src + 31) / 32, cols = (c_dst + 31) / 32;
-  const double blocks = (double)(a.transpose_w ? plan->stages_in : plan->stages_out) * cols / num_cus();
-  const double chain = a.k_vol * (a.transpose_w && cols % 2 == 0 ? 1.23 : 1.0);      // (64 columns a tile; small forward launches: 32)
-  return 9.5 + slabs * (a.reduced ? 0.30 * chain + 0.155 * blocks : 0.41 * chain + 0.293 * blocks);
+  const double blocks = (double)(a.transpose_w ? plan->stages_in : plan->stages_out) * cols / num_cus() *
+                        (cols % 2 == 0 || cols == 1 ? 1 : a.reduced ? 1.66 : 1.36);      // (32 columns a tile: rows gathered once for each)
+  const double chain = a.k_vol * (a.transpose_w && cols % 2 == 0 ? 1.3 : 1.0);           // (64; small forward launches take 32)
+  return a.reduced ? 9.6 + slabs * (0.293 * chain + 0.139 * blocks) : 9.8 + slabs * (0.41 * chain + 0.271 * blocks);
 }
 double pair_view_us(const GmsArgs &a, double pairs) {
   const int c_src = a.transpose_w ? a.c_out : a.c_in, c_dst = a.transpose_w ? a.c_in : a.c_out;
