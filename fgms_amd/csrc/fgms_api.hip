@@ -478,7 +478,8 @@ int check_common(const void *a, const void *b, const void *c, const int32_t *kpo
 // 140 / 207; 128 -> 128 input gradient over 50 k scattered 117 / 239; with its weight gradient, which the output-stationary
 // kernel's grid hides, 64 -> 64 over 50 k 130 / 101, 128 -> 128 225 / 253.
 double rows_us(const GmsArgs &a, const Plan *plan) {
-  const int c_src = a.transpose_w ? a.c_out : a.c_in, c_dst = a.transpose_w ? a.c_in : a.c_out, slabs = (c_src + 31) / 32, cols = (c_dst + 31) / 32;
+  const int c_src = a.transpose_w ? a.c_out : a.c_in, c_dst = a.transpose_w ? a.c_in : a.c_out;
+  const int slabs = (c_src + 31) / 32, cols = (c_dst + 31) / 32;
   const double blocks = (double)(a.transpose_w ? plan->stages_in : plan->stages_out) * cols / num_cus() *
                         (cols % 2 == 0 || cols == 1 ? 1 : a.reduced ? 1.66 : 1.36);      // (32 columns a tile: rows gathered once for each)
   const double chain = a.k_vol * (a.transpose_w && cols % 2 == 0 ? 1.3 : 1.0);           // (64; small forward launches take 32)
@@ -643,7 +644,8 @@ bool padded_gms_channels(const GmsArgs &a, const Plan *plan, int *c_in, int *c_o
 // Layers whose channels fill no whole tile go straight to kernels that mask the rest, where the map
 // is dense enough for the output-stationary kernel (else the pair-stationary kernels over padded copies).
 bool takes_ragged(const GmsArgs &a, const Plan *plan) {
-  return g_policy == 0 && plan && a.n_pairs > 0 && a.dense_k < 0 && !narrow_gms_supported(a, plan) && !small_gms_supported(a, plan) && !sparse_rows(a, plan, true);
+  return g_policy == 0 && plan && a.n_pairs > 0 && a.dense_k < 0 && !narrow_gms_supported(a, plan) &&
+         !small_gms_supported(a, plan) && !sparse_rows(a, plan, true);
 }
 
 // fp32 counts that are no multiple of 32: over the masked tiles where another matrix kernel takes them as they are or the
@@ -758,7 +760,8 @@ int run_gms_padded(const GmsArgs &a, const Plan *plan, int c_in, int c_out, bool
                dst_bytes = (size_t)a.n_dst * p_dst * esz;
   const int src_slot = a.transpose_w ? kSlotPadOut : kSlotPadIn;
   // (rows that fill whole tiles as they are need no copy, nor do results)
-  const bool copy_src = p_src != c_src || reinterpret_cast<uintptr_t>(a.src) % 16, crop = p_dst != c_dst || reinterpret_cast<uintptr_t>(a.dst) % 16;
+  const bool copy_src = p_src != c_src || reinterpret_cast<uintptr_t>(a.src) % 16;
+  const bool crop = p_dst != c_dst || reinterpret_cast<uintptr_t>(a.dst) % 16;
   *done = workspaces_fit(a.stream, {{src_slot, copy_src ? src_bytes : 0}, {kSlotPadWeights, w_bytes}, {kSlotPadResult, crop ? dst_bytes : 0}});
   if (!*done) return FGMS_OK;
   GmsArgs p = a;
@@ -806,7 +809,8 @@ bool padded_wgrad_channels(const WgradArgs &a, int *c_in, int *c_out) {
 // they are added to the caller's tensor.
 int run_wgrad_padded(const WgradArgs &a, int c_in, int c_out, bool *done) {
   const size_t esz = elem_size(a.dtype);
-  const bool copy_in = c_in != a.c_in || reinterpret_cast<uintptr_t>(a.in) % 16, copy_gout = c_out != a.c_out || reinterpret_cast<uintptr_t>(a.gout) % 16;
+  const bool copy_in = c_in != a.c_in || reinterpret_cast<uintptr_t>(a.in) % 16;
+  const bool copy_gout = c_out != a.c_out || reinterpret_cast<uintptr_t>(a.gout) % 16;
   const size_t in_bytes = copy_in ? (size_t)a.n_in * c_in * esz : 0, gout_bytes = copy_gout ? (size_t)a.n_out * c_out * esz : 0;
   *done = workspaces_fit(a.stream, {{kSlotPadIn, in_bytes}, {kSlotPadOut, gout_bytes}, {1, (size_t)a.k_vol * c_in * c_out * sizeof(float)}});
   if (!*done) return FGMS_OK;
@@ -901,7 +905,8 @@ bool masked_bwd_pays(const GmsArgs &d, const Plan *p, const WgradArgs &w) {
   const GmsArgs pd = with_channels(d, up_to_32(d.c_in), up_to_32(d.c_out));
   if (sparse_rows(pd, p)) return false;
   const double in_alone = tuned_gms(d, p) ? padded_us(d, p) : std::min(padded_us(pd, p), vector_alu_us(d, p));
-  const double cells = (double)(pd.c_in / 32) * (pd.c_out / 32), w_alone = 12.3 + 6e-4 * (double)w.n_out + 1e-3 * (double)w.n_pairs * (0.045 + 0.05 * std::min(cells, 4.0));
+  const double cells = (double)(pd.c_in / 32) * (pd.c_out / 32);
+  const double w_alone = 12.3 + 6e-4 * (double)w.n_out + 1e-3 * (double)w.n_pairs * (0.045 + 0.05 * std::min(cells, 4.0));
   return masked_us(d, p) < 0.95 * (in_alone + w_alone);
 }
 

@@ -297,7 +297,7 @@ int launch_side_job(const SideJob &job, hipStream_t stream);
 // 32-wide tiles, 53.9 with 96; 96 -> 96 over 40 k scattered ones, 3.3 pairs a row, forward and backward 100 us
 // against 108; the submanifold maps that gain by it have 10.)
 inline bool worth_96_columns(int64_t n_pairs, int64_t n_a, int64_t n_b) { return n_pairs >= 5 * (n_a > n_b ? n_a : n_b); }
-bool split_bf16_enabled();   // products of fp32 tensors in split bf16 where the caller allows tf32 precision
+bool split_bf16_enabled();   // products of fp32 tensors in bf16 parts: three a value, two where the caller allows tf32 precision
 bool small_gms_supported(const GmsArgs &a, const Plan *p);
 int launch_small_gms(const GmsArgs &a, const Plan *p);
 // Narrow input sides on the matrix cores (fgms_narrow.hip): the forward pass, and the weight gradient.

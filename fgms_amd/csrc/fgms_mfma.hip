@@ -243,8 +243,8 @@ __device__ __forceinline__ void mma_slab_rawt(float16v (&acc)[MT][NT], const int
 // 64 -> 64 forward over 40 k voxels 88 / 76 us, 200 k 227 / 165; backward 116 / 91, 398 / 319; 128 -> 128 over 40 k 249 / 161
 // and 349 / 271; 32 -> 32 over 20 k 25.4 / 23.2 and 25.6 / 24.0.
 // What the parts cannot hold goes to fp32 MFMAs (RAW = 7 and 8): sums that an infinite value reaches come out as NaN or infinite
-// whatever else is in them, and a value too small for them (below 2^-102 at most) is noted when it is split, so that a workgroup that has met either does its
-// work again before it writes its tile, in that tile at the price of both.
+// whatever else is in them, and a value too small for them (below 2^-102 at most) is noted when it is split, so that a
+// workgroup that has met either does its work again before it writes its tile, in that tile at the price of both.
 //
 // Slot (16 bytes = 8 bf16) of a split tile of P parts: row-major, a row holds its 32 values of the slab
 // as 4 chunks of each part; the XOR spreads the rows one b128 read pass (16 lanes) touches over all banks: rows of
@@ -279,8 +279,8 @@ __device__ __forceinline__ void gather_commit_parts(int4v *__restrict__ a_lds, i
 // acc[mt][nt] += A(slab) x W(slab), both split.  Weights in LDS as [k-step][nt][part][lane], or (AS_ROWS: the input
 // gradient) as a split tile of the NT*32 rows of W[k], the slab's 32 columns.
 template <int P, bool AS_ROWS, int NT, int MT>
-__device__ __forceinline__ void mma_slab_parts(float16v (&acc)[MT][NT], float16v (&low)[P == 3 ? MT : 1][P == 3 ? NT : 1], const int4v *__restrict__ a_lds,
-                                               const int4v *__restrict__ w_lds, int lane) {
+__device__ __forceinline__ void mma_slab_parts(float16v (&acc)[MT][NT], float16v (&low)[P == 3 ? MT : 1][P == 3 ? NT : 1],
+                                               const int4v *__restrict__ a_lds, const int4v *__restrict__ w_lds, int lane) {
   const int h = lane / 32, r = lane % 32;
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
@@ -289,7 +289,8 @@ __device__ __forceinline__ void mma_slab_parts(float16v (&acc)[MT][NT], float16v
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
       for (int q = 0; q < P; ++q)
-        b[nt][q] = __builtin_bit_cast(bf16x8, w_lds[AS_ROWS ? part_slot<P>(nt * 32 + r, q, s * 2 + h) : ((s * NT + nt) * P + q) * 64 + lane]);
+        b[nt][q] = __builtin_bit_cast(bf16x8, w_lds[AS_ROWS ? part_slot<P>(nt * 32 + r, q, s * 2 + h)
+                                                            : ((s * NT + nt) * P + q) * 64 + lane]);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       bf16x8 a[P];
@@ -306,7 +307,8 @@ __device__ __forceinline__ void mma_slab_parts(float16v (&acc)[MT][NT], float16v
 // holds the 8 values op(W[k])[slab*32 + s*16 + (lane/32)*8 + 0..7][nt*32 + lane%32] of that part.
 // One thread per P chunks.
 // (Channels that fill no whole tile: zeros behind them.)
-// A chunk with a weight that three parts do not hold is marked with a NaN, which takes every tile that meets it to fp32 MFMAs and the weights as they are.
+// A chunk with a weight that three parts do not hold is marked with a NaN, which takes every tile that meets it to fp32 MFMAs
+// and the weights as they are.
 template <int P>
 __global__ void pack_weights_parts_kernel(const float *__restrict__ w, int4v *__restrict__ packed,
                                           int k_vol, int c_in, int c_out, bool transpose) {
@@ -1042,7 +1044,6 @@ struct Shape {
   int c_src, c_dst, S, NT, E;
   int NTR, SR;            // 32-column tiles per wave and k-steps per slab in the output-stationary kernel
   size_t lds_bytes;       // pair-stationary kernel
-  size_t lds_rows_bytes;  // output-stationary kernel
   bool ok;
 };
 
@@ -1073,12 +1074,11 @@ Shape shape_of(const GmsArgs &a) {
   // time, so that more waves are worth more than fewer gathers (96 -> 96 over 40 k: 127.5 us against 184.8
   // with 96); in tf32 mode the forward pass takes 96 once there are tiles enough (over 150 k 243.9 ->
   // 166.2 us, over 40 k the same).
-  const bool cols96 = s.c_dst % 96 == 0 && worth_96_columns(a.n_pairs, a.n_src, a.n_dst) && (a.dtype == FGMS_F16 || (a.reduced && !a.transpose_w && s.S == 4 && split_bf16_enabled() &&
-                      (a.n_dst + kTileRows - 1) / kTileRows * (s.c_dst / 96) * 2 >= 3 * (int64_t)num_cus()));
+  const bool tf32_fills_96 = a.reduced && !a.transpose_w && s.S == 4 && split_bf16_enabled() &&
+                             (a.n_dst + kTileRows - 1) / kTileRows * (s.c_dst / 96) * 2 >= 3 * (int64_t)num_cus();
+  const bool cols96 = s.c_dst % 96 == 0 && worth_96_columns(a.n_pairs, a.n_src, a.n_dst) && (a.dtype == FGMS_F16 || tf32_fills_96);
   s.NTR = (s.c_dst % 128 == 0 && wide) ? 4 : s.c_dst % 64 == 0 ? 2 : cols96 ? 3 : 1;
   s.SR = s.S < 4 && s.c_src % (6 * s.E) == 0 ? 3 : s.S;
-  s.lds_rows_bytes = 2 * (size_t)s.SR * s.NTR * 64 * 16          // two stages of weights
-                     + (size_t)kWaves * kWaveRows * 2 * s.SR * 16 + (size_t)kWaves * 3 * kWaveRows * sizeof(int);
   s.ok = s.lds_bytes <= 128 * 1024;
   return s;
 }
@@ -1132,8 +1132,6 @@ Shape ragged_shape(const GmsArgs &a) {
     return s;
   s.NTR = f16 ? ragged_tiles(s.c_dst, worth_96_columns(a.n_pairs, a.n_src, a.n_dst)) : (s.c_dst + 31) / 32 % 2 ? 1 : 2;
   s.SR = f16 ? ragged_steps(s.c_src) : 4;
-  s.lds_rows_bytes = 2 * (size_t)s.SR * s.NTR * 64 * 16 + (size_t)kWaves * kWaveRows * 2 * s.SR * 16 +
-                     (size_t)kWaves * 3 * kWaveRows * sizeof(int);
   s.ok = s.NTR > 0;
   return s;
 }
@@ -1336,8 +1334,9 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
   // (Three parts take 6 bytes a weight, at 32-bit offsets: a stream under capture whose workspace holds only the 4 of the other
   // layouts stays on fp32 MFMAs.  Masked channel counts come here with room for them.)
   const size_t bytes = (size_t)a.k_vol * a.c_in * a.c_out * 6;
+  auto room = [&]() { return bytes <= 0xfffffff0u && (!is_capturing(a.stream) || workspace_bytes(a.stream, 0) >= bytes); };
   const bool split = kCanSplit && !a.transpose_w && !a.prepacked && split_bf16_enabled() &&
-                     (a.reduced || RAGGED || (three_parts && bytes <= 0xfffffff0u && (!is_capturing(a.stream) || workspace_bytes(a.stream, 0) >= bytes)));
+                     (a.reduced || RAGGED || (three_parts && room()));
   if (kCanSplit && raw == 2 && split_bf16_enabled()) raw = a.reduced ? 4 : three_parts ? 6 : 2;   // (the input gradient splits as it reads)
   const T *packed = raw ? (const T *)a.w : (const T *)a.prepacked;
   if (split) {
@@ -1362,7 +1361,8 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
   const unsigned gx = rg.gx;
   if (gx == 0) return a.side.kind ? launch_side_job(a.side, a.stream) : FGMS_OK;
   constexpr bool kCanRaw = NT != 4;
-  constexpr int kRaw6 = kCanSplit && NT != 3 ? 6 : 0, kRaw5 = kCanSplit && NT != 3 ? 5 : 0, kRaw4 = kCanSplit ? 4 : 0, kRaw3 = kCanSplit ? 3 : 0, kRaw2 = kCanRaw ? 2 : 0, kRaw1 = kCanRaw && sizeof(T) == 2 ? 1 : 0;
+  constexpr int kRaw6 = kCanSplit && NT != 3 ? 6 : 0, kRaw5 = kCanSplit && NT != 3 ? 5 : 0;
+  constexpr int kRaw4 = kCanSplit ? 4 : 0, kRaw3 = kCanSplit ? 3 : 0, kRaw2 = kCanRaw ? 2 : 0, kRaw1 = kCanRaw && sizeof(T) == 2 ? 1 : 0;
   constexpr int kRagRaw = !RAGGED ? 0 : sizeof(T) == 2 ? kRaw1 : kRaw3, kRagRaw5 = !RAGGED ? 0 : sizeof(T) == 2 ? kRaw1 : kRaw5;
   // (raw is one of those the type and the tile allow)
 #define FGMS_BY_RAW(MTv, KGv)                                                                                       \
@@ -1390,7 +1390,9 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
   const int part_stages = rg.gz > 1 ? rg.part_stages : 0;
   const unsigned gz = rg.gz;
   {
-    ProfileScope prof(pair_view ? (a.transpose_w ? "gms_rows_kernel(dgrad, pair view)" : "gms_rows_kernel(fwd, pair view)") : raw == 4 ? "gms_rows_kernel(dgrad, bf16x3)"
+    ProfileScope prof(pair_view  ? (a.transpose_w ? "gms_rows_kernel(dgrad, pair view)" : "gms_rows_kernel(fwd, pair view)")
+                      : RAGGED   ? (raw == 3 ? "gms_rows_kernel(fwd, masked, bf16x3)" : "gms_rows_kernel(fwd, masked)")
+                      : raw == 4 ? "gms_rows_kernel(dgrad, bf16x3)"
                       : raw == 3 ? "gms_rows_kernel(fwd, bf16x3)"
                       : a.transpose_w ? "gms_rows_kernel(dgrad)" : "gms_rows_kernel(fwd)",
                       a.stream);
@@ -1419,7 +1421,8 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
 // (2 waves per SIMD where the weight gradient's tile is 128 x 128: its 64 accumulators per lane and
 // the rows in flight spill at 3.  128 -> 128 over 40k voxels, forward and backward: tf32 mode 477 -> 327 us.)
 template <typename T, int NT, int S, int BI, int BJ, int RAWD, int MT = 2, bool RAGGED = false>
-__global__ __launch_bounds__(kThreads, NT >= 3 || RAWD == 6 || BI * BJ == 16 || ((BI == 3 || BJ == 3) && BI * BJ >= 6) ? 2 : 3) void bwd_fused_kernel(
+__global__ __launch_bounds__(kThreads, NT >= 3 || RAWD == 6 || BI * BJ == 16 || ((BI == 3 || BJ == 3) && BI * BJ >= 6) ? 2 : 3)
+void bwd_fused_kernel(
     const T *__restrict__ gout, const T *__restrict__ w, T *__restrict__ gin,
     const int32_t *__restrict__ nbr, const unsigned long long *__restrict__ block_masks,
     const int32_t *__restrict__ perm, const int32_t *__restrict__ tile_order, int n_in, int k_vol,
@@ -1442,8 +1445,8 @@ __global__ __launch_bounds__(kThreads, NT >= 3 || RAWD == 6 || BI * BJ == 16 || 
   } else {
     const int j = blockIdx.x - rows_total;
     if constexpr (BI <= 3 && BJ <= 3)
-      wgrad_wave_body<T, BI, BJ, RAWD == 6 && BI * BJ == 1 ? 0 : split_parts_of(RAWD), RAGGED>(in, gout, gw32, kpos, imap, omap, k_vol, c_in, c_out, smap,
-                                            j % wgrad_x, j / wgrad_x, in_bytes, gout_bytes);
+      wgrad_wave_body<T, BI, BJ, RAWD == 6 && BI * BJ == 1 ? 0 : split_parts_of(RAWD), RAGGED>(      // (see wave_geometry)
+          in, gout, gw32, kpos, imap, omap, k_vol, c_in, c_out, smap, j % wgrad_x, j / wgrad_x, in_bytes, gout_bytes);
     else
       wgrad_wg_body<T, BI, BJ, RAWD == 4>(in, gout, gw32, kpos, imap, omap, k_vol, c_in, c_out, smap,
                                           j % wgrad_x, j / wgrad_x);
@@ -1494,7 +1497,10 @@ int launch_fused(const GmsArgs &d, const Shape &s, const Plan *p, const WgradArg
   if (lds < lds_rows) lds = lds_rows;
   { const int rc_lds = allow_dynamic_lds(reinterpret_cast<const void *>(kern), (size_t)lds); if (rc_lds != FGMS_OK) return rc_lds; }
   {
-    ProfileScope prof(raw == 4 ? "bwd_fused_kernel(bf16x3)" : "bwd_fused_kernel", d.stream);
+    ProfileScope prof(RAGGED     ? (raw == 4 ? "bwd_fused_kernel(masked, bf16x3)" : "bwd_fused_kernel(masked)")
+                      : raw == 4 ? "bwd_fused_kernel(bf16x3)"
+                      : g.smap.by_xcd ? "bwd_fused_kernel(by XCD)" : "bwd_fused_kernel",
+                      d.stream);
     SideJob check{};
     (void)plan_take_check(p, &check);
     kern<<<row_x * row_y * row_z + (unsigned)(g.tiles * g.ty) + (unsigned)check.blocks, kThreads, lds, d.stream>>>(
@@ -1693,7 +1699,7 @@ int launch_side_job(const SideJob &job, hipStream_t stream) {
   return FGMS_OK;
 }
 
-// FGMS_SPLIT_BF16=0 keeps fp32 tensors on fp32 MFMAs in "tf32" mode too (for comparison).
+// FGMS_SPLIT_BF16=0 keeps fp32 tensors on fp32 MFMAs, in full precision and in "tf32" mode (for comparison).
 bool split_bf16_enabled() {
   static const bool on = !(getenv("FGMS_SPLIT_BF16") && atoi(getenv("FGMS_SPLIT_BF16")) == 0);
   return on;

@@ -8,9 +8,9 @@
 //   forward          out[row][co] = sum over (k, ci) of in[nbr[k][row]][ci] * W[k][ci][co]
 //   weight gradient  dW[(k, ci)][co] = sum over rows of in[nbr[k][row]][ci] * gout[row][co]
 //
-// The forward pass (fp16; on fp32 the matrix cores are no faster than the vector ALUs) needs no LDS for its rows: a lane of v_mfma_f32_32x32x16_f16 wants 8 consecutive
-// contraction values of one row, i.e. two gathered rows of 4 channels or one of 8, which is what its
-// gathers bring.  The weight gradient reads every output-gradient row once per row and not once per pair,
+// The forward pass (fp16; on fp32 the matrix cores are no faster than the vector ALUs) needs no LDS for its rows: a lane of
+// v_mfma_f32_32x32x16_f16 wants 8 consecutive contraction values of one row, i.e. two gathered rows of 4 channels or one of
+// 8, which is what its gathers bring.  The weight gradient reads every output-gradient row once per row and not once per pair,
 // and its gathers of 8-byte rows stay in the L2.
 //
 // Rows of 3, 5 or 7 halfs lie at odd 2-byte addresses: the aligned words around one are fetched and
@@ -18,7 +18,7 @@
 //
 // Bound by latency: a wave's few dependent loads (mask, index, row) and the launches.  4 -> 32 fp16 over 200 k voxels:
 // forward 14 us (one lane per row and products on the vector ALUs: 20), weight gradient 18 + 4 (pair by pair: 33 + 4).
-// 3 -> 32 over 125 offsets and 78 k voxels, both: 94 us with padded copies and the vector ALUs' kernels, 63 here.
+// 3 -> 32 over 125 offsets and 78 k voxels, both: 93 us with padded copies and the vector ALUs' kernels, 54 here.
 #include "fgms_device.h"
 #include "fgms_internal.h"
 #include "fgms_mma.h"
@@ -515,7 +515,8 @@ int launch_fwd(const GmsArgs &a, const Plan *p, size_t lds) {
 
 constexpr int kSlotPartials = 8;                // workspace of the workgroups' sums
 
-// Workgroups of a weight gradient: one a CU at most (each leaves a tile of sums), and blockIdx.y's range.
+// Workgroups of a weight gradient, one a CU or eight for each of blockIdx.y's range, whichever is more (each leaves a tile of
+// sums), and that range.
 struct NarrowGrid {
   size_t walkers;
   int ny, col_blocks;
@@ -617,7 +618,8 @@ bool narrow_wgrad_supported(const WgradArgs &a, const Plan *p) {
          reinterpret_cast<uintptr_t>(a.in) % 4 == 0 && reinterpret_cast<uintptr_t>(a.gout) % 16 == 0 &&
          buffer_range((size_t)a.n_in * a.c_in * esz) <= kMaxBufferBytes &&
          // (a workspace cannot grow under stream capture)
-         (!is_capturing(a.stream) || workspace_bytes(a.stream, kSlotPartials) >= wgrad_grid(a).bytes()) && (size_t)a.n_out * a.c_out * esz <= kMaxBufferBytes;
+         (!is_capturing(a.stream) || workspace_bytes(a.stream, kSlotPartials) >= wgrad_grid(a).bytes()) &&
+         (size_t)a.n_out * a.c_out * esz <= kMaxBufferBytes;
 }
 
 int launch_narrow_wgrad(const WgradArgs &a, const Plan *p) {

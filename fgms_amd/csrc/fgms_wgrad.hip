@@ -275,7 +275,8 @@ void tile_blocks(const WgradArgs &a, bool shares_grid, int *bi, int *bj) {
   // 500 voxels 25 / 54, 2 k 61 / 60, scattered 20 k 181 / 150.)
   if (a.dtype != FGMS_F16 && !a.reduced && split_bf16_enabled()) {
     const int64_t tiles = (int64_t)(a.c_in / 128) * (a.c_out / 128), rows = a.n_in > a.n_out ? a.n_in : a.n_out;
-    const bool whole = !shares_grid && *bi * *bj == 16 && ((tiles <= 2 && a.n_pairs < 7 * rows) || (tiles >= 2 && a.n_pairs * tiles < 70000));
+    const bool whole = !shares_grid && *bi * *bj == 16 &&
+                       ((tiles <= 2 && a.n_pairs < 7 * rows) || (tiles >= 2 && a.n_pairs * tiles < 70000));
     if (*bi > 2 && !whole) *bi = 2;
     if (*bj > 2 && !whole) *bj = 2;
   }
@@ -428,7 +429,8 @@ static bool mfma_wgrad_shape(const WgradArgs &a) {
 bool mfma_wgrad_supported(const WgradArgs &a) { return takes_narrow(a) || mfma_wgrad_shape(a); }
 
 // One cell's walk waits for the rows it meets -- 3.3 times the cloud's rows to a cell, or its pairs where these
-// are fewer, by what a row of the tile costs -- and the chip multiplies 40 pairs x 32 x 32 channels a nanosecond.  On dense maps the copies always pay, twice over; on thin ones there are too few pairs to cut more
+// are fewer, by what a row of the tile costs -- and the chip multiplies 40 pairs x 32 x 32 channels a nanosecond.
+// On dense maps the copies always pay, twice over; on thin ones there are too few pairs to cut more
 // cells, where the vector ALUs take pieces of 512 pairs x 32 x 32 channels.  Thinned clouds, fp32, copies / vector ALUs:
 // 48 x 48 over 10 k voxels 39 / 42 us, 20 k 67 / 68, 40 k 122 / 88; 128 x 20 over 5 k 30 / 39, 40 k 171 / 90;
 // 32 x 20 over 40 k 49 / 60 (tf32 mode 69 / 61).

@@ -47,3 +47,25 @@ def test_against_float64(n, shape, mode, overwrite):
         bound = (1.1 * roundings * 2.0 ** -24 + (2.0 ** -15 if tf else 0)) * most + 1e-30
         assert ((got.double() - ref).abs() <= bound).all(), ((got.double() - ref).abs() / bound).max()
         assert (f[got.numel():] == 7.0).all()
+
+
+@pytest.mark.parametrize("mode", ["fp32", "tf32"])
+@pytest.mark.parametrize("n,shape,masked", [(30000, (48, 48), True), (30000, (40, 56), True), (30000, (64, 64), False)])
+def test_which_kernels_run(n, shape, masked, mode):
+    """Dense maps and such counts go to the masked tiles, in both passes; whole tiles do not."""
+    from fgms_amd import capi
+    capi.set_kernel_policy(0)
+    vox = clouds.cloud_indoor(clouds.rng_for(4), target=n)
+    imap, omap, knnz, kpos = clouds.build_kernel_map(vox, vox, clouds.offsets_cube(3))
+    x, w, g = (torch.randn(*s, device="cuda") for s in ((len(vox), shape[0]), (27, *shape), (len(vox), shape[1])))
+    maps = tuple(torch.from_numpy(np.ascontiguousarray(t.astype(np.int32))).cuda() for t in (kpos, imap, omap))
+    plan = capi.Plan(*maps, len(vox), len(vox))
+    capi.profile_reset()
+    capi.profile_enable(True)
+    capi.conv_fwd(x, w, torch.empty_like(g), *maps, arch80=mode == "tf32", plan=plan)
+    capi.conv_bwd(g, x, w, torch.empty_like(x), torch.empty_like(w), *maps, arch80=mode == "tf32", plan=plan)
+    capi.profile_enable(False)
+    names = [r[0] for r in capi.profile_records()]
+    capi.profile_reset()
+    assert [q.split("(")[0] for q in names] == ["gms_rows_kernel", "bwd_fused_kernel"], names
+    assert [("masked" in q, "bf16x3" in q) for q in names] == [(masked, mode == "tf32")] * 2, names

@@ -35,3 +35,21 @@ def test_against_float64(n, shape, offsets):
     # fp32 sums (a rounding for each 16 products, one for each workgroup of an offset), rounded to fp16 once
     bound = 2.0 ** -11 * want.abs() + 1.1 * (int(knnz.max()) // 16 + 600) * 2.0 ** -24 * most + 2.0 ** -24
     assert ((gw.double() - want).abs() <= bound).all(), ((gw.double() - want).abs() / bound).max()
+
+
+@pytest.mark.parametrize("n,by_xcd", [(4000, False), (17000, True)])
+def test_either_side_of_the_size(n, by_xcd):
+    from fgms_amd import capi
+    capi.set_kernel_policy(0)
+    vox = clouds.cloud_indoor(clouds.rng_for(6), target=n)
+    imap, omap, knnz, kpos = clouds.build_kernel_map(vox, vox, clouds.offsets_cube(3))
+    x, w, g = (torch.randn(*s, device="cuda").half() for s in ((len(vox), 128), (27, 128, 128), (len(vox), 128)))
+    maps = tuple(torch.from_numpy(np.ascontiguousarray(t.astype(np.int32))).cuda() for t in (kpos, imap, omap))
+    plan = capi.Plan(*maps, len(vox), len(vox))
+    capi.profile_reset()
+    capi.profile_enable(True)
+    capi.conv_bwd(g, x, w, torch.empty_like(x), torch.empty_like(w), *maps, plan=plan)
+    capi.profile_enable(False)
+    names = [r[0] for r in capi.profile_records()]
+    capi.profile_reset()
+    assert ("bwd_fused_kernel(by XCD)" in names) == by_xcd and any(q.startswith("bwd_fused_kernel") for q in names), names
