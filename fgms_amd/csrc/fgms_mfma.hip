@@ -1327,10 +1327,10 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
   // fp32 tensors: products of bf16 parts, two to a value in "tf32" mode, else three (three or eight 16-bit MFMAs instead
   // of sixteen fp32 ones per product tile); needs whole 32-channel slabs
   constexpr bool kCanSplit = sizeof(T) == 4 && S == 4 && NT != 4;
-  // (The pair view at 32 columns gathers as much for half the products, and its atomics bound it: fp32 MFMAs / three parts
-  // 32 -> 32 over 5 k scattered voxels 16 / 18 us, 96 -> 96 over 60 k LiDAR ones 144 / 162; at 64 columns 64 -> 64 over 60 k 97 / 97,
-  // 256 -> 256 over 5 k scattered ones 84 / 63.)
-  const bool three_parts = NT != 3 && !(pair_view && NT == 1);
+  // (The pair view's atomics hide fp32 products where there are workgroups enough, and better at three of them to a CU than at two;
+  // at 32 columns a tile always.  fp32 MFMAs / three parts: 32 -> 32 over 5 k scattered voxels 16 / 18 us, 96 -> 96 over 60 k LiDAR ones
+  // 144 / 162, 128 -> 128 over 20 k scattered ones 67 / 71, 256 -> 256 over 50 k 245 / 266, over 5 k 84 / 63, 64 -> 64 over 20 k 34 / 32.)
+  const bool three_parts = NT != 3 && !(pair_view && (NT == 1 || (int64_t)rg.gx * gy > (int64_t)num_cus() * 2));
   // (Three parts take 6 bytes a weight, at 32-bit offsets: a stream under capture whose workspace holds only the 4 of the other
   // layouts stays on fp32 MFMAs.  Masked channel counts come here with room for them.)
   const size_t bytes = (size_t)a.k_vol * a.c_in * a.c_out * 6;
