@@ -441,11 +441,18 @@ def main():
             # the backward call's single launch computes both gradients
             parts = ("dgrad", "wgrad") if dom.startswith("bwd_fused") else \
                 (("dgrad",) if "dgrad" in dom else (("wgrad",) if "wgrad" in dom else ("fwd",)))
-            # fp32 tensors: every product is several bf16 MFMAs of the values' parts (three in tf32 mode, six in
-            # fp32 mode), so the matrix pipes do that many times the algorithmic flop, at the 16-bit rate
-            six = (arith == "f32" and not arch80 and dom.startswith(("gms_rows", "bwd_fused", "wgrad_wave")) and
-                   L["c_in"] % 32 == 0 and L["c_out"] % 32 == 0 and os.environ.get("FGMS_SPLIT_BF16") != "0")
-            factor = 3 if "bf16x3" in dom else 6 if six else 1
+            # fp32 tensors: every product is several bf16 MFMAs of the values' parts (three in tf32 mode, eight in
+            # fp32 mode), so the matrix pipes do that many times the algorithmic flop, at the 16-bit rate; fp32 MFMAs
+            # (the pair view at 32 columns or over two workgroups a CU, weight-gradient tiles of 32 x 32) take the time of sixteen
+            odd_in, odd_out = L["c_in"] // 32 % 2 == 1, L["c_out"] // 32 % 2 == 1
+            eight = (arith == "f32" and not arch80 and dom.startswith(("gms_rows", "bwd_fused", "wgrad_wave")) and
+                     L["c_in"] % 32 == 0 and L["c_out"] % 32 == 0 and os.environ.get("FGMS_SPLIT_BF16") != "0" and
+                     not ("pair view" in dom and ((odd_in if "dgrad" in dom else odd_out) or
+                                                  len(L["imap"]) / 256 * (L["c_in"] if "dgrad" in dom else L["c_out"]) / 64 > 512)) and
+                     not (dom.startswith("wgrad_wave") and odd_in and odd_out))
+            factor = 3 if "bf16x3" in dom else 8 if eight else 1
+            if eight and dom.startswith("bwd_fused") and odd_in and odd_out:
+                factor = 12
             peak = PEAK_TFLOPS["f16" if factor > 1 else arith]
             ach = factor * len(parts) * flops_pass / avg_s / 1e12
             flow = sum(dataflow_bytes(L, w_) for w_ in parts)
@@ -454,7 +461,7 @@ def main():
                         "unit": "TFLOP/s", "frac": ach / peak, "traffic": traffic,
                         "traffic_source": TRAFFIC_SOURCE if traffic is not None else None,
                         "mfma_flop_per_algorithmic_flop": factor,
-                        # `frac` prices the matrix pipes' work (for bf16 parts: three or six MFMA flop per
+                        # `frac` prices the matrix pipes' work (for bf16 parts: three or eight MFMA flop per
                         # algorithmic flop); frac_algorithmic prices the useful work alone, against
                         # the same 16-bit peak and against the fp32 MFMA peak the tensors' type has
                         "frac_algorithmic": len(parts) * flops_pass / avg_s / 1e12 / peak,
