@@ -1024,7 +1024,9 @@ __global__ __launch_bounds__(kThreads * KG, RAW >= 5 ? (MT == 2 || KG == 2 ? 2 :
     const int32_t *__restrict__ nbr, const unsigned long long *__restrict__ block_masks,
     const int32_t *__restrict__ perm, const int32_t *__restrict__ tile_order, int n_dst, int k_vol,
     int c_src, int c_dst, int part_stages, SideJob side, int pair_view, unsigned src_bytes, int overwrite,
-    int flip, unsigned long long centre, const T *__restrict__ w_raw) {
+    int flip_centre, const T *__restrict__ w_raw) {
+  // (flip, and the centre offset + 1 behind its 8 bits: as an argument of eight bytes its own, the centre's bit made every
+  // launch 0.07 us longer, 10.20 instead of 10.13 us for 32 -> 32 fp16 over 2 k voxels)
   // the leading workgroups of the grid run the side job, if there is one
   int block_x = blockIdx.x;
   if (side.blocks) {
@@ -1036,7 +1038,7 @@ __global__ __launch_bounds__(kThreads * KG, RAW >= 5 ? (MT == 2 || KG == 2 ? 2 :
   }
   gms_rows_body<T, NT, S, RAW, MT, KG, RAGGED>(src, packed, dst, nbr, block_masks, perm, tile_order, n_dst, k_vol, c_src,
                                    c_dst, part_stages, block_x, blockIdx.y, blockIdx.z, gridDim.z, src_bytes, pair_view,
-                                   overwrite, flip, centre, w_raw);
+                                   overwrite, flip_centre & 255, flip_centre >> 8 ? 1ull << ((flip_centre >> 8) - 1) : 0ull, w_raw);
 }
 
 // ---------------------------------------------------------------------------
@@ -1399,7 +1401,7 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
     kern<<<dim3(gx + (unsigned)a.side.blocks, gy, gz), kThreads * kg, lds_rows, a.stream>>>(
         (const T *)a.src, packed, (T *)a.dst, nbr, masks, perm, tile_order, (int)a.n_dst, a.k_vol,
         s.c_src, s.c_dst, part_stages > 0 ? part_stages : 1, a.side, pair_view ? 1 : 0,
-        (unsigned)((size_t)a.n_src * s.c_src * sizeof(T)), overwrite ? 1 : 0, flip, a.centre ? 1ull << (a.centre - 1) : 0ull, (const T *)a.w);
+        (unsigned)((size_t)a.n_src * s.c_src * sizeof(T)), overwrite ? 1 : 0, flip | a.centre << 8, (const T *)a.w);
   }
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;
