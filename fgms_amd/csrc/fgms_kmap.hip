@@ -10,18 +10,18 @@
 //
 //   1. fill     everything that has to start from a value
 //   2. insert   every input row enters its block of 2 x 2 x 4 voxels; the blocks are found through
-//               an open-addressing hash table (linear probing, load <= 0.5); equal coordinates keep the
+//               an open-addressing hash table (linear probing, load <= 0.8); equal coordinates keep the
 //               smallest row
 //   3. lookup   a table of the output rows, [n_out][offsets] -> input row or -1, the
 //               set of offsets every row has a pair through, hits per (offset, 256 rows)
-//   4. scan     prefix sum over those counts
-//   5. lists    hits compacted in (offset, row) order; next to it the histogram of the plan's sort
-//   6. plan     row order and tables (fgms_plan.hip), from the table of step 3: no atomics per
+//   4. lists    prefix sums over those counts, hits compacted in (offset, row) order
+//   5. plan     row order and tables (fgms_plan_sort.h, fgms_plan.hip), from the masks and the table of step 3: no atomics per
 //               pair, no second pass over the lists.  A submanifold map (one coordinate list on
 //               both sides, mirrored offsets) is its own mirror image, so one order and one table
-//               serve both directions.
-// At 100 k voxels x 27 offsets the whole build takes 110 us of the stream; lists alone and a plan from
-// them afterwards took 140 and 195 us, each behind a wait of the host for the one before.
+//               serve both directions.  Steps 4 and 5 share launches (kmap_sizes_kernel).
+// Bound by latencies: eight launches of one or two waves' worth of dependent accesses each.  At 100 k LiDAR voxels x 27 offsets they
+// take 77 us of the stream; with a scan of its own and the lists in front of the plan's sort 98 us; lists alone and a plan from
+// them afterwards 140 and 195 us, each behind a wait of the host for the one before.
 #include <immintrin.h>
 #include <stdlib.h>
 #include <string.h>
@@ -33,6 +33,7 @@
 #include "fgms_device.h"
 #include "fgms_internal.h"
 #include "fgms_plan_build.h"
+#include "fgms_plan_sort.h"
 
 namespace fgms {
 namespace {
@@ -44,16 +45,21 @@ constexpr int kListRows = 256;              // output rows per count
 constexpr int kKernargOffsets = 128;        // offsets that travel as a kernel argument
 // pinned read-back: [0] coordinates looked at, [1] bad one among them, [2] shared ones; [3] sizes there, [4] pairs, [16 ...] sizes
 constexpr int kHostInts = 16 + 1024;
+// A plan's offsets are also counted over all rows: in copies, a row of 64 sums each, so that the atomics of the lookup's workgroups
+// spread over as many lines (all in one: a launch of 1 564 workgroups would wait for its 42 k atomics one behind the other).
+constexpr int kTotalCopies = 64;
 
 struct Offsets {
   int xyz[kKernargOffsets * 3];
 };
 
-// Voxels are found by blocks of 2 x 2 x 4: the hash table holds one row number per block in use (its
-// representative: the row that got there first), and a block's 16 voxels lie in one 64-byte piece of
-// `cells`, at the representative's number.  The 27 neighbours of a voxel lie in 8 blocks, and
+// Voxels are found by blocks of 2 x 2 x 4: the hash table holds the blocks in use, and a block's 16 voxels lie in one 64-byte piece
+// of `cells`, at its slot's number.  The 27 neighbours of a voxel lie in 8 blocks, and
 // neighbouring rows share them: an eighth of the random accesses that a table of voxels costs, which
-// is what such a table is bound by (100 k rows x 27 offsets: 2.7 M probes of a line each).
+// is what such a table is bound by (100 k rows x 27 offsets: 2.7 M probes of a line each).  A slot holds its block's coordinates
+// themselves (59 bits), so that a search is one access to it and one to the cells.  (A row number in the slot, its coordinates
+// behind a load of their own, cells by row: insertion of 29 k rows 6.5 -> 4.8 us,
+// of 200 k 15.6 -> 14.6, the lookup the same.)
 constexpr int kBlockX = 1, kBlockY = 1, kBlockZ = 2;      // bits of a coordinate inside its block
 constexpr int kCells = 1 << (kBlockX + kBlockY + kBlockZ);
 constexpr int kNoRow = INT32_MAX;
@@ -68,12 +74,20 @@ __device__ __forceinline__ unsigned slot_of(int bx, int by, int bz, unsigned mas
   return h & mask;
 }
 __device__ __forceinline__ int cell_of(int x, int y, int z) { return (x & 1) << 3 | (y & 1) << 2 | (z & 3); }
-__device__ __forceinline__ bool same_block(const int32_t *__restrict__ coords, int row, int bx, int by, int bz) {
-  return coords[3 * row] >> kBlockX == bx && coords[3 * row + 1] >> kBlockY == by && coords[3 * row + 2] >> kBlockZ == bz;
+// A block as a slot holds it.  (Blocks of accepted coordinates only, block_exists; a free slot's ones are none of them.)
+typedef unsigned long long BlockKey;
+constexpr BlockKey kFreeSlot = ~0ull;
+__device__ __forceinline__ bool block_exists(int bx, int by, int bz) {
+  constexpr int x = kCoordLimit >> kBlockX, y = kCoordLimit >> kBlockY, z = kCoordLimit >> kBlockZ;
+  return bx >= -x && bx < x && by >= -y && by < y && bz >= -z && bz < z;
+}
+__device__ __forceinline__ BlockKey block_key(int bx, int by, int bz) {
+  constexpr int x = kCoordLimit >> kBlockX, y = kCoordLimit >> kBlockY, z = kCoordLimit >> kBlockZ;
+  return (BlockKey)(unsigned)(bx + x) << 40 | (BlockKey)(unsigned)(by + y) << 20 | (unsigned)(bz + z);
 }
 
 // flags[0]: an input coordinate is outside the range; flags[1]: two input rows share their coordinates
-__global__ __launch_bounds__(256) void kmap_insert_kernel(const int32_t *__restrict__ coords, int n, int32_t *__restrict__ slots,
+__global__ __launch_bounds__(256) void kmap_insert_kernel(const int32_t *__restrict__ coords, int n, BlockKey *__restrict__ slots,
                                                           unsigned mask, int32_t *__restrict__ cells, int *__restrict__ flags) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
@@ -84,27 +98,25 @@ __global__ __launch_bounds__(256) void kmap_insert_kernel(const int32_t *__restr
   }
   const int bx = x >> kBlockX, by = y >> kBlockY, bz = z >> kBlockZ;
   unsigned slot = slot_of(bx, by, bz, mask);
-  int rep = i;
-  while (true) {                       // ends: the table has two slots per row and more
-    const int prev = atomicCAS(&slots[slot], -1, i);
-    if (prev < 0) break;
-    if (same_block(coords, prev, bx, by, bz)) {
-      rep = prev;
-      break;
-    }
+  const BlockKey key = block_key(bx, by, bz);
+  while (true) {                       // ends: the table has more slots than rows
+    const BlockKey prev = atomicCAS(&slots[slot], kFreeSlot, key);
+    if (prev == kFreeSlot || prev == key) break;
     slot = (slot + 1) & mask;
   }
-  if (atomicMin(&cells[(size_t)rep * kCells + cell_of(x, y, z)], i) != kNoRow) flags[1] = 1;
+  if (atomicMin(&cells[(size_t)slot * kCells + cell_of(x, y, z)], i) != kNoRow) flags[1] = 1;
 }
 
 struct LookupArgs {
-  const int32_t *in_coords, *out_coords;
+  const int32_t *out_coords;
   int n_out, k_vol, stride, skip_offset, row_ld;
-  const int32_t *slots, *cells;
+  const BlockKey *slots;
+  const int32_t *cells;
   unsigned mask;
   const int32_t *offsets;                      // device; nullptr: `offs`
   int32_t *rows;                               // [n_out][row_ld]
   int32_t *counts;                             // [k_vol][blocks of kListRows rows]
+  int32_t *totals;                             // [kTotalCopies][64], nullptr: no plan
   int blocks;
   unsigned long long *rmask_out, *rmask_in;    // nullptr: no plan / a mirrored one
   const int *flags;
@@ -120,41 +132,32 @@ __device__ __forceinline__ void publish_coordinates(const int *__restrict__ flag
   __hip_atomic_store(&host[0], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// The representatives of N blocks (-1: not in use; want = false: not asked for), all probed together.
+// The slots of N blocks (-1: not in use; want = false: not asked for), all probed together.
 template <int N>
 __device__ __forceinline__ void find_blocks(const LookupArgs &a, const int (&bx)[N], const int (&by)[N], const int (&bz)[N],
-                                            const bool (&want)[N], int (&rep)[N]) {
+                                            const bool (&want)[N], int (&at)[N]) {
   unsigned slot[N];
+  BlockKey key[N];
   bool open[N], any = false;
 #pragma unroll
   for (int u = 0; u < N; ++u) {
-    rep[u] = -1;
-    open[u] = want[u];
+    at[u] = -1;
+    open[u] = want[u] && block_exists(bx[u], by[u], bz[u]);
     any = any || open[u];
     slot[u] = slot_of(bx[u], by[u], bz[u], a.mask);
+    key[u] = block_key(bx[u], by[u], bz[u]);
   }
-  while (any) {                        // ends: every chain meets its block or an empty slot
-    int cand[N];
+  while (any) {                        // ends: every chain meets its block or a free slot
+    BlockKey cand[N];
 #pragma unroll
-    for (int u = 0; u < N; ++u) cand[u] = open[u] ? a.slots[slot[u]] : -1;
-    int cx[N], cy[N], cz[N];
-#pragma unroll
-    for (int u = 0; u < N; ++u) {
-      const int c = cand[u] < 0 ? 0 : cand[u];
-      cx[u] = a.in_coords[3 * c]; cy[u] = a.in_coords[3 * c + 1]; cz[u] = a.in_coords[3 * c + 2];
-    }
+    for (int u = 0; u < N; ++u) cand[u] = open[u] ? a.slots[slot[u]] : kFreeSlot;
     any = false;
 #pragma unroll
     for (int u = 0; u < N; ++u) {
-      if (cand[u] < 0) {
-        open[u] = false;
-      } else if (cx[u] >> kBlockX == bx[u] && cy[u] >> kBlockY == by[u] && cz[u] >> kBlockZ == bz[u]) {
-        rep[u] = cand[u];
-        open[u] = false;
-      } else if (open[u]) {
-        slot[u] = (slot[u] + 1) & a.mask;
-        any = true;
-      }
+      if (cand[u] == key[u] && open[u]) at[u] = (int)slot[u];
+      open[u] = open[u] && cand[u] != key[u] && cand[u] != kFreeSlot;
+      slot[u] = open[u] ? (slot[u] + 1) & a.mask : slot[u];
+      any = any || open[u];
     }
   }
 }
@@ -163,8 +166,8 @@ __device__ __forceinline__ void find_blocks(const LookupArgs &a, const int (&bx)
 // each.  NEAR (every offset within one voxel): its four waves find two of
 // each row's eight blocks each, then every wave reads every fourth offset's cell from them.  Else
 // (wider kernels) a lane finds the blocks of up to seven offsets at a time for itself.
-// Bound by latency -- slot, representative's coordinates, cell: three dependent loads, with two to
-// seven of each in flight per lane.  17 us at 100 k rows x 27 offsets; one probe chain per thread in a
+// Bound by latency -- slot, cell: two dependent loads, with two to
+// seven of each in flight per lane.  16.5 us at 100 k rows x 27 offsets; one probe chain per thread in a
 // table of voxels took 14.5 us for half of the offsets, a table of voxels probed like this 116 us.
 constexpr int kLookupRows = 64, kLookupChunk = 28;
 template <bool NEAR>
@@ -172,12 +175,13 @@ __global__ __launch_bounds__(256) void kmap_lookup_kernel(LookupArgs a, Offsets 
   constexpr int kMine = kLookupChunk / 4;
   __shared__ int32_t found[kLookupRows][kLookupChunk + 1];
   __shared__ unsigned long long wave_mask[4][kLookupRows];
-  __shared__ int32_t near_rep[8][kLookupRows];
+  __shared__ int32_t near_slot[8][kLookupRows];
   if (blockIdx.x == gridDim.x - 1) {
     publish_coordinates(a.flags, a.host);
     return;
   }
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+  __shared__ int count_of[kLookupChunk];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
   const int o = blockIdx.x * kLookupRows + lane;
   const bool live = o < a.n_out;
   const int oc = live ? o : a.n_out - 1;
@@ -189,7 +193,7 @@ __global__ __launch_bounds__(256) void kmap_lookup_kernel(LookupArgs a, Offsets 
   const int block = blockIdx.x * kLookupRows / kListRows;
   if constexpr (NEAR) {
     // block j of a row: the row's own (bits 0) or the nearer neighbour along x (bit 2), y (bit 1), z (bit 0)
-    int bx[2], by[2], bz[2], rep[2];
+    int bx[2], by[2], bz[2], at[2];
     bool want[2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
@@ -200,25 +204,25 @@ __global__ __launch_bounds__(256) void kmap_lookup_kernel(LookupArgs a, Offsets 
       bz[u] = (z0 >> kBlockZ) + (j & 1 ? dz : 0);
       want[u] = sane && !((j & 1) && dz == 0);
     }
-    find_blocks<2>(a, bx, by, bz, want, rep);
+    find_blocks<2>(a, bx, by, bz, want, at);
 #pragma unroll
-    for (int u = 0; u < 2; ++u) near_rep[wave * 2 + u][lane] = rep[u];
+    for (int u = 0; u < 2; ++u) near_slot[wave * 2 + u][lane] = at[u];
     __syncthreads();
   }
   unsigned long long mine = 0;
   for (int k0 = 0; k0 < a.k_vol; k0 += kLookupChunk) {
-    int hit[kMine], rep[kMine], cell[kMine];
+    int hit[kMine], at[kMine], cell[kMine];
     if constexpr (NEAR) {
 #pragma unroll
       for (int u = 0; u < kMine; ++u) {
         const int k = k0 + u * 4 + wave;
-        rep[u] = -1;
+        at[u] = -1;
         cell[u] = 0;
         if (k < a.k_vol && k != a.skip_offset) {
           const int *d = a.offsets ? a.offsets + 3 * k : offs.xyz + 3 * k;
           const int x = x0 + d[0], y = y0 + d[1], z = z0 + d[2];
           const int j = (x >> kBlockX != x0 >> kBlockX) << 2 | (y >> kBlockY != y0 >> kBlockY) << 1 | (z >> kBlockZ != z0 >> kBlockZ);
-          rep[u] = near_rep[j][lane];
+          at[u] = near_slot[j][lane];
           cell[u] = cell_of(x, y, z);
         }
       }
@@ -239,18 +243,18 @@ __global__ __launch_bounds__(256) void kmap_lookup_kernel(LookupArgs a, Offsets 
           cell[u] = cell_of((int)x, (int)y, (int)z);
         }
       }
-      find_blocks<kMine>(a, bx, by, bz, want, rep);
+      find_blocks<kMine>(a, bx, by, bz, want, at);
     }
 #pragma unroll
-    for (int u = 0; u < kMine; ++u) hit[u] = a.cells[(size_t)(rep[u] < 0 ? 0 : rep[u]) * kCells + cell[u]];
+    for (int u = 0; u < kMine; ++u) hit[u] = a.cells[(size_t)(at[u] < 0 ? 0 : at[u]) * kCells + cell[u]];
 #pragma unroll
     for (int u = 0; u < kMine; ++u) {
       const int k = k0 + u * 4 + wave;
       if (k >= a.k_vol) break;
-      if (rep[u] < 0 || hit[u] == kNoRow) hit[u] = -1;
+      if (at[u] < 0 || hit[u] == kNoRow) hit[u] = -1;
       found[lane][k - k0] = hit[u];
       const unsigned long long b = __ballot(hit[u] >= 0);
-      if (lane == 0 && b) atomicAdd(&a.counts[(size_t)k * a.blocks + block], __builtin_popcountll(b));
+      if (lane == 0) count_of[k - k0] = __builtin_popcountll(b);
       if (a.rmask_out && hit[u] >= 0) {
         mine |= 1ull << k;
         if (a.rmask_in)
@@ -259,6 +263,15 @@ __global__ __launch_bounds__(256) void kmap_lookup_kernel(LookupArgs a, Offsets 
       }
     }
     __syncthreads();
+    // (the workgroup's counts in one instruction: a lane of every wave for itself took 3 us longer)
+    if (threadIdx.x < kLookupChunk && k0 + (int)threadIdx.x < a.k_vol) {
+      const int k = k0 + threadIdx.x;
+      const int n = count_of[threadIdx.x];
+      if (n) {
+        atomicAdd(&a.counts[(size_t)k * a.blocks + block], n);
+        if (a.totals) atomicAdd(&a.totals[blockIdx.x % kTotalCopies * 64 + k], n);
+      }
+    }
     // the chunk's part of every row, 16 bytes a thread
     const int width = min(kLookupChunk, a.row_ld - k0) / 4;
     for (int e = threadIdx.x; e < kLookupRows * width; e += 256) {
@@ -283,7 +296,6 @@ struct ScanArgs {
   int32_t *bases;             // pairs before each of them, and the total behind
   int k_vol, blocks;
   int32_t *kernel_nnz, *kpos, *qkpos;      // (qkpos: nullptr: not wanted)
-  int *plan_flags;            // flags[12] of the plan: its pair count
 };
 
 // Exclusive prefix sum by one workgroup, 4096 values a round: every thread takes four neighbouring
@@ -362,7 +374,6 @@ __global__ __launch_bounds__(1024) void kmap_scan_kernel(ScanArgs a) {
   if (lane == 0) {
     a.kpos[a.k_vol] = carry;
     if (a.qkpos) a.qkpos[0] = 0;
-    if (a.plan_flags) a.plan_flags[12] = carry;
   }
 }
 
@@ -379,31 +390,24 @@ struct ListArgs {
   int *host;                  // pinned
 };
 
-// Workgroup 0 sends the sizes to the host.  Workgroups [1, list_blocks]: 256 output rows each, 28 offsets at a time through LDS; a wave takes
-// every fourth offset and ranks its hits with ballots.  The rest: the histogram of the plan's sort,
-// which needs the row masks only.
-__global__ __launch_bounds__(256) void kmap_lists_kernel(ListArgs a, SortArgs sort, int list_blocks) {
-  constexpr int kWidth = 28;
-  __shared__ int32_t tile[kListRows * (kWidth + 1) > kBins ? kListRows * (kWidth + 1) : kBins];
-  if (blockIdx.x == 0) {
-    if (threadIdx.x >= 64) return;
-    for (int k = threadIdx.x; k < min(a.k_vol, kHostInts - 16); k += 64) a.host[16 + k] = a.kernel_nnz[k];
-    if (threadIdx.x == 0) a.host[4] = a.kpos[a.k_vol];
-    __threadfence_system();
-    if (threadIdx.x == 0) __hip_atomic_store(&a.host[3], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-    if (a.flags) publish_coordinates(a.flags, a.host);
-    return;
-  }
-  const int list_block = blockIdx.x - 1;
-  if (list_block >= list_blocks) {
-    const int b = list_block - list_blocks;
-    const int side = b < sort.side[0].chunks ? 0 : 1;
-    sort_hist_body<256>(sort.side[side], sort, side ? b - sort.side[0].chunks : b, tile);
-    return;
-  }
+// The sizes to the host; threads of the first wave.
+__device__ __forceinline__ void publish_sizes(int k_vol, const int32_t *__restrict__ kernel_nnz, int pairs, int *__restrict__ host) {
+  for (int k = threadIdx.x; k < min(k_vol, kHostInts - 16); k += 64) host[16 + k] = kernel_nnz[k];
+  if (threadIdx.x == 0) host[4] = pairs;
+  __threadfence_system();
+  if (threadIdx.x == 0) __hip_atomic_store(&host[3], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// 256 output rows by THREADS threads, 28 offsets at a time through LDS (`tile`); a wave takes every (THREADS / 64)th offset
+// and ranks its hits with ballots.
+constexpr int kListWidth = 28, kListTile = kListRows * (kListWidth + 1);
+template <int THREADS>
+__device__ __forceinline__ void lists_body(const ListArgs &a, int list_block, int list_blocks, int32_t *__restrict__ tile) {
+  constexpr int kWidth = kListWidth, kWaves = THREADS / 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
   const int row0 = list_block * kListRows;
-  constexpr int kTurns = kWidth / 4;      // 16-byte chunks of a row per thread, and offsets per wave
+  constexpr int kLoads = (kListRows * kWidth / 4 + THREADS - 1) / THREADS;      // 16-byte chunks of rows per thread
+  constexpr int kTurns = (kWidth + kWaves - 1) / kWaves;                        // offsets per wave
   // bounds of the plan's row bands that fall into this block of rows (the last block has those behind
   // it, too): what lies below them inside the block is in the ballots anyway
   int bands = 0, band_rows = 1, c_first = 1, c_last = 0;
@@ -416,31 +420,31 @@ __global__ __launch_bounds__(256) void kmap_lists_kernel(ListArgs a, SortArgs so
   for (int k0 = 0; k0 < a.k_vol; k0 += kWidth) {
     const int width = min(kWidth, a.row_ld - k0) / 4, k_end = min(k0 + kWidth, a.k_vol);
     // (all of a part's loads in flight together)
-    int4v_ v[kTurns];
+    int4v_ v[kLoads];
     int block_first[kTurns], first[kTurns];
 #pragma unroll
-    for (int i = 0; i < kTurns; ++i) {
-      const int e = threadIdx.x + 256 * i, row = row0 + e / width;
+    for (int i = 0; i < kLoads; ++i) {
+      const int e = threadIdx.x + THREADS * i, row = row0 + e / width;
       v[i] = int4v_{-1, -1, -1, -1};
-      if (i < width && row < a.n_out) v[i] = *reinterpret_cast<const int4v_ *>(a.rows + (size_t)row * a.row_ld + k0 + e % width * 4);
+      if (e < kListRows * width && row < a.n_out) v[i] = *reinterpret_cast<const int4v_ *>(a.rows + (size_t)row * a.row_ld + k0 + e % width * 4);
     }
 #pragma unroll
     for (int i = 0; i < kTurns; ++i) {
-      const size_t line = (size_t)min(k0 + wave + 4 * i, a.k_vol - 1) * a.blocks;
+      const size_t line = (size_t)min(k0 + wave + kWaves * i, a.k_vol - 1) * a.blocks;
       block_first[i] = a.bases[line + list_block];
       first[i] = a.bases[line];
     }
 #pragma unroll
-    for (int i = 0; i < kTurns; ++i) {
-      if (i >= width) break;
-      const int e = threadIdx.x + 256 * i;
+    for (int i = 0; i < kLoads; ++i) {
+      const int e = threadIdx.x + THREADS * i;
+      if (e >= kListRows * width) break;
 #pragma unroll
       for (int q = 0; q < 4; ++q) tile[e / width * (kWidth + 1) + e % width * 4 + q] = v[i][q];
     }
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < kTurns; ++i) {
-      const int k = k0 + wave + 4 * i;
+      const int k = k0 + wave + kWaves * i;
       if (k >= k_end) break;
       const int before = block_first[i] - first[i];
       long long pos = block_first[i];
@@ -472,6 +476,146 @@ __global__ __launch_bounds__(256) void kmap_lists_kernel(ListArgs a, SortArgs so
     }
     __syncthreads();
   }
+}
+
+// Maps without a plan.  Workgroup 0 sends the sizes to the host, the others write the lists.
+__global__ __launch_bounds__(256) void kmap_lists_kernel(ListArgs a, int list_blocks) {
+  __shared__ int32_t tile[kListTile];
+  if (blockIdx.x == 0) {
+    if (threadIdx.x >= 64) return;
+    publish_sizes(a.k_vol, a.kernel_nnz, a.kpos[a.k_vol], a.host);
+    if (a.flags) publish_coordinates(a.flags, a.host);
+    return;
+  }
+  lists_body<256>(a, blockIdx.x - 1, list_blocks, tile);
+}
+
+// Maps with a plan: its sort needs the row masks and the offsets' sizes only, so the lists keep out of its way.  Three launches,
+// each of which runs what is ready side by side:
+//   sizes   per-offset tables, and the sizes to the host (workgroup 0); the sort's histogram
+//   bases   the sort's scan; pairs before every block of an offset (a workgroup per offset)
+//   (the sort's scatter)
+//   lists   the sort's windows, and next to them the lists
+// (One workgroup scanning all counts, then lists and histogram, then scan, scatter and windows: 100 k LiDAR voxels x 27 offsets
+// 8.3 + 12.7 + 5.4 + 9.7 + 11.6 us, so 7.0 + 4.5 + 8.9 + 13.4.  The lists next to the scatter instead, which needs 1 024 threads
+// a workgroup: 200 k indoor voxels 25.2 us there and 11.4 for the windows, so 8.6 and 15.4.)
+struct SizeArgs {
+  const int32_t *totals;
+  int32_t *kernel_nnz, *kpos, *qkpos;      // (qkpos: nullptr: not wanted)
+  int *plan_flags;                         // flags[12] of the plan: its pair count
+  int *host;                               // pinned
+};
+__global__ __launch_bounds__(kSortThreads) void kmap_sizes_kernel(SizeArgs a, SortArgs sort) {
+  __shared__ int part[kSortThreads / 64][64];
+  __shared__ int size_of[64];
+  __shared__ int hist[kBins];
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+  auto sizes = [&]() -> const int * {
+    constexpr int kWaves = kSortThreads / 64;
+    int sum = 0;
+#pragma unroll
+    for (int c = 0; c < kTotalCopies / kWaves; ++c) sum += a.totals[(wave + kWaves * c) * 64 + lane];      // (0 from k_vol on)
+    part[wave][lane] = sum;
+    __syncthreads();
+    if (wave == 0) {
+      sum = 0;
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) sum += part[w][lane];
+      size_of[lane] = sum;
+    }
+    __syncthreads();
+    return size_of;
+  };
+  if (blockIdx.x > 0) {
+    const int b = blockIdx.x - 1, side = b < sort.side[0].chunks ? 0 : 1;
+    sort_hist_body(sort.side[side], sort, side ? b - sort.side[0].chunks : b, hist, sizes);
+    return;
+  }
+  (void)sizes();
+  if (wave != 0) return;
+  const int mine = size_of[lane], k_vol = sort.k_vol;
+  int upto = mine, padded = (mine + 255) / 256 * 256;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int up = __shfl_up(upto, d, 64), padded_up = __shfl_up(padded, d, 64);
+    if (lane >= d) {
+      upto += up;
+      padded += padded_up;
+    }
+  }
+  if (lane < k_vol) {
+    a.kernel_nnz[lane] = mine;
+    a.kpos[lane] = upto - mine;
+    if (a.qkpos) a.qkpos[lane + 1] = padded;
+    a.host[16 + lane] = mine;
+  }
+  const int pairs = __shfl(upto, 63, 64);
+  if (lane == 0) {
+    a.kpos[k_vol] = pairs;
+    if (a.qkpos) a.qkpos[0] = 0;
+    a.plan_flags[12] = pairs;
+    a.host[4] = pairs;
+  }
+  __threadfence_system();
+  if (lane == 0) __hip_atomic_store(&a.host[3], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+struct BaseArgs {
+  const int32_t *counts, *kpos;
+  int32_t *bases;
+  int blocks, scans;          // workgroups of the sort's scan per side
+};
+__global__ __launch_bounds__(256) void kmap_bases_kernel(BaseArgs a, SortArgs sort) {
+  const int sides = sort.side[1].n > 0 ? 2 : 1;
+  int k = blockIdx.x - a.scans * sides;
+  if (k < 0) {
+    sort_scan_body(sort.side[blockIdx.x / a.scans], blockIdx.x % a.scans);
+    return;
+  }
+  // exclusive prefix sum of an offset's line, four counts a thread and round
+  __shared__ int wave_total[2][4];
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+  const int32_t *__restrict__ from = a.counts + (size_t)k * a.blocks;
+  int32_t *__restrict__ to = a.bases + (size_t)k * a.blocks;
+  int carry = a.kpos[k], round = 0;
+  for (int base = 0; base < a.blocks; base += 1024, round ^= 1) {
+    int v[4], mine = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int i = base + threadIdx.x * 4 + j;
+      v[j] = i < a.blocks ? from[i] : 0;
+      mine += v[j];
+    }
+    int incl = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int up = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += up;
+    }
+    if (lane == 63) wave_total[round][wave] = incl;
+    __syncthreads();         // (the other buffer is written next round, after every wave has passed this barrier)
+    int run = carry + incl - mine;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const int t = wave_total[round][w];
+      run += w < wave ? t : 0;
+      carry += t;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int i = base + threadIdx.x * 4 + j;
+      if (i < a.blocks) to[i] = run;
+      run += v[j];
+    }
+  }
+}
+
+__global__ __launch_bounds__(kWindowThreads) void kmap_window_lists_kernel(ListArgs a, SortArgs sort, int windows, int list_blocks) {
+  constexpr int kBuf = 2 * kWindow * (int)(sizeof(unsigned long long) / sizeof(int32_t));
+  __shared__ __attribute__((aligned(16))) int32_t lds[kListTile > kBuf ? kListTile : kBuf];
+  const int sides = sort.side[1].n > 0 ? 2 : 1, b = blockIdx.x;
+  if (b < windows * sides) sort_window_body(sort, b / windows, b % windows, reinterpret_cast<unsigned long long *>(lds));
+  else lists_body<kWindowThreads>(a, b - windows * sides, list_blocks, lds);
 }
 
 // Pinned read-back blocks, kept.
@@ -546,8 +690,9 @@ int map_build_begin(MapBuild **build, const int32_t *in_coords, int64_t n_in, co
     for (int c = 0; c < 3; ++c)
       if (offsets_host[3 * (k_vol - 1 - k) + c] != -offsets_host[3 * k + c]) mirror = false;
 
+  // (a quarter more slots than rows at least; surfaces have two to four rows to a block)
   size_t slots = 256;
-  while (slots < 2 * (size_t)n_in) slots <<= 1;
+  while (slots * 4 < 5 * (size_t)n_in) slots <<= 1;
   const int blocks = (int)((n_out + kListRows - 1) / kListRows);
   const int row_ld = (k_vol + 3) / 4 * 4;
   const size_t n_counts = (size_t)k_vol * blocks;
@@ -560,14 +705,16 @@ int map_build_begin(MapBuild **build, const int32_t *in_coords, int64_t n_in, co
   int cap_out = 0, cap_in = 0;
   const int tiles_out = with_plan ? tile_table(n_out, &cap_out) : 0, tiles_in = with_plan ? tile_table(n_in, &cap_in) : 0;
   const size_t so = (size_t)n_out * k_vol, si = mirror ? 0 : (size_t)n_in * k_vol;
-  int32_t *slot_table = nullptr, *cells = nullptr, *rows = nullptr, *counts = nullptr, *bases = nullptr, *offs_dev = nullptr, *flags = nullptr;
+  BlockKey *slot_table = nullptr;
+  int32_t *cells = nullptr, *rows = nullptr, *counts = nullptr, *totals = nullptr, *bases = nullptr, *offs_dev = nullptr, *flags = nullptr;
   unsigned long long *rmask_out = nullptr, *rmask_in = nullptr;
   void *scratch = nullptr;
   auto layout = [&](Arena &keep, Arena &tmp) {
     tmp.take(slot_table, slots);
-    tmp.take(cells, (size_t)n_in * kCells);
+    tmp.take(cells, slots * kCells);
     tmp.take(rows, (size_t)n_out * row_ld);
     tmp.take(flags, 64);
+    if (with_plan) tmp.take(totals, (size_t)kTotalCopies * 64);
     tmp.take(counts, n_counts);                     // (behind the flags: one fill)
     tmp.take(bases, n_counts + 1);
     if (k_vol > kKernargOffsets) tmp.take(offs_dev, (size_t)k_vol * 3);
@@ -631,8 +778,8 @@ int map_build_begin(MapBuild **build, const int32_t *in_coords, int64_t n_in, co
     }
   }
   FillBatch fills{};
-  fills.add(slot_table, slots * sizeof(int32_t), -1);
-  fills.add(cells, (size_t)n_in * kCells * sizeof(int32_t), kNoRow);
+  fills.add(slot_table, slots * sizeof(BlockKey), -1);
+  fills.add(cells, slots * kCells * sizeof(int32_t), kNoRow);
   fills.add(flags, (size_t)((char *)(counts + n_counts) - (char *)flags), 0);
   if (p) {
     fills.add(p->flags, kPlanFlags * sizeof(int), 0);
@@ -658,30 +805,35 @@ int map_build_begin(MapBuild **build, const int32_t *in_coords, int64_t n_in, co
   }
   if (n_out > 0 && n_in > 0) {
     ProfileScope prof("kmap_lookup_kernel", s);
-    LookupArgs la{in_coords, out_coords, (int)n_out, k_vol, stride, skip_offset, row_ld, slot_table, cells, mask, offs_dev,
-                  rows, counts, blocks, rmask_out, rmask_in, flags, host_dev};
+    LookupArgs la{out_coords, (int)n_out, k_vol, stride, skip_offset, row_ld, slot_table, cells, mask, offs_dev,
+                  rows, counts, totals, blocks, rmask_out, rmask_in, flags, host_dev};
     bool near = true;
     for (int q = 0; q < 3 * k_vol; ++q) near = near && offsets_host[q] >= -1 && offsets_host[q] <= 1;
     auto kern = near ? kmap_lookup_kernel<true> : kmap_lookup_kernel<false>;
     kern<<<(unsigned)((n_out + kLookupRows - 1) / kLookupRows) + 1, 256, 0, s>>>(la, offs);
   }
-  {
-    ScanArgs sc{counts, bases, k_vol, blocks, kernel_nnz, kpos, qkpos, p ? p->flags : nullptr};
-    kmap_scan_kernel<<<1, 1024, 0, s>>>(sc);
-  }
-  {
+  ListArgs la{rows, (int)n_out, k_vol, row_ld, blocks, bases, in_map, out_map, (long long)capacity, p ? p->band_start : nullptr, num_cus(),
+              kernel_nnz, kpos, n_out > 0 && n_in > 0 ? nullptr : flags, host_dev};
+  const int list_blocks = n_in > 0 ? blocks : 0;
+  if (p) {
+    sort.by_mask = plan_sorts_rows();
+    if (!sort.by_mask) sort.side[0].chunks = sort.side[1].chunks = 0;
+    const int chunks = sort.side[0].chunks + sort.side[1].chunks, scans = chunks ? kBins / kScanBins : 0, sides = mirror ? 1 : 2;
+    kmap_sizes_kernel<<<(unsigned)(1 + chunks), kSortThreads, 0, s>>>(SizeArgs{totals, kernel_nnz, kpos, qkpos, p->flags, host_dev}, sort);
+    kmap_bases_kernel<<<(unsigned)(scans * sides + k_vol), 256, 0, s>>>(BaseArgs{counts, kpos, bases, blocks, scans}, sort);
+    if (chunks && (rc = launch_sort_scatter(sort, s))) return fail(rc);
     ProfileScope prof("kmap_write_kernel", s);
-    ListArgs la{rows, (int)n_out, k_vol, row_ld, blocks, bases, in_map, out_map, (long long)capacity, p ? p->band_start : nullptr, num_cus(),
-                kernel_nnz, kpos, n_out > 0 && n_in > 0 ? nullptr : flags, host_dev};
-    const int hist_blocks = p ? sort.side[0].chunks + sort.side[1].chunks : 0;
-    const int list_blocks = n_in > 0 ? blocks : 0;
-    kmap_lists_kernel<<<(unsigned)(1 + list_blocks + hist_blocks), 256, 0, s>>>(la, sort, list_blocks);
+    const int windows = (int)(((mirror || n_out > n_in ? n_out : n_in) + kWindow - 1) / kWindow);
+    kmap_window_lists_kernel<<<(unsigned)(windows * sides + list_blocks), kWindowThreads, 0, s>>>(la, sort, windows, list_blocks);
+  } else {
+    kmap_scan_kernel<<<1, 1024, 0, s>>>(ScanArgs{counts, bases, k_vol, blocks, kernel_nnz, kpos, qkpos});
+    ProfileScope prof("kmap_write_kernel", s);
+    kmap_lists_kernel<<<(unsigned)(1 + list_blocks), 256, 0, s>>>(la, list_blocks);
   }
   if (hipGetLastError() != hipSuccess) {
     set_error("fgms_build_kernel_map: a kernel launch failed");
     return fail(FGMS_E_HIP);
   }
-  if (p && (rc = launch_sort(sort, true, s))) return fail(rc);
   if (p) {
     TablesArgs ta{};
     p->n_pairs = (int64_t)k_vol * n_out;         // (a bound; the count is known to the device only)

@@ -15,6 +15,7 @@
 #include "fgms_device.h"
 #include "fgms_internal.h"
 #include "fgms_plan_build.h"
+#include "fgms_plan_sort.h"
 
 namespace fgms {
 namespace {
@@ -104,238 +105,19 @@ __global__ __launch_bounds__(kSortThreads) void sort_hist_kernel(SortArgs a) {
   const SortSide &sd = a.side[blockIdx.y];
   if ((int)blockIdx.x >= sd.chunks) return;
   __shared__ int hist[kBins];
-  sort_hist_body<kSortThreads>(sd, a, blockIdx.x, hist);
+  sort_hist_body(sd, a, blockIdx.x, hist, [] { return (const int *)nullptr; });
 }
 
-// hist[chunk][bin] -> hist_before[chunk][bin] = rows of the bin in earlier chunks, and
-// bin_total[bin].  Bins are independent: 64 of them per workgroup of 256 threads, a quarter of the
-// chunks each (one workgroup alone reads the 800 KB of counts at 30 GB/s).
-constexpr int kScanBins = 64;
-__global__ __launch_bounds__(256) void sort_scan_kernel(SortArgs a) {
-  const SortSide &sd = a.side[blockIdx.y];
-  if (sd.chunks == 0) return;
-  __shared__ int part_sum[4][kScanBins];
-  const int part = threadIdx.x / kScanBins, b = threadIdx.x % kScanBins;
-  const int bin = blockIdx.x * kScanBins + b;
-  const int per = (sd.chunks + 3) / 4, c0 = min(part * per, sd.chunks), c1 = min(c0 + per, sd.chunks);
-  const int32_t *__restrict__ h = sd.hist + bin;
-  int32_t *__restrict__ hb = sd.hist_before + bin;
-  int sum = 0;
-#pragma unroll 8
-  for (int c = c0; c < c1; ++c) sum += h[(size_t)c * kBins];
-  part_sum[part][b] = sum;
-  __syncthreads();
-  int run = 0;
-  for (int q = 0; q < part; ++q) run += part_sum[q][b];
-#pragma unroll 8
-  for (int c = c0; c < c1; ++c) {
-    const int v = h[(size_t)c * kBins];
-    hb[(size_t)c * kBins] = run;
-    run += v;
-  }
-  if (part == 3) sd.bin_start[bin] = run;        // (the bin's total; the scatter kernel turns totals into starts)
-}
+__global__ __launch_bounds__(256) void sort_scan_kernel(SortArgs a) { sort_scan_body(a.side[blockIdx.y], blockIdx.x); }
 
-// Value of the lane whose number differs from this lane's in bit J.
-template <int J>
-__device__ __forceinline__ unsigned lane_xor(unsigned v) {
-  const int x = (int)v;
-  if constexpr (J == 1) return (unsigned)__builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, true);           // quad_perm [1,0,3,2]
-  else if constexpr (J == 2) return (unsigned)__builtin_amdgcn_mov_dpp(x, 0x4E, 0xF, 0xF, true);      // quad_perm [2,3,0,1]
-  else if constexpr (J == 4)                                                                          // row_half_mirror, quad_perm [3,2,1,0]
-    return (unsigned)__builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(x, 0x141, 0xF, 0xF, true), 0x1B, 0xF, 0xF, true);
-  else if constexpr (J == 8) return (unsigned)__builtin_amdgcn_mov_dpp(x, 0x128, 0xF, 0xF, true);     // row_ror:8
-  else return (unsigned)__shfl_xor(x, J);
-}
-template <int J>
-__device__ __forceinline__ unsigned long long lane_xor(unsigned long long v) {
-  return (unsigned long long)lane_xor<J>((unsigned)v) | (unsigned long long)lane_xor<J>((unsigned)(v >> 32)) << 32;
-}
-
-// Bitonic sort of kWindow keys, ascending, by kWindowThreads threads: wave w holds elements w * 128 ...
-// in two registers per lane (element w * 128 + r * 64 + lane in key[r]), so that 49 of the 55 phases
-// are register exchanges inside a wave (most of them on the vector ALUs alone) and only the 6 with
-// partners 128 or more apart go through LDS (`buf`: 2 x kWindow keys).  The vector ALUs are its
-// limit, hence small windows on many CUs: 2048 keys by 1024 threads took 13 us, with every phase in LDS 25.
-template <typename K, int K2, int J>
-__device__ __forceinline__ void bitonic_phases(K (&key)[2], K *buf, int base, int lane, int &flip) {
-  if constexpr (J >= 128) {
-    K *to = buf + flip * kWindow;
-    flip ^= 1;
-    to[base + lane] = key[0];
-    to[base + 64 + lane] = key[1];
-    __syncthreads();
-    const bool low = ((base & J) == 0) == ((base & K2) == 0);      // (J, K2 >= 128: bits of the wave's number)
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      const K o = to[(base ^ J) + r * 64 + lane];
-      key[r] = (o < key[r]) == low ? o : key[r];
-    }
-  } else if constexpr (J == 64) {
-    const bool asc = (base & K2) == 0;
-    const K lo = key[0] < key[1] ? key[0] : key[1], hi = key[0] < key[1] ? key[1] : key[0];
-    key[0] = asc ? lo : hi;
-    key[1] = asc ? hi : lo;
-  } else {
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      const int i = base + r * 64 + lane;
-      const K o = lane_xor<J>(key[r]);
-      const bool low = ((lane & J) == 0) == ((i & K2) == 0);
-      key[r] = (o < key[r]) == low ? o : key[r];
-    }
-  }
-  if constexpr (J > 1) bitonic_phases<K, K2, J / 2>(key, buf, base, lane, flip);
-}
-template <typename K, int K2 = 2>
-__device__ __forceinline__ void bitonic_window(K (&key)[2], K *buf, int base, int lane, int &flip) {
-  bitonic_phases<K, K2, K2 / 2>(key, buf, base, lane, flip);
-  if constexpr (K2 < kWindow) bitonic_window<K, K2 * 2>(key, buf, base, lane, flip);
-}
-
-// Stable scatter of a chunk's rows into bin order.  Lanes of a wave that share a bin find each other
-// with one ballot per bit of the bin; the waves then take their bins' counters in turn, the rows of a
-// wave as one addition per bin.  (Sorting the chunk instead, in registers as above: 9 us.)
 __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(SortArgs a) {
-  const SortSide &sd = a.side[blockIdx.y];
-  const int chunk = blockIdx.x;
-  if (chunk >= sd.chunks) return;
-  __shared__ int next[kBins];          // where the bin's next row goes
-  __shared__ int part[kSortThreads / 64];
-  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-  constexpr int kBatches = kChunk / kSortThreads;
-  int bin[kBatches], rank[kBatches], peers[kBatches];
-  bool first[kBatches];
-#pragma unroll
-  for (int r = 0; r < kBatches; ++r) {
-    const int row = chunk * kChunk + (wave * kBatches + r) * 64 + lane;
-    const bool live = row < sd.n;
-    bin[r] = live ? top_bits(sd.key[row], a.k_vol) : -1;
-    unsigned long long same = __ballot(live);
-#pragma unroll
-    for (int bit = 0; bit < kBinBits; ++bit) {
-      const bool set = bin[r] >> bit & 1;
-      const unsigned long long b = __ballot(set);
-      same &= set ? b : ~b;
-    }
-    const unsigned long long below = same & ((1ull << lane) - 1);
-    rank[r] = __builtin_popcountll(below);
-    peers[r] = __builtin_popcountll(same);
-    first[r] = live && below == 0;
-  }
-  // rows in smaller bins: exclusive scan of the bin totals (thread, wave, workgroup)
-  {
-    constexpr int kPer = kBins / kSortThreads;
-    int mine[kPer], local = 0;
-#pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-      mine[q] = sd.bin_start[threadIdx.x * kPer + q];
-      local += mine[q];
-    }
-    int incl = local;
-    for (int d = 1; d < 64; d <<= 1) {
-      const int up = __shfl_up(incl, d);
-      if (lane >= d) incl += up;
-    }
-    if (lane == 63) part[wave] = incl;
-    __syncthreads();
-    int before = incl - local;
-    for (int wv = 0; wv < wave; ++wv) before += part[wv];
-#pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-      const int b = threadIdx.x * kPer + q;
-      next[b] = before + sd.hist_before[(size_t)chunk * kBins + b];
-      before += mine[q];
-    }
-  }
-  __syncthreads();
-  int at[kBatches];
-  for (int turn = 0; turn < kSortThreads / 64; ++turn) {
-    if (wave == turn) {
-#pragma unroll
-      for (int r = 0; r < kBatches; ++r) {
-        at[r] = bin[r] >= 0 ? next[bin[r]] : 0;
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        if (first[r]) next[bin[r]] = at[r] + peers[r];
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-      }
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int r = 0; r < kBatches; ++r)
-    if (bin[r] >= 0) sd.perm_tmp[at[r] + rank[r]] = chunk * kChunk + (wave * kBatches + r) * 64 + lane;
+  __shared__ int next[kBins];
+  if ((int)blockIdx.x < a.side[blockIdx.y].chunks) sort_scatter_body(a.side[blockIdx.y], a, blockIdx.x, next);
 }
 
-// Full sort by (key, row) of a window of positions (of keys over more than 32 offsets: by the top
-// 32 bits); writes the final order and its inverse, and what the window's blocks of 64 positions use:
-// block_mask = the OR of their rows' masks, flags[4 + side] += (block, offset) combinations in use,
-// flags[10 + side] += offset bits of all rows.  chunks == 0: the window starts from the identity
-// order (sides of one window).
 __global__ __launch_bounds__(kWindowThreads) void sort_window_kernel(SortArgs a) {
-  const SortSide &sd = a.side[blockIdx.y];
-  const int p0 = blockIdx.x * kWindow;
-  if (p0 >= sd.n) return;
   __shared__ unsigned long long buf[2 * kWindow];
-  __shared__ int sums[kWindowThreads / 64][2];
-  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, base = wave * 128;
-  const int shift = a.k_vol > 32 ? a.k_vol - 32 : 0;
-  unsigned long long key[2];
-  __shared__ unsigned char order[64];
-  if (a.by_mask && sd.chunks == 0) {           // (no histogram has left keys)
-    sort_offset_order(a.kpos, a.k_vol, order);
-    __syncthreads();
-  }
-#pragma unroll
-  for (int r = 0; r < 2; ++r) {
-    const int p = p0 + base + r * 64 + lane;
-    key[r] = ~0ull;
-    if (p < sd.n) {
-      const int row = sd.chunks ? sd.perm_tmp[p] : p;
-      const unsigned long long full = !a.by_mask ? 0ull : sd.chunks ? sd.key[row] : sort_key(sd.rmask[row], a.k_vol, order);
-      key[r] = (full >> shift) << 32 | (unsigned)row;
-    }
-  }
-  int flip = 0;
-  bitonic_window(key, buf, base, lane, flip);
-  int bits = 0, row_bits = 0;
-  const int centre = empty_centre(a.kpos, a.k_vol);
-  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) a.flags[kFlagCentre] = centre >= 0;
-#pragma unroll
-  for (int r = 0; r < 2; ++r) {
-    const int p = p0 + base + r * 64 + lane;
-    unsigned long long m = 0;
-    if (p < sd.n) {
-      const int row = (int)(unsigned)key[r];
-      sd.perm[p] = row;
-      if (centre >= 0) sd.nbr[(size_t)centre * sd.n + p] = row;
-      sd.inv[row] = p;
-      m = sd.rmask[row];
-    }
-    int rb = __popcll(m);
-    for (int d = 32; d > 0; d >>= 1) {
-      m |= __shfl_xor(m, d);
-      rb += __shfl_xor(rb, d);
-    }
-    if (p0 + base + r * 64 < sd.n) {
-      const int block = (p0 + base) / 64 + r;
-      if (lane == 0) sd.block_mask[block] = m;
-      bits += __popcll(m);
-      row_bits += rb;
-    }
-  }
-  if (lane == 0) {
-    sums[wave][0] = bits;
-    sums[wave][1] = row_bits;
-  }
-  __syncthreads();
-  if (threadIdx.x < 2) {
-    int sum = 0;
-    for (int i = 0; i < kWindowThreads / 64; ++i) sum += sums[i][threadIdx.x];
-    if (sum) atomicAdd(&a.flags[(threadIdx.x ? 10 : 4) + blockIdx.y], sum);
-  }
+  sort_window_body(a, blockIdx.y, blockIdx.x, buf);
 }
 
 // Pair view: the pair lists with every offset's run padded to a multiple of 64 rows
@@ -546,8 +328,9 @@ __device__ __forceinline__ void tile_order_body(const TileSide &sd, int cus_per_
 __device__ __forceinline__ void bands_body(const TablesArgs &a, int x, int shift, int32_t *__restrict__ lds) {
   const int k_vol = a.k_vol, bands = a.bands ? a.bands : band_count_of(a.kpos[a.k_vol], a.k_vol, a.cus);
   const int per_xcd = (bands / 8) * k_vol;
-  int *count = lds;                       // [per_xcd]
-  int *group = lds + per_xcd;             // [per_xcd]
+  // [per_xcd], the last four's worth rounded up: the smaller, the earlier
+  unsigned *key = reinterpret_cast<unsigned *>(lds);
+  const int padded = (per_xcd + 3) & ~3;
   auto below = [&](int first, int n, long long target) {      // first pair with omap >= target
     int lo = 0, hi = n;
     while (lo < hi) {
@@ -568,23 +351,26 @@ __device__ __forceinline__ void bands_body(const TablesArgs &a, int x, int shift
       b0 = below(first, n, (long long)band * a.band_rows);
       b1 = band + 1 == bands ? n : below(first, n, (long long)(band + 1) * a.band_rows);
     }
-    count[o] = b1 - b0;
-    group[o] = q >> shift;
+    key[o] = (unsigned)(q >> shift) << 27 | ((1u << 27) - 1 - min((unsigned)(b1 - b0), (1u << 27) - 1));
     if (shift == 0 && !a.bands_known) {
       a.band_start[k * (bands + 1) + band] = b0;
       if (band + 1 == bands) a.band_start[k * (bands + 1) + bands] = n;
     }
   }
+  for (int o = per_xcd + threadIdx.x; o < padded; o += blockDim.x) key[o] = ~0u;
   __syncthreads();
+  typedef unsigned uint4v_ __attribute__((ext_vector_type(4)));
   for (int c = threadIdx.x; c < per_xcd; c += blockDim.x) {
-    const int mine = count[c], my_group = group[c];
+    const unsigned mine = key[c];
     int rank = 0;
-#pragma unroll 8      // (independent LDS reads in flight: the loop is bound by their latency)
-    for (int o = 0; o < per_xcd; ++o) {
-      const int theirs = count[o], their_group = group[o];
-      const bool before = their_group != my_group ? their_group < my_group
-                                                   : (theirs > mine || (theirs == mine && o < c));
-      rank += before ? 1 : 0;
+    // (Bound by the reads' latency: four keys a read, four reads in flight.  Count and group of one cell at a time, 108 cells 14 us and
+    // 216 cells 26, were what the launch waited for: over 100 k LiDAR and 200 k indoor voxels, 27 offsets, 17.2 -> 11.6 us
+    // and 28.8 -> 17.2.)
+#pragma unroll 4
+    for (int o = 0; o < padded; o += 4) {
+      const uint4v_ theirs = *reinterpret_cast<const uint4v_ *>(key + o);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) rank += theirs[e] < mine || (theirs[e] == mine && o + e < c) ? 1 : 0;
     }
     a.band_cells[(size_t)shift * bands * k_vol + rank * 8 + x] = (c % k_vol) * 65536 + (c / k_vol) * 8 + x;
   }
@@ -732,21 +518,33 @@ void sort_side_layout(SortSide &sd, int64_t n, Arena &tmp) {
   }
 }
 
-int launch_sort(const SortArgs &args, bool hist_done, hipStream_t s) {
-  // FGMS_PLAN_SORT=0 keeps the rows in their natural order (for comparison).
+// FGMS_PLAN_SORT=0 keeps the rows in their natural order (for comparison).
+bool plan_sorts_rows() {
   static const bool sort_rows = !(getenv("FGMS_PLAN_SORT") && atoi(getenv("FGMS_PLAN_SORT")) == 0);
+  return sort_rows;
+}
+
+static unsigned sides_of(const SortArgs &a) { return a.side[1].n > 0 ? 2 : 1; }
+static int most_chunks(const SortArgs &a) { return a.side[0].chunks > a.side[1].chunks ? a.side[0].chunks : a.side[1].chunks; }
+
+int launch_sort_scatter(const SortArgs &a, hipStream_t s) {
+  sort_scatter_kernel<<<dim3((unsigned)most_chunks(a), sides_of(a)), kSortThreads, 0, s>>>(a);
+  FGMS_HIP_TRY(hipGetLastError());
+  return FGMS_OK;
+}
+
+int launch_sort(const SortArgs &args, hipStream_t s) {
   SortArgs a = args;
-  a.by_mask = sort_rows;
-  if (!sort_rows) a.side[0].chunks = a.side[1].chunks = 0;
-  const int most = a.side[0].n > a.side[1].n ? a.side[0].n : a.side[1].n;
-  const int chunks = a.side[0].chunks > a.side[1].chunks ? a.side[0].chunks : a.side[1].chunks;
-  const unsigned sides = a.side[1].n > 0 ? 2 : 1;
-  if (chunks) {
-    if (!hist_done) sort_hist_kernel<<<dim3((unsigned)chunks, sides), kSortThreads, 0, s>>>(a);
-    sort_scan_kernel<<<dim3(kBins / kScanBins, sides), 256, 0, s>>>(a);
-    sort_scatter_kernel<<<dim3((unsigned)chunks, sides), kSortThreads, 0, s>>>(a);
+  a.by_mask = plan_sorts_rows();
+  if (!a.by_mask) a.side[0].chunks = a.side[1].chunks = 0;
+  if (const int chunks = most_chunks(a)) {
+    sort_hist_kernel<<<dim3((unsigned)chunks, sides_of(a)), kSortThreads, 0, s>>>(a);
+    sort_scan_kernel<<<dim3(kBins / kScanBins, sides_of(a)), 256, 0, s>>>(a);
+    const int rc = launch_sort_scatter(a, s);
+    if (rc != FGMS_OK) return rc;
   }
-  if (most) sort_window_kernel<<<dim3((unsigned)((most + kWindow - 1) / kWindow), sides), kWindowThreads, 0, s>>>(a);
+  const int most = a.side[0].n > a.side[1].n ? a.side[0].n : a.side[1].n;
+  if (most) sort_window_kernel<<<dim3((unsigned)((most + kWindow - 1) / kWindow), sides_of(a)), kWindowThreads, 0, s>>>(a);
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;
 }
@@ -757,7 +555,7 @@ int launch_tables(TablesArgs a, hipStream_t s) {
   a.tile_blocks = 8;                               // (two at work; the parts behind start on a multiple of eight)
   a.band_blocks = 0;
   if (a.band_start) {
-    const size_t need = (size_t)2 * ((a.bands ? a.bands : 64) / 8) * a.k_vol * sizeof(int32_t);
+    const size_t need = ((size_t)((a.bands ? a.bands : 64) / 8) * a.k_vol + 3) * sizeof(int32_t);
     if (need > lds) lds = need;
     a.band_blocks = 32;
   }
@@ -930,7 +728,7 @@ int plan_create(fgms_plan_t **plan_out, const int32_t *kpos, const int32_t *in_m
       pair_masks_kernel<<<(unsigned)((n_pairs + 255) / 256) + kPrintParts, 256, 0, s>>>(
           kpos, in_map, out_map, k_vol, (int)n_pairs, (int)n_in, (int)n_out, rmask, rmask + n_out, p->flags,
           want_bands ? p->band_start : nullptr, p->band_count, p->band_rows > 0 ? p->band_rows : 1);
-    if ((rc = launch_sort(sa, false, s))) return fail(rc);
+    if ((rc = launch_sort(sa, s))) return fail(rc);
     ta.inv_out = sa.side[0].inv; ta.inv_in = sa.side[1].inv;
     ta.nbr_out = p->nbr_out; ta.nbr_in = p->nbr_in;
     ta.bands_known = true;

@@ -70,84 +70,12 @@ __device__ __forceinline__ int empty_centre(const int32_t *__restrict__ kpos, in
   return k_vol % 2 == 1 && kpos[mid] == kpos[mid + 1] ? mid : -1;
 }
 
-// Bin of a key.
-__device__ __forceinline__ int top_bits(unsigned long long key, int k_vol) {
-  const int shift = k_vol > kBinBits ? k_vol - kBinBits : 0;
-  return (int)((key >> shift) & (kBins - 1));
-}
-
-// The order of the offsets in a sort key, most significant first: by the number of their pairs,
-// rarest first.  `order`: 64 bytes of LDS; the caller's barrier publishes it.  (A lane per offset, compared through
-// shuffles: one trip to memory instead of one per offset.)
-__device__ __forceinline__ void sort_offset_order(const int32_t *__restrict__ kpos, int k_vol, unsigned char *order) {
-  const int k = threadIdx.x;
-  if (k >= 64) return;
-  const int mine = k < k_vol ? kpos[k + 1] - kpos[k] : 0;
-  int rank = 0;
-  for (int o = 0; o < k_vol; ++o) {
-    const int theirs = __shfl(mine, o);
-    rank += theirs < mine || (theirs == mine && o < k) ? 1 : 0;
-  }
-  if (k < k_vol) order[rank] = (unsigned char)k;
-}
-
-// A row's place among all sets of offsets: the set as a number whose high bits are the rare offsets,
-// counted in Gray code, so that sets next to each other differ in few offsets.  Rows that have a rare
-// offset are few: kept together they load few blocks with it.  (Counted with bins and
-// windows of the sort's sizes, 64-row blocks x offsets over pairs / 64 on 120 k LiDAR voxels: by the mask
-// as a number 1.39, rarest first 1.30, in Gray code too 1.28; 256-row tiles x offsets over pairs / 256
-// 1.62, 1.47, 1.45; on 200 k indoor voxels 1.13, 1.12, 1.11 and 1.32, 1.28, 1.25.)
-template <int N>
-__device__ __forceinline__ void sort_keys(unsigned long long (&mask)[N], int k_vol, const unsigned char *order) {
-  unsigned long long key[N] = {};
-  for (int b = 0; b < k_vol; ++b) {
-    const int bit = order[b];
-#pragma unroll
-    for (int r = 0; r < N; ++r) key[r] = key[r] << 1 | (mask[r] >> bit & 1);
-  }
-#pragma unroll
-  for (int r = 0; r < N; ++r) {
-#pragma unroll
-    for (int s = 1; s < 64; s <<= 1) key[r] ^= key[r] >> s;
-    mask[r] = key[r];
-  }
-}
-__device__ __forceinline__ unsigned long long sort_key(unsigned long long mask, int k_vol, const unsigned char *order) {
-  unsigned long long key[1] = {mask};
-  sort_keys<1>(key, k_vol, order);
-  return key[0];
-}
-
-// Keys and rows per bin of one chunk; `hist`: kBins ints of LDS.  A thread's rows are loaded and turned into keys side by
-// side, not one after the other: latencies bound this, not bytes.  (Launch of the lists and the histogram, together with
-// the offsets' order from shuffles and the list blocks' loads in flight together: 27 offsets over 100 k LiDAR voxels 14.5 -> 13.0
-// us, over the 30 k of the next level 13.3 -> 10.7, the 8 between them 10.2 -> 8.1.)
-template <int THREADS>
-__device__ __forceinline__ void sort_hist_body(const SortSide &sd, const SortArgs &a, int chunk, int *hist) {
-  constexpr int kRows = kChunk / THREADS;
-  __shared__ unsigned char order[64];
-  const int first = chunk * kChunk + threadIdx.x;
-  unsigned long long key[kRows];
-#pragma unroll
-  for (int r = 0; r < kRows; ++r) key[r] = first + r * THREADS < sd.n ? sd.rmask[first + r * THREADS] : 0ull;
-  sort_offset_order(a.kpos, a.k_vol, order);
-  for (int i = threadIdx.x; i < kBins; i += THREADS) hist[i] = 0;
-  __syncthreads();
-  sort_keys<kRows>(key, a.k_vol, order);
-#pragma unroll
-  for (int r = 0; r < kRows; ++r) {
-    if (first + r * THREADS >= sd.n) break;
-    sd.key[first + r * THREADS] = key[r];
-    atomicAdd(&hist[top_bits(key[r], a.k_vol)], 1);
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < kBins; i += THREADS) sd.hist[(size_t)chunk * kBins + i] = hist[i];
-}
-
 // Lays out a side's temporaries.
 void sort_side_layout(SortSide &sd, int64_t n, Arena &tmp);
-// Histogram (unless the caller's own launch took it), scan, scatter, window sort.
-int launch_sort(const SortArgs &a, bool hist_done, hipStream_t s);
+bool plan_sorts_rows();                                  // false: rows stay in their natural order
+int launch_sort_scatter(const SortArgs &a, hipStream_t s);
+// Histogram, scan, scatter, window sort.
+int launch_sort(const SortArgs &a, hipStream_t s);
 
 // Weight-gradient row bands: 8, 16, 32 or 64 (the XCDs take them in groups of 1, 2, 4 or 8;
 // other counts measured worse), the fewest that leave an (offset, band) cell at most ~1 900

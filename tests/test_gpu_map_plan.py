@@ -70,6 +70,46 @@ def test_kinds_of_maps(oracle):
     check(oracle, vox[:700], vox[:700], np.concatenate([clouds.offsets_cube(5), clouds.offsets_cube(3) * 4]))   # 152
 
 
+@pytest.mark.parametrize("k_vol", [1, 8, 9, 33, 41, 63, 64])
+def test_numbers_of_offsets(oracle, k_vol):
+    """Whole and part bytes of a row's set of offsets, keys of more than 32 bits."""
+    check(oracle, cloud(2500), cloud(2500), clouds.offsets_cube(5)[30:30 + k_vol])
+
+
+def test_sides_of_one_window_and_of_many(oracle):
+    vox = cloud(2600)
+    coarse = clouds.downsample_coords(vox, 2)
+    assert len(coarse) < 1024 < len(vox)
+    check(oracle, vox, coarse, clouds.offsets_cube(2), 2, same=False)
+    check(oracle, coarse, vox, clouds.offsets_cube(3), 1, same=False)
+
+
+def test_corners_of_the_coordinate_range():
+    """Against the dictionary: the numpy builder's keys of neighbours outside the range meet others'."""
+    import FGMS.nn as fnn
+    ends = np.array([-(1 << 20), -(1 << 20) + 1, -1, 0, 1, (1 << 20) - 2, (1 << 20) - 1])
+    vox = np.stack(np.meshgrid(ends, ends, ends, indexing="ij"), -1).reshape(-1, 3).astype(np.int32)
+    offsets, c = clouds.offsets_cube(3), torch.from_numpy(vox).cuda()
+    for out, stride in ((vox, 1), (vox // 2, 2)):
+        imap, omap, knnz, _ = clouds.build_kernel_map_bruteforce(vox, out, offsets, stride)
+        kmap = fnn.KernelMap.from_coords(c, c if stride == 1 else torch.from_numpy(out).cuda(), offsets, stride)
+        assert np.array_equal(kmap.in_map.cpu().numpy(), imap) and np.array_equal(kmap.out_map.cpu().numpy(), omap)
+        assert np.array_equal(kmap.kernel_nnz.numpy(), knnz)
+
+
+def test_blocks_of_rows_past_a_thousand():
+    """More than 1024 counts to an offset: the lists' prefix sums go round again."""
+    import FGMS.nn as fnn
+    grid = np.stack(np.meshgrid(np.arange(700), np.arange(400), indexing="ij"), -1).reshape(-1, 2)
+    vox = np.concatenate([grid, (grid.sum(1) // 7 % 3)[:, None]], 1).astype(np.int32)
+    offsets = clouds.offsets_cube(3)
+    imap, omap, knnz, _ = clouds.build_kernel_map(vox, vox, offsets)
+    c = torch.from_numpy(vox).cuda()
+    kmap = fnn.KernelMap.from_coords(c, c, offsets)
+    assert np.array_equal(kmap.in_map.cpu().numpy(), imap) and np.array_equal(kmap.out_map.cpu().numpy(), omap)
+    assert np.array_equal(kmap.kernel_nnz.numpy(), knnz)
+
+
 def test_coordinate_out_of_range():
     import FGMS.nn as fnn
     v = torch.tensor([[0, 0, 0], [1 << 20, 0, 0]], dtype=torch.int32, device="cuda")
