@@ -511,7 +511,7 @@ Route route_of(const GmsArgs &a, const Plan *plan) {
   const bool dense = a.dense_k >= 0;
   if (g_policy == 1) return Route::kGeneric;
   const bool pair_view = !dense && pair_view_gms_supported(a, plan);
-  if (g_policy == 5 && pair_view) return Route::kPairView;
+  if (g_policy == 5 && pair_view && plan_pair_view(plan, a)) return Route::kPairView;
   // (16 -> 64 channels fill the output-stationary kernel's tiles: 150 k voxels 20 us, 39 us here; the others 1.1 .. 3 times
   // faster than on the vector ALUs from 2 k to 150 k voxels)
   if (!dense && (g_policy == 0 || g_policy == 4) && narrow_gms_supported(a, plan) &&
@@ -527,7 +527,7 @@ Route route_of(const GmsArgs &a, const Plan *plan) {
   // block's weights of one offset.  Measured (same clouds): fp32 a tie up to 128 channels,
   // 245 against 341 us at 256 -> 256 over 50 k voxels; fp16 14.2 against 18.3 us at 64
   // channels over 35 k voxels, a tie from 128 channels on (96.6 against 96.3 us at 256).
-  if (g_policy == 0 && pair_view && (a.dtype == FGMS_F32 || (a.transpose_w ? a.c_out : a.c_in) <= 64))
+  if (g_policy == 0 && pair_view && (a.dtype == FGMS_F32 || (a.transpose_w ? a.c_out : a.c_in) <= 64) && plan_pair_view(plan, a))
     return Route::kPairView;
   if (g_policy == 0 && wide_gms_supported(a)) return Route::kWide;
   return mfma_gms_supported(a) ? Route::kPairs : Route::kGeneric;

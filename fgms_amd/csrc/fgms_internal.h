@@ -129,7 +129,7 @@ struct Plan {
   int64_t pairs_counted;  // pairs the build saw (kpos[k_vol] - kpos[0]); n_pairs is the caller's bound
   std::vector<Plan *> groups;   // k_vol > 64: one plan per 64 offsets (owned)
   bool has_tables;        // k_vol <= 64: neighbour tables and masks exist (else the plan is the weight gradient's bands only)
-  const int32_t *kpos, *in_map, *out_map;    // the caller's lists (for the pair view, built on first use)
+  const int32_t *kpos, *in_map, *out_map;    // the caller's lists (for the fingerprint)
   hipStream_t pv_stream;        // the stream the pair view was built on
   hipEvent_t pv_ready;          // fires behind its last kernel (launches on other streams wait for it)
   hipStream_t create_stream;    // the stream the build was queued on
@@ -190,10 +190,10 @@ struct Plan {
   // of 64 (padding = -1), so that a 64-row block of pv_in / pv_out belongs to one offset,
   // bit k of pv_mask[b] says which.  The output-stationary kernel walks these "virtual
   // rows" like a plan whose rows have one neighbour each and adds its results with
-  // atomics.  nullptr: not built.
+  // atomics.  nullptr: not built yet (plan_pair_view).
   int32_t *pv_in, *pv_out;        // [pv_rows]
   unsigned long long *pv_mask;    // [pv_rows / 64]
-  int64_t pv_rows;                // a multiple of 256
+  int64_t pv_rows;                // a multiple of 256; 0: this map has none
   // The middle offset of an odd number of them has no pairs (the caller keeps it out of the lists): its lines
   // of the tables then hold the row order, through which every row is its own neighbour.  No mask names
   // the offset, so that only a launch that asks for it (GmsArgs::centre) sees them.
@@ -309,6 +309,7 @@ bool planned_gms_supported(const GmsArgs &a, const Plan *p);
 int launch_planned_gms(const GmsArgs &a, const Plan *p);
 // The same kernel over the plan's pair view (no wasted row slots, atomic adds).
 bool pair_view_gms_supported(const GmsArgs &a, const Plan *p);
+bool plan_pair_view(const Plan *p, const GmsArgs &a);      // builds it if need be (false: cannot be had now)
 int launch_pair_view_gms(const GmsArgs &a, const Plan *p);
 // Notes that a launch on `stream` reads the plan.
 inline void plan_touch(const Plan *p, hipStream_t stream) {

@@ -1792,7 +1792,8 @@ int launch_ragged_gms(const GmsArgs &a, const Plan *p) {
 }
 
 bool pair_view_gms_supported(const GmsArgs &a, const Plan *p) {
-  if (!p || !p->pv_in || a.dense_k >= 0 || a.k_vol != p->k_vol) return false;
+  if (!p || !p->pv_rows || a.dense_k >= 0 || a.k_vol != p->k_vol) return false;
+  if (!p->pv_in && is_capturing(a.stream)) return false;
   if (a.transpose_w ? (a.n_dst != p->n_in || a.n_src != p->n_out) : (a.n_dst != p->n_out || a.n_src != p->n_in))
     return false;
   if (reinterpret_cast<uintptr_t>(a.dst) % 16 || !rows_fit_buffer(a)) return false;
@@ -1800,7 +1801,7 @@ bool pair_view_gms_supported(const GmsArgs &a, const Plan *p) {
 }
 
 int launch_pair_view_gms(const GmsArgs &a, const Plan *p) {
-  if (!pair_view_gms_supported(a, p)) {
+  if (!pair_view_gms_supported(a, p) || !plan_pair_view(p, a)) {
     set_error("launch_pair_view_gms: unsupported shape or plan");
     return FGMS_E_INVALID;
   }

@@ -822,12 +822,54 @@ static bool plan_is_stale(const Plan *p) {
   return false;
 }
 
-static int fill_pair_view(const Plan *p, int64_t rows, hipStream_t s) {
+// The pair view of `p`, built by the first launch that is to walk it, from that call's own lists.
+static bool build_pair_view(Plan *p, const int32_t *kpos, const int32_t *in_map, const int32_t *out_map, hipStream_t s) {
+  std::lock_guard<std::mutex> lock(p->mutex);
+  if (p->pv_in) return true;
+  if (!p->pv_rows || is_capturing(s)) return false;
+  if (Plan *b = p->base) {                     // (a transposed view: the base's, the sides swapped)
+    if (!build_pair_view(b, kpos, out_map, in_map, s)) return false;
+    p->pv_stream = b->pv_stream; p->pv_ready = b->pv_ready;
+    p->pv_out = b->pv_in; p->pv_mask = b->pv_mask; p->pv_in = b->pv_out;
+    return true;
+  }
+  const int64_t rows = p->pv_rows;
+  int32_t *in = nullptr, *out = nullptr;
+  unsigned long long *mask = nullptr;
   FillBatch fills{};
-  fills.add(p->pv_in, (size_t)rows * sizeof(int32_t), -1);
-  fills.add(p->pv_out, (size_t)rows * sizeof(int32_t), -1);
-  fills.add(p->pv_mask, (size_t)(rows / 64) * sizeof(unsigned long long), 0);
-  return launch_fills(fills, s);
+  bool ok = pool_alloc((void **)&in, (size_t)rows * sizeof(int32_t), s) == FGMS_OK &&
+            pool_alloc((void **)&out, (size_t)rows * sizeof(int32_t), s) == FGMS_OK &&
+            pool_alloc((void **)&mask, (size_t)(rows / 64) * sizeof(unsigned long long), s) == FGMS_OK;
+  if (ok) {
+    fills.add(in, (size_t)rows * sizeof(int32_t), -1);
+    fills.add(out, (size_t)rows * sizeof(int32_t), -1);
+    fills.add(mask, (size_t)(rows / 64) * sizeof(unsigned long long), 0);
+    ok = launch_fills(fills, s) == FGMS_OK;
+  }
+  if (!ok) {
+    if (in) pool_free(in, s, false);
+    if (out) pool_free(out, s, false);
+    if (mask) pool_free(mask, s, false);
+    p->pv_rows = 0;
+    return false;
+  }
+  pair_view_kernel<<<(unsigned)((p->n_pairs + 255) / 256), 256, 0, s>>>(kpos, in_map, out_map, p->k_vol, (int)p->n_pairs, (long long)rows,
+                                                                       in, out, mask);
+  // launches on other streams wait for this event (launch_pair_view_gms, the destroy path)
+  if (hipGetLastError() != hipSuccess || hipEventCreateWithFlags(&p->pv_ready, hipEventDisableTiming) != hipSuccess ||
+      hipEventRecord(p->pv_ready, s) != hipSuccess) {
+    // without the event nothing else can be ordered behind the build: finish it here
+    (void)hipStreamSynchronize(s);
+    if (p->pv_ready) (void)hipEventDestroy(p->pv_ready);
+    p->pv_ready = nullptr;
+  }
+  p->pv_stream = s;
+  p->pv_out = out; p->pv_mask = mask; p->pv_in = in;
+  return true;
+}
+
+bool plan_pair_view(const Plan *p, const GmsArgs &a) {
+  return build_pair_view(const_cast<Plan *>(p), a.kpos, a.transpose_w ? a.smap : a.gmap, a.transpose_w ? a.gmap : a.smap, a.stream);
 }
 
 const Plan *plan_resolve(fgms_plan_t *plan, hipStream_t stream, int *rc) {
@@ -853,8 +895,7 @@ const Plan *plan_resolve(fgms_plan_t *plan, hipStream_t stream, int *rc) {
       p->tile_grid_out = b->tile_grid_in; p->tile_grid_in = b->tile_grid_out;
       p->stages_out = b->stages_in; p->stages_in = b->stages_out;
       p->fwd_ok = b->dgrad_ok; p->dgrad_ok = b->fwd_ok;
-      p->pv_in = b->pv_out; p->pv_out = b->pv_in; p->pv_mask = b->pv_mask; p->pv_rows = b->pv_rows;
-      p->pv_ready = b->pv_ready; p->pv_stream = b->pv_stream;
+      p->pv_rows = b->pv_rows;
       p->has_tables = b->has_tables;
       p->centre_line = b->centre_line;
       p->pairs_counted = b->pairs_counted;
@@ -890,46 +931,14 @@ const Plan *plan_resolve(fgms_plan_t *plan, hipStream_t stream, int *rc) {
       p->stages_in = h[5];
       p->pairs_counted = p->has_tables ? h[12] : p->n_pairs;
       // The pair view, for maps sparse enough that some layer would take it (fp32 layers prefer
-      // it from about 1 + 45 / channels row slots per pair on, never below 1.4, where the products are many): built now that
-      // the counts are known, so that dense maps pay nothing.
+      // it from about 1 + 45 / channels row slots per pair on, never below 1.4, where the products are many).  Its size is known now;
+      // it is built when a layer does take it (plan_pair_view): fp16 layers want twice as sparse a map, and over 100 k LiDAR
+      // voxels, 1.5 slots a pair, its two launches were 15 us that a network in fp16 never saw again.
       static const bool pair_view = !(getenv("FGMS_PAIR_VIEW") && atoi(getenv("FGMS_PAIR_VIEW")) == 0);
       const int most = p->stages_out > p->stages_in ? p->stages_out : p->stages_in;
       if (!p->invalid && pair_view && p->has_tables && p->pairs_counted > 0 &&
-          (kernel_policy() == 5 || (double)most * 64.0 >= 1.35 * (double)p->pairs_counted)) {
-        // (a caller that names no stream -- fgms_plan_usable, fgms_plan_stats -- must not put the
-        // view on the legacy null stream, which the streams torch makes do not wait for: the
-        // stream the plan itself was built on takes it)
-        hipStream_t s = stream ? stream : p->create_stream;
-        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-        const bool capturing = s && hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
-        const int64_t rows = (p->pairs_counted + 64 * (int64_t)p->k_vol + 255) / 256 * 256;
-        if (!capturing &&
-            pool_alloc((void **)&p->pv_in, (size_t)rows * sizeof(int32_t), s) == FGMS_OK &&
-            pool_alloc((void **)&p->pv_out, (size_t)rows * sizeof(int32_t), s) == FGMS_OK &&
-            pool_alloc((void **)&p->pv_mask, (size_t)(rows / 64) * sizeof(unsigned long long), s) == FGMS_OK &&
-            fill_pair_view(p, rows, s) == FGMS_OK) {
-          pair_view_kernel<<<(unsigned)((p->n_pairs + 255) / 256), 256, 0, s>>>(
-              p->kpos, p->in_map, p->out_map, p->k_vol, (int)p->n_pairs, (long long)rows, p->pv_in, p->pv_out,
-              p->pv_mask);
-          // launches on other streams wait for this event (launch_pair_view_gms, the destroy path)
-          if (hipGetLastError() != hipSuccess ||
-              hipEventCreateWithFlags(&p->pv_ready, hipEventDisableTiming) != hipSuccess ||
-              hipEventRecord(p->pv_ready, s) != hipSuccess) {
-            // without the event nothing else can be ordered behind the build: finish it here
-            (void)hipStreamSynchronize(s);
-            if (p->pv_ready) (void)hipEventDestroy(p->pv_ready);
-            p->pv_ready = nullptr;
-          }
-          p->pv_rows = rows;
-          p->pv_stream = s;
-        } else {
-          if (p->pv_in) pool_free(p->pv_in, s, false);
-          if (p->pv_out) pool_free(p->pv_out, s, false);
-          if (p->pv_mask) pool_free(p->pv_mask, s, false);
-          p->pv_in = p->pv_out = nullptr;
-          p->pv_mask = nullptr;
-        }
-      }
+          (kernel_policy() == 5 || (double)most * 64.0 >= 1.35 * (double)p->pairs_counted))
+        p->pv_rows = (p->pairs_counted + 64 * (int64_t)p->k_vol + 255) / 256 * 256;
       // (a plan over more than 64 offsets: its groups)
       for (Plan *g : p->groups) {
         int grc = FGMS_OK;
@@ -1064,7 +1073,7 @@ int fgms_plan_stats(const fgms_plan_t *plan, int64_t stats[4]) {
   stats[0] = p->groups.empty() ? p->pairs_counted : p->n_pairs;
   stats[1] = p->stages_out;
   stats[2] = p->stages_in;
-  stats[3] = p->pv_in ? p->pv_rows : 0;
+  stats[3] = p->pv_rows;
   return FGMS_OK;
 }
 

@@ -264,3 +264,52 @@ def test_backend_cache_drops_a_plan_whose_map_was_rewritten(capi, oracle):
         forward()
     G.assert_close(forward(), reference(), "fp16", "second map, after the stale plan was dropped")
     backend.fgms_plan_cache_clear()
+
+
+def test_pair_view_is_built_by_the_first_layer_that_walks_it(capi, oracle):
+    """A thinned cloud: an fp16 layer does without the view, a captured fp32 layer too while there is none; the first fp32 layer
+    outside a capture builds it, from a transposed plan on a stream of its own, and the plan itself walks the same one."""
+    vox = clouds.cloud_indoor(clouds.rng_for(2), target=60000)
+    vox = np.ascontiguousarray(vox[np.sort(np.random.default_rng(1).permutation(len(vox))[:20000])])
+    rng = np.random.default_rng(5)
+    L = clouds.submanifold_case(vox, 64, 64, np.float32, rng)
+    D = G.to_dev(L)
+    maps = (D["kpos"], D["imap"], D["omap"])
+    plan = capi.Plan(*maps, D["n_in"], D["n_out"])
+    view = plan.transposed()
+    assert plan.stats()["pair_view_rows"] == view.stats()["pair_view_rows"] > 0
+    swapped = (maps[0], maps[2], maps[1])
+    want = oracle.c_fwd(L["in_feats"], L["kernel"], L["knnz"], L["imap"], L["omap"], L["n_out"])
+    want_up = oracle.c_fwd(L["in_feats"], L["kernel"], L["knnz"], L["omap"], L["imap"], L["n_in"])
+    out = torch.empty_like(D["out_grad"])
+
+    def kernels(x, w, y, m, p):
+        capi.profile_reset(); capi.profile_enable(True)
+        capi.conv_fwd(x, w, y, *m, plan=p)
+        torch.cuda.synchronize()
+        capi.profile_enable(False)
+        return [n for n, _ in capi.profile_records()]
+
+    half = [t.half() for t in (D["in_feats"], D["kernel"], out)]
+    assert not any("pair view" in n for n in kernels(*half, maps, plan))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):                         # (workspaces for the capture, without a plan)
+        capi.conv_fwd(D["in_feats"], D["kernel"], out, *maps)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    captured = torch.empty_like(out)
+    with torch.cuda.graph(graph, stream=side, capture_error_mode="thread_local"):
+        capi.conv_fwd(D["in_feats"], D["kernel"], captured, *maps, plan=plan)
+    for _ in range(3):
+        captured.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        G.assert_close(captured.cpu().numpy(), want, "fp32", "captured")
+        with torch.cuda.stream(side):
+            assert any("pair view" in n for n in kernels(D["in_feats"], D["kernel"], out, swapped, view))
+        G.assert_close(out.cpu().numpy(), want_up, "fp32", "through the transposed plan")
+        assert any("pair view" in n for n in kernels(D["in_feats"], D["kernel"], out, maps, plan))
+        G.assert_close(out.cpu().numpy(), want, "fp32", "through the plan")
+    view.close()
+    plan.close()
