@@ -20,6 +20,8 @@
 
 #include <stdlib.h>
 
+#include <algorithm>
+
 #include <map>
 #include <mutex>
 
@@ -289,7 +291,9 @@ void tile_blocks(const WgradArgs &a, bool shares_grid, int *bi, int *bj) {
 // Slices per offset: from the plan's row bands when it has them, `stride` bands to
 // a slice so that about `want_wgs` workgroups result; else equal pair counts,
 // enough to fill the chip a few times with at least ~16 stages of pairs per slice
-// on average.  A multiple of 8 (one per XCD).
+// on average, or eight of 64 pairs while there is a workgroup to a CU at most (a workgroup's chain of stages is then what the launch
+// takes, beyond it the atomics of the flushes: the transposed layer 128 -> 64 over a stride-2 map, backward launch, 192 / 256 / 384
+// workgroups over 200 k pairs 28.5 / 25.9 / 31.1 us, 64 / 128 over 60 k 21.0 / 15.0).  A multiple of 8 (one per XCD).
 SliceMap choose_slices(const WgradArgs &a, int ty, int stage_pairs, int64_t want_wgs) {
   SliceMap m{};
   if (a.plan && a.plan->bands_ok && a.plan->band_start && a.plan->k_vol == a.k_vol &&
@@ -311,7 +315,8 @@ SliceMap choose_slices(const WgradArgs &a, int ty, int stage_pairs, int64_t want
     return m;
   }
   int64_t slices = want_wgs / ((int64_t)a.k_vol * ty);
-  const int64_t by_work = a.n_pairs / ((int64_t)a.k_vol * 16 * stage_pairs);
+  int64_t by_work = a.n_pairs / ((int64_t)a.k_vol * 16 * stage_pairs);
+  if (stage_pairs == 64) by_work = std::max(by_work, std::min(a.n_pairs / ((int64_t)a.k_vol * 8 * stage_pairs), num_cus() / ((int64_t)a.k_vol * ty)));
   if (slices > by_work) slices = by_work;
   slices = (slices + 7) / 8 * 8;
   m.slices = (int)(slices < 8 ? 8 : slices);
@@ -486,7 +491,7 @@ int wgrad_geometry(const WgradArgs &a, WgradGeometry *g, bool shares_grid) {
   const size_t esz = f16 ? 2 : 4;
   int bi, bj;
   tile_blocks(a, shares_grid, &bi, &bj);
-  const int pad = f16 ? WT<__half>::pad : WT<float>::pad;
+  const int pad = f16 ? 0 : WT<float>::pad;
   *g = WgradGeometry{};
   g->bi = bi;
   g->bj = bj;

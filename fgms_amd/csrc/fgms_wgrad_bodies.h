@@ -38,15 +38,20 @@ __device__ __forceinline__ half8 tr_frag(const __half *tile, int ld, int p0, int
   return __builtin_bit_cast(half8, v);
 }
 
-// The same from a tile without row padding (rows of exactly `ld` = 32, 64 or 96 halfs).  One
-// transposing read touches rows p .. p + 3 and p + 8 .. p + 11, 64 bytes of each; with 128-byte
+// The same from a tile without row padding (rows of exactly `ld` = 32, 64, 96 or 128 halfs; p0 a multiple of 4).  One
+// transposing read touches rows p .. p + 3 and p + 8 .. p + 11, 64 bytes of each.  With 128-byte
 // rows, rows p and p + 2 would meet in the same banks, so the writer exchanges the two 64-byte
-// halves of every row whose (row >> 1) is odd (wave tile below) and the read does the same.
+// halves of every row whose (row >> 1) is odd, with 256-byte rows all four would, and it exchanges the 64-byte quarters by
+// row & 3 (dense_chunk); the read does the same.
+template <int LD>
+__device__ __forceinline__ int dense_chunk(int row, int chunk) {      // where a 16-byte chunk of a row goes
+  return chunk ^ (LD == 64 ? ((row >> 1) & 1) * 4 : LD == 128 ? (row & 3) * 4 : 0);
+}
 template <int LD>
 __device__ __forceinline__ half8 tr_frag_dense(const __half *tile, int p0, int c0, int lane) {
-  static_assert(LD == 32 || LD == 64 || LD == 96, "dense tile: 32, 64 or 96 channels a row");
+  static_assert(LD == 32 || LD == 64 || LD == 96 || LD == 128, "dense tile: 32, 64, 96 or 128 channels a row");
   const int b = lane >> 4, i = lane & 15, h = lane >> 5;
-  const int sw = LD == 64 ? ((lane >> 3) & 1) * 32 : 0;
+  const int sw = LD == 64 ? ((lane >> 3) & 1) * 32 : LD == 128 ? (i >> 2) * 32 : 0;
   const __half *base = tile + (size_t)(p0 + h * 8 + (i >> 2)) * LD + (c0 ^ sw) + (b & 1) * 16 + (i & 3) * 4;
   typedef __attribute__((address_space(3))) short4v lds_v4;
   const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4 *)(base));
@@ -313,7 +318,7 @@ __device__ __forceinline__ void wgrad_wave_body(
         store_split_chunk<P>(xs, SP * LDIh, LDIh, e / NCI, e % NCI, xr[i],
                              st * SP + e / NCI < count && (!RAGGED || ci0 + e % NCI * E < c_in), lost);
       else if constexpr (kBufW)
-        *reinterpret_cast<int4v *>(x + x_row(i) * LDI + ((x_chunk(i) ^ (CI == 64 ? ((x_row(i) >> 1) & 1) * 4 : 0)) * E)) = xr[i];
+        *reinterpret_cast<int4v *>(x + x_row(i) * LDI + dense_chunk<CI>(x_row(i), x_chunk(i)) * E) = xr[i];
       else
         *reinterpret_cast<int4v *>(x + (e / NCI) * LDI + (e % NCI) * E) =
             st * SP + e / NCI < count && (!RAGGED || ci0 + e % NCI * E < c_in) ? xr[i] : int4v{0, 0, 0, 0};
@@ -325,7 +330,7 @@ __device__ __forceinline__ void wgrad_wave_body(
         store_split_chunk<P>(gs, SP * LDOh, LDOh, e / NCO, e % NCO, gr[i],
                              st * SP + e / NCO < count && (!RAGGED || co0 + e % NCO * E < c_out), lost);
       else if constexpr (kBufW)
-        *reinterpret_cast<int4v *>(g + g_row(i) * LDO + ((g_chunk(i) ^ (CO == 64 ? ((g_row(i) >> 1) & 1) * 4 : 0)) * E)) = gr[i];
+        *reinterpret_cast<int4v *>(g + g_row(i) * LDO + dense_chunk<CO>(g_row(i), g_chunk(i)) * E) = gr[i];
       else
         *reinterpret_cast<int4v *>(g + (e / NCO) * LDO + (e % NCO) * E) =
             st * SP + e / NCO < count && (!RAGGED || co0 + e % NCO * E < c_out) ? gr[i] : int4v{0, 0, 0, 0};
@@ -502,7 +507,12 @@ __device__ __forceinline__ void wgrad_wg_body(
   using G = WaveGrid<BI, BJ>;
   constexpr int E = W::E, SP = W::stage_pairs, KP = W::step_pairs;
   constexpr int CI = BI * 32, CO = BJ * 32;
-  constexpr int LDI = CI + W::pad, LDO = CO + W::pad;
+  // (fp16: rows without padding, see tr_frag_dense.  Padded by 32 bytes the reads met in the banks, 0.87 conflict cycles to an LDS
+  // instruction over 128 x 128, and the stages of 64 x 128 left room for two workgroups on a CU instead of three.  Backward launch,
+  // padded / dense: 128 -> 64 over 60 k indoor voxels 69.8 / 61.9 us, 64 -> 128 over 100 k 92 / 89, stride 2 transposed 128 -> 64
+  // over 200 k 31.8 / 27.8, 128 -> 128 over 120 k LiDAR ones 170 / 158 .. 166.)
+  constexpr bool kDense = sizeof(T) == 2;
+  constexpr int LDI = CI + (kDense ? 0 : W::pad), LDO = CO + (kDense ? 0 : W::pad);
   constexpr int NCI = CI / E, NCO = CO / E;   // 16-byte chunks per staged row
   constexpr int NX = BI, NG = BJ;             // chunks per thread and stage
   extern __shared__ int4v lds[];
@@ -575,7 +585,7 @@ __device__ __forceinline__ void wgrad_wg_body(
         __half *xh = stage0h + buf * kBufHalfs;
         store_split_chunk<2>(xh, SP * LDIh, LDIh, e / NCI, e % NCI, xr[i], st * SP + e / NCI < count, lost);
       } else {
-        *reinterpret_cast<int4v *>(stage0 + buf * kBufElems + (e / NCI) * LDI + (e % NCI) * E) =
+        *reinterpret_cast<int4v *>(stage0 + buf * kBufElems + (e / NCI) * LDI + (kDense ? dense_chunk<CI>(e / NCI, e % NCI) : e % NCI) * E) =
             st * SP + e / NCI < count ? xr[i] : int4v{0, 0, 0, 0};
       }
     }
@@ -586,7 +596,7 @@ __device__ __forceinline__ void wgrad_wg_body(
         __half *gh = stage0h + buf * kBufHalfs + SP * 2 * LDIh;
         store_split_chunk<2>(gh, SP * LDOh, LDOh, e / NCO, e % NCO, gr[i], st * SP + e / NCO < count, lost);
       } else {
-        *reinterpret_cast<int4v *>(stage0 + buf * kBufElems + SP * LDI + (e / NCO) * LDO + (e % NCO) * E) =
+        *reinterpret_cast<int4v *>(stage0 + buf * kBufElems + SP * LDI + (e / NCO) * LDO + (kDense ? dense_chunk<CO>(e / NCO, e % NCO) : e % NCO) * E) =
             st * SP + e / NCO < count ? gr[i] : int4v{0, 0, 0, 0};
       }
     }
@@ -626,9 +636,9 @@ __device__ __forceinline__ void wgrad_wg_body(
       if constexpr (sizeof(T) == 2) {
         half8 a[G::TI], b[G::TJ];
 #pragma unroll
-        for (int ti = 0; ti < G::TI; ++ti) a[ti] = tr_frag(x, LDI, p0, (wi * G::TI + ti) * 32, lane);
+        for (int ti = 0; ti < G::TI; ++ti) a[ti] = tr_frag_dense<CI>(x, p0, (wi * G::TI + ti) * 32, lane);
 #pragma unroll
-        for (int tj = 0; tj < G::TJ; ++tj) b[tj] = tr_frag(g, LDO, p0, (wj * G::TJ + tj) * 32, lane);
+        for (int tj = 0; tj < G::TJ; ++tj) b[tj] = tr_frag_dense<CO>(g, p0, (wj * G::TJ + tj) * 32, lane);
 #pragma unroll
         for (int ti = 0; ti < G::TI; ++ti)
 #pragma unroll

@@ -53,3 +53,28 @@ def test_either_side_of_the_size(n, by_xcd):
     names = [r[0] for r in capi.profile_records()]
     capi.profile_reset()
     assert ("bwd_fused_kernel(by XCD)" in names) == by_xcd and any(q.startswith("bwd_fused_kernel") for q in names), names
+
+
+@pytest.mark.parametrize("shape", [(32, 128), (128, 32), (64, 128), (128, 64), (128, 128), (256, 128)], ids=lambda s: "%dx%d" % s)
+def test_tiles_of_128_channels_are_exact(shape):
+    """Whole numbers small enough for every sum to be one: whatever a stage's rows meet in the wrong place shows.  Lists that
+    end inside, at and behind a stage of 64 pairs, both with the input gradient and alone, forward and swapped lists (no bands)."""
+    from fgms_amd import capi
+    capi.set_kernel_policy(0)
+    sizes = [1, 63, 64, 65, 127, 129, 700, 0, 1500]
+    n, rng = 1600, np.random.default_rng(4)
+    rows = [np.sort(rng.permutation(n)[:s]) for s in sizes]
+    omap = np.concatenate(rows).astype(np.int32)
+    imap = np.concatenate([rng.permutation(n)[:s] for s in sizes]).astype(np.int32)
+    kpos = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    x, g = (torch.from_numpy(rng.integers(-1, 2, (n, c)).astype(np.float16)).cuda() for c in shape)
+    w = torch.from_numpy(rng.integers(-1, 2, (len(sizes), *shape)).astype(np.float16)).cuda()
+    for a, b in ((imap, omap), (omap, imap)):
+        maps = tuple(torch.from_numpy(t).cuda() for t in (kpos, a, b))
+        want = exact(x.float(), w.float(), g.float(), kpos.tolist(), maps[1].long(), maps[2].long())[2]
+        assert want.abs().max() < 2048
+        plan = capi.Plan(*maps, n, n)
+        gi, gw, alone = torch.empty_like(x), torch.full_like(w, float("nan")), torch.zeros_like(w)
+        capi.conv_bwd(g, x, w, gi, gw, *maps, plan=plan)
+        capi.wgrad(x, g, alone, *maps, plan=plan)
+        assert torch.equal(gw.double(), want) and torch.equal(alone.double(), want)
