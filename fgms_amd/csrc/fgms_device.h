@@ -14,14 +14,14 @@ namespace fgms {
 // reference does this with a bisection over the caller's 256-padded qkpos
 // (backend/utils.cuh:6-27, backend/spconv.cuh:484-485); walking kpos instead
 // makes the result independent of the padding quantum and skips empty offsets
-// the same way.  t is wave-uniform, so the walk runs on the scalar unit.
+// the same way.  t is wave-uniform, so the walk runs on the scalar unit.  (skip: an offset without tiles.)
 __device__ __forceinline__ bool locate_tile(const int32_t *__restrict__ kpos, int k_vol,
-                                            int rows, int t, int &k, int &first, int &count) {
+                                            int rows, int t, int &k, int &first, int &count, int skip = -1) {
   int lo = kpos[0];
   for (int i = 0; i < k_vol; ++i) {
     int hi = kpos[i + 1];
     int n = hi - lo;
-    int nt = (n + rows - 1) / rows;
+    int nt = i == skip ? 0 : (n + rows - 1) / rows;
     if (t < nt) {
       k = i;
       first = lo + t * rows;

@@ -78,8 +78,19 @@ struct GmsArgs {
   bool overwrite;          // dst = the sums instead of dst += (rows without a pair become zero)
   double beside_us;        // input gradient of fp32 tensors: what the output-stationary grid hides of the weight gradient's time
   const void *prepacked;   // output-stationary kernel only: the weights are already re-laid here
+  int first_offset;        // pair-stationary kernels: k + 1: offset k meets every destination row exactly once (see Plan::full_out)
   SideJob side;            // rides along with the launch (not the shape-agnostic kernel's)
 };
+// What a launch of a pair-stationary kernel walks: all pairs, the pairs of all offsets but one, or one offset's list (or the identity
+// map), whose rows nothing else of the launch meets.
+enum { kWalkAll = 0, kWalkRest = 1, kWalkOwn = 2 };
+// How it leaves its tiles.
+enum { kTileAdd = 0, kTileAtomic = 1, kTileStore = 2 };
+// The launch's offset as the kernels take it: kWalkRest, the one left out; kWalkOwn, twice its own, and one if it is to store and not to
+// add.  (One argument, and not one more than without the others: they cost a launch of 25 us 0.3.)
+inline int walk_offset(const GmsArgs &a, bool first) {
+  return first ? 2 * (a.first_offset - 1) + 1 : a.dense_k >= 0 ? 2 * a.dense_k + (a.overwrite ? 1 : 0) : a.first_offset - 1;
+}
 
 struct WgradArgs {
   const void *in;     // [n_in, c_in]
@@ -111,6 +122,7 @@ struct WgradArgs {
 constexpr int kPlanFlags = 32;      // ints the plan build reports back (see fgms_plan.hip)
 constexpr int kFlagStale = 13;      // flags[13]: a later check found another fingerprint (fgms_plan_check)
 constexpr int kFlagCentre = 14;     // flags[14]: see Plan::centre_line
+constexpr int kFlagFull = 15;       // flags[15]: see Plan::full_out (+ 1, that of the input side << 8)
 constexpr int kFlagPrint = 16;      // flags[16 .. 31]: fingerprint of the pair lists (kPrintParts 64-bit words)
 constexpr int kPrintParts = 8;      // ... each over an eighth of the sample, so that as many workgroups take it
 
@@ -198,6 +210,8 @@ struct Plan {
   // of the tables then hold the row order, through which every row is its own neighbour.  No mask names
   // the offset, so that only a launch that asks for it (GmsArgs::centre) sees them.
   bool centre_line;
+  // An offset that meets every output (input) row exactly once, as a submanifold map's middle one does; -1: none.
+  int full_out, full_in;
   bool fwd_ok;        // no offset maps two pairs onto one output row
   bool dgrad_ok;      // no offset maps two pairs from one input row
 };

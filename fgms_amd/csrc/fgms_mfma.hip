@@ -428,12 +428,13 @@ __device__ __forceinline__ void gather_commit_parts_buf(int4v *__restrict__ a_ld
 // Pair-stationary kernel.
 // SPLIT: fp32 tensors whose caller allows tf32 precision, products in split bf16 (see
 // mma_slab_parts); `packed` from pack_weights_parts_kernel.
-template <typename T, int NT, int S, bool SPLIT>
+// WALK: see kWalkAll.
+template <typename T, int NT, int S, bool SPLIT, int WALK>
 __global__ __launch_bounds__(kThreads) void gms_pairs_kernel(
     const T *__restrict__ src, const T *__restrict__ packed, T *__restrict__ dst,
     const int32_t *__restrict__ kpos, const int32_t *__restrict__ gmap,
     const int32_t *__restrict__ smap, int k_vol, int c_src, int c_dst, int tiles_per_wg,
-    int dense_k, int dense_rows, SideJob side) {
+    int offset, int dense_rows, SideJob side) {
   // the leading workgroups of the grid run the side job, if there is one
   int block_x = blockIdx.x;
   if (side.blocks) {
@@ -461,12 +462,14 @@ __global__ __launch_bounds__(kThreads) void gms_pairs_kernel(
   const int t_begin = block_x * tiles_per_wg;
   for (int t = t_begin; t < t_begin + tiles_per_wg; ++t) {
     int k, first, count;
-    if (dense_k >= 0) {
-      k = dense_k;
+    if constexpr (WALK == kWalkOwn) {
+      k = offset >> 1;
+      const int rows = gmap ? min(dense_rows, kpos[k + 1] - kpos[k]) : dense_rows;
       first = t * kTileRows;
-      if (first >= dense_rows) break;
-      count = min(kTileRows, dense_rows - first);
-    } else if (!locate_tile(kpos, k_vol, kTileRows, t, k, first, count)) {
+      if (first >= rows) break;
+      count = min(kTileRows, rows - first);
+      if (gmap) first += kpos[k];
+    } else if (!locate_tile(kpos, k_vol, kTileRows, t, k, first, count, WALK == kWalkRest ? offset : -1)) {
       break;
     }
     if (k != cur_k) {  // uniform over the workgroup
@@ -508,7 +511,9 @@ __global__ __launch_bounds__(kThreads) void gms_pairs_kernel(
       else mma_slab<T, NT, S>(acc, a_lds, w_lds, slab, lane);
       wave_lds_fence();
     }
-    write_tile<T, NT, true>(acc, dst, sidx, c_dst, nt0 * 32, lane);
+    if constexpr (WALK != kWalkOwn) write_tile<T, NT, kTileAtomic>(acc, dst, sidx, c_dst, nt0 * 32, lane);
+    else if (offset & 1) write_tile<T, NT, kTileStore>(acc, dst, sidx, c_dst, nt0 * 32, lane);
+    else write_tile<T, NT, kTileAdd>(acc, dst, sidx, c_dst, nt0 * 32, lane);
     wave_lds_fence();
   }
 }
@@ -1190,22 +1195,30 @@ int launch_pairs(const GmsArgs &a, const Shape &s) {
     int rc = pack_weights<T>(a, S, &packed);
     if (rc != FGMS_OK) return rc;
   }
-  const bool dense = a.dense_k >= 0;
-  const int64_t tiles = dense ? (a.n_dense + kTileRows - 1) / kTileRows
-                              : (a.n_pairs + kTileRows - 1) / kTileRows + a.k_vol;
-  // a few workgroups per CU, each walking a contiguous run of tiles
-  const int64_t want_wgs = (int64_t)num_cus() * 8;
-  const int tiles_per_wg = (int)((tiles + want_wgs - 1) / want_wgs);
-  const unsigned gx = (unsigned)((tiles + tiles_per_wg - 1) / tiles_per_wg);
-  auto kern = split ? gms_pairs_kernel<T, NT, S, kCanSplit> : gms_pairs_kernel<T, NT, S, false>;
-  { const int rc_lds = allow_dynamic_lds(reinterpret_cast<const void *>(kern), (size_t)s.lds_bytes); if (rc_lds != FGMS_OK) return rc_lds; }
-  {
+  // (a first launch for the offset that meets every row once, if there is one, then one for the other pairs)
+  SideJob side = a.side;
+  for (int part = a.first_offset ? 0 : 1; part < 2; ++part) {
+    const bool dense = part == 0 || a.dense_k >= 0;
+    const int64_t rows = part == 0 ? a.n_dst : dense ? a.n_dense : a.n_pairs - (a.first_offset ? a.n_dst : 0);
+    if (rows <= 0 && part == 1 && a.first_offset) continue;
+    constexpr int kRest = sizeof(T) == 2 ? kWalkRest : kWalkAll;      // (first offsets: fp16)
+    auto kern = dense            ? (split ? gms_pairs_kernel<T, NT, S, kCanSplit, kWalkOwn> : gms_pairs_kernel<T, NT, S, false, kWalkOwn>)
+                : a.first_offset ? gms_pairs_kernel<T, NT, S, false, kRest>
+                : split          ? gms_pairs_kernel<T, NT, S, kCanSplit, kWalkAll>
+                                 : gms_pairs_kernel<T, NT, S, false, kWalkAll>;
+    { const int rc_lds = allow_dynamic_lds(reinterpret_cast<const void *>(kern), (size_t)s.lds_bytes); if (rc_lds != FGMS_OK) return rc_lds; }
+    const int64_t tiles = (rows + kTileRows - 1) / kTileRows + (dense ? 0 : a.k_vol);
+    // a few workgroups per CU, each walking a contiguous run of tiles
+    const int64_t want_wgs = (int64_t)num_cus() * 8;
+    const int tiles_per_wg = (int)((tiles + want_wgs - 1) / want_wgs);
+    const unsigned gx = (unsigned)((tiles + tiles_per_wg - 1) / tiles_per_wg);
     ProfileScope prof(split ? (a.transpose_w ? "gms_pairs_kernel(dgrad, bf16x3)" : "gms_pairs_kernel(fwd, bf16x3)")
                             : (a.transpose_w ? "gms_pairs_kernel(dgrad)" : "gms_pairs_kernel(fwd)"),
                       a.stream);
-    kern<<<dim3(gx + (unsigned)a.side.blocks, (unsigned)(s.c_dst / (32 * NT))), kThreads, s.lds_bytes, a.stream>>>(
+    kern<<<dim3(gx + (unsigned)side.blocks, (unsigned)(s.c_dst / (32 * NT))), kThreads, s.lds_bytes, a.stream>>>(
         (const T *)a.src, packed, (T *)a.dst, a.kpos, a.gmap, a.smap, a.k_vol, s.c_src, s.c_dst,
-        tiles_per_wg, a.dense_k, (int)a.n_dense, a.side);
+        tiles_per_wg, walk_offset(a, part == 0), (int)rows, side);
+    side = SideJob{};
   }
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;

@@ -898,6 +898,7 @@ const Plan *plan_resolve(fgms_plan_t *plan, hipStream_t stream, int *rc) {
       p->pv_rows = b->pv_rows;
       p->has_tables = b->has_tables;
       p->centre_line = b->centre_line;
+      p->full_out = b->full_in; p->full_in = b->full_out;
       p->pairs_counted = b->pairs_counted;
       p->ordered = false;
       // (the weight gradient's row bands follow the base's output rows: not valid for the swapped lists)
@@ -927,6 +928,8 @@ const Plan *plan_resolve(fgms_plan_t *plan, hipStream_t stream, int *rc) {
       p->ordered = !h[0] && !h[3];
       p->bands_ok = p->has_bands && p->ordered;
       p->centre_line = p->has_tables && h[kFlagCentre];
+      p->full_out = p->fwd_ok ? (h[kFlagFull] & 255) - 1 : -1;
+      p->full_in = p->dgrad_ok ? (h[kFlagFull] >> 8) - 1 : -1;
       p->stages_out = h[4];
       p->stages_in = h[5];
       p->pairs_counted = p->has_tables ? h[12] : p->n_pairs;

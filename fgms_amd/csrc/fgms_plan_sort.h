@@ -264,7 +264,15 @@ __device__ __forceinline__ void sort_window_body(const SortArgs &a, int side, in
   bitonic_window(key, buf, base, lane, flip);
   int bits = 0, row_bits = 0;
   const int centre = empty_centre(a.kpos, a.k_vol);
-  if (window == 0 && side == 0 && threadIdx.x == 0) a.flags[kFlagCentre] = centre >= 0;
+  if (window == 0 && side == 0 && wave == 0) {
+    // (as many pairs as rows; that they are of different rows is for the reader of the flags to ask)
+    const int size = lane < a.k_vol ? a.kpos[lane + 1] - a.kpos[lane] : -1;
+    const unsigned long long out = __ballot(size == a.side[0].n), in = __ballot(size == (a.side[1].n > 0 ? a.side[1].n : a.side[0].n));
+    if (lane == 0) {
+      a.flags[kFlagCentre] = centre >= 0;
+      a.flags[kFlagFull] = (out ? __builtin_ctzll(out) + 1 : 0) | (in ? __builtin_ctzll(in) + 1 : 0) << 8;
+    }
+  }
 #pragma unroll
   for (int r = 0; r < 2; ++r) {
     const int p = p0 + base + r * 64 + lane;

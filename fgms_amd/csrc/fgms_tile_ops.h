@@ -81,8 +81,9 @@ __device__ __forceinline__ void zero_rows(T *__restrict__ dst, const int *__rest
 // Writes a wave's accumulators.  Accumulator register r of lane l holds row
 // (r / 4) * 8 + (l / 32) * 4 + r % 4 and column l % 32 of its 32x32 tile.  For
 // fp16 two lanes swap one value each so that every lane owns two neighbouring
-// columns of one row and can issue a packed 4-byte update.
-template <typename T, int NT, bool ATOMIC, bool RAGGED = false, int MT>
+// columns of one row and can issue a packed 4-byte update.  HOW: kTileAtomic, kTileAdd where the caller owns the rows, or
+// kTileStore where nothing is in them yet.
+template <typename T, int NT, int HOW, bool RAGGED = false, int MT>
 __device__ __forceinline__ void write_tile(const float16v (&acc)[MT][NT], T *__restrict__ dst,
                                            const int *__restrict__ rows, int c_dst, int cd0,
                                            int lane) {
@@ -98,7 +99,8 @@ __device__ __forceinline__ void write_tile(const float16v (&acc)[MT][NT], T *__r
           const int row = rows[mt * 32 + (r / 4) * 8 + h * 4 + (r % 4)];
           if (row >= 0 && column) {
             float *p = reinterpret_cast<float *>(dst) + (size_t)row * c_dst + cd0 + nt * 32 + col;
-            if constexpr (ATOMIC) atomic_add(p, acc[mt][nt][r]);
+            if constexpr (HOW == kTileAtomic) atomic_add(p, acc[mt][nt][r]);
+            else if constexpr (HOW == kTileStore) *p = acc[mt][nt][r];
             else *p += acc[mt][nt][r];
           }
         }
@@ -113,8 +115,10 @@ __device__ __forceinline__ void write_tile(const float16v (&acc)[MT][NT], T *__r
           const int row = rows[mt * 32 + (r / 4) * 8 + h * 4 + (r % 4)];
           if (row >= 0 && column) {
             __half *p = reinterpret_cast<__half *>(dst) + (size_t)row * c_dst + cd0 + nt * 32 + (col & ~1);
-            if constexpr (ATOMIC) {
+            if constexpr (HOW == kTileAtomic) {
               atomic_add_pk(p, lo, hi);
+            } else if constexpr (HOW == kTileStore) {
+              *reinterpret_cast<__half2 *>(p) = __floats2half2_rn(lo, hi);
             } else {
               __half2 *q = reinterpret_cast<__half2 *>(p);
               const float2 old = __half22float2(*q);
@@ -204,7 +208,7 @@ __device__ __forceinline__ void add_rows_lds(const float16v (&acc)[MT][NT], T *_
   constexpr int FIT = (WR * 2 * S * 16) / (COLS * 4);
   constexpr int R = FIT >= 32 ? 32 : FIT >= 16 ? 16 : FIT >= 8 ? 8 : 0;
   if constexpr (R < 8) {
-    if constexpr (ATOMIC) write_tile<T, NT, true, RAGGED>(acc, dst, rows, c_dst, cd0, lane);
+    if constexpr (ATOMIC) write_tile<T, NT, kTileAtomic, RAGGED>(acc, dst, rows, c_dst, cd0, lane);
     else {
       if constexpr (OVERWRITE) {
         zero_rows<T, NT, WR, RAGGED>(dst, rows, c_dst, cd0, lane);

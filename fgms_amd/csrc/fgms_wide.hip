@@ -26,11 +26,13 @@ constexpr int kWideCols = 256;       // destination channels per workgroup
 constexpr int kWideThreads = 1024;   // 16 waves
 constexpr int kSlabChunks = kWideRows * 8;   // 16-byte chunks of a slab of rows, and of a slab of weights
 
+// WALK: see kWalkAll.
+template <int WALK>
 __global__ __launch_bounds__(kWideThreads) void gms_wide_kernel(
     const __half *__restrict__ src, const int4v *__restrict__ packed, __half *__restrict__ dst,
     const int32_t *__restrict__ kpos, const int32_t *__restrict__ gmap,
     const int32_t *__restrict__ smap, int k_vol, int c_src, int c_dst, int tiles_per_wg,
-    int dense_k, int dense_rows, SideJob side) {
+    int offset, int dense_rows, SideJob side) {
   // the leading workgroups of the grid run the side job, if there is one
   int block_x = blockIdx.x;
   if (side.blocks) {
@@ -56,13 +58,15 @@ __global__ __launch_bounds__(kWideThreads) void gms_wide_kernel(
   const size_t packed_per_k = (size_t)c_src * c_dst / 8;   // chunks
 
   auto tile_at = [&](int t, int &k, int &first, int &count) {
-    if (dense_k >= 0) {
-      k = dense_k;
+    if constexpr (WALK == kWalkOwn) {
+      k = offset >> 1;
+      const int rows = gmap ? min(dense_rows, kpos[k + 1] - kpos[k]) : dense_rows;
       first = t * kWideRows;
-      count = min(kWideRows, dense_rows - first);
-      return first < dense_rows;
+      count = min(kWideRows, rows - first);
+      if (gmap) first += kpos[k];
+      return t * kWideRows < rows;
     }
-    return locate_tile(kpos, k_vol, kWideRows, t, k, first, count);
+    return locate_tile(kpos, k_vol, kWideRows, t, k, first, count, WALK == kWalkRest ? offset : -1);
   };
   // the indices of a tile's pairs -> LDS (buffer `par`)
   auto load_indices = [&](int par, int first, int count) {
@@ -144,7 +148,10 @@ __global__ __launch_bounds__(kWideThreads) void gms_wide_kernel(
     }
     if (has_next) commit(buf ^ 1);
     if (last_slab) {
-      write_tile<__half, 2, true>(acc, dst, sidx + par * kWideRows + rg * 64, c_dst, nt0 * 32 + cg * 64, lane);
+      const int *rows = sidx + par * kWideRows + rg * 64;
+      if constexpr (WALK != kWalkOwn) write_tile<__half, 2, kTileAtomic>(acc, dst, rows, c_dst, nt0 * 32 + cg * 64, lane);
+      else if (offset & 1) write_tile<__half, 2, kTileStore>(acc, dst, rows, c_dst, nt0 * 32 + cg * 64, lane);
+      else write_tile<__half, 2, kTileAdd>(acc, dst, rows, c_dst, nt0 * 32 + cg * 64, lane);
       clear();
     }
     if (!has_next) break;
@@ -186,23 +193,27 @@ int launch_wide_gms(const GmsArgs &a) {
     int rc = pack_weights_any(a, 4, &packed);
     if (rc != FGMS_OK) return rc;
   }
-  const bool dense = a.dense_k >= 0;
-  const int64_t tiles = dense ? (a.n_dense + kWideRows - 1) / kWideRows
-                              : (a.n_pairs + kWideRows - 1) / kWideRows + a.k_vol;
-  if (tiles <= 0) return FGMS_OK;
-  // one workgroup per CU at a time: each takes a contiguous run of tiles (mostly one offset,
-  // whose weights then stay in the L2 between its tiles)
-  const int64_t want_wgs = (int64_t)num_cus() / (c_dst / kWideCols > 1 ? c_dst / kWideCols : 1);
-  const int tiles_per_wg = (int)((tiles + want_wgs - 1) / (want_wgs > 0 ? want_wgs : 1));
-  const unsigned gx = (unsigned)((tiles + tiles_per_wg - 1) / tiles_per_wg);
-  const size_t lds_bytes = 4 * (size_t)kSlabChunks * 16 + 4 * kWideRows * sizeof(int);
-  const int rc_lds = allow_dynamic_lds(reinterpret_cast<const void *>(gms_wide_kernel), lds_bytes);
-  if (rc_lds != FGMS_OK) return rc_lds;
-  {
+  // (a first launch for the offset that meets every row once, if there is one, then one for the other pairs)
+  SideJob side = a.side;
+  for (int part = a.first_offset ? 0 : 1; part < 2; ++part) {
+    const bool dense = part == 0 || a.dense_k >= 0;
+    const int64_t rows = part == 0 ? a.n_dst : dense ? a.n_dense : a.n_pairs - (a.first_offset ? a.n_dst : 0);
+    if (rows <= 0) continue;
+    const int64_t tiles = (rows + kWideRows - 1) / kWideRows + (dense ? 0 : a.k_vol);
+    // one workgroup per CU at a time: each takes a contiguous run of tiles (mostly one offset,
+    // whose weights then stay in the L2 between its tiles)
+    const int64_t want_wgs = (int64_t)num_cus() / (c_dst / kWideCols > 1 ? c_dst / kWideCols : 1);
+    const int tiles_per_wg = (int)((tiles + want_wgs - 1) / (want_wgs > 0 ? want_wgs : 1));
+    const unsigned gx = (unsigned)((tiles + tiles_per_wg - 1) / tiles_per_wg);
+    const size_t lds_bytes = 4 * (size_t)kSlabChunks * 16 + 4 * kWideRows * sizeof(int);
+    auto kern = dense ? gms_wide_kernel<kWalkOwn> : a.first_offset ? gms_wide_kernel<kWalkRest> : gms_wide_kernel<kWalkAll>;
+    const int rc_lds = allow_dynamic_lds(reinterpret_cast<const void *>(kern), lds_bytes);
+    if (rc_lds != FGMS_OK) return rc_lds;
     ProfileScope prof(a.transpose_w ? "gms_wide_kernel(dgrad)" : "gms_wide_kernel(fwd)", a.stream);
-    gms_wide_kernel<<<dim3(gx + (unsigned)a.side.blocks, (unsigned)(c_dst / kWideCols)), kWideThreads, lds_bytes, a.stream>>>(
+    kern<<<dim3(gx + (unsigned)side.blocks, (unsigned)(c_dst / kWideCols)), kWideThreads, lds_bytes, a.stream>>>(
         (const __half *)a.src, (const int4v *)packed, (__half *)a.dst, a.kpos, a.gmap, a.smap, a.k_vol, c_src,
-        c_dst, tiles_per_wg, a.dense_k, (int)a.n_dense, a.side);
+        c_dst, tiles_per_wg, walk_offset(a, part == 0), (int)rows, side);
+    side = SideJob{};
   }
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;
