@@ -49,6 +49,15 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_resource(const void *base
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
 }
 
+// Half a 16-byte chunk at a row's end (fp16 rows of 4 channels more than a multiple of 8): loaded kTailBytes further to the front, so that
+// no load leaves its row, and moved into place, zeros behind it, on the way to LDS.  (What lies behind the row may be infinite, and
+// zeros in the other operand would make NaN of it.)  Rows start on 8 bytes then; buffer loads ask for 4.
+constexpr unsigned kTailBytes = 8;
+template <typename V>
+__device__ __forceinline__ V take_tail(V v, bool tail) {
+  return V{tail ? v[2] : v[0], tail ? v[3] : v[1], tail ? 0 : v[2], tail ? 0 : v[3]};
+}
+
 __device__ __forceinline__ float to_float(float v) { return v; }
 __device__ __forceinline__ float to_float(__half v) { return __half2float(v); }
 

@@ -377,22 +377,37 @@ __device__ __forceinline__ void gather_commit(int4v *__restrict__ a_lds, int4v (
 // `offs` holds a byte offset per row of the wave's tile, kAbsentRow for a row that has no
 // neighbour through this offset, which then arrives as zeros by itself: no select on the way
 // to LDS, no row index kept per load, 32-bit address arithmetic.
-// (RAGGED: the slab's chunks from row_bytes on do not exist either)
-template <int S, bool RAGGED = false, int N>
+// (RAGGED: the slab's chunks from row_bytes on do not exist either; TAILS: of a row's last chunk the first half does, see take_tail)
+template <int S, bool RAGGED = false, bool TAILS = false, int N>
 __device__ __forceinline__ void gather_issue_buf(int4v (&v)[N], const unsigned *__restrict__ offs,
                                                  __amdgpu_buffer_rsrc_t rsrc, int slab, int lane, unsigned row_bytes = 0) {
   constexpr int C = 2 * S;
   unsigned off[N];
 #pragma unroll
   for (int it = 0; it < N; ++it) off[it] = offs[(it * 64 + lane) / C] + (unsigned)((64 % C == 0 ? lane % C : (it * 64 + lane) % C) * 16);
-  if constexpr (RAGGED) {
+  if constexpr (TAILS) {
+    // (the slab in the lane's offset: a row's half chunk may start in front of it)
+#pragma unroll
+    for (int it = 0; it < N; ++it) {
+      const unsigned at = (unsigned)((slab * C + (it * 64 + lane) % C) * 16);
+      off[it] = at >= row_bytes ? kAbsentRow : off[it] + (unsigned)(slab * (C * 16)) - (at + 16 > row_bytes ? kTailBytes : 0u);
+    }
+  } else if constexpr (RAGGED) {
 #pragma unroll
     for (int it = 0; it < N; ++it)
       if ((unsigned)((slab * C + (it * 64 + lane) % C) * 16) >= row_bytes) off[it] = kAbsentRow;
   }
 #pragma unroll
   for (int it = 0; it < N; ++it)
-    v[it] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off[it], slab * (C * 16), 0));
+    v[it] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off[it], TAILS ? 0 : slab * (C * 16), 0));
+}
+
+// The rows of a slab that ends in half a chunk.
+template <int S, int N>
+__device__ __forceinline__ void take_row_tails(int4v (&v)[N], int slab, int lane, unsigned row_bytes) {
+  constexpr int C = 2 * S;
+#pragma unroll
+  for (int it = 0; it < N; ++it) v[it] = take_tail(v[it], (unsigned)((slab * C + (it * 64 + lane) % C) * 16) + 16 > row_bytes);
 }
 
 template <int S, int N>
@@ -558,8 +573,10 @@ constexpr int rows_sum_chunks() { return kWaves * MT * NT * 4 * 64; }      // ..
 
 // RAGGED (fp16, RAW 1 and 2; fp32, RAW 3 to 6): channel counts that fill no whole tile.  Chunks of rows and weights from
 // c_src on, and of weights from c_dst on, are loaded from outside their buffers and arrive as zeros (re-laid weights hold
-// zeros there); columns from c_dst on are not written.
-template <typename T, int NT, int S, int RAW, int MT = 2, int KG = 1, bool RAGGED = false>
+// zeros there); columns from c_dst on are not written.  TAILS (with it): 4 output channels more
+// than a multiple of 8, so that rows of that side end in half a chunk (see take_tail); a variant of its own, because the moves into
+// place and the addresses cost the masked tiles a tenth (48 -> 96 over 90 k LiDAR voxels, drop-in call 99.9 -> 112.3 us).
+template <typename T, int NT, int S, int RAW, int MT = 2, int KG = 1, bool RAGGED = false, bool TAILS = false>
 __device__ __forceinline__ void gms_rows_body(
     const T *__restrict__ src, const T *__restrict__ packed, T *__restrict__ dst,
     const int32_t *__restrict__ nbr, const unsigned long long *__restrict__ block_masks,
@@ -740,6 +757,10 @@ __device__ __forceinline__ void gms_rows_body(
     else if constexpr (P > 0) wvoff[i] = (unsigned)(((e / (NT * 64 * P)) * nts * 64 * P + e % (NT * 64 * P)) * 16);
     else wvoff[i] = (unsigned)(((e / (NT * 64)) * nts * 64 + e % (NT * 64)) * 16);
   }
+  // is chunk e of the stage's weights a row's last one, of which only half exists?
+  auto weight_tail = [&](int e, int slab) {
+    return kAsLies ? nt0 * 32 + e % WP * E + E > c_dst : slab * (C * E) + e % C * E + E > c_src;
+  };
   // (flip: the tables number the offsets from the other end, see Plan)
   auto weights_issue = [&](int4v (&wreg)[NW], int k_, int slab) {
     const int k = flip ? flip - k_ : k_;
@@ -770,16 +791,24 @@ __device__ __forceinline__ void gms_rows_body(
       const int e = tid + kThreads * i;
       if (NW * kThreads == WLD || e < WLD) {
         unsigned off = wvoff[i];
-        if constexpr (RAGGED && RAW != 3 && RAW != 5) {
+        if constexpr (TAILS) {
+          const int from = slab * (C * E) + (kAsLies ? e / WP : e % C * E);
+          const int to = nt0 * 32 + (kAsLies ? e % WP * E : e / C);
+          off = from >= c_src || to >= c_dst ? kAbsentRow : off + soff - (weight_tail(e, slab) ? kTailBytes : 0u);
+        } else if constexpr (RAGGED && RAW != 3 && RAW != 5) {
           const int from = slab * (C * E) + (kAsLies ? e / WP : e % C * E);
           const int to = nt0 * 32 + (kAsLies ? e % WP * E : e / C);
           if (from >= c_src || to >= c_dst) off = kAbsentRow;
         }
-        wreg[i] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(wrsrc, off, soff, 0));
+        wreg[i] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(wrsrc, off, TAILS ? 0 : soff, 0));
       }
     }
   };
-  auto weights_commit = [&](const int4v (&wreg)[NW], int buf) {
+  auto weights_commit = [&](int4v (&wreg)[NW], int buf, int slab) {
+    if constexpr (TAILS) {
+#pragma unroll
+      for (int i = 0; i < NW; ++i) wreg[i] = take_tail(wreg[i], weight_tail(tid + kThreads * i, slab));
+    }
 #pragma unroll
     for (int i = 0; i < NW; ++i) {
       const int e = tid + kThreads * i;
@@ -809,10 +838,11 @@ __device__ __forceinline__ void gms_rows_body(
   int4v v[NV];
   int gsel[kBuf ? 1 : NV];
   auto rows_issue = [&](int slab_, int slot_ = 0) {
-    if constexpr (kBuf) gather_issue_buf<S, RAGGED>(v, goff + slot_ * WR, rsrc, slab_, lane, row_bytes);
+    if constexpr (kBuf) gather_issue_buf<S, RAGGED, TAILS && kAsRows>(v, goff + slot_ * WR, rsrc, slab_, lane, row_bytes);
     else gather_issue<T, S>(v, gsel, gidx, src, c_src, slab_, lane);
   };
-  auto rows_commit = [&]() {
+  auto rows_commit = [&](int slab_) {
+    if constexpr (TAILS && kAsRows) take_row_tails<S>(v, slab_, lane, row_bytes);
     if constexpr (P > 0) gather_commit_parts_buf<P>(a_lds, v, lane, lost);
     else if constexpr (kBuf) gather_commit_buf<S>(a_lds, v, lane);
     else gather_commit<S>(a_lds, v, gsel, lane);
@@ -825,8 +855,8 @@ __device__ __forceinline__ void gms_rows_body(
   wave_lds_fence();
   weights_issue(wreg, k, 0);
   if (active) rows_issue(0);
-  weights_commit(wreg, 0);
-  if (active) rows_commit();
+  weights_commit(wreg, 0, 0);
+  if (active) rows_commit(0);
   __syncthreads();
 
   int buf = 0;
@@ -886,8 +916,8 @@ __device__ __forceinline__ void gms_rows_body(
       }
       if (active) mma_stage();
       wave_lds_fence();
-      rows_commit();
-      weights_commit(wreg, buf ^ 1);
+      rows_commit(nslab);
+      weights_commit(wreg, buf ^ 1, nslab);
       __syncthreads();
       buf ^= 1;
       active = (wave_mask >> nk) & 1;
@@ -954,8 +984,8 @@ __device__ __forceinline__ void gms_rows_body(
       }
       if (!has_next) break;
       wave_lds_fence();
-      if (next_active) rows_commit();
-      weights_commit(wreg, buf ^ 1);
+      if (next_active) rows_commit(nslab);
+      weights_commit(wreg, buf ^ 1, nslab);
       if (nk != k) {
         k_nxt = todo ? __builtin_ctzll(todo) : -1;
         if (todo) todo &= todo - 1;
@@ -1022,7 +1052,7 @@ __device__ __forceinline__ void gms_rows_body(
   }
 }
 
-template <typename T, int NT, int S, int RAW, int MT = 2, int KG = 1, bool RAGGED = false>
+template <typename T, int NT, int S, int RAW, int MT = 2, int KG = 1, bool RAGGED = false, bool TAILS = false>
 __global__ __launch_bounds__(kThreads * KG, RAW >= 5 ? (MT == 2 || KG == 2 ? 2 : KG == 4 ? 4 : 3)
                                                       : MT == 1 ? (NT == 3 ? 3 : 4) : (NT >= 3 ? 2 : 3)) void gms_rows_kernel(
     const T *__restrict__ src, const T *__restrict__ packed, T *__restrict__ dst,
@@ -1041,7 +1071,7 @@ __global__ __launch_bounds__(kThreads * KG, RAW >= 5 ? (MT == 2 || KG == 2 ? 2 :
     }
     block_x -= side.blocks;
   }
-  gms_rows_body<T, NT, S, RAW, MT, KG, RAGGED>(src, packed, dst, nbr, block_masks, perm, tile_order, n_dst, k_vol, c_src,
+  gms_rows_body<T, NT, S, RAW, MT, KG, RAGGED, TAILS>(src, packed, dst, nbr, block_masks, perm, tile_order, n_dst, k_vol, c_src,
                                    c_dst, part_stages, block_x, blockIdx.y, blockIdx.z, gridDim.z, src_bytes, pair_view,
                                    overwrite, flip_centre & 255, flip_centre >> 8 ? 1ull << ((flip_centre >> 8) - 1) : 0ull, w_raw);
 }
@@ -1118,15 +1148,19 @@ int ragged_steps(int c) {
 // The shapes that take it: multiples of 8 channels (16-byte chunks) that no whole tile fits -- a source of a pass
 // that is no multiple of 16, anything else that is none of 32 -- or an odd number of 32s from five
 // on (160), which whole tiles take 32 columns at a time.  Kernels on the vector ALUs keep the narrow ones.
+// fp16 output layers of 20 and 28 channels too (half_chunk; counts of 4 more than a multiple of 8 above a tile are rare, and every tile of
+// theirs would be one more instantiation): no copies of the gradient's rows and of the weights, no crop of either result; four launches
+// instead of seven, 96 -> 20 over 60 k voxels 77.5 -> 69.2 us.
 // fp32 (in bf16 parts): what is no multiple of 32 on either side.  Without (fp32 MFMAs, padded copies) / with masks:
 // 48 -> 48 over 30 k voxels forward 83 / 50 us, both gradients 123 / 65; 48 -> 64 over 120 k 121 / 108 and 303 / 189, in
 // tf32 mode 121 / 65 and 180 / 131.
 bool ragged_channels(int c_in, int c_out, bool forward, bool f16) {
-  if (c_in % 8 || c_out % 8 || c_in < 16 || c_out < 16 || c_in * c_out <= 256) return false;
+  if (c_in % 8 || c_out % (f16 && c_out <= 32 ? 4 : 8) || c_in < 16 || c_out < 16 || c_in * c_out <= 256) return false;
   if (!f16) return c_in % 32 != 0 || c_out % 32 != 0;
   auto odd = [](int c, int whole) { return c % whole != 0 || (c % 32 == 0 && c / 32 % 2 == 1 && c / 32 >= 5 && c / 32 % 3 != 0); };
   return odd(c_in, forward ? 16 : 32) || odd(c_out, 32);
 }
+bool half_chunk(const GmsArgs &a) { return a.c_out % 8 != 0; }      // (of the masked shapes)
 Shape ragged_shape(const GmsArgs &a) {
   Shape s{};
   s.c_src = a.transpose_w ? a.c_out : a.c_in;
@@ -1295,7 +1329,7 @@ RowsGrid rows_grid(int64_t n_dst, unsigned gy, int stages, bool can_half, bool h
   return g;
 }
 
-template <typename T, int NT, int S, bool RAGGED = false>
+template <typename T, int NT, int S, bool RAGGED = false, bool TAILS = false>
 int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
                 const unsigned long long *masks, const int32_t *perm, const int32_t *tile_order,
                 int tile_grid, int flip, bool pair_view = false) {
@@ -1312,14 +1346,14 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
   // 47.2 / 66.4 -> 40.9; tf32 mode over 5 k 35.2 / 31.6 -> 27.4; 128 -> 128 fp16 over 2 k 21.8 / 24.1 -> 19.5.
   if constexpr (NT == 2 || NT == 3) {
     if (rg.groups == 4 && (int64_t)rg.gx * gy * NT <= num_cus())
-      return launch_rows<T, 1, S, RAGGED>(a, s, nbr, masks, perm, tile_order, tile_grid, flip, pair_view);
+      return launch_rows<T, 1, S, RAGGED, TAILS>(a, s, nbr, masks, perm, tile_order, tile_grid, flip, pair_view);
     // ... and where 96-column tiles would be partly empty and 32-column ones fit the chip in one round
     // (128 -> 160 fp16 over 20 k voxels 48.6 -> 37.5 us)
     if (RAGGED && NT == 3 && (s.c_dst + 31) / 32 % 3 != 0 &&
         (a.n_dst + 127) / 128 * ((s.c_dst + 31) / 32) <= (int64_t)num_cus() * 4) {
       if (s.c_dst % 32 == 0 && s.c_src % (2 * S * s.E) == 0)      // (nothing left to mask)
         return launch_rows<T, 1, S>(a, s, nbr, masks, perm, tile_order, tile_grid, flip, pair_view);
-      return launch_rows<T, 1, S, RAGGED>(a, s, nbr, masks, perm, tile_order, tile_grid, flip, pair_view);
+      return launch_rows<T, 1, S, RAGGED, TAILS>(a, s, nbr, masks, perm, tile_order, tile_grid, flip, pair_view);
     }
   }
   // With 64-column wave tiles the input gradient and the fp16 forward pass read the weight
@@ -1381,8 +1415,8 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
   constexpr int kRagRaw = !RAGGED ? 0 : sizeof(T) == 2 ? kRaw1 : kRaw3, kRagRaw5 = !RAGGED ? 0 : sizeof(T) == 2 ? kRaw1 : kRaw5;
   // (raw is one of those the type and the tile allow)
 #define FGMS_BY_RAW(MTv, KGv)                                                                                       \
-  (RAGGED && raw == 5 ? gms_rows_kernel<T, NT, S, kRagRaw5, MTv, KGv == 4 && NT == 2 && sizeof(T) == 4 ? 2 : KGv, RAGGED> \
-   : RAGGED   ? gms_rows_kernel<T, NT, S, kRagRaw, MTv, KGv, RAGGED>                                                \
+  (RAGGED && raw == 5 ? gms_rows_kernel<T, NT, S, kRagRaw5, MTv, KGv == 4 && NT == 2 && sizeof(T) == 4 ? 2 : KGv, RAGGED, TAILS> \
+   : RAGGED   ? gms_rows_kernel<T, NT, S, kRagRaw, MTv, KGv, RAGGED, TAILS>                                         \
    : raw == 6 ? gms_rows_kernel<T, NT, S, kRaw6, MTv, 1>                                                            \
    : raw == 5 ? gms_rows_kernel<T, NT, S, kRaw5, MTv, KGv == 4 && NT == 2 ? 2 : KGv>                                \
    : raw == 4 ? gms_rows_kernel<T, NT, S, kRaw4, MTv, KGv>                                                          \
@@ -1435,7 +1469,7 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
 // plan's XCD-aware orders of either kind assume.
 // (2 waves per SIMD where the weight gradient's tile is 128 x 128: its 64 accumulators per lane and
 // the rows in flight spill at 3.  128 -> 128 over 40k voxels, forward and backward: tf32 mode 477 -> 327 us.)
-template <typename T, int NT, int S, int BI, int BJ, int RAWD, int MT = 2, bool RAGGED = false>
+template <typename T, int NT, int S, int BI, int BJ, int RAWD, int MT = 2, bool RAGGED = false, bool TAILS = false>
 __global__ __launch_bounds__(kThreads, NT >= 3 || RAWD == 6 || BI * BJ == 16 || ((BI == 3 || BJ == 3) && BI * BJ >= 6) ? 2 : 3)
 void bwd_fused_kernel(
     const T *__restrict__ gout, const T *__restrict__ w, T *__restrict__ gin,
@@ -1455,12 +1489,12 @@ void bwd_fused_kernel(
   }
   if ((int)blockIdx.x < rows_total) {
     const int bx = blockIdx.x % row_x, rest = blockIdx.x / row_x;
-    gms_rows_body<T, NT, S, RAWD, MT, 1, RAGGED>(gout, w, gin, nbr, block_masks, perm, tile_order, n_in, k_vol, c_out, c_in,
+    gms_rows_body<T, NT, S, RAWD, MT, 1, RAGGED, TAILS>(gout, w, gin, nbr, block_masks, perm, tile_order, n_in, k_vol, c_out, c_in,
                                       part_stages, bx, rest % row_y, rest / row_y, row_z, gout_bytes, 0, overwrite, flip, 0, nullptr);
   } else {
     const int j = blockIdx.x - rows_total;
     if constexpr (BI <= 3 && BJ <= 3)
-      wgrad_wave_body<T, BI, BJ, RAWD == 6 && BI * BJ == 1 ? 0 : split_parts_of(RAWD), RAGGED>(      // (see wave_geometry)
+      wgrad_wave_body<T, BI, BJ, RAWD == 6 && BI * BJ == 1 ? 0 : split_parts_of(RAWD), RAGGED, TAILS>(      // (see wave_geometry)
           in, gout, gw32, kpos, imap, omap, k_vol, c_in, c_out, smap, j % wgrad_x, j / wgrad_x, in_bytes, gout_bytes);
     else
       wgrad_wg_body<T, BI, BJ, RAWD == 4>(in, gout, gw32, kpos, imap, omap, k_vol, c_in, c_out, smap,
@@ -1474,7 +1508,7 @@ bool fused_bwd_enabled() {
   return on;
 }
 
-template <typename T, int NT, int S, int BI, int BJ, bool RAGGED = false>
+template <typename T, int NT, int S, int BI, int BJ, bool RAGGED = false, bool TAILS = false>
 int launch_fused(const GmsArgs &d, const Shape &s, const Plan *p, const WgradArgs &w, const WgradGeometry &g,
                  float *acc32) {
   // the input gradient's grid, as launch_rows lays it out (tiles padded to a multiple of 8)
@@ -1501,12 +1535,12 @@ int launch_fused(const GmsArgs &d, const Shape &s, const Plan *p, const WgradArg
   constexpr int kRaw2 = RAGGED && sizeof(T) == 4 ? 4 : 2;        // (masked fp32 shapes come in parts only)
   constexpr int kHalfMT = kCanHalf ? 1 : 2;
   constexpr int kRaw4 = kCanSplit ? 4 : 2, kRaw6 = kCan3 ? 6 : 2;
-  auto kern = rg.half_tiles ? (raw == 6 ? bwd_fused_kernel<T, NT, S, BI, BJ, kRaw6, kHalfMT, RAGGED>
-                               : raw == 4 ? bwd_fused_kernel<T, NT, S, BI, BJ, kRaw4, kHalfMT, RAGGED>
-                                          : bwd_fused_kernel<T, NT, S, BI, BJ, kRaw2, kHalfMT, RAGGED>)
-              : raw == 6    ? bwd_fused_kernel<T, NT, S, BI, BJ, kRaw6, 2, RAGGED>
-              : raw == 4    ? bwd_fused_kernel<T, NT, S, BI, BJ, kRaw4, 2, RAGGED>
-                            : bwd_fused_kernel<T, NT, S, BI, BJ, kRaw2, 2, RAGGED>;
+  auto kern = rg.half_tiles ? (raw == 6 ? bwd_fused_kernel<T, NT, S, BI, BJ, kRaw6, kHalfMT, RAGGED, TAILS>
+                               : raw == 4 ? bwd_fused_kernel<T, NT, S, BI, BJ, kRaw4, kHalfMT, RAGGED, TAILS>
+                                          : bwd_fused_kernel<T, NT, S, BI, BJ, kRaw2, kHalfMT, RAGGED, TAILS>)
+              : raw == 6    ? bwd_fused_kernel<T, NT, S, BI, BJ, kRaw6, 2, RAGGED, TAILS>
+              : raw == 4    ? bwd_fused_kernel<T, NT, S, BI, BJ, kRaw4, 2, RAGGED, TAILS>
+                            : bwd_fused_kernel<T, NT, S, BI, BJ, kRaw2, 2, RAGGED, TAILS>;
   size_t lds = g.lds;
   const size_t lds_rows = rg.half_tiles ? rows_group_chunks<T, NT, S, kHalfMT>(raw) * 16 : rows_group_chunks<T, NT, S, 2>(raw) * 16;
   if (lds < lds_rows) lds = lds_rows;
@@ -1667,11 +1701,19 @@ int launch_ragged_bwd(const GmsArgs &d, const Plan *p, const WgradArgs &w, bool 
   FGMS_FRF(1, 1) FGMS_FRF(1, 2) FGMS_FRF(2, 1) FGMS_FRF(2, 2)
 #undef FGMS_FRF
 #define FGMS_FR(NTv, Sv, BJv)                                                                                     \
-  if (!found && f16 && s.NTR == NTv && s.SR == Sv && g.bi == NTv && g.bj == BJv) {                                \
+  if (!found && f16 && !half_chunk(d) && s.NTR == NTv && s.SR == Sv && g.bi == NTv && g.bj == BJv) {                                \
     found = true;                                                                                                 \
     if ((rc = wgrad_accumulator(w, &acc32)) == FGMS_OK)                                                           \
       rc = launch_fused<__half, NTv, Sv, NTv, BJv, true>(d, s, p, w, g, acc32);                                   \
   }
+#define FGMS_FT(NTv)                                                                                              \
+  if (!found && f16 && half_chunk(d) && s.NTR == NTv && s.SR == 2 && g.bi == NTv && g.bj == 1) {                  \
+    found = true;                                                                                                 \
+    if ((rc = wgrad_accumulator(w, &acc32)) == FGMS_OK)                                                           \
+      rc = launch_fused<__half, NTv, 2, NTv, 1, true, true>(d, s, p, w, g, acc32);                                \
+  }
+  FGMS_FT(1) FGMS_FT(2) FGMS_FT(3)
+#undef FGMS_FT
   FGMS_FR(1, 2, 1) FGMS_FR(1, 3, 2) FGMS_FR(1, 4, 2) FGMS_FR(1, 3, 3) FGMS_FR(1, 4, 3)
   FGMS_FR(2, 2, 1) FGMS_FR(2, 3, 2) FGMS_FR(2, 4, 2) FGMS_FR(2, 3, 3) FGMS_FR(2, 4, 3)
   FGMS_FR(3, 2, 1) FGMS_FR(3, 3, 2) FGMS_FR(3, 4, 2) FGMS_FR(3, 3, 3) FGMS_FR(3, 4, 3)
@@ -1794,6 +1836,13 @@ int launch_ragged_gms(const GmsArgs &a, const Plan *p) {
     if (s.NTR == 2)
       return launch_rows<float, 2, 4, true>(a_, s, p->nbr_out, p->mask_out, p->perm_out, p->tile_out, p->tile_grid_out, p->flip_out);
     return launch_rows<float, 1, 4, true>(a_, s, p->nbr_out, p->mask_out, p->perm_out, p->tile_out, p->tile_grid_out, p->flip_out);
+  }
+  if (half_chunk(a)) {                        // (one column tile)
+    auto go = [&](auto sv) {
+      return launch_rows<__half, 1, decltype(sv)::value, true, true>(a_, s, p->nbr_out, p->mask_out, p->perm_out, p->tile_out, p->tile_grid_out,
+                                                                     p->flip_out);
+    };
+    return s.SR == 2 ? go(std::integral_constant<int, 2>{}) : s.SR == 3 ? go(std::integral_constant<int, 3>{}) : go(std::integral_constant<int, 4>{});
   }
 #define FGMS_RG(NTv, Sv)                   \
   if (s.NTR == NTv && s.SR == Sv)          \

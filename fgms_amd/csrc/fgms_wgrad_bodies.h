@@ -171,8 +171,8 @@ template <> struct WTW<float> { static constexpr int stage_pairs = 16; };
 // Three parts: a workgroup whose sums are not all finite (an infinite value has no parts), or that has met a value too small for
 // them, does its work again on fp32 MFMAs before anything is flushed.
 // RAGGED (not fp32 MFMAs alone): the tile's channels from c_in / c_out on do not exist; they are loaded from outside the
-// buffers, or another chunk in their place, and count as zeros, and are not flushed.
-template <typename T, int BI, int BJ, int SPLIT = 0, bool RAGGED = false>
+// buffers, or another chunk in their place, and count as zeros, and are not flushed.  TAILS (with it): output rows end in half a chunk, see take_tail.
+template <typename T, int BI, int BJ, int SPLIT = 0, bool RAGGED = false, bool TAILS = false>
 __device__ __forceinline__ void wgrad_wave_body(
     const T *__restrict__ in, const T *__restrict__ gout, float *__restrict__ gw32,
     const int32_t *__restrict__ kpos, const int32_t *__restrict__ imap,
@@ -239,6 +239,8 @@ __device__ __forceinline__ void wgrad_wave_body(
   auto g_row = [&](int i) { return !kBufW ? (lane + 64 * i) / NCO : NG == 6 ? lane / 4 + 16 * (i / 3) : (lane / NCO) * NG + i; };
   auto x_chunk = [&](int i) { return !kBufW ? (lane + 64 * i) % NCI : NX == 6 ? lane % 4 + 4 * (i % 3) : lane % NCI; };
   auto g_chunk = [&](int i) { return !kBufW ? (lane + 64 * i) % NCO : NG == 6 ? lane % 4 + 4 * (i % 3) : lane % NCO; };
+  static_assert(!TAILS || (RAGGED && kBufW), "half chunks: fp16");
+  auto g_tail = [&](int i) { return TAILS && co0 + g_chunk(i) * E + E > c_out; };      // (or beyond the row: zeros either way)
 
   // Everything is issued unconditionally and nothing touches a loaded register before
   // its consumer: an index or a row that is selected, copied or loaded under a branch
@@ -304,13 +306,17 @@ __device__ __forceinline__ void wgrad_wave_body(
         const bool live = st_ * SP + g_row(i) < count && (!RAGGED || co0 + cc * E < c_out);
         const unsigned off = live ? (unsigned)gi[i] * (unsigned)(c_out * (int)sizeof(T)) : kAbsentRow;
         gr[i] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(
-                                              gout_rsrc, off + (unsigned)((co0 + cc * E) * (int)sizeof(T)), 0, 0));
+                                              gout_rsrc, off + (unsigned)((co0 + cc * E) * (int)sizeof(T)) - (g_tail(i) && live ? kTailBytes : 0u), 0, 0));
       } else {
         gr[i] = *reinterpret_cast<const int4v *>(gout + (size_t)gi[i] * c_out + (RAGGED ? min(co0 + cc * E, c_out - E) : co0 + cc * E));
       }
     }
   };
   auto store_rows = [&](int st) {     // st: the stage the rows in flight belong to
+    if constexpr (TAILS) {
+#pragma unroll
+      for (int i = 0; i < NG; ++i) gr[i] = take_tail(gr[i], g_tail(i));
+    }
 #pragma unroll
     for (int i = 0; i < NX; ++i) {
       const int e = lane + 64 * i;
