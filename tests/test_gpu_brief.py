@@ -1,0 +1,89 @@
+"""Small fp16 forward launches, whose tiles take all offsets at once: whole numbers small enough for every sum to be one, over the
+channel counts and numbers of offsets it takes, first and last rows of a tile, and the plan's forms (a map with its centre kept
+apart, a mirrored one, empty offsets, rows without a pair)."""
+import numpy as np
+import pytest
+import torch
+
+from fgms_amd import clouds
+from tests.test_gpu_fp32_parts import exact
+
+pytestmark = pytest.mark.gpu
+
+CUBE, WIDE = clouds.offsets_cube(3).tolist(), clouds.offsets_cube(5).tolist()
+OFFSETS = {"cube": CUBE, "17": WIDE[54:71], "32": WIDE[40:72], "gaps": [[900, 900, 900]] + CUBE[:9] + [[901, 900, 900]] + CUBE[9:]}
+
+
+@pytest.mark.parametrize("offsets", sorted(OFFSETS))
+@pytest.mark.parametrize("n,shape", [(1, (32, 32)), (31, (16, 64)), (33, (48, 32)), (64, (64, 64)), (321, (32, 96)), (2000, (64, 32)), (2047, (32, 32)),
+                                     (500, (24, 40)), (700, (56, 16)), (900, (40, 72))],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_whole_numbers(n, shape, offsets):
+    from fgms_amd import capi
+    capi.set_kernel_policy(0)
+    vox = clouds.cloud_indoor(clouds.rng_for(4), target=n)
+    n = len(vox)
+    offs = np.ascontiguousarray(np.array(OFFSETS[offsets], dtype=np.int32))
+    imap, omap, _, kpos = clouds.build_kernel_map(vox, vox, offs)
+    maps = tuple(torch.from_numpy(np.ascontiguousarray(t.astype(np.int32))).cuda() for t in (kpos, imap, omap))
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(n)
+    few = lambda *s: torch.randint(-2, 3, s, generator=gen, device="cuda").half()
+    x, w = few(n, shape[0]), few(len(offs), *shape)
+    zeros = torch.zeros(n, shape[1], device="cuda")
+    want = exact(x.float(), w.float(), zeros, kpos.tolist(), maps[1].long(), maps[2].long())[0]
+    assert want.abs().max() <= 2048
+    plan = capi.Plan(*maps, n, n)
+    out = torch.full_like(zeros, float("nan")).half()
+    capi.conv_fwd(x, w, out, *maps, plan=plan)
+    assert torch.equal(out.double(), want)
+    start = few(n, shape[1])
+    out = start.clone()
+    capi.fusion_fwd(x, w, 0, out, maps[0], None, maps[1], maps[2], False, False, plan=plan)
+    assert torch.equal(out.double(), want + start.double())
+    plan.close()
+
+
+@pytest.mark.parametrize("n", [95, 2000])
+def test_mirrored_plan_and_centre(n):
+    from FGMS.nn import KernelMap, sparse_conv
+    from fgms_amd import capi
+    capi.set_kernel_policy(0)
+    vox = torch.from_numpy(clouds.cloud_indoor(clouds.rng_for(4), target=n)).cuda()
+    n = len(vox)
+    x = torch.randint(-2, 3, (n, 32), device="cuda").half()
+    w = torch.randint(-2, 3, (27, 32, 64), device="cuda").half()
+    imap, omap, knnz, kpos = capi.build_kernel_map(vox, vox, clouds.offsets_cube(3))
+    want = exact(x.float(), w.float(), torch.zeros(n, 64, device="cuda"), kpos.tolist(), imap.long(), omap.long())[0]
+    with torch.no_grad():
+        got = sparse_conv(x, w, KernelMap.from_coords(vox, vox, clouds.offsets_cube(3)), False)
+    assert torch.equal(got.double(), want)
+    imap, omap, knnz, kpos = capi.build_kernel_map(vox, vox, clouds.offsets_cube(3), skip_offset=13)
+    plan = capi.Plan(kpos, imap.clone(), omap.clone(), n, n)
+    out = torch.zeros(n, 64, device="cuda").half()
+    capi.fusion_fwd(x, w, 0, out, kpos, None, imap, omap, True, False, plan=plan)
+    assert torch.equal(out.double(), want)
+    plan.close()
+
+
+@pytest.mark.parametrize("shape", [(16, 32), (32, 64), (64, 32)])
+def test_infinite_weights_reach_their_pairs_only(shape):
+    from fgms_amd import capi
+    capi.set_kernel_policy(0)
+    vox = clouds.cloud_indoor(clouds.rng_for(4), target=1000)
+    n = len(vox)
+    imap, omap, _, kpos = clouds.build_kernel_map(vox, vox, clouds.offsets_cube(3))
+    maps = tuple(torch.from_numpy(np.ascontiguousarray(t.astype(np.int32))).cuda() for t in (kpos, imap, omap))
+    x, w = torch.randn(n, shape[0], device="cuda").half(), torch.randn(27, *shape, device="cuda").half() / 8
+    plan = capi.Plan(*maps, n, n)
+    clean, out = (torch.full((n, shape[1]), float("nan"), device="cuda").half() for _ in range(2))
+    capi.conv_fwd(x, w, clean, *maps, plan=plan)
+    w[5], w[22] = float("inf"), float("nan")
+    capi.conv_fwd(x, w, out, *maps, plan=plan)
+    hit = torch.zeros(n, dtype=torch.bool, device="cuda")
+    for k in (5, 22):
+        hit[maps[2][kpos[k]:kpos[k + 1]].long()] = True
+    assert hit.any() and not hit.all() and not torch.isfinite(out[hit]).any()
+    # (the same products; a wave's two offsets are added up before they meet the others' or each by itself: fp32 roundings)
+    assert torch.allclose(out[~hit].float(), clean[~hit].float(), rtol=2.0 ** -10, atol=2.0 ** -20 * 27 * shape[0])
+    plan.close()
