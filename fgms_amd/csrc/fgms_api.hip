@@ -669,7 +669,7 @@ int run_gms_padded(const GmsArgs &a, const Plan *plan, int c_in, int c_out, bool
 // a forward and a backward call, 125 -> 98 us.)
 bool centre_rides(const GmsArgs &a, const Plan *plan) {
   if (!plan || a.n_pairs == 0 || !plan->groups.empty() || !plan->centre_line || a.centre - 1 != a.k_vol / 2 || a.n_src != a.n_dst) return false;
-  if (brief_gms_pays(a, plan)) return true;
+  if (brief_gms_pays(a, plan) || held_gms_pays(a, plan)) return true;
   if (takes_ragged(a, plan) && ragged_gms_supported(a, plan) && ragged_pays(a, plan)) return true;
   int pi, po;
   return route_of(padded_gms_channels(a, plan, &pi, &po) ? with_channels(a, pi, po) : a, plan) == Route::kRows;
@@ -696,6 +696,10 @@ int run_gms(GmsArgs a, const Plan *plan) {
   if (brief_gms_pays(a, plan)) {
     plan_touch(plan, a.stream);
     return launch_brief_gms(a, plan);
+  }
+  if (held_gms_pays(a, plan)) {
+    plan_touch(plan, a.stream);
+    return launch_held_gms(a, plan);
   }
   if (takes_ragged(a, plan) && ragged_gms_supported(a, plan) && ragged_pays(a, plan)) {
     plan_touch(plan, a.stream);

@@ -315,6 +315,9 @@ bool split_bf16_enabled();   // products of fp32 tensors in bf16 parts: three a 
 // Small fp16 forward launches, all offsets of a tile at once (fgms_brief.hip).
 bool brief_gms_pays(const GmsArgs &a, const Plan *p);
 int launch_brief_gms(const GmsArgs &a, const Plan *p);
+// ... and of up to 32 channels, all weights in LDS, in the place of the output-stationary kernel (whole tiles and masked).
+bool held_gms_pays(const GmsArgs &a, const Plan *p);
+int launch_held_gms(const GmsArgs &a, const Plan *p);
 bool small_gms_supported(const GmsArgs &a, const Plan *p);
 int launch_small_gms(const GmsArgs &a, const Plan *p);
 // Narrow input sides on the matrix cores (fgms_narrow.hip): the forward pass, and the weight gradient.

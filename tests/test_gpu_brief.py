@@ -12,6 +12,7 @@ pytestmark = pytest.mark.gpu
 
 CUBE, WIDE = clouds.offsets_cube(3).tolist(), clouds.offsets_cube(5).tolist()
 OFFSETS = {"cube": CUBE, "17": WIDE[54:71], "32": WIDE[40:72], "gaps": [[900, 900, 900]] + CUBE[:9] + [[901, 900, 900]] + CUBE[9:]}
+FEW = {"9": CUBE[9:18], "16": CUBE[5:21], **OFFSETS}
 
 
 @pytest.mark.parametrize("offsets", sorted(OFFSETS))
@@ -19,11 +20,22 @@ OFFSETS = {"cube": CUBE, "17": WIDE[54:71], "32": WIDE[40:72], "gaps": [[900, 90
                                      (500, (24, 40)), (700, (56, 16)), (900, (40, 72))],
                          ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
 def test_whole_numbers(n, shape, offsets):
+    whole_numbers(n, shape, offsets)
+
+
+# up to 32 channels with all weights in LDS: few offsets at any size, more of them above what the other kernel takes
+@pytest.mark.parametrize("n,shape,offsets", [(1, (32, 32), "9"), (257, (24, 24), "16"), (3001, (32, 16), "9"), (3001, (40, 32), "16"), (40001, (32, 32), "cube"),
+                                             (40001, (24, 32), "gaps"), (33000, (32, 24), "32"), (50000, (16, 16), "17")])
+def test_whole_numbers_with_the_weights_held(n, shape, offsets):
+    whole_numbers(n, shape, offsets)
+
+
+def whole_numbers(n, shape, offsets):
     from fgms_amd import capi
     capi.set_kernel_policy(0)
     vox = clouds.cloud_indoor(clouds.rng_for(4), target=n)
     n = len(vox)
-    offs = np.ascontiguousarray(np.array(OFFSETS[offsets], dtype=np.int32))
+    offs = np.ascontiguousarray(np.array(FEW[offsets], dtype=np.int32))
     imap, omap, _, kpos = clouds.build_kernel_map(vox, vox, offs)
     maps = tuple(torch.from_numpy(np.ascontiguousarray(t.astype(np.int32))).cuda() for t in (kpos, imap, omap))
     gen = torch.Generator(device="cuda")
@@ -66,11 +78,11 @@ def test_mirrored_plan_and_centre(n):
     plan.close()
 
 
-@pytest.mark.parametrize("shape", [(16, 32), (32, 64), (64, 32)])
-def test_infinite_weights_reach_their_pairs_only(shape):
+@pytest.mark.parametrize("n,shape", [(1000, (16, 32)), (1000, (32, 64)), (1000, (64, 32)), (40000, (16, 32)), (40000, (32, 24))])
+def test_infinite_weights_reach_their_pairs_only(n, shape):
     from fgms_amd import capi
     capi.set_kernel_policy(0)
-    vox = clouds.cloud_indoor(clouds.rng_for(4), target=1000)
+    vox = clouds.cloud_indoor(clouds.rng_for(4), target=n)
     n = len(vox)
     imap, omap, _, kpos = clouds.build_kernel_map(vox, vox, clouds.offsets_cube(3))
     maps = tuple(torch.from_numpy(np.ascontiguousarray(t.astype(np.int32))).cuda() for t in (kpos, imap, omap))
@@ -84,6 +96,6 @@ def test_infinite_weights_reach_their_pairs_only(shape):
     for k in (5, 22):
         hit[maps[2][kpos[k]:kpos[k + 1]].long()] = True
     assert hit.any() and not hit.all() and not torch.isfinite(out[hit]).any()
-    # (the same products; a wave's two offsets are added up before they meet the others' or each by itself: fp32 roundings)
+    # (the same products; sums of a few offsets before they meet the others', or of each by itself: fp32 roundings)
     assert torch.allclose(out[~hit].float(), clean[~hit].float(), rtol=2.0 ** -10, atol=2.0 ** -20 * 27 * shape[0])
     plan.close()
