@@ -208,15 +208,11 @@ __device__ __forceinline__ void add_rows_lds(const float16v (&acc)[MT][NT], T *_
   constexpr int FIT = (WR * 2 * S * 16) / (COLS * 4);
   constexpr int R = FIT >= 32 ? 32 : FIT >= 16 ? 16 : FIT >= 8 ? 8 : 0;
   if constexpr (R < 8) {
+    // (Written as they are, not added to zeros behind a fence, which every wave of a launch waited for: forward launches of half tiles,
+    // 16 -> 64 fp16 over 100 k voxels 112 -> 17 us, 32 -> 96 137 -> 24, over 18 k 30 -> 14.)
     if constexpr (ATOMIC) write_tile<T, NT, kTileAtomic, RAGGED>(acc, dst, rows, c_dst, cd0, lane);
-    else {
-      if constexpr (OVERWRITE) {
-        zero_rows<T, NT, WR, RAGGED>(dst, rows, c_dst, cd0, lane);
-        __builtin_amdgcn_s_waitcnt(0x0F70);      // vmcnt(0): the zeros are on their way before the rows are read
-        __threadfence();
-      }
-      add_rows<T, NT, RAGGED>(acc, dst, rows, c_dst, cd0, lane);
-    }
+    else if constexpr (OVERWRITE) write_tile<T, NT, kTileStore, RAGGED>(acc, dst, rows, c_dst, cd0, lane);
+    else add_rows<T, NT, RAGGED>(acc, dst, rows, c_dst, cd0, lane);
   } else {
     constexpr int CH = COLS / 4;            // 16-byte chunks per staged row
     constexpr int IT = R * CH / 64;         // chunks per lane and pass
