@@ -129,7 +129,7 @@ __global__ __launch_bounds__(kBriefWaves * 64, 4) void gms_brief_kernel(BriefArg
   }
 }
 
-// Layers of up to 32 channels on either side, at any size: all weights of the layer stay in LDS, and a wave walks the offsets of its own 32 rows.
+// Layers of up to 32 channels in, 32 columns a workgroup: all weights of the layer stay in LDS, and a wave walks the offsets of its own 32 rows.
 // Four offsets make a batch; the next batch's rows and the indices of the one behind it are in flight, and after the weights have come in
 // there is no barrier: a stage of the output-stationary kernel, which brings 2 KB of weights and waits for four waves, does 32 channels' work of
 // 128 clocks.  Bound by the L1's gathers where the launch is long: whole rows by neighbouring lanes, and through LDS to the lanes that want them
@@ -157,7 +157,7 @@ __global__ __launch_bounds__(kHeldWaves * 64, 4) void gms_held_kernel(BriefArgs 
   int block_x = blockIdx.x;
   if (a.side.blocks) {
     if (block_x < a.side.blocks) {
-      run_side_job(a.side, block_x);
+      if (blockIdx.y == 0) run_side_job(a.side, block_x);
       return;
     }
     block_x -= a.side.blocks;
@@ -171,7 +171,7 @@ __global__ __launch_bounds__(kHeldWaves * 64, 4) void gms_held_kernel(BriefArgs 
   extern __shared__ int4v lds[];
   __shared__ int out_rows[kHeldWaves][32];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int h = lane >> 5;
+  const int h = lane >> 5, nt0 = blockIdx.y * 32;
   const int pos0 = tile * (kHeldWaves * 32) + wave * 32, pos = pos0 + (lane & 31), safe_pos = min(pos, a.n_dst - 1);
   const bool in_range = pos < a.n_dst;
   unsigned long long mask = a.block_masks[min(pos0, a.n_dst - 1) / 64] | a.centre;
@@ -224,7 +224,7 @@ __global__ __launch_bounds__(kHeldWaves * 64, 4) void gms_held_kernel(BriefArgs 
   int4v wreg[NW];
 #pragma unroll
   for (int i = 0; i < NW; ++i) {
-    const int e = tid + i * kThreads_, k = e / kChunks, c = e % kChunks / 4, to = e % 4 * 8;
+    const int e = tid + i * kThreads_, k = e / kChunks, c = e % kChunks / 4, to = nt0 + e % 4 * 8;
     const unsigned off = k < a.k_vol && c < a.c_src && to < a.c_dst ? (unsigned)((k * a.c_src + c) * a.c_dst + to) * 2u : kAbsentRow;
     wreg[i] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(wrsrc, off, 0, 0));
   }
@@ -272,8 +272,8 @@ __global__ __launch_bounds__(kHeldWaves * 64, 4) void gms_held_kernel(BriefArgs 
         if (rows >> ((r / 4) * 8 + h * 4 + r % 4) & 1) acc[0][0][r] += own[r];
     }
   }
-  if (a.overwrite) write_tile<__half, 1, kTileStore, true>(acc, a.dst, out_rows[wave], a.c_dst, 0, lane);
-  else if (mask) write_tile<__half, 1, kTileAdd, true>(acc, a.dst, out_rows[wave], a.c_dst, 0, lane);
+  if (a.overwrite) write_tile<__half, 1, kTileStore, true>(acc, a.dst, out_rows[wave], a.c_dst, nt0, lane);
+  else if (mask) write_tile<__half, 1, kTileAdd, true>(acc, a.dst, out_rows[wave], a.c_dst, nt0, lane);
 }
 
 int brief_steps(const GmsArgs &a) { return (a.c_in + 15) / 16; }
@@ -346,10 +346,13 @@ int launch_brief_gms(const GmsArgs &a, const Plan *p) {
 // order: 32 -> 32 over 35 k 10.7 / 10.3 and 11.2 / 10.4, 60 k 12.1 / 10.5 and 14.2 / 11.3, 100 k 17.3 / 12.3 and 20.0 / 15.9, 130 k 19.2 / 14.0
 // and 22.2 / 19.6, 200 k, where some workgroups wait for a second round, 22.6 / 22.2 and 28.3 / 28.9; 16 -> 32 over 60 k 10.1 / 7.6 and 10.6 / 8.0,
 // 200 k 27.7 / 15.6 and 32.4 / 21.0; 32 -> 16 over 60 k 21.7 / 10.4 and 25.4 / 11.0, 200 k 50.1 / 21.4 and 57.1 / 27.8; 16 -> 16 over 100 k 11.4 / 8.1 and
-// 14.9 / 11.7.)
+// 14.9 / 11.7.  More than 32 columns gather their rows twice: 16 -> 48 over 60 k 13.5 / 11.0, 200 k 37.9 / 26.5; 16 -> 64 over 30 k 10.7 / 8.3, 100 k
+// 17.1 / 14.7 and 20.3 / 19.4, 200 k 22.2 / 27.3; 32 -> 64 over 30 k 12.2 / 11.7, 60 k 14.5 / 17.1.)
 bool held_gms_pays(const GmsArgs &a, const Plan *p) {
-  if (!brief_layer(a, p, 32) || a.c_out > 32 || a.k_vol <= 8) return false;
-  return a.c_in <= 16 || a.c_out <= 16 || (a.n_dst + kHeldWaves * 32 - 1) / (kHeldWaves * 32) <= 2 * (int64_t)num_cus();
+  if (!brief_layer(a, p, 32) || a.c_out > 64 || a.k_vol <= 8) return false;
+  const int64_t workgroups = (a.n_dst + kHeldWaves * 32 - 1) / (kHeldWaves * 32) * ((a.c_out + 31) / 32);
+  if (a.c_in <= 16) return a.c_out <= 48 || workgroups <= 4 * (int64_t)num_cus();
+  return a.c_out <= 16 || (a.c_out <= 32 && workgroups <= 2 * (int64_t)num_cus());
 }
 
 int launch_held_gms(const GmsArgs &a, const Plan *p) {
@@ -361,7 +364,7 @@ int launch_held_gms(const GmsArgs &a, const Plan *p) {
   const unsigned tiles = p->tile_out ? (unsigned)p->tile_grid_out : (unsigned)((a.n_dst + kHeldWaves * 32 - 1) / (kHeldWaves * 32));
   {
     ProfileScope prof("gms_rows_kernel(fwd)", a.stream);
-    kern<<<tiles + (unsigned)b.side.blocks, kHeldWaves * 64, lds, a.stream>>>(b, p->tile_out);
+    kern<<<dim3(tiles + (unsigned)b.side.blocks, (unsigned)((a.c_out + 31) / 32)), kHeldWaves * 64, lds, a.stream>>>(b, p->tile_out);
   }
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;

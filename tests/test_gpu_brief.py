@@ -25,7 +25,8 @@ def test_whole_numbers(n, shape, offsets):
 
 # up to 32 channels with all weights in LDS: few offsets at any size, more of them above what the other kernel takes
 @pytest.mark.parametrize("n,shape,offsets", [(1, (32, 32), "9"), (257, (24, 24), "16"), (3001, (32, 16), "9"), (3001, (40, 32), "16"), (40001, (32, 32), "cube"),
-                                             (40001, (24, 32), "gaps"), (33000, (32, 24), "32"), (50000, (16, 16), "17")])
+                                             (40001, (24, 32), "gaps"), (33000, (32, 24), "32"), (50000, (16, 16), "17"), (1500, (24, 40), "16"),
+                                             (3001, (16, 64), "9"), (35000, (32, 64), "cube")])
 def test_whole_numbers_with_the_weights_held(n, shape, offsets):
     whole_numbers(n, shape, offsets)
 
