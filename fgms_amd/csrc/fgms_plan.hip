@@ -383,7 +383,7 @@ __device__ __forceinline__ void bands_body(const TablesArgs &a, int x, int shift
 // workgroups of the same launch: tile orders, row bands, the fingerprint of the lists, the findings'
 // way to the host.  (Five launches of 3-12 us each and a second stream before.)
 __global__ __launch_bounds__(256) void tables_kernel(TablesArgs a) {
-  extern __shared__ int32_t lds[];
+  extern __shared__ __align__(16) int32_t lds[];      // (bands_body reads 16 bytes at a time; the static LDS in front of it ends anywhere)
   int b = blockIdx.x;
   if (b < a.tile_blocks) {
     if (b == 0 && threadIdx.x < kPlanFlags) {

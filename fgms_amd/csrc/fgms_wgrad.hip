@@ -133,7 +133,7 @@ __global__ __launch_bounds__(kSkinnyThreads) void wgrad_skinny_kernel(
   constexpr int PPS = 64 / GD;                // pairs per step
   constexpr int XW = CS * (int)sizeof(T) / 4; // 32-bit words of an input row
   static_assert(CD % KD == 0 && 64 % GD == 0 && XW >= 1, "shape");
-  extern __shared__ float red[];            // [waves - 1][CS][CD]
+  extern __shared__ __align__(16) float red[];            // [waves - 1][CS][CD]
   constexpr int kWavesS = kSkinnyThreads / 64;
   int k, first, count;
   if (!locate_slice(kpos, smap, k_vol, block_x, k, first, count)) return;
