@@ -10,7 +10,7 @@
 //
 //   1. fill     everything that has to start from a value
 //   2. insert   every input row enters its block of 2 x 2 x 4 voxels; the blocks are found through
-//               an open-addressing hash table (linear probing, load <= 0.8); equal coordinates keep the
+//               an open-addressing hash table (buckets of four, load <= 0.5); equal coordinates keep the
 //               smallest row
 //   3. lookup   a table of the output rows, [n_out][offsets] -> input row or -1, the
 //               set of offsets every row has a pair through, hits per (offset, 256 rows)
@@ -57,21 +57,28 @@ struct Offsets {
 // of `cells`, at its slot's number.  The 27 neighbours of a voxel lie in 8 blocks, and
 // neighbouring rows share them: an eighth of the random accesses that a table of voxels costs, which
 // is what such a table is bound by (100 k rows x 27 offsets: 2.7 M probes of a line each).  A slot holds its block's coordinates
-// themselves (59 bits), so that a search is one access to it and one to the cells.  (A row number in the slot, its coordinates
-// behind a load of their own, cells by row: insertion of 29 k rows 6.5 -> 4.8 us,
-// of 200 k 15.6 -> 14.6, the lookup the same.)
+// themselves (59 bits), so that a search is one access to it and one to the cells.
+// A search waits for one bucket after another, and a wave for the longest chain of its lanes, most of which look for blocks that are not
+// there.  Four slots to a bucket, read together, and two slots a row, whatever the number of rows: longest chain of a workgroup of the
+// lookup, in the mean, 1.1 buckets over indoor and LiDAR surfaces, 2.0 over an indoor cloud thinned to a quarter, 2.7 to an
+// eighth, 5.3 over 104 k voxels with a block each.  Single slots, two to four a row: 2.5, 4.6, 6.6 and 12; 1.25 to 2.5 a row: 3,
+// 10, 18 and 141.  Whole builds with either of these / this, us: 200 k indoor voxels x 27 offsets 146 / 117 / 118, the eighth of them x 27
+// 85 / 87 / 77 and x 125 144 / 231 / 105, 104 k with a block each x 27 123 / 277 / 104 and x 125 379 / 2 379 / 223.  (Three slots to
+// two rows: 80 k with a block each x 125 314, of two a row 205, of two to four single ones 273.)
 constexpr int kBlockX = 1, kBlockY = 1, kBlockZ = 2;      // bits of a coordinate inside its block
 constexpr int kCells = 1 << (kBlockX + kBlockY + kBlockZ);
 constexpr int kNoRow = INT32_MAX;
+constexpr int kBucket = 4;
+constexpr unsigned kNoSlot = ~0u;
 
 // (Factors: the first three 32-bit primes of xxHash, Y. Collet; finaliser: prospector32, C. Wellons, "Prospecting for
 // hash functions", 2018.)
-__device__ __forceinline__ unsigned slot_of(int bx, int by, int bz, unsigned mask) {
+__device__ __forceinline__ unsigned bucket_of(int bx, int by, int bz, unsigned buckets) {
   unsigned h = (unsigned)bx * 0x9E3779B1u ^ (unsigned)by * 0x85EBCA77u ^ (unsigned)bz * 0xC2B2AE3Du;
   h ^= h >> 15; h *= 0x2C1B3C6Du;
   h ^= h >> 12; h *= 0x297A2D39u;
   h ^= h >> 15;
-  return h & mask;
+  return __umulhi(h, buckets);
 }
 __device__ __forceinline__ int cell_of(int x, int y, int z) { return (x & 1) << 3 | (y & 1) << 2 | (z & 3); }
 // A block as a slot holds it.  (Blocks of accepted coordinates only, block_exists; a free slot's ones are none of them.)
@@ -85,10 +92,20 @@ __device__ __forceinline__ BlockKey block_key(int bx, int by, int bz) {
   constexpr int x = kCoordLimit >> kBlockX, y = kCoordLimit >> kBlockY, z = kCoordLimit >> kBlockZ;
   return (BlockKey)(unsigned)(bx + x) << 40 | (BlockKey)(unsigned)(by + y) << 20 | (unsigned)(bz + z);
 }
+// The slots of a bucket.  They fill from the front and keep what they hold, so that a free one ends every search.
+typedef BlockKey keys2_ __attribute__((ext_vector_type(2)));
+struct Bucket {
+  keys2_ front, back;
+  __device__ __forceinline__ BlockKey operator[](int e) const { return e < 2 ? front[e] : back[e - 2]; }
+};
+__device__ __forceinline__ Bucket bucket_at(const BlockKey *__restrict__ slots, unsigned bucket) {
+  const keys2_ *const p = reinterpret_cast<const keys2_ *>(slots + (size_t)bucket * kBucket);
+  return Bucket{p[0], p[1]};
+}
 
 // flags[0]: an input coordinate is outside the range; flags[1]: two input rows share their coordinates
 __global__ __launch_bounds__(256) void kmap_insert_kernel(const int32_t *__restrict__ coords, int n, BlockKey *__restrict__ slots,
-                                                          unsigned mask, int32_t *__restrict__ cells, int *__restrict__ flags) {
+                                                          unsigned buckets, int32_t *__restrict__ cells, int *__restrict__ flags) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
   const int x = coords[3 * i], y = coords[3 * i + 1], z = coords[3 * i + 2];
@@ -97,14 +114,26 @@ __global__ __launch_bounds__(256) void kmap_insert_kernel(const int32_t *__restr
     return;
   }
   const int bx = x >> kBlockX, by = y >> kBlockY, bz = z >> kBlockZ;
-  unsigned slot = slot_of(bx, by, bz, mask);
+  unsigned bucket = bucket_of(bx, by, bz, buckets);
   const BlockKey key = block_key(bx, by, bz);
+  int e = 0;
   while (true) {                       // ends: the table has more slots than rows
-    const BlockKey prev = atomicCAS(&slots[slot], kFreeSlot, key);
+    const BlockKey prev = atomicCAS(&slots[(size_t)bucket * kBucket + e], kFreeSlot, key);
     if (prev == kFreeSlot || prev == key) break;
-    slot = (slot + 1) & mask;
+    // (what is read here may be old: a slot taken since then still looks free, and the exchange above tells)
+    const Bucket b = bucket_at(slots, bucket);
+    int next = kBucket;
+#pragma unroll
+    for (int q = kBucket - 1; q > 0; --q)
+      if (q > e && (b[q] == kFreeSlot || b[q] == key)) next = q;
+    e = next;
+    if (e == kBucket) {
+      e = 0;
+      bucket = bucket + 1 == buckets ? 0 : bucket + 1;
+    }
   }
-  if (atomicMin(&cells[(size_t)slot * kCells + cell_of(x, y, z)], i) != kNoRow) flags[1] = 1;
+  const size_t slot = (size_t)bucket * kBucket + e;
+  if (atomicMin(&cells[slot * kCells + cell_of(x, y, z)], i) != kNoRow) flags[1] = 1;
 }
 
 struct LookupArgs {
@@ -112,7 +141,7 @@ struct LookupArgs {
   int n_out, k_vol, stride, skip_offset, row_ld;
   const BlockKey *slots;
   const int32_t *cells;
-  unsigned mask;
+  unsigned buckets;
   const int32_t *offsets;                      // device; nullptr: `offs`
   int32_t *rows;                               // [n_out][row_ld]
   int32_t *counts;                             // [k_vol][blocks of kListRows rows]
@@ -132,31 +161,36 @@ __device__ __forceinline__ void publish_coordinates(const int *__restrict__ flag
   __hip_atomic_store(&host[0], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// The slots of N blocks (-1: not in use; want = false: not asked for), all probed together.
+// The slots of N blocks (kNoSlot: not in use; want = false: not asked for), all searched together.
 template <int N>
 __device__ __forceinline__ void find_blocks(const LookupArgs &a, const int (&bx)[N], const int (&by)[N], const int (&bz)[N],
-                                            const bool (&want)[N], int (&at)[N]) {
-  unsigned slot[N];
+                                            const bool (&want)[N], unsigned (&at)[N]) {
+  unsigned bucket[N];
   BlockKey key[N];
   bool open[N], any = false;
 #pragma unroll
   for (int u = 0; u < N; ++u) {
-    at[u] = -1;
+    at[u] = kNoSlot;
     open[u] = want[u] && block_exists(bx[u], by[u], bz[u]);
     any = any || open[u];
-    slot[u] = slot_of(bx[u], by[u], bz[u], a.mask);
+    bucket[u] = bucket_of(bx[u], by[u], bz[u], a.buckets);
     key[u] = block_key(bx[u], by[u], bz[u]);
   }
   while (any) {                        // ends: every chain meets its block or a free slot
-    BlockKey cand[N];
+    Bucket b[N];
 #pragma unroll
-    for (int u = 0; u < N; ++u) cand[u] = open[u] ? a.slots[slot[u]] : kFreeSlot;
+    for (int u = 0; u < N; ++u)
+      if (open[u]) b[u] = bucket_at(a.slots, bucket[u]);
     any = false;
 #pragma unroll
     for (int u = 0; u < N; ++u) {
-      if (cand[u] == key[u] && open[u]) at[u] = (int)slot[u];
-      open[u] = open[u] && cand[u] != key[u] && cand[u] != kFreeSlot;
-      slot[u] = open[u] ? (slot[u] + 1) & a.mask : slot[u];
+      if (open[u]) {
+#pragma unroll
+        for (int e = 0; e < kBucket; ++e)
+          if (b[u][e] == key[u]) at[u] = bucket[u] * kBucket + e;
+      }
+      open[u] = open[u] && at[u] == kNoSlot && b[u][kBucket - 1] != kFreeSlot;
+      bucket[u] = bucket[u] + 1 == a.buckets ? 0 : bucket[u] + 1;
       any = any || open[u];
     }
   }
@@ -175,7 +209,7 @@ __global__ __launch_bounds__(256) void kmap_lookup_kernel(LookupArgs a, Offsets 
   constexpr int kMine = kLookupChunk / 4;
   __shared__ int32_t found[kLookupRows][kLookupChunk + 1];
   __shared__ unsigned long long wave_mask[4][kLookupRows];
-  __shared__ int32_t near_slot[8][kLookupRows];
+  __shared__ unsigned near_slot[8][kLookupRows];
   if (blockIdx.x == gridDim.x - 1) {
     publish_coordinates(a.flags, a.host);
     return;
@@ -193,7 +227,8 @@ __global__ __launch_bounds__(256) void kmap_lookup_kernel(LookupArgs a, Offsets 
   const int block = blockIdx.x * kLookupRows / kListRows;
   if constexpr (NEAR) {
     // block j of a row: the row's own (bits 0) or the nearer neighbour along x (bit 2), y (bit 1), z (bit 0)
-    int bx[2], by[2], bz[2], at[2];
+    int bx[2], by[2], bz[2];
+    unsigned at[2];
     bool want[2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
@@ -211,12 +246,13 @@ __global__ __launch_bounds__(256) void kmap_lookup_kernel(LookupArgs a, Offsets 
   }
   unsigned long long mine = 0;
   for (int k0 = 0; k0 < a.k_vol; k0 += kLookupChunk) {
-    int hit[kMine], at[kMine], cell[kMine];
+    int hit[kMine], cell[kMine];
+    unsigned at[kMine];
     if constexpr (NEAR) {
 #pragma unroll
       for (int u = 0; u < kMine; ++u) {
         const int k = k0 + u * 4 + wave;
-        at[u] = -1;
+        at[u] = kNoSlot;
         cell[u] = 0;
         if (k < a.k_vol && k != a.skip_offset) {
           const int *d = a.offsets ? a.offsets + 3 * k : offs.xyz + 3 * k;
@@ -246,12 +282,12 @@ __global__ __launch_bounds__(256) void kmap_lookup_kernel(LookupArgs a, Offsets 
       find_blocks<kMine>(a, bx, by, bz, want, at);
     }
 #pragma unroll
-    for (int u = 0; u < kMine; ++u) hit[u] = a.cells[(size_t)(at[u] < 0 ? 0 : at[u]) * kCells + cell[u]];
+    for (int u = 0; u < kMine; ++u) hit[u] = a.cells[(size_t)(at[u] == kNoSlot ? 0 : at[u]) * kCells + cell[u]];
 #pragma unroll
     for (int u = 0; u < kMine; ++u) {
       const int k = k0 + u * 4 + wave;
       if (k >= a.k_vol) break;
-      if (at[u] < 0 || hit[u] == kNoRow) hit[u] = -1;
+      if (at[u] == kNoSlot || hit[u] == kNoRow) hit[u] = -1;
       found[lane][k - k0] = hit[u];
       const unsigned long long b = __ballot(hit[u] >= 0);
       if (lane == 0) count_of[k - k0] = __builtin_popcountll(b);
@@ -690,9 +726,9 @@ int map_build_begin(MapBuild **build, const int32_t *in_coords, int64_t n_in, co
     for (int c = 0; c < 3; ++c)
       if (offsets_host[3 * (k_vol - 1 - k) + c] != -offsets_host[3 * k + c]) mirror = false;
 
-  // (a quarter more slots than rows at least; surfaces have two to four rows to a block)
-  size_t slots = 256;
-  while (slots * 4 < 5 * (size_t)n_in) slots <<= 1;
+  // (144 bytes of scratch a row, slots and cells, at every size)
+  const unsigned buckets = (unsigned)((2 * (size_t)n_in + kBucket - 1) / kBucket + 1);
+  const size_t slots = (size_t)buckets * kBucket;
   const int blocks = (int)((n_out + kListRows - 1) / kListRows);
   const int row_ld = (k_vol + 3) / 4 * 4;
   const size_t n_counts = (size_t)k_vol * blocks;
@@ -798,14 +834,13 @@ int map_build_begin(MapBuild **build, const int32_t *in_coords, int64_t n_in, co
     memcpy(offs.xyz, offsets_host, (size_t)k_vol * 3 * sizeof(int32_t));
   }
   if ((rc = launch_fills(fills, s))) return fail(rc);
-  const unsigned mask = (unsigned)(slots - 1);
   if (n_in > 0) {
     ProfileScope prof("kmap_insert_kernel", s);
-    kmap_insert_kernel<<<(unsigned)((n_in + 255) / 256), 256, 0, s>>>(in_coords, (int)n_in, slot_table, mask, cells, flags);
+    kmap_insert_kernel<<<(unsigned)((n_in + 255) / 256), 256, 0, s>>>(in_coords, (int)n_in, slot_table, buckets, cells, flags);
   }
   if (n_out > 0 && n_in > 0) {
     ProfileScope prof("kmap_lookup_kernel", s);
-    LookupArgs la{out_coords, (int)n_out, k_vol, stride, skip_offset, row_ld, slot_table, cells, mask, offs_dev,
+    LookupArgs la{out_coords, (int)n_out, k_vol, stride, skip_offset, row_ld, slot_table, cells, buckets, offs_dev,
                   rows, counts, totals, blocks, rmask_out, rmask_in, flags, host_dev};
     bool near = true;
     for (int q = 0; q < 3 * k_vol; ++q) near = near && offsets_host[q] >= -1 && offsets_host[q] <= 1;

@@ -151,3 +151,43 @@ def test_tiles_of_very_different_weight(oracle):
     vox = vox[np.lexsort(vox.T[::-1])]
     vox = np.concatenate([np.zeros((len(vox), cloud(1).shape[1] - 3), np.int32), vox], 1) if cloud(1).shape[1] > 3 else vox
     check(oracle, vox, vox, clouds.offsets_cube(3), 1, 64, 64)
+
+
+def alone(n, seed=5):
+    """Voxels with a block of 2 x 2 x 4 each, an eighth of the blocks of a cube or less: as many searches for a block that is
+    there as rows, and most others in vain."""
+    rng = np.random.default_rng(seed)
+    side = 2 * int(np.ceil(n ** (1 / 3))) + 1
+    at = np.sort(rng.choice(side ** 3, n, replace=False))
+    return (np.stack([at // side ** 2, at // side % side, at % side], 1) * [2, 2, 4] + rng.integers(0, [2, 2, 4], (n, 3))).astype(np.int32)
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 6, 7, 170, 171, 5461, 5462, 20001])
+def test_a_block_for_every_row(n):
+    """The block table as full as it gets, around sizes that fill its last bucket."""
+    import FGMS.nn as fnn
+    vox = alone(n)
+    c = torch.from_numpy(vox).cuda()
+    for offsets in (clouds.offsets_cube(3), clouds.offsets_cube(5)):
+        imap, omap, knnz, _ = clouds.build_kernel_map(vox, vox, offsets)
+        kmap = fnn.KernelMap.from_coords(c, c, offsets)
+        assert np.array_equal(kmap.in_map.cpu().numpy(), imap) and np.array_equal(kmap.out_map.cpu().numpy(), omap)
+        assert np.array_equal(kmap.kernel_nnz.numpy(), knnz)
+
+
+def test_thin_clouds_take_no_longer_at_one_size_than_at_the_next():
+    """Just below and just above 4/5 of 2^17 rows with a block each: the larger map is no cheaper.  (With a table of 2^n single slots,
+    5/4 a row at least, the smaller one took 6.6 times as long: chains of a hundred dependent probes.)"""
+    import FGMS.nn as fnn
+    offsets, best = clouds.offsets_cube(5), {}
+    coords = {n: torch.from_numpy(alone(n)).cuda() for n in (104000, 106000)}
+    for turn in range(6):
+        for n, c in coords.items():
+            start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(5):
+                fnn.KernelMap.from_coords(c, c, offsets).in_map
+            stop.record()
+            torch.cuda.synchronize()
+            best[n] = min(best.get(n, 1e9), start.elapsed_time(stop))
+    assert best[104000] < 2 * best[106000], best
