@@ -740,6 +740,13 @@ bool full_offset_pays(const GmsArgs &a, Route route) {
   return saved > costs + 2.5;
 }
 
+// That offset, or -1.  (A plan of another map, which the kernels that walk the lists do without, says nothing about these lists.)
+int full_offset_of(const GmsArgs &a, const Plan *plan) {
+  if (!plan || a.k_vol != plan->k_vol) return -1;
+  if (a.transpose_w) return a.n_dst == plan->n_in && a.n_src == plan->n_out ? plan->full_in : -1;
+  return a.n_dst == plan->n_out && a.n_src == plan->n_in ? plan->full_out : -1;
+}
+
 int run_gms_one(GmsArgs a, const Plan *plan) {
   if (plan) plan_touch(plan, a.stream);
   const bool dense = a.dense_k >= 0;
@@ -757,7 +764,7 @@ int run_gms_one(GmsArgs a, const Plan *plan) {
   // (these kernels add with atomics, several workgroups to a row.  Where the identity map, or the list of one offset, meets
   // every row once, its products are written in the place of the zeros.)
   const bool pairs = route == Route::kWide || route == Route::kPairs;
-  if (pairs && a.overwrite && !dense && plan && full_offset_pays(a, route)) a.first_offset = (a.transpose_w ? plan->full_in : plan->full_out) + 1;
+  if (pairs && a.overwrite && !dense && full_offset_pays(a, route)) a.first_offset = full_offset_of(a, plan) + 1;
   const bool written = pairs && a.overwrite && (a.first_offset || (dense && a.n_dense == a.n_dst));
   if (a.overwrite && !written && (pairs || route == Route::kGeneric)) {
     const int rc = zero_result();

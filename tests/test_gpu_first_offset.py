@@ -66,6 +66,27 @@ def test_whole_numbers(n, c_in, c_out, full, launches):
     plan.close()
 
 
+@pytest.mark.parametrize("c_in,c_out", [(256, 256), (256, 128)])
+@pytest.mark.parametrize("other", [(55000, 27), (52001, 32)], ids=["rows", "offsets"])
+def test_plan_of_another_map(other, c_in, c_out):
+    """Rows or offsets that do not fit the call's: what that plan says about an offset is not taken over."""
+    from fgms_amd import capi
+    capi.set_kernel_policy(0)
+    n = 52001
+    maps, others = thin_map(n, None), thin_map(other[0], other[1] - 1, other[1])
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(n)
+    few = lambda *s: (torch.randint(0, 64, s, generator=gen, device="cuda") < 3).half() - (torch.randint(0, 64, s, generator=gen, device="cuda") < 3).half()
+    x, w, g = few(n, c_in), few(27, c_in, c_out), few(n, c_out)
+    want = exact(x.float(), w.float(), g.float(), maps[0].tolist(), maps[1].long(), maps[2].long())
+    plan = capi.Plan(*others, other[0], other[0])
+    out, gin = torch.full_like(g, float("nan")), torch.full_like(x, float("nan"))
+    capi.conv_fwd(x, w, out, *maps, plan=plan)
+    capi.conv_bwd(g, x, w, gin, None, *maps, plan=plan)
+    assert torch.equal(out.double(), want[0]) and torch.equal(gin.double(), want[1])
+    plan.close()
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 @pytest.mark.parametrize("c_in,c_out", [(64, 64), (128, 256), (32, 96)])
 def test_identity_map_added_and_written(c_in, c_out, dtype):
