@@ -82,7 +82,8 @@ struct GmsArgs {
   SideJob side;            // rides along with the launch (not the shape-agnostic kernel's)
 };
 // What a launch of a pair-stationary kernel walks: all pairs, the pairs of all offsets but one, or one offset's list (or the identity
-// map), whose rows nothing else of the launch meets.
+// map), entry i of which meets row i.  The lists may be others than the plan has seen (rewritten in place): kWalkOwn clears a row whose
+// entry is of another one, and kWalkRest adds what kWalkOwn has left out (see Strays).
 enum { kWalkAll = 0, kWalkRest = 1, kWalkOwn = 2 };
 // How it leaves its tiles.
 enum { kTileAdd = 0, kTileAtomic = 1, kTileStore = 2 };
@@ -120,6 +121,7 @@ struct WgradArgs {
 };
 
 constexpr int kPlanFlags = 32;      // ints the plan build reports back (see fgms_plan.hip)
+constexpr int kFlagInput = 9;       // flags[9]: an offset with as many pairs as input rows does not list these in order (or nobody looked)
 constexpr int kFlagStale = 13;      // flags[13]: a later check found another fingerprint (fgms_plan_check)
 constexpr int kFlagCentre = 14;     // flags[14]: see Plan::centre_line
 constexpr int kFlagFull = 15;       // flags[15]: see Plan::full_out (+ 1, that of the input side << 8)
@@ -210,7 +212,7 @@ struct Plan {
   // of the tables then hold the row order, through which every row is its own neighbour.  No mask names
   // the offset, so that only a launch that asks for it (GmsArgs::centre) sees them.
   bool centre_line;
-  // An offset that meets every output (input) row exactly once, as a submanifold map's middle one does; -1: none.
+  // An offset that meets every output (input) row exactly once and lists them in order, as a submanifold map's middle one does; -1: none.
   int full_out, full_in;
   bool fwd_ok;        // no offset maps two pairs onto one output row
   bool dgrad_ok;      // no offset maps two pairs from one input row

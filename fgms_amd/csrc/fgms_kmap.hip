@@ -538,7 +538,7 @@ __global__ __launch_bounds__(256) void kmap_lists_kernel(ListArgs a, int list_bl
 struct SizeArgs {
   const int32_t *totals;
   int32_t *kernel_nnz, *kpos, *qkpos;      // (qkpos: nullptr: not wanted)
-  int *plan_flags;                         // flags[12] of the plan: its pair count
+  int *plan_flags;                         // flags[12] of the plan: its pair count; flags[9]
   int *host;                               // pinned
 };
 __global__ __launch_bounds__(kSortThreads) void kmap_sizes_kernel(SizeArgs a, SortArgs sort) {
@@ -590,6 +590,7 @@ __global__ __launch_bounds__(kSortThreads) void kmap_sizes_kernel(SizeArgs a, So
     a.kpos[k_vol] = pairs;
     if (a.qkpos) a.qkpos[0] = 0;
     a.plan_flags[12] = pairs;
+    a.plan_flags[kFlagInput] = sort.side[1].n > 0;      // (a mirrored map's middle offset has every row for its own neighbour)
     a.host[4] = pairs;
   }
   __threadfence_system();

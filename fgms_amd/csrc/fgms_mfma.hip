@@ -27,6 +27,7 @@
 // operand do not collide on banks.
 #include <stdlib.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "fgms_device.h"
@@ -473,17 +474,21 @@ __global__ __launch_bounds__(kThreads) void gms_pairs_kernel(
   const int nt0 = blockIdx.y * NT;
   const size_t packed_per_k = (size_t)c_src * c_dst / E;  // chunks
 
+  Strays strays;
+  if constexpr (WALK == kWalkRest) {
+    const int blocks = gridDim.x - side.blocks;
+    strays = look_for_strays(kpos, smap, offset, block_x);
+    tiles_per_wg = rest_tiles(kpos, k_vol, offset, kTileRows, tiles_per_wg, blocks);
+  }
   int cur_k = -1;
   const int t_begin = block_x * tiles_per_wg;
   for (int t = t_begin; t < t_begin + tiles_per_wg; ++t) {
     int k, first, count;
     if constexpr (WALK == kWalkOwn) {
       k = offset >> 1;
-      const int rows = gmap ? min(dense_rows, kpos[k + 1] - kpos[k]) : dense_rows;
       first = t * kTileRows;
-      if (first >= rows) break;
-      count = min(kTileRows, rows - first);
-      if (gmap) first += kpos[k];
+      if (first >= dense_rows) break;
+      count = min(kTileRows, dense_rows - first);
     } else if (!locate_tile(kpos, k_vol, kTileRows, t, k, first, count, WALK == kWalkRest ? offset : -1)) {
       break;
     }
@@ -501,8 +506,14 @@ __global__ __launch_bounds__(kThreads) void gms_pairs_kernel(
     if (nrows <= 0) continue;
     const bool live = lane < nrows;
     const int j = first + wfirst + lane;
-    gidx[lane] = !live ? -1 : (gmap ? gmap[j] : j);
-    sidx[lane] = !live ? -1 : (smap ? smap[j] : j);
+    if constexpr (WALK == kWalkOwn) {
+      const int source = live ? own_source(kpos, gmap, smap, k, j) : -1;
+      gidx[lane] = source;
+      sidx[lane] = live ? own_row(source, j) : -1;
+    } else {
+      gidx[lane] = !live ? -1 : (gmap ? gmap[j] : j);
+      sidx[lane] = !live ? -1 : (smap ? smap[j] : j);
+    }
     wave_lds_fence();
 
     float16v acc[2][NT];
@@ -529,8 +540,13 @@ __global__ __launch_bounds__(kThreads) void gms_pairs_kernel(
     if constexpr (WALK != kWalkOwn) write_tile<T, NT, kTileAtomic>(acc, dst, sidx, c_dst, nt0 * 32, lane);
     else if (offset & 1) write_tile<T, NT, kTileStore>(acc, dst, sidx, c_dst, nt0 * 32, lane);
     else write_tile<T, NT, kTileAdd>(acc, dst, sidx, c_dst, nt0 * 32, lane);
+    if constexpr (WALK == kWalkOwn && sizeof(T) == 2)
+      if (gmap) clear_rows<NT>(dst, sidx, c_dst, nt0 * 32, lane);
     wave_lds_fence();
   }
+  if constexpr (WALK == kWalkRest)
+    add_strays<S>(strays, src, reinterpret_cast<const int4v *>(packed) + packed_per_k * offset, dst, gmap, smap, dense_rows, c_src, c_dst,
+                  nt0 * 32, NT * 32, gridDim.x - side.blocks);
 }
 
 // ---------------------------------------------------------------------------
@@ -1233,8 +1249,7 @@ int launch_pairs(const GmsArgs &a, const Shape &s) {
   SideJob side = a.side;
   for (int part = a.first_offset ? 0 : 1; part < 2; ++part) {
     const bool dense = part == 0 || a.dense_k >= 0;
-    const int64_t rows = part == 0 ? a.n_dst : dense ? a.n_dense : a.n_pairs - (a.first_offset ? a.n_dst : 0);
-    if (rows <= 0 && part == 1 && a.first_offset) continue;
+    const int64_t rows = part == 0 ? a.n_dst : dense ? a.n_dense : std::max<int64_t>(a.n_pairs - (a.first_offset ? a.n_dst : 0), 0);
     constexpr int kRest = sizeof(T) == 2 ? kWalkRest : kWalkAll;      // (first offsets: fp16)
     auto kern = dense            ? (split ? gms_pairs_kernel<T, NT, S, kCanSplit, kWalkOwn> : gms_pairs_kernel<T, NT, S, false, kWalkOwn>)
                 : a.first_offset ? gms_pairs_kernel<T, NT, S, false, kRest>
@@ -1251,7 +1266,7 @@ int launch_pairs(const GmsArgs &a, const Shape &s) {
                       a.stream);
     kern<<<dim3(gx + (unsigned)side.blocks, (unsigned)(s.c_dst / (32 * NT))), kThreads, s.lds_bytes, a.stream>>>(
         (const T *)a.src, packed, (T *)a.dst, a.kpos, a.gmap, a.smap, a.k_vol, s.c_src, s.c_dst,
-        tiles_per_wg, walk_offset(a, part == 0), (int)rows, side);
+        tiles_per_wg, walk_offset(a, part == 0), (int)(dense ? rows : a.n_dst), side);
     side = SideJob{};
   }
   FGMS_HIP_TRY(hipGetLastError());

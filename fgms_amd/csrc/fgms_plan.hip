@@ -35,7 +35,7 @@ __global__ __launch_bounds__(256) void fills_kernel(FillBatch batch) {
 // an output row; flags[2]: two pairs of one offset share an input row;
 // flags[3]: inside some offset the pairs are not ordered by output row;
 // flags[4], flags[5]: (64-position block, offset) combinations in use, output / input side;
-// flags[6..9]: unused; flags[10], flags[11]: offset bits
+// flags[6..8]: unused; flags[9]: see kFlagInput; flags[10], flags[11]: offset bits
 // set over all row masks of the output / input side; flags[12]: pairs in the map.  Two pairs of
 // one offset that share a row set one bit between them, so a side whose bits do not add up to
 // the pair count has such a pair (what flags[1] / flags[2] used to say).
@@ -71,6 +71,7 @@ __global__ void pair_masks_kernel(const int32_t *__restrict__ kpos, const int32_
   }
   const int before = j > kpos[k] ? omap[j - 1] : -1;
   if (before > o) flags[3] = 1;
+  if (i != j - kpos[k] && kpos[k + 1] - kpos[k] == n_in) flags[kFlagInput] = 1;
   // the bounds of the weight gradient's row bands that fall between this pair and the one before it
   // (pre-set to 0; meaningful where the pairs are ordered by output row, in bounds always)
   if (band_start) {
@@ -928,8 +929,8 @@ const Plan *plan_resolve(fgms_plan_t *plan, hipStream_t stream, int *rc) {
       p->ordered = !h[0] && !h[3];
       p->bands_ok = p->has_bands && p->ordered;
       p->centre_line = p->has_tables && h[kFlagCentre];
-      p->full_out = p->fwd_ok ? (h[kFlagFull] & 255) - 1 : -1;
-      p->full_in = p->dgrad_ok ? (h[kFlagFull] >> 8) - 1 : -1;
+      p->full_out = p->fwd_ok && p->ordered ? (h[kFlagFull] & 255) - 1 : -1;
+      p->full_in = p->dgrad_ok && !h[kFlagInput] ? (h[kFlagFull] >> 8) - 1 : -1;
       p->stages_out = h[4];
       p->stages_in = h[5];
       p->pairs_counted = p->has_tables ? h[12] : p->n_pairs;

@@ -265,7 +265,7 @@ __device__ __forceinline__ void sort_window_body(const SortArgs &a, int side, in
   int bits = 0, row_bits = 0;
   const int centre = empty_centre(a.kpos, a.k_vol);
   if (window == 0 && side == 0 && wave == 0) {
-    // (as many pairs as rows; that they are of different rows is for the reader of the flags to ask)
+    // (as many pairs as rows; that they are of different rows, and in order, is for the reader of the flags to ask)
     const int size = lane < a.k_vol ? a.kpos[lane + 1] - a.kpos[lane] : -1;
     const unsigned long long out = __ballot(size == a.side[0].n), in = __ballot(size == (a.side[1].n > 0 ? a.side[1].n : a.side[0].n));
     if (lane == 0) {

@@ -78,6 +78,81 @@ __device__ __forceinline__ void zero_rows(T *__restrict__ dst, const int *__rest
   }
 }
 
+// kWalkOwn: the source row of result row `row`, -1 if the list's entry there is of another one or there is none.
+__device__ __forceinline__ int own_source(const int32_t *__restrict__ kpos, const int32_t *__restrict__ gmap,
+                                          const int32_t *__restrict__ smap, int k, int row) {
+  if (!gmap) return row;
+  const int at = kpos[k] + row, safe = at < kpos[k + 1] ? at : 0;      // (both loads at once)
+  const int source = gmap[safe], meets = smap[safe];
+  return at < kpos[k + 1] && meets == row ? source : -1;
+}
+// ... its place in the rows that write_tile writes: not there, and for clear_rows to find, if it has no source.
+__device__ __forceinline__ int own_row(int source, int row) { return source >= 0 ? row : -2 - row; }
+
+// Clears those rows, of the 64 of a wave.
+template <int NT>
+__device__ __forceinline__ void clear_rows(__half *__restrict__ dst, const int *__restrict__ rows, int c_dst, int cd0, int lane) {
+  if (!__builtin_amdgcn_ballot_w64(rows[lane] < -1)) [[likely]] return;
+  constexpr int CH = NT * 16;      // pairs of columns
+#pragma unroll 1
+  for (int e = lane; e < 64 * CH; e += 64) {
+    const int row = -2 - rows[e / CH];
+    if (row >= 0) *reinterpret_cast<__half2 *>(dst + (size_t)row * c_dst + cd0 + e % CH * 2) = __half2{};
+  }
+}
+
+// kWalkRest: entries of the left-out offset that kWalkOwn has left out too, because entry i is not of row i: none as long as the lists
+// are those the plan was made from.  Every workgroup looks at 256 of them (and 256 more `blocks` further on, ...), a load each thread
+// that is in flight while the workgroup walks its tiles; a wave that finds some adds their products, `cols` columns from cd0 on, on the
+// vector ALUs.
+constexpr int kStrayChunk = 256;
+struct Strays {
+  int at, size;             // the offset's entries
+  int i, row;               // this thread's first one, and the row it meets
+};
+__device__ __forceinline__ Strays look_for_strays(const int32_t *__restrict__ kpos, const int32_t *__restrict__ smap, int k, int block) {
+  Strays s;
+  s.at = kpos[k];
+  s.size = threadIdx.x < kStrayChunk ? kpos[k + 1] - s.at : 0;
+  s.i = block * kStrayChunk + threadIdx.x;
+  s.row = s.i < s.size ? smap[s.at + s.i] : -1;
+  return s;
+}
+template <int S>
+__device__ __forceinline__ void add_strays(Strays s, const __half *__restrict__ src, const int4v *__restrict__ packed_k,
+                                           __half *__restrict__ dst, const int32_t *__restrict__ gmap, const int32_t *__restrict__ smap,
+                                           int n_dst, int c_src, int c_dst, int cd0, int cols, int blocks) {
+  const __half *const w = reinterpret_cast<const __half *>(packed_k);
+  const int lane = threadIdx.x % 64, nts = c_dst / 32;
+  while (__builtin_amdgcn_ballot_w64(s.i < s.size)) {
+    unsigned long long found = __builtin_amdgcn_ballot_w64(s.i < s.size && (s.row != s.i || s.i >= n_dst));
+    for (; found; found &= found - 1) {
+      const int from = __builtin_ctzll(found), row = __shfl(s.row, from);
+      const __half *const x = src + (size_t)gmap[s.at + __shfl(s.i, from)] * c_src;
+#pragma unroll 1
+      for (int col = cd0 + lane * 2; col < cd0 + cols; col += 128) {
+        float lo = 0.f, hi = 0.f;
+#pragma unroll 1
+        for (int c = 0; c < c_src; ++c) {      // (as pack_weight_elements lays them)
+          const int chunk = c / 8 % (2 * S), q = c / (16 * S) * S + chunk % S;
+          const __half *const p = w + (((size_t)q * nts + col / 32) * 64 + chunk / S * 32 + col % 32) * 8 + c % 8;
+          const float v = __half2float(x[c]);
+          lo = __builtin_fmaf(v, __half2float(p[0]), lo);
+          hi = __builtin_fmaf(v, __half2float(p[8]), hi);
+        }
+        atomic_add_pk(dst + (size_t)row * c_dst + col, lo, hi);
+      }
+    }
+    s.i = s.i < s.size - blocks * kStrayChunk ? s.i + blocks * kStrayChunk : s.size;
+    s.row = s.i < s.size ? smap[s.at + s.i] : -1;
+  }
+}
+// Tiles a workgroup walks: more than the launch has planned for if the other offsets have got more pairs since.
+__device__ __forceinline__ int rest_tiles(const int32_t *__restrict__ kpos, int k_vol, int k, int rows, int planned, int blocks) {
+  const int rest = (kpos[k_vol] - kpos[0] - (kpos[k + 1] - kpos[k])) / rows + k_vol;
+  return rest <= planned * blocks ? planned : (rest + blocks - 1) / blocks;
+}
+
 // Writes a wave's accumulators.  Accumulator register r of lane l holds row
 // (r / 4) * 8 + (l / 32) * 4 + r % 4 and column l % 32 of its 32x32 tile.  For
 // fp16 two lanes swap one value each so that every lane owns two neighbouring

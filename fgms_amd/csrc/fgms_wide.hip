@@ -13,6 +13,8 @@
 // next tile if need be, are in flight while the current one is multiplied.  The reference
 // re-gathers per column tile as well (backend/spconv.cuh:1397-1449 walks its 64- or
 // 128-column blocks in blockIdx.y).
+#include <algorithm>
+
 #include "fgms_device.h"
 #include "fgms_internal.h"
 #include "fgms_mma.h"
@@ -60,11 +62,9 @@ __global__ __launch_bounds__(kWideThreads) void gms_wide_kernel(
   auto tile_at = [&](int t, int &k, int &first, int &count) {
     if constexpr (WALK == kWalkOwn) {
       k = offset >> 1;
-      const int rows = gmap ? min(dense_rows, kpos[k + 1] - kpos[k]) : dense_rows;
       first = t * kWideRows;
-      count = min(kWideRows, rows - first);
-      if (gmap) first += kpos[k];
-      return t * kWideRows < rows;
+      count = min(kWideRows, dense_rows - first);
+      return first < dense_rows;
     }
     return locate_tile(kpos, k_vol, kWideRows, t, k, first, count, WALK == kWalkRest ? offset : -1);
   };
@@ -73,8 +73,14 @@ __global__ __launch_bounds__(kWideThreads) void gms_wide_kernel(
     if (tid < kWideRows) {
       const bool live = tid < count;
       const int j = first + tid;
-      gidx[par * kWideRows + tid] = !live ? -1 : (gmap ? gmap[j] : j);
-      sidx[par * kWideRows + tid] = !live ? -1 : (smap ? smap[j] : j);
+      if constexpr (WALK == kWalkOwn) {
+        const int source = live ? own_source(kpos, gmap, smap, offset >> 1, j) : -1;
+        gidx[par * kWideRows + tid] = source;
+        sidx[par * kWideRows + tid] = live ? own_row(source, j) : -1;
+      } else {
+        gidx[par * kWideRows + tid] = !live ? -1 : (gmap ? gmap[j] : j);
+        sidx[par * kWideRows + tid] = !live ? -1 : (smap ? smap[j] : j);
+      }
     }
   };
   int4v av[2], wv[2];
@@ -110,10 +116,20 @@ __global__ __launch_bounds__(kWideThreads) void gms_wide_kernel(
   };
   clear();
 
+  Strays strays;
+  if constexpr (WALK == kWalkRest) {
+    const int blocks = gridDim.x - side.blocks;
+    strays = look_for_strays(kpos, smap, offset, block_x);
+    tiles_per_wg = rest_tiles(kpos, k_vol, offset, kWideRows, tiles_per_wg, blocks);
+  }
+  auto finish = [&]() {
+    if constexpr (WALK == kWalkRest)
+      add_strays<S>(strays, src, packed + packed_per_k * offset, dst, gmap, smap, dense_rows, c_src, c_dst, nt0 * 32, kWideCols, gridDim.x - side.blocks);
+  };
   int t = block_x * tiles_per_wg;
   const int t_end = t + tiles_per_wg;
   int k, first, count;
-  if (!tile_at(t, k, first, count)) return;
+  if (!tile_at(t, k, first, count)) return finish();
   load_indices(0, first, count);
   __syncthreads();
   issue(0, k, 0);
@@ -152,6 +168,8 @@ __global__ __launch_bounds__(kWideThreads) void gms_wide_kernel(
       if constexpr (WALK != kWalkOwn) write_tile<__half, 2, kTileAtomic>(acc, dst, rows, c_dst, nt0 * 32 + cg * 64, lane);
       else if (offset & 1) write_tile<__half, 2, kTileStore>(acc, dst, rows, c_dst, nt0 * 32 + cg * 64, lane);
       else write_tile<__half, 2, kTileAdd>(acc, dst, rows, c_dst, nt0 * 32 + cg * 64, lane);
+      if constexpr (WALK == kWalkOwn)
+        if (gmap) clear_rows<2>(dst, rows, c_dst, nt0 * 32 + cg * 64, lane);
       clear();
     }
     if (!has_next) break;
@@ -169,6 +187,7 @@ __global__ __launch_bounds__(kWideThreads) void gms_wide_kernel(
       ++slab;
     }
   }
+  finish();
 }
 
 }  // namespace
@@ -197,8 +216,8 @@ int launch_wide_gms(const GmsArgs &a) {
   SideJob side = a.side;
   for (int part = a.first_offset ? 0 : 1; part < 2; ++part) {
     const bool dense = part == 0 || a.dense_k >= 0;
-    const int64_t rows = part == 0 ? a.n_dst : dense ? a.n_dense : a.n_pairs - (a.first_offset ? a.n_dst : 0);
-    if (rows <= 0) continue;
+    const int64_t rows = part == 0 ? a.n_dst : dense ? a.n_dense : std::max<int64_t>(a.n_pairs - (a.first_offset ? a.n_dst : 0), 0);
+    if (rows == 0 && !a.first_offset) continue;
     const int64_t tiles = (rows + kWideRows - 1) / kWideRows + (dense ? 0 : a.k_vol);
     // one workgroup per CU at a time: each takes a contiguous run of tiles (mostly one offset,
     // whose weights then stay in the L2 between its tiles)
@@ -212,7 +231,7 @@ int launch_wide_gms(const GmsArgs &a) {
     ProfileScope prof(a.transpose_w ? "gms_wide_kernel(dgrad)" : "gms_wide_kernel(fwd)", a.stream);
     kern<<<dim3(gx + (unsigned)side.blocks, (unsigned)(c_dst / kWideCols)), kWideThreads, lds_bytes, a.stream>>>(
         (const __half *)a.src, (const int4v *)packed, (__half *)a.dst, a.kpos, a.gmap, a.smap, a.k_vol, c_src,
-        c_dst, tiles_per_wg, walk_offset(a, part == 0), (int)rows, side);
+        c_dst, tiles_per_wg, walk_offset(a, part == 0), (int)(dense ? rows : a.n_dst), side);
     side = SideJob{};
   }
   FGMS_HIP_TRY(hipGetLastError());

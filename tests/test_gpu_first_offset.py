@@ -66,6 +66,58 @@ def test_whole_numbers(n, c_in, c_out, full, launches):
     plan.close()
 
 
+@pytest.mark.parametrize("how", ["shuffled", "fewer", "more", "none"])
+@pytest.mark.parametrize("c_in,c_out", [(256, 256), (128, 128), (256, 128), (128, 256)])
+def test_lists_rewritten_under_the_plan(c_in, c_out, how):
+    """The offset that met every row, in order, when the plan was made, meets others since (in any order, not all of them, some of them
+    twice, or none), and the other offsets have its pairs: the sums are those of the lists as they are."""
+    from fgms_amd import capi
+    capi.set_kernel_policy(0)
+    n, full = 52001, 13
+    rng = np.random.default_rng(c_in + c_out)
+    sizes = [n if k == full else n // 8 + k for k in range(27)]
+    ins, outs = ([np.arange(n) if k == full else pick(rng.permutation(n)[:m]) for k, m in enumerate(sizes)] for pick in (lambda r: r, np.sort))
+    lists = lambda parts: torch.from_numpy(np.concatenate(parts).astype(np.int32)).cuda()
+    starts = lambda parts: torch.from_numpy(np.cumsum([0] + [len(p) for p in parts]).astype(np.int32)).cuda()
+    maps = starts(outs), lists(ins), lists(outs)
+    plan = capi.Plan(*maps, n, n)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(n)
+    few = lambda *s: (torch.randint(0, 64, s, generator=gen, device="cuda") < 3).half() - (torch.randint(0, 64, s, generator=gen, device="cuda") < 3).half()
+    x, w, g = few(n, c_in), few(27, c_in, c_out), few(n, c_out)
+
+    def check(beyond=False):
+        m = tuple(t.long() for t in maps[1:])
+        kpos = maps[0].tolist()
+        want = exact(x.float(), w.float(), g.float(), kpos, *m)
+        hit = [torch.zeros(n, dtype=torch.bool, device="cuda") for _ in range(2)]
+        if beyond:
+            w[full, 3, 5], w[full, 2, 1] = float("inf"), float("nan")
+            for h, q in zip(hit, (m[1], m[0])):
+                h[q[kpos[full]:kpos[full + 1]]] = True
+        out, gin = torch.full_like(g, float("nan")), torch.full_like(x, float("nan"))
+        capi.conv_fwd(x, w, out, *maps, plan=plan)
+        capi.conv_bwd(g, x, w, gin, None, *maps, plan=plan)
+        for got, ref, h in ((out, want[0], hit[0]), (gin, want[1], hit[1])):
+            assert torch.equal(got[~h].double(), ref[~h])
+
+    check()
+    changed = {"shuffled": n, "fewer": n - 777, "more": n + 555, "none": 0}[how]
+    rows = [rng.permutation(n) for _ in range(2)]
+    rows = [np.concatenate([r, r[:555]])[:changed] for r in rows]
+    extra = sizes[full] - changed
+    ins[full], outs[full] = rows
+    if extra < 0:
+        ins[0], outs[0] = ins[0][:extra], outs[0][:extra]
+    else:
+        ins[20], outs[20] = (np.concatenate([q[20], rng.permutation(n)[:extra]]) for q in (ins, outs))
+    for t, new in zip(maps, (starts(outs), lists(ins), lists(outs))):
+        t.copy_(new)
+    check()
+    check(beyond=True)
+    plan.close()
+
+
 @pytest.mark.parametrize("c_in,c_out", [(256, 256), (256, 128)])
 @pytest.mark.parametrize("other", [(55000, 27), (52001, 32)], ids=["rows", "offsets"])
 def test_plan_of_another_map(other, c_in, c_out):
