@@ -506,12 +506,13 @@ bool sparse_rows(const GmsArgs &a, const Plan *plan, bool masked = false) {
 
 enum class Route { kNarrow, kSkinny, kRows, kPairView, kWide, kPairs, kGeneric };
 
-// Which kernel a forward / input-gradient pass takes.
-Route route_of(const GmsArgs &a, const Plan *plan) {
+// Which kernel a forward / input-gradient pass takes.  (A question only, asked for estimates too: a pair view that is not there yet is
+// built by the call that walks it.  with_view = false: it could not be had.)
+Route route_of(const GmsArgs &a, const Plan *plan, bool with_view = true) {
   const bool dense = a.dense_k >= 0;
   if (g_policy == 1) return Route::kGeneric;
-  const bool pair_view = !dense && pair_view_gms_supported(a, plan);
-  if (g_policy == 5 && pair_view && plan_pair_view(plan, a)) return Route::kPairView;
+  const bool pair_view = !dense && with_view && pair_view_gms_supported(a, plan);
+  if (g_policy == 5 && pair_view) return Route::kPairView;
   // (16 -> 64 channels fill the output-stationary kernel's tiles: 150 k voxels 20 us, 39 us here; the others 1.1 .. 3 times
   // faster than on the vector ALUs from 2 k to 150 k voxels)
   if (!dense && (g_policy == 0 || g_policy == 4) && narrow_gms_supported(a, plan) &&
@@ -527,7 +528,7 @@ Route route_of(const GmsArgs &a, const Plan *plan) {
   // block's weights of one offset.  Measured (same clouds): fp32 a tie up to 128 channels,
   // 245 against 341 us at 256 -> 256 over 50 k voxels; fp16 14.2 against 18.3 us at 64
   // channels over 35 k voxels, a tie from 128 channels on (96.6 against 96.3 us at 256).
-  if (g_policy == 0 && pair_view && (a.dtype == FGMS_F32 || (a.transpose_w ? a.c_out : a.c_in) <= 64) && plan_pair_view(plan, a))
+  if (g_policy == 0 && pair_view && (a.dtype == FGMS_F32 || (a.transpose_w ? a.c_out : a.c_in) <= 64))
     return Route::kPairView;
   if (g_policy == 0 && wide_gms_supported(a)) return Route::kWide;
   return mfma_gms_supported(a) ? Route::kPairs : Route::kGeneric;
@@ -754,7 +755,8 @@ int run_gms_one(GmsArgs a, const Plan *plan) {
     return launch_fill_zero(a.dst, (size_t)a.n_dst * (a.transpose_w ? a.c_in : a.c_out) * elem_size(a.dtype), a.stream);
   };
   if ((!dense && a.n_pairs == 0) || (dense && a.n_dense == 0)) return a.overwrite ? zero_result() : FGMS_OK;
-  const Route route = route_of(a, plan);
+  Route route = route_of(a, plan);
+  if (route == Route::kPairView && !plan_pair_view(plan, a)) route = route_of(a, plan, false);
   if (a.centre && route != Route::kRows) {      // (the copies it was to run over could not be had)
     const int rc = run_centre(a);
     if (rc != FGMS_OK) return rc;

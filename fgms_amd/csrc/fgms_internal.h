@@ -207,7 +207,7 @@ struct Plan {
   // atomics.  nullptr: not built yet (plan_pair_view).
   int32_t *pv_in, *pv_out;        // [pv_rows]
   unsigned long long *pv_mask;    // [pv_rows / 64]
-  int64_t pv_rows;                // a multiple of 256; 0: this map has none
+  int64_t pv_rows;                // a multiple of 256: what it has once built; 0: this map has none
   // The middle offset of an odd number of them has no pairs (the caller keeps it out of the lists): its lines
   // of the tables then hold the row order, through which every row is its own neighbour.  No mask names
   // the offset, so that only a launch that asks for it (GmsArgs::centre) sees them.

@@ -1878,11 +1878,11 @@ bool pair_view_gms_supported(const GmsArgs &a, const Plan *p) {
 }
 
 int launch_pair_view_gms(const GmsArgs &a, const Plan *p) {
-  if (!pair_view_gms_supported(a, p) || !plan_pair_view(p, a)) {
+  if (!pair_view_gms_supported(a, p) || !p->pv_in) {      // (plan_pair_view comes first)
     set_error("launch_pair_view_gms: unsupported shape or plan");
     return FGMS_E_INVALID;
   }
-  // (the view was built on the stream that first resolved the plan)
+  // (the view was built on the stream of the first call that walked it)
   if (p->pv_ready && a.stream != p->pv_stream) FGMS_HIP_TRY(hipStreamWaitEvent(a.stream, p->pv_ready, 0));
   // the virtual rows stand in for the destination rows: tiles, the in-range test and the
   // choice of the wave tile's width go by their number

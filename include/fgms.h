@@ -113,8 +113,9 @@ int fgms_plan_usable(const fgms_plan_t *plan, int for_dgrad);
 /* What the build counted (no counterpart in the reference): stats[0] = pairs in the map,
  * stats[1] / stats[2] = (64-row block, offset) combinations with at least one pair in the
  * forward / input-gradient direction (the output-stationary kernels run 64 row slots for
- * each, so stats[1] * 64 / stats[0] is their row slots per pair), stats[3] = rows of the
- * pair view (0: the plan keeps none).  Returns FGMS_OK or FGMS_E_INVALID. */
+ * each, so stats[1] * 64 / stats[0] is their row slots per pair), stats[3] = rows that the
+ * pair view has once a layer has asked for it (0: the map is too dense for one, or there was
+ * no memory for it).  Returns FGMS_OK or FGMS_E_INVALID. */
 int fgms_plan_stats(const fgms_plan_t *plan, int64_t stats[4]);
 
 /*

@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from fgms_amd import clouds
+from tests import gpu_trace
 from tests import gpu_util as G
 
 pytestmark = pytest.mark.gpu
@@ -313,3 +314,26 @@ def test_pair_view_is_built_by_the_first_layer_that_walks_it(capi, oracle):
         G.assert_close(out.cpu().numpy(), want, "fp32", "through the plan")
     view.close()
     plan.close()
+
+
+def test_pair_view_is_not_built_for_an_estimate(capi, oracle):
+    """fp32 layers over a thin map that end on another kernel, however their prices over the view compare (20 channels out: the vector ALUs
+    as long as the padded copies' launches cost more; a backward call's masked tiles), build no view; one that walks it does, once."""
+    vox = clouds.cloud_indoor(clouds.rng_for(2), target=60000)
+    rng = np.random.default_rng(6)
+    vox = np.ascontiguousarray(vox[np.sort(rng.permutation(len(vox))[:1500])])
+    for shape, walks in (((32, 20), False), ((24, 40), False), ((128, 128), True)):
+        L = clouds.submanifold_case(vox, *shape, np.float32, rng)
+        D = G.to_dev(L)
+        maps = (D["kpos"], D["imap"], D["omap"])
+        plan = capi.Plan(*maps, D["n_in"], D["n_out"])
+        plan.stats()                                                 # (the build has ended)
+        out, gin, gw = (torch.empty_like(D[q]) for q in ("out_grad", "in_feats", "kernel"))
+
+        def both():
+            capi.conv_fwd(D["in_feats"], D["kernel"], out, *maps, plan=plan)
+            capi.conv_bwd(D["out_grad"], D["in_feats"], D["kernel"], gin, gw, *maps, plan=plan)
+
+        assert [gpu_trace.kernels(both).count("pair_view_kernel") for _ in range(2)] == [int(walks), 0], shape
+        G.assert_close(out.cpu().numpy(), oracle.c_fwd(L["in_feats"], L["kernel"], L["knnz"], L["imap"], L["omap"], L["n_out"]), "fp32", "fwd")
+        plan.close()
