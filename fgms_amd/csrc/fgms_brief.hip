@@ -335,7 +335,7 @@ int launch_brief_gms(const GmsArgs &a, const Plan *p) {
   const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kern), lds);
   if (rc != FGMS_OK) return rc;
   {
-    ProfileScope prof("gms_rows_kernel(fwd)", a.stream);
+    ProfileScope prof("gms_brief_kernel", a.stream);
     kern<<<dim3((unsigned)((a.n_dst + kBriefRows - 1) / kBriefRows) + (unsigned)b.side.blocks, (unsigned)((a.c_out + 31) / 32)), kBriefWaves * 64, lds, a.stream>>>(b);
   }
   FGMS_HIP_TRY(hipGetLastError());
@@ -363,7 +363,7 @@ int launch_held_gms(const GmsArgs &a, const Plan *p) {
   if (rc != FGMS_OK) return rc;
   const unsigned tiles = p->tile_out ? (unsigned)p->tile_grid_out : (unsigned)((a.n_dst + kHeldWaves * 32 - 1) / (kHeldWaves * 32));
   {
-    ProfileScope prof("gms_rows_kernel(fwd)", a.stream);
+    ProfileScope prof("gms_held_kernel", a.stream);
     kern<<<dim3(tiles + (unsigned)b.side.blocks, (unsigned)((a.c_out + 31) / 32)), kHeldWaves * 64, lds, a.stream>>>(b, p->tile_out);
   }
   FGMS_HIP_TRY(hipGetLastError());

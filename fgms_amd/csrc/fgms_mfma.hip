@@ -1455,7 +1455,7 @@ int launch_rows(const GmsArgs &a, const Shape &s, const int32_t *nbr,
   const unsigned gz = rg.gz;
   {
     ProfileScope prof(pair_view  ? (a.transpose_w ? "gms_rows_kernel(dgrad, pair view)" : "gms_rows_kernel(fwd, pair view)")
-                      : RAGGED && !TAILS ? (raw == 3 ? "gms_rows_kernel(fwd, masked, bf16x3)" : "gms_rows_kernel(fwd, masked)")
+                      : RAGGED   ? (raw == 3 ? "gms_rows_kernel(fwd, masked, bf16x3)" : "gms_rows_kernel(fwd, masked)")
                       : raw == 4 ? "gms_rows_kernel(dgrad, bf16x3)"
                       : raw == 3 ? "gms_rows_kernel(fwd, bf16x3)"
                       : a.transpose_w ? "gms_rows_kernel(dgrad)" : "gms_rows_kernel(fwd)",

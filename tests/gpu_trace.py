@@ -1,5 +1,5 @@
 """Names of the device kernels that a call runs, as the tracer of torch.profiler sees them (the library's own profile records
-name a launch by the pass it is of)."""
+name the main launches only)."""
 import re
 
 import torch

@@ -10,9 +10,22 @@ from tests.test_gpu_fp32_parts import exact
 
 pytestmark = pytest.mark.gpu
 
+BRIEF, HELD = "gms_brief_kernel", "gms_held_kernel"
 CUBE, WIDE = clouds.offsets_cube(3).tolist(), clouds.offsets_cube(5).tolist()
 OFFSETS = {"cube": CUBE, "17": WIDE[54:71], "32": WIDE[40:72], "gaps": [[900, 900, 900]] + CUBE[:9] + [[901, 900, 900]] + CUBE[9:]}
 FEW = {"9": CUBE[9:18], "16": CUBE[5:21], **OFFSETS}
+
+
+def assert_runs(kernel, call):
+    """One launch, and of this kernel; None: neither of the two."""
+    from fgms_amd import capi
+    capi.profile_reset()
+    capi.profile_enable(True)
+    call()
+    capi.profile_enable(False)
+    names = [q for q, _ in capi.profile_records() if q.startswith("gms_")]
+    capi.profile_reset()
+    assert names == [kernel] if kernel else not {BRIEF, HELD} & set(names), names
 
 
 @pytest.mark.parametrize("offsets", sorted(OFFSETS))
@@ -20,18 +33,41 @@ FEW = {"9": CUBE[9:18], "16": CUBE[5:21], **OFFSETS}
                                      (500, (24, 40)), (700, (56, 16)), (900, (40, 72))],
                          ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
 def test_whole_numbers(n, shape, offsets):
-    whole_numbers(n, shape, offsets)
+    whole_numbers(n, shape, offsets, BRIEF)
 
 
-# up to 32 channels with all weights in LDS: few offsets at any size, more of them above what the other kernel takes
+# up to 32 channels with all weights in LDS: few offsets at any size, more of them above what the other kernel takes; and what neither takes
+# (too many channels in or columns, or offsets, for the rows)
 @pytest.mark.parametrize("n,shape,offsets", [(1, (32, 32), "9"), (257, (24, 24), "16"), (3001, (32, 16), "9"), (3001, (40, 32), "16"), (40001, (32, 32), "cube"),
                                              (40001, (24, 32), "gaps"), (33000, (32, 24), "32"), (50000, (16, 16), "17"), (1500, (24, 40), "16"),
                                              (3001, (16, 64), "9"), (35000, (32, 64), "cube")])
 def test_whole_numbers_with_the_weights_held(n, shape, offsets):
-    whole_numbers(n, shape, offsets)
+    whole_numbers(n, shape, offsets, None if shape in ((40, 32), (24, 40), (32, 64)) else HELD)
 
 
-def whole_numbers(n, shape, offsets):
+# the rows on either side of each rule: 1 024 tiles of 32 rows and columns in two workgroups a CU, 384 in one; 512 and 1 024 workgroups of 256 rows
+# with the weights held
+@pytest.mark.parametrize("n,shape,kernel", [(32768, (32, 32), BRIEF), (32769, (32, 32), HELD), (16384, (32, 64), BRIEF), (16385, (32, 64), None),
+                                            (12288, (64, 32), BRIEF), (12289, (64, 32), None), (6144, (48, 64), BRIEF), (6145, (48, 64), None),
+                                            (131072, (32, 32), HELD), (131073, (32, 32), None), (131073, (32, 16), HELD),
+                                            (131072, (16, 64), HELD), (131073, (16, 64), None), (131073, (16, 48), HELD)])
+def test_sides_of_the_rules(n, shape, kernel):
+    from fgms_amd import capi
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("sizes for 256 CUs")
+    capi.set_kernel_policy(0)
+    vox = clouds.cloud_indoor(clouds.rng_for(4), target=n + 4000)[:n]
+    assert len(vox) == n
+    imap, omap, _, kpos = clouds.build_kernel_map(vox, vox, clouds.offsets_cube(3))
+    maps = tuple(torch.from_numpy(np.ascontiguousarray(t.astype(np.int32))).cuda() for t in (kpos, imap, omap))
+    x, w = torch.randn(n, shape[0], device="cuda").half(), torch.randn(27, *shape, device="cuda").half()
+    out = torch.empty(n, shape[1], device="cuda").half()
+    plan = capi.Plan(*maps, n, n)
+    assert_runs(kernel, lambda: capi.conv_fwd(x, w, out, *maps, plan=plan))
+    plan.close()
+
+
+def whole_numbers(n, shape, offsets, kernel):
     from fgms_amd import capi
     capi.set_kernel_policy(0)
     vox = clouds.cloud_indoor(clouds.rng_for(4), target=n)
@@ -48,11 +84,11 @@ def whole_numbers(n, shape, offsets):
     assert want.abs().max() <= 2048
     plan = capi.Plan(*maps, n, n)
     out = torch.full_like(zeros, float("nan")).half()
-    capi.conv_fwd(x, w, out, *maps, plan=plan)
+    assert_runs(kernel, lambda: capi.conv_fwd(x, w, out, *maps, plan=plan))
     assert torch.equal(out.double(), want)
     start = few(n, shape[1])
     out = start.clone()
-    capi.fusion_fwd(x, w, 0, out, maps[0], None, maps[1], maps[2], False, False, plan=plan)
+    assert_runs(kernel, lambda: capi.fusion_fwd(x, w, 0, out, maps[0], None, maps[1], maps[2], False, False, plan=plan))
     assert torch.equal(out.double(), want + start.double())
     plan.close()
 
@@ -68,13 +104,14 @@ def test_mirrored_plan_and_centre(n):
     w = torch.randint(-2, 3, (27, 32, 64), device="cuda").half()
     imap, omap, knnz, kpos = capi.build_kernel_map(vox, vox, clouds.offsets_cube(3))
     want = exact(x.float(), w.float(), torch.zeros(n, 64, device="cuda"), kpos.tolist(), imap.long(), omap.long())[0]
+    got = []
     with torch.no_grad():
-        got = sparse_conv(x, w, KernelMap.from_coords(vox, vox, clouds.offsets_cube(3)), False)
-    assert torch.equal(got.double(), want)
+        assert_runs(BRIEF, lambda: got.append(sparse_conv(x, w, KernelMap.from_coords(vox, vox, clouds.offsets_cube(3)), False)))
+    assert torch.equal(got[0].double(), want)
     imap, omap, knnz, kpos = capi.build_kernel_map(vox, vox, clouds.offsets_cube(3), skip_offset=13)
     plan = capi.Plan(kpos, imap.clone(), omap.clone(), n, n)
     out = torch.zeros(n, 64, device="cuda").half()
-    capi.fusion_fwd(x, w, 0, out, kpos, None, imap, omap, True, False, plan=plan)
+    assert_runs(BRIEF, lambda: capi.fusion_fwd(x, w, 0, out, kpos, None, imap, omap, True, False, plan=plan))
     assert torch.equal(out.double(), want)
     plan.close()
 
@@ -90,7 +127,7 @@ def test_infinite_weights_reach_their_pairs_only(n, shape):
     x, w = torch.randn(n, shape[0], device="cuda").half(), torch.randn(27, *shape, device="cuda").half() / 8
     plan = capi.Plan(*maps, n, n)
     clean, out = (torch.full((n, shape[1]), float("nan"), device="cuda").half() for _ in range(2))
-    capi.conv_fwd(x, w, clean, *maps, plan=plan)
+    assert_runs(BRIEF if n == 1000 else HELD, lambda: capi.conv_fwd(x, w, clean, *maps, plan=plan))
     w[5], w[22] = float("inf"), float("nan")
     capi.conv_fwd(x, w, out, *maps, plan=plan)
     hit = torch.zeros(n, dtype=torch.bool, device="cuda")

@@ -39,10 +39,13 @@ def test_against_oracle(oracle, n, shape, dtype, arch80):
         plan.close()
 
 
-@pytest.mark.parametrize("shape", [(64, 64), (48, 96), (96, 20)])
-def test_one_main_launch(shape):
+# (policy 4: small fp16 layers on the output-stationary kernel too)
+@pytest.mark.parametrize("shape,policy,kernel", [((64, 64), 0, "gms_brief_kernel"), ((48, 96), 0, "gms_brief_kernel"), ((64, 64), 4, "gms_rows_kernel(fwd)"),
+                                                 ((128, 64), 0, "gms_rows_kernel(fwd)"), ((72, 96), 0, "gms_rows_kernel(fwd, masked)"),
+                                                 ((96, 20), 0, "gms_rows_kernel(fwd, masked)")])
+def test_one_main_launch(shape, policy, kernel):
     from fgms_amd import capi
-    capi.set_kernel_policy(0)
+    capi.set_kernel_policy(policy)
     L, D = centre_layer(1500, *shape, np.float16)
     plan = capi.Plan(D["kpos"], D["imap"], D["omap"], D["n_in"], D["n_out"])
     G.run_fwd(capi, D, True, True, False, plan)
@@ -52,4 +55,6 @@ def test_one_main_launch(shape):
     capi.profile_enable(False)
     names = [r[0] for r in capi.profile_records()]
     capi.profile_reset()
-    assert names == ["gms_rows_kernel(fwd)"]
+    plan.close()
+    capi.set_kernel_policy(0)
+    assert names == [kernel]

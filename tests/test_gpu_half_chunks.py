@@ -45,7 +45,7 @@ def test_whole_numbers(n, shape):
     capi.profile_enable(False)
     names = [q[0] for q in capi.profile_records()]
     capi.profile_reset()
-    assert names == ["gms_rows_kernel(fwd)", "bwd_fused_kernel(masked)"], names
+    assert names == ["gms_rows_kernel(fwd, masked)", "bwd_fused_kernel(masked)"], names
     for got, ref in zip((out, gi, gw), want):
         assert torch.equal(got.double(), ref)
     assert torch.isnan(around[:64]).all() and torch.isnan(around[-64:]).all()

@@ -327,7 +327,7 @@ def test_plan_stats(capi):
 def test_scattered_wide_layer_takes_the_pair_stationary_kernel(capi, oracle, dtype):
     """A 256 -> 256 layer over a scattered cloud (few pairs per 64-row block and offset):
     automatic dispatch weighs the empty row slots of the output-stationary kernel against
-    the atomics of the pair-stationary one and picks the latter; a dense 64 -> 64 layer
+    the atomics of the pair-stationary one and picks the latter; a dense 128 -> 64 layer
     stays output-stationary.  Results against the oracle either way."""
     L = clouds.config_case(5, dtype, scale=0.08)
     D = G.to_dev(L)
@@ -364,7 +364,7 @@ def test_scattered_wide_layer_takes_the_pair_stationary_kernel(capi, oracle, dty
     assert np.array_equal(first, second)
     G.assert_close(first, ref, G.mode_of(L["in_feats"].dtype, False), "fwd, policy 4")
 
-    L = layer(5, 64, 64, np.float16)
+    L = layer(5, 128, 64, np.float16)         # (up to 64 channels in: the small launches' kernel)
     D = G.to_dev(L)
     plan = capi.Plan(D["kpos"], D["imap"], D["omap"], D["n_in"], D["n_out"])
     capi.profile_enable(True)
