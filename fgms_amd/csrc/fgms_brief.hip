@@ -286,7 +286,7 @@ size_t brief_lds(const GmsArgs &a) {
 
 // What either kernel asks of a layer of up to `most` channels in.
 static bool brief_layer(const GmsArgs &a, const Plan *p, int most) {
-  if (a.dtype != FGMS_F16 || a.transpose_w || a.prepacked || a.dense_k >= 0 || a.n_pairs == 0 || a.n_dst == 0 || kernel_policy() != 0) return false;
+  if (a.dtype != FGMS_F16 || a.transpose_w || a.prepacked || a.dense_k >= 0 || a.n_pairs == 0 || a.n_dst == 0 || kernel_policy() != 0 || !raw_weights_enabled()) return false;
   if (!p || !p->groups.empty() || !p->has_tables || !p->fwd_ok || a.k_vol != p->k_vol || a.n_dst != p->n_out || a.n_src != p->n_in) return false;
   if (a.c_in % 8 || a.c_in < 16 || a.c_in > most || a.c_out % 8 || a.c_out < 16 || a.k_vol > kBriefOffsets) return false;
   if (reinterpret_cast<uintptr_t>(a.w) % 16 || reinterpret_cast<uintptr_t>(a.src) % 16 || reinterpret_cast<uintptr_t>(a.dst) % 4) return false;
@@ -322,7 +322,7 @@ static BriefArgs brief_args(const GmsArgs &a, const Plan *p) {
 // 64 -> 64 over 2 k 12.4 / 6.7 and 10.0 / 6.6, 4 k (250) 12.5 / 8.2 and 10.0 / 7.6, 6 k (376) 12.5 / 10.3, 8 k (500) 12.5 / 12.1 and 9.9 / 11.1;
 // 48 -> 48 over 4 k 11.9 / 7.1 and 17.6 / 7.0; 64 -> 128 over 2 k (252) 12.5 / 8.2 and 10.5 / 7.6.
 bool brief_gms_pays(const GmsArgs &a, const Plan *p) {
-  if (!brief_layer(a, p, 64) || a.k_vol <= kBriefWaves) return false;
+  if (!brief_layer(a, p, 64) || a.k_vol <= kBriefWaves || !half_tiles_enabled()) return false;
   const int64_t tiles = (a.n_dst + kBriefRows - 1) / kBriefRows * ((a.c_out + 31) / 32);
   return 2 * tiles <= (int64_t)num_cus() * (brief_lds(a) <= 80 << 10 ? 8 : 3);
 }

@@ -314,6 +314,8 @@ int launch_side_job(const SideJob &job, hipStream_t stream);
 // against 108; the submanifold maps that gain by it have 10.)
 inline bool worth_96_columns(int64_t n_pairs, int64_t n_a, int64_t n_b) { return n_pairs >= 5 * (n_a > n_b ? n_a : n_b); }
 bool split_bf16_enabled();   // products of fp32 tensors in bf16 parts: three a value, two where the caller allows tf32 precision
+bool raw_weights_enabled();  // fp16 weights read as they lie where that pays
+bool half_tiles_enabled();   // tiles of less than 256 rows for launches that do not fill the chip
 // Small fp16 forward launches, all offsets of a tile at once (fgms_brief.hip).
 bool brief_gms_pays(const GmsArgs &a, const Plan *p);
 int launch_brief_gms(const GmsArgs &a, const Plan *p);

@@ -1136,12 +1136,6 @@ Shape shape_of(const GmsArgs &a) {
   return s;
 }
 
-// FGMS_RAW_WEIGHTS=0 keeps the forward pass on re-laid weights (for comparison).
-bool raw_weights_enabled() {
-  static const bool on = !(getenv("FGMS_RAW_WEIGHTS") && atoi(getenv("FGMS_RAW_WEIGHTS")) == 0);
-  return on;
-}
-
 // --- channel counts that fill no whole tile (RAGGED) --------------------------------------
 // 32-column tiles per wave (and blocks of a weight-gradient tile) for c columns, 0: not served.
 int ragged_tiles(int c, bool three) {
@@ -1271,12 +1265,6 @@ int launch_pairs(const GmsArgs &a, const Shape &s) {
   }
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;
-}
-
-// FGMS_HALF_TILES=0 keeps small launches on 256-row tiles (for comparison).
-bool half_tiles_enabled() {
-  static const bool on = !(getenv("FGMS_HALF_TILES") && atoi(getenv("FGMS_HALF_TILES")) == 0);
-  return on;
 }
 
 // Grid of an output-stationary launch over n_dst destination rows: tiles of 256 rows from the
@@ -1769,6 +1757,18 @@ int launch_side_job(const SideJob &job, hipStream_t stream) {
   side_job_kernel<<<(unsigned)job.blocks, 256, 0, stream>>>(job);
   FGMS_HIP_TRY(hipGetLastError());
   return FGMS_OK;
+}
+
+// FGMS_RAW_WEIGHTS=0 keeps the forward pass on re-laid weights (for comparison).
+bool raw_weights_enabled() {
+  static const bool on = !(getenv("FGMS_RAW_WEIGHTS") && atoi(getenv("FGMS_RAW_WEIGHTS")) == 0);
+  return on;
+}
+
+// FGMS_HALF_TILES=0 keeps small launches on 256-row tiles (for comparison).
+bool half_tiles_enabled() {
+  static const bool on = !(getenv("FGMS_HALF_TILES") && atoi(getenv("FGMS_HALF_TILES")) == 0);
+  return on;
 }
 
 // FGMS_SPLIT_BF16=0 keeps fp32 tensors on fp32 MFMAs, in full precision and in "tf32" mode (for comparison).

@@ -91,6 +91,40 @@ def test_small_launches_on_256_row_tiles():
     assert "bwd_fused_kernel" in names and "gms_rows_kernel(fwd)" in names, names
 
 
+DISPATCH_CHILD = r"""
+import json, sys
+import numpy as np, torch
+sys.path.insert(0, %r)
+from fgms_amd import capi, clouds
+from oracle import fgms_oracle as oracle
+from tests import gpu_util as G
+capi.set_kernel_policy(0)
+for n, c_in, c_out in ((2000, 64, 64), (60000, 32, 32)):
+    vox = clouds.cloud_indoor(clouds.rng_for(4), target=n)
+    L = clouds.submanifold_case(vox, c_in, c_out, np.float16, np.random.default_rng(n))
+    D = G.to_dev(L)
+    plan = capi.Plan(D["kpos"], D["imap"], D["omap"], D["n_in"], D["n_out"])
+    capi.profile_reset(); capi.profile_enable(True)
+    out = G.run_fwd(capi, D, fused=True, plan=plan)
+    capi.profile_enable(False)
+    print("KERNELS", json.dumps([n for n, _ in capi.profile_records()]))
+    G.assert_close(out, oracle.c_fwd(L["in_feats"], L["kernel"], L["knnz"], L["imap"], L["omap"], L["n_out"]), "fp16", "fwd")
+    plan.close()
+""" % ROOT
+
+
+@pytest.mark.parametrize("env,kernels", [({}, ["gms_brief_kernel", "gms_held_kernel"]), ({"FGMS_RAW_WEIGHTS": "0"}, ["gms_rows_kernel(fwd)"] * 2),
+                                         ({"FGMS_HALF_TILES": "0"}, ["gms_rows_kernel(fwd)", "gms_held_kernel"])],
+                         ids=["default", "re-laid weights", "256-row tiles"])
+def test_switches_reach_the_layers_with_kernels_of_their_own(env, kernels):
+    """Small fp16 layers, and such of up to 32 channels, under automatic dispatch: their kernels read the weights as they lie, and the
+    small ones' tiles have 32 rows, so that the switches turn them off."""
+    r = subprocess.run([sys.executable, "-c", DISPATCH_CHILD], env={**os.environ, **env}, cwd=ROOT, stdout=subprocess.PIPE,
+                       stderr=subprocess.STDOUT, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout[-3000:]
+    assert [json.loads(l[8:]) for l in r.stdout.splitlines() if l.startswith("KERNELS ")] == [[k] for k in kernels]
+
+
 FULL_SIZE_CHILD = r"""
 import sys
 import numpy as np, torch
