@@ -337,3 +337,40 @@ def test_pair_view_is_not_built_for_an_estimate(capi, oracle):
         assert [gpu_trace.kernels(both).count("pair_view_kernel") for _ in range(2)] == [int(walks), 0], shape
         G.assert_close(out.cpu().numpy(), oracle.c_fwd(L["in_feats"], L["kernel"], L["knnz"], L["imap"], L["omap"], L["n_out"]), "fp32", "fwd")
         plan.close()
+
+
+def test_layer_captured_after_an_eager_call_of_it_walks_the_pair_view(capi, oracle):
+    """An fp32 layer over a thinned cloud, captured after eager fp16 calls on its map and after an eager call of its own: the kernels of
+    the replays (the pair-stationary ones, and the view's), the results of both."""
+    vox = clouds.cloud_indoor(clouds.rng_for(2), target=60000)
+    vox = np.ascontiguousarray(vox[np.sort(np.random.default_rng(1).permutation(len(vox))[:20000])])
+    L = clouds.submanifold_case(vox, 128, 128, np.float32, np.random.default_rng(5))
+    D = G.to_dev(L)
+    maps = (D["kpos"], D["imap"], D["omap"])
+    plan = capi.Plan(*maps, D["n_in"], D["n_out"])
+    want = oracle.c_fwd(L["in_feats"], L["kernel"], L["knnz"], L["imap"], L["omap"], L["n_out"])
+    out = torch.empty_like(D["out_grad"])
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+
+    def captured():
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side, capture_error_mode="thread_local"):
+            capi.conv_fwd(D["in_feats"], D["kernel"], out, *maps, plan=plan)
+        for _ in range(2):
+            out.fill_(7.0)
+            ran = gpu_trace.kernels(graph.replay)
+            G.assert_close(out.cpu().numpy(), want, "fp32", "captured")
+        return ran
+
+    with torch.cuda.stream(side):
+        capi.conv_fwd(D["in_feats"], D["kernel"], out, *maps)                             # (workspaces, without a plan)
+        capi.conv_fwd(D["in_feats"].half(), D["kernel"].half(), out.half(), *maps, plan=plan)
+    torch.cuda.synchronize()
+    assert "gms_pairs_kernel" in captured()
+    with torch.cuda.stream(side):
+        capi.conv_fwd(D["in_feats"], D["kernel"], out, *maps, plan=plan)
+    torch.cuda.synchronize()
+    ran = captured()
+    assert "gms_rows_kernel" in ran and "gms_pairs_kernel" not in ran, ran
+    plan.close()
