@@ -288,13 +288,33 @@ void tile_blocks(const WgradArgs &a, bool shares_grid, int *bi, int *bj) {
   }
 }
 
+// Slices of fewer stages, for launches of few workgroups, which last as long as one of them: of eight stages (64 pairs each) for at most
+// `most` workgroups, to the multiple of eight below or above.  Every slice more is a tile more to flush with atomics, as long as two or three
+// stages, and the shorter a pair's work and the bigger the tile the sooner that is more than it saves.
+int64_t slices_of_eight(const WgradArgs &a, int ty, int64_t most, bool above = false) {
+  const int64_t slices = a.n_pairs / ((int64_t)a.k_vol * 8 * 64), room = most / ((int64_t)a.k_vol * ty);
+  return std::min((slices + 7) / 8 * 8, (room + (above ? 7 : 0)) / 8 * 8);
+}
+// The fp16 workgroup body's.  Beside the input gradient: three quarters of the CUs, and all of them from twelve stages on where the input
+// channels are the wide ones (the input gradient then contracts over few channels and is the shorter part).
+// Transposed layers over stride-2 maps, slices of 16 stages / these, us.  Backward launch, 8 offsets: 64 -> 128 over 60 k pairs 23.0 / 17.8, 100 k 24.1 /
+// 21.5, over 145 k 26.9 and with all CUs 31.0; 128 -> 64 24.3 / 19.3, 26.6 / 26.0, 22.4 and 24.6, over 200 k 27.8 / 26.5.  27 offsets, with 432
+// workgroups: 64 -> 128 over 130 k 30.6 and 34.1, 128 -> 64 over 142 k 28.1 and 29.6, but 128 -> 32 over 167 k 26.2 and 24.2.  Alone, 27 offsets: 32 -> 128
+// over 130 k 15.2 / 12.7, 128 -> 64 17.7 and 19.0, over 206 k 23.5 / 21.5.
+int64_t shortest_chain(const WgradArgs &a, int ty, int bi, int bj, bool shares_grid) {
+  const int64_t cus = num_cus(), room = cus / ((int64_t)a.k_vol * ty);
+  auto nearest = [&](int stages) { return (a.n_pairs / ((int64_t)a.k_vol * stages * 64) + 4) / 8 * 8; };
+  const int64_t nearest_eight = std::min(nearest(8), (room + 7) / 8 * 8);
+  const bool small = bi * bj == 4;
+  if (!shares_grid) return small ? slices_of_eight(a, ty, cus, true) : std::max(slices_of_eight(a, ty, cus), nearest_eight);
+  return std::max(slices_of_eight(a, ty, cus * 3 / 4), bi <= bj ? 0 : small ? nearest_eight : std::min(nearest(12), room / 8 * 8));
+}
+
 // Slices per offset: from the plan's row bands when it has them, `stride` bands to
 // a slice so that about `want_wgs` workgroups result; else equal pair counts,
 // enough to fill the chip a few times with at least ~16 stages of pairs per slice
-// on average, or eight of 64 pairs while there is a workgroup to a CU at most (a workgroup's chain of stages is then what the launch
-// takes, beyond it the atomics of the flushes: the transposed layer 128 -> 64 over a stride-2 map, backward launch, 192 / 256 / 384
-// workgroups over 200 k pairs 28.5 / 25.9 / 31.1 us, 64 / 128 over 60 k 21.0 / 15.0).  A multiple of 8 (one per XCD).
-SliceMap choose_slices(const WgradArgs &a, int ty, int stage_pairs, int64_t want_wgs) {
+// on average, or `at_least` however few these are (see shortest_chain).  A multiple of 8 (one per XCD).
+SliceMap choose_slices(const WgradArgs &a, int ty, int stage_pairs, int64_t want_wgs, int64_t at_least = 0) {
   SliceMap m{};
   if (a.plan && a.plan->bands_ok && a.plan->band_start && a.plan->k_vol == a.k_vol &&
       a.plan->n_pairs == a.n_pairs && a.plan->n_out == a.n_out) {
@@ -315,8 +335,7 @@ SliceMap choose_slices(const WgradArgs &a, int ty, int stage_pairs, int64_t want
     return m;
   }
   int64_t slices = want_wgs / ((int64_t)a.k_vol * ty);
-  int64_t by_work = a.n_pairs / ((int64_t)a.k_vol * 16 * stage_pairs);
-  if (stage_pairs == 64) by_work = std::max(by_work, std::min(a.n_pairs / ((int64_t)a.k_vol * 8 * stage_pairs), num_cus() / ((int64_t)a.k_vol * ty)));
+  const int64_t by_work = std::max(a.n_pairs / ((int64_t)a.k_vol * 16 * stage_pairs), at_least);
   if (slices > by_work) slices = by_work;
   slices = (slices + 7) / 8 * 8;
   m.slices = (int)(slices < 8 ? 8 : slices);
@@ -369,6 +388,15 @@ bool skinny_shape(const WgradArgs &a) {
          (size_t)a.c_in * esz % 8 == 0;
 }
 
+// (Lists without bands, slices of 16 stages / these, us.  fp32, 8 offsets, 120 k pairs: 16 -> 64 32.4 / 23.7, 8 -> 64 18.4 / 15.3; 27 offsets, where the
+// multiple of eight above the CUs are 432 workgroups, 167 k: 8 -> 64 17.6 / 16.3, but 16 -> 64 31.9 and 37.6.  fp16 walks a pair in less time:
+// 27 offsets, 130 k, 16 -> 64 30.2 and 43.7, 16 -> 16 19.0 and 24.4; 8 offsets, 60 k, 16 -> 64 32.0 / 26.8, 16 -> 16 19.7 and 20.2.)
+SliceMap skinny_slices(const WgradArgs &a, int wgs_per_cu) {
+  const int64_t cus = num_cus();
+  const int64_t at_least = a.dtype == FGMS_F32 ? slices_of_eight(a, 1, cus, a.c_in <= 8) : a.c_out == 64 ? slices_of_eight(a, 1, cus / 2) : 0;
+  return choose_slices(a, 1, 64, cus * wgs_per_cu, at_least);
+}
+
 template <typename T, int CS, int CD>
 int launch_skinny(const WgradArgs &a, float *acc32) {
   // Few, big workgroups (about two to a CU): measured on the 4 -> 32 layer over 2.1 M
@@ -377,7 +405,7 @@ int launch_skinny(const WgradArgs &a, float *acc32) {
   // work on the same offset and their closing atomic adds queue on the same addresses),
   // and 40-68 us with 16-wave workgroups.
   static const int wgs_per_cu = getenv("FGMS_SKINNY_WGS") ? atoi(getenv("FGMS_SKINNY_WGS")) : 2;
-  const SliceMap smap = choose_slices(a, 1, 64, (int64_t)num_cus() * wgs_per_cu);
+  const SliceMap smap = skinny_slices(a, wgs_per_cu);
   const int64_t tiles = (int64_t)smap.slices * a.k_vol;
   const size_t lds = (size_t)(kSkinnyThreads / 64 - 1) * CS * CD * sizeof(float);
   auto kern = wgrad_skinny_kernel<T, CS, CD>;
@@ -444,7 +472,7 @@ double padded_wgrad_us(const WgradArgs &p) {
   WgradGeometry g;
   if (skinny_shape(p)) {
     per_row = 0.076 / 512 * p.c_in * p.c_out;
-    cells = (double)choose_slices(p, 1, 64, (int64_t)num_cus() * 2).slices * p.k_vol;
+    cells = (double)skinny_slices(p, 2).slices * p.k_vol;
   } else if (wgrad_geometry(p, &g) == FGMS_OK) {
     const int blocks = g.bi * g.bj;
     per_row = blocks == 1 ? (g.split ? 0.083 : 0.05) : blocks == 2 ? (g.split ? 0.122 : 0.095)
@@ -516,7 +544,7 @@ int wgrad_geometry(const WgradArgs &a, WgradGeometry *g, bool shares_grid) {
     g->smap.by_xcd = ((size_t)a.n_in * a.c_in + (size_t)a.n_out * a.c_out) * esz > 8 << 20;
     g->tiles = g->smap.by_xcd ? tiles_by_xcd(a.n_pairs, chunk, a.k_vol) : (a.n_pairs + chunk - 1) / chunk + a.k_vol;
   } else {
-    g->smap = choose_slices(a, g->ty, sp, (int64_t)num_cus() * 4);
+    g->smap = choose_slices(a, g->ty, sp, (int64_t)num_cus() * 4, f16 ? shortest_chain(a, g->ty, bi, bj, shares_grid) : 0);
     g->tiles = (int64_t)g->smap.slices * a.k_vol;
   }
   g->split = !f16 && a.reduced && split_bf16_enabled() ? 2 : 0;
