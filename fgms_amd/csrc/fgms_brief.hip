@@ -168,6 +168,7 @@ __global__ __launch_bounds__(kHeldWaves * 64, 4) void gms_held_kernel(BriefArgs 
     if (tile < 0) return;
     tile &= 0xFFFFFF;
   }
+  if (tile * (kHeldWaves * 32) >= a.n_dst) return;
   extern __shared__ int4v lds[];
   __shared__ int out_rows[kHeldWaves][32];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -272,8 +273,10 @@ __global__ __launch_bounds__(kHeldWaves * 64, 4) void gms_held_kernel(BriefArgs 
         if (rows >> ((r / 4) * 8 + h * 4 + r % 4) & 1) acc[0][0][r] += own[r];
     }
   }
+  // (Added to what is there: all old values requested before the first sum.  One by one, each behind the store before it, 32 -> 32 over 35 k
+  // indoor voxels 13.6 us and 16 -> 64 over 60 k 15.8, 12.2 and 13.6 with the kernels that had these layers before; this way 12.4 and 12.2.)
   if (a.overwrite) write_tile<__half, 1, kTileStore, true>(acc, a.dst, out_rows[wave], a.c_dst, nt0, lane);
-  else if (mask) write_tile<__half, 1, kTileAdd, true>(acc, a.dst, out_rows[wave], a.c_dst, nt0, lane);
+  else if (mask) add_rows<__half, 1, true>(acc, a.dst, out_rows[wave], a.c_dst, nt0, lane);
 }
 
 int brief_steps(const GmsArgs &a) { return (a.c_in + 15) / 16; }
@@ -347,11 +350,12 @@ int launch_brief_gms(const GmsArgs &a, const Plan *p) {
 // and 22.2 / 19.6, 200 k, where some workgroups wait for a second round, 22.6 / 22.2 and 28.3 / 28.9; 16 -> 32 over 60 k 10.1 / 7.6 and 10.6 / 8.0,
 // 200 k 27.7 / 15.6 and 32.4 / 21.0; 32 -> 16 over 60 k 21.7 / 10.4 and 25.4 / 11.0, 200 k 50.1 / 21.4 and 57.1 / 27.8; 16 -> 16 over 100 k 11.4 / 8.1 and
 // 14.9 / 11.7.  More than 32 columns gather their rows twice: 16 -> 48 over 60 k 13.5 / 11.0, 200 k 37.9 / 26.5; 16 -> 64 over 30 k 10.7 / 8.3, 100 k
-// 17.1 / 14.7 and 20.3 / 19.4, 200 k 22.2 / 27.3; 32 -> 64 over 30 k 12.2 / 11.7, 60 k 14.5 / 17.1.)
+// 17.1 / 14.7 and 20.3 / 19.4, 200 k 22.2 / 27.3, added to a result over 100 k 20.2 / 16.7 and 21.1 / 20.1, 120 k 21.5 / 20.8 and 22.4 / 24.9;
+// 32 -> 64 over 30 k 12.2 / 11.7, 60 k 14.5 / 17.1.)
 bool held_gms_pays(const GmsArgs &a, const Plan *p) {
   if (!brief_layer(a, p, 32) || a.c_out > 64 || a.k_vol <= 8) return false;
   const int64_t workgroups = (a.n_dst + kHeldWaves * 32 - 1) / (kHeldWaves * 32) * ((a.c_out + 31) / 32);
-  if (a.c_in <= 16) return a.c_out <= 48 || workgroups <= 4 * (int64_t)num_cus();
+  if (a.c_in <= 16) return a.c_out <= 48 || 2 * workgroups <= (a.overwrite ? 8 : 7) * (int64_t)num_cus();
   return a.c_out <= 16 || (a.c_out <= 32 && workgroups <= 2 * (int64_t)num_cus());
 }
 
@@ -361,7 +365,9 @@ int launch_held_gms(const GmsArgs &a, const Plan *p) {
   const size_t lds = (size_t)(a.k_vol + kHeldWaves) * brief_steps(a) * 1024;
   const int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kern), lds);
   if (rc != FGMS_OK) return rc;
-  const unsigned tiles = p->tile_out ? (unsigned)p->tile_grid_out : (unsigned)((a.n_dst + kHeldWaves * 32 - 1) / (kHeldWaves * 32));
+  // (without the plan's table a multiple of eight: the two workgroups of a tile of 64 columns write halves of the same lines, and belong on the
+  // same XCD)
+  const unsigned tiles = p->tile_out ? (unsigned)p->tile_grid_out : (unsigned)((a.n_dst + kHeldWaves * 32 - 1) / (kHeldWaves * 32) + 7) / 8 * 8;
   {
     ProfileScope prof("gms_held_kernel", a.stream);
     kern<<<dim3(tiles + (unsigned)b.side.blocks, (unsigned)((a.c_out + 31) / 32)), kHeldWaves * 64, lds, a.stream>>>(b, p->tile_out);

@@ -67,6 +67,24 @@ def test_sides_of_the_rules(n, shape, kernel):
     plan.close()
 
 
+@pytest.mark.parametrize("n,kernel", [(114688, HELD), (114689, None)])
+def test_sixteen_channels_added_to_64_columns(n, kernel):
+    """Results that are added to, of two column tiles a row: up to 896 workgroups of 256 rows."""
+    from fgms_amd import capi
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("sizes for 256 CUs")
+    capi.set_kernel_policy(0)
+    vox = clouds.cloud_indoor(clouds.rng_for(4), target=n + 4000)[:n]
+    imap, omap, _, kpos = clouds.build_kernel_map(vox, vox, clouds.offsets_cube(3))
+    maps = tuple(torch.from_numpy(np.ascontiguousarray(t.astype(np.int32))).cuda() for t in (kpos, imap, omap))
+    x, w, start = (torch.randint(-2, 3, s, device="cuda").half() for s in ((n, 16), (27, 16, 64), (n, 64)))
+    want = exact(x.float(), w.float(), torch.zeros_like(start, dtype=torch.float32), kpos.tolist(), maps[1].long(), maps[2].long())[0]
+    plan, out = capi.Plan(*maps, n, n), start.clone()
+    assert_runs(kernel, lambda: capi.fusion_fwd(x, w, 0, out, maps[0], None, maps[1], maps[2], False, False, plan=plan))
+    assert torch.equal(out.double(), want + start.double())
+    plan.close()
+
+
 def whole_numbers(n, shape, offsets, kernel):
     from fgms_amd import capi
     capi.set_kernel_policy(0)
