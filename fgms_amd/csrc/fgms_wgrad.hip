@@ -510,6 +510,8 @@ static void wave_geometry(const WgradArgs &a, WgradGeometry *g, bool shares_grid
   g->lds = lds < red ? red : lds;
 }
 
+constexpr size_t kTwoToACu = 56 << 10;      // bytes of LDS that leave no room for a third workgroup
+
 int wgrad_geometry(const WgradArgs &a, WgradGeometry *g, bool shares_grid) {
   if (skinny_shape(a) || !mfma_wgrad_shape(a)) {
     set_error("wgrad_geometry: not a shape of the MFMA weight-gradient kernels");
@@ -550,6 +552,12 @@ int wgrad_geometry(const WgradArgs &a, WgradGeometry *g, bool shares_grid) {
   g->split = !f16 && a.reduced && split_bf16_enabled() ? 2 : 0;
   g->lds = g->split ? 2 * (size_t)sp * 2 * ((bi * 32 + 16) + (bj * 32 + 16)) * 2
                     : 2 * (size_t)sp * ((bi * 32 + pad) + (bj * 32 + pad)) * esz;
+  // A third workgroup on a CU slows the other two down.  Where the launch, alone and of one tile an offset, takes as many rounds of the chip with
+  // two, there are two.  (128 -> 64, 864 cells, over 85 k indoor voxels with three / two 46.6 / 44.9 us, 140 k 69.9 / 65.2, 120 k LiDAR 63.1 /
+  // 56.7; 1 728 cells, 200 k 88.9 / 92.9.  Two tiles share their rows: 64 -> 256 over 70 k 72.0 / 80.1.)
+  const int64_t cus = num_cus();
+  if (f16 && bi * bj == 8 && g->ty == 1 && !shares_grid && (g->tiles - 1) / (cus * 3) == (g->tiles - 1) / (cus * 2) && g->lds < kTwoToACu)
+    g->lds = kTwoToACu;
   return FGMS_OK;
 }
 
