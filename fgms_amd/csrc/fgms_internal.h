@@ -93,6 +93,8 @@ inline int walk_offset(const GmsArgs &a, bool first) {
   return first ? 2 * (a.first_offset - 1) + 1 : a.dense_k >= 0 ? 2 * a.dense_k + (a.overwrite ? 1 : 0) : a.first_offset - 1;
 }
 
+constexpr size_t kTwoToACu = 56 << 10;      // bytes of LDS that leave no room for a third workgroup on a CU
+
 struct WgradArgs {
   const void *in;     // [n_in, c_in]
   const void *gout;   // [n_out, c_out]

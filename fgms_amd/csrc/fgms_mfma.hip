@@ -1547,6 +1547,20 @@ int launch_fused(const GmsArgs &d, const Shape &s, const Plan *p, const WgradArg
   size_t lds = g.lds;
   const size_t lds_rows = rg.half_tiles ? rows_group_chunks<T, NT, S, kHalfMT>(raw) * 16 : rows_group_chunks<T, NT, S, 2>(raw) * 16;
   if (lds < lds_rows) lds = lds_rows;
+  // Tiles of 64 x 128 leave room for a third workgroup on a CU, which slows the other two down: it pays where workgroups wait for a slot, not
+  // where nearly all of them start at once and the last to end is what the launch takes.  So two where the input gradient's tiles are
+  // shared (it fills the chip about once) and there are cells for a round and a half of it, and up to seven workgroups to two CUs over dense maps.
+  // Backward call, with three / two (indoor voxels, 27 offsets): 64 -> 128 over 30 k (672 workgroups) 38.8 / 36.4 us, 50 k (832) 55.5 / 51.7, 60 k (912)
+  // 64.8 / 58.7, 70 k (1 056) 78.0 / 68.3, LiDAR 50 k 59.8 / 55.6 but 70 k 82.8 / 88.8; not shared 85 k (1 200) 70.6 / 73.4, 100 k 80.9 / 83.8, 120 k
+  // 99.8 / 96.8, LiDAR 112.0 / 114.7.  128 -> 64 30 k (912, shared) 42.1 / 38.3, 50 k (832) 52.0 / 48.4, 60 k (902) 59.1 / 62.7, 70 k 71.7 / 75.1, 150 k
+  // 107.5 / 107.6.  Transposed lists of a stride-2 map, 27 offsets, 64 -> 128 over 297 k pairs (704, 432 of them cells) 43.3 / 39.8, over 212 k (584, 216) 35.1 /
+  // 41.0.  Over 140 launches of either kind the rule is 0.7 % over the better of the two, always three 1.5 %, always two 2.5 %.
+  if constexpr (sizeof(T) == 2 && BI * BJ == 8) {
+    const int64_t cus = num_cus(), wgs = (int64_t)row_x * row_y * row_z + g.tiles;
+    const bool shared = row_z > 1 && 2 * g.tiles > 3 * cus;
+    const bool dense = g.smap.band_start && w.n_pairs >= 5 * std::max(w.n_in, w.n_out);
+    if (g.ty == 1 && (shared || (dense && 2 * wgs < 7 * cus)) && lds < kTwoToACu) lds = kTwoToACu;
+  }
   { const int rc_lds = allow_dynamic_lds(reinterpret_cast<const void *>(kern), (size_t)lds); if (rc_lds != FGMS_OK) return rc_lds; }
   {
     ProfileScope prof(RAGGED     ? (raw == 4 ? "bwd_fused_kernel(masked, bf16x3)" : "bwd_fused_kernel(masked)")

@@ -510,8 +510,6 @@ static void wave_geometry(const WgradArgs &a, WgradGeometry *g, bool shares_grid
   g->lds = lds < red ? red : lds;
 }
 
-constexpr size_t kTwoToACu = 56 << 10;      // bytes of LDS that leave no room for a third workgroup
-
 int wgrad_geometry(const WgradArgs &a, WgradGeometry *g, bool shares_grid) {
   if (skinny_shape(a) || !mfma_wgrad_shape(a)) {
     set_error("wgrad_geometry: not a shape of the MFMA weight-gradient kernels");

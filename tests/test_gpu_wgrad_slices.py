@@ -58,3 +58,25 @@ def test_whole_numbers_on_either_side_of_the_rules(shape, dtype, offsets, pairs)
     assert torch.equal(alone.float(), want) and torch.equal(both.float(), want)
     view.close()
     plan.close()
+
+
+# voxels on either side of what leaves a third workgroup on a CU beside 64 x 128 tiles
+@pytest.mark.parametrize("shape,n", [((64, 128), 72001), ((64, 128), 85001), ((128, 64), 36001), ((128, 64), 50001), ((128, 64), 62001)],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_whole_numbers_beside_the_input_gradient(shape, n):
+    from fgms_amd import capi, clouds
+    from tests.test_gpu_fp32_parts import exact
+    capi.set_kernel_policy(0)
+    vox = clouds.cloud_indoor(clouds.rng_for(4), target=n)
+    n = len(vox)
+    imap, omap, _, kpos = clouds.build_kernel_map(vox, vox, clouds.offsets_cube(3))
+    maps = tuple(torch.from_numpy(np.ascontiguousarray(t.astype(np.int32))).cuda() for t in (kpos, imap, omap))
+    few = lambda *s: (torch.randint(0, 32, s, device="cuda").lt(1).float() - torch.randint(0, 32, s, device="cuda").lt(1).float()).half()
+    x, g, w = few(n, shape[0]), few(n, shape[1]), few(27, *shape)
+    _, want_x, want_w = exact(x, w, g, kpos.tolist(), maps[1].long(), maps[2].long())
+    assert max(want_x.abs().max(), want_w.abs().max()) < 2048
+    gin, gw = torch.full_like(x, float("nan")), torch.full_like(w, float("nan"))
+    plan = capi.Plan(*maps, n, n)
+    capi.conv_bwd(g, x, w, gin, gw, *maps, plan=plan)
+    assert torch.equal(gin.double(), want_x) and torch.equal(gw.double(), want_w)
+    plan.close()
