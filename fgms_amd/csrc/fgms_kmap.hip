@@ -20,7 +20,7 @@
 //               both sides, mirrored offsets) is its own mirror image, so one order and one table
 //               serve both directions.  Steps 4 and 5 share launches (kmap_sizes_kernel).
 // Bound by latencies: eight launches of one or two waves' worth of dependent accesses each.  At 100 k LiDAR voxels x 27 offsets they
-// take 77 us of the stream; with a scan of its own and the lists in front of the plan's sort 98 us; lists alone and a plan from
+// take 81 us of the stream; with a scan of its own and the lists in front of the plan's sort 98 us; lists alone and a plan from
 // them afterwards 140 and 195 us, each behind a wait of the host for the one before.
 #include <immintrin.h>
 #include <stdlib.h>

@@ -516,7 +516,7 @@ __device__ __forceinline__ void wgrad_wg_body(
   // (fp16: rows without padding, see tr_frag_dense.  Padded by 32 bytes the reads met in the banks, 0.87 conflict cycles to an LDS
   // instruction over 128 x 128, and the stages of 64 x 128 left room for two workgroups on a CU instead of three.  Backward launch,
   // padded / dense: 128 -> 64 over 60 k indoor voxels 69.8 / 61.9 us, 64 -> 128 over 100 k 92 / 89, stride 2 transposed 128 -> 64
-  // over 200 k 31.8 / 27.8, 128 -> 128 over 120 k LiDAR ones 170 / 158 .. 166.)
+  // over 200 k 31.8 / 27.8, 128 -> 128 over 120 k LiDAR ones 145.2 / 144.6, 50 k scattered 90.9 / 87.2.)
   constexpr bool kDense = sizeof(T) == 2;
   constexpr int LDI = CI + (kDense ? 0 : W::pad), LDO = CO + (kDense ? 0 : W::pad);
   constexpr int NCI = CI / E, NCO = CO / E;   // 16-byte chunks per staged row
